@@ -31,6 +31,10 @@ inline void bind_decoder(py::module_& m) {
      py::arg("R"), py::arg("ldr"), py::arg("M"), py::arg("N"), py::arg("K"), py::arg("act"), py::arg("out_f32"),
      py::arg("st"), py::arg("wsh") = 0, py::arg("rowstat") = 0, py::arg("colsum") = 0, py::arg("ws") = 0,
      py::arg("ws_bytes") = 0);
+  m.def("gemm_set_mid", [](int tile, int splits) { return dnn_gemm_set_mid(tile, splits); });
+  m.def("gemm_is_skinny", [](int M, int N, int K, int norm, int frag, long long ws_bytes) {
+    return dnn_gemm_is_skinny(M, N, K, norm, frag, ws_bytes);
+  });
   m.def("sample_topk", [](u64 x, int ld, int M, int N, u64 out, float temperature, int topk, unsigned seed, u64 step,
                           u64 st) {
     return dnn_sample_topk(CP(x), ld, M, N, reinterpret_cast<int*>(out), temperature, topk, seed,

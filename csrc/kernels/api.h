@@ -14,6 +14,10 @@ int dnn_gemm_bf16(const void* A, int lda, const void* W, int ldw, void* C, int l
                   long long ws_bytes = 0);
 int dnn_row_stats(const void* x, int ldx, float* stats, int M, int N, float eps, int rms, hipStream_t st);
 int dnn_gemm_set_tile(int tile);
+// tile of gemm_mid.h's table and K split for every call above 64 rows (tests, A/B; -1: chosen)
+int dnn_gemm_set_mid(int tile, int splits);
+// whether M rows run on the decode kernels (norm: dnn_gemm_skinny_norm; frag: the weight has its fragment-order copy)
+int dnn_gemm_is_skinny(int M, int N, int K, int norm, int frag, long long ws_bytes);
 int dnn_gemm_set_anatomy(int bits);
 int dnn_gemm_set_skinny_pin(int id, int ks, int n, int k);
 int dnn_gemm_bf16_qkv_scatter(const void* A, int lda, const void* W, int ldw, const float* bias, const float* rowstat,

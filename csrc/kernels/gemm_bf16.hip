@@ -8,125 +8,20 @@
 // nanoGPT c_attn / c_proj / c_fc / lm_head (partitions/gpt_model_parts.py:20-21,
 // 32-33,46-49) and the Llama projections.
 //
-// Structure (cdna_hip_programming.md §5, "minimum 2-phase"): 128x128x64 tiles,
-// 4 waves in 2x2, each wave 64x64 = 4x4 mfma_f32_16x16x32_bf16 tiles; operands
-// staged global->LDS with 16-byte global_load_lds into a double buffer whose
-// 128-B rows are XOR-swizzled on the SOURCE address (chunk ^= (row>>1)&7), which
-// makes the ds_read_b128 fragment reads conflict-free (rule 21 / T2).
-// Block ids are remapped so tiles sharing A panels run on one XCD (T1).
-//
-// Decode-sized M (<= 64) goes to the weight-streaming kernels of gemm_skinny.hip.
+// Decode-sized M (<= 64) goes to the weight-streaming kernels of gemm_skinny.hip,
+// row counts between that and a full chip of 256 x 256 tiles (gemm_tile.h) to the
+// smaller tiles of gemm_mid.h.  Operands are staged global->LDS with 16-byte
+// global_load_lds into buffers whose 128-B rows are XOR-swizzled on the SOURCE
+// address (chunk ^= (row>>1)&7), which makes the ds_read_b128 fragment reads
+// conflict-free.  Block ids are remapped so tiles sharing A panels run on one XCD.
 #include <type_traits>
 
 #include "api.h"
 #include "gemm_epilogue.h"
+#include "gemm_mid_api.h"
 #include "gemm_tile.h"
 
 namespace dnn {
-
-// Epilogue on a TRANSPOSED accumulator: the MFMAs are issued as W.A^T, so a
-// lane holds 4 consecutive output columns n..n+3 of one row m (C/D map of the
-// 16x16 MFMA with the operands swapped) and writes them as one 8-B (bf16) or
-// 16-B (fp32) store instead of four scattered 2-B stores.
-template <int ACT, bool OUT_F32>
-__global__ __launch_bounds__(256, 2) void gemm_bf16_tn_kernel(
-    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int ldw, void* __restrict__ Cv,
-    int ldc, const float* __restrict__ bias, const bf16_t* __restrict__ R, int ldr, int M, int N, int K,
-    const float2* __restrict__ rowstat, const float* __restrict__ colsum) {
-  __shared__ __attribute__((aligned(16))) char smem[4 * G_TILE_BYTES];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int ntn = (N + GB_N - 1) / GB_N, ntm = (M + GB_M - 1) / GB_M;
-  int tm, tn;
-  tile_coords(xcd_remap(blockIdx.x, ntm * ntn), ntm, ntn, tm, tn);
-  const int m0 = tm * GB_M, n0 = tn * GB_N;
-  const int wm = wave >> 1, wn = wave & 1;
-
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int nk = K / GB_K;
-  stage_tile(A, lda, m0, M, 0, smem, wave, lane);
-  stage_tile(W, ldw, n0, N, 0, smem + G_TILE_BYTES, wave, lane);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-
-  // two K-tiles per trip: the double-buffer index is a compile-time constant
-  auto ktile = [&](const int t, auto ccst) {
-    constexpr int cur = decltype(ccst)::value;
-    char* a_s = smem + cur * 2 * G_TILE_BYTES;
-    char* b_s = a_s + G_TILE_BYTES;
-    if (t + 1 < nk) {
-      char* na = smem + (cur ^ 1) * 2 * G_TILE_BYTES;
-      stage_tile(A, lda, m0, M, (t + 1) * GB_K, na, wave, lane);
-      stage_tile(W, ldw, n0, N, (t + 1) * GB_K, na + G_TILE_BYTES, wave, lane);
-    }
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int chunk = s * 4 + (lane >> 4);
-      bf16x8 af[4], bfr[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) af[i] = lds_frag(a_s, wm * 64 + i * 16 + (lane & 15), chunk);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bfr[j] = lds_frag(b_s, wn * 64 + j * 16 + (lane & 15), chunk);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[j], af[i], acc[i][j], 0, 0, 0);
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-  };
-  int t = 0;
-  for (; t + 1 < nk; t += 2) {
-    ktile(t, std::integral_constant<int, 0>{});
-    ktile(t + 1, std::integral_constant<int, 1>{});
-  }
-  if (t < nk) ktile(t, std::integral_constant<int, 0>{});
-
-  // Epilogue (transposed accumulators): lane holds row m = .. + (lane&15), cols n..n+3.
-  if (rowstat != nullptr) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        acc[i][j] = epi_norm4(acc[i][j], m0 + wm * 64 + i * 16 + (lane & 15), n0 + wn * 64 + j * 16 + (lane >> 4) * 4,
-                              M, N, rowstat, colsum);
-  }
-  const bool vec = epi_vec_ok(Cv, ldc, bias, R, ldr);
-  const bool pair = vec && epi_pair_ok(Cv, ldc, bias, R, ldr);
-  const f32x2 xc = act_consts<ACT>(bias, N);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + wm * 64 + i * 16 + (lane & 15);
-    if (is_glu(ACT)) {
-#pragma unroll
-      for (int jp = 0; jp < 2; ++jp)
-        epi_glu_pair<ACT, OUT_F32>(acc[i][2 * jp], acc[i][2 * jp + 1], m, (n0 + wn * 64 + jp * 32) / 2, M, N / 2, Cv,
-                               ldc, vec, lane);
-    } else if (!OUT_F32 && pair) {
-#pragma unroll
-      for (int jp = 0; jp < 2; ++jp) {
-        const int nb = n0 + wn * 64 + jp * 32;
-        if (nb + 31 < N)
-          epi_pair_bf16<ACT>(acc[i][2 * jp], acc[i][2 * jp + 1], m, nb, M, reinterpret_cast<bf16_t*>(Cv), ldc, bias,
-                             R, ldr, lane, {}, {}, xc);
-        else
-#pragma unroll
-          for (int j = 2 * jp; j < 2 * jp + 2; ++j)
-            epi_t4<ACT, OUT_F32>(acc[i][j], m, n0 + wn * 64 + j * 16 + (lane >> 4) * 4, M, N, Cv, ldc, bias, R, ldr,
-                                 vec, nullptr, 1.f, nullptr, xc);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        epi_t4<ACT, OUT_F32>(acc[i][j], m, n0 + wn * 64 + j * 16 + (lane >> 4) * 4, M, N, Cv, ldc, bias, R, ldr, vec,
-                             nullptr, 1.f, nullptr, xc);
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------
 // fp8 (OCP e4m3fn) on the same 256^2 4-phase schedule: a K-tile is 128 fp8 =
@@ -525,9 +420,20 @@ __global__ void silu_mul_packed_kernel(const bf16_t* __restrict__ gu, int ld_in,
 // ------------------------------- host API ----------------------------------
 using namespace dnn;
 
-// Large-GEMM tile selection: 0 = auto (256x256 when it still yields >= 256
-// blocks), 128 / 256 force a tile (A/B benchmarking, tests).
+// Large-GEMM tile selection: 0 = auto (gemm_mid.hip mid_plan), 128 / 255 / 256
+// force a tile (A/B benchmarking, tests).
 static int g_gemm_tile = 0;
+// Forced tile of gemm_mid.h's table and K split (tests, A/B); -1: chosen
+static int g_mid_tile = -1, g_mid_splits = 1;
+extern "C" int dnn_gemm_set_mid(int tile, int splits) {
+  if (tile < -1 || tile > 5 || splits < 1 || splits > 16) return -1;
+  g_mid_tile = tile;
+  g_mid_splits = splits;
+  return 0;
+}
+extern "C" int dnn_gemm_is_skinny(int M, int N, int K, int norm, int frag, long long ws_bytes) {
+  return g_gemm_tile == 0 && g_mid_tile < 0 ? mid_skinny(M, N, K, norm != 0, frag != 0, ws_bytes - 4096) : M <= 64;
+}
 
 // Rows up to which every bf16 GEMM streams its weights on the skinny kernels
 // (A/B switch).  At M = 64 a wide-N head with warm weights runs faster on the
@@ -604,41 +510,39 @@ extern "C" int dnn_gemm_set_half_cost(float c) {
 }
 
 template <int ACT, bool F32>
-static void launch_gemm(const void* A, int lda, const void* W, int ldw, void* C, int ldc, const float* bias,
+static int launch_gemm(const void* A, int lda, const void* W, int ldw, void* C, int ldc, const float* bias,
                         const void* R, int ldr, int M, int N, int K, hipStream_t st, const void* Wsh,
                         const float2* rowstat, const float* colsum, void* ws, long long ws_bytes) {
-  // decode-sized: the weight-streaming skinny kernels (gemm_skinny.hip); medium
-  // M (<= 256) too while the 128^2 tiles would not fill 3/4 of the CUs (same
-  // rule as ops/gemm.py skinny_rows)
-  // (a folded-norm GEMM (rowstat) always takes the tile kernels: the skinny
-  // path folds its norm itself, dnn_gemm_skinny_norm)
-  if (rowstat == nullptr &&
-      (M <= g_skinny_max_m || (M <= 256 && ((M + GB_M - 1) / GB_M) * ((N + GB_N - 1) / GB_N) < 192))) {
-    dnn_gemm_skinny(A, lda, nullptr, W, ldw, nullptr, C, ldc, bias, R, ldr, M, N, K, ACT, F32 ? 1 : 0, 0, st, Wsh, ws,
-                    ws_bytes);
-    return;
+  // decode-sized: the weight-streaming kernels (gemm_skinny.hip); a folded-norm
+  // GEMM (rowstat) always takes the tile kernels: the skinny path folds its norm
+  // itself, dnn_gemm_skinny_norm
+  const long long part_bytes = mid_ws(ws, ws_bytes);
+  const bool pinned = g_gemm_tile != 0 || g_mid_tile >= 0;
+  if (rowstat == nullptr && (M <= g_skinny_max_m || (M > 64 && !pinned && mid_skinny(M, N, K, false, Wsh != nullptr, part_bytes)))) {
+    return dnn_gemm_skinny(A, lda, nullptr, W, ldw, nullptr, C, ldc, bias, R, ldr, M, N, K, ACT, F32 ? 1 : 0, 0, st, Wsh,
+                           ws, ws_bytes);
   }
-  // Auto choice by wave quantisation: the 256^2 kernel runs 1 block/CU (256
-  // slots) and is ~1.3x the 128^2 kernel (2 blocks/CU, 512 slots) per slot
-  // when both fill the chip; 1.4 also sends M=32768 N=768 (1.5 waves of 256^2
-  // tiles) to the 256^2 kernel, 6 % faster at K=3072 and equal at K=768
-  // (profiles/archive/r1_gemm_bench_v2_widened_epilogue.jsonl).
+  // Tiles of gemm_mid.h, or 256 x 256 (and its tail split below) by estimated time
   const int tiles256 = ((M + BG_M - 1) / BG_M) * ((N + BG_N - 1) / BG_N);
-  const int tiles128 = ((M + GB_M - 1) / GB_M) * ((N + GB_N - 1) / GB_N);
-  auto fill = [](int tiles, int slots) {
-    const int waves = (tiles + slots - 1) / slots;
-    return (double)tiles / ((double)waves * slots);
-  };
-  const bool big = g_gemm_tile == 256 || g_gemm_tile == 255 ||
-                   (g_gemm_tile == 0 && M >= 256 && N >= 256 && 1.4 * fill(tiles256, 256) > fill(tiles128, 512));
+  MidPlan plan{-1, 1, 0.f};
+  if (lda >= 1 << 23 || ldw >= 1 << 23) {  // the small tiles address a tile's rows with 32 bits
+  } else if (g_mid_tile >= 0) plan = {g_mid_tile, (long long)g_mid_splits * M * N * 4 <= part_bytes ? g_mid_splits : 1, 0.f};
+  else if (g_gemm_tile == 128) plan.tile = 2;
+  else if (g_gemm_tile == 0 && (is_glu(ACT) || has_consts(ACT) || tail_split_cols(M, N) == 0))
+    plan = mid_plan(M, N, K, part_bytes, false);
+  if (plan.tile >= 0) {
+    const MidArgs a{(const bf16_t*)A, (const bf16_t*)W, C, bias, (const bf16_t*)R, rowstat, colsum, (float*)ws, lda, ldw,
+                    ldc, ldr, M, N, K, plan.splits, ACT, F32 ? 1 : 0};
+    return mid_launch(plan.tile, a, nullptr, st);
+  }
   const int tilesH = ((M + BG_M - 1) / BG_M) * ((N + 127) / 128);
   const bool half = g_gemm_tile == 255 ||
-                    (big && g_gemm_tile == 0 && (float)((tilesH + 255) / 256) * g_half_cost < (float)((tiles256 + 255) / 256));
+                    (g_gemm_tile == 0 && (float)((tilesH + 255) / 256) * g_half_cost < (float)((tiles256 + 255) / 256));
   if (half) {
     hipLaunchKernelGGL((gemm_bf16_256_kernel<ACT, F32, false, 1>), dim3(tilesH), dim3(512), 0, st, (const bf16_t*)A,
                        lda, (const bf16_t*)W, ldw, C, ldc, bias, (const bf16_t*)R, ldr, M, N, K, g_res_prefetch,
                        rowstat, colsum);
-    return;
+    return (int)hipGetLastError();
   }
   // Tail split (round 4): when the 256^2 grid is full rounds plus a last
   // column of tiles that fills at most one more round as 256x128 tiles (GPT-2's
@@ -647,7 +551,7 @@ static void launch_gemm(const void* A, int lda, const void* W, int ldw, void* C,
   // in a second launch — 1 + 1/2 rounds instead of 2 full ones, no workspace
   // and no reduction (the two launches write disjoint columns).
   const int ntm256 = (M + BG_M - 1) / BG_M;
-  const int Na = (big && !is_glu(ACT) && !has_consts(ACT)) ? tail_split_cols(M, N) : 0;  // constants lie behind all N
+  const int Na = (!is_glu(ACT) && !has_consts(ACT)) ? tail_split_cols(M, N) : 0;  // constants lie behind all N
   if (Na > 0) {
     const int Nt = N - Na;
     const size_t cb = F32 ? sizeof(float) : sizeof(bf16_t);
@@ -659,16 +563,12 @@ static void launch_gemm(const void* A, int lda, const void* W, int ldw, void* C,
                        (void*)((char*)C + (size_t)Na * cb), ldc, bias != nullptr ? bias + Na : nullptr,
                        R != nullptr ? (const bf16_t*)R + Na : nullptr, ldr, M, Nt, K, g_res_prefetch, rowstat,
                        colsum != nullptr ? colsum + Na : nullptr);
-    return;
+    return (int)hipGetLastError();
   }
-  if (big) {
-    hipLaunchKernelGGL((gemm_bf16_256_kernel<ACT, F32>), dim3(tiles256), dim3(512), 0, st, (const bf16_t*)A, lda,
-                       (const bf16_t*)W, ldw, C, ldc, bias, (const bf16_t*)R, ldr, M, N, K, g_res_prefetch, rowstat,
-                       colsum);
-    return;
-  }
-  hipLaunchKernelGGL((gemm_bf16_tn_kernel<ACT, F32>), dim3(tiles128), dim3(256), 0, st, (const bf16_t*)A, lda,
-                     (const bf16_t*)W, ldw, C, ldc, bias, (const bf16_t*)R, ldr, M, N, K, rowstat, colsum);
+  hipLaunchKernelGGL((gemm_bf16_256_kernel<ACT, F32>), dim3(tiles256), dim3(512), 0, st, (const bf16_t*)A, lda,
+                     (const bf16_t*)W, ldw, C, ldc, bias, (const bf16_t*)R, ldr, M, N, K, g_res_prefetch, rowstat,
+                     colsum);
+  return (int)hipGetLastError();
 }
 
 // rowstat (M float2 {rstd, -mean rstd}) / colsum (N floats, LayerNorm only):
@@ -683,9 +583,8 @@ extern "C" int dnn_gemm_bf16(const void* A, int lda, const void* W, int ldw, voi
   const float2* rs = reinterpret_cast<const float2*>(rowstat);
 #define DISPATCH(a)                                                                                  \
   if (act == a) {                                                                                    \
-    if (out_f32) launch_gemm<a, true>(A, lda, W, ldw, C, ldc, bias, R, ldr, M, N, K, st, Wsh, rs, colsum, ws, ws_bytes); \
-    else launch_gemm<a, false>(A, lda, W, ldw, C, ldc, bias, R, ldr, M, N, K, st, Wsh, rs, colsum, ws, ws_bytes);        \
-    return (int)hipGetLastError();                                                                   \
+    if (out_f32) return launch_gemm<a, true>(A, lda, W, ldw, C, ldc, bias, R, ldr, M, N, K, st, Wsh, rs, colsum, ws, ws_bytes); \
+    return launch_gemm<a, false>(A, lda, W, ldw, C, ldc, bias, R, ldr, M, N, K, st, Wsh, rs, colsum, ws, ws_bytes); \
   }
   DISPATCH(ACT_NONE)
 #ifndef DNN_DECODER_ONLY  // the other families' epilogues: not in the decoder subset (ops/build.py)
@@ -696,8 +595,7 @@ extern "C" int dnn_gemm_bf16(const void* A, int lda, const void* W, int ldw, voi
 #undef DISPATCH
 #define DISPATCH_BF16(a)                                                                                             \
   if (act == a && !out_f32) {                                                                                        \
-    launch_gemm<a, false>(A, lda, W, ldw, C, ldc, bias, R, ldr, M, N, K, st, Wsh, rs, colsum, ws, ws_bytes);         \
-    return (int)hipGetLastError();                                                                                   \
+    return launch_gemm<a, false>(A, lda, W, ldw, C, ldc, bias, R, ldr, M, N, K, st, Wsh, rs, colsum, ws, ws_bytes); \
   }
   DISPATCH_BF16(ACT_GELU_TANH_MUL)
   if (act == ACT_XIELU && bias == nullptr) return -2;
@@ -728,10 +626,20 @@ extern "C" int dnn_gemm_bf16_qkv_scatter(const void* A, int lda, const void* W, 
                                          hipStream_t st) {
   const int M = B * T, N = (H + 2 * Hkv) * hd;
   if (K % 64 != 0 || M <= 0 || hd % 8 != 0 || (colsum != nullptr && rowstat == nullptr)) return -1;
-  if (N % 32 != 0 || M < 256 || ((uintptr_t)bias & 15) != 0) return -3;
+  if (N % 32 != 0 || ((uintptr_t)bias & 15) != 0) return -3;
   const int tiles = ((M + BG_M - 1) / BG_M) * ((N + BG_N - 1) / BG_N);
   if ((hd & (hd - 1)) != 0 || M >= (1 << 24)) return -3;
   QkvScatter sc{(bf16_t*)q, (bf16_t*)kc, (bf16_t*)vc, pos, T, H, Hkv, __builtin_ctz(hd), S, 1.0f / (float)T};
+  if (g_gemm_tile == 0 && tail_split_cols(M, N) == 0 && lda < 1 << 23 && ldw < 1 << 23) {
+    MidPlan plan = mid_plan(M, N, K, 0, true);
+    if (g_mid_tile >= 0) plan.tile = g_mid_tile;
+    if (plan.tile >= 0) {
+      const MidArgs a{(const bf16_t*)A, (const bf16_t*)W, q, bias, nullptr, reinterpret_cast<const float2*>(rowstat),
+                      colsum, nullptr, lda, ldw, hd, 0, M, N, K, 1, ACT_NONE, 0};
+      return mid_launch(plan.tile, a, &sc, st);
+    }
+  }
+  if (M < 256) return -3;
   // tail split as launch_gemm's (GPT-2 c_attn at M = 32768: 1024 + 128 tiles
   // -> 4 rounds of 256^2 + 1 round of 256x128); the bias is indexed by the
   // global column (c_off), the folded norm's colsum by the launch's own

@@ -1,0 +1,334 @@
+// bf16 GEMM for row counts between decode and large prefill (65 to a few thousand
+// rows, where 256 x 256 tiles leave most CUs idle): tiles of 64 to 256 rows with a
+// deep LDS pipeline, and the K range over several workgroups where the tiles alone
+// do not fill the chip (gemm_bf16.hip mid_plan chooses).
+#pragma once
+#include "common.h"
+#include "gemm_epilogue.h"
+#include "gemm_mid_api.h"
+#include "gemm_tile.h"
+
+namespace dnn {
+
+template <int BM_, int BN_, int WM_, int WN_, int S_>
+struct MidTile {
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, S = S_;
+  static constexpr int NW = WM * WN;                           // waves
+  static constexpr int I = BM / WM / 16, J = BN / WN / 16;      // 16 x 16 tiles of a wave
+  static constexpr int PA = BM / 8 / NW, PB = BN / 8 / NW;      // 1-KiB pieces a wave stages of either operand
+  static constexpr int STAGE = (BM + BN) * 128;                 // bytes of one K-tile of both operands
+  static_assert(J % 2 == 0 && PA >= 1 && PB >= 1 && S >= 2, "");
+};
+
+// s_waitcnt operand: at most `vm` vector-memory and `lgkm` LDS operations outstanding
+constexpr int wait_imm(int vm, int lgkm) { return (vm & 15) | (vm >> 4) << 14 | 7 << 4 | lgkm << 8; }
+
+// Columns n .. n + 3 of a vector of N.
+__device__ __forceinline__ f32x4 mid_cols(const float* b, int n, int N) {
+  if (n + 3 < N && (reinterpret_cast<uintptr_t>(b) & 15) == 0) return *reinterpret_cast<const f32x4*>(b + n);
+  f32x4 v;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v[r] = n + r < N ? b[n + r] : 0.f;
+  return v;
+}
+
+template <int ACT>
+__device__ __forceinline__ f32x4 mid_act(f32x4 v, const f32x2& xc) {
+  if constexpr (ACT == ACT_GELU) {
+    const f32x2 g0 = gelu_erf2(f32x2{v[0], v[1]}), g1 = gelu_erf2(f32x2{v[2], v[3]});
+    return f32x4{g0[0], g0[1], g1[0], g1[1]};
+  }
+  act_xielu<ACT>(v, xc);
+  if constexpr (ACT == ACT_RELU) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.f);
+  }
+  return v;
+}
+
+// 4 finished columns of a row: residual and store, bf16 or fp32.
+__device__ __forceinline__ void epi_t4_any(const f32x4& v, int m, int n, int M, int N, const MidArgs& p, const bf16_t* R,
+                                           bool vec) {
+  if (p.f32) epi_t4<ACT_NONE, true>(v, m, n, M, N, p.C, p.ldc, nullptr, R, p.ldr, vec);
+  else epi_t4<ACT_NONE, false>(v, m, n, M, N, p.C, p.ldc, nullptr, R, p.ldr, vec);
+}
+
+// Bias and an elementwise activation on a wave's accumulators.
+template <int I, int J>
+__device__ __forceinline__ void mid_bias_act(f32x4 (&acc)[I][J], const float* bias, int act, int n0, int N) {
+  if (bias != nullptr) {
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const f32x4 b4 = mid_cols(bias, n0 + j * 16, N);
+#pragma unroll
+      for (int i = 0; i < I; ++i) acc[i][j] += b4;
+    }
+  }
+  if (act == ACT_GELU) {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int j = 0; j < J; ++j) acc[i][j] = mid_act<ACT_GELU>(acc[i][j], f32x2{});
+  } else if (act == ACT_RELU) {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int j = 0; j < J; ++j) acc[i][j] = mid_act<ACT_RELU>(acc[i][j], f32x2{});
+  } else if (act == ACT_XIELU) {
+    const f32x2 xc = act_consts<ACT_XIELU>(bias, N);
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int j = 0; j < J; ++j) acc[i][j] = mid_act<ACT_XIELU>(acc[i][j], xc);
+  }
+}
+
+enum MidOut { MID_ROWS = 0, MID_SCATTER = 1, MID_PART = 2 };
+
+// Loop: a K-tile of 64 is multiplied in two halves of 32; the second half's
+// fragments are read behind the first row of products of the first, the next
+// tile's first half behind the first row of the second, one barrier a tile.  The
+// requests for tile t + S - 1 go out between the rows of products.
+//
+// What bounds it: the operands' way from L2 to LDS.  With 128 x 128 tiles on 192
+// CUs a K-tile takes 0.47 us (32 KB a CU: 13 TB/s over the chip) where its products
+// take 0.22 and its LDS traffic 0.33; larger tiles need fewer bytes per product but
+// more splits.  Touching later lines from a wave of its own, waves of 64 x 32 in
+// place of 64 x 64, or padded rows did not change that.
+template <class T, MidOut OUT>
+__global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvScatter scat) {
+  constexpr bool PART = OUT == MID_PART;
+  constexpr int I = T::I, J = T::J, S = T::S, L = T::PA + T::PB;
+  // S * STAGE bytes, given at launch: with the size in the kernel the compiler sees one
+  // wave per SIMD and moves accumulators of the four-wave tiles to AGPRs and back in
+  // the loop (192 x 128 at 700 x 6144 x 4096: 47 -> 78 us)
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int M = p.M, N = p.N;
+  const int ntn = (N + T::BN - 1) / T::BN, ntm = (M + T::BM - 1) / T::BM, tiles = ntm * ntn;
+  int id = xcd_remap(blockIdx.x, tiles * p.splits), sp = 0;
+  if constexpr (PART) {
+    sp = id / tiles;
+    id -= sp * tiles;
+  }
+  int tm, tn;
+  tile_coords(id, ntm, ntn, tm, tn);
+  const int m0 = tm * T::BM, n0 = tn * T::BN;
+  const int wm = wave / T::WN, wn = wave % T::WN;
+  int nk = p.K >> 6, k0 = 0;
+  if constexpr (PART) {
+    k0 = (int)((long long)nk * sp / p.splits);
+    nk = (int)((long long)nk * (sp + 1) / p.splits) - k0;
+  }
+  // staging: uniform tile bases, per-lane offsets of the wave's pieces
+  const char* a0 = reinterpret_cast<const char*>(p.A + (size_t)m0 * p.lda) + (size_t)k0 * 128;
+  const char* b0 = reinterpret_cast<const char*>(p.W + (size_t)n0 * p.ldw) + (size_t)k0 * 128;
+  uint32_t oa[T::PA], ob[T::PB];
+#pragma unroll
+  for (int q = 0; q < T::PA; ++q) {
+    const int rl = (q * T::NW + wave) * 8 + (lane >> 3);
+    oa[q] = (uint32_t)min(rl, M - 1 - m0) * (uint32_t)p.lda * 2u + (uint32_t)((lane & 7) ^ swz_chunk(rl)) * 16u;
+  }
+#pragma unroll
+  for (int q = 0; q < T::PB; ++q) {
+    const int rl = (q * T::NW + wave) * 8 + (lane >> 3);
+    ob[q] = (uint32_t)min(rl, N - 1 - n0) * (uint32_t)p.ldw * 2u + (uint32_t)((lane & 7) ^ swz_chunk(rl)) * 16u;
+  }
+  // pieces [q0, q1) of K-tile t; past the end: a harmless refill, so that the waits count alike
+  auto stage_a = [&](int t, int buf, int q0, int q1) {
+    const char* as = a0 + (size_t)min(t, nk - 1) * 128;
+#pragma unroll
+    for (int q = q0; q < q1; ++q) glds16(as + oa[q], smem + buf * T::STAGE + (q * T::NW + wave) * 1024);
+  };
+  auto stage_b = [&](int t, int buf, int q0, int q1) {
+    const char* bs = b0 + (size_t)min(t, nk - 1) * 128;
+#pragma unroll
+    for (int q = q0; q < q1; ++q) glds16(bs + ob[q], smem + buf * T::STAGE + T::BM * 128 + (q * T::NW + wave) * 1024);
+  };
+  // fragment reads: lane (r, g) reads 16 B of row r at chunks g and 4 + g
+  const int fr = lane & 15, fg = lane >> 4;
+  const int arow = wm * (I * 16) + fr, brow = wn * (J * 16) + fr;
+  const int ao[2] = {arow * 128 + ((fg ^ swz_chunk(arow)) << 4), arow * 128 + (((4 + fg) ^ swz_chunk(arow)) << 4)};
+  const int bo[2] = {T::BM * 128 + brow * 128 + ((fg ^ swz_chunk(brow)) << 4),
+                     T::BM * 128 + brow * 128 + (((4 + fg) ^ swz_chunk(brow)) << 4)};
+  // The operands of a K-tile in two halves of 32: F[x] = 16 x 32 fragments of A, then of B.
+  bf16x8 f[2][I + J];
+  auto read = [&](auto hc, int buf) {
+    constexpr int h = decltype(hc)::value;
+    const char* d = smem + buf * T::STAGE;
+#pragma unroll
+    for (int j = 0; j < J; ++j) f[h][I + j] = *reinterpret_cast<const bf16x8*>(d + bo[h] + j * 2048);
+#pragma unroll
+    for (int i = 0; i < I; ++i) f[h][i] = *reinterpret_cast<const bf16x8*>(d + ao[h] + i * 2048);
+  };
+  f32x4 acc[I][J];
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int j = 0; j < J; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto mma = [&](auto hc, int i) {
+    constexpr int h = decltype(hc)::value;
+#pragma unroll
+    for (int j = 0; j < J; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[h][I + j], f[h][i], acc[i][j], 0, 0, 0);
+  };
+  constexpr auto h0 = std::integral_constant<int, 0>{};
+  constexpr auto h1 = std::integral_constant<int, 1>{};
+#pragma unroll
+  for (int q = 0; q < S - 1; ++q) {
+    stage_a(q, q, 0, T::PA);
+    stage_b(q, q, 0, T::PB);
+  }
+  __builtin_amdgcn_s_waitcnt(wait_imm((S - 2) * L, 0));
+  bg_barrier();
+  read(h0, 0);
+  int cur = 0;
+  for (int t = 0; t < nk; ++t) {
+    const int prev = cur == 0 ? S - 1 : cur - 1, next = cur == S - 1 ? 0 : cur + 1;
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      mma(h0, i);
+      __builtin_amdgcn_sched_barrier(0);
+      if (i == 0) read(h1, cur);
+      stage_a(t + S - 1, prev, T::PA * i / I, T::PA * (i + 1) / I);
+      stage_b(t + S - 1, prev, T::PB * i / I, T::PB * (i + 1) / I);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_waitcnt(wait_imm((S - 2) * L, 0));  // tile t + 1 landed, tile t read
+    bg_barrier();
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      mma(h1, i);
+      __builtin_amdgcn_sched_barrier(0);
+      if (i == 0) read(h0, next);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    cur = next;
+  }
+  __builtin_amdgcn_s_waitcnt(wait_imm(0, 0));
+
+  if constexpr (PART) {
+    float* d = p.part + (size_t)sp * M * N;
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      const int m = m0 + wm * (I * 16) + i * 16 + fr;
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        const int n = n0 + wn * (J * 16) + j * 16 + fg * 4;  // host: N % 4 == 0
+        if (m < M && n < N) *reinterpret_cast<f32x4*>(d + (size_t)m * N + n) = acc[i][j];
+      }
+    }
+    return;
+  }
+  const int mw = m0 + wm * (I * 16) + fr, nw = n0 + wn * (J * 16);  // the lane's first row, the wave's first column
+  if (p.rowstat != nullptr) {  // the folded norm, in the 256 x 256 kernel's order of operations
+    float2 rs[I];
+    f32x4 cs[J];
+#pragma unroll
+    for (int i = 0; i < I; ++i) rs[i] = p.rowstat[min(mw + i * 16, M - 1)];
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+      cs[j] = p.colsum != nullptr ? mid_cols(p.colsum, nw + j * 16 + fg * 4, N) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int j = 0; j < J; ++j) acc[i][j] = acc[i][j] * rs[i].x + rs[i].y * cs[j];
+  }
+  if constexpr (OUT == MID_SCATTER) {
+    int spos[I];
+#pragma unroll
+    for (int i = 0; i < I; ++i) spos[i] = qkv_row_pos(scat, min(mw + i * 16, M - 1));
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int jp = 0; jp < J / 2; ++jp)
+        if (nw + jp * 32 < N)  // host: N % 32 == 0
+          epi_pair_scatter(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, nw + jp * 32, M, p.bias, lane, scat, spos[i]);
+    return;
+  }
+  const bool vec = epi_vec_ok(p.C, p.ldc, p.bias, p.R, p.ldr);
+  if (is_glu(p.act)) {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int jp = 0; jp < J / 2; ++jp) {
+        const f32x4 &x0 = acc[i][2 * jp], &x1 = acc[i][2 * jp + 1];
+        const int m = mw + i * 16, c = (nw + jp * 32) / 2;
+        if (p.act == ACT_GELU_TANH_MUL) epi_glu_pair<ACT_GELU_TANH_MUL, false>(x0, x1, m, c, M, N / 2, p.C, p.ldc, vec, lane);
+        else if (p.f32) epi_glu_pair<ACT_SILU_MUL, true>(x0, x1, m, c, M, N / 2, p.C, p.ldc, vec, lane);
+        else epi_glu_pair<ACT_SILU_MUL, false>(x0, x1, m, c, M, N / 2, p.C, p.ldc, vec, lane);
+      }
+    return;
+  }
+  mid_bias_act<I, J>(acc, p.bias, p.act, nw + fg * 4, N);
+  bf16_t* C = reinterpret_cast<bf16_t*>(p.C);
+  const bool pair = vec && !p.f32 && epi_pair_ok(p.C, p.ldc, p.bias, p.R, p.ldr) && nw + J * 16 <= N;
+  if (pair && p.R != nullptr) {  // every residual load before the first output
+    bf16x4 rr[I][J / 2][2];
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int jp = 0; jp < J / 2; ++jp)
+        epi_pair_res_load(mw + i * 16, nw + jp * 32, M, p.R, p.ldr, lane, rr[i][jp][0], rr[i][jp][1]);
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int jp = 0; jp < J / 2; ++jp)
+        epi_pair_bf16<ACT_NONE, true>(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, nw + jp * 32, M, C, p.ldc, nullptr,
+                                      p.R, p.ldr, lane, rr[i][jp][0], rr[i][jp][1]);
+  } else if (pair) {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int jp = 0; jp < J / 2; ++jp)
+        epi_pair_bf16<ACT_NONE>(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, nw + jp * 32, M, C, p.ldc, nullptr, nullptr,
+                                0, lane);
+  } else if (p.f32) {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        epi_t4<ACT_NONE, true>(acc[i][j], mw + i * 16, nw + j * 16 + fg * 4, M, N, p.C, p.ldc, nullptr, p.R, p.ldr, vec);
+  } else {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        epi_t4<ACT_NONE, false>(acc[i][j], mw + i * 16, nw + j * 16 + fg * 4, M, N, p.C, p.ldc, nullptr, p.R, p.ldr, vec);
+  }
+}
+
+// Sum of the parts and the epilogue.  A thread: 4 columns of one row (gated: 4
+// gate columns and the 4 up columns that belong to them).  Bound by reading the
+// parts (they were just written: mostly from the last-level cache).
+template <int GLU>
+__global__ __launch_bounds__(256) void gemm_mid_reduce(MidArgs p) {
+  const int m = blockIdx.y, M = p.M, N = p.N;
+  const int q = blockIdx.x * 256 + threadIdx.x;  // group of 4 output columns
+  const int n = GLU ? (q >> 1) * 16 + (q & 1) * 4 : q * 4;
+  if (n >= N) return;
+  const size_t slab = (size_t)M * N;
+  const float* d = p.part + (size_t)m * N + n;
+  f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f}, u = v;
+  for (int s = 0; s < p.splits; ++s) {
+    v += *reinterpret_cast<const f32x4*>(d + s * slab);
+    if (GLU) u += *reinterpret_cast<const f32x4*>(d + s * slab + 8);
+  }
+  if (p.rowstat != nullptr) {
+    v = epi_norm4(v, m, n, M, N, p.rowstat, p.colsum);
+    if (GLU) u = epi_norm4(u, m, n + 8, M, N, p.rowstat, p.colsum);
+  }
+  const bool vec = epi_vec_ok(p.C, p.ldc, p.bias, p.R, p.ldr);
+  if (GLU) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = (p.act == ACT_GELU_TANH_MUL ? gelu_tanh(v[r]) : silu(v[r])) * u[r];
+    epi_t4_any(v, m, q * 4, M, N / 2, p, nullptr, vec);
+    return;
+  }
+  f32x4 a[1][1] = {{v}};
+  mid_bias_act<1, 1>(a, p.bias, p.act, n, N);
+  epi_t4_any(a[0][0], m, n, M, N, p, p.R, vec);
+}
+
+}  // namespace dnn

@@ -1,0 +1,120 @@
+// bf16 GEMM for 65 to a few thousand rows: the choice of tile and K split, and
+// the launches (kernels: gemm_mid.h).
+#include "gemm_mid.h"
+
+namespace dnn {
+
+// Tile table: rows, columns, whether two workgroups share a CU, and the two
+// constants of a tile's time in us: a (launch, first loads, epilogue) and s (a
+// K-tile of 64).  Fitted to 310 shapes (65 to 32768 rows, 768 to 28672 columns, K of
+// 768 to 18432, weights cold) that every tile ran, with 1 to 8 splits: the estimate
+// is off by 9 % (rms), and what it picks is within 1 % of the best measured on
+// average, 20 % at worst.  The last entry is the 256 x 256 kernel (gemm_tile.h).
+struct MidCost {
+  int bm, bn, pairs;
+  float a, s;
+};
+static constexpr MidCost MID[] = {{64, 64, 1, 1.89f, 0.252f},   {128, 64, 0, 2.78f, 0.332f},
+                                  {128, 128, 0, 2.99f, 0.472f}, {192, 128, 0, 3.71f, 0.637f},
+                                  {256, 128, 0, 4.14f, 0.707f}, {128, 256, 0, 4.07f, 0.754f},
+                                  {256, 256, 0, 4.93f, 1.198f}};
+static constexpr int MID_TILES = 6, CUS = 256;
+typedef MidTile<64, 64, 2, 2, 4> Mid0;
+typedef MidTile<128, 64, 2, 2, 6> Mid1;
+typedef MidTile<128, 128, 2, 4, 4> Mid2;
+typedef MidTile<192, 128, 2, 2, 3> Mid3;
+typedef MidTile<256, 128, 4, 2, 3> Mid4;
+typedef MidTile<128, 256, 2, 4, 3> Mid5;
+
+// Time of one tile size and split: K-tiles of the fullest CU, beside the time that
+// reading the weights (4.3 TB/s) and moving the activations (2 TB/s) takes; a split
+// adds its sum (5 us and 3 us for one more launch from the host, which bounds the
+// smallest steps, and the parts written and read at 3.2 TB/s).
+static float mid_time(const MidCost& c, int M, int N, int K, int splits) {
+  const long long wgs = (long long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * splits;
+  const int kt = (K / 64 + splits - 1) / splits, n = (int)((wgs + CUS - 1) / CUS);
+  const float rounds = c.pairs ? (n / 2) * 1.73f + (n & 1) : (float)n;
+  const float a = c.pairs ? c.a : c.a * (1.f + 0.5f * (n - 1));
+  const float t = rounds * kt * c.s, w = (float)N * K * 2.f / 4.27e6f + (float)M * (K + N) * 2.f / 2.0e6f;
+  const float us = a + cbrtf(t * t * t + w * w * w);
+  return splits == 1 ? us : us + 8.f + (splits + 0.5f) * M * N * 4.f / 3.16e6f;
+}
+
+static MidPlan best_plan(int M, int N, int K, long long ws_bytes, bool scatter) {
+  // the 256 x 256 kernel needs to be 5 % slower to lose: the estimate's error at
+  // its sizes (12352 columns of 3000 rows: 257 us, 267 as 256 x 128)
+  MidPlan best{-1, 1, M < 256 || N < 256 ? 1e30f : 0.95f * mid_time(MID[MID_TILES], M, N, K, 1)};
+  for (int i = 0; i < MID_TILES; ++i)
+    for (int s = 1; s <= 8; ++s) {
+      if (s > 1 && (scatter || N % 4 != 0 || M > 65535 || K / 64 / s < 3 || (long long)s * M * N * 4 > ws_bytes)) break;
+      const float t = mid_time(MID[i], M, N, K, s);
+      if (t < best.us) best = {i, s, t};
+    }
+  return best;
+}
+
+// The same by sizes: 48 estimates take 3 us of host time, a table entry (per thread)
+// nothing beside a launch.
+MidPlan mid_plan(int M, int N, int K, long long ws_bytes, bool scatter) {
+  struct Entry {
+    int M = 0, N = 0, K = 0, scatter = 0;
+    long long ws = 0;
+    MidPlan plan{};
+  };
+  static thread_local Entry table[256];
+  Entry& e = table[((unsigned)M * 2654435761u ^ (unsigned)N * 40503u ^ (unsigned)K * 97u ^ (scatter ? 77u : 0u)) >> 7 & 255];
+  if (e.M != M || e.N != N || e.K != K || e.scatter != (int)scatter || e.ws != ws_bytes)
+    e = {M, N, K, scatter ? 1 : 0, ws_bytes, best_plan(M, N, K, ws_bytes, scatter)};
+  return e.plan;
+}
+
+// Decode kernels (gemm_skinny.hip) on more than 64 rows: every 16 rows read the
+// weights once more (from the cache): 4 times the time of the tiles at 256 x 4096 x
+// 18432 (236 us : 53), little more at the smallest (96 x 768 x 768: 5.4 : 5.0), where
+// a folded norm that rides in them saves a launch (3.5 us on the device, 8 where
+// the host bounds such steps).  `frag`: the weight has its fragment-order copy.
+bool mid_skinny(int M, int N, int K, bool norm, bool frag, long long ws_bytes) {
+  if (M <= 64) return true;
+  if (M > 256) return false;
+  return 4.2f + (frag ? 2.0e-7f : 3.2e-7f) * N * K * ((M + 15) / 16) < mid_plan(M, N, K, ws_bytes, false).us + (norm ? 8.f : 0.f);
+}
+
+template <class T, MidOut OUT>
+static int start(const MidArgs& a, const QkvScatter& scat, hipStream_t st) {
+  constexpr int LDS = T::S * T::STAGE;
+  static const hipError_t room =
+      hipFuncSetAttribute((const void*)gemm_mid_kernel<T, OUT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  if (room != hipSuccess) return (int)room;
+  const int tiles = ((a.M + T::BM - 1) / T::BM) * ((a.N + T::BN - 1) / T::BN);
+  hipLaunchKernelGGL((gemm_mid_kernel<T, OUT>), dim3(tiles * a.splits), dim3(T::NW * 64), LDS, st, a, scat);
+  return (int)hipGetLastError();
+}
+
+template <class T>
+static int launch(const MidArgs& a, const QkvScatter* scat, hipStream_t st) {
+  if (scat != nullptr) return start<T, MID_SCATTER>(a, *scat, st);
+  if (a.splits == 1) return start<T, MID_ROWS>(a, QkvScatter{}, st);
+  if (const int rc = start<T, MID_PART>(a, QkvScatter{}, st)) return rc;
+  const bool glu = is_glu(a.act);
+  const dim3 grid(((glu ? a.N / 2 : a.N) / 4 + 255) / 256, a.M);
+  if (glu) hipLaunchKernelGGL((gemm_mid_reduce<1>), grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((gemm_mid_reduce<0>), grid, dim3(256), 0, st, a);
+  return (int)hipGetLastError();
+}
+
+int mid_launch(int tile, const MidArgs& a, const QkvScatter* scat, hipStream_t st) {
+  if (a.splits < 1 || (a.splits > 1 && (scat != nullptr || a.part == nullptr || a.N % 4 != 0 || a.K / 64 < a.splits ||
+                                        a.M > 65535)))
+    return -1;
+  switch (tile) {
+    case 0: return launch<Mid0>(a, scat, st);
+    case 1: return launch<Mid1>(a, scat, st);
+    case 2: return launch<Mid2>(a, scat, st);
+    case 3: return launch<Mid3>(a, scat, st);
+    case 4: return launch<Mid4>(a, scat, st);
+    case 5: return launch<Mid5>(a, scat, st);
+  }
+  return -1;
+}
+
+}  // namespace dnn

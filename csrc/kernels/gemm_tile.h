@@ -9,26 +9,7 @@
 
 namespace dnn {
 
-constexpr int GB_M = 128, GB_N = 128, GB_K = 64;
-constexpr int G_TILE_BYTES = GB_M * GB_K * 2;  // 16 KiB per operand tile
-
 __device__ __forceinline__ int swz_chunk(int row) { return (row >> 1) & 7; }
-
-// Stage one 128x64 bf16 tile (rows r0.., clamped to nrows-1) into LDS `dst`.
-__device__ __forceinline__ void stage_tile(const bf16_t* __restrict__ src, int ld, int r0, int nrows,
-                                           int k0, char* dst, int wave, int lane) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int piece = wave * 4 + i;            // 1 KiB = 8 rows per wave-instruction
-    const int rl = piece * 8 + (lane >> 3);    // row within the tile
-    const int cp = lane & 7;                   // destination 16B chunk (linear)
-    const int cs = cp ^ swz_chunk(rl);         // source chunk (inverse swizzle)
-    int r = r0 + rl;
-    r = r < nrows ? r : nrows - 1;
-    const bf16_t* g = src + (size_t)r * ld + k0 + cs * 8;
-    glds16(g, dst + piece * 1024);
-  }
-}
 
 __device__ __forceinline__ bf16x8 lds_frag(const char* tile, int row, int chunk) {
   return *reinterpret_cast<const bf16x8*>(tile + row * 128 + ((chunk ^ swz_chunk(row)) << 4));

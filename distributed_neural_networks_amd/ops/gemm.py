@@ -6,6 +6,7 @@ the last dim must be contiguous and K a multiple of 64.
 """
 from __future__ import annotations
 
+import functools
 from typing import Optional
 
 import torch
@@ -20,14 +21,24 @@ SKINNY_MAX_M = 256
 SKINNY_ALWAYS_M = 64  # bf16: rows up to which the skinny kernels always run (gemm_bf16.hip g_skinny_max_m)
 
 
-def skinny_rows(M: int, N: int, w8: bool = False) -> bool:
+def skinny_rows(M: int, N: int, w8: bool = False, K: int = 0, norm: bool = False, frag: bool = True,
+                ws: Optional[torch.Tensor] = None) -> bool:
     """Decode-sized GEMM -> the weight-streaming skinny kernels: M <= 64 (always
     for fp8 weights: W8A16 keeps bf16 activations in decode; bf16 per
-    ``set_skinny_max_m``), or medium M (<= 256, M split into 16-row tiles) while
-    128^2 tiles would not fill 3/4 of the CUs (same rule as gemm_bf16.hip
-    launch_gemm)."""
-    always = 64 if w8 else SKINNY_ALWAYS_M
-    return M <= always or (M <= SKINNY_MAX_M and -(-M // 128) * -(-N // 128) < 192)
+    ``set_skinny_max_m``); up to 256 rows bf16 by estimated time beside the tiles of
+    gemm_mid.h (the rule gemm_bf16.hip uses too; ``norm``: a norm that rides
+    along, ``frag``: the weight has its fragment-order copy), fp8 while 128^2 tiles
+    would not fill 3/4 of the CUs."""
+    if w8:
+        return M <= 64 or (M <= SKINNY_MAX_M and -(-M // 128) * -(-N // 128) < 192)
+    if M <= SKINNY_ALWAYS_M or M > SKINNY_MAX_M:
+        return M <= SKINNY_ALWAYS_M
+    return _is_skinny(M, N, K, norm, frag, 0 if ws is None else ws.nbytes)
+
+
+@functools.lru_cache(maxsize=4096)
+def _is_skinny(M: int, N: int, K: int, norm: bool, frag: bool, ws_bytes: int) -> bool:
+    return bool(lib().gemm_is_skinny(M, N, K, int(norm), int(frag), ws_bytes))
 
 
 def set_skinny_max_m(m: int = 64) -> None:
@@ -41,6 +52,17 @@ _ACTS = {None: ACT_NONE, "none": ACT_NONE, "relu": ACT_RELU, "gelu": ACT_GELU, "
 
 DECODE_WS_BYTES = 16 << 20
 _decode_ws = {}
+PREFILL_WS_BYTES = 64 << 20
+
+
+def prefill_workspace(rows: int, cols: int, device) -> Optional[torch.Tensor]:
+    """Workspace of the GEMMs of up to ``rows`` rows (more than decode brings) and
+    ``cols`` columns that split K over workgroups (gemm_mid.h): fp32 parts of one
+    projection at a time, at most 8.  One per stage, used in stream order like
+    its scratch rows; zeroed, its last 4 KiB are tickets (``decode_workspace``)."""
+    if rows <= SKINNY_ALWAYS_M:
+        return None
+    return torch.zeros(min(PREFILL_WS_BYTES, 8 * 4 * rows * cols) + 4096, dtype=torch.uint8, device=device)
 
 
 def decode_workspace(device, slot: int = 0) -> torch.Tensor:
@@ -120,7 +142,7 @@ def rowstats_written() -> bool:
 
 
 def _ws_args(ws: Optional[torch.Tensor]):
-    return (0, 0) if ws is None else (ws.data_ptr(), ws.numel() * ws.element_size())
+    return (0, 0) if ws is None else (ws.data_ptr(), ws.nbytes)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, act=None,
@@ -131,7 +153,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     """``w_shuf``: ``shuffle_weight(w)``, streamed instead of ``w`` on the skinny path (``skinny_rows``).
     ``rs_out`` (decode): row-statistics partials of the output (``rowstats_buffer``);
     ``rowstats_written()`` tells whether the kernel that ran wrote them.
-    ``ws``: ``decode_workspace`` for the decode stream GEMM's split-K partials.
+    ``ws``: ``decode_workspace`` (``prefill_workspace``) for the partials of a K split.
     ``rowstat`` ((M, 2) fp32 from ``transformer_ops.row_stats``) / ``colsum``: a
     folded pre-norm applied in the epilogue, ``rstd (x W^T) - mean rstd colsum``
     (MFMA tile kernels only).  ``ACT_XIELU``: c0 z^2 + z / 2 above zero, c1 (exp(z) - 1 - z) + z / 2
@@ -181,8 +203,16 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
 
 
 def set_gemm_tile(tile: int = 0) -> None:
-    """Force the large-GEMM tile (128, 256, or 255 = 256x128) or restore the auto choice (0)."""
+    """Force the large-GEMM tile (128, 256, or 255 = 256x128) or restore the choice by estimated time (0)."""
     check(lib().gemm_set_tile(int(tile)), "gemm_set_tile")
+    _is_skinny.cache_clear()
+
+
+def set_gemm_mid(tile: int = -1, splits: int = 1) -> None:
+    """Force a tile of gemm_mid.h's table (0..5) and a K split for GEMMs above the
+    decode sizes (tests, A/B probes); -1 restores the choice by estimated time."""
+    check(lib().gemm_set_mid(int(tile), int(splits)), "gemm_set_mid")
+    _is_skinny.cache_clear()
 
 
 def set_gemm_split_tail(on=True) -> None:
@@ -282,7 +312,7 @@ def linear_norm(x: torch.Tensor, f: FoldedLinear, act=None, residual: Optional[t
     N = f.w.shape[0]
     if (not w8 and f.w.shape[1] != K) or x.dtype != torch.bfloat16 or x.stride(1) != 1:
         raise ValueError(f"linear_norm: x {tuple(x.shape)} {x.dtype} vs w {tuple(f.w.shape)}")
-    if not skinny_rows(M, N, w8):
+    if not skinny_rows(M, N, w8, K, True, f.ws is not None, ws):
         from .transformer_ops import layernorm, layernorm_q8
         if std_buf is None or ones is None:
             raise ValueError("linear_norm: large M needs std_buf and ones")
@@ -311,9 +341,9 @@ def linear_norm(x: torch.Tensor, f: FoldedLinear, act=None, residual: Optional[t
             from .transformer_ops import row_stats
             st = std_buf.reshape(-1)[:4 * M].view(torch.float32).view(M, 2)
             row_stats(x, st, f.eps, f.norm == NORM_RMS, rows=M, ldx=x.stride(0))
-            return linear(x, f.w, f.bias, a, residual, out, rowstat=st, colsum=f.colsum)
+            return linear(x, f.w, f.bias, a, residual, out, rowstat=st, colsum=f.colsum, ws=ws)
         xs = layernorm(x, ones, None, std_buf[:M], f.eps, f.norm == NORM_RMS, rows=M, ldx=x.stride(0))
-        return linear(xs[:M], f.w, f.bias, a, residual, out)
+        return linear(xs[:M], f.w, f.bias, a, residual, out, ws=ws)
     if w8:
         return linear_w8(x, f.w, f.bias, a, residual, out, f.norm, f.colsum, f.eps, ws=ws, rs_in=rs_in)
     if K % 32:
@@ -359,7 +389,7 @@ def qkv_scatter_norm(x: torch.Tensor, f: FoldedLinear, std_buf: torch.Tensor, q:
         return False
     M, K = x.shape
     N = f.w.shape[0]
-    if M != B * T or N != (H + 2 * Hkv) * hd or skinny_rows(M, N, w8) or x.stride(1) != 1:
+    if M != B * T or N != (H + 2 * Hkv) * hd or skinny_rows(M, N, w8, K, True, w8 or f.ws is not None) or x.stride(1) != 1:
         return False
     if not (kc.is_contiguous() and vc.is_contiguous()) or q.numel() < M * H * hd or pos.dtype != torch.int32:
         return False

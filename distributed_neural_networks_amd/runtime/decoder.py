@@ -33,7 +33,7 @@ from ..models import DECODERS, model_info
 from ..ops import decoder_ops as D_
 from ..ops import mixer_ops as M_
 from ..ops import transformer_ops as T_
-from ..ops.gemm import decode_workspace
+from ..ops.gemm import decode_workspace, prefill_workspace
 from .decoder_layers import LAYERS, DynamicTanh, ScalarNorm, Weights, pad
 from .paging import LatentHeads, StepBatch, pages_for, tile_lists
 from .stages import StageCompute, StageOutput
@@ -160,6 +160,8 @@ class DecoderStage(StageCompute):
             self.amx_part = torch.empty((max(self.max_batch, 1) * 2 * T_.ARGMAX_PART_PER_ROW,), dtype=torch.int32,
                                         device=dev)
         self.ws: Optional[torch.Tensor] = None        # decode-attention partials (engine steps)
+        widest = max(w.shape[1] for w in (self.h, *self.buf.values()))
+        self.pws = None if self.f32 else prefill_workspace(n, widest, dev)  # K splits of steps of more than 64 rows
 
     def flat(self, name: str, s: slice, cols: int) -> torch.Tensor:
         """Rows ``s`` of a scratch buffer as dense rows of ``cols`` (buffers of
@@ -293,7 +295,7 @@ class DecoderStage(StageCompute):
                 self.ws = torch.empty((need,), dtype=torch.float32, device=self.device)
         ids = self._enter(x, b.ids, 0, b.M)
         gws = decode_workspace(self.device) if not self.f32 and b.M <= 64 else None
-        self._layers(b, ids, 0, gws, self.ws)
+        self._layers(b, ids, 0, self.pws if gws is None else gws, self.ws)
         if not self.last:
             return self._leave(ids, 0, b.M, None)
         if not b.n_want:
@@ -393,7 +395,7 @@ class DecoderStage(StageCompute):
                 ws = self._ring_ws[per * b0:]
         ids = self._enter(x, x.view(-1) if self.first else None, r0, M)
         gws = decode_workspace(self.device, b0 // B) if T == 1 and not self.f32 else None
-        self._layers(b, ids, r0, gws, ws)
+        self._layers(b, ids, r0, self.pws if gws is None else gws, ws)
         if not self.last:
             return self._leave(ids, r0, M, out)
         c = self._ring[(B, T, b0)]

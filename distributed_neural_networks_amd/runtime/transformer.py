@@ -348,6 +348,7 @@ class TransformerStage(StageCompute):
         self.head_part = (torch.empty((self.max_batch * 2 * HEAD_PART_PER_ROW,), dtype=torch.int32, device=dev)
                           if self.last else None)
         self.rowstat = G_.rowstats_buffer(self.max_batch, d, dev)  # decode rows only
+        self.pws = None if self.fp8 else G_.prefill_workspace(ntok, max((H + 2 * Hkv) * hd, d, ffn), dev)
         self.q8 = self.s8 = None
         self.sx8 = self.q8b = self.sx8b = None
         if self.fp8:
@@ -443,7 +444,7 @@ class TransformerStage(StageCompute):
             s8 = self.s8[r0:]
         ws = self.ws[r0 * self.ws_per_seq:] if T == 1 else self.ws
         # decode stream-GEMM split-K workspace: one per concurrent microbatch slot
-        gws = decode_workspace(self.device, b0 // B) if T == 1 else None
+        gws = decode_workspace(self.device, b0 // B) if T == 1 else self.pws
         # decode row statistics produced by the residual-writing projections
         # (O, c_proj: per-16-column {mean, M2} partials of h) and merged by the
         # next folded pre-norm projection (c_fc, the next layer's QKV) instead

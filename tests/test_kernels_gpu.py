@@ -493,3 +493,101 @@ def test_fp8_gemm_tail_split_matches_single_grid(N, K, split, act, res):
         ref = ref + r.float()
     err = ((outs[0].float() - ref).norm() / ref.norm()).item()
     assert err < (3e-2 if split else 8e-2), err
+
+
+MID_TILES = ((64, 64), (128, 64), (128, 128), (192, 128), (256, 128), (128, 256))  # csrc/kernels/gemm_mid.hip MID
+
+
+def _mid_reference(x, w, b, r, act, norm, consts):
+    y = x.float() @ w.float().t()
+    if norm is not None:
+        st, cs = norm
+        y = y * st[:, :1] + st[:, 1:] * cs
+    if act in (3, 4):  # packed gate | up
+        g = y.view(y.shape[0], -1, 2, 8)
+        f = torch.nn.functional.silu if act == 3 else lambda z: torch.nn.functional.gelu(z, approximate="tanh")
+        return (f(g[:, :, 0]) * g[:, :, 1]).reshape(y.shape[0], -1)
+    if b is not None:
+        y = y + b
+    if act == 1:
+        y = torch.relu(y)
+    elif act == 2:
+        y = torch.nn.functional.gelu(y)
+    elif act == 6:
+        y = torch.where(y > 0, consts[0] * y * y, consts[1] * (torch.expm1(y.clamp(max=0)) - y)) + y / 2
+    return y if r is None else y + r.float()
+
+
+@pytest.mark.parametrize("tile", range(6))
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("dm,dn,K", [(1, 36, 192), (0, 0, 448), (-1, -8, 576), (3, 20, 4096)])
+def test_gemm_mid_tiles(tile, splits, dm, dn, K):
+    """Every tile of the mid-size GEMM, whole and with K over three workgroups, at
+    sizes around its borders: plain, bias, activations, residual, gated, folded
+    norm and fp32 outputs, strided operands and rows that no vector store fits.
+    Inputs are bf16 and sums fp32, so a result is off by its rounding to bf16 (2^-9
+    at most, 1.1e-3 rms) and an fp32 one by the order of its sums."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    bm, bn = MID_TILES[tile]
+    M, N = bm * (2 if bm == 64 else 1) + dm, bn + dn
+    g = torch.Generator(device=DEV).manual_seed(tile * 10 + splits)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    x, w = rnd(M, K + 8).bfloat16()[:, :K], (rnd(N, K + 16) * K ** -0.5).bfloat16()[:, :K]
+    b, ws = rnd(N), torch.zeros((4 * 3 * M * 2 * N) + 4096, dtype=torch.uint8, device=DEV)
+    st, cs = torch.rand(M, 2, device=DEV, generator=g) + 0.5, w.float().sum(1).contiguous()
+    r, odd = rnd(M, N).bfloat16(), torch.empty((M, N + 3), dtype=torch.bfloat16, device=DEV)[:, :N]
+    consts = torch.tensor([0.7, 1.3], device=DEV)
+    wg = (rnd(2 * (-(-N // 16) * 16), K) * K ** -0.5).bfloat16()
+    calls = [(dict(bias=b, act=a, residual=r), w, b, r, a, None) for a in (0, 1, 2)]
+    calls += [(dict(rowstat=st, colsum=cs, bias=b), w, b, None, 0, (st, cs)), (dict(out_dtype=torch.float32), w, None, None, 0, None),
+              (dict(bias=torch.cat([b, consts]), act=6), w, b, None, 6, None), (dict(out=odd, residual=r), w, None, r, 0, None),
+              (dict(act=3), wg, None, None, 3, None), (dict(act=4), wg, None, None, 4, None)]
+    G.set_gemm_mid(tile, splits)
+    try:
+        for kw, wt, bias, res, act, norm in calls:
+            y = G.linear(x, wt, ws=ws, **kw)
+            assert torch.isfinite(y).all()
+            assert _rel(y, _mid_reference(x, wt, bias, res, act, norm, consts)) < (1e-5 if y.dtype == torch.float32 else 2.5e-3), kw.keys()
+    finally:
+        G.set_gemm_mid()
+    assert not ws[-4096:].any()  # the tickets of a decode workspace are not parts
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 768, 3072), (96, 4096, 14336), (200, 6144, 4096), (256, 768, 768), (257, 4800, 1600),
+                                   (700, 4096, 14336), (1071, 2304, 768), (4097, 768, 3072)])
+@pytest.mark.parametrize("room", [0, 1 << 22, 1 << 26])
+def test_gemm_chosen_tiles(M, N, K, room):
+    """The tile, split or decode kernel that the estimate picks, with and without room for parts."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x, w = torch.randn(M, K, device=DEV, generator=g).bfloat16(), torch.randn(N, K, device=DEV, generator=g).bfloat16()
+    w = (w.float() * K ** -0.5).bfloat16()
+    ws = torch.zeros(room + 4096, dtype=torch.uint8, device=DEV) if room else None
+    for sh in (None, G.shuffle_weight(w)):
+        assert _rel(G.linear(x, w, ws=ws, w_shuf=sh), x.float() @ w.float().t()) < 2.5e-3
+
+
+@pytest.mark.parametrize("B,T,H,Hkv,hd,pos0,S", [(1, 65, 12, 12, 64, 0, 80), (3, 43, 4, 2, 128, 5, 60), (1, 255, 25, 25, 64, 9, 300)])
+def test_qkv_scatter_small_prefill(B, T, H, Hkv, hd, pos0, S):
+    """Fewer rows than a 256 x 256 tile: scattered on every small tile == qkv rows + qkv_split."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    from distributed_neural_networks_amd.ops import transformer_ops as T_
+    g = torch.Generator(device=DEV).manual_seed(B * T)
+    d, N = 320, (H + 2 * Hkv) * hd
+    x = torch.randn(B * T, d, device=DEV, generator=g).bfloat16()
+    f = G.fold_norm(torch.randn(N, d, device=DEV, generator=g) * 0.05, torch.ones(d, device=DEV), torch.zeros(d, device=DEV),
+                    torch.randn(N, device=DEV, generator=g) * 0.02, False, 1e-5, DEV)
+    std, pos = torch.empty(B * T, d, device=DEV, dtype=torch.bfloat16), torch.full((B,), pos0, device=DEV, dtype=torch.int32)
+    for tile in range(6):
+        caches = [torch.zeros(B, Hkv, S, hd, device=DEV).bfloat16() for _ in range(4)]
+        q, q2 = (torch.empty(B * H * T * hd, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+        G.set_gemm_mid(tile)
+        try:
+            assert G.qkv_scatter_norm(x, f, std, q, caches[0], caches[1], pos, B, T, H, Hkv, hd)
+            qkv = G.linear_norm(x, f, std_buf=std, ones=torch.ones(d, device=DEV))
+        finally:
+            G.set_gemm_mid()
+        T_.qkv_split(qkv, q2, caches[2], caches[3], B, T, H, Hkv, hd, pos)
+        keep = pos0 + torch.arange(T, device=DEV) < S
+        assert torch.equal(q.view(B, H, T, hd)[:, :, keep], q2.view(B, H, T, hd)[:, :, keep])
+        assert torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3])
