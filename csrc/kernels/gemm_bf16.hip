@@ -19,6 +19,7 @@
 #include "api.h"
 #include "gemm_epilogue.h"
 #include "gemm_mid_api.h"
+#include "gemm_mid_fp8.h"
 #include "gemm_tile.h"
 
 namespace dnn {
@@ -529,10 +530,10 @@ static int launch_gemm(const void* A, int lda, const void* W, int ldw, void* C, 
   } else if (g_mid_tile >= 0) plan = {g_mid_tile, (long long)g_mid_splits * M * N * 4 <= part_bytes ? g_mid_splits : 1, 0.f};
   else if (g_gemm_tile == 128) plan.tile = 2;
   else if (g_gemm_tile == 0 && (is_glu(ACT) || has_consts(ACT) || tail_split_cols(M, N) == 0))
-    plan = mid_plan(M, N, K, part_bytes, false);
+    plan = mid_plan(M, N, K, part_bytes, MID_BF16);
   if (plan.tile >= 0) {
-    const MidArgs a{(const bf16_t*)A, (const bf16_t*)W, C, bias, (const bf16_t*)R, rowstat, colsum, (float*)ws, lda, ldw,
-                    ldc, ldr, M, N, K, plan.splits, ACT, F32 ? 1 : 0};
+    const MidArgs a{{C, bias, (const bf16_t*)R, ldc, ldr, M, N, ACT, F32 ? 1 : 0}, (const bf16_t*)A, (const bf16_t*)W,
+                    rowstat, colsum, (float*)ws, lda, ldw, K, plan.splits};
     return mid_launch(plan.tile, a, nullptr, st);
   }
   const int tilesH = ((M + BG_M - 1) / BG_M) * ((N + 127) / 128);
@@ -631,11 +632,11 @@ extern "C" int dnn_gemm_bf16_qkv_scatter(const void* A, int lda, const void* W, 
   if ((hd & (hd - 1)) != 0 || M >= (1 << 24)) return -3;
   QkvScatter sc{(bf16_t*)q, (bf16_t*)kc, (bf16_t*)vc, pos, T, H, Hkv, __builtin_ctz(hd), S, 1.0f / (float)T};
   if (g_gemm_tile == 0 && tail_split_cols(M, N) == 0 && lda < 1 << 23 && ldw < 1 << 23) {
-    MidPlan plan = mid_plan(M, N, K, 0, true);
+    MidPlan plan = mid_plan(M, N, K, 0, MID_BF16);
     if (g_mid_tile >= 0) plan.tile = g_mid_tile;
     if (plan.tile >= 0) {
-      const MidArgs a{(const bf16_t*)A, (const bf16_t*)W, q, bias, nullptr, reinterpret_cast<const float2*>(rowstat),
-                      colsum, nullptr, lda, ldw, hd, 0, M, N, K, 1, ACT_NONE, 0};
+      const MidArgs a{{q, bias, nullptr, hd, 0, M, N, ACT_NONE, 0}, (const bf16_t*)A, (const bf16_t*)W,
+                      reinterpret_cast<const float2*>(rowstat), colsum, nullptr, lda, ldw, K, 1};
       return mid_launch(plan.tile, a, &sc, st);
     }
   }
@@ -726,7 +727,15 @@ extern "C" int dnn_gemm_fp8_256(const void* A, const float* sa, const void* W, c
   return -2;
 }
 
-// MX-scaled W8A8 GEMM on the 256^2 kernel: A8 [M][Kb]
+// Tile of gemm_mid.h for an MX product, -1: the 256 x 256 kernel.  A K-tile of 128
+// bytes takes a tile as long as the bf16 kernel's K-tile of 64: the same estimate.
+static int mx_mid_tile(int M, int N, int Kb, bool quant) {
+  if (g_gemm_tile != 0) return -1;
+  if (g_mid_tile >= 0) return g_mid_tile == 3 || (quant && g_mid_tile < 2) ? 2 : g_mid_tile;
+  return mid_plan(M, N, Kb / 2, 0, quant ? MID_MX_QUANT : MID_MX).tile;
+}
+
+// MX-scaled W8A8 GEMM: A8 [M][Kb]
 // e4m3 with e8m0 scales sx per (row, 128-column K-tile) (common.h mx_index;
 // dnn_quant_fp8_mx / dnn_layernorm_q8_mx / a QOUT epilogue write them), W8 /
 // sw per-channel e4m3.  qo != nullptr (act GELU): the output is quantised in
@@ -744,6 +753,12 @@ extern "C" int dnn_gemm_fp8_mx(const void* A8, const void* sx, const void* W8, c
   if (is_glu(act) && N % 16 != 0) return -1;
   const int tiles = ((M + BG_M - 1) / BG_M) * ((N + BG_N - 1) / BG_N);
   const uint32_t* sxw = reinterpret_cast<const uint32_t*>(sx);
+  const int mid = mx_mid_tile(M, N, Kb, qo != nullptr);
+  if (mid >= 0 && act <= ACT_SILU_MUL) {
+    const Mid8Args a{{C, bias, (const bf16_t*)R, ldc, ldr, M, N, act, 0}, (const uint8_t*)A8, (const uint8_t*)W8, sxw, sw,
+                     (uint8_t*)qo, (uint8_t*)sxo, Kb, ldq, kpo};
+    return mid8_launch(mid, a, nullptr, st);
+  }
   if (qo != nullptr) {
     hipLaunchKernelGGL((gemm_fp8_256_kernel<ACT_GELU, false, 2, true, true>), dim3(tiles), dim3(512), 0, st,
                        (const uint8_t*)A8, (const float*)nullptr, (const uint8_t*)W8, sw, (bf16_t*)nullptr, 0, bias,
@@ -772,6 +787,12 @@ extern "C" int dnn_gemm_fp8_qkv_scatter_mx(const void* A8, const void* sx, const
   if (N % 32 != 0 || M < 256 || N < 256 || ((uintptr_t)bias & 15) != 0) return -3;
   if ((hd & (hd - 1)) != 0 || M >= (1 << 24)) return -3;
   QkvScatter sc{(bf16_t*)q, (bf16_t*)kc, (bf16_t*)vc, pos, T, H, Hkv, __builtin_ctz(hd), S, 1.0f / (float)T};
+  const int mid = mx_mid_tile(M, N, Kb, false);
+  if (mid >= 0) {
+    const Mid8Args a{{q, bias, nullptr, hd, 0, M, N, ACT_NONE, 0}, (const uint8_t*)A8, (const uint8_t*)W8,
+                     reinterpret_cast<const uint32_t*>(sx), sw, nullptr, nullptr, Kb, 0, 0};
+    return mid8_launch(mid, a, &sc, st);
+  }
   const int tiles = ((M + BG_M - 1) / BG_M) * ((N + BG_N - 1) / BG_N);
   hipLaunchKernelGGL((gemm_fp8_256_kernel<ACT_NONE, true, 2, true>), dim3(tiles), dim3(512), 0, st, (const uint8_t*)A8,
                      (const float*)nullptr, (const uint8_t*)W8, sw, (bf16_t*)q, hd, bias, (const bf16_t*)nullptr, 0, M,

@@ -20,6 +20,14 @@ struct MidTile {
   static_assert(J % 2 == 0 && PA >= 1 && PB >= 1 && S >= 2, "");
 };
 
+// The tile table (costs: gemm_mid.hip MID)
+typedef MidTile<64, 64, 2, 2, 4> Mid0;
+typedef MidTile<128, 64, 2, 2, 6> Mid1;
+typedef MidTile<128, 128, 2, 4, 4> Mid2;
+typedef MidTile<192, 128, 2, 2, 3> Mid3;
+typedef MidTile<256, 128, 4, 2, 3> Mid4;
+typedef MidTile<128, 256, 2, 4, 3> Mid5;
+
 // s_waitcnt operand: at most `vm` vector-memory and `lgkm` LDS operations outstanding
 constexpr int wait_imm(int vm, int lgkm) { return (vm & 15) | (vm >> 4) << 14 | 7 << 4 | lgkm << 8; }
 
@@ -47,14 +55,14 @@ __device__ __forceinline__ f32x4 mid_act(f32x4 v, const f32x2& xc) {
 }
 
 // 4 finished columns of a row: residual and store, bf16 or fp32.
-__device__ __forceinline__ void epi_t4_any(const f32x4& v, int m, int n, int M, int N, const MidArgs& p, const bf16_t* R,
+__device__ __forceinline__ void epi_t4_any(const f32x4& v, int m, int n, int M, int N, const MidRows& p, const bf16_t* R,
                                            bool vec) {
   if (p.f32) epi_t4<ACT_NONE, true>(v, m, n, M, N, p.C, p.ldc, nullptr, R, p.ldr, vec);
   else epi_t4<ACT_NONE, false>(v, m, n, M, N, p.C, p.ldc, nullptr, R, p.ldr, vec);
 }
 
 // Bias and an elementwise activation on a wave's accumulators.
-template <int I, int J>
+template <int I, int J, bool ALL = true>
 __device__ __forceinline__ void mid_bias_act(f32x4 (&acc)[I][J], const float* bias, int act, int n0, int N) {
   if (bias != nullptr) {
 #pragma unroll
@@ -74,12 +82,121 @@ __device__ __forceinline__ void mid_bias_act(f32x4 (&acc)[I][J], const float* bi
     for (int i = 0; i < I; ++i)
 #pragma unroll
       for (int j = 0; j < J; ++j) acc[i][j] = mid_act<ACT_RELU>(acc[i][j], f32x2{});
-  } else if (act == ACT_XIELU) {
+  } else if (ALL && act == ACT_XIELU) {
     const f32x2 xc = act_consts<ACT_XIELU>(bias, N);
 #pragma unroll
     for (int i = 0; i < I; ++i)
 #pragma unroll
       for (int j = 0; j < J; ++j) acc[i][j] = mid_act<ACT_XIELU>(acc[i][j], xc);
+  }
+}
+
+// Staging of K-tiles (128 bytes of a row): uniform tile bases, per-lane offsets of
+// the wave's 1-KiB pieces of 8 rows, 16-byte chunks swizzled by row.
+template <class T>
+struct MidSource {
+  const char* a;
+  const char* b;
+  char* lds;
+  int nk, wave;
+  uint32_t oa[T::PA], ob[T::PB];
+  __device__ __forceinline__ void init(const char* A, int lda, int m0, int M, const char* W, int ldw, int n0, int N, int k0,
+                                       int nk_, char* smem, int wave_, int lane) {
+    a = A + (size_t)m0 * lda + (size_t)k0 * 128;
+    b = W + (size_t)n0 * ldw + (size_t)k0 * 128;
+    lds = smem, nk = nk_, wave = wave_;
+#pragma unroll
+    for (int q = 0; q < T::PA; ++q) {
+      const int rl = (q * T::NW + wave) * 8 + (lane >> 3);
+      oa[q] = (uint32_t)min(rl, M - 1 - m0) * (uint32_t)lda + (uint32_t)((lane & 7) ^ swz_chunk(rl)) * 16u;
+    }
+#pragma unroll
+    for (int q = 0; q < T::PB; ++q) {
+      const int rl = (q * T::NW + wave) * 8 + (lane >> 3);
+      ob[q] = (uint32_t)min(rl, N - 1 - n0) * (uint32_t)ldw + (uint32_t)((lane & 7) ^ swz_chunk(rl)) * 16u;
+    }
+  }
+  // Part i of n of K-tile t; past the end: a harmless refill, so that the waits count alike
+  __device__ __forceinline__ void stage(int t, int buf, int i, int n) const {
+    const size_t k = (size_t)min(t, nk - 1) * 128;
+    char* d = lds + buf * T::STAGE + wave * 1024;
+#pragma unroll
+    for (int q = T::PA * i / n; q < T::PA * (i + 1) / n; ++q) glds16(a + k + oa[q], d + q * T::NW * 1024);
+#pragma unroll
+    for (int q = T::PB * i / n; q < T::PB * (i + 1) / n; ++q) glds16(b + k + ob[q], d + T::BM * 128 + q * T::NW * 1024);
+  }
+};
+
+// A wave's accumulators to head-major q / K / V (host: N % 32 == 0).
+template <int I, int J>
+__device__ __forceinline__ void mid_scatter(const f32x4 (&acc)[I][J], int mw, int nw, int M, int N, const float* bias, int lane,
+                                            const QkvScatter& scat) {
+  int spos[I];
+#pragma unroll
+  for (int i = 0; i < I; ++i) spos[i] = qkv_row_pos(scat, min(mw + i * 16, M - 1));
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int jp = 0; jp < J / 2; ++jp)
+      if (nw + jp * 32 < N)
+        epi_pair_scatter(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, nw + jp * 32, M, bias, lane, scat, spos[i]);
+}
+
+// A wave's accumulators (rows mw + 16 i of this lane, columns from nw on) through the epilogue to C.
+// ALL: with fp32 rows and the activations that only bf16 weights have.
+template <int I, int J, bool ALL = true>
+__device__ __forceinline__ void mid_rows(f32x4 (&acc)[I][J], int mw, int nw, int lane, const MidRows& p) {
+  const int M = p.M, N = p.N, fg = lane >> 4;
+  const bool f32 = ALL && p.f32;
+  const bool vec = epi_vec_ok(p.C, p.ldc, p.bias, p.R, p.ldr);
+  if (is_glu(p.act)) {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int jp = 0; jp < J / 2; ++jp) {
+        const f32x4 &x0 = acc[i][2 * jp], &x1 = acc[i][2 * jp + 1];
+        const int m = mw + i * 16, c = (nw + jp * 32) / 2;
+        if (ALL && p.act == ACT_GELU_TANH_MUL) epi_glu_pair<ACT_GELU_TANH_MUL, false>(x0, x1, m, c, M, N / 2, p.C, p.ldc, vec, lane);
+        else if (f32) epi_glu_pair<ACT_SILU_MUL, true>(x0, x1, m, c, M, N / 2, p.C, p.ldc, vec, lane);
+        else epi_glu_pair<ACT_SILU_MUL, false>(x0, x1, m, c, M, N / 2, p.C, p.ldc, vec, lane);
+      }
+    return;
+  }
+  mid_bias_act<I, J, ALL>(acc, p.bias, p.act, nw + fg * 4, N);
+  bf16_t* C = reinterpret_cast<bf16_t*>(p.C);
+  const bool pair = vec && !f32 && epi_pair_ok(p.C, p.ldc, p.bias, p.R, p.ldr) && nw + J * 16 <= N;
+  if (pair && p.R != nullptr) {  // every residual load before the first output
+    bf16x4 rr[I][J / 2][2];
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int jp = 0; jp < J / 2; ++jp)
+        epi_pair_res_load(mw + i * 16, nw + jp * 32, M, p.R, p.ldr, lane, rr[i][jp][0], rr[i][jp][1]);
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int jp = 0; jp < J / 2; ++jp)
+        epi_pair_bf16<ACT_NONE, true>(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, nw + jp * 32, M, C, p.ldc, nullptr,
+                                      p.R, p.ldr, lane, rr[i][jp][0], rr[i][jp][1]);
+  } else if (pair) {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int jp = 0; jp < J / 2; ++jp)
+        epi_pair_bf16<ACT_NONE>(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, nw + jp * 32, M, C, p.ldc, nullptr, nullptr,
+                                0, lane);
+  } else if (f32) {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        epi_t4<ACT_NONE, true>(acc[i][j], mw + i * 16, nw + j * 16 + fg * 4, M, N, p.C, p.ldc, nullptr, p.R, p.ldr, vec);
+  } else {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        epi_t4<ACT_NONE, false>(acc[i][j], mw + i * 16, nw + j * 16 + fg * 4, M, N, p.C, p.ldc, nullptr, p.R, p.ldr, vec);
   }
 }
 
@@ -120,31 +237,9 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvS
     k0 = (int)((long long)nk * sp / p.splits);
     nk = (int)((long long)nk * (sp + 1) / p.splits) - k0;
   }
-  // staging: uniform tile bases, per-lane offsets of the wave's pieces
-  const char* a0 = reinterpret_cast<const char*>(p.A + (size_t)m0 * p.lda) + (size_t)k0 * 128;
-  const char* b0 = reinterpret_cast<const char*>(p.W + (size_t)n0 * p.ldw) + (size_t)k0 * 128;
-  uint32_t oa[T::PA], ob[T::PB];
-#pragma unroll
-  for (int q = 0; q < T::PA; ++q) {
-    const int rl = (q * T::NW + wave) * 8 + (lane >> 3);
-    oa[q] = (uint32_t)min(rl, M - 1 - m0) * (uint32_t)p.lda * 2u + (uint32_t)((lane & 7) ^ swz_chunk(rl)) * 16u;
-  }
-#pragma unroll
-  for (int q = 0; q < T::PB; ++q) {
-    const int rl = (q * T::NW + wave) * 8 + (lane >> 3);
-    ob[q] = (uint32_t)min(rl, N - 1 - n0) * (uint32_t)p.ldw * 2u + (uint32_t)((lane & 7) ^ swz_chunk(rl)) * 16u;
-  }
-  // pieces [q0, q1) of K-tile t; past the end: a harmless refill, so that the waits count alike
-  auto stage_a = [&](int t, int buf, int q0, int q1) {
-    const char* as = a0 + (size_t)min(t, nk - 1) * 128;
-#pragma unroll
-    for (int q = q0; q < q1; ++q) glds16(as + oa[q], smem + buf * T::STAGE + (q * T::NW + wave) * 1024);
-  };
-  auto stage_b = [&](int t, int buf, int q0, int q1) {
-    const char* bs = b0 + (size_t)min(t, nk - 1) * 128;
-#pragma unroll
-    for (int q = q0; q < q1; ++q) glds16(bs + ob[q], smem + buf * T::STAGE + T::BM * 128 + (q * T::NW + wave) * 1024);
-  };
+  MidSource<T> src;
+  src.init(reinterpret_cast<const char*>(p.A), p.lda * 2, m0, M, reinterpret_cast<const char*>(p.W), p.ldw * 2, n0, N, k0,
+           nk, smem, wave, lane);
   // fragment reads: lane (r, g) reads 16 B of row r at chunks g and 4 + g
   const int fr = lane & 15, fg = lane >> 4;
   const int arow = wm * (I * 16) + fr, brow = wn * (J * 16) + fr;
@@ -175,8 +270,7 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvS
   constexpr auto h1 = std::integral_constant<int, 1>{};
 #pragma unroll
   for (int q = 0; q < S - 1; ++q) {
-    stage_a(q, q, 0, T::PA);
-    stage_b(q, q, 0, T::PB);
+    src.stage(q, q, 0, 1);
   }
   __builtin_amdgcn_s_waitcnt(wait_imm((S - 2) * L, 0));
   bg_barrier();
@@ -190,8 +284,7 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvS
       mma(h0, i);
       __builtin_amdgcn_sched_barrier(0);
       if (i == 0) read(h1, cur);
-      stage_a(t + S - 1, prev, T::PA * i / I, T::PA * (i + 1) / I);
-      stage_b(t + S - 1, prev, T::PB * i / I, T::PB * (i + 1) / I);
+      src.stage(t + S - 1, prev, i, I);
       __builtin_amdgcn_sched_barrier(0);
     }
     __builtin_amdgcn_s_waitcnt(wait_imm((S - 2) * L, 0));  // tile t + 1 landed, tile t read
@@ -235,68 +328,8 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvS
 #pragma unroll
       for (int j = 0; j < J; ++j) acc[i][j] = acc[i][j] * rs[i].x + rs[i].y * cs[j];
   }
-  if constexpr (OUT == MID_SCATTER) {
-    int spos[I];
-#pragma unroll
-    for (int i = 0; i < I; ++i) spos[i] = qkv_row_pos(scat, min(mw + i * 16, M - 1));
-#pragma unroll
-    for (int i = 0; i < I; ++i)
-#pragma unroll
-      for (int jp = 0; jp < J / 2; ++jp)
-        if (nw + jp * 32 < N)  // host: N % 32 == 0
-          epi_pair_scatter(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, nw + jp * 32, M, p.bias, lane, scat, spos[i]);
-    return;
-  }
-  const bool vec = epi_vec_ok(p.C, p.ldc, p.bias, p.R, p.ldr);
-  if (is_glu(p.act)) {
-#pragma unroll
-    for (int i = 0; i < I; ++i)
-#pragma unroll
-      for (int jp = 0; jp < J / 2; ++jp) {
-        const f32x4 &x0 = acc[i][2 * jp], &x1 = acc[i][2 * jp + 1];
-        const int m = mw + i * 16, c = (nw + jp * 32) / 2;
-        if (p.act == ACT_GELU_TANH_MUL) epi_glu_pair<ACT_GELU_TANH_MUL, false>(x0, x1, m, c, M, N / 2, p.C, p.ldc, vec, lane);
-        else if (p.f32) epi_glu_pair<ACT_SILU_MUL, true>(x0, x1, m, c, M, N / 2, p.C, p.ldc, vec, lane);
-        else epi_glu_pair<ACT_SILU_MUL, false>(x0, x1, m, c, M, N / 2, p.C, p.ldc, vec, lane);
-      }
-    return;
-  }
-  mid_bias_act<I, J>(acc, p.bias, p.act, nw + fg * 4, N);
-  bf16_t* C = reinterpret_cast<bf16_t*>(p.C);
-  const bool pair = vec && !p.f32 && epi_pair_ok(p.C, p.ldc, p.bias, p.R, p.ldr) && nw + J * 16 <= N;
-  if (pair && p.R != nullptr) {  // every residual load before the first output
-    bf16x4 rr[I][J / 2][2];
-#pragma unroll
-    for (int i = 0; i < I; ++i)
-#pragma unroll
-      for (int jp = 0; jp < J / 2; ++jp)
-        epi_pair_res_load(mw + i * 16, nw + jp * 32, M, p.R, p.ldr, lane, rr[i][jp][0], rr[i][jp][1]);
-#pragma unroll
-    for (int i = 0; i < I; ++i)
-#pragma unroll
-      for (int jp = 0; jp < J / 2; ++jp)
-        epi_pair_bf16<ACT_NONE, true>(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, nw + jp * 32, M, C, p.ldc, nullptr,
-                                      p.R, p.ldr, lane, rr[i][jp][0], rr[i][jp][1]);
-  } else if (pair) {
-#pragma unroll
-    for (int i = 0; i < I; ++i)
-#pragma unroll
-      for (int jp = 0; jp < J / 2; ++jp)
-        epi_pair_bf16<ACT_NONE>(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, nw + jp * 32, M, C, p.ldc, nullptr, nullptr,
-                                0, lane);
-  } else if (p.f32) {
-#pragma unroll
-    for (int i = 0; i < I; ++i)
-#pragma unroll
-      for (int j = 0; j < J; ++j)
-        epi_t4<ACT_NONE, true>(acc[i][j], mw + i * 16, nw + j * 16 + fg * 4, M, N, p.C, p.ldc, nullptr, p.R, p.ldr, vec);
-  } else {
-#pragma unroll
-    for (int i = 0; i < I; ++i)
-#pragma unroll
-      for (int j = 0; j < J; ++j)
-        epi_t4<ACT_NONE, false>(acc[i][j], mw + i * 16, nw + j * 16 + fg * 4, M, N, p.C, p.ldc, nullptr, p.R, p.ldr, vec);
-  }
+  if constexpr (OUT == MID_SCATTER) mid_scatter<I, J>(acc, mw, nw, M, N, p.bias, lane, scat);
+  else mid_rows<I, J>(acc, mw, nw, lane, p);
 }
 
 // Sum of the parts and the epilogue.  A thread: 4 columns of one row (gated: 4

@@ -19,12 +19,6 @@ static constexpr MidCost MID[] = {{64, 64, 1, 1.89f, 0.252f},   {128, 64, 0, 2.7
                                   {256, 128, 0, 4.14f, 0.707f}, {128, 256, 0, 4.07f, 0.754f},
                                   {256, 256, 0, 4.93f, 1.198f}};
 static constexpr int MID_TILES = 6, CUS = 256;
-typedef MidTile<64, 64, 2, 2, 4> Mid0;
-typedef MidTile<128, 64, 2, 2, 6> Mid1;
-typedef MidTile<128, 128, 2, 4, 4> Mid2;
-typedef MidTile<192, 128, 2, 2, 3> Mid3;
-typedef MidTile<256, 128, 4, 2, 3> Mid4;
-typedef MidTile<128, 256, 2, 4, 3> Mid5;
 
 // Time of one tile size and split: K-tiles of the fullest CU, beside the time that
 // reading the weights (4.3 TB/s) and moving the activations (2 TB/s) takes; a split
@@ -40,31 +34,34 @@ static float mid_time(const MidCost& c, int M, int N, int K, int splits) {
   return splits == 1 ? us : us + 8.f + (splits + 0.5f) * M * N * 4.f / 3.16e6f;
 }
 
-static MidPlan best_plan(int M, int N, int K, long long ws_bytes, bool scatter) {
+static MidPlan best_plan(int M, int N, int K, long long ws_bytes, unsigned kind) {
   // the 256 x 256 kernel needs to be 5 % slower to lose: the estimate's error at
   // its sizes (12352 columns of 3000 rows: 257 us, 267 as 256 x 128)
   MidPlan best{-1, 1, M < 256 || N < 256 ? 1e30f : 0.95f * mid_time(MID[MID_TILES], M, N, K, 1)};
-  for (int i = 0; i < MID_TILES; ++i)
+  for (int i = 0; i < MID_TILES; ++i) {
+    if (kind != MID_BF16 && (i == 3 || (kind == MID_MX_QUANT && MID[i].bn < 128))) continue;
     for (int s = 1; s <= 8; ++s) {
-      if (s > 1 && (scatter || N % 4 != 0 || M > 65535 || K / 64 / s < 3 || (long long)s * M * N * 4 > ws_bytes)) break;
+      if (s > 1 && ( N % 4 != 0 || M > 65535 || K / 64 / s < 3 || (long long)s * M * N * 4 > ws_bytes)) break;
       const float t = mid_time(MID[i], M, N, K, s);
       if (t < best.us) best = {i, s, t};
     }
+  }
   return best;
 }
 
 // The same by sizes: 48 estimates take 3 us of host time, a table entry (per thread)
 // nothing beside a launch.
-MidPlan mid_plan(int M, int N, int K, long long ws_bytes, bool scatter) {
+MidPlan mid_plan(int M, int N, int K, long long ws_bytes, unsigned kind) {
   struct Entry {
-    int M = 0, N = 0, K = 0, scatter = 0;
+    int M = 0, N = 0, K = 0;
+    unsigned kind = 0;
     long long ws = 0;
     MidPlan plan{};
   };
   static thread_local Entry table[256];
-  Entry& e = table[((unsigned)M * 2654435761u ^ (unsigned)N * 40503u ^ (unsigned)K * 97u ^ (scatter ? 77u : 0u)) >> 7 & 255];
-  if (e.M != M || e.N != N || e.K != K || e.scatter != (int)scatter || e.ws != ws_bytes)
-    e = {M, N, K, scatter ? 1 : 0, ws_bytes, best_plan(M, N, K, ws_bytes, scatter)};
+  Entry& e = table[((unsigned)M * 2654435761u ^ (unsigned)N * 40503u ^ (unsigned)K * 97u ^ kind * 77u) >> 7 & 255];
+  if (e.M != M || e.N != N || e.K != K || e.kind != kind || e.ws != ws_bytes)
+    e = {M, N, K, kind, ws_bytes, best_plan(M, N, K, ws_bytes, kind)};
   return e.plan;
 }
 
@@ -76,7 +73,7 @@ MidPlan mid_plan(int M, int N, int K, long long ws_bytes, bool scatter) {
 bool mid_skinny(int M, int N, int K, bool norm, bool frag, long long ws_bytes) {
   if (M <= 64) return true;
   if (M > 256) return false;
-  return 4.2f + (frag ? 2.0e-7f : 3.2e-7f) * N * K * ((M + 15) / 16) < mid_plan(M, N, K, ws_bytes, false).us + (norm ? 8.f : 0.f);
+  return 4.2f + (frag ? 2.0e-7f : 3.2e-7f) * N * K * ((M + 15) / 16) < mid_plan(M, N, K, ws_bytes, MID_BF16).us + (norm ? 8.f : 0.f);
 }
 
 template <class T, MidOut OUT>

@@ -5,16 +5,21 @@
 
 namespace dnn {
 
-struct MidArgs {
-  const bf16_t* A;
-  const bf16_t* W;
+// Output rows and their epilogue.
+struct MidRows {
   void* C;
   const float* bias;
   const bf16_t* R;
+  int ldc, ldr, M, N, act, f32;
+};
+
+struct MidArgs : MidRows {
+  const bf16_t* A;
+  const bf16_t* W;
   const float2* rowstat;
   const float* colsum;
   float* part;  // splits > 1: fp32 parts [splits][M][N]
-  int lda, ldw, ldc, ldr, M, N, K, splits, act, f32;
+  int lda, ldw, K, splits;
 };
 
 struct QkvScatter;
@@ -24,8 +29,10 @@ struct MidPlan {
   float us;    // estimated time
 };
 
-// `ws_bytes`: room for parts (0: no split).  `scatter`: head-major output, no split.
-MidPlan mid_plan(int M, int N, int K, long long ws_bytes, bool scatter);
+// `ws_bytes`: room for parts (0: no split).  `kind`: MID_BF16, or tiles that the MX
+// e4m3 kernel has (K then in 128-byte K-tiles x 64), all or with whole 128 columns.
+enum MidKind : unsigned { MID_BF16 = 0, MID_MX = 1, MID_MX_QUANT = 2 };
+MidPlan mid_plan(int M, int N, int K, long long ws_bytes, unsigned kind);
 // Whether M rows still run faster on the decode kernels (`norm`: with a folded norm; `frag`: with the weight's fragment-order copy).
 bool mid_skinny(int M, int N, int K, bool norm, bool frag, long long ws_bytes);
 // Bytes of a decode workspace that parts may use: its last 4 KiB hold the decode stream kernel's tickets.

@@ -47,6 +47,7 @@ PER_FILE_FLAGS = {"cifar_fused.hip": ["-ffast-math"],
                   "moe.hip": NO_SLP,
                   "gemm_skinny.hip": NO_SLP,
                   "gemm_mid.hip": NO_SLP,
+                  "gemm_mid_fp8.hip": NO_SLP,
                   "gemm_bf16.hip": NO_SLP}
 
 

@@ -1557,3 +1557,50 @@ def test_fp8_fidelity_vs_unquantised():
     # the weights, not the activation format, set the error: e4m3 activations
     # stay within 2x of the split format's prefill error
     assert r["fp8-e4m3"]["prefill_logits_rel"] < 2 * r["fp8-split"]["prefill_logits_rel"]
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 4, 5])
+@pytest.mark.parametrize("M,N,K", [(256, 256, 64), (257, 300, 200), (383, 520, 1600), (513, 388, 384)])
+def test_gemm_fp8_mx_small_tiles(tile, M, N, K):
+    """The MX product on the tiles below 256 x 256, at sizes around their borders:
+    bias, residual, activations, gated, and the epilogue that quantises its own
+    output, equal to the 256 x 256 kernel's up to the order of its rounding to bf16
+    (the same products in the same order; 2^-9 relative where a contraction
+    differs), quantised bytes up to a step of e4m3."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    from distributed_neural_networks_amd.ops.fp8 import (kpad_of, linear_fp8, mx_scale_bytes, quant_rows_mx, quantize_weight)
+    g = torch.Generator(device=DEV).manual_seed(M + tile)
+    x = torch.randn(M, K, device=DEV, generator=g).bfloat16()
+    w = quantize_weight(torch.randn(N, K, device=DEV, generator=g) * 0.05, DEV)
+    wg = quantize_weight(torch.randn(-(-N // 16) * 16, K, device=DEV, generator=g) * 0.05, DEV)
+    b, r = torch.randn(N, device=DEV, generator=g), torch.randn(M, N, device=DEV, generator=g).bfloat16()
+    kp, kpo = kpad_of(K), kpad_of(N)
+    q, sx = (torch.empty(n, dtype=torch.uint8, device=DEV) for n in (M * kp, mx_scale_bytes(M, kp)))
+    quant_rows_mx(x, q, sx)
+    xd = _mx_dequant(q.view(M, kp), sx, M, kp)[:, :K]
+    ref = (xd.double() @ (w.q[:, :K].float() * w.scale[:, None]).double().t()).float() + b
+
+    def run():
+        out = [linear_fp8(x, w, b, act, res, None, q, None, prequantized=True, sx=sx)
+               for act, res in ((0, r), (1, r), (2, None))]
+        out.append(linear_fp8(x, wg, None, 3, None, None, q, None, prequantized=True, sx=sx))
+        qo = torch.full((M * kpo,), 77, dtype=torch.uint8, device=DEV)
+        sxo = torch.full((mx_scale_bytes(M, kpo),), 127, dtype=torch.uint8, device=DEV)
+        linear_fp8(x, w, b, 2, None, None, q, None, prequantized=True, sx=sx, q_out=(qo, sxo))
+        return out, _mx_dequant(qo.view(M, kpo), sxo, M, kpo)
+    G.set_gemm_mid(tile)
+    try:
+        got, gq = run()
+    finally:
+        G.set_gemm_mid()
+    G.set_gemm_tile(256)
+    try:
+        want, wq = run()
+    finally:
+        G.set_gemm_tile(0)
+    for y, z in zip(got, want):
+        assert _rel(y, z) < 2e-3
+    assert _rel(got[0], ref + r.float()) < 3e-3
+    assert torch.equal(gq[:, N:], torch.zeros_like(gq[:, N:]))
+    assert _rel(gq, wq) < 1e-3
+    assert _rel(gq[:, :N], torch.nn.functional.gelu(ref)) < 4e-2
