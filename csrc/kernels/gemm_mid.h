@@ -200,8 +200,6 @@ __device__ __forceinline__ void mid_rows(f32x4 (&acc)[I][J], int mw, int nw, int
   }
 }
 
-enum MidOut { MID_ROWS = 0, MID_SCATTER = 1, MID_PART = 2 };
-
 // Loop: a K-tile of 64 is multiplied in two halves of 32; the second half's
 // fragments are read behind the first row of products of the first, the next
 // tile's first half behind the first row of the second, one barrier a tile.  The
@@ -212,34 +210,9 @@ enum MidOut { MID_ROWS = 0, MID_SCATTER = 1, MID_PART = 2 };
 // take 0.22 and its LDS traffic 0.33; larger tiles need fewer bytes per product but
 // more splits.  Touching later lines from a wave of its own, waves of 64 x 32 in
 // place of 64 x 64, or padded rows did not change that.
-template <class T, MidOut OUT>
-__global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvScatter scat) {
-  constexpr bool PART = OUT == MID_PART;
+template <class T>
+__device__ __forceinline__ void mid_loop(const MidSource<T>& src, int wm, int wn, int lane, f32x4 (&acc)[T::I][T::J]) {
   constexpr int I = T::I, J = T::J, S = T::S, L = T::PA + T::PB;
-  // S * STAGE bytes, given at launch: with the size in the kernel the compiler sees one
-  // wave per SIMD and moves accumulators of the four-wave tiles to AGPRs and back in
-  // the loop (192 x 128 at 700 x 6144 x 4096: 47 -> 78 us)
-  extern __shared__ __attribute__((aligned(1024))) char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int M = p.M, N = p.N;
-  const int ntn = (N + T::BN - 1) / T::BN, ntm = (M + T::BM - 1) / T::BM, tiles = ntm * ntn;
-  int id = xcd_remap(blockIdx.x, tiles * p.splits), sp = 0;
-  if constexpr (PART) {
-    sp = id / tiles;
-    id -= sp * tiles;
-  }
-  int tm, tn;
-  tile_coords(id, ntm, ntn, tm, tn);
-  const int m0 = tm * T::BM, n0 = tn * T::BN;
-  const int wm = wave / T::WN, wn = wave % T::WN;
-  int nk = p.K >> 6, k0 = 0;
-  if constexpr (PART) {
-    k0 = (int)((long long)nk * sp / p.splits);
-    nk = (int)((long long)nk * (sp + 1) / p.splits) - k0;
-  }
-  MidSource<T> src;
-  src.init(reinterpret_cast<const char*>(p.A), p.lda * 2, m0, M, reinterpret_cast<const char*>(p.W), p.ldw * 2, n0, N, k0,
-           nk, smem, wave, lane);
   // fragment reads: lane (r, g) reads 16 B of row r at chunks g and 4 + g
   const int fr = lane & 15, fg = lane >> 4;
   const int arow = wm * (I * 16) + fr, brow = wn * (J * 16) + fr;
@@ -250,13 +223,12 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvS
   bf16x8 f[2][I + J];
   auto read = [&](auto hc, int buf) {
     constexpr int h = decltype(hc)::value;
-    const char* d = smem + buf * T::STAGE;
+    const char* d = src.lds + buf * T::STAGE;
 #pragma unroll
     for (int j = 0; j < J; ++j) f[h][I + j] = *reinterpret_cast<const bf16x8*>(d + bo[h] + j * 2048);
 #pragma unroll
     for (int i = 0; i < I; ++i) f[h][i] = *reinterpret_cast<const bf16x8*>(d + ao[h] + i * 2048);
   };
-  f32x4 acc[I][J];
 #pragma unroll
   for (int i = 0; i < I; ++i)
 #pragma unroll
@@ -269,14 +241,12 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvS
   constexpr auto h0 = std::integral_constant<int, 0>{};
   constexpr auto h1 = std::integral_constant<int, 1>{};
 #pragma unroll
-  for (int q = 0; q < S - 1; ++q) {
-    src.stage(q, q, 0, 1);
-  }
+  for (int q = 0; q < S - 1; ++q) src.stage(q, q, 0, 1);
   __builtin_amdgcn_s_waitcnt(wait_imm((S - 2) * L, 0));
   bg_barrier();
   read(h0, 0);
   int cur = 0;
-  for (int t = 0; t < nk; ++t) {
+  for (int t = 0; t < src.nk; ++t) {
     const int prev = cur == 0 ? S - 1 : cur - 1, next = cur == S - 1 ? 0 : cur + 1;
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
@@ -300,6 +270,40 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvS
     cur = next;
   }
   __builtin_amdgcn_s_waitcnt(wait_imm(0, 0));
+}
+
+enum MidOut { MID_ROWS = 0, MID_SCATTER = 1, MID_PART = 2 };
+
+template <class T, MidOut OUT>
+__global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvScatter scat) {
+  constexpr bool PART = OUT == MID_PART;
+  constexpr int I = T::I, J = T::J;
+  // S * STAGE bytes, given at launch: with the size in the kernel the compiler sees one
+  // wave per SIMD and moves accumulators of the four-wave tiles to AGPRs and back in
+  // the loop (192 x 128 at 700 x 6144 x 4096: 47 -> 78 us)
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int M = p.M, N = p.N;
+  const int ntn = (N + T::BN - 1) / T::BN, ntm = (M + T::BM - 1) / T::BM, tiles = ntm * ntn;
+  int id = xcd_remap(blockIdx.x, tiles * p.splits), sp = 0;
+  if constexpr (PART) {
+    sp = id / tiles;
+    id -= sp * tiles;
+  }
+  int tm, tn;
+  tile_coords(id, ntm, ntn, tm, tn);
+  const int m0 = tm * T::BM, n0 = tn * T::BN;
+  const int wm = wave / T::WN, wn = wave % T::WN, fr = lane & 15, fg = lane >> 4;
+  int nk = p.K >> 6, k0 = 0;
+  if constexpr (PART) {
+    k0 = (int)((long long)nk * sp / p.splits);
+    nk = (int)((long long)nk * (sp + 1) / p.splits) - k0;
+  }
+  MidSource<T> src;
+  src.init(reinterpret_cast<const char*>(p.A), p.lda * 2, m0, M, reinterpret_cast<const char*>(p.W), p.ldw * 2, n0, N, k0,
+           nk, smem, wave, lane);
+  f32x4 acc[I][J];
+  mid_loop<T>(src, wm, wn, lane, acc);
 
   if constexpr (PART) {
     float* d = p.part + (size_t)sp * M * N;

@@ -4,12 +4,12 @@
 // gemm_f32).  W has few rows (the side dimension, padded to 64), so a plain
 // GEMM grid would leave most CUs idle:
 //
-//   rows <= 256   a workgroup takes 16 columns of 16 rows; eight waves split
-//                 K (one round trip for K <= 4096) over W in fragment order
-//                 (ops/gemm.py shuffle_weight) and reduce through LDS
-//   more rows     64 x 64 or 64 x 128 tiles, six LDS stages of the K loop,
-//                 five in flight (the K loop is latency-bound at one workgroup per CU)
+//   few rows    a workgroup takes 16 columns of 16 rows; eight waves split
+//               K (one round trip for K <= 4096) over W in fragment order
+//               (ops/gemm.py shuffle_weight) and reduce through LDS
+//   more rows   64 x 64 tiles on the loop of gemm_mid.h
 #include "common.h"
+#include "gemm_mid.h"
 #include "residual_api.h"
 
 namespace dnn {
@@ -76,81 +76,30 @@ __global__ __launch_bounds__(64 * (TG_WAVES + 1)) void token_gate_skinny_kernel(
   __syncthreads();
 }
 
-constexpr int TG_BM = 64, TG_BK = 64, TG_ST = 6;
-
-// One wave-instruction copies 8 rows x 128 B; 16-B chunk p of row r holds
-// logical chunk p ^ (r & 7).
-__device__ __forceinline__ void tg_stage8(const bf16_t* src, int ld, int row0, int rows, int k, char* lds, int lane) {
-  const int r = lane >> 3, c = (lane & 7) ^ r;
-  glds16(src + (size_t)min(row0 + r, rows - 1) * ld + k + c * 8, lds);
-}
-__device__ __forceinline__ bf16x8 tg_frag(const char* lds, int r, int c) {
-  return *reinterpret_cast<const bf16x8*>(lds + r * 128 + ((c ^ (r & 7)) << 4));
-}
-
-template <int BN>
-__global__ __launch_bounds__(256) void token_gate_tile_kernel(const bf16_t* __restrict__ x, int ldx,
-                                                              const bf16_t* __restrict__ w, int ldw, int np, int K,
-                                                              TokenGate t) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  constexpr int STAGE = (TG_BM + BN) * 128, NI = (TG_BM + BN) / 32;  // NI: copies per wave and stage
-  constexpr int NJ = BN / 32;                                         // 16-column tiles of a wave
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int ntn = np / BN, b = xcd_remap(blockIdx.x, gridDim.x);
-  const int m0 = b / ntn * TG_BM, n0 = b % ntn * BN, nk = K / TG_BK;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * (BN / 2);
-  // Every workgroup starts at another K tile: in step, the 64 rows of all of
-  // them would ask the same few memory channels at a time (power-of-two strides)
-  const int k0 = (int)((b * 7u) % (unsigned)nk);
-  auto issue = [&](int s) __attribute__((always_inline)) {
-    const int kt = (s + k0 < nk ? s + k0 : s + k0 - nk) * TG_BK;
-    char* lds = smem + (s % TG_ST) * STAGE;
+template <class T>
+__global__ __launch_bounds__(T::NW * 64, 2) void token_gate_tile_kernel(const bf16_t* __restrict__ x, int ldx,
+                                                                        const bf16_t* __restrict__ w, int ldw, int np, int K,
+                                                                        TokenGate t) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  constexpr int I = T::I, J = T::J;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ntn = np / T::BN, b = xcd_remap(blockIdx.x, gridDim.x);
+  const int m0 = b / ntn * T::BM, n0 = b % ntn * T::BN, wm = wave / T::WN, wn = wave % T::WN;
+  const int mw = m0 + wm * (I * 16) + (lane & 15), cw = n0 + wn * (J * 16) + (lane >> 4) * 4;
+  float e[I][J][4];  // gathered ahead of the loop
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int q = wave * NI + i;  // 8-row group: first the x rows, then the weight rows
-      if (q < TG_BM / 8) tg_stage8(x, ldx, m0 + q * 8, t.M, kt, lds + q * 1024, lane);
-      else tg_stage8(w, ldw, n0 + (q - TG_BM / 8) * 8, np, kt, lds + q * 1024, lane);
-    }
-  };
-  f32x4 acc[2][NJ];
+  for (int i = 0; i < I; ++i)
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int j = 0; j < J; ++j) token_gate_row(t, mw + i * 16, cw + j * 16, e[i][j]);
+  MidSource<T> src;
+  src.init(reinterpret_cast<const char*>(x), ldx * 2, m0, t.M, reinterpret_cast<const char*>(w), ldw * 2, n0, np, 0, K / 64,
+           smem, wave, lane);
+  f32x4 acc[I][J];
+  mid_loop<T>(src, wm, wn, lane, acc);
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < TG_ST - 1 && s < nk; ++s) issue(s);
-  for (int k = 0; k < nk; ++k) {
-    // stage k has landed when only the stages issued after it are in flight
-    if (k + TG_ST - 2 < nk) asm volatile("s_waitcnt vmcnt(%0)" ::"i"((TG_ST - 2) * NI) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    // every wave's part of stage k landed, and stage k - 1 is read
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    if (k + TG_ST - 1 < nk) issue(k + TG_ST - 1);
-    const char* as = smem + (k % TG_ST) * STAGE;
-    const char* bs = as + TG_BM * 128;
+  for (int i = 0; i < I; ++i)
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int c = s * 4 + (lane >> 4);
-      bf16x8 af[2], bf[NJ];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) af[i] = tg_frag(as, wm + i * 16 + (lane & 15), c);
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) bf[j] = tg_frag(bs, wn + j * 16 + (lane & 15), c);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j], af[i], acc[i][j], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int m = m0 + wm + i * 16 + (lane & 15), c = n0 + wn + j * 16 + (lane >> 4) * 4;
-      float e[4];
-      token_gate_row(t, m, c, e);
-      token_gate_store(t, acc[i][j], m, c, e);
-    }
+    for (int j = 0; j < J; ++j) token_gate_store(t, acc[i][j], mw + i * 16, cw + j * 16, e[i][j]);
 }
 
 // g[m, c] = gelu_tanh(z[m, c]) * table[token[m], off + c] for c < n, 0 up to np.
@@ -181,15 +130,19 @@ extern "C" int dnn_token_gate(const void* x, int ldx, const void* w, int ldw, co
   if (ldx % 8 != 0 || ldw % 8 != 0 || ldx < K || ldw < K || ldg % 4 != 0 || ldg < np || wsh == nullptr) return -1;
   if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)wsh) & 15) != 0 || ((uintptr_t)g & 7) != 0) return -1;
   const TokenGate t{(const bf16_t*)table, tok, (bf16_t*)g, ldt, off, V, ldg, M, n};
-#define TGT(BN)                                                                                                    \
-  hipLaunchKernelGGL((token_gate_tile_kernel<BN>), dim3((unsigned)((M + TG_BM - 1) / TG_BM * (np / BN))), dim3(256), \
-                     TG_ST * (TG_BM + BN) * 128, st, (const bf16_t*)x, ldx, (const bf16_t*)w, ldw, np, K, t)
-  if (M <= 256)
+  // Few rows: rounds of 256 workgroups of 16 x 16 outputs, 6.4 us each for K up to
+  // 4096 (512 x 256 x 4096: 13.9 us, as tiles 17.0); tiles: 0.225 us a K-tile of 64
+  // (1024 x 256 x 4096: 16.9 us, as rounds 26.5; 30 with the six-stage loop of its own
+  // that read a tile's fragments between two barriers)
+  const float rounds = (float)(((M + 15) / 16 * (np / 16) + 255) / 256), passes = (float)((K + 4095) / 4096);
+  if (M <= 64 || 1.f + 6.4f * rounds * passes < 2.5f + 0.225f * K / 64) {
     hipLaunchKernelGGL(token_gate_skinny_kernel, dim3(np / 16, (M + 15) / 16), dim3(64 * (TG_WAVES + 1)), 0, st,
                        (const bf16_t*)x, ldx, (const uint8_t*)wsh, K, t);
-  else if (np % 128 == 0 && M > 4096) TGT(128);
-  else TGT(64);
-#undef TGT
+  } else {
+    typedef Mid0 T;
+    hipLaunchKernelGGL((token_gate_tile_kernel<T>), dim3((unsigned)((M + T::BM - 1) / T::BM * (np / T::BN))), dim3(T::NW * 64),
+                       T::S * T::STAGE, st, (const bf16_t*)x, ldx, (const bf16_t*)w, ldw, np, K, t);
+  }
   return (int)hipGetLastError();
 }
 

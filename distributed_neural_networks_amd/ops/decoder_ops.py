@@ -154,8 +154,12 @@ class TokenShift:
             _index(t, M, "token shift index")
         a.sh_mu, a.sh_state, a.sh_nslots = ptr(self.mu), ptr(self.state), self.state.shape[0]
         a.sh_start, a.sh_last, a.sh_slots, a.sh_pos = (ptr(t) for t in self.rows)
-        # neighbouring rows of a group of threads: a workgroup's, a wave's where rows are short
-        a.sh_rows = 1 if M <= 256 else 4 if self.mu.numel() <= 1024 else 8
+        # neighbouring rows of a group of threads (a workgroup's; a wave's where rows
+        # are short): more of them form fewer rows twice, but the rows of a group are a
+        # chain, so only what four workgroups a CU leave over.  4096 wide: 640 rows
+        # 11 us (8 at a time 29), 2048 24 (37), 4096 38 (41), 8192 92 (one at a time 124)
+        short = self.mu.numel() <= 1024
+        a.sh_rows = min(4 if short else 8, -(-M // (4096 if short and M > 256 else 1024)))
 
 
 def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor) -> torch.Tensor:
