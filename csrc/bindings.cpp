@@ -143,6 +143,11 @@ PYBIND11_MODULE(_dnn_hip, m) {
   m.def("cifar_head_tail_x3", [](u64 hid, u64 w2h, u64 w2l, u64 b2, u64 probs, u64 pred, int B, u64 st) {
     return dnn_cifar_head_tail_x3(CFP(hid), CP(w2h), CP(w2l), CFP(b2), FP(probs), IP(pred), B, ST(st));
   });
+  m.def("cifar_head_few", [](u64 a, int blocked, u64 wh, u64 wl, u64 b1, u64 part, u64 hid, u64 w2h, u64 w2l, u64 b2,
+                             u64 probs, u64 pred, int M, u64 st) {
+    return dnn_cifar_head_few(CFP(a), blocked, CP(wh), CP(wl), CFP(b1), FP(part), FP(hid), CP(w2h), CP(w2l), CFP(b2),
+                              FP(probs), IP(pred), M, ST(st));
+  });
   m.def("cifar_head_tail", [](u64 hid, u64 w2p, u64 b2, u64 probs, u64 pred, int B, u64 st) {
     return dnn_cifar_head_tail(CP(hid), CP(w2p), CFP(b2), FP(probs), IP(pred), B, ST(st));
   });

@@ -97,6 +97,9 @@ int dnn_cifar_fc1_x3(const float* A, int lda, const void* Wh, const void* Wl, in
 int dnn_cifar_split_blocked(const float* a, float* o, int M, int K, int dir, hipStream_t st);
 int dnn_cifar_head_tail_x3(const float* hid, const void* w2h, const void* w2l, const float* b2, float* probs, int* pred,
                            int B, hipStream_t st);
+int dnn_cifar_head_few(const float* A, int blocked, const void* Wh, const void* Wl, const float* b1, float* part,
+                       float* hid, const void* w2h, const void* w2l, const float* b2, float* probs, int* pred, int M,
+                       hipStream_t st);
 int dnn_cifar_head_tail(const void* hid, const void* w2p, const float* b2, float* probs, int* pred, int B,
                         hipStream_t st);
 // split: rows of 2 kpad bytes, e4m3 hi plane then the residual plane (W8A8 prefill with split activations)

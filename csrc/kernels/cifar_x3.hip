@@ -28,8 +28,10 @@
 //    tiles, 8 waves of 128x64, per k32 step 3 x 32 mfma_f32_16x16x32_bf16 per
 //    wave (A_hi W_hi + A_hi W_lo + A_lo W_hi) on 24 conflict-free ds_read_b128.
 //  * cifar_split3_kernel: fp32 (B,K) -> bf16 (B,3K) = [hi | hi | lo], the A
-//    operand of the small-batch fc1 (one skinny bf16 GEMM over K' = 3K against
+//    operand of the mid-batch fc1 (one bf16 GEMM over K' = 3K against
 //    W' = [W_hi | W_lo | W_hi]) when the 256^2 tiles cannot fill the chip.
+//  * cifar_stage0_x3_band_kernel, cifar_fc1_few_kernel, cifar_head_few_kernel: the
+//    same stages where the batch is too small to fill the chip with whole images.
 //  * cifar_head_tail_x3_kernel: fc2 (512->10) + bias + softmax + per-row argmax
 //    on fp32 hidden rows, 3-term split on mfma_f32_16x16x32_bf16.
 #include <type_traits>
@@ -97,6 +99,106 @@ __device__ __forceinline__ void c2_step(const uint32_t (&b)[3][2], const bf16x8 
   acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur[3], wh[S], acc[1], 0, 0, 0);
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (S + 1 < 18) c2_step<S + 1>(b, wh, wl, acc, nxt, cur);
+}
+
+// hi / lo planes of the pooled conv1 map: bias + ReLU + 2x2 max-pool of tile t in
+// registers (max(a)+b == max(a+b) exactly), quad-DPP gather of 4 channels of one
+// pooled pixel per lane, hi/lo split, one 8-B store per plane
+__device__ __forceinline__ void conv1_store(char* a1, int t, const f32x16& acc, float bias, int lane) {
+  const int h = lane >> 5, r32 = lane & 31;
+  const int q = ((r32 & 1) ? 2 : 0) + ((r32 & 2) ? 1 : 0);
+  const int cb = r32 & ~3;
+  const int ty = t >> 2, tx = t & 3;
+  float v[4];
+#pragma unroll
+  for (int qy = 0; qy < 2; ++qy)
+#pragma unroll
+    for (int qx = 0; qx < 2; ++qx) {
+      const int g0 = (2 * qy) * 4 + 2 * qx;
+      v[qy * 2 + qx] = fmaxf(fmax_nan(fmax_nan(acc[g0], acc[g0 + 1]), fmax_nan(acc[g0 + 4], acc[g0 + 5])) + bias, 0.f);
+    }
+  const bool odd = r32 & 1;
+  const int s0 = __float_as_int(odd ? v[0] : v[2]), s1 = __float_as_int(odd ? v[1] : v[3]);
+  const float r0 = __int_as_float(dpp_xor1(s0)), r1 = __int_as_float(dpp_xor1(s1));
+  uint32_t u0h, u0l, u1h, u1l;
+  if (!odd) {
+    split2(v[0], r0, u0h, u0l);
+    split2(v[1], r1, u1h, u1l);
+  } else {
+    split2(r0, v[2], u0h, u0l);
+    split2(r1, v[3], u1h, u1l);
+  }
+  const bool hi2 = r32 & 2;
+  const uint32_t rch = (uint32_t)dpp_xor2((int)(hi2 ? u0h : u1h));
+  const uint32_t rcl = (uint32_t)dpp_xor2((int)(hi2 ? u0l : u1l));
+  const uint32_t mh = hi2 ? u1h : u0h, ml = hi2 ? u1l : u0l;
+  uint2 wh, wl;
+  wh.x = hi2 ? rch : mh;
+  wh.y = hi2 ? mh : rch;
+  wl.x = hi2 ? rcl : ml;
+  wl.y = hi2 ? ml : rcl;
+  const int Y = 2 * ty + (q >> 1) + 1, X = 4 * tx + 2 * h + (q & 1) + 1;
+  const int o = (Y * 18 + X) * 64 + ((((cb >> 3) ^ (Y & 3))) << 4) + (cb & 7) * 2;
+  *reinterpret_cast<uint2*>(a1 + o) = wh;
+  *reinterpret_cast<uint2*>(a1 + A1PL + o) = wl;
+}
+
+// two conv1 tiles of the staged image xh (lo plane XPL behind) at once: all 24
+// A-fragment reads up front, two accumulation chains interleaved
+__device__ __forceinline__ void conv1_pair(const char* xh, char* a1, int ta, int tb, const bf16x8 (&w1hf)[3],
+                                           const bf16x8 (&w1lf)[3], float bias, int lane) {
+  const int h = lane >> 5, r32 = lane & 31;
+  const int c1_lane = ((r32 >> 3) * XW + (r32 & 7) + 2 * h) * 8;
+  const int oa = c1_lane + ((4 * (ta >> 2)) * XW + 8 * (ta & 3)) * 8;
+  const int ob = c1_lane + ((4 * (tb >> 2)) * XW + 8 * (tb & 3)) * 8;
+  auto frag = [&](const char* p) {
+    const uint2 a = *reinterpret_cast<const uint2*>(p);
+    const uint2 b = *reinterpret_cast<const uint2*>(p + 8);
+    return __builtin_bit_cast(bf16x8, make_uint4(a.x, a.y, b.x, b.y));
+  };
+  bf16x8 fah[3], fal[3], fbh[3], fbl[3];
+#pragma unroll
+  for (int s = 0; s < 3; ++s) {
+    fah[s] = frag(xh + oa + s * XW * 8);
+    fbh[s] = frag(xh + ob + s * XW * 8);
+    fal[s] = frag(xh + XPL + oa + s * XW * 8);
+    fbl[s] = frag(xh + XPL + ob + s * XW * 8);
+  }
+  f32x16 acca = {}, accb = {};
+#pragma unroll
+  for (int s = 0; s < 3; ++s) {
+    acca = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fah[s], w1hf[s], acca, 0, 0, 0);
+    accb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fbh[s], w1hf[s], accb, 0, 0, 0);
+    acca = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fah[s], w1lf[s], acca, 0, 0, 0);
+    accb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fbh[s], w1lf[s], accb, 0, 0, 0);
+    acca = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fal[s], w1hf[s], acca, 0, 0, 0);
+    accb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fbl[s], w1hf[s], accb, 0, 0, 0);
+  }
+  conv1_store(a1, ta, acca, bias, lane);
+  conv1_store(a1, tb, accb, bias, lane);
+}
+
+// bias + ReLU + 2x2 max-pool of conv2 tile (ty2, i) and channel oc2 -> row `out` of
+// the (B,4096) boundary: 8-B stores of two pooled columns
+template <bool SPLIT_OUT>
+__device__ __forceinline__ void conv2_store(float* out, int oc2, int ty2, int i, const f32x16& acc, float bias, int h) {
+#pragma unroll
+  for (int qy = 0; qy < 2; ++qy) {
+    float2 pv;
+    const int g0 = (2 * qy) * 4;
+    pv.x = fmaxf(fmax_nan(fmax_nan(acc[g0], acc[g0 + 1]), fmax_nan(acc[g0 + 4], acc[g0 + 5])) + bias, 0.f);
+    pv.y = fmaxf(fmax_nan(fmax_nan(acc[g0 + 2], acc[g0 + 3]), fmax_nan(acc[g0 + 6], acc[g0 + 7])) + bias, 0.f);
+    const int PY = 2 * ty2 + qy, PX = 4 * i + 2 * h;
+    if constexpr (SPLIT_OUT) {
+      uint32_t hi, lo;
+      split2(pv.x, pv.y, hi, lo);
+      char* bp = reinterpret_cast<char*>(out) + (oc2 * 2 + (PY >> 2)) * 128 + ((PY & 3) * 8 + PX) * 2;
+      *reinterpret_cast<uint32_t*>(bp) = hi;
+      *reinterpret_cast<uint32_t*>(bp + 64) = lo;
+    } else {
+      *reinterpret_cast<float2*>(out + oc2 * 64 + PY * 8 + PX) = pv;
+    }
+  }
 }
 
 template <int N>
@@ -168,79 +270,6 @@ __global__ __launch_bounds__(512, 1) void cifar_stage0_x3_kernel(
         *reinterpret_cast<uint2*>(xl + o) = vl;
       }
     };
-    const int c1_lane = ((r32 >> 3) * XW + (r32 & 7) + 2 * h) * 8;
-    const int q = ((r32 & 1) ? 2 : 0) + ((r32 & 2) ? 1 : 0);
-    const int cb = r32 & ~3;
-
-    // bias + ReLU + 2x2 max-pool in registers (max(a)+b == max(a+b) exactly), quad-DPP
-    // gather of 4 channels of one pooled pixel per lane, hi/lo split, one 8-B store per plane
-    auto conv1_epi = [&](int t, const f32x16& acc, int k) {
-      const int ty = t >> 2, tx = t & 3;
-      float v[4];
-#pragma unroll
-      for (int qy = 0; qy < 2; ++qy)
-#pragma unroll
-        for (int qx = 0; qx < 2; ++qx) {
-          const int g0 = (2 * qy) * 4 + 2 * qx;
-          v[qy * 2 + qx] = fmaxf(fmax_nan(fmax_nan(acc[g0], acc[g0 + 1]), fmax_nan(acc[g0 + 4], acc[g0 + 5])) + bias, 0.f);
-        }
-      const bool odd = r32 & 1;
-      const int s0 = __float_as_int(odd ? v[0] : v[2]), s1 = __float_as_int(odd ? v[1] : v[3]);
-      const float r0 = __int_as_float(dpp_xor1(s0)), r1 = __int_as_float(dpp_xor1(s1));
-      uint32_t u0h, u0l, u1h, u1l;
-      if (!odd) {
-        split2(v[0], r0, u0h, u0l);
-        split2(v[1], r1, u1h, u1l);
-      } else {
-        split2(r0, v[2], u0h, u0l);
-        split2(r1, v[3], u1h, u1l);
-      }
-      const bool hi2 = r32 & 2;
-      const uint32_t rch = (uint32_t)dpp_xor2((int)(hi2 ? u0h : u1h));
-      const uint32_t rcl = (uint32_t)dpp_xor2((int)(hi2 ? u0l : u1l));
-      const uint32_t mh = hi2 ? u1h : u0h, ml = hi2 ? u1l : u0l;
-      uint2 wh, wl;
-      wh.x = hi2 ? rch : mh;
-      wh.y = hi2 ? mh : rch;
-      wl.x = hi2 ? rcl : ml;
-      wl.y = hi2 ? ml : rcl;
-      const int Y = 2 * ty + (q >> 1) + 1, X = 4 * tx + 2 * h + (q & 1) + 1;
-      const int o = (Y * 18 + X) * 64 + ((((cb >> 3) ^ (Y & 3))) << 4) + (cb & 7) * 2;
-      *reinterpret_cast<uint2*>(smem + a1_off(k, 0) + o) = wh;
-      *reinterpret_cast<uint2*>(smem + a1_off(k, 1) + o) = wl;
-    };
-    auto frag = [&](const char* p) {
-      const uint2 a = *reinterpret_cast<const uint2*>(p);
-      const uint2 b = *reinterpret_cast<const uint2*>(p + 8);
-      return __builtin_bit_cast(bf16x8, make_uint4(a.x, a.y, b.x, b.y));
-    };
-    // two conv1 tiles at once: all 24 A-fragment reads up front, two accumulation chains interleaved
-    auto conv1_pair = [&](int ta, int tb, int k) {
-      const char* xh = smem + xin_off(k, 0);
-      const int oa = c1_lane + ((4 * (ta >> 2)) * XW + 8 * (ta & 3)) * 8;
-      const int ob = c1_lane + ((4 * (tb >> 2)) * XW + 8 * (tb & 3)) * 8;
-      bf16x8 fah[3], fal[3], fbh[3], fbl[3];
-#pragma unroll
-      for (int s = 0; s < 3; ++s) {
-        fah[s] = frag(xh + oa + s * XW * 8);
-        fbh[s] = frag(xh + ob + s * XW * 8);
-        fal[s] = frag(xh + XPL + oa + s * XW * 8);
-        fbl[s] = frag(xh + XPL + ob + s * XW * 8);
-      }
-      f32x16 acca = {}, accb = {};
-#pragma unroll
-      for (int s = 0; s < 3; ++s) {
-        acca = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fah[s], w1hf[s], acca, 0, 0, 0);
-        accb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fbh[s], w1hf[s], accb, 0, 0, 0);
-        acca = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fah[s], w1lf[s], acca, 0, 0, 0);
-        accb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fbh[s], w1lf[s], accb, 0, 0, 0);
-        acca = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fal[s], w1hf[s], acca, 0, 0, 0);
-        accb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fbl[s], w1hf[s], accb, 0, 0, 0);
-      }
-      conv1_epi(ta, acca, k);
-      conv1_epi(tb, accb, k);
-    };
-
     if (n > 0) {
       load_img(0);
       stage_img(0);
@@ -250,7 +279,8 @@ __global__ __launch_bounds__(512, 1) void cifar_stage0_x3_kernel(
     for (int it = 0; it <= n; ++it) {
       if (it < n) {
 #pragma unroll 1
-        for (int t = rw; t < 32; t += 8) conv1_pair(t, t + 4, it);
+        for (int t = rw; t < 32; t += 8)
+          conv1_pair(smem + xin_off(it, 0), smem + a1_off(it, 0), t, t + 4, w1hf, w1lf, bias, lane);
         if (it + 1 < n) {
           stage_img(it + 1);
           if (it + 2 < n) load_img(it + 2);
@@ -330,26 +360,7 @@ __global__ __launch_bounds__(512, 1) void cifar_stage0_x3_kernel(
           }
         } else {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-#pragma unroll
-          for (int qy = 0; qy < 2; ++qy) {
-            float2 pv;
-            const int g0 = (2 * qy) * 4;
-            pv.x = fmaxf(fmax_nan(fmax_nan(acc[i][g0], acc[i][g0 + 1]), fmax_nan(acc[i][g0 + 4], acc[i][g0 + 5])) + bias, 0.f);
-            pv.y = fmaxf(fmax_nan(fmax_nan(acc[i][g0 + 2], acc[i][g0 + 3]), fmax_nan(acc[i][g0 + 6], acc[i][g0 + 7])) + bias,
-                         0.f);
-            const int PY = 2 * ty2 + qy, PX = 4 * i + 2 * h;
-            if constexpr (SPLIT_OUT) {
-              uint32_t hi, lo;
-              split2(pv.x, pv.y, hi, lo);
-              char* bp = reinterpret_cast<char*>(ob - oc2 * 64) + (oc2 * 2 + (PY >> 2)) * 128 + ((PY & 3) * 8 + PX) * 2;
-              *reinterpret_cast<uint32_t*>(bp) = hi;
-              *reinterpret_cast<uint32_t*>(bp + 64) = lo;
-            } else {
-              *reinterpret_cast<float2*>(ob + PY * 8 + PX) = pv;
-            }
-          }
-        }
+          for (int i = 0; i < 2; ++i) conv2_store<SPLIT_OUT>(ob - oc2 * 64, oc2, ty2, i, acc[i], bias, h);
         }
       }
     };
@@ -359,6 +370,87 @@ __global__ __launch_bounds__(512, 1) void cifar_stage0_x3_kernel(
       if (it >= 1) conv2_img(it - 1);
       __syncthreads();
     }
+  }
+}
+
+// Stage 0 of a few images: one workgroup per image and band of 4 conv2 rows
+// (ty2), so that 4 B workgroups share what one of the persistent kernel does in a
+// row: conv1 of the 3 or 4 tile rows that the band's pooled map touches (waves
+// 0-3, two pairs of tiles each; 1.5x the work of one image over the 4 bands), then
+// conv2 of the band, one 32x32 tile a wave (waves 4-7, their weights loaded while
+// conv1 runs).  Tiles, products and their order are those of the persistent kernel:
+// the results are the same bits.  Bound by its chain (load, stage, conv1, barrier,
+// 54 dependent MFMAs, store): 7.3 us where the persistent kernel takes 11.0 for one
+// image.  Taken while the bands of all images run at once (4 B <= grid): with 256
+// VGPRs a CU holds one workgroup, so beyond that the bands would queue.
+template <bool SPLIT_OUT>
+__global__ __launch_bounds__(512, 1) void cifar_stage0_x3_band_kernel(
+    const float* __restrict__ x, float* __restrict__ out, const bf16_t* __restrict__ w1h,
+    const bf16_t* __restrict__ w1l, const float* __restrict__ b1, const bf16_t* __restrict__ w2h,
+    const bf16_t* __restrict__ w2l, const float* __restrict__ b2) {
+  constexpr int A1 = 2 * XPL;  // xin hi | lo, pooled map hi | lo
+  __shared__ __attribute__((aligned(16))) char smem[A1 + 2 * A1PL];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rw = wave & 3, h = lane >> 5, r32 = lane & 31;
+  const int ty2 = blockIdx.x & 3;
+  const size_t img = blockIdx.x >> 2;
+
+  float px[2][3];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) px[i][c] = x[img * 3072 + c * 1024 + tid + 512 * i];
+  for (int i = tid; i < (A1 + 2 * A1PL) / 16; i += 512) reinterpret_cast<uint4*>(smem)[i] = make_uint4(0, 0, 0, 0);
+  __syncthreads();  // halos are zero before the interior is written
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int p = tid + 512 * i, o = (((p >> 5) + 1) * XW + (p & 31) + 1) * 8;
+    uint2 vh, vl;
+    split2(px[i][0], px[i][1], vh.x, vl.x);
+    split2(px[i][2], 0.f, vh.y, vl.y);
+    *reinterpret_cast<uint2*>(smem + o) = vh;
+    *reinterpret_cast<uint2*>(smem + XPL + o) = vl;
+  }
+  if (wave < 4) {
+    bf16x8 w1hf[3], w1lf[3];
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      w1hf[s] = *reinterpret_cast<const bf16x8*>(w1h + r32 * 48 + s * 16 + h * 8);
+      w1lf[s] = *reinterpret_cast<const bf16x8*>(w1l + r32 * 48 + s * 16 + h * 8);
+    }
+    const float bias = b1[r32];
+    __syncthreads();
+    const int ty = 2 * ty2 - 1 + rw;  // conv1 tile row: pooled rows 2 ty, 2 ty + 1
+    if (ty >= 0 && ty < 8) {
+      conv1_pair(smem, smem + A1, 4 * ty, 4 * ty + 1, w1hf, w1lf, bias, lane);
+      conv1_pair(smem, smem + A1, 4 * ty + 2, 4 * ty + 3, w1hf, w1lf, bias, lane);
+    }
+    __syncthreads();
+  } else {
+    const int oc2 = (rw & 1) * 32 + r32, i = rw >> 1;
+    bf16x8 w2hf[18], w2lf[18];
+#pragma unroll
+    for (int s = 0; s < 18; ++s) {
+      w2hf[s] = *reinterpret_cast<const bf16x8*>(w2h + oc2 * 288 + s * 16 + h * 8);
+      w2lf[s] = *reinterpret_cast<const bf16x8*>(w2l + oc2 * 288 + s * 16 + h * 8);
+    }
+    const float bias = b2[oc2];
+    resident_fence(w2hf);
+    resident_fence(w2lf);
+    __syncthreads();
+    __syncthreads();
+    f32x16 acc = {};
+#pragma unroll
+    for (int s = 0; s < 18; ++s) {
+      const int ky = (s >> 1) / 3, kx = (s >> 1) % 3, yr = (r32 >> 3) + ky;
+      const char* p = smem + A1 + ((4 * ty2 + yr) * 18 + 8 * i + (r32 & 7) + kx) * 64 + (((2 * (s & 1) + h) ^ (yr & 3)) << 4);
+      const bf16x8 hi = *reinterpret_cast<const bf16x8*>(p), lo = *reinterpret_cast<const bf16x8*>(p + A1PL);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, w2hf[s], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, w2lf[s], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, w2hf[s], acc, 0, 0, 0);
+    }
+    conv2_store<SPLIT_OUT>(out + img * 4096, oc2, ty2, i, acc, bias, h);
   }
 }
 
@@ -691,6 +783,160 @@ __global__ __launch_bounds__(256) void cifar_head_tail_x3_kernel(const float* __
   }
 }
 
+// ---------------------------------------------------------------------------
+// The head of a few images: fc1 as HS_S slices of K over HS_S x 32 workgroups, each
+// reading its 16 columns x 512 k of W_hi and W_lo once for all rows, and a finish
+// that sums the slices in order and, one workgroup a row, goes on to fc2, softmax
+// and argmax.
+//
+// One row costs 8 MB of weights and nothing else: the GEMM over K' = 3 K that larger
+// batches take reads 12.6 MB on 32 workgroups.  A wave holds its 64 k of the weights
+// in registers and takes the rows 16 at a time (products and split of the fp32 rows
+// as in the other fc1 paths); the 8 waves meet in LDS and the slice's sums leave as
+// part[slice][row][512].  Slice = block & 7: the workgroups of one XCD share one
+// slice of the rows in its L2.  One row: 3.8 + 3.4 us for the two launches; split,
+// GEMM and tail took 3.2 + 16.8 + 9.8 us.
+constexpr int HS_S = 8, HS_N = 512, HS_K = 4096;
+
+template <bool BLOCKED>
+__global__ __launch_bounds__(512) void cifar_fc1_few_kernel(const float* __restrict__ A, const bf16_t* __restrict__ Wh,
+                                                            const bf16_t* __restrict__ Wl, float* __restrict__ part,
+                                                            int M) {
+  __shared__ __attribute__((aligned(16))) float red[2][8][32 * 16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r16 = lane & 15, kq = (lane >> 4) * 8;
+  const int slice = blockIdx.x & (HS_S - 1), n0 = (blockIdx.x / HS_S) * 16;
+  const int k0 = slice * (HS_K / HS_S) + wave * 64;
+  const size_t wo = (size_t)(n0 + r16) * HS_K + k0 + kq;
+  bf16x8 wh[2], wl[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    wh[s] = *reinterpret_cast<const bf16x8*>(Wh + wo + s * 32);
+    wl[s] = *reinterpret_cast<const bf16x8*>(Wl + wo + s * 32);
+  }
+  uint4 a[2][2][2];  // 16-row tile, k32 step, 32 B of the lane's row (fp32 k 0-3, 4-7 or hi, lo)
+  auto load = [&](int m0) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int m = min(m0 + i * 16 + r16, M - 1);
+      const char* p = reinterpret_cast<const char*>(A + (size_t)m * HS_K + k0);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        a[i][s][0] = *reinterpret_cast<const uint4*>(p + s * 128 + (BLOCKED ? kq * 2 : kq * 4));
+        a[i][s][1] = *reinterpret_cast<const uint4*>(p + s * 128 + (BLOCKED ? kq * 2 + 64 : kq * 4 + 16));
+      }
+    }
+  };
+  load(0);
+  int buf = 0;
+  for (int m0 = 0; m0 < M; m0 += 32, buf ^= 1) {
+    f32x4 acc[2] = {f32x4{}, f32x4{}};
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        uint4 hi = a[i][s][0], lo = a[i][s][1];
+        if constexpr (!BLOCKED) {
+          const float4 u = __builtin_bit_cast(float4, a[i][s][0]), v = __builtin_bit_cast(float4, a[i][s][1]);
+          split2(u.x, u.y, hi.x, lo.x);
+          split2(u.z, u.w, hi.y, lo.y);
+          split2(v.x, v.y, hi.z, lo.z);
+          split2(v.z, v.w, hi.w, lo.w);
+        }
+        const bf16x8 ah = __builtin_bit_cast(bf16x8, hi), al = __builtin_bit_cast(bf16x8, lo);
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wh[s], ah, acc[i], 0, 0, 0);
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wl[s], ah, acc[i], 0, 0, 0);
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wh[s], al, acc[i], 0, 0, 0);
+      }
+    if (m0 + 32 < M) load(m0 + 32);
+    // acc[i][r] = (row i * 16 + (lane & 15), column n0 + (lane >> 4) * 4 + r)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      *reinterpret_cast<f32x4*>(&red[buf][wave][(i * 16 + r16) * 16 + (lane >> 4) * 4]) = acc[i];
+    __syncthreads();
+    float v = red[buf][0][tid];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) v += red[buf][w][tid];
+    const int m = m0 + (tid >> 4);
+    if (m < M) part[((size_t)slice * M + m) * HS_N + n0 + (tid & 15)] = v;
+  }
+}
+
+// Row blockIdx.x: hid = relu(sum of the slices + b1) (stored where hid is given),
+// then, with TAIL, logits = hid . W2^T + b2 (fp32 products with W2 = hi + lo, exact in
+// fp32), softmax and the smallest class that attains the maximum.
+template <bool TAIL>
+__global__ __launch_bounds__(256) void cifar_head_few_kernel(const float* __restrict__ part,
+                                                             const float* __restrict__ b1, float* __restrict__ hid,
+                                                             const bf16_t* __restrict__ w2h,
+                                                             const bf16_t* __restrict__ w2l,
+                                                             const float* __restrict__ b2, float* __restrict__ probs,
+                                                             int* __restrict__ pred, int M) {
+  __shared__ __attribute__((aligned(16))) float hs[16 * 36];  // 32 k per slice of 36: 16-B reads of 4 slices, 4 banks apart
+  __shared__ float zs[4][16];
+  const int tid = threadIdx.x, m = blockIdx.x;
+  const int cls = tid & 15, ks = tid >> 4;
+  uint4 wh[4], wl[4];
+  if constexpr (TAIL) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      wh[j] = *reinterpret_cast<const uint4*>(w2h + cls * HS_N + ks * 32 + j * 8);
+      wl[j] = *reinterpret_cast<const uint4*>(w2l + cls * HS_N + ks * 32 + j * 8);
+    }
+  }
+  float2 p[HS_S];
+#pragma unroll
+  for (int s = 0; s < HS_S; ++s)
+    p[s] = *reinterpret_cast<const float2*>(part + ((size_t)s * M + m) * HS_N + 2 * tid);
+  const float2 bb = *reinterpret_cast<const float2*>(b1 + 2 * tid);
+  float2 v = p[0];
+#pragma unroll
+  for (int s = 1; s < HS_S; ++s) {
+    v.x += p[s].x;
+    v.y += p[s].y;
+  }
+  v.x = fmaxf(v.x + bb.x, 0.f);
+  v.y = fmaxf(v.y + bb.y, 0.f);
+  if (hid != nullptr) *reinterpret_cast<float2*>(hid + (size_t)m * HS_N + 2 * tid) = v;
+  if constexpr (TAIL) {
+    *reinterpret_cast<float2*>(hs + (tid >> 4) * 36 + (2 * tid & 31)) = v;
+    __syncthreads();
+    float z = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float4 u = *reinterpret_cast<const float4*>(hs + ks * 36 + j * 8);
+      const float4 t = *reinterpret_cast<const float4*>(hs + ks * 36 + j * 8 + 4);
+      const float hv[8] = {u.x, u.y, u.z, u.w, t.x, t.y, t.z, t.w};
+      const uint32_t ph[4] = {wh[j].x, wh[j].y, wh[j].z, wh[j].w}, pl[4] = {wl[j].x, wl[j].y, wl[j].z, wl[j].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        z = fmaf(hv[2 * e], __uint_as_float(ph[e] << 16) + __uint_as_float(pl[e] << 16), z);
+        z = fmaf(hv[2 * e + 1], __uint_as_float(ph[e] & 0xffff0000u) + __uint_as_float(pl[e] & 0xffff0000u), z);
+      }
+    }
+    z += __shfl_xor(z, 16, 64);
+    z += __shfl_xor(z, 32, 64);
+    if ((tid & 63) < 16) zs[tid >> 6][cls] = z;
+    __syncthreads();
+    if (tid < 16) {
+      z = tid < 10 ? zs[0][tid] + zs[1][tid] + zs[2][tid] + zs[3][tid] + b2[tid] : -INFINITY;
+      float mx = z;
+#pragma unroll
+      for (int o = 1; o < 16; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+      const float e = tid < 10 ? expf(z - mx) : 0.f;
+      float sum = e;
+      int cand = (z == mx) ? tid : 16;
+#pragma unroll
+      for (int o = 1; o < 16; o <<= 1) {
+        sum += __shfl_xor(sum, o, 64);
+        cand = min(cand, __shfl_xor(cand, o, 64));
+      }
+      if (tid < 10) probs[(size_t)m * 10 + tid] = e / sum;
+      if (tid == 0) pred[m] = cand;
+    }
+  }
+}
+
 }  // namespace dnn
 
 using namespace dnn;
@@ -721,6 +967,15 @@ extern "C" int dnn_cifar_stage0_x3(const float* x, float* out, const void* w1h, 
                                    hipStream_t st, int split_out) {
   if (B <= 0) return 0;
   if (grid <= 0) grid = 256;
+  if (4L * B <= grid) {
+    if (split_out)
+      hipLaunchKernelGGL(cifar_stage0_x3_band_kernel<true>, dim3(4 * B), dim3(512), 0, st, x, out, (const bf16_t*)w1h,
+                         (const bf16_t*)w1l, b1, (const bf16_t*)w2h, (const bf16_t*)w2l, b2);
+    else
+      hipLaunchKernelGGL(cifar_stage0_x3_band_kernel<false>, dim3(4 * B), dim3(512), 0, st, x, out, (const bf16_t*)w1h,
+                         (const bf16_t*)w1l, b1, (const bf16_t*)w2h, (const bf16_t*)w2l, b2);
+    return (int)hipGetLastError();
+  }
   if (grid > B) grid = B;
   return split_out ? launch_stage0_x3<true>(x, out, w1h, w1l, b1, w2h, w2l, b2, B, grid, st)
                    : launch_stage0_x3<false>(x, out, w1h, w1l, b1, w2h, w2l, b2, B, grid, st);
@@ -768,5 +1023,27 @@ extern "C" int dnn_cifar_head_tail_x3(const float* hid, const void* w2h, const v
   if (blocks > 1024) blocks = 1024;
   hipLaunchKernelGGL(cifar_head_tail_x3_kernel, dim3(blocks), dim3(256), 0, st, hid, (const bf16_t*)w2h,
                      (const bf16_t*)w2l, b2, probs, pred, B);
+  return (int)hipGetLastError();
+}
+
+// fc1 of a few rows into hid (M,512) and, where probs is given, fc2 + softmax + argmax
+// (hid may then be null).  part: HS_S x M x 512 floats of scratch.
+extern "C" int dnn_cifar_head_few(const float* A, int blocked, const void* Wh, const void* Wl, const float* b1,
+                                  float* part, float* hid, const void* w2h, const void* w2l, const float* b2,
+                                  float* probs, int* pred, int M, hipStream_t st) {
+  if (M <= 0) return 0;
+  if (probs == nullptr && hid == nullptr) return -1;
+  if (blocked)
+    hipLaunchKernelGGL(cifar_fc1_few_kernel<true>, dim3(HS_S * HS_N / 16), dim3(512), 0, st, A, (const bf16_t*)Wh,
+                       (const bf16_t*)Wl, part, M);
+  else
+    hipLaunchKernelGGL(cifar_fc1_few_kernel<false>, dim3(HS_S * HS_N / 16), dim3(512), 0, st, A, (const bf16_t*)Wh,
+                       (const bf16_t*)Wl, part, M);
+  if (probs != nullptr)
+    hipLaunchKernelGGL(cifar_head_few_kernel<true>, dim3(M), dim3(256), 0, st, part, b1, hid, (const bf16_t*)w2h,
+                       (const bf16_t*)w2l, b2, probs, pred, M);
+  else
+    hipLaunchKernelGGL(cifar_head_few_kernel<false>, dim3(M), dim3(256), 0, st, part, b1, hid, (const bf16_t*)w2h,
+                       (const bf16_t*)w2l, b2, probs, pred, M);
   return (int)hipGetLastError();
 }

@@ -148,6 +148,10 @@ STAGE0_GRID = 0  # persistent stage-0 workgroups; 0 = one per CU (256)
 # fused fp32 fc1 from this batch on: 2 x B/256 tiles of 128 k32 steps each need
 # >= 128 tiles to occupy the chip; below, split3 + the K-concat GEMM is faster
 FC1_X3_MIN_ROWS = 16384
+# fp32 head up to this batch: fc1 in slices of K and a finish of one workgroup a row
+# (pipeline pass, us, with and without: 1 row 27.7 / 44.3, 64 29.7 / 57.4, 256 50.6 /
+# 84.9, 512 79.1 / 88.3, 768 104.4 / 96.2: each 32 rows are a round of every workgroup)
+FC1_FEW_ROWS = 512
 
 
 def set_stage0_grid(grid: int = 0) -> None:
@@ -211,6 +215,28 @@ def stage0_forward(x: torch.Tensor, w: CifarStage0Weights, out: Optional[torch.T
     return out
 
 
+def _head_few(h: torch.Tensor, w: CifarHeadWeights, hid: Optional[torch.Tensor], probs: Optional[torch.Tensor],
+              pred: Optional[torch.Tensor], scratch: Optional[torch.Tensor], split: int) -> None:
+    B = h.shape[0]
+    part = _fc1_scratch(scratch, B, h.device)  # 8 x B x 512 floats of the 12288 bf16 a row
+    check(lib().cifar_head_few(ptr(h), split, ptr(w.w_fc1h), ptr(w.w_fc1l), ptr(w.b_fc1), ptr(part), ptr(hid),
+                               ptr(w.w_fc2h), ptr(w.w_fc2l), ptr(w.b_fc2), ptr(probs), ptr(pred), B, stream_ptr()),
+          "cifar_head_few")
+
+
+def _fc1_scratch(scratch: Optional[torch.Tensor], B: int, device) -> torch.Tensor:
+    if scratch is None or scratch.shape[0] < B or tuple(scratch.shape[1:]) != (3 * 4096,):
+        scratch = torch.empty((B, 3 * 4096), dtype=torch.bfloat16, device=device)
+    return scratch
+
+
+def _few_rows(h: torch.Tensor, w: CifarHeadWeights, hid: Optional[torch.Tensor]) -> bool:
+    """One row a workgroup of the finish; a strided or typed ``hid`` is the GEMM's."""
+    B = h.shape[0]
+    return w.precision == "fp32" and 0 < B <= FC1_FEW_ROWS and (
+        hid is None or (tuple(hid.shape) == (B, 512) and hid.dtype == torch.float32 and hid.is_contiguous()))
+
+
 def fc1_forward(h: torch.Tensor, w: CifarHeadWeights, out: Optional[torch.Tensor] = None,
                 scratch: Optional[torch.Tensor] = None, boundary: str = "fp32") -> torch.Tensor:
     """Unit 2: (B,4096) -> relu(fc1) (B,512) on the MFMA GEMM (fp32: split operand,
@@ -228,9 +254,11 @@ def fc1_forward(h: torch.Tensor, w: CifarHeadWeights, out: Optional[torch.Tensor
         check(lib().cifar_fc1_x3(ptr(h), 4096, ptr(w.w_fc1h), ptr(w.w_fc1l), 4096, ptr(w.b_fc1), ptr(out), 512,
                                  B, 512, 4096, stream_ptr(), split), "cifar_fc1_x3")
         return out
-    if scratch is None or scratch.shape[0] < B or tuple(scratch.shape[1:]) != (3 * 4096,):
-        scratch = torch.empty((B, 3 * 4096), dtype=torch.bfloat16, device=h.device)
-    a3 = scratch[:B]
+    if _few_rows(h, w, out):
+        out = torch.empty((B, 512), dtype=torch.float32, device=h.device) if out is None else out
+        _head_few(h, w, out, None, None, scratch, split)
+        return out
+    a3 = _fc1_scratch(scratch, B, h.device)[:B]
     check(lib().cifar_split3(ptr(h), 4096, ptr(a3), 3 * 4096, B, 4096, stream_ptr(), split), "cifar_split3")
     if out is None:
         out = torch.empty((B, 512), dtype=torch.float32, device=h.device)
@@ -255,7 +283,15 @@ def head_tail(hid: torch.Tensor, w: CifarHeadWeights, probs: Optional[torch.Tens
 
 def head_forward(h: torch.Tensor, w: CifarHeadWeights, hid: Optional[torch.Tensor] = None,
                  probs: Optional[torch.Tensor] = None, pred: Optional[torch.Tensor] = None,
-                 boundary: str = "fp32") -> Tuple[torch.Tensor, torch.Tensor]:
-    """Units 2-3: h (B,4096) -> (probs (B,10) fp32, pred (B,) int32)."""
-    hid = fc1_forward(h, w, out=hid, boundary=boundary)
+                 boundary: str = "fp32", scratch: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Units 2-3: h (B,4096) -> (probs (B,10) fp32, pred (B,) int32); ``hid`` (if given) holds
+    relu(fc1) afterwards, ``scratch`` as in ``fc1_forward``."""
+    if _few_rows(h, w, hid):
+        split = _split_boundary(boundary, w.precision)
+        _check_act(h, (4096,), torch.float32, "fc1 input")
+        probs = probs if probs is not None else torch.empty((h.shape[0], 10), dtype=torch.float32, device=h.device)
+        pred = pred if pred is not None else torch.empty((h.shape[0],), dtype=torch.int32, device=h.device)
+        _head_few(h, w, hid, probs, pred, scratch, split)
+        return probs, pred
+    hid = fc1_forward(h, w, out=hid, scratch=scratch, boundary=boundary)
     return head_tail(hid, w, probs, pred)

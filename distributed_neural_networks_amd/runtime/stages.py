@@ -130,12 +130,14 @@ class CifarHipStage(StageCompute):
                 return h
         elif h.dtype != self.adt:
             h = h.to(self.adt)
-        if self.start <= 2 <= self.end:
-            h = self._cops.fc1_forward(h.contiguous(), self.wh, out if self.end == 2 else buf["hid"],
-                                       scratch=buf.get("split"), boundary=self.boundary)
-            if self.end == 2:
-                return h
-        probs, pred = self._cops.head_tail(h.contiguous(), self.wh, out, buf["pred"])
+        if self.end == 2:
+            return self._cops.fc1_forward(h.contiguous(), self.wh, out, scratch=buf.get("split"),
+                                          boundary=self.boundary)
+        if self.start <= 2:
+            probs, pred = self._cops.head_forward(h.contiguous(), self.wh, buf["hid"], out, buf["pred"],
+                                                  boundary=self.boundary, scratch=buf.get("split"))
+        else:
+            probs, pred = self._cops.head_tail(h.contiguous(), self.wh, out, buf["pred"])
         return StageOutput(probs, pred)
 
 

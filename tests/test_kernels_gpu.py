@@ -366,6 +366,39 @@ def test_cifar_fc1_x3_kernel(M, N, K, split_in):
 
 
 @pytest.mark.parametrize("boundary", ["fp32", "split"])
+@pytest.mark.parametrize("B", [1, 2, 15, 16, 17, 32, 33, 64, 65, 500, 512])
+def test_cifar_few_images(B, boundary):
+    """Bands of one image against whole images a workgroup (the same bits) and the
+    head in slices of K against fp64: a product of the 3-term split is off by at
+    most 2^-16 of itself, and 4096 + 512 fp32 sums stay below 2^-17 of the sum of
+    magnitudes."""
+    from distributed_neural_networks_amd.ops import cifar as cops
+    assert B <= cops.FC1_FEW_ROWS
+    sd, x, _, _ = _cifar_golden(B, B)
+    w0, wh = cops.pack_stage0(sd, DEV), cops.pack_head(sd, DEV)
+    x = x.to(DEV)
+    h = cops.stage0_forward(x, w0, boundary=boundary)
+    whole = cops.stage0_forward(x, w0, grid=B, boundary=boundary)  # B workgroups: no bands
+    assert torch.equal(h, whole)
+    hid = torch.full((B, 512), float("nan"), device=DEV)
+    probs, pred = cops.head_forward(h, wh, hid=hid, boundary=boundary)
+    alone = cops.fc1_forward(h, wh, boundary=boundary)
+    assert torch.equal(hid, alone)
+    p2, k2 = cops.head_forward(h, wh, boundary=boundary)
+    assert torch.equal(probs, p2) and torch.equal(pred, k2)
+    hv = cops.decode_boundary(h) if boundary == "split" else h
+    W, b = sd["fc1.weight"].to(DEV).double(), sd["fc1.bias"].to(DEV).double()
+    ref = torch.relu(hv.double() @ W.t() + b)
+    bound = (hv.double().abs() @ W.abs().t() + b.abs()) * 3 * 2.0 ** -17
+    assert bool(((hid.double() - ref).abs() <= bound).all())
+    W2, b2 = sd["fc2.weight"].to(DEV).double(), sd["fc2.bias"].to(DEV).double()
+    z = hid.double() @ W2.t() + b2
+    err = (hid.double() @ W2.abs().t() + b2.abs()).max() * 2.0 ** -16
+    assert (probs.double() - z.softmax(1)).abs().max() <= err + 2.0 ** -20
+    assert torch.equal(pred.long(), probs.argmax(1))
+
+
+@pytest.mark.parametrize("boundary", ["fp32", "split"])
 def test_cifar_fp32_pipeline_large_batch_fused_fc1(boundary):
     """The large-batch fp32 head (fused fc1) on 20000 images: max |dprob| <= 1e-5
     vs the fp32 torch model and argmax agreement on every decidable row."""

@@ -96,6 +96,13 @@ def test_token_gate(dtype, M, n, np_, K):
     assert (out[:, n:np_] == 0).all() and (out[:, np_:] == 1).all()
 
 
+@pytest.mark.parametrize("M", [64, 65, 500, 2049, 4100])
+@pytest.mark.parametrize("n,np_", [(60, 64), (300, 320)])
+def test_token_gate_long_rows(M, n, np_):
+    """Rows of 4096: the few-row kernel beyond 256 rows and the 64x64 tiles, either side of the rule."""
+    test_token_gate("bf16", M, n, np_, 4096)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 6, 64), (33, 200, 128), (70, 331, 192), (129, 64, 1024)])
 def test_linear_f32(M, N, K):
     from distributed_neural_networks_amd.ops import decoder_ops as D_
