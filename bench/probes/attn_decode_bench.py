@@ -53,12 +53,11 @@ def main():
                "auto_splits": decode_splits(S, B, Hkv, G)}
         kv_bytes = 2 * B * Hkv * (pos + 1) * hd * 2
         ref = None
-        modes = {"": "0", "m": "1"}
-        for sp, mode in [(int(v), m) for v in args.splits.split(",") for m in modes]:
+        mode = ""
+        for sp in [int(v) for v in args.splits.split(",")]:
             sp = sp or res["auto_splits"]
             if sp < decode_splits(S, B, Hkv, G) and sp < res["auto_splits"]:
                 continue
-            os.environ["DNN_DECODE_MFMA"] = modes[mode]
             ws = torch.empty(B * Hkv * sp * G * (hd + 2), device=dev, dtype=torch.float32)
 
             def run():

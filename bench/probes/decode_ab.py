@@ -38,10 +38,6 @@ def apply(switch: str, v: int) -> None:
         gemm.set_stream_gemm(1, 0, v)
     elif switch == "stream":  # decode stream GEMM: 0 off, 1 where it measured faster, 2 forced (gemm_stream.h)
         gemm.set_stream_gemm(v)
-    elif switch == "decode_1p":  # one-pass decode attention: 0 batched kernel, 1 default, 2 forced (attention.hip)
-        os.environ["DNN_DECODE_1P"] = str(v)
-    elif switch == "decode_1p_kf":  # one-pass decode attention: K/V loads issued before q (attention.hip KF)
-        os.environ["DNN_DECODE_1P_KF"] = str(v)
     elif switch == "flash_db":  # flash prefill with double-buffered K/V LDS (attention.hip DNN_FLASH_DB)
         os.environ["DNN_FLASH_DB"] = str(v)
     elif switch == "epi_pre":  # decode GEMM epilogue operands issued with the first loads (gemm_oneshot.h / skinny)
@@ -58,8 +54,6 @@ def apply(switch: str, v: int) -> None:
         gemm.set_gemm_tile(v)
     elif switch == "half_cost":  # auto 256x128 rule: relative tile cost x 100
         gemm.set_gemm_half_cost(v / 100.0)
-    elif switch == "decode_1p_ns":  # one-pass decode attention: at least v key splits (attention.hip)
-        os.environ["DNN_DECODE_1P_NS"] = str(v)
     elif switch == "split_tail":  # prefill 256^2 + 256x128 tail split (gemm_bf16.hip): mask 1 bf16, 2 fp8
         gemm.set_gemm_split_tail(int(v))
     elif switch == "fused_head":  # decode head + argmax partials in one launch (gemm_head.h)

@@ -18,25 +18,10 @@
 // XOR-swizzled so the A-fragment ds_read_b128 reads are conflict-free.
 #include "common.h"
 
+#include <algorithm>
 #include <cstdlib>
 
 namespace dnn {
-
-// Phase timestamps of decode-attention block (0,0), thread 0: only in the
-// bench-only probe build (-DDNN_DEC_PROBE, bench/attn_probe.py).
-#ifdef DNN_DEC_PROBE
-__device__ unsigned long long dec_probe_ts[32];
-#define DEC_PROBE(i, dep)                                                             \
-  do {                                                                                \
-    asm volatile("" ::"v"(dep));                                                      \
-    if (threadIdx.x == 0 && (blockIdx.x | blockIdx.y) == 0) {                         \
-      dec_probe_ts[i] = __builtin_amdgcn_s_memrealtime();                             \
-      dec_probe_ts[16 + i] = __builtin_amdgcn_s_memtime();                             \
-    }                                                                                 \
-  } while (0)
-#else
-#define DEC_PROBE(i, dep) do { } while (0)
-#endif
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
@@ -473,11 +458,10 @@ __global__ __launch_bounds__(256, 2) void flash_attn_kernel(const bf16_t* __rest
 // Decode attention (one query token per sequence), split over the key axis.
 // grid = (B*Hkv, NS); each workgroup handles the G = H/Hkv query heads of one
 // kv head over keys [split*chunk, (split+1)*chunk) ∩ [0, lens[b]) and writes an
-// unnormalised partial (o, m, l) to ws; decode_combine merges the splits.
+// unnormalised partial (o, m, l) to ws; decode_combine merges the splits.  bf16
+// caches: attention_stream.h; e4m3 caches: attn_decode_kernel.
 // ---------------------------------------------------------------------------
 constexpr int DEC_MAXG = 8;
-constexpr int DEC_U = 8;  // key/value rows in flight per thread
-static_assert(DEC_U % 2 == 0, "P.V folds key pairs");
 
 // 8 consecutive head-dim elements [8*sub, 8*sub+8) of one head row, RoPE'd
 // (rotate-half: element i pairs with i +- hd/2) when ROPE, and
@@ -556,7 +540,7 @@ __device__ __forceinline__ void kv8_unpack(const i32x4& w, uint32_t (&p)[8]) {
 // halve; entries are converted to bf16 in registers (exact) before the same
 // v_dot2 math, and the new key/value row is rounded to e4m3 once — its score
 // uses the rounded copy, so the current step sees what later steps will read.
-template <int HD, int G, int FM, bool NT, bool MF = false, bool KV8 = false, int RU = 0>
+template <int HD, int G, int FM, bool NT, bool MF = false, int RU = 10>
 __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restrict__ q, int ldq,
                                                           bf16_t* __restrict__ kc, bf16_t* __restrict__ vc,
                                                           float* __restrict__ ws, int H, int Hkv, int S,
@@ -565,27 +549,21 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
                                                           int chunk_cap, bf16_t* __restrict__ o_direct) {
   constexpr bool FUSED = FM != 0;  // FM: 0 = q head-major + cached keys, 1 = fused QKV rows, 2 = fused + RoPE
   constexpr bool ROPE = FM == 2;
-  // rows in flight per thread (RU > 0 overrides): KV8 rows are half the bytes,
-  // so 10 rows keep the same bytes in flight and one batch covers 640 keys at
-  // hd 64 (the 512-567-token benchmark contexts take one K and one V round
-  // trip, not two).  bf16 MHA with 10 or 12 rows measured neutral (GPT-2 B=64
-  // 0.585 / 0.584 / 0.590 ms, profiles/archive/r2_decode_rows_in_flight_bf16_ab.jsonl):
-  // that path is bound by the K/V bytes, not by its round trips
-  constexpr int DEC_U = RU > 0 ? RU : (KV8 ? 10 : dnn::DEC_U);
+  // rows in flight per thread: one batch covers 640 keys at hd 64 (the 512-567-token
+  // benchmark contexts take one K and one V round trip, not two)
+  constexpr int DEC_U = RU;
   static_assert(DEC_U % 2 == 0, "P.V folds key pairs");
-  constexpr int ELT = KV8 ? 16 : 8;     // head dims per 16-B lane load
+  constexpr int ELT = 16;               // head dims per 16-B lane load
   constexpr int LPK = HD / ELT;         // lanes per key row (16 B each)
   constexpr int GPB = 256 / LPK;        // key groups per block
   extern __shared__ __attribute__((aligned(16))) float dsm[];   // [G][chunk_cap] scores, then reduction scratch
   const int bk = blockIdx.x, split = blockIdx.y, NS = gridDim.y;
-  DEC_PROBE(0, 0);
   const int b = bk / Hkv, kvh = bk % Hkv;
   const int p_new = FUSED ? lens[b] : 0;  // FUSED: lens = positions already cached
   const int len = FUSED ? min(p_new + 1, S) : min(lens[b], S);  // never read past the cache capacity
   // splits share the *runtime* length evenly (one captured graph serves every step)
   const int chunk = (len + NS - 1) / NS;
   const int k0 = split * chunk, k1 = min(len, k0 + chunk);
-  DEC_PROBE(1, k1);
   const int tid = threadIdx.x, sub = tid % LPK, grp = tid / LPK;
   float* wsp = ws + ((size_t)bk * NS + split) * G * (HD + 2);
   if (k0 >= k1) {
@@ -595,11 +573,8 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
     }
     return;
   }
-  bf16_t* kb = kc + ((size_t)b * Hkv + kvh) * S * HD;
-  bf16_t* vb = vc + ((size_t)b * Hkv + kvh) * S * HD;
-  constexpr int EB = KV8 ? 1 : 2;  // cache bytes per element
-  uint8_t* kb8 = reinterpret_cast<uint8_t*>(kc) + ((size_t)b * Hkv + kvh) * S * HD * EB;
-  uint8_t* vb8 = reinterpret_cast<uint8_t*>(vc) + ((size_t)b * Hkv + kvh) * S * HD * EB;
+  uint8_t* kb8 = reinterpret_cast<uint8_t*>(kc) + ((size_t)b * Hkv + kvh) * S * HD;
+  uint8_t* vb8 = reinterpret_cast<uint8_t*>(vc) + ((size_t)b * Hkv + kvh) * S * HD;
   float qv[G][ELT];
   float nk[ELT] = {}, nv[ELT] = {};
   // FUSED: is the new key inside this split (and inside the cache)?
@@ -641,21 +616,13 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
       for (int j = 0; j < ELT / 2; ++j) qp[g][j] = pack2bf(qv[g][2 * j], qv[g][2 * j + 1]);
   }
   uint32_t nvp[ELT / 2];
-  i32x4 nk8 = {0, 0, 0, 0}, nv8 = {0, 0, 0, 0};  // KV8: the new row as stored (e4m3)
-  if constexpr (KV8) {
-    kv8_pack(nk, nk8);
-    kv8_pack(nv, nv8);
-    kv8_unpack(nk8, nkp);  // the register copy = what the cache will hold
-    kv8_unpack(nv8, nvp);
-  } else {
-#pragma unroll
-    for (int j = 0; j < ELT / 2; ++j) nkp[j] = pack2bf(nk[j * 2], nk[j * 2 + 1]);
-#pragma unroll
-    for (int j = 0; j < ELT / 2; ++j) nvp[j] = pack2bf(nv[j * 2], nv[j * 2 + 1]);
-  }
+  i32x4 nk8 = {0, 0, 0, 0}, nv8 = {0, 0, 0, 0};  // the new row as stored (e4m3)
+  kv8_pack(nk, nk8);
+  kv8_pack(nv, nv8);
+  kv8_unpack(nk8, nkp);  // the register copy = what the cache will hold
+  kv8_unpack(nv8, nvp);
   float* sc = dsm;  // [G][chunk]
   const int n = k1 - k0;
-  DEC_PROBE(2, nvp[0]);
   if constexpr (MF) {
     static_assert(G <= 16, "MFMA score tile has 16 head columns");
     constexpr int NKC = HD / 32;  // k-steps of 32 dims
@@ -679,8 +646,8 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
         load_head8<HD, ROPE>(q + (size_t)b * ldq + (H + kvh) * HD, c4 + 4 * m, cosT, sinT, min(p_new, S - 1), t8);
 #pragma unroll
         for (int j = 0; j < 8; ++j) nkA[m][j] = (short)f2bf(t8[j]);
-        if constexpr (KV8)  // the register copy = the stored e4m3 row
-          nkA[m] = __builtin_bit_cast(bf16x8, kv8_unpack8(kv8_pack8(__builtin_bit_cast(i32x4, nkA[m]))));
+        // the register copy = the stored e4m3 row
+        nkA[m] = __builtin_bit_cast(bf16x8, kv8_unpack8(kv8_pack8(__builtin_bit_cast(i32x4, nkA[m]))));
       }
     }
     const int ntile = (n + 15) / 16;
@@ -691,19 +658,14 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
         const int kk = min((t0 + tb * 4 + wave) * 16 + hj, n - 1);
 #pragma unroll
         for (int m = 0; m < NKC; ++m) {
-          if constexpr (KV8) {  // 8 e4m3 entries -> the same bf16 A fragment
-            typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-            const u32x2* kp8 = reinterpret_cast<const u32x2*>(kb8 + (size_t)(k0 + kk) * HD + (c4 + 4 * m) * 8);
-            const u32x2 w = NT ? __builtin_nontemporal_load(kp8) : *kp8;
-            ka[tb][m] = __builtin_bit_cast(bf16x8, kv8_unpack8(make_uint2(w[0], w[1])));
-          } else {
-            const bf16x8* kp = reinterpret_cast<const bf16x8*>(kb + (size_t)(k0 + kk) * HD + (c4 + 4 * m) * 8);
-            ka[tb][m] = NT ? __builtin_nontemporal_load(kp) : *kp;
-          }
+          // 8 e4m3 entries -> the same bf16 A fragment
+          typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+          const u32x2* kp8 = reinterpret_cast<const u32x2*>(kb8 + (size_t)(k0 + kk) * HD + (c4 + 4 * m) * 8);
+          const u32x2 w = NT ? __builtin_nontemporal_load(kp8) : *kp8;
+          ka[tb][m] = __builtin_bit_cast(bf16x8, kv8_unpack8(make_uint2(w[0], w[1])));
         }
       }
       __builtin_amdgcn_sched_barrier(0);
-      if (t0 == 0) DEC_PROBE(8, ka[0][0][0]);
 #pragma unroll
       for (int tb = 0; tb < TB; ++tb) {
         const int t = t0 + tb * 4 + wave;
@@ -715,7 +677,6 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int m = 0; m < NKC; ++m) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[tb][m], qB[m], acc, 0, 0, 0);
-        if (t0 == 0 && tb == 0) DEC_PROBE(9, acc[0]);
         if (hj < G) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
@@ -737,7 +698,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
       // per step, so stream them non-temporally (GPT-2 B=64: 0.658 -> 0.590 ms
       // per decode step); small caches (batch 1) stay cacheable: they live in
       // the MALL from one step to the next
-      const bf16x8* kp = reinterpret_cast<const bf16x8*>(kb8 + ((size_t)(k0 + kk) * HD + sub * ELT) * EB);
+      const bf16x8* kp = reinterpret_cast<const bf16x8*>(kb8 + (size_t)(k0 + kk) * HD + sub * ELT);
       kr[u] = NT ? __builtin_nontemporal_load(kp) : *kp;
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -746,12 +707,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
       if (kb0 + u * GPB >= n) break;  // workgroup-uniform: the rest of the batch is past the context
       const int kk = kb0 + u * GPB + grp;
       uint32_t kp[ELT / 2];
-      if constexpr (KV8) {
-        kv8_unpack(__builtin_bit_cast(i32x4, kr[u]), kp);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) kp[j] = (uint32_t)(uint16_t)kr[u][2 * j] | ((uint32_t)(uint16_t)kr[u][2 * j + 1] << 16);
-      }
+      kv8_unpack(__builtin_bit_cast(i32x4, kr[u]), kp);
       if (FUSED && kk == knew) {
 #pragma unroll
         for (int j = 0; j < ELT / 2; ++j) kp[j] = nkp[j];
@@ -767,7 +723,6 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
     }
   }
   }
-  DEC_PROBE(10, 0);
   // first batch of value rows: requested now, in flight across the barrier and
   // the softmax (they depend only on the key range).  Issuing it before the
   // score loop instead measured slower on the e4m3 path (GPT-2 B=64 0.523 ->
@@ -776,11 +731,10 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
 #pragma unroll
   for (int u = 0; u < DEC_U; ++u) {
     const int kk = min(u * GPB + grp, n - 1);
-    const bf16x8* vp = reinterpret_cast<const bf16x8*>(vb8 + ((size_t)(k0 + kk) * HD + sub * ELT) * EB);
+    const bf16x8* vp = reinterpret_cast<const bf16x8*>(vb8 + (size_t)(k0 + kk) * HD + sub * ELT);
     vr0[u] = NT ? __builtin_nontemporal_load(vp) : *vp;
   }
   __syncthreads();
-  DEC_PROBE(3, 0);
   // per-head max and exp (one wave per head, strided)
   __shared__ float mh[DEC_MAXG], lh[DEC_MAXG];
   const int wave = tid >> 6, lane = tid & 63;
@@ -798,7 +752,6 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
     if (lane == 0) { mh[g] = mx; lh[g] = s; }
   }
   __syncthreads();
-  DEC_PROBE(4, 0);
   // P.V: thread owns d chunk `sub` for key group `grp`
   float acc[G][ELT];
 #pragma unroll
@@ -814,7 +767,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
 #pragma unroll
       for (int u = 0; u < DEC_U; ++u) {
         const int kk = min(kb0 + u * GPB + grp, n - 1);
-        const bf16x8* vp = reinterpret_cast<const bf16x8*>(vb8 + ((size_t)(k0 + kk) * HD + sub * ELT) * EB);
+        const bf16x8* vp = reinterpret_cast<const bf16x8*>(vb8 + (size_t)(k0 + kk) * HD + sub * ELT);
         vr[u] = NT ? __builtin_nontemporal_load(vp) : *vp;
       }
     }
@@ -827,16 +780,8 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
       if (kb0 + u * GPB >= n) break;  // workgroup-uniform, as in the score loop
       const int ka = kb0 + u * GPB + grp, kz = ka + GPB;
       uint32_t wa[ELT / 2], wz[ELT / 2];
-      if constexpr (KV8) {
-        kv8_unpack(__builtin_bit_cast(i32x4, vr[u]), wa);
-        kv8_unpack(__builtin_bit_cast(i32x4, vr[u + 1]), wz);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          wa[j] = (uint32_t)(uint16_t)vr[u][2 * j] | ((uint32_t)(uint16_t)vr[u][2 * j + 1] << 16);
-          wz[j] = (uint32_t)(uint16_t)vr[u + 1][2 * j] | ((uint32_t)(uint16_t)vr[u + 1][2 * j + 1] << 16);
-        }
-      }
+      kv8_unpack(__builtin_bit_cast(i32x4, vr[u]), wa);
+      kv8_unpack(__builtin_bit_cast(i32x4, vr[u + 1]), wz);
       if (FUSED && ka == knew) {
 #pragma unroll
         for (int j = 0; j < ELT / 2; ++j) wa[j] = nvp[j];
@@ -862,7 +807,6 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
       }
     }
   }
-  DEC_PROBE(5, acc[0][0]);
   __syncthreads();  // scores no longer needed: reuse dsm as [GPB][G][HD] reduction scratch
   float* red = dsm;
 #pragma unroll
@@ -886,395 +830,13 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const bf16_t* __restri
   }
   // the new key / value row into the cache, last: a store issued before the
   // K/V loads would sit in front of them in this wave's vmcnt queue
-  if (KV8 && FUSED && own_new && grp == 0) {
+  if (FUSED && own_new && grp == 0) {
     *reinterpret_cast<i32x4*>(kb8 + (size_t)p_new * HD + sub * 16) = nk8;
     *reinterpret_cast<i32x4*>(vb8 + (size_t)p_new * HD + sub * 16) = nv8;
-  } else if (FUSED && own_new && grp == 0) {
-    uint4 wk, wv;
-    uint32_t* pk = reinterpret_cast<uint32_t*>(&wk);
-    uint32_t* pv = reinterpret_cast<uint32_t*>(&wv);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      pk[j] = nkp[j];
-      pv[j] = nvp[j];
-    }
-    *reinterpret_cast<uint4*>(kb + (size_t)p_new * HD + sub * 8) = wk;
-    *reinterpret_cast<uint4*>(vb + (size_t)p_new * HD + sub * 8) = wv;
-  }
-  DEC_PROBE(7, 0);
-}
-
-// ---------------------------------------------------------------------------
-// One-pass decode attention (round 3): every key and value row of a split is
-// requested before the first score is formed, so a workgroup's whole K/V
-// range is in flight at once instead of one batch per round trip.
-//
-// attn_decode_kernel above runs K batch -> scores -> softmax pass -> V batch
-// -> P.V -> V batch ...: at Llama-3 8B B=32 (B*Hkv = 256, 3 splits of ~180
-// keys) that chain ran at 3.5 TB/s plus a 4.8 us combine launch, at GPT-2
-// B=64 at 5.0 TB/s.  Here, for a split of at most CAP = NW*KT*16 keys:
-//   1. q / new key / new value (first in the vmcnt queue), then every K tile
-//      of the wave (KT x HD/32 16-B loads per lane), then the first VE value
-//      rows of the thread;
-//   2. scores on MFMA as K lands (16 keys x 16 head columns per tile, lane =
-//      key row, B = q^T), written to LDS, and each wave's per-head max kept
-//      in registers -> LDS (no separate max pass);
-//   3. the remaining value rows are issued as soon as the K registers are
-//      free, then one barrier;
-//   4. P.V on v_dot2 (thread = 8 dims of VU rows), exponentials taken where
-//      they are used, row sums carried beside the accumulators;
-//   5. one LDS reduction over the row groups, output written directly (one
-//      split) or as the (o, m, l) partial decode_combine_kernel merges.
-// Cache rows past the runtime length are never scored: their loads are
-// clamped to the last valid row (same address: coalesced).
-template <int HD, int G, int FM, bool NT, int NW, int KT, int VE, int VU, bool RS = false, bool KNT = NT,
-          bool KF = false>
-__global__ __launch_bounds__(NW * 64) void attn_decode_1p_kernel(const bf16_t* __restrict__ q, int ldq,
-                                                               bf16_t* __restrict__ kc, bf16_t* __restrict__ vc,
-                                                               float* __restrict__ ws, int H, int Hkv, int S,
-                                                               const int* __restrict__ lens,
-                                                               const float* __restrict__ cosT,
-                                                               const float* __restrict__ sinT, float scale_log2,
-                                                               bf16_t* __restrict__ o_direct) {
-  // RS: scores in the row layout (thread = 8 dims of key rows grp + GPB*u, dot2
-  // + DPP row sum, as the value rows) instead of MFMA key tiles; KNT: the key
-  // loads non-temporal (NT: the value loads)
-  constexpr bool FUSED = FM != 0, ROPE = FM == 2;
-  constexpr int NTH = NW * 64;
-  constexpr int LPK = HD / 8;          // lanes per value row (16 B = 8 dims each)
-  constexpr int GPB = NTH / LPK;       // value row groups
-  constexpr int NKC = HD / 32;         // MFMA k-steps of a key tile
-  constexpr int CAP = RS ? GPB * VU : NW * KT * 16;  // keys per split (host-checked)
-  constexpr int KR = RS ? VU : 1;      // key rows per thread (RS)
-  static_assert(GPB * VU >= CAP, "value rows must cover the key tiles");
-  static_assert(VE <= VU && VU % 2 == 0 && G <= 16, "bad shape");
-  __shared__ __attribute__((aligned(16))) float sc[CAP * G];  // scaled scores, [key][head] (one LDS read per key)
-  __shared__ float wmax[NW][G];        // per-wave score max per head
-  extern __shared__ __attribute__((aligned(16))) float red1p[];  // [NW][G][HD] + [NW][G]
-
-  const int bk = blockIdx.x, split = blockIdx.y, NS = gridDim.y;
-  const int b = bk / Hkv, kvh = bk % Hkv;
-  const int p_new = FUSED ? lens[b] : 0;
-  const int len = FUSED ? min(p_new + 1, S) : min(lens[b], S);
-  const int chunk = (len + NS - 1) / NS;
-  const int k0 = split * chunk, k1 = min(len, k0 + chunk);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int hj = lane & 15, c4 = lane >> 4;
-  const int sub = tid % LPK, grp = tid / LPK;
-  float* wsp = ws + ((size_t)bk * NS + split) * G * (HD + 2);
-  if (k0 >= k1) {  // empty split (short context): neutral partial
-    for (int i = tid; i < G * (HD + 2); i += NTH) wsp[i] = (i % (HD + 2)) == HD ? -INFINITY : 0.f;
-    return;
-  }
-  const int n = k1 - k0;
-  bf16_t* kb = kc + ((size_t)b * Hkv + kvh) * S * HD + (size_t)k0 * HD;
-  bf16_t* vb = vc + ((size_t)b * Hkv + kvh) * S * HD + (size_t)k0 * HD;
-  const bool own_new = FUSED && p_new < S && p_new >= k0 && p_new < k1;
-  const int knew = own_new ? p_new - k0 : -1;
-  const int pr = min(p_new, S - 1);
-
-  // ---- K: MFMA tiles t = wave + NW*i (lane loads key row t*16 + hj, dims
-  // (c4 + 4m)*8), or RS rows grp + GPB*u (dims sub*8); then the first VE value
-  // rows (row grp + GPB*u, dims sub*8).  KF: issued before q, so the K/V
-  // stream starts without waiting for q (and the RoPE tables); q then lands
-  // behind them in the vmcnt queue, which the scores wait for anyway
-  bf16x8 ka[RS ? 1 : KT][NKC];
-  bf16x8 kr[KR];
-  bf16x8 vr[VU];
-  auto issue_kv = [&]() __attribute__((always_inline)) {
-    if constexpr (!RS) {
-#pragma unroll
-      for (int i = 0; i < KT; ++i) {
-        const int kk = min((wave + NW * i) * 16 + hj, n - 1);
-#pragma unroll
-        for (int m = 0; m < NKC; ++m) {
-          const bf16x8* kp = reinterpret_cast<const bf16x8*>(kb + (size_t)kk * HD + (c4 + 4 * m) * 8);
-          ka[i][m] = KNT ? __builtin_nontemporal_load(kp) : *kp;
-        }
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < KR; ++u) {
-        const bf16x8* kp = reinterpret_cast<const bf16x8*>(kb + (size_t)min(grp + GPB * u, n - 1) * HD + sub * 8);
-        kr[u] = KNT ? __builtin_nontemporal_load(kp) : *kp;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < VE; ++u) {
-      const bf16x8* vp = reinterpret_cast<const bf16x8*>(vb + (size_t)min(grp + GPB * u, n - 1) * HD + sub * 8);
-      vr[u] = NT ? __builtin_nontemporal_load(vp) : *vp;
-    }
-  };
-  if constexpr (KF) {
-    issue_kv();
-    __builtin_amdgcn_sched_barrier(0);
-  }
-
-  // ---- 1. q (MFMA: q^T B operand with columns >= G zero, new key in A layout;
-  // RS: bf16 pairs of this thread's 8 dims per head), new k/v (row layout)
-  bf16x8 qB[NKC], nkA[NKC];
-  uint32_t qp[RS ? G : 1][4];
-  if constexpr (!RS) {
-#pragma unroll
-    for (int m = 0; m < NKC; ++m) {
-      float t8[8];
-      const int hq = min(hj, G - 1);
-      if constexpr (FUSED) {
-        load_head8<HD, ROPE>(q + (size_t)b * ldq + (kvh * G + hq) * HD, c4 + 4 * m, cosT, sinT, pr, t8);
-      } else {
-        const bf16x8 pq =
-            *reinterpret_cast<const bf16x8*>(q + ((size_t)b * H + kvh * G + hq) * HD + (c4 + 4 * m) * 8);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) t8[j] = bf2f_s(pq[j]);
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) qB[m][j] = hj < G ? (short)f2bf(t8[j]) : (short)0;
-      if constexpr (FUSED) {
-        load_head8<HD, ROPE>(q + (size_t)b * ldq + (H + kvh) * HD, c4 + 4 * m, cosT, sinT, pr, t8);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) nkA[m][j] = (short)f2bf(t8[j]);
-      }
-    }
-  } else {
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      float t8[8];
-      if constexpr (FUSED) {
-        load_head8<HD, ROPE>(q + (size_t)b * ldq + (kvh * G + g) * HD, sub, cosT, sinT, pr, t8);
-      } else {
-        const bf16x8 pq = *reinterpret_cast<const bf16x8*>(q + ((size_t)b * H + kvh * G + g) * HD + sub * 8);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) t8[j] = bf2f_s(pq[j]);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) qp[g][j] = pack2bf(t8[2 * j], t8[2 * j + 1]);
-    }
-  }
-  uint32_t nkp[4] = {0, 0, 0, 0}, nvp[4] = {0, 0, 0, 0};  // this thread's 8 dims of the new row (bf16 pairs)
-  if constexpr (FUSED) {
-    float nk[8], nv[8];
-    load_head8<HD, ROPE>(q + (size_t)b * ldq + (H + kvh) * HD, sub, cosT, sinT, pr, nk);
-    load_head8<HD, false>(q + (size_t)b * ldq + (H + Hkv + kvh) * HD, sub, nullptr, nullptr, 0, nv);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      nkp[j] = pack2bf(nk[2 * j], nk[2 * j + 1]);
-      nvp[j] = pack2bf(nv[2 * j], nv[2 * j + 1]);
-    }
-  }
-  if constexpr (!KF) issue_kv();
-  __builtin_amdgcn_sched_barrier(0);
-
-  // ---- 2. scores (scaled to log2 units) + this wave's max per head
-  if constexpr (!RS) {
-    float mx = -INFINITY;  // lane's head hj
-#pragma unroll
-    for (int i = 0; i < KT; ++i) {
-      const int t = wave + NW * i;
-      if (t * 16 >= n) break;  // wave-uniform
-      if (FUSED && t * 16 + hj == knew) {
-#pragma unroll
-        for (int m = 0; m < NKC; ++m) ka[i][m] = nkA[m];
-      }
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int m = 0; m < NKC; ++m) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[i][m], qB[m], acc, 0, 0, 0);
-      if (hj < G) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int key = t * 16 + c4 * 4 + r;
-          if (key < n) {
-            const float s = acc[r] * scale_log2;
-            sc[key * G + hj] = s;
-            mx = fmaxf(mx, s);
-          }
-        }
-      }
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    if (lane < G) wmax[wave][lane] = mx;
-  } else {
-    float mx[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) mx[g] = -INFINITY;
-#pragma unroll
-    for (int u = 0; u < KR; ++u) {
-      if (GPB * u >= n) break;  // workgroup-uniform
-      const int row = grp + GPB * u;
-      uint32_t kp[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) kp[j] = (uint32_t)(uint16_t)kr[u][2 * j] | ((uint32_t)(uint16_t)kr[u][2 * j + 1] << 16);
-      if (FUSED && row == knew) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) kp[j] = nkp[j];
-      }
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        float d = 0.f;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          d = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2v, qp[g][j]), __builtin_bit_cast(bf16x2v, kp[j]),
-                                              d, false);
-        d = group_sum<LPK>(d) * scale_log2;
-        if (row < n) {
-          if (sub == 0) sc[row * G + g] = d;
-          mx[g] = fmaxf(mx[g], d);
-        }
-      }
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const float m = wave_max(mx[g]);
-      if (lane == 0) wmax[wave][g] = m;
-    }
-  }
-  // ---- 3. the remaining value rows (the K registers are free now)
-#pragma unroll
-  for (int u = VE; u < VU; ++u) {
-    const bf16x8* vp = reinterpret_cast<const bf16x8*>(vb + (size_t)min(grp + GPB * u, n - 1) * HD + sub * 8);
-    vr[u] = NT ? __builtin_nontemporal_load(vp) : *vp;
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  __syncthreads();
-  float mg[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    float m = wmax[0][g];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) m = fmaxf(m, wmax[w][g]);
-    mg[g] = m;
-  }
-  // ---- 4. probabilities, once per (key, head): the whole workgroup
-  // exponentiates the score array in place (a thread of P.V would otherwise
-  // take the same exponential as the other LPK - 1 lanes of its row)
-  for (int i = tid; i < n * G; i += NTH) {
-    const int g = i % G;
-    float m = mg[0];
-#pragma unroll
-    for (int gg = 1; gg < G; ++gg) m = g == gg ? mg[gg] : m;
-    sc[i] = __builtin_amdgcn_exp2f(sc[i] - m);
-  }
-  __syncthreads();
-  // ---- 5. P.V: key pairs (u, u+1) share this thread's 8 dims; the
-  // probabilities of 4 rows are read together (one ds_read per row) so the
-  // LDS round trips overlap instead of one read -> wait -> use per head
-  float acc[G][8], ls[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    ls[g] = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
-  }
-  static_assert(VU % 4 == 0, "P.V reads probabilities 4 rows at a time");
-#pragma unroll
-  for (int u0 = 0; u0 < VU; u0 += 4) {
-    if (GPB * u0 >= n) break;  // workgroup-uniform
-    float pr4[4][G];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int row = grp + GPB * (u0 + q);
-      const float* sp = sc + min(row, n - 1) * G;
-      if constexpr (G == 4) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(sp);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) pr4[q][g] = row < n ? v[g] : 0.f;
-      } else if constexpr (G == 2) {
-        const f32x2 v = *reinterpret_cast<const f32x2*>(sp);
-#pragma unroll
-        for (int g = 0; g < 2; ++g) pr4[q][g] = row < n ? v[g] : 0.f;
-      } else {
-#pragma unroll
-        for (int g = 0; g < G; ++g) pr4[q][g] = row < n ? sp[g] : 0.f;
-      }
-    }
-#pragma unroll
-    for (int u = u0; u < u0 + 4; u += 2) {
-      const int ka_ = grp + GPB * u, kz = ka_ + GPB;
-      uint32_t wa[4], wz[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        wa[j] = (uint32_t)(uint16_t)vr[u][2 * j] | ((uint32_t)(uint16_t)vr[u][2 * j + 1] << 16);
-        wz[j] = (uint32_t)(uint16_t)vr[u + 1][2 * j] | ((uint32_t)(uint16_t)vr[u + 1][2 * j + 1] << 16);
-      }
-      if (FUSED && ka_ == knew) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) wa[j] = nvp[j];
-      }
-      if (FUSED && kz == knew) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) wz[j] = nvp[j];
-      }
-      uint32_t prr[8];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        prr[2 * j] = __builtin_amdgcn_perm(wz[j], wa[j], 0x05040100u);
-        prr[2 * j + 1] = __builtin_amdgcn_perm(wz[j], wa[j], 0x07060302u);
-      }
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const float pa = pr4[u - u0][g], pz = pr4[u - u0 + 1][g];
-        ls[g] += pa + pz;
-        const bf16x2v pp = __builtin_bit_cast(bf16x2v, pack2bf(pa, pz));
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          acc[g][j] = __builtin_amdgcn_fdot2_f32_bf16(pp, __builtin_bit_cast(bf16x2v, prr[j]), acc[g][j], false);
-      }
-    }
-  }
-  // ---- 6. reduce over the row groups: first across the wave's 64 / LPK row
-  // groups by lane shuffles (xor LPK, 2 LPK, ...), then the NW wave sums
-  // through LDS -- [NW][G][HD] instead of [GPB][G][HD] (Llama-3 8B: 16 KB
-  // instead of 64 KB of LDS, so two GQA workgroups fit on a CU)
-  float* red = red1p;                  // [NW][G][HD]
-  float* lred = red1p + NW * G * HD;   // [NW][G]
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-#pragma unroll
-    for (int off = LPK; off < 64; off <<= 1) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) acc[g][j] += __shfl_xor(acc[g][j], off, 64);
-      ls[g] += __shfl_xor(ls[g], off, 64);
-    }
-  }
-  if (lane < LPK) {
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      f32x4* dst = reinterpret_cast<f32x4*>(red + ((size_t)wave * G + g) * HD + sub * 8);
-      dst[0] = f32x4{acc[g][0], acc[g][1], acc[g][2], acc[g][3]};
-      dst[1] = f32x4{acc[g][4], acc[g][5], acc[g][6], acc[g][7]};
-      if (sub == 0) lred[wave * G + g] = ls[g];
-    }
-  }
-  __syncthreads();
-  for (int i = tid; i < G * HD; i += NTH) {
-    const int g = i / HD, d = i % HD;
-    float s = 0.f, l = 0.f;
-#pragma unroll
-    for (int r = 0; r < NW; ++r) {
-      s += red[((size_t)r * G + g) * HD + d];
-      l += lred[r * G + g];
-    }
-    if (NS == 1) {
-      o_direct[(size_t)b * H * HD + (kvh * G + g) * HD + d] = f2bf(l > 0.f ? s / l : 0.f);
-    } else {
-      wsp[g * (HD + 2) + d] = s;
-      if (d == 0) {
-        wsp[g * (HD + 2) + HD] = mg[g];
-        wsp[g * (HD + 2) + HD + 1] = l;
-      }
-    }
-  }
-  // the new key / value row into the cache, last (behind every K/V load of this wave)
-  if (own_new && grp == 0) {
-    uint4 wk, wv;
-    wk.x = nkp[0]; wk.y = nkp[1]; wk.z = nkp[2]; wk.w = nkp[3];
-    wv.x = nvp[0]; wv.y = nvp[1]; wv.z = nvp[2]; wv.w = nvp[3];
-    bf16_t* kr = kc + ((size_t)b * Hkv + kvh) * S * HD + (size_t)p_new * HD + sub * 8;
-    bf16_t* vrp = vc + ((size_t)b * Hkv + kvh) * S * HD + (size_t)p_new * HD + sub * 8;
-    *reinterpret_cast<uint4*>(kr) = wk;
-    *reinterpret_cast<uint4*>(vrp) = wv;
   }
 }
+
+#include "attention_stream.h"
 
 // (Folding this pass into the attention kernel — the last-arriving split
 // combines, tickets behind an agent-scope release / acquire — measured 20 %
@@ -1429,14 +991,18 @@ extern "C" int dnn_flash_attn_qkv(const void* qkv, int ldqkv, void* kc, void* vc
   return (int)hipGetLastError();
 }
 
-// the split merge: the one-round-trip kernel for up to 8 splits (head dim <= 256)
+// the split merge: the one-round-trip kernel for up to 32 splits (head dim <= 256)
 static void launch_decode_combine(const float* ws, bf16_t* o, int B, int H, int Hkv, int hd, int ns, hipStream_t st) {
-  if (ns <= 8 && hd <= 256) {
+  if (ns <= 32 && hd <= 256) {
     const int th = hd <= 64 ? 64 : (hd <= 128 ? 128 : 256);
     if (ns <= 2)
       hipLaunchKernelGGL(decode_combine_fast_kernel<2>, dim3(B * H), dim3(th), 0, st, ws, o, B, H, Hkv, hd, ns);
     else if (ns <= 4)
       hipLaunchKernelGGL(decode_combine_fast_kernel<4>, dim3(B * H), dim3(th), 0, st, ws, o, B, H, Hkv, hd, ns);
+    else if (ns > 16)
+      hipLaunchKernelGGL(decode_combine_fast_kernel<32>, dim3(B * H), dim3(th), 0, st, ws, o, B, H, Hkv, hd, ns);
+    else if (ns > 8)
+      hipLaunchKernelGGL(decode_combine_fast_kernel<16>, dim3(B * H), dim3(th), 0, st, ws, o, B, H, Hkv, hd, ns);
     else
       hipLaunchKernelGGL(decode_combine_fast_kernel<8>, dim3(B * H), dim3(th), 0, st, ws, o, B, H, Hkv, hd, ns);
     return;
@@ -1444,7 +1010,7 @@ static void launch_decode_combine(const float* ws, bf16_t* o, int B, int H, int 
   hipLaunchKernelGGL(decode_combine_kernel, dim3(B * H), dim3(128), 0, st, ws, o, B, H, Hkv, hd, ns);
 }
 
-struct Dec1pArgs {
+struct StreamArgs {
   const bf16_t* q;
   int ldq;
   bf16_t *kc, *vc;
@@ -1454,88 +1020,47 @@ struct Dec1pArgs {
   const float *cosT, *sinT;
   float sl2;
   bf16_t* o;
-  bool kf;  // K/V loads issued before q (attn_decode_1p_kernel KF)
 };
-template <int HD, int G, int NW, int KT, int VE, int VU, bool RS, int FM, bool NT, bool KNT>
-static void launch_1p_k(const Dec1pArgs& a, dim3 grid, hipStream_t st) {
-  const size_t smem = sizeof(float) * (size_t)NW * G * (HD + 1);  // [NW][G][HD] + [NW][G] (step 6)
-  if (a.kf)
-    hipLaunchKernelGGL((attn_decode_1p_kernel<HD, G, FM, NT, NW, KT, VE, VU, RS, KNT, true>), grid, dim3(NW * 64),
-                       smem, st, a.q, a.ldq, a.kc, a.vc, a.ws, a.H, a.Hkv, a.S, a.lens, a.cosT, a.sinT, a.sl2, a.o);
-  else
-    hipLaunchKernelGGL((attn_decode_1p_kernel<HD, G, FM, NT, NW, KT, VE, VU, RS, KNT, false>), grid, dim3(NW * 64),
-                       smem, st, a.q, a.ldq, a.kc, a.vc, a.ws, a.H, a.Hkv, a.S, a.lens, a.cosT, a.sinT, a.sl2, a.o);
-}
-template <int HD, int G, int NW, int KT, int VE, int VU, bool RS, int FM>
-static void launch_1p_f(const Dec1pArgs& a, bool nt, bool knt, dim3 grid, hipStream_t st) {
-  if (!nt)
-    launch_1p_k<HD, G, NW, KT, VE, VU, RS, FM, false, false>(a, grid, st);
-  else if (knt)
-    launch_1p_k<HD, G, NW, KT, VE, VU, RS, FM, true, true>(a, grid, st);
-  else
-    launch_1p_k<HD, G, NW, KT, VE, VU, RS, FM, true, false>(a, grid, st);
-}
-template <int HD, int G, int NW, int KT, int VE, int VU, bool RS>
-static void launch_1p(const Dec1pArgs& a, int fm, bool nt, bool knt, dim3 grid, hipStream_t st) {
-  if (fm == 2)
-    launch_1p_f<HD, G, NW, KT, VE, VU, RS, 2>(a, nt, knt, grid, st);
-  else if (fm == 1)
-    launch_1p_f<HD, G, NW, KT, VE, VU, RS, 1>(a, nt, knt, grid, st);
-  else
-    launch_1p_f<HD, G, NW, KT, VE, VU, RS, 0>(a, nt, knt, grid, st);
+template <int HD, int G, int NW>
+static void launch_stream(const StreamArgs& a, int fm, bool nt, dim3 grid, hipStream_t st) {
+#define DECS(FMV, NTV)                                                                                             \
+  if (fm == FMV && nt == NTV)                                                                                      \
+    hipLaunchKernelGGL((attn_decode_stream_kernel<HD, G, FMV, NTV, NW, 4>), grid, dim3(NW * 64), 0, st, a.q, a.ldq, \
+                       a.kc, a.vc, a.ws, a.H, a.Hkv, a.S, a.lens, a.cosT, a.sinT, a.sl2, a.o);
+  DECS(0, false) DECS(0, true) DECS(1, false) DECS(1, true) DECS(2, false) DECS(2, true)
+#undef DECS
 }
 
-// One-pass decode attention (bf16 cache): returns 1 when the shape is not
-// covered (the caller falls back to the batched kernel).  Splits of at most
-// DEC1P_CAP keys; more than one split only when the caller's workspace holds
-// them; grids below 128 workgroups keep the split-K kernel (its splits fill
-// the chip at batch 1).
-constexpr int DEC1P_CAP = 640;
-static int attn_decode_1p_launch(const void* q, int ldq, void* kc, void* vc, void* o, int B, int H, int Hkv, int hd,
-                                 int S, const int* lens, const float* cosT, const float* sinT, float sl2, int splits,
-                                 float* ws, int fm, bool nt, bool force, hipStream_t st) {
-  const int G = H / Hkv;
-  int ns = (S + DEC1P_CAP - 1) / DEC1P_CAP;
-  // DNN_DECODE_1P_NS=n: at least n key splits (A/B; needs the caller's workspace)
-  const char* ns_e = getenv("DNN_DECODE_1P_NS");
-  const int ns_min = ns_e != nullptr ? atoi(ns_e) : 0;
-  if (ns_min > ns) ns = ns_min;
-  if (ns > 1 && ns > splits) return 1;
-  if (!force && (long)B * Hkv * ns < 128) return 1;
-  // GQA past one workgroup per CU: the 86 KiB of LDS per workgroup keeps one
-  // resident per CU, so a second round of workgroups runs serially and the
-  // batched kernel wins (Llama-3 B=64: 36.5 vs 30.9 us,
-  // profiles/r3_attn_1p_shapes.jsonl); MHA's 4-wave workgroups are small
-  if (!force && ns_min <= 1 && G > 1 && (long)B * Hkv * ns > 256) return 1;
-  dim3 grid(B * Hkv, ns);
-  // row-layout scores for MHA, MFMA key tiles for GQA: at MHA hd 64 an MFMA tile
-  // uses 1 of 16 head columns and its half-row key loads ran 10 % slower than
-  // whole rows (GPT-2 B=64 22.0 vs 19.9 us, profiles/r3_attn_1p_probe.jsonl)
-  const char* rs_e = getenv("DNN_DECODE_1P_RS");    // A/B override: 0 MFMA tiles, 1 row layout
-  const char* kn_e = getenv("DNN_DECODE_1P_KNT");   // key loads non-temporal (A/B; default: as the values)
-  const bool rs = rs_e != nullptr ? atoi(rs_e) == 1 : G == 1;
-  // key loads: non-temporal for MHA, default policy for GQA (Llama-3 B=32
-  // 19.54 -> 19.11 us; GPT-2 B=64 19.28 -> 20.01 the other way)
-  const bool knt = nt && (kn_e != nullptr ? atoi(kn_e) != 0 : G == 1);
-  // K/V loads before q for GQA (Llama-3 B=32 19.40 -> 19.12 us, decode 3.930 -> 3.902 ms/step), after q for
-  // MHA (GPT-2 B=64 19.50 -> 19.91 us the other way; profiles/r3_attn_1p_probe_v3.jsonl)
-  const char* kf_e = getenv("DNN_DECODE_1P_KF");    // A/B override: 1 before q, 0 after
-  const bool kf = kf_e != nullptr ? atoi(kf_e) == 1 : G > 1;
-  Dec1pArgs a{(const bf16_t*)q, ldq, (bf16_t*)kc, (bf16_t*)vc, ws, H, Hkv, S, lens, cosT, sinT, sl2, (bf16_t*)o, kf};
-  // hd 128 GQA (Llama-3 G = 4, llama3-tiny G = 2): 8 waves x 5 key tiles; hd 64 MHA (GPT-2): 4 waves x 10
-  // (row-layout scores for GQA measured 22.3 vs 19.0 us at Llama-3 B=32: not built)
-  if (hd == 128 && G == 4)
-    launch_1p<128, 4, 8, 5, 8, 20, false>(a, fm, nt, knt, grid, st);
-  else if (hd == 128 && G == 2)
-    launch_1p<128, 2, 8, 5, 8, 20, false>(a, fm, nt, knt, grid, st);
-  else if (hd == 64 && G == 1 && rs)
-    launch_1p<64, 1, 4, 10, 2, 20, true>(a, fm, nt, knt, grid, st);
-  else if (hd == 64 && G == 1)
-    launch_1p<64, 1, 4, 10, 6, 20, false>(a, fm, nt, knt, grid, st);
-  else
-    return 1;
-  if (ns > 1)
-    launch_decode_combine(ws, (bf16_t*)o, B, H, Hkv, hd, ns, st);
+// Waves of a workgroup and key splits of the stream kernel (bf16 cache).
+//
+// 8 waves while that leaves the chip with at most two workgroups a CU (one with
+// grouped heads, whose waves hold more registers), else 4.  us at 8 / 4 waves: GPT-2
+// B=8 of 300 keys 4.6 / 5.0, B=20 of 500 8.2 / 8.6, B=64 of 512 17.4 / 16.9, XL B=64 of
+// 60 12.0 / 8.4; Llama-3 B=32 of 1100 22.8 / 25.3, B=64 of 150 11.8 / 10.1.
+//
+// Splits cost a second launch (2.5 us and more).  Grouped heads: as many as put one
+// workgroup on every CU, of at least 128 keys (B=1 of 2048 keys 1 / 4 / 8 splits 21.4 /
+// 11.0 / 9.6 us, B=16 of 1000 1 / 2 / 4: 15.7 / 15.1 / 17.5; B=1 of 200 1 / 2: 5.7 / 6.6).
+// One head a row: a block of 8 waves takes 256 keys in the time of 64 here, so the line
+// is at 1024 keys (B=1 of 960 1 / 4 / 8: 6.4 / 6.6 / 6.5).
+static int attn_stream_launch(const StreamArgs& a, int B, int hd, int splits, int fm, bool nt, hipStream_t st) {
+  const int G = a.H / a.Hkv;
+  const long wgs = (long)B * a.Hkv;
+  long ns = (256 + wgs - 1) / wgs;
+  ns = std::min(ns, (long)(a.S / (G > 1 ? 128 : 1024)));
+  ns = std::max(1L, std::min(ns, (long)splits));
+  const bool w8 = wgs * ns <= (G > 1 ? 256 : 512);
+  const dim3 grid(B * a.Hkv, (unsigned)ns);
+#define STR(HDV, GV)                                    \
+  if (hd == HDV && G == GV) {                           \
+    if (w8)                                             \
+      launch_stream<HDV, GV, 8>(a, fm, nt, grid, st);   \
+    else                                                \
+      launch_stream<HDV, GV, 4>(a, fm, nt, grid, st);   \
+  } else
+  STR(64, 1) STR(64, 2) STR(64, 4) STR(64, 8) STR(128, 1) STR(128, 2) STR(128, 4) STR(128, 8) { return -2; }
+#undef STR
+  if (ns > 1) launch_decode_combine(a.ws, a.o, B, a.H, a.Hkv, hd, (int)ns, st);
   return (int)hipGetLastError();
 }
 
@@ -1544,20 +1069,9 @@ static int attn_decode_launch(const void* q, int ldq, void* kc, void* vc, void* 
                               float* ws, bool fused, hipStream_t st, bool kv8 = false) {
   const int G = H / Hkv;
   if (H % Hkv != 0 || G > DEC_MAXG || splits <= 0) return -1;
-  if (!kv8) {
-    // DNN_DECODE_1P=0 keeps the batched kernel everywhere (A/B), =2 takes the
-    // one-pass kernel on small grids too (tests)
-    const char* e1 = getenv("DNN_DECODE_1P");
-    const int m1 = e1 != nullptr ? atoi(e1) : 1;
-    if (m1 != 0) {
-      const bool nt1 = (double)B * Hkv * S * hd * 4.0 > 32.0 * 1024 * 1024;
-      const int r = attn_decode_1p_launch(q, ldq, kc, vc, o, B, H, Hkv, hd, S, lens, cosT, sinT,
-                                          scale * 1.4426950408889634f, splits, ws,
-                                          fused ? (cosT != nullptr ? 2 : 1) : 0, nt1, m1 == 2, st);
-      if (r != 1) return r;
-    }
-  }
   if (kv8 && G != 1 && hd != 128) return -4;  // e4m3 cache: MHA, or GQA at hd 128 (Llama-3)
+  // a split's keys per head are bounded for both caches by what the e4m3 kernel's LDS
+  // holds of their scores (the caller's splits grow with the capacity)
   const int chunk_cap = (S + splits - 1) / splits;
   const int gpb = 256 / (hd / (kv8 ? 16 : 8));
   size_t smem = sizeof(float) * (size_t)G * (size_t)(chunk_cap > gpb * hd ? chunk_cap : gpb * hd);
@@ -1566,82 +1080,43 @@ static int attn_decode_launch(const void* q, int ldq, void* kc, void* vc, void* 
   dim3 grid(B * Hkv, splits);
   // cache bytes this launch may stream (capacity bound): > 32 MB -> non-temporal
   const bool nt = (double)B * Hkv * S * hd * (kv8 ? 2.0 : 4.0) > 32.0 * 1024 * 1024;
-  // MFMA scores: GQA (G >= 2) by default; DNN_DECODE_MFMA=0/1 forces it off/on (A/B)
-  const char* mf_e = getenv("DNN_DECODE_MFMA");
-  const bool mf = mf_e ? atoi(mf_e) == 1 : G >= 2;
   const int fm = fused ? (cosT != nullptr ? 2 : 1) : 0;
-  if (kv8) {
-    // DNN_KV8_U=8: 8 rows in flight per thread instead of 10 (A/B)
-    const char* u_e = getenv("DNN_KV8_U");
-    const bool u8 = u_e != nullptr && atoi(u_e) == 8;
+  if (!kv8)
+    return attn_stream_launch({(const bf16_t*)q, ldq, (bf16_t*)kc, (bf16_t*)vc, ws, H, Hkv, S, lens, cosT, sinT, sl2,
+                               (bf16_t*)o}, B, hd, splits, fm, nt, st);
+  // DNN_KV8_U=8: 8 rows in flight per thread instead of 10 (A/B)
+  const char* u_e = getenv("DNN_KV8_U");
+  const bool u8 = u_e != nullptr && atoi(u_e) == 8;
 #define DEC8(HDV, NTV, FMV)                                                                                          \
   if (hd == HDV && nt == NTV && fm == FMV) {                                                                          \
     if (u8)                                                                                                           \
-      hipLaunchKernelGGL((attn_decode_kernel<HDV, 1, FMV, NTV, false, true, 8>), grid, dim3(256), smem, st,           \
+      hipLaunchKernelGGL((attn_decode_kernel<HDV, 1, FMV, NTV, false, 8>), grid, dim3(256), smem, st,           \
                          (const bf16_t*)q, ldq, (bf16_t*)kc, (bf16_t*)vc, ws, H, Hkv, S, lens, nullptr, nullptr, sl2,  \
                          chunk_cap, (bf16_t*)o);                                                                      \
     else                                                                                                              \
-      hipLaunchKernelGGL((attn_decode_kernel<HDV, 1, FMV, NTV, false, true, 10>), grid, dim3(256), smem, st,          \
+      hipLaunchKernelGGL((attn_decode_kernel<HDV, 1, FMV, NTV, false, 10>), grid, dim3(256), smem, st,          \
                          (const bf16_t*)q, ldq, (bf16_t*)kc, (bf16_t*)vc, ws, H, Hkv, S, lens, nullptr, nullptr, sl2,  \
                          chunk_cap, (bf16_t*)o);                                                                      \
   } else
-    if (G > 1) {  // GQA: MFMA key tiles (hd 128: Llama-3 G = 4, llama3-tiny G = 2)
+  if (G > 1) {  // GQA: MFMA key tiles (hd 128: Llama-3 G = 4, llama3-tiny G = 2)
 #define DEC8G(GV, NTV, FMV)                                                                                           \
   if (G == GV && nt == NTV && fm == FMV)                                                                              \
-    hipLaunchKernelGGL((attn_decode_kernel<128, GV, FMV, NTV, true, true>), grid, dim3(256), smem, st,                \
+    hipLaunchKernelGGL((attn_decode_kernel<128, GV, FMV, NTV, true>), grid, dim3(256), smem, st,                \
                        (const bf16_t*)q, ldq, (bf16_t*)kc, (bf16_t*)vc, ws, H, Hkv, S, lens, cosT, sinT, sl2,         \
                        chunk_cap, (bf16_t*)o);                                                                        \
   else
-      DEC8G(4, true, 2) DEC8G(4, false, 2) DEC8G(4, true, 1) DEC8G(4, false, 1) DEC8G(4, true, 0) DEC8G(4, false, 0)
-      DEC8G(2, true, 2) DEC8G(2, false, 2) DEC8G(2, true, 1) DEC8G(2, false, 1) DEC8G(2, true, 0) DEC8G(2, false, 0)
-      { return -2; }
+    DEC8G(4, true, 2) DEC8G(4, false, 2) DEC8G(4, true, 1) DEC8G(4, false, 1) DEC8G(4, true, 0) DEC8G(4, false, 0)
+    DEC8G(2, true, 2) DEC8G(2, false, 2) DEC8G(2, true, 1) DEC8G(2, false, 1) DEC8G(2, true, 0) DEC8G(2, false, 0)
+    { return -2; }
 #undef DEC8G
-    } else
-    DEC8(64, true, 1) DEC8(64, false, 1) DEC8(128, true, 1) DEC8(128, false, 1) DEC8(64, true, 0) DEC8(64, false, 0)
-    DEC8(128, true, 0) DEC8(128, false, 0) { return -2; }
-#undef DEC8
-    if (splits > 1)
-      launch_decode_combine(ws, (bf16_t*)o, B, H, Hkv, hd, splits, st);
-    return (int)hipGetLastError();
-  }
-#define DEC_FM(HDV, GV, NTV, MFV)                                                                                     \
-  if (fm == 2)                                                                                                        \
-    hipLaunchKernelGGL((attn_decode_kernel<HDV, GV, 2, NTV, MFV>), grid, dim3(256), smem, st, (const bf16_t*)q, ldq,  \
-                       (bf16_t*)kc, (bf16_t*)vc, ws, H, Hkv, S, lens, cosT, sinT, sl2, chunk_cap, (bf16_t*)o);        \
-  else if (fm == 1)                                                                                                   \
-    hipLaunchKernelGGL((attn_decode_kernel<HDV, GV, 1, NTV, MFV>), grid, dim3(256), smem, st, (const bf16_t*)q, ldq,  \
-                       (bf16_t*)kc, (bf16_t*)vc, ws, H, Hkv, S, lens, nullptr, nullptr, sl2, chunk_cap, (bf16_t*)o);  \
-  else                                                                                                                \
-    hipLaunchKernelGGL((attn_decode_kernel<HDV, GV, 0, NTV, MFV>), grid, dim3(256), smem, st, (const bf16_t*)q, ldq,  \
-                       (bf16_t*)kc, (bf16_t*)vc, ws, H, Hkv, S, lens, nullptr, nullptr, sl2, chunk_cap, (bf16_t*)o);
-#define DEC_NT(HDV, GV, NTV)                                                                                          \
-  if (mf) {                                                                                                           \
-    DEC_FM(HDV, GV, NTV, true)                                                                                        \
-  } else {                                                                                                            \
-    DEC_FM(HDV, GV, NTV, false)                                                                                       \
-  }
-#define DEC(HDV, GV)                                                                                                  \
-  if (hd == HDV && G == GV) {                                                                                         \
-    if (nt) {                                                                                                         \
-      DEC_NT(HDV, GV, true)                                                                                           \
-    } else {                                                                                                          \
-      DEC_NT(HDV, GV, false)                                                                                          \
-    }                                                                                                                 \
   } else
-  DEC(64, 1) DEC(64, 2) DEC(64, 4) DEC(64, 8) DEC(128, 1) DEC(128, 2) DEC(128, 4) DEC(128, 8) { return -2; }
-#undef DEC
-#undef DEC_NT
-#undef DEC_FM
+  DEC8(64, true, 1) DEC8(64, false, 1) DEC8(128, true, 1) DEC8(128, false, 1) DEC8(64, true, 0) DEC8(64, false, 0)
+  DEC8(128, true, 0) DEC8(128, false, 0) { return -2; }
+#undef DEC8
   if (splits > 1)
     launch_decode_combine(ws, (bf16_t*)o, B, H, Hkv, hd, splits, st);
   return (int)hipGetLastError();
 }
-
-#ifdef DNN_DEC_PROBE
-extern "C" int dnn_dec_probe_read(unsigned long long* out) {
-  return (int)hipMemcpyFromSymbol(out, HIP_SYMBOL(dec_probe_ts), sizeof(unsigned long long) * 32);
-}
-#endif
 
 extern "C" int dnn_attn_decode(const void* q, const void* kc, const void* vc, void* o, int B, int H, int Hkv, int hd,
                                int S, const int* lens, float scale, int splits, float* ws, hipStream_t st, int kv8) {

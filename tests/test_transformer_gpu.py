@@ -238,6 +238,58 @@ def test_attn_decode(B, H, Hkv, hd, S, lens, mfma, monkeypatch):
         assert _rel(out[b], ref) < 2e-2, b
 
 
+@pytest.mark.parametrize("H,Hkv,hd", [(3, 3, 64), (4, 2, 64), (8, 2, 64), (8, 1, 64), (2, 2, 128), (4, 2, 128),
+                                      (8, 2, 128), (16, 2, 128)])
+@pytest.mark.parametrize("B,S,rope", [(1, 130, True), (4, 700, False), (2, 5000, True), (150, 40, True)])
+def test_attn_decode_stream(H, Hkv, hd, B, S, rope):
+    """One key, blocks cut anywhere, a full cache, one past it; one and several splits,
+    4 and 8 waves: a step from the projection rows (RoPE, new row appended) and over
+    cached keys, against fp64.  Probabilities and the result are rounded to bf16
+    (8 bits: 2^-8 each of the sum of |p v|), the rest is fp32."""
+    from distributed_neural_networks_amd.ops import transformer_ops as T
+    g = torch.Generator(device=DEV).manual_seed(B + hd + H)
+    rn = lambda *s: torch.randn(*s, device=DEV, generator=g).bfloat16()  # noqa: E731
+    kc, vc, qkv = rn(B, Hkv, S, hd), rn(B, Hkv, S, hd), rn(B, (H + 2 * Hkv) * hd)
+    edge = [0, S - 1, S, 15, 16, 31, 32, 33, 63, 64, 127, 128, 129, S // 2, S - 2]
+    pos = torch.tensor([min(edge[(b + H) % len(edge)], S) for b in range(B)], dtype=torch.int32, device=DEV)
+    cos = sin = None
+    if rope:
+        t = torch.arange(S, device=DEV)[:, None] * torch.rand(hd // 2, device=DEV, generator=g)[None]
+        cos, sin = torch.cos(t), torch.sin(t)
+    G = H // Hkv
+    splits = T.decode_splits(S, B, Hkv, G)
+    ws = torch.full((B * Hkv * splits * G * (hd + 2),), float("nan"), device=DEV)
+    out = torch.empty(B, H * hd, device=DEV, dtype=torch.bfloat16)
+    k1, v1 = kc.clone(), vc.clone()
+    T.attn_decode_qkv(qkv, k1, v1, out, B, H, Hkv, hd, pos, ws, splits, cos, sin)
+    q, k, v = (t.view(B, -1, hd) for t in qkv.split([H * hd, Hkv * hd, Hkv * hd], 1))
+    if rope:
+        c, s = (t[pos.long().clamp(max=S - 1)][:, None] for t in (cos, sin))
+        rot = lambda t: torch.cat([t[..., :hd // 2].float() * c - t[..., hd // 2:].float() * s,  # noqa: E731
+                                   t[..., hd // 2:].float() * c + t[..., :hd // 2].float() * s], -1).bfloat16()
+        q, k = rot(q), rot(k)
+    lens = []
+    for b in range(B):
+        p = int(pos[b])
+        if p < S:
+            # the rotation may be contracted to FMAs: one bf16 step
+            assert torch.allclose(k1[b, :, p].float(), k[b].float(), rtol=2 ** -7, atol=2 ** -7)
+            assert torch.equal(v1[b, :, p], v[b])
+            kc[b, :, p], vc[b, :, p] = k1[b, :, p], v[b]
+        lens.append(min(p + 1, S))
+    assert torch.equal(k1, kc) and torch.equal(v1, vc)
+    tol = 2.0 ** -6 if rope else 0.0  # q may differ by a bf16 step where the rotation is contracted
+    cached = torch.empty_like(out)
+    T.attn_decode(q.contiguous(), kc, vc, cached, B, H, Hkv, hd, torch.tensor(lens, dtype=torch.int32, device=DEV), ws,
+                  splits)
+    for b in range(B):
+        kk, vv = (t[b, :, :lens[b]].double().repeat_interleave(G, 0) for t in (kc, vc))
+        p = (torch.matmul(kk, q[b].double()[..., None])[..., 0] / math.sqrt(hd)).softmax(-1)
+        ref, mag = (torch.matmul(p[:, None], t)[:, 0].reshape(-1) for t in (vv, vv.abs()))
+        assert ((cached[b].double() - ref).abs() <= (2.0 ** -7 + 2.0 ** -12) * mag).all(), b
+        assert ((out[b].double() - ref).abs() <= (2.0 ** -7 + 2.0 ** -12 + tol) * mag).all(), b
+
+
 @pytest.mark.parametrize("B,H,Hkv,hd,S,rope,ns", [(32, 32, 8, 128, 600, True, 0), (64, 12, 12, 64, 560, False, 0),
                                                   (64, 25, 25, 64, 1300, False, 0), (32, 32, 8, 128, 600, True, 2),
                                                   (32, 32, 8, 128, 600, True, 3), (64, 12, 12, 64, 560, False, 3)])
