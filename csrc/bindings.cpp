@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "bindings_decoder.h"
+#include "prefill_blocks.h"
 
 PYBIND11_MODULE(_dnn_hip, m) {
   m.doc() = "distributed_neural_networks_amd HIP/CDNA4 kernels (gfx950)";
@@ -152,6 +153,48 @@ PYBIND11_MODULE(_dnn_hip, m) {
     return dnn_cifar_head_tail(CP(hid), CP(w2p), CFP(b2), FP(probs), IP(pred), B, ST(st));
   });
 #ifdef DNN_HAVE_TRANSFORMER
+  // blocks: 20 pointers each (qkv, o, up, down x weight, scale, bias, row sums, fragment copy); returns
+  // (code, launch that failed); -100: not a pass of this kind, nothing launched
+  m.def("prefill_blocks", [](const std::vector<int>& n, const std::vector<u64>& b, float eps, float scale,
+                             long long kv_block, long long ws_bytes, u64 st,
+                             const std::vector<u64>& blocks) -> py::tuple {
+    if (n.size() != 15 || b.size() != 19 || blocks.size() % 20 != 0)
+      throw std::runtime_error("prefill_blocks: ragged arguments");
+    dnn::PrefillPass a{};
+    int* dims[] = {&a.B, &a.T, &a.d, &a.H, &a.Hkv, &a.hd, &a.S, &a.ffn, &a.n_up, &a.act, &a.norm, &a.skinny_rows,
+                   &a.skinny_max, &a.fp8, &a.scatter};
+    for (size_t i = 0; i < n.size(); ++i) *dims[i] = n[i];
+    void** bufs[] = {&a.h, &a.a, &a.qkv, &a.q, &a.att, &a.f, &a.q8, &a.sx, &a.q8b, &a.sxb, &a.ws};
+    for (size_t i = 0; i < 11; ++i) *bufs[i] = P(b[i]);
+    a.x = CP(b[11]);
+    a.ones = CFP(b[12]);
+    a.kc = static_cast<char*>(P(b[13]));
+    a.vc = static_cast<char*>(P(b[14]));
+    a.pos = CIP(b[15]);
+    a.cosT = CFP(b[16]);
+    a.sinT = CFP(b[17]);
+    a.s8 = FP(b[18]);
+    a.eps = eps;
+    a.scale = scale;
+    a.kv_block = kv_block;
+    a.ws_bytes = ws_bytes;
+    a.st = ST(st);
+    std::vector<dnn::PrefillBlock> L(blocks.size() / 20);
+    for (size_t i = 0; i < L.size(); ++i) {
+      dnn::PrefillProj* p[] = {&L[i].qkv, &L[i].o, &L[i].up, &L[i].down};
+      for (int j = 0; j < 4; ++j) {
+        const u64* w = &blocks[i * 20 + j * 5];
+        *p[j] = {CP(w[0]), CFP(w[1]), CFP(w[2]), CFP(w[3]), CP(w[4])};
+      }
+    }
+    if (!a.covered()) return py::make_tuple(-100, "");
+    int rc;
+    {
+      py::gil_scoped_release nogil;
+      rc = a.run(L);
+    }
+    return py::make_tuple(rc, a.what);
+  });
   m.def("row_stats", [](u64 x, int ldx, u64 stats, int M, int N, float eps, int rms, u64 st) {
     return dnn_row_stats(CP(x), ldx, FP(stats), M, N, eps, rms, ST(st));
   });

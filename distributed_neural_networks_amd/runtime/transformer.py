@@ -34,6 +34,8 @@ import torch
 
 from ..models import DECODERS, model_info
 from ..models.llama3 import rope_tables
+from ..ops import _lib
+from ..ops import fp8 as F8_
 from ..ops import gemm as G_
 from ..ops.fp8 import mx_ok as fp8_mx_ok
 from ..ops import transformer_ops as T_
@@ -451,7 +453,8 @@ class TransformerStage(StageCompute):
         # of every column-tile workgroup re-deriving them
         rs = self.rowstat[r0:r1] if (T == 1 and self.fuse_norm and G_.ROWSTATS) else None
         have_rs = False
-        for li, L in enumerate(self.layers):
+        one_call = T > 1 and self._prefill_blocks(h_in, pos, B, T, b0)
+        for li, L in enumerate(() if one_call else self.layers):
             kc, vc = self.kc[li, b0:b0 + B], self.vc[li, b0:b0 + B]
             att = self.buf_att[r0:r1]
             scattered = (T > 1 and self.cos is None and self.fuse_norm and
@@ -535,6 +538,44 @@ class TransformerStage(StageCompute):
         part = self.amx_part[r0 * 2 * T_.ARGMAX_PART_PER_ROW:] if last_only else None
         T_.argmax_rows(logits, dst, n=self.V, also=also, advance=adv, part=part, hist=hist)
         return StageOutput(logits[:, :self.V], dst)
+
+    def _prefill_blocks(self, x: torch.Tensor, pos: torch.Tensor, B: int, T: int, b0: int) -> bool:
+        """The launches of ``step``'s block loop for a prefill pass, issued by one
+        native call (csrc/prefill_blocks.h) from the layers' weights as they are now.
+        False, with nothing launched, where the loop has to issue them: e4m3 caches,
+        split activations, a switch off its default, input the loop's checks are for."""
+        if not (self.layers and self.fuse_norm and G_.FOLD_NORM_PREFILL and self.kc.dtype == torch.bfloat16 and self.hd in (64, 128)
+                and pos.dtype == torch.int32 and x.dtype == torch.bfloat16 and x.is_contiguous()) or _lib.DEBUG_SYNC:
+            return False
+        if self.fp8 and (self.sx8 is None or not F8_.MX_PREFILL):
+            return False
+        blocks = []
+        for L in self.layers:
+            for w, bias, colsum, frag in ((L.w_qkv.w, L.w_qkv.bias, L.w_qkv.colsum, L.w_qkv.ws),
+                                          (L.w_o, L.b_o, None, L.w_o_s),
+                                          (L.w_up.w, L.w_up.bias, L.w_up.colsum, L.w_up.ws),
+                                          (L.w_down, L.b_down, None, L.w_down_s)):
+                scale = None
+                if self.fp8:
+                    w, scale, frag = w.q, w.scale, w.shuf
+                blocks += [w.data_ptr(), 0 if scale is None else scale.data_ptr(), 0 if bias is None else
+                           bias.data_ptr(), 0 if colsum is None else colsum.data_ptr(),
+                           0 if frag is None else frag.data_ptr()]
+        up = self.layers[0].w_up
+        S = self.kc.shape[3]
+        rc, what = _lib.lib().prefill_blocks(
+            [B, T, self.d, self.H, self.Hkv, self.hd, S, self.buf_f.shape[1], up.w.shape[0],
+             ACT_GELU if self.family == "gpt2" else ACT_SILU_MUL, up.norm, G_.SKINNY_ALWAYS_M, G_.SKINNY_MAX_M,
+             int(self.fp8), int(G_.QKV_SCATTER)],
+            [_lib.ptr(t) for t in (self.buf_h, self.buf_a, self.buf_qkv, self.buf_q, self.buf_att, self.buf_f, self.q8,
+                                   self.sx8, self.q8b, self.sx8b, self.pws, x, self.ones, self.kc[0, b0], self.vc[0, b0],
+                                   pos, self.cos, self.sin, self.s8)],
+            self.eps, 1.0 / math.sqrt(self.hd), self.kc.stride(0) * 2, 0 if self.pws is None else self.pws.nbytes,
+            _lib.stream_ptr(), blocks)
+        if rc == -100:
+            return False
+        _lib.check(rc, what)
+        return True
 
     def forward(self, x: torch.Tensor, out: Optional[torch.Tensor] = None):
         """Full-prefix forward of one request (the reference stage call,

@@ -1656,3 +1656,35 @@ def test_gemm_fp8_mx_small_tiles(tile, M, N, K):
     assert torch.equal(gq[:, N:], torch.zeros_like(gq[:, N:]))
     assert _rel(gq, wq) < 1e-3
     assert _rel(gq[:, :N], torch.nn.functional.gelu(ref)) < 4e-2
+
+
+@pytest.mark.parametrize("model,dtype", [("gpt2-tiny", "bf16"), ("gpt2", "bf16"), ("llama3-tiny", "bf16"), ("gpt2", "fp8"),
+                                         ("llama3-tiny", "fp8")])
+@pytest.mark.parametrize("B,T", [(1, 2), (2, 32), (1, 65), (3, 70), (2, 127), (1, 256), (2, 130), (3, 357)])
+def test_prefill_one_call(model, dtype, B, T, monkeypatch):
+    """The blocks of a prefill pass issued by one native call against the loop over
+    the layers: the same launches, so the same bits, into rows of a larger cache."""
+    from distributed_neural_networks_amd import checkpoint as ckpt
+    from distributed_neural_networks_amd.models import model_info
+    from distributed_neural_networks_amd.runtime.transformer import TransformerStage, build_device_stage
+    cfg = model_info(model).cfg
+    if T + 4 > (getattr(cfg, "block_size", None) or 10 ** 9):
+        pytest.skip("past the model's positions")
+    n = min(2, cfg.n_layer)
+    sd = ckpt.random_stage_state_dict(model, 0, n - 1, True, False, 3, nontrivial=cfg.__class__.__name__ == "GPTConfig")
+    st = build_device_stage(model, sd, 0, n - 1, True, False, DEV, dtype=dtype, max_batch=B + 2, max_seq=T + 4,
+                            max_tokens=B * T)
+    ids = torch.randint(0, cfg.vocab_size, (B, T), dtype=torch.int32, device=DEV)
+    pos = torch.arange(B, dtype=torch.int32, device=DEV)
+    native, calls = TransformerStage._prefill_blocks, []
+    got = []
+    for on in (True, False):
+        monkeypatch.setattr(TransformerStage, "_prefill_blocks",
+                            lambda self, *a: calls.append(native(self, *a)) or calls[-1] if on else False)
+        st.kc.zero_(), st.vc.zero_()
+        y = st.step(ids, pos, B, T, b0=1)
+        got.append((y.clone(), st.kc.clone(), st.vc.clone()))
+    assert calls == [True]
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    assert got[0][1][:, 1:1 + B].abs().sum() > 0 and got[0][1][:, 1 + B].abs().sum() == 0
