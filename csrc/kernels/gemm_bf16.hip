@@ -427,7 +427,7 @@ static int g_gemm_tile = 0;
 // Forced tile of gemm_mid.h's table and K split (tests, A/B); -1: chosen
 static int g_mid_tile = -1, g_mid_splits = 1;
 extern "C" int dnn_gemm_set_mid(int tile, int splits) {
-  if (tile < -1 || tile > 5 || splits < 1 || splits > 16) return -1;
+  if (tile < -1 || tile > 4 || splits < 1 || splits > 16) return -1;
   g_mid_tile = tile;
   g_mid_splits = splits;
   return 0;
@@ -525,15 +525,26 @@ static int launch_gemm(const void* A, int lda, const void* W, int ldw, void* C, 
   }
   // Tiles of gemm_mid.h, or 256 x 256 (and its tail split below) by estimated time
   const int tiles256 = ((M + BG_M - 1) / BG_M) * ((N + BG_N - 1) / BG_N);
-  MidPlan plan{-1, 1, 0.f};
+  MidPlan plan{-1, 1, 0.f, 0};
   if (lda >= 1 << 23 || ldw >= 1 << 23) {  // the small tiles address a tile's rows with 32 bits
-  } else if (g_mid_tile >= 0) plan = {g_mid_tile, (long long)g_mid_splits * M * N * 4 <= part_bytes ? g_mid_splits : 1, 0.f};
+  } else if (g_mid_tile >= 0) plan = {g_mid_tile, (long long)g_mid_splits * M * N * 4 <= part_bytes ? g_mid_splits : 1, 0.f, 0};
   else if (g_gemm_tile == 128) plan.tile = 2;
   else if (g_gemm_tile == 0 && (is_glu(ACT) || has_consts(ACT) || tail_split_cols(M, N) == 0))
-    plan = mid_plan(M, N, K, part_bytes, MID_BF16);
+    plan = mid_plan(M, N, K, part_bytes, has_consts(ACT) ? MID_BF16_WHOLE : MID_BF16);  // constants lie behind all N
   if (plan.tile >= 0) {
-    const MidArgs a{{C, bias, (const bf16_t*)R, ldc, ldr, M, N, ACT, F32 ? 1 : 0}, (const bf16_t*)A, (const bf16_t*)W,
-                    rowstat, colsum, (float*)ws, lda, ldw, K, plan.splits};
+    MidArgs a{{C, bias, (const bf16_t*)R, ldc, ldr, M, N, ACT, F32 ? 1 : 0}, (const bf16_t*)A, (const bf16_t*)W,
+              rowstat, colsum, (float*)ws, lda, ldw, K, plan.splits};
+    if (const int n = plan.cols) {  // disjoint columns
+      hipLaunchKernelGGL((gemm_bf16_256_kernel<ACT, F32>), dim3(((M + BG_M - 1) / BG_M) * (n / BG_N)), dim3(512), 0, st,
+                         a.A, lda, a.W, ldw, C, ldc, bias, a.R, ldr, M, n, K, g_res_prefetch, rowstat, colsum);
+      if (const hipError_t e = hipGetLastError()) return (int)e;
+      a.C = (char*)C + (size_t)(is_glu(ACT) ? n / 2 : n) * (F32 ? 4 : 2);
+      a.W += (size_t)n * ldw;
+      a.N -= n;
+      if (bias != nullptr) a.bias += n;
+      if (a.R != nullptr) a.R += n;
+      if (colsum != nullptr) a.colsum += n;
+    }
     return mid_launch(plan.tile, a, nullptr, st);
   }
   const int tilesH = ((M + BG_M - 1) / BG_M) * ((N + 127) / 128);
@@ -632,7 +643,7 @@ extern "C" int dnn_gemm_bf16_qkv_scatter(const void* A, int lda, const void* W, 
   if ((hd & (hd - 1)) != 0 || M >= (1 << 24)) return -3;
   QkvScatter sc{(bf16_t*)q, (bf16_t*)kc, (bf16_t*)vc, pos, T, H, Hkv, __builtin_ctz(hd), S, 1.0f / (float)T};
   if (g_gemm_tile == 0 && tail_split_cols(M, N) == 0 && lda < 1 << 23 && ldw < 1 << 23) {
-    MidPlan plan = mid_plan(M, N, K, 0, MID_BF16);
+    MidPlan plan = mid_plan(M, N, K, 0, MID_BF16_WHOLE);
     if (g_mid_tile >= 0) plan.tile = g_mid_tile;
     if (plan.tile >= 0) {
       const MidArgs a{{q, bias, nullptr, hd, 0, M, N, ACT_NONE, 0}, (const bf16_t*)A, (const bf16_t*)W,
@@ -731,7 +742,7 @@ extern "C" int dnn_gemm_fp8_256(const void* A, const float* sa, const void* W, c
 // bytes takes a tile as long as the bf16 kernel's K-tile of 64: the same estimate.
 static int mx_mid_tile(int M, int N, int Kb, bool quant) {
   if (g_gemm_tile != 0) return -1;
-  if (g_mid_tile >= 0) return g_mid_tile == 3 || (quant && g_mid_tile < 2) ? 2 : g_mid_tile;
+  if (g_mid_tile >= 0) return quant && g_mid_tile < 2 ? 2 : g_mid_tile;
   return mid_plan(M, N, Kb / 2, 0, quant ? MID_MX_QUANT : MID_MX).tile;
 }
 

@@ -24,9 +24,8 @@ struct MidTile {
 typedef MidTile<64, 64, 2, 2, 4> Mid0;
 typedef MidTile<128, 64, 2, 2, 6> Mid1;
 typedef MidTile<128, 128, 2, 4, 4> Mid2;
-typedef MidTile<192, 128, 2, 2, 3> Mid3;
-typedef MidTile<256, 128, 4, 2, 3> Mid4;
-typedef MidTile<128, 256, 2, 4, 3> Mid5;
+typedef MidTile<256, 128, 4, 2, 3> Mid3;
+typedef MidTile<128, 256, 2, 4, 3> Mid4;
 
 // s_waitcnt operand: at most `vm` vector-memory and `lgkm` LDS operations outstanding
 constexpr int wait_imm(int vm, int lgkm) { return (vm & 15) | (vm >> 4) << 14 | 7 << 4 | lgkm << 8; }

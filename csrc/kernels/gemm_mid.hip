@@ -15,15 +15,13 @@ struct MidCost {
   float a, s;
 };
 static constexpr MidCost MID[] = {{64, 64, 1, 1.89f, 0.252f},   {128, 64, 0, 2.78f, 0.332f},
-                                  {128, 128, 0, 2.99f, 0.472f}, {192, 128, 0, 3.71f, 0.637f},
-                                  {256, 128, 0, 4.14f, 0.707f}, {128, 256, 0, 4.07f, 0.754f},
-                                  {256, 256, 0, 4.93f, 1.198f}};
-static constexpr int MID_TILES = 6, CUS = 256;
+                                  {128, 128, 0, 2.99f, 0.472f}, {256, 128, 0, 4.14f, 0.707f},
+                                  {128, 256, 0, 4.07f, 0.754f}, {256, 256, 0, 4.93f, 1.198f}};
+static constexpr int MID_TILES = 5, CUS = 256;
 
 // Time of one tile size and split: K-tiles of the fullest CU, beside the time that
 // reading the weights (4.3 TB/s) and moving the activations (2 TB/s) takes; a split
-// adds its sum (5 us and 3 us for one more launch from the host, which bounds the
-// smallest steps, and the parts written and read at 3.2 TB/s).
+// adds its sum (one more launch, and the parts written and read at 3.2 TB/s).
 static float mid_time(const MidCost& c, int M, int N, int K, int splits) {
   const long long wgs = (long long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * splits;
   const int kt = (K / 64 + splits - 1) / splits, n = (int)((wgs + CUS - 1) / CUS);
@@ -31,19 +29,40 @@ static float mid_time(const MidCost& c, int M, int N, int K, int splits) {
   const float a = c.pairs ? c.a : c.a * (1.f + 0.5f * (n - 1));
   const float t = rounds * kt * c.s, w = (float)N * K * 2.f / 4.27e6f + (float)M * (K + N) * 2.f / 2.0e6f;
   const float us = a + cbrtf(t * t * t + w * w * w);
-  return splits == 1 ? us : us + 8.f + (splits + 0.5f) * M * N * 4.f / 3.16e6f;
+  return splits == 1 ? us : us + 4.f + (splits + 0.5f) * M * N * 4.f / 3.16e6f;
+}
+
+// The best tile and split of M x N, at most `best`.
+static MidPlan best_tile(int M, int N, int K, long long ws_bytes, unsigned kind, MidPlan best) {
+  for (int i = 0; i < MID_TILES; ++i) {
+    if (kind == MID_MX_QUANT && MID[i].bn < 128) continue;
+    for (int s = 1; s <= 8; ++s) {
+      if (s > 1 && (N % 4 != 0 || M > 65535 || K / 64 / s < 3 || (long long)s * M * N * 4 > ws_bytes)) break;
+      const float t = mid_time(MID[i], M, N, K, s);
+      if (t < best.us) best = {i, s, t, 0};
+    }
+  }
+  return best;
 }
 
 static MidPlan best_plan(int M, int N, int K, long long ws_bytes, unsigned kind) {
   // the 256 x 256 kernel needs to be 5 % slower to lose: the estimate's error at
   // its sizes (12352 columns of 3000 rows: 257 us, 267 as 256 x 128)
-  MidPlan best{-1, 1, M < 256 || N < 256 ? 1e30f : 0.95f * mid_time(MID[MID_TILES], M, N, K, 1)};
-  for (int i = 0; i < MID_TILES; ++i) {
-    if (kind != MID_BF16 && (i == 3 || (kind == MID_MX_QUANT && MID[i].bn < 128))) continue;
-    for (int s = 1; s <= 8; ++s) {
-      if (s > 1 && ( N % 4 != 0 || M > 65535 || K / 64 / s < 3 || (long long)s * M * N * 4 > ws_bytes)) break;
-      const float t = mid_time(MID[i], M, N, K, s);
-      if (t < best.us) best = {i, s, t};
+  const MidCost& big = MID[MID_TILES];
+  MidPlan best = best_tile(M, N, K, ws_bytes, kind,
+                           {-1, 1, M < 256 || N < 256 ? 1e30f : 0.95f * mid_time(big, M, N, K, 1), 0});
+  // Full rounds of 256 x 256 tiles and the columns that are left on the tile that
+  // suits them: a last round that fills a third of the chip costs a whole one.  us as
+  // the best single tile and in two: 700 x 28672 x 4096 168 : 155, 1700 rows 356 : 320,
+  // 2600 x 12352 x 4096 256 : 222, 2600 x 6400 x 1600 80 : 65.
+  const long long ntm = (M + 255) / 256, tiles = ntm * ((N + 255) / 256);
+  if (kind == MID_BF16 && M >= 256 && tiles > CUS && tiles % CUS != 0) {
+    const int cols = (int)(tiles / CUS * CUS / ntm) * 256;
+    if (cols > 0 && cols < N) {
+      MidPlan two = best_tile(M, N - cols, K, ws_bytes, kind, {-1, 1, 1e30f, 0});
+      two.us += mid_time(big, M, cols, K, 1);
+      two.cols = cols;
+      if (two.us < 0.95f * best.us) best = two;
     }
   }
   return best;
@@ -66,14 +85,17 @@ MidPlan mid_plan(int M, int N, int K, long long ws_bytes, unsigned kind) {
 }
 
 // Decode kernels (gemm_skinny.hip) on more than 64 rows: every 16 rows read the
-// weights once more (from the cache): 4 times the time of the tiles at 256 x 4096 x
-// 18432 (236 us : 53), little more at the smallest (96 x 768 x 768: 5.4 : 5.0), where
-// a folded norm that rides in them saves a launch (3.5 us on the device, 8 where
-// the host bounds such steps).  `frag`: the weight has its fragment-order copy.
+// weights once more (from the cache).  us beside the tiles, a folded norm that rides
+// along (its launch takes 2.5 beside them): 66 rows x 768 x 768 4.1 : 5.3, 192 x 768 x 3072 13.6
+// : 10.3, 66 x 2048 x 7680 25.4 : 15.3, 256 x 4096 x 4096 88 : 18; with the norm 66 x 2304
+// x 768 6.7 : 8.0, 128 rows 8.2 : 8.0, 256 rows 11.0 : 8.1.  `frag`: the weight has its
+// fragment-order copy.
 bool mid_skinny(int M, int N, int K, bool norm, bool frag, long long ws_bytes) {
   if (M <= 64) return true;
   if (M > 256) return false;
-  return 4.2f + (frag ? 2.0e-7f : 3.2e-7f) * N * K * ((M + 15) / 16) < mid_plan(M, N, K, ws_bytes, MID_BF16).us + (norm ? 8.f : 0.f);
+  const float nk = (float)N * K;
+  return 3.8f + nk * 2.f / 4.27e6f + (frag ? 2.1e-7f : 3.2e-7f) * nk * ((M + 15) / 16) <
+         mid_plan(M, N, K, ws_bytes, MID_BF16).us + (norm ? 2.5f : 0.f);
 }
 
 template <class T, MidOut OUT>
@@ -109,7 +131,6 @@ int mid_launch(int tile, const MidArgs& a, const QkvScatter* scat, hipStream_t s
     case 2: return launch<Mid2>(a, scat, st);
     case 3: return launch<Mid3>(a, scat, st);
     case 4: return launch<Mid4>(a, scat, st);
-    case 5: return launch<Mid5>(a, scat, st);
   }
   return -1;
 }

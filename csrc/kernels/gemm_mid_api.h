@@ -27,11 +27,13 @@ struct MidPlan {
   int tile;    // index into the tile table, < 0: the 256 x 256 kernel is the faster one
   int splits;  // workgroups over K
   float us;    // estimated time
+  int cols;    // leading columns as 256 x 256 tiles in a launch of their own, the rest as above (0: none)
 };
 
-// `ws_bytes`: room for parts (0: no split).  `kind`: MID_BF16, or tiles that the MX
-// e4m3 kernel has (K then in 128-byte K-tiles x 64), all or with whole 128 columns.
-enum MidKind : unsigned { MID_BF16 = 0, MID_MX = 1, MID_MX_QUANT = 2 };
+// `ws_bytes`: room for parts (0: no split).  `kind`: bf16, with the columns in one launch
+// or in two, or tiles that the MX e4m3 kernel has (K then in 128-byte K-tiles x 64),
+// all or with whole 128 columns.
+enum MidKind : unsigned { MID_BF16 = 0, MID_BF16_WHOLE = 1, MID_MX = 2, MID_MX_QUANT = 3 };
 MidPlan mid_plan(int M, int N, int K, long long ws_bytes, unsigned kind);
 // Whether M rows still run faster on the decode kernels (`norm`: with a folded norm; `frag`: with the weight's fragment-order copy).
 bool mid_skinny(int M, int N, int K, bool norm, bool frag, long long ws_bytes);

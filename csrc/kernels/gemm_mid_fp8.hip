@@ -214,8 +214,8 @@ int mid8_launch(int tile, const Mid8Args& a, const QkvScatter* scat, hipStream_t
     case 0: return launch<Mid0>(a, scat, st);
     case 1: return launch<Mid1>(a, scat, st);
     case 2: return launch<Mid2>(a, scat, st);
+    case 3: return launch<Mid3>(a, scat, st);
     case 4: return launch<Mid4>(a, scat, st);
-    case 5: return launch<Mid5>(a, scat, st);
   }
   return -1;
 }

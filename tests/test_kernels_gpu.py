@@ -528,7 +528,7 @@ def test_fp8_gemm_tail_split_matches_single_grid(N, K, split, act, res):
     assert err < (3e-2 if split else 8e-2), err
 
 
-MID_TILES = ((64, 64), (128, 64), (128, 128), (192, 128), (256, 128), (128, 256))  # csrc/kernels/gemm_mid.hip MID
+MID_TILES = ((64, 64), (128, 64), (128, 128), (256, 128), (128, 256))  # csrc/kernels/gemm_mid.hip MID
 
 
 def _mid_reference(x, w, b, r, act, norm, consts):
@@ -551,7 +551,7 @@ def _mid_reference(x, w, b, r, act, norm, consts):
     return y if r is None else y + r.float()
 
 
-@pytest.mark.parametrize("tile", range(6))
+@pytest.mark.parametrize("tile", range(5))
 @pytest.mark.parametrize("splits", [1, 3])
 @pytest.mark.parametrize("dm,dn,K", [(1, 36, 192), (0, 0, 448), (-1, -8, 576), (3, 20, 4096)])
 def test_gemm_mid_tiles(tile, splits, dm, dn, K):
@@ -600,6 +600,29 @@ def test_gemm_chosen_tiles(M, N, K, room):
         assert _rel(G.linear(x, w, ws=ws, w_shuf=sh), x.float() @ w.float().t()) < 2.5e-3
 
 
+@pytest.mark.parametrize("M,N,K", [(700, 22064, 768), (700, 22068, 2048), (1600, 12352, 2048)])
+def test_gemm_columns_in_two(M, N, K):
+    """Sizes whose columns are full rounds of 256 x 256 tiles and a rest on smaller ones (whole or
+    split over K): every operand of the rest starts at its column.  Tolerances: test_gemm_mid_tiles."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    g = torch.Generator(device=DEV).manual_seed(M)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    x, w, b, r = rnd(M, K).bfloat16(), (rnd(N, K) * K ** -0.5).bfloat16(), rnd(N), rnd(M, N).bfloat16()
+    ws = torch.zeros((64 << 20) + 4096, dtype=torch.uint8, device=DEV)
+    st, cs = torch.rand(M, 2, device=DEV, generator=g) + 0.5, w.float().sum(1).contiguous()
+    consts = torch.tensor([0.7, 1.3], device=DEV)
+    calls = [(dict(bias=b, act=2, residual=r), b, r, 2, None), (dict(rowstat=st, colsum=cs, bias=b), b, None, 0, (st, cs)),
+             (dict(out_dtype=torch.float32, bias=b), b, None, 0, None), (dict(bias=torch.cat([b, consts]), act=6), b, None, 6, None)]
+    if N % 16 == 0:
+        calls += [(dict(act=3), None, None, 3, None), (dict(act=4), None, None, 4, None)]
+    for kw, bias, res, act, norm in calls:
+        y = G.linear(x, w, ws=ws, **kw)
+        ref = _mid_reference(x, w, bias, res, act, norm, consts)
+        tol = 1e-5 if y.dtype == torch.float32 else 2.5e-3
+        for cols in (slice(0, 64), slice(y.shape[1] - 64, None), slice(None)):
+            assert _rel(y[:, cols], ref[:, cols]) < tol, kw.keys()
+
+
 @pytest.mark.parametrize("B,T,H,Hkv,hd,pos0,S", [(1, 65, 12, 12, 64, 0, 80), (3, 43, 4, 2, 128, 5, 60), (1, 255, 25, 25, 64, 9, 300)])
 def test_qkv_scatter_small_prefill(B, T, H, Hkv, hd, pos0, S):
     """Fewer rows than a 256 x 256 tile: scattered on every small tile == qkv rows + qkv_split."""
@@ -611,7 +634,7 @@ def test_qkv_scatter_small_prefill(B, T, H, Hkv, hd, pos0, S):
     f = G.fold_norm(torch.randn(N, d, device=DEV, generator=g) * 0.05, torch.ones(d, device=DEV), torch.zeros(d, device=DEV),
                     torch.randn(N, device=DEV, generator=g) * 0.02, False, 1e-5, DEV)
     std, pos = torch.empty(B * T, d, device=DEV, dtype=torch.bfloat16), torch.full((B,), pos0, device=DEV, dtype=torch.int32)
-    for tile in range(6):
+    for tile in range(5):
         caches = [torch.zeros(B, Hkv, S, hd, device=DEV).bfloat16() for _ in range(4)]
         q, q2 = (torch.empty(B * H * T * hd, device=DEV, dtype=torch.bfloat16) for _ in range(2))
         G.set_gemm_mid(tile)

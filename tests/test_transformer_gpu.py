@@ -1611,7 +1611,7 @@ def test_fp8_fidelity_vs_unquantised():
     assert r["fp8-e4m3"]["prefill_logits_rel"] < 2 * r["fp8-split"]["prefill_logits_rel"]
 
 
-@pytest.mark.parametrize("tile", [0, 1, 2, 4, 5])
+@pytest.mark.parametrize("tile", range(5))
 @pytest.mark.parametrize("M,N,K", [(256, 256, 64), (257, 300, 200), (383, 520, 1600), (513, 388, 384)])
 def test_gemm_fp8_mx_small_tiles(tile, M, N, K):
     """The MX product on the tiles below 256 x 256, at sizes around their borders:
