@@ -815,7 +815,7 @@ extern "C" int dnn_gemm_set_stream(int on, long long min_bytes, int fold) {
 //   M <= 8     : 1 tile, 4 chunks in flight, 8 waves/WG (within 3% of the best
 //                row-major config on every Llama-3 / GPT-2 XL shape); with the
 //                fragment-order copy (Wsh) the per-class rules below
-//   M <= 16    : wide N (>= 16K): 4 tiles x 2 chunks, 2 waves; else 2 tiles x 2
+//   M <= 16    : N <= 4096: as M <= 8; wide N (>= 16K): 4 tiles x 2 chunks, 2 waves; else 2 tiles x 2
 //                chunks pipelined, 4 waves
 //   M <= 64    : by N class (wide >= 16K / mid / narrow <= 4K): 4 / 2 / 1 column
 //                tiles x 2 chunks, 4 waves (activation re-reads dominate as M
@@ -925,6 +925,15 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
     CFG(1, 1, 4, false, 8);
   }
   if (M <= 16) {
+    // narrow N: one column tile a workgroup, as for M <= 8.  Two put 64 to 128 workgroups
+    // on 256 CUs.  us, 16 rows, two tiles : one: 4096 x 14336 32.3 : 24.2, 4096 x 4096 11.5
+    // : 9.1, 768 x 3072 8.9 : 6.8, 2304 x 768 5.8 : 5.1; row-major 4096 x 14336 50.4 : 33.3,
+    // 2048 x 7680 30.4 : 19.8; e4m3 4096 x 14336 23.9 : 19.0, 1600 x 6400 11.9 : 10.4 (the
+    // last four on 4 waves: 8 are up to 10 % slower there and faster above)
+    if (!FP8 && N <= 4096) CFG(1, 1, 4, false, (W8 || Wsh == nullptr) ? 4 : 8);
+    // wide N in fragment order, K from 2048: 28672 x 4096, 12 rows 45.9 : 40.7, 16 rows
+    // 45.2 : 44.0, 32768 x 4096 49.9 : 46.2 (50257 x 768 the other way, 19.8 : 23.2)
+    if (!FP8 && !W8 && wide && Wsh != nullptr && kbytes >= 4096) CFG(1, 1, 4, false, 4);
     if (wide) CFG(1, 4, 2, false, 2);
     CFG(1, 2, 2, true, 4);
   }

@@ -600,6 +600,27 @@ def test_gemm_chosen_tiles(M, N, K, room):
         assert _rel(G.linear(x, w, ws=ws, w_shuf=sh), x.float() @ w.float().t()) < 2.5e-3
 
 
+@pytest.mark.parametrize("M", [9, 16, 17])
+@pytest.mark.parametrize("N,K", [(20, 64), (4096, 192), (4112, 2048), (16384, 1984), (16400, 2048)])
+def test_gemm_9_to_16_rows(M, N, K):
+    """Either side of the lines of the 9 to 16 row rule: bf16 row-major and in fragment order, e4m3 weights.
+    Tolerances: test_gemm_mid_tiles (the e4m3 product is exact in its weights)."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    from distributed_neural_networks_amd.ops.fp8 import linear_w8, quantize_weight
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x, w = torch.randn(M, K, device=DEV, generator=g).bfloat16(), torch.randn(N, K, device=DEV, generator=g) * K ** -0.5
+    b, r = torch.randn(N, device=DEV, generator=g), torch.randn(M, N, device=DEV, generator=g).bfloat16()
+    wb = w.bfloat16()
+    ref = x.float() @ wb.float().t() + b + r.float()
+    for sh in (None, G.shuffle_weight(wb)):
+        assert _rel(G.linear(x, wb, b, residual=r, w_shuf=sh), ref) < 2.5e-3
+    w8 = quantize_weight(w, DEV)
+    ref8 = x.float() @ (w8.q[:, :K].float() * w8.scale[:, None]).t() + b + r.float()
+    for _ in range(2):
+        assert _rel(linear_w8(x, w8, b, residual=r), ref8) < 2.5e-3
+        G.attach_shuffled(w8)
+
+
 @pytest.mark.parametrize("M,N,K", [(700, 22064, 768), (700, 22068, 2048), (1600, 12352, 2048)])
 def test_gemm_columns_in_two(M, N, K):
     """Sizes whose columns are full rounds of 256 x 256 tiles and a rest on smaller ones (whole or
