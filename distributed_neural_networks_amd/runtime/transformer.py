@@ -549,33 +549,38 @@ class TransformerStage(StageCompute):
             return False
         if self.fp8 and (self.sx8 is None or not F8_.MX_PREFILL):
             return False
-        blocks = []
-        for L in self.layers:
-            for w, bias, colsum, frag in ((L.w_qkv.w, L.w_qkv.bias, L.w_qkv.colsum, L.w_qkv.ws),
-                                          (L.w_o, L.b_o, None, L.w_o_s),
-                                          (L.w_up.w, L.w_up.bias, L.w_up.colsum, L.w_up.ws),
-                                          (L.w_down, L.b_down, None, L.w_down_s)):
-                scale = None
-                if self.fp8:
-                    w, scale, frag = w.q, w.scale, w.shuf
-                blocks += [w.data_ptr(), 0 if scale is None else scale.data_ptr(), 0 if bias is None else
-                           bias.data_ptr(), 0 if colsum is None else colsum.data_ptr(),
-                           0 if frag is None else frag.data_ptr()]
         up = self.layers[0].w_up
-        S = self.kc.shape[3]
-        rc, what = _lib.lib().prefill_blocks(
-            [B, T, self.d, self.H, self.Hkv, self.hd, S, self.buf_f.shape[1], up.w.shape[0],
+        n = [B, T, self.d, self.H, self.Hkv, self.hd, self.kc.shape[3], self.buf_f.shape[1], up.w.shape[0],
              ACT_GELU if self.family == "gpt2" else ACT_SILU_MUL, up.norm, G_.SKINNY_ALWAYS_M, G_.SKINNY_MAX_M,
-             int(self.fp8), int(G_.QKV_SCATTER)],
-            [_lib.ptr(t) for t in (self.buf_h, self.buf_a, self.buf_qkv, self.buf_q, self.buf_att, self.buf_f, self.q8,
-                                   self.sx8, self.q8b, self.sx8b, self.pws, x, self.ones, self.kc[0, b0], self.vc[0, b0],
-                                   pos, self.cos, self.sin, self.s8)],
-            self.eps, 1.0 / math.sqrt(self.hd), self.kc.stride(0) * 2, 0 if self.pws is None else self.pws.nbytes,
-            _lib.stream_ptr(), blocks)
-        if rc == -100:
-            return False
-        _lib.check(rc, what)
+             int(self.fp8), int(G_.QKV_SCATTER)]
+        bufs = [_lib.ptr(t) for t in (self.buf_h, self.buf_a, self.buf_qkv, self.buf_q, self.buf_att, self.buf_f,
+                                      self.q8, self.sx8, self.q8b, self.sx8b, self.pws, x, self.ones, self.kc[0, b0],
+                                      self.vc[0, b0], pos, self.cos, self.sin, self.s8)]
+        block, wsb = self.kc.stride(0) * 2, 0 if self.pws is None else self.pws.nbytes
+        st = _lib.stream_ptr()
+        # the first block by itself: the device works on it while the pointers of the rest are collected
+        for layers in (self.layers[:1], self.layers[1:]):
+            if not layers:
+                break
+            w = [p for L in layers for p in self._block_ptrs(L)]
+            rc, what = _lib.lib().prefill_blocks(n, bufs, self.eps, 1.0 / math.sqrt(self.hd), block, wsb, st, w)
+            if rc == -100:  # the same answer for every block
+                return False
+            _lib.check(rc, what)
+            bufs[11] = bufs[0]  # the next block reads what this one wrote
+            bufs[13], bufs[14] = bufs[13] + block, bufs[14] + block
         return True
+
+    def _block_ptrs(self, L: LayerW) -> List[int]:
+        """Weight, scale, bias, row sums and fragment-order copy of a block's four projections."""
+        q, u, out = L.w_qkv, L.w_up, []
+        for w, bias, colsum, frag in ((q.w, q.bias, q.colsum, q.ws), (L.w_o, L.b_o, None, L.w_o_s),
+                                      (u.w, u.bias, u.colsum, u.ws), (L.w_down, L.b_down, None, L.w_down_s)):
+            scale = None
+            if self.fp8:
+                w, scale, frag = w.q, w.scale, w.shuf
+            out += [0 if t is None else t.data_ptr() for t in (w, scale, bias, colsum, frag)]
+        return out
 
     def forward(self, x: torch.Tensor, out: Optional[torch.Tensor] = None):
         """Full-prefix forward of one request (the reference stage call,
