@@ -172,14 +172,14 @@ __global__ __launch_bounds__(256, 2) void flash_attn_kernel(const bf16_t* __rest
   const int qb = (int)(gridDim.z - 1 - blockIdx.z), hh = blockIdx.x, b = blockIdx.y;
   const int kvh = hh / (H / Hkv);
   const int p0 = pos != nullptr ? pos[b] : 0;
-  const int kv_len = p0 + T;
+  const int kv_len = min(p0 + T, S);  // rows of the cache: none past its end is fetched or counted
   const int qrow0 = qb * FA_QB + wave * 32;            // this wave's first query (chunk-relative)
   const int qrow = qrow0 + r32;                        // this lane's query
   const int q_abs = p0 + min(qrow, T - 1);
   const int wave_qmax = p0 + min(qrow0 + 31, T - 1);   // wave-uniform
   const int wave_qmin = p0 + min(qrow0, T - 1);
   const int blk_qmax = p0 + min(qb * FA_QB + FA_QB - 1, T - 1);
-  const int kv_end = min(min(kv_len, blk_qmax + 1), S);  // never read past the cache
+  const int kv_end = min(kv_len, blk_qmax + 1);
 
   const bf16_t* krow_new = nullptr;  // QKV: this sequence's new-key rows (position p0 + t = row b*T + t)
   const bf16_t* vrow_new = nullptr;

@@ -192,6 +192,36 @@ def test_flash_attn_spike_rescale():
     assert _rel(out, ref) < 2e-2
 
 
+@pytest.mark.parametrize("B,Tn,H,Hkv,hd,pos0,S", [(1, 161, 3, 3, 64, 0, 161), (2, 200, 4, 2, 64, 33, 240), (1, 320, 2, 2, 64, 0, 300),
+                                                  (1, 449, 4, 2, 128, 0, 512), (1, 513, 2, 1, 128, 70, 600)])
+def test_flash_two_key_groups(B, Tn, H, Hkv, hd, pos0, S, monkeypatch):
+    """Every other key block in a group of its own (the default on small grids) against
+    one group: a last round with one block, a causal edge inside a block, a cache that
+    ends first.  The sums differ in their order and in the maximum the probabilities
+    are rounded against: 2^-8 each way, and the result's rounding to bf16."""
+    from distributed_neural_networks_amd.ops import transformer_ops as T
+    g = torch.Generator(device=DEV).manual_seed(Tn)
+    q = torch.randn(B * H * Tn * hd, device=DEV, generator=g).bfloat16()
+    kc, vc = (torch.randn(B, Hkv, S, hd, device=DEV, generator=g).bfloat16() for _ in range(2))
+    qkv = torch.randn(B * Tn, (H + 2 * Hkv) * hd, device=DEV, generator=g).bfloat16()
+    pos = torch.full((B,), pos0, device=DEV, dtype=torch.int32)
+    outs = []
+    for db in (None, "1"):
+        monkeypatch.setenv("DNN_FLASH_DB", db) if db else monkeypatch.delenv("DNN_FLASH_DB", raising=False)
+        k2, v2 = kc.clone(), vc.clone()
+        o, o2 = (torch.full((B * Tn, H * hd), float("nan"), device=DEV, dtype=torch.bfloat16) for _ in range(2))
+        T.flash_attn(q, kc, vc, o, B, Tn, H, Hkv, hd, pos)
+        T.flash_attn_qkv(qkv, k2, v2, o2, B, Tn, H, Hkv, hd, pos)
+        outs.append((o, o2, k2, v2))
+    (a, a2, ka, va), (b, b2, kb, vb) = outs
+    assert torch.equal(ka, kb) and torch.equal(va, vb)
+    for x, y in ((a, b), (a2, b2)):
+        assert torch.isfinite(x).all()
+        # sum of |p v| <= the largest |v|: an absolute bound
+        assert (x.float() - y.float()).abs().max() <= 3 * 2.0 ** -8 * max(vc.abs().max().item(), qkv.abs().max().item())
+        assert _rel(x, y) < 4e-3
+
+
 def _decode_path(monkeypatch, path):
     """'0' / '1': the batched kernel with DPP / MFMA scores; '1p': the one-pass
     kernel, forced onto grids of any size."""
