@@ -151,8 +151,13 @@ __device__ __forceinline__ int k_swz(int key, int chunk) {
 // (profiles/r5_flash_pipe_ab.jsonl): the second accumulator takes the kernel
 // from 144 to 212 VGPRs and three buffers to 60 KB of LDS, i.e. from 3 to 2
 // workgroups per CU — the lost wave per SIMD overlapped the chain better.
-template <int HD, bool QKV = false, bool KV8 = false, bool DB = false, bool PIPE = false>
-__global__ __launch_bounds__(256, 2) void flash_attn_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
+//
+// KS = 2 (DB): two groups of 4 waves take every other key block of the same 128
+// queries into buffers of their own and merge at the end.  A workgroup's blocks are
+// a chain (fetch, barrier, S, softmax, P.V: 1 us at hd 64) that nothing hides where
+// the grid leaves a workgroup a CU: FA_KS_WGS below.
+template <int HD, bool QKV = false, bool KV8 = false, bool DB = false, bool PIPE = false, int KS = 1>
+__global__ __launch_bounds__(256 * KS, 2) void flash_attn_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                                                             const bf16_t* __restrict__ vc, bf16_t* __restrict__ o, int T,
                                                             int H, int Hkv, int S, const int* __restrict__ pos,
                                                             float scale_log2, int ldq = 0,
@@ -161,13 +166,16 @@ __global__ __launch_bounds__(256, 2) void flash_attn_kernel(const bf16_t* __rest
   using SM = FaSmem<HD>;
   // DB: two K/V buffers, one barrier per block (the block after next is staged
   // into the other buffer while this one is read)
-  __shared__ __attribute__((aligned(16))) char smem[SM::TOTAL * (PIPE ? 3 : DB ? 2 : 1)];
-  char* ks = smem;
-  char* vs = smem + SM::K_BYTES;
+  __shared__ __attribute__((aligned(16))) char smem[SM::TOTAL * (PIPE ? 3 : DB ? 2 : 1) * KS];
+  static_assert(KS == 1 || (DB && !PIPE), "key groups have two buffers each");
+  const int kg = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);  // key group
+  char* const buf0 = smem + kg * 2 * SM::TOTAL;
+  char* ks = buf0;
+  char* vs = buf0 + SM::K_BYTES;
   constexpr int NKS = HD / 16;  // k-steps of the QK^T contraction
   constexpr int NDT = HD / 32;  // 32-wide d tiles of O
   constexpr int CH = HD / 8;    // 16-B chunks per row
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
   const int h = lane >> 5, r32 = lane & 31;
   const int qb = (int)(gridDim.z - 1 - blockIdx.z), hh = blockIdx.x, b = blockIdx.y;
   const int kvh = hh / (H / Hkv);
@@ -189,7 +197,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_kernel(const bf16_t* __rest
     if (hh % (H / Hkv) == 0) {  // cache write of rows t in [qb*128, qb*128+128), once per kv head
       bf16_t* kd = kc_out + ((size_t)b * Hkv + kvh) * S * HD;
       bf16_t* vd = vc_out + ((size_t)b * Hkv + kvh) * S * HD;
-      for (int e = tid; e < FA_QB * CH; e += 256) {
+      for (int e = threadIdx.x; e < FA_QB * CH; e += 256 * KS) {
         const int t = qb * FA_QB + e / CH, c = e % CH;
         if (t < T && p0 + t < S) {
           if constexpr (KV8) {
@@ -416,26 +424,51 @@ __global__ __launch_bounds__(256, 2) void flash_attn_kernel(const bf16_t* __rest
       __syncthreads();
     }
   } else {
-    if (kv_end > 0) {
-      fetch(0, pkA, pvA);
+    const int first = kg * FA_KB;
+    constexpr int STEP = KS * FA_KB;
+    if (first < kv_end) {
+      fetch(first, pkA, pvA);
       stage(pkA, pvA);
-      if (FA_KB < kv_end) fetch(FA_KB, pkA, pvA);
+      if (first + STEP < kv_end) fetch(first + STEP, pkA, pvA);
     }
     int buf = 0;
-    for (int kb0 = 0; kb0 < kv_end; kb0 += FA_KB) {
+    for (int kb = 0; kb < kv_end; kb += STEP) {  // as many rounds in every group
+      const int kb0 = kb + first;
       // block kb0 is in buffer `buf` and every wave is done with the other one
       __syncthreads();
-      ks = smem + buf * SM::TOTAL;
+      ks = buf0 + buf * SM::TOTAL;
       vs = ks + SM::K_BYTES;
-      compute(kb0);
-      if (kb0 + FA_KB < kv_end) {
-        ks = smem + (buf ^ 1) * SM::TOTAL;
+      if (KS == 1 || kb0 < kv_end) compute(kb0);
+      if (kb0 + STEP < kv_end) {
+        ks = buf0 + (buf ^ 1) * SM::TOTAL;
         vs = ks + SM::K_BYTES;
         stage(pkA, pvA);
-        if (kb0 + 2 * FA_KB < kv_end) fetch(kb0 + 2 * FA_KB, pkA, pvA);
+        if (kb0 + 2 * STEP < kv_end) fetch(kb0 + 2 * STEP, pkA, pvA);
       }
       buf ^= 1;
     }
+  }
+  if constexpr (KS == 2) {  // group 1 hands (m, l, O) over; a group without a block has m = -inf, l = 0
+    static_assert(4 * (NDT * 16 + 2) * 256 <= SM::TOTAL * 4, "the sums fit the key and value buffers");
+    float* mb = reinterpret_cast<float*>(smem) + wave * (NDT * 16 + 2) * 64 + lane;
+    __syncthreads();
+    if (kg == 1) {
+      mb[0] = m_i;
+      mb[64] = l_i;
+#pragma unroll
+      for (int i = 0; i < NDT; ++i)
+#pragma unroll
+        for (int g = 0; g < 16; ++g) mb[(2 + i * 16 + g) * 64] = oacc[i][g];
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    const float m1 = mb[0], m = fmax_nan(m_i, m1), mu = m == -INFINITY ? 0.f : m;
+    const float f0 = __builtin_amdgcn_exp2f(m_i - mu), f1 = __builtin_amdgcn_exp2f(m1 - mu);
+    l_i = l_i * f0 + mb[64] * f1;
+#pragma unroll
+    for (int i = 0; i < NDT; ++i)
+#pragma unroll
+      for (int g = 0; g < 16; ++g) oacc[i][g] = oacc[i][g] * f0 + mb[(2 + i * 16 + g) * 64] * f1;
   }
   // ---- normalise + store: lane = query, regs = d ----
   if (qrow < T) {
@@ -919,6 +952,15 @@ extern "C" int dnn_qkv_split(const void* qkv, void* q, void* kc, void* vc, int B
   return (int)hipGetLastError();
 }
 
+// Two key groups: at most one workgroup a CU and a chain of a few blocks.  us, one :
+// two groups: GPT-2 200 tokens 7.2 : 6.6, 3 x 357 10.0 : 8.8, 960 19.2 : 14.7, 4 x 600
+// 14.6 : 11.8, but 100 5.3 : 5.7; XL 8 x 256 (400 workgroups) 9.4 : 12.9; Llama-3 700
+// 21.4 : 19.2, 1000 29.6 : 26.1, 300 11.2 : 11.5.
+constexpr int FA_KS_WGS = 256;
+template <int HD>
+static bool flash_two_groups(long wgs, int T) {
+  return wgs <= FA_KS_WGS && T > (HD == 64 ? 160 : 448);
+}
 template <int HD, bool QKV, bool KV8>
 static void launch_flash(dim3 grid, hipStream_t st, const bf16_t* q, const bf16_t* kc, const bf16_t* vc, bf16_t* o,
                          int T, int H, int Hkv, int S, const int* pos, float sl2, int ldq, bf16_t* kco, bf16_t* vco) {
@@ -934,7 +976,11 @@ static void launch_flash(dim3 grid, hipStream_t st, const bf16_t* q, const bf16_
       return;
     }
   }
-  if (e == nullptr || atoi(e) != 0)
+  const long wgs = (long)grid.x * grid.y * grid.z;
+  if (e == nullptr && flash_two_groups<HD>(wgs, T))  // DNN_FLASH_DB pins a one-group variant
+    hipLaunchKernelGGL((flash_attn_kernel<HD, QKV, KV8, true, false, 2>), grid, dim3(512), 0, st, q, kc, vc, o, T, H,
+                       Hkv, S, pos, sl2, ldq, kco, vco);
+  else if (e == nullptr || atoi(e) != 0)
     hipLaunchKernelGGL((flash_attn_kernel<HD, QKV, KV8, true>), grid, dim3(256), 0, st, q, kc, vc, o, T, H, Hkv, S,
                        pos, sl2, ldq, kco, vco);
   else
