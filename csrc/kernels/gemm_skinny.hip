@@ -29,6 +29,7 @@
 // and so the step time halve.  KS is chosen on the host so that N/16 x KS waves
 // cover the CUs.
 #include <algorithm>
+#include <cstdlib>
 #include "gemm_epilogue.h"
 #include "gemm_head.h"
 #include "gemm_oneshot.h"
@@ -115,24 +116,23 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const uint8_t* __restr
   // wave index via readfirstlane: the K-slice bounds and the surplus-chunk tests
   // below are then scalar (s_cbranch), not exec-masked VALU branches
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), KS = blockDim.x >> 6;
-  // MS (M split): one workgroup per (column tile, 16-row M tile), so M = 32..64
-  // runs 2-4x the workgroups (narrow N, e.g. GPT-2's 768-wide projections, has
+  // MS (M split): one workgroup per (column tile, MT 16-row M tiles), so M = 32..64
+  // runs 2-4x the workgroups (MT = 1) (narrow N, e.g. GPT-2's 768-wide projections, has
   // too few column tiles to fill 256 CUs otherwise).  The M tiles of a column
   // tile are consecutive logical ids on one XCD, so its weight slice is read
   // from HBM once and re-read from that XCD's L2.
   int n0;
   if constexpr (MS) {
-    static_assert(MT == 1, "MS: one M tile per workgroup");
-    const int mtiles = (M + 15) >> 4;
+    const int mtiles = (M + 16 * MT - 1) / (16 * MT);
     const int lgc = xcd_remap(blockIdx.x, gridDim.x);
-    const int mo = (lgc % mtiles) * 16;
+    const int mo = (lgc % mtiles) * (16 * MT);
     n0 = (lgc / mtiles) * (16 * NT);
     A += (size_t)mo * lda_b;
     if (sa != nullptr) sa += mo;
     Cv = reinterpret_cast<char*>(Cv) + (size_t)mo * ldc * (OUT_F32 ? 4 : 2);
     if (R != nullptr) R += (size_t)mo * ldr;
     if (rs_out != nullptr) rs_out += (size_t)mo * rs_ld;
-    M = min(16, M - mo);
+    M = min(16 * MT, M - mo);
   } else {
     n0 = blockIdx.x * (16 * NT);
   }
@@ -839,7 +839,7 @@ template <int ACT, bool F32, bool FP8, int MT, int NT, int U, bool PIPE, int NOR
 static int launch_skinny_cfg(const void* A, int lda_b, const float* sa, const void* W, int ldw_b, const float* sw,
                              void* C, int ldc, const float* bias, const void* R, int ldr, int M, int N, int kbytes,
                              int ks, const float* colsum, float eps, hipStream_t st, const void* Wsh) {
-  const int groups = (N + 16 * NT - 1) / (16 * NT) * (MS ? (M + 15) / 16 : 1);
+  const int groups = (N + 16 * NT - 1) / (16 * NT) * (MS ? (M + 16 * MT - 1) / (16 * MT) : 1);
   while (ks > 1 && kbytes / 64 < ks) ks >>= 1;
   size_t smem = (size_t)ks * NT * MT * 64 * sizeof(f32x4);
   if (NORM != NORM_NONE) smem += (size_t)ks * MT * 2 * 16 * sizeof(float);
@@ -888,6 +888,9 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
   return launch_skinny_cfg<ACT, F32, FP8, 1, NTV, UV, PV, NORM, W8, true>(A, lda_b, sa, W, ldw_b, sw, C, ldc, bias, \
                                                                            R, ldr, M, N, kbytes, KSV, colsum, eps, st, \
                                                                            Wsh)
+#define CFG_MM(MTV, NTV)                                                                                             \
+  return launch_skinny_cfg<ACT, F32, FP8, MTV, NTV, 2, false, NORM, W8, true>(A, lda_b, sa, W, ldw_b, sw, C, ldc, bias, \
+                                                                             R, ldr, M, N, kbytes, 4, colsum, eps, st, Wsh)
   const bool pinned = g_skinny_pin.id != 0 && !FP8 && !W8 && Wsh != nullptr && M > 16 && M <= 64 &&
                       (g_skinny_pin.n == 0 || g_skinny_pin.n == N) &&
                       (g_skinny_pin.k == 0 || g_skinny_pin.k * 2 == kbytes);
@@ -903,11 +906,19 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
       default: break;
     }
   }
-  // medium M (64, 256], decode of larger batches: always the M split, one
-  // 16-row tile per workgroup; the weight slice of a column tile is re-read
+  // medium M (64, 256], decode of larger batches: always the M split; the weight slice of a column tile is re-read
   // from its XCD's L2 by the M tiles (the 128^2 GEMM would launch only a
   // handful of tiles at these shapes)
   if (M > 64) {
+    // e4m3 weights (bf16 has the tiles of gemm_mid.h here): 64 rows a workgroup, so the
+    // weights and their conversion serve four M tiles.  us, 16 : 64 rows: 256 x 4096 x
+    // 14336 126 : 62, 256 x 6400 x 1600 34.7 : 23.7, 190 x 4800 x 1600 22.5 : 14.9, 100 x 4096 x 4096
+    // 22.3 : 21.9, but 66 x 4096 x 4096 17.9 : 21.9; narrow N on 2 column tiles 256 x 1600 x
+    // 6400 32.5 : 28.9, 190 rows 25.6 : 28.6
+    if constexpr (W8) {
+      if (N >= 4096 && M > 80) CFG_MM(4, 4);
+      if (N < 4096 && N > 1024 && M > 208) CFG_MM(4, 2);
+    }
     if (N <= 1024) CFG_MS(1, 4, false, 4);
     CFG_MS(2, 2, false, 4);
   }
@@ -966,6 +977,7 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
     if (N <= 2048 || (W8 && N <= 4096)) CFG_MS(2, 2, true, 4);
   }
 #undef CFG_MS
+#undef CFG_MM
   const bool deep = kbytes >= 16384;
   const bool narrow = N <= 4096;
   if (M <= 32) {

@@ -621,6 +621,27 @@ def test_gemm_9_to_16_rows(M, N, K):
         G.attach_shuffled(w8)
 
 
+@pytest.mark.parametrize("M", [80, 81, 129, 193, 208, 209, 256])
+@pytest.mark.parametrize("N,K", [(1040, 64), (4092, 192), (4112, 448)])
+def test_gemm_w8_65_to_256_rows(M, N, K):
+    """Either side of the lines to 64 rows a workgroup, a last group of one row, columns cut
+    inside a tile: e4m3 weights with bias and residual, GELU behind a folded norm, row-major
+    and in fragment order.  Tolerances: test_gemm_9_to_16_rows."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    from distributed_neural_networks_amd.ops.fp8 import linear_w8, quantize_weight
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x, w = torch.randn(M, K, device=DEV, generator=g).bfloat16(), torch.randn(N, K, device=DEV, generator=g) * K ** -0.5
+    b, r = torch.randn(N, device=DEV, generator=g), torch.randn(M, N, device=DEV, generator=g).bfloat16()
+    w8 = quantize_weight(w, DEV)
+    wd = w8.q[:, :K].float() * w8.scale[:, None]
+    xn = torch.nn.functional.layer_norm(x.float(), (K,), eps=1e-5)
+    ref, gelu = x.float() @ wd.t() + b + r.float(), torch.nn.functional.gelu(xn @ wd.t() + b)
+    for _ in range(2):
+        assert _rel(linear_w8(x, w8, b, residual=r), ref) < 2.5e-3
+        assert _rel(linear_w8(x, w8, b, act=2, norm=2, colsum=wd.sum(1), eps=1e-5), gelu) < 2.5e-3
+        G.attach_shuffled(w8)
+
+
 @pytest.mark.parametrize("M,N,K", [(700, 22064, 768), (700, 22068, 2048), (1600, 12352, 2048)])
 def test_gemm_columns_in_two(M, N, K):
     """Sizes whose columns are full rounds of 256 x 256 tiles and a rest on smaller ones (whole or
