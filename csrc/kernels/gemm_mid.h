@@ -279,7 +279,7 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvS
   constexpr int I = T::I, J = T::J;
   // S * STAGE bytes, given at launch: with the size in the kernel the compiler sees one
   // wave per SIMD and moves accumulators of the four-wave tiles to AGPRs and back in
-  // the loop (192 x 128 at 700 x 6144 x 4096: 47 -> 78 us)
+  // the loop (a tile of 192 x 128 rows at 700 x 6144 x 4096: 47 -> 78 us)
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int M = p.M, N = p.N;

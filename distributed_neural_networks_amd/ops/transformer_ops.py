@@ -181,9 +181,11 @@ def decode_splits(S: int, B: int, Hkv: int, G: int = 1) -> int:
     split per 256 keys of cache capacity.  Each split takes
     ``ceil(len/splits)`` of the *runtime* length, so short contexts stay
     balanced; with one split the kernel writes the output itself (no combine).
-    Long contexts: a split keeps its G x chunk scores in LDS (160 KiB), so the
-    split count never drops below ceil(S / floor(40960 / G)) (14 for a 128 K-token
-    Llama-3 cache, G = 4), whatever the batch."""
+    The kernel for bf16 caches takes fewer where they do not pay (attention.hip
+    attn_stream_launch); the workspace is sized for all.  Long contexts: a split of the
+    e4m3 kernel keeps its G x chunk scores in LDS (160 KiB), so the split count never
+    drops below ceil(S / floor(40960 / G)) (14 for a 128 K-token Llama-3 cache, G = 4),
+    whatever the batch."""
     lds_min = max(1, -(-S // (DEC_LDS_SCORES // max(1, G))))  # ceil(S/splits) * G <= 40960
     if os.environ.get("DNN_DECODE_SPLITS"):  # A/B override
         return max(lds_min, int(os.environ["DNN_DECODE_SPLITS"]))
