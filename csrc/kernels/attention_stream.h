@@ -213,7 +213,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
           s[t][r] = t * 16 + r < last ? s[t][r] * scale_log2 : -INFINITY;
           mx = fmaxf(mx, s[t][r]);
         }
-      const float mn = fmaxf(m, max_over_quarters(mx));
+      const float mn = fmaxf(m, max_over_quarters(mx)), base = mn == -INFINITY ? 0.f : mn;  // no finite score yet: all 0
       const float al = mn == m ? 1.f : __builtin_amdgcn_exp2f(m - mn);
       m = mn;
       float sum = 0.f;
@@ -221,7 +221,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
       for (int t = 0; t < NT16; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float p = __builtin_amdgcn_exp2f(s[t][r] - mn);
+          const float p = __builtin_amdgcn_exp2f(s[t][r] - base);
           sum += p;
           const int row = t * 16 + c4 * 4 + r, u = row / RG;
           if (hj < G) pl[wave][((row % RG) * (U / 2) + (u >> 1)) * G * 2 + hj * 2 + (u & 1)] = f2bf(p);
@@ -266,12 +266,12 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
 #pragma unroll
       for (int u = 0; u < U; ++u)
         if (u * RG < last) mn = fmaxf(mn, p[u]);
-      const float al = mn == m ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+      const float al = mn == m ? 1.f : __builtin_amdgcn_exp2f(m - mn), base = mn == -INFINITY ? 0.f : mn;
       m = mn;
       float sum = 0.f;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        p[u] = u * RG < last ? __builtin_amdgcn_exp2f(p[u] - mn) : 0.f;
+        p[u] = u * RG < last ? __builtin_amdgcn_exp2f(p[u] - base) : 0.f;
         sum += p[u];
       }
       l = l * al + sum;

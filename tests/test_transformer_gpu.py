@@ -320,6 +320,31 @@ def test_attn_decode_stream(H, Hkv, hd, B, S, rope):
         assert ((out[b].double() - ref).abs() <= (2.0 ** -7 + 2.0 ** -12 + tol) * mag).all(), b
 
 
+@pytest.mark.parametrize("H,Hkv,hd", [(3, 3, 64), (8, 2, 64), (2, 2, 128), (8, 2, 128)])
+@pytest.mark.parametrize("S,keys", [(40, (0, 3)), (300, (0, 256)), (300, (0, 299)), (2000, (100, 1999)), (40, (39, 40))])
+def test_attn_decode_infinite_scores(H, Hkv, hd, S, keys):
+    """Keys with a score of -inf have probability 0, also where a wave's first keys, a block or
+    a split hold no others.  Bound: test_attn_decode_stream."""
+    from distributed_neural_networks_amd.ops import transformer_ops as T
+    g = torch.Generator(device=DEV).manual_seed(S + H)
+    B, G, (k0, k1) = 2, H // Hkv, keys
+    q, kc, vc = (torch.randn(B, n, hd, device=DEV, generator=g).bfloat16() for n in (H, Hkv * S, Hkv * S))
+    kc, vc = kc.view(B, Hkv, S, hd), vc.view(B, Hkv, S, hd)
+    q[..., 5] = 1.0
+    kc[:, :, k0:k1, 5] = float("-inf")
+    splits = T.decode_splits(S, B, Hkv, G)
+    ws = torch.full((B * Hkv * splits * G * (hd + 2),), float("nan"), device=DEV)
+    out = torch.full((B, H * hd), float("nan"), device=DEV, dtype=torch.bfloat16)
+    lens = torch.full((B,), S, dtype=torch.int32, device=DEV)
+    T.attn_decode(q, kc, vc, out, B, H, Hkv, hd, lens, ws, splits)
+    for b in range(B):
+        kk, vv = (t[b].double().repeat_interleave(G, 0) for t in (kc, vc))
+        p = (torch.matmul(kk, q[b].double()[..., None])[..., 0] / math.sqrt(hd)).softmax(-1)
+        assert (p[:, k0:k1] == 0).all()
+        ref, mag = (torch.matmul(p[:, None], t)[:, 0].reshape(-1) for t in (vv, vv.abs()))
+        assert ((out[b].double() - ref).abs() <= (2.0 ** -7 + 2.0 ** -12) * mag).all()
+
+
 @pytest.mark.parametrize("B,H,Hkv,hd,S,rope,ns", [(32, 32, 8, 128, 600, True, 0), (64, 12, 12, 64, 560, False, 0),
                                                   (64, 25, 25, 64, 1300, False, 0), (32, 32, 8, 128, 600, True, 2),
                                                   (32, 32, 8, 128, 600, True, 3), (64, 12, 12, 64, 560, False, 3)])
