@@ -287,8 +287,8 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
       else
         nv = i32x4{(int)nvp[0], (int)nvp[1], (int)nvp[2], (int)nvp[3]};
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (blk * R + u * RG + grp == knew) vr[u] = nv;
+      for (int u = 0; u < U; ++u)  // and past it (knew = n - 1): copies of the row as a slot's last owner left it
+        if (blk * R + u * RG + grp >= knew) vr[u] = nv;
     }
 #pragma unroll
     for (int u = 0; u < U; u += 2) {

@@ -345,6 +345,28 @@ def test_attn_decode_infinite_scores(H, Hkv, hd, S, keys):
         assert ((out[b].double() - ref).abs() <= (2.0 ** -7 + 2.0 ** -12) * mag).all()
 
 
+@pytest.mark.parametrize("H,Hkv,hd", [(3, 3, 64), (8, 2, 64), (2, 2, 128), (8, 2, 128), (16, 2, 128)])
+@pytest.mark.parametrize("S,p", [(40, 0), (40, 7), (300, 128), (300, 298), (2000, 1500)])
+def test_attn_decode_rows_not_written_yet(H, Hkv, hd, S, p):
+    """What the cache holds at the new token's row and after it (NaN here, of the slot's last
+    owner) is never part of a result: the same bits as with zeros there."""
+    from distributed_neural_networks_amd.ops import transformer_ops as T
+    g = torch.Generator(device=DEV).manual_seed(S + p)
+    B, G = 2, H // Hkv
+    kc, vc = (torch.randn(B, Hkv, S, hd, device=DEV, generator=g).bfloat16() for _ in range(2))
+    qkv = torch.randn(B, (H + 2 * Hkv) * hd, device=DEV, generator=g).bfloat16()
+    pos = torch.full((B,), p, dtype=torch.int32, device=DEV)
+    splits = T.decode_splits(S, B, Hkv, G)
+    ws, outs = torch.empty(B * Hkv * splits * G * (hd + 2), device=DEV), []
+    for fill in (0.0, float("nan"), float("inf")):
+        k, v = kc.clone(), vc.clone()
+        k[:, :, p:], v[:, :, p:] = fill, fill
+        outs.append(torch.empty(B, H * hd, device=DEV, dtype=torch.bfloat16))
+        T.attn_decode_qkv(qkv, k, v, outs[-1], B, H, Hkv, hd, pos, ws, splits)
+        assert torch.equal(v[:, :, p].reshape(B, -1), qkv[:, (H + Hkv) * hd:])
+    assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 @pytest.mark.parametrize("B,H,Hkv,hd,S,rope,ns", [(32, 32, 8, 128, 600, True, 0), (64, 12, 12, 64, 560, False, 0),
                                                   (64, 25, 25, 64, 1300, False, 0), (32, 32, 8, 128, 600, True, 2),
                                                   (32, 32, 8, 128, 600, True, 3), (64, 12, 12, 64, 560, False, 3)])
