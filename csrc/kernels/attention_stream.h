@@ -22,6 +22,8 @@
 //    128 dims and 4 heads against 250), one softmax a wave, and its probabilities
 //    reach the row layout as bf16 pairs through 64 B of LDS a row group, private to
 //    the wave.
+typedef uint16_t u16x2v __attribute__((ext_vector_type(2)));
+
 __device__ __forceinline__ float max_over_quarters(float v) {  // lanes l, l ^ 16, l ^ 32, l ^ 48
   const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
@@ -227,13 +229,16 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
           if (hj < G) pl[wave][((row % RG) * (U / 2) + (u >> 1)) * G * 2 + hj * 2 + (u & 1)] = f2bf(p);
         }
       l = l * al + sum;
-      __builtin_amdgcn_wave_barrier();
+      // other lanes read what this one stored: the fence keeps the order (a wave's LDS
+      // operations run in it), the vector type lets 16-bit stores be read in pairs
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
       for (int w = 0; w < U / 2; ++w)
 #pragma unroll
         for (int g = 0; g < G; ++g)
-          pp[w][g] = *reinterpret_cast<const uint32_t*>(&pl[wave][((grp * (U / 2) + w) * G + g) * 2]);
-      __builtin_amdgcn_wave_barrier();
+          pp[w][g] = __builtin_bit_cast(
+              uint32_t, *reinterpret_cast<const u16x2v*>(&pl[wave][((grp * (U / 2) + w) * G + g) * 2]));
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       if (!__all(al == 1.f)) {
 #pragma unroll
         for (int g = 0; g < G; ++g) {
