@@ -18,6 +18,7 @@ ACTS_GLU = (ACT_SILU_MUL, ACT_GELU_TANH_MUL, ACT_CLAMP_MUL)  # packed gate|up we
 SKINNY_MAX_M = 256
 
 
+ROW_STATS_MAX_K = 8192  # widest row of transformer_ops.row_stats
 SKINNY_ALWAYS_M = 64  # bf16: rows up to which the skinny kernels always run (gemm_bf16.hip g_skinny_max_m)
 
 
@@ -34,6 +35,19 @@ def skinny_rows(M: int, N: int, w8: bool = False, K: int = 0, norm: bool = False
     if M <= SKINNY_ALWAYS_M or M > SKINNY_MAX_M:
         return M <= SKINNY_ALWAYS_M
     return _is_skinny(M, N, K, norm, frag, 0 if ws is None else ws.nbytes)
+
+
+def _norm_skinny(x: torch.Tensor, f: "FoldedLinear", act: int, buffers: bool, ws: Optional[torch.Tensor] = None) -> bool:
+    """``skinny_rows`` of a folded norm with bf16 weights, where both sides can take it.
+    Up to 191 tiles of 128 x 128 (65 to 256 rows) what the tile kernels cannot take runs on
+    the decode kernels -- no ``buffers``, K not of whole 64s, rows wider than the statistics
+    kernel's; beyond, an activation that the decode kernels lack runs on tiles.  What a
+    call may bring then does not depend on the estimate."""
+    (M, K), N = x.shape, f.w.shape[0]
+    few = M <= SKINNY_MAX_M and -(-M // 128) * -(-N // 128) < 192
+    if skinny_rows(M, N, False, K, True, f.ws is not None, ws):
+        return few or M <= SKINNY_ALWAYS_M or act in SKINNY_NORM_ACTS[f.norm]
+    return few and (not buffers or K % 64 != 0 or K > ROW_STATS_MAX_K)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -246,6 +260,7 @@ def pack_gate_up(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
 
 
 NORM_RMS, NORM_LN = 1, 2
+SKINNY_NORM_ACTS = {NORM_RMS: (ACT_NONE, ACT_SILU_MUL), NORM_LN: (ACT_NONE, ACT_GELU)}  # dnn_gemm_skinny_norm
 FOLD_NORM_PREFILL = True  # prefill (non-skinny) folded norms: row statistics + GEMM epilogue (A/B switch)
 
 
@@ -312,9 +327,10 @@ def linear_norm(x: torch.Tensor, f: FoldedLinear, act=None, residual: Optional[t
     N = f.w.shape[0]
     if (not w8 and f.w.shape[1] != K) or x.dtype != torch.bfloat16 or x.stride(1) != 1:
         raise ValueError(f"linear_norm: x {tuple(x.shape)} {x.dtype} vs w {tuple(f.w.shape)}")
-    if not skinny_rows(M, N, w8, K, True, f.ws is not None, ws):
+    buffers = std_buf is not None and ones is not None
+    if not (skinny_rows(M, N, True) if w8 else _norm_skinny(x, f, a, buffers, ws)):
         from .transformer_ops import layernorm, layernorm_q8
-        if std_buf is None or ones is None:
+        if not buffers:
             raise ValueError("linear_norm: large M needs std_buf and ones")
         if w8 and q8 is not None and sx is not None and fp8_mx_ok(M, N, f.w):
             # standardise + MX-quantise in one pass (e8m0 per 128 columns); the
@@ -389,7 +405,8 @@ def qkv_scatter_norm(x: torch.Tensor, f: FoldedLinear, std_buf: torch.Tensor, q:
         return False
     M, K = x.shape
     N = f.w.shape[0]
-    if M != B * T or N != (H + 2 * Hkv) * hd or skinny_rows(M, N, w8, K, True, w8 or f.ws is not None) or x.stride(1) != 1:
+    if M != B * T or N != (H + 2 * Hkv) * hd or x.stride(1) != 1 or (
+            skinny_rows(M, N, True) if w8 else _norm_skinny(x, f, ACT_NONE, True)):
         return False
     if not (kc.is_contiguous() and vc.is_contiguous()) or q.numel() < M * H * hd or pos.dtype != torch.int32:
         return False

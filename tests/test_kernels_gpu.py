@@ -665,6 +665,34 @@ def test_gemm_columns_in_two(M, N, K):
             assert _rel(y[:, cols], ref[:, cols]) < tol, kw.keys()
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 2304, 768), (200, 4096, 4096), (256, 768, 3072), (128, 24448, 64), (200, 6144, 160),
+                                   (256, 4096, 1056), (256, 2048, 8224), (256, 2048, 8256), (65, 24576, 64)])
+@pytest.mark.parametrize("buffers", [False, True])
+def test_linear_norm_65_to_256_rows(M, N, K, buffers):
+    """Up to 191 tiles of 128 x 128 a folded norm runs on the decode kernels where the tiles cannot take it: without
+    buffers, K of whole 32s, rows wider than the statistics kernel's; and a scatter says that it does not apply.
+    Tolerance: bf16 products with fp32 sums and the result's rounding, the norm off by its rounding in fp32."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    x = torch.randn(M, K, device=DEV, generator=g).bfloat16()
+    f = G.fold_norm(torch.randn(N, K, device=DEV, generator=g) * K ** -0.5, torch.ones(K, device=DEV), torch.zeros(K, device=DEV),
+                    torch.randn(N, device=DEV, generator=g), False, 1e-5, DEV)
+    kw = dict(std_buf=torch.empty(M, K, device=DEV, dtype=torch.bfloat16), ones=torch.ones(K, device=DEV)) if buffers else {}
+    ref = torch.nn.functional.layer_norm(x.float(), (K,), eps=1e-5) @ f.w.float().t() + f.bias
+    for ws in (None, G.shuffle_weight(f.w)):
+        f.ws = ws
+        if not buffers and -(-M // 128) * -(-N // 128) >= 192:
+            continue
+        assert _rel(G.linear_norm(x, f, **kw), ref) < 4e-3
+        if buffers and -(-M // 128) * -(-N // 128) >= 192:  # an activation that only the tiles have
+            assert _rel(G.linear_norm(x, f, act="relu", **kw), torch.relu(ref)) < 4e-3
+    if buffers and (K % 64 or K > 8192):
+        q, cache = torch.empty(M * N, device=DEV, dtype=torch.bfloat16), torch.empty(1, 1, M, 16, device=DEV, dtype=torch.bfloat16)
+        H = N // 16 - 2
+        assert not G.qkv_scatter_norm(x, f, kw["std_buf"], q, cache, cache.clone(), torch.zeros(1, device=DEV, dtype=torch.int32), 1, M,
+                                      H, 1, 16)
+
+
 @pytest.mark.parametrize("B,T,H,Hkv,hd,pos0,S", [(1, 65, 12, 12, 64, 0, 80), (3, 43, 4, 2, 128, 5, 60), (1, 255, 25, 25, 64, 9, 300)])
 def test_qkv_scatter_small_prefill(B, T, H, Hkv, hd, pos0, S):
     """Fewer rows than a 256 x 256 tile: scattered on every small tile == qkv rows + qkv_split."""
