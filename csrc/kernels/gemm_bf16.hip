@@ -510,6 +510,11 @@ extern "C" int dnn_gemm_set_half_cost(float c) {
   return 0;
 }
 
+// Rows that 16-byte LDS-DMA may fetch.
+static bool dma_rows(const void* A, int lda, const void* W, int ldw) {
+  return (((uintptr_t)A | (uintptr_t)W) & 15) == 0 && lda % 8 == 0 && ldw % 8 == 0;
+}
+
 template <int ACT, bool F32>
 static int launch_gemm(const void* A, int lda, const void* W, int ldw, void* C, int ldc, const float* bias,
                         const void* R, int ldr, int M, int N, int K, hipStream_t st, const void* Wsh,
@@ -519,14 +524,19 @@ static int launch_gemm(const void* A, int lda, const void* W, int ldw, void* C, 
   // itself, dnn_gemm_skinny_norm
   const long long part_bytes = mid_ws(ws, ws_bytes);
   const bool pinned = g_gemm_tile != 0 || g_mid_tile >= 0;
-  if (rowstat == nullptr && (M <= g_skinny_max_m || (M > 64 && !pinned && mid_skinny(M, N, K, false, Wsh != nullptr, part_bytes)))) {
+  // up to 256 rows what the small tiles cannot stage (dma_rows) goes to the decode kernels, whose loads are plain
+  const bool narrow = lda < 1 << 23 && ldw < 1 << 23;  // the small tiles address a tile's rows with 32 bits
+  if (rowstat == nullptr &&
+      (M <= g_skinny_max_m || (M > 64 && M <= 256 && !pinned &&
+                               (!narrow || !dma_rows(A, lda, W, ldw) ||
+                                mid_skinny(M, N, K, false, Wsh != nullptr, part_bytes))))) {
     return dnn_gemm_skinny(A, lda, nullptr, W, ldw, nullptr, C, ldc, bias, R, ldr, M, N, K, ACT, F32 ? 1 : 0, 0, st, Wsh,
                            ws, ws_bytes);
   }
   // Tiles of gemm_mid.h, or 256 x 256 (and its tail split below) by estimated time
   const int tiles256 = ((M + BG_M - 1) / BG_M) * ((N + BG_N - 1) / BG_N);
   MidPlan plan{-1, 1, 0.f, 0};
-  if (lda >= 1 << 23 || ldw >= 1 << 23) {  // the small tiles address a tile's rows with 32 bits
+  if (!narrow) {
   } else if (g_mid_tile >= 0) plan = {g_mid_tile, (long long)g_mid_splits * M * N * 4 <= part_bytes ? g_mid_splits : 1, 0.f, 0};
   else if (g_gemm_tile == 128) plan.tile = 2;
   else if (g_gemm_tile == 0 && (is_glu(ACT) || has_consts(ACT) || tail_split_cols(M, N) == 0))
@@ -638,7 +648,7 @@ extern "C" int dnn_gemm_bf16_qkv_scatter(const void* A, int lda, const void* W, 
                                          hipStream_t st) {
   const int M = B * T, N = (H + 2 * Hkv) * hd;
   if (K % 64 != 0 || M <= 0 || hd % 8 != 0 || (colsum != nullptr && rowstat == nullptr)) return -1;
-  if (N % 32 != 0 || ((uintptr_t)bias & 15) != 0) return -3;
+  if (N % 32 != 0 || ((uintptr_t)bias & 15) != 0 || (M < 256 && !dma_rows(A, lda, W, ldw))) return -3;
   const int tiles = ((M + BG_M - 1) / BG_M) * ((N + BG_N - 1) / BG_N);
   if ((hd & (hd - 1)) != 0 || M >= (1 << 24)) return -3;
   QkvScatter sc{(bf16_t*)q, (bf16_t*)kc, (bf16_t*)vc, pos, T, H, Hkv, __builtin_ctz(hd), S, 1.0f / (float)T};

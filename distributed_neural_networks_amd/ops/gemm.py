@@ -41,13 +41,15 @@ def _norm_skinny(x: torch.Tensor, f: "FoldedLinear", act: int, buffers: bool, ws
     """``skinny_rows`` of a folded norm with bf16 weights, where both sides can take it.
     Up to 191 tiles of 128 x 128 (65 to 256 rows) what the tile kernels cannot take runs on
     the decode kernels -- no ``buffers``, K not of whole 64s, rows wider than the statistics
-    kernel's; beyond, an activation that the decode kernels lack runs on tiles.  What a
-    call may bring then does not depend on the estimate."""
+    kernel's, rows that 16-byte LDS-DMA does not fetch; beyond, an activation that the
+    decode kernels lack runs on tiles.  What a call may bring then does not depend on the
+    estimate."""
     (M, K), N = x.shape, f.w.shape[0]
     few = M <= SKINNY_MAX_M and -(-M // 128) * -(-N // 128) < 192
     if skinny_rows(M, N, False, K, True, f.ws is not None, ws):
         return few or M <= SKINNY_ALWAYS_M or act in SKINNY_NORM_ACTS[f.norm]
-    return few and (not buffers or K % 64 != 0 or K > ROW_STATS_MAX_K)
+    return few and (not buffers or K % 64 != 0 or K > ROW_STATS_MAX_K or
+                    (x.data_ptr() | f.w.data_ptr() | 2 * x.stride(0) | 2 * f.w.stride(0)) % 16 != 0)
 
 
 @functools.lru_cache(maxsize=4096)

@@ -545,7 +545,8 @@ class TransformerStage(StageCompute):
         False, with nothing launched, where the loop has to issue them: e4m3 caches,
         split activations, a switch off its default, input the loop's checks are for."""
         if not (self.layers and self.fuse_norm and G_.FOLD_NORM_PREFILL and self.kc.dtype == torch.bfloat16 and self.hd in (64, 128)
-                and pos.dtype == torch.int32 and x.dtype == torch.bfloat16 and x.is_contiguous()) or _lib.DEBUG_SYNC:
+                and pos.dtype == torch.int32 and x.dtype == torch.bfloat16 and x.is_contiguous()
+                and x.data_ptr() % 16 == 0) or _lib.DEBUG_SYNC:
             return False
         if self.fp8 and (self.sx8 is None or not F8_.MX_PREFILL):
             return False

@@ -693,6 +693,27 @@ def test_linear_norm_65_to_256_rows(M, N, K, buffers):
                                       H, 1, 16)
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 2304, 768), (200, 4096, 1024), (256, 768, 3072), (130, 12544, 64)])
+def test_gemm_65_to_256_rows_off_16_bytes(M, N, K):
+    """Operands that start off 16 bytes or whose rows do: plain loads (the decode kernels) instead of the
+    tiles' LDS-DMA.  Tolerance: test_gemm_mid_tiles."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g).bfloat16()  # noqa: E731
+    x0, w0 = rnd(M * K + 3), rnd(N * K + 1)
+    xs = [x0[3:].view(M, K), rnd(M, K + 5)[:, :K], rnd(M, K + 8)[:, 1:K + 1], rnd(M, K)]
+    ws = [rnd(N, K)] * 3 + [w0[1:].view(N, K)]
+    few = -(-M // 128) * -(-N // 128) < 192
+    f = G.fold_norm(ws[0].float(), torch.ones(K, device=DEV), torch.zeros(K, device=DEV), None, False, 1e-5, DEV)
+    for x, w in zip(xs, ws):
+        w = (w.float() * K ** -0.5).bfloat16() if w.data_ptr() % 16 == 0 else w
+        assert _rel(G.linear(x, w), x.float() @ w.float().t()) < 2.5e-3
+        if few:
+            ref = torch.nn.functional.layer_norm(x.float(), (K,), eps=1e-5) @ f.w.float().t()
+            y = G.linear_norm(x, f, std_buf=torch.empty(M, K, device=DEV, dtype=torch.bfloat16), ones=torch.ones(K, device=DEV))
+            assert _rel(y, ref) < 4e-3
+
+
 @pytest.mark.parametrize("B,T,H,Hkv,hd,pos0,S", [(1, 65, 12, 12, 64, 0, 80), (3, 43, 4, 2, 128, 5, 60), (1, 255, 25, 25, 64, 9, 300)])
 def test_qkv_scatter_small_prefill(B, T, H, Hkv, hd, pos0, S):
     """Fewer rows than a 256 x 256 tile: scattered on every small tile == qkv rows + qkv_split."""

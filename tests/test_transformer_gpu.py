@@ -1765,3 +1765,18 @@ def test_prefill_one_call(model, dtype, B, T, monkeypatch):
     for a, b in zip(*got):
         assert torch.equal(a, b)
     assert got[0][1][:, 1:1 + B].abs().sum() > 0 and got[0][1][:, 1 + B].abs().sum() == 0
+
+
+@pytest.mark.parametrize("T", [70, 200])
+def test_prefill_rows_off_16_bytes(T):
+    """Hidden rows that start off 16 bytes: issued by the loop, whose kernels look at the alignment."""
+    from distributed_neural_networks_amd import checkpoint as ckpt
+    from distributed_neural_networks_amd.runtime.transformer import build_device_stage
+    sd = ckpt.random_stage_state_dict("gpt2", 1, 2, False, False, 3, nontrivial=True)
+    st = build_device_stage("gpt2", sd, 1, 2, False, False, DEV, max_batch=1, max_seq=T + 4, max_tokens=T)
+    flat = torch.randn(T * st.d + 8, device=DEV).bfloat16()
+    pos, outs = torch.zeros(1, dtype=torch.int32, device=DEV), []
+    for off in (0, 3):
+        flat[off:off + T * st.d] = torch.linspace(-2, 2, T * st.d, device=DEV).sin().bfloat16()
+        outs.append(st.step(flat[off:off + T * st.d].view(T, st.d), pos, 1, T).clone())
+    assert _rel(outs[1], outs[0]) < 1e-2
