@@ -751,7 +751,7 @@ extern "C" int dnn_gemm_fp8_256(const void* A, const float* sa, const void* W, c
 // Tile of gemm_mid.h for an MX product, -1: the 256 x 256 kernel.  A K-tile of 128
 // bytes takes a tile as long as the bf16 kernel's K-tile of 64: the same estimate.
 static int mx_mid_tile(int M, int N, int Kb, bool quant) {
-  if (g_gemm_tile != 0) return -1;
+  if (g_gemm_tile != 0 || Kb >= 1 << 24) return -1;  // the small tiles address a tile's rows with 32 bits
   if (g_mid_tile >= 0) return quant && g_mid_tile < 2 ? 2 : g_mid_tile;
   return mid_plan(M, N, Kb / 2, 0, quant ? MID_MX_QUANT : MID_MX).tile;
 }

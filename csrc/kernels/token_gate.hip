@@ -135,7 +135,8 @@ extern "C" int dnn_token_gate(const void* x, int ldx, const void* w, int ldw, co
   // (1024 x 256 x 4096: 16.9 us, as rounds 26.5; 30 with the six-stage loop of its own
   // that read a tile's fragments between two barriers)
   const float rounds = (float)(((M + 15) / 16 * (np / 16) + 255) / 256), passes = (float)((K + 4095) / 4096);
-  if (M <= 64 || 1.f + 6.4f * rounds * passes < 2.5f + 0.225f * K / 64) {
+  const bool narrow = ldx < 1 << 23 && ldw < 1 << 23;  // the tiles address their 64 rows with 32 bits
+  if (M <= 64 || !narrow || 1.f + 6.4f * rounds * passes < 2.5f + 0.225f * K / 64) {
     hipLaunchKernelGGL(token_gate_skinny_kernel, dim3(np / 16, (M + 15) / 16), dim3(64 * (TG_WAVES + 1)), 0, st,
                        (const bf16_t*)x, ldx, (const uint8_t*)wsh, K, t);
   } else {

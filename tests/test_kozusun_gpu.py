@@ -96,6 +96,22 @@ def test_token_gate(dtype, M, n, np_, K):
     assert (out[:, n:np_] == 0).all() and (out[:, np_:] == 1).all()
 
 
+def test_token_gate_rows_far_apart():
+    """Rows whose distance times 64 passes 32 bits (4.9 GB of them), at a size that the tiles would take."""
+    from distributed_neural_networks_amd.ops import decoder_ops as D_
+    g = torch.Generator().manual_seed(0)
+    M, n, K, ld = 70, 60, 64, 35_000_000
+    xs, tab = torch.randn(M, K, generator=g).bfloat16(), torch.randn(11, n, generator=g).bfloat16()
+    x = torch.empty(M * ld, dtype=torch.bfloat16, device=dev()).as_strided((M, K), (ld, 1))
+    x.copy_(xs)
+    w, ids = torch.zeros(64, K), torch.randint(0, 11, (M,), generator=g, dtype=torch.int32)
+    w[:n] = torch.randn(n, K, generator=g).bfloat16().float() / math.sqrt(K)
+    lin, out = D_.Linear(w, None, torch.bfloat16, dev()), torch.empty(M, 64, dtype=torch.bfloat16, device=dev())
+    D_.token_gate(x, lin, tab.to(dev()), 0, ids.to(dev()), out, n)
+    ref = O.gelu_tanh(xs.double() @ lin.w.double().cpu()[:n].t()) * tab[ids.long()].double()
+    assert ((out[:, :n].double().cpu() - ref).norm(dim=1) / ref.norm(dim=1)).max().item() < 8e-3
+
+
 @pytest.mark.parametrize("M", [64, 65, 500, 2049, 4100])
 @pytest.mark.parametrize("n,np_", [(60, 64), (300, 320)])
 def test_token_gate_long_rows(M, n, np_):
