@@ -225,7 +225,11 @@ def _head_few(h: torch.Tensor, w: CifarHeadWeights, hid: Optional[torch.Tensor],
 
 
 def _fc1_scratch(scratch: Optional[torch.Tensor], B: int, device) -> torch.Tensor:
-    if scratch is None or scratch.shape[0] < B or tuple(scratch.shape[1:]) != (3 * 4096,):
+    """``scratch`` where its first ``B`` rows are 24 KB each, one behind the other."""
+    if scratch is not None and scratch.dtype != torch.bfloat16:
+        raise TypeError(f"fc1 scratch: bf16 rows expected, got {scratch.dtype}")
+    if (scratch is None or scratch.shape[0] < B or tuple(scratch.shape[1:]) != (3 * 4096,)
+            or not scratch[:B].is_contiguous()):
         scratch = torch.empty((B, 3 * 4096), dtype=torch.bfloat16, device=device)
     return scratch
 
