@@ -123,7 +123,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const uint8_t* __restr
   // from HBM once and re-read from that XCD's L2.
   int n0;
   if constexpr (MS) {
-    const int mtiles = (M + 16 * MT - 1) / (16 * MT);
+    const int mtiles = (unsigned)(M + 16 * MT - 1) / (16 * MT);
     const int lgc = xcd_remap(blockIdx.x, gridDim.x);
     const int mo = (lgc % mtiles) * (16 * MT);
     n0 = (lgc / mtiles) * (16 * NT);
@@ -835,6 +835,26 @@ extern "C" int dnn_gemm_set_skinny_pin(int id, int ks, int n, int k) {
   return 0;
 }
 
+// e4m3 weights, 65 to 256 rows (bf16 has the tiles of gemm_mid.h here): whether 64 rows a
+// workgroup, whose weights and their conversion serve four M tiles, run faster than 16.
+//
+// Both by estimate, from the workgroups of the fullest CU: 16 rows on 2 column tiles
+// share a CU and add up; 64 rows on 4 (N from 4096) or 2 hold 64 or 32 KB of LDS and queue
+// in rounds.  us over M, 16 : 64 rows, the faster one taken: 4800 x 1600 90 12.6 : 13.3,
+// 112 14.5 : 13.5, 190 20.7 : 13.7, 240 22.9 : 20.4; 6400 x 1600 130 19.7 : 20.5, 175 22.9
+// : 20.4; 4096 x 14336 90 53.4 : 61.5, 130 81.5 : 61.7, 256 132 : 64; 1600 x 6400 240 25.9
+// : 29.0, 256 32.9 : 29.1.  K below 1024 on narrow outputs: 2304 x 768 256 9.9 : 11.6.
+// The estimates are within 10 % of 150 shapes each; 2 % and a folded norm's 0.7 us (its
+// sums take longer with 64 rows) go to the 16 rows.
+static bool w8_rows64(int M, int N, int K, bool norm) {
+  if (N <= 1024 || (N < 4096 && K < 1024)) return false;
+  const int n16 = ((M + 15) / 16 * ((N + 31) / 32) + 255) / 256, cols = N >= 4096 ? 64 : 32;
+  const int n64 = ((M + 63) / 64 * ((N + cols - 1) / cols) + 255) / 256;
+  const float t16 = 4.3f + n16 * (0.35f + 0.00105f * K);
+  const float t64 = N >= 4096 ? 6.3f + n64 * (0.9f + 0.0038f * K) : 5.6f + n64 * 0.00366f * K;
+  return t64 + (norm ? 0.7f : 0.f) < 0.98f * t16;
+}
+
 template <int ACT, bool F32, bool FP8, int MT, int NT, int U, bool PIPE, int NORM, bool W8, bool MS = false>
 static int launch_skinny_cfg(const void* A, int lda_b, const float* sa, const void* W, int ldw_b, const float* sw,
                              void* C, int ldc, const float* bias, const void* R, int ldr, int M, int N, int kbytes,
@@ -910,14 +930,11 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
   // from its XCD's L2 by the M tiles (the 128^2 GEMM would launch only a
   // handful of tiles at these shapes)
   if (M > 64) {
-    // e4m3 weights (bf16 has the tiles of gemm_mid.h here): 64 rows a workgroup, so the
-    // weights and their conversion serve four M tiles.  us, 16 : 64 rows: 256 x 4096 x
-    // 14336 126 : 62, 256 x 6400 x 1600 34.7 : 23.7, 190 x 4800 x 1600 22.5 : 14.9, 100 x 4096 x 4096
-    // 22.3 : 21.9, but 66 x 4096 x 4096 17.9 : 21.9; narrow N on 2 column tiles 256 x 1600 x
-    // 6400 32.5 : 28.9, 190 rows 25.6 : 28.6
     if constexpr (W8) {
-      if (N >= 4096 && M > 80) CFG_MM(4, 4);
-      if (N < 4096 && N > 1024 && M > 208) CFG_MM(4, 2);
+      if (w8_rows64(M, N, kbytes, NORM != NORM_NONE)) {
+        if (N >= 4096) CFG_MM(4, 4);
+        CFG_MM(4, 2);
+      }
     }
     if (N <= 1024) CFG_MS(1, 4, false, 4);
     CFG_MS(2, 2, false, 4);

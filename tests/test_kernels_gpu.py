@@ -621,11 +621,11 @@ def test_gemm_9_to_16_rows(M, N, K):
         G.attach_shuffled(w8)
 
 
-@pytest.mark.parametrize("M", [80, 81, 129, 193, 208, 209, 256])
-@pytest.mark.parametrize("N,K", [(1040, 64), (4092, 192), (4112, 448)])
+@pytest.mark.parametrize("M", [80, 81, 113, 129, 193, 208, 209, 240, 241, 256])
+@pytest.mark.parametrize("N,K", [(1040, 64), (4092, 192), (4112, 448), (1600, 1600), (4092, 1600), (4112, 1600)])
 def test_gemm_w8_65_to_256_rows(M, N, K):
-    """Either side of the lines to 64 rows a workgroup, a last group of one row, columns cut
-    inside a tile: e4m3 weights with bias and residual, GELU behind a folded norm, row-major
+    """16 rows a workgroup (the first three sizes) and either side of the rule to 64 rows, on 2 and on 4 column
+    tiles (K of 1600), a last group of one row, columns cut inside a tile: e4m3 weights with bias and residual, GELU behind a folded norm, row-major
     and in fragment order.  Tolerances: test_gemm_9_to_16_rows."""
     from distributed_neural_networks_amd.ops import gemm as G
     from distributed_neural_networks_amd.ops.fp8 import linear_w8, quantize_weight
