@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256 * KS, 2) void flash_attn_kernel(const bf16_t* _
   constexpr int NKS = HD / 16;  // k-steps of the QK^T contraction
   constexpr int NDT = HD / 32;  // 32-wide d tiles of O
   constexpr int CH = HD / 8;    // 16-B chunks per row
-  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+  const int tid = KS == 1 ? threadIdx.x : threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
   const int h = lane >> 5, r32 = lane & 31;
   const int qb = (int)(gridDim.z - 1 - blockIdx.z), hh = blockIdx.x, b = blockIdx.y;
   const int kvh = hh / (H / Hkv);
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(256 * KS, 2) void flash_attn_kernel(const bf16_t* _
   const int kv_len = min(p0 + T, S);  // rows of the cache: none past its end is fetched or counted
   const int qrow0 = qb * FA_QB + wave * 32;            // this wave's first query (chunk-relative)
   const int qrow = qrow0 + r32;                        // this lane's query
-  const int q_abs = p0 + min(qrow, T - 1);
+  const int key_max = min(p0 + min(qrow, T - 1), kv_len - 1);  // last key this lane's query attends
   const int wave_qmax = p0 + min(qrow0 + 31, T - 1);   // wave-uniform
   const int wave_qmin = p0 + min(qrow0, T - 1);
   const int blk_qmax = p0 + min(qb * FA_QB + FA_QB - 1, T - 1);
@@ -298,7 +298,7 @@ __global__ __launch_bounds__(256 * KS, 2) void flash_attn_kernel(const bf16_t* _
 #pragma unroll
           for (int g = 0; g < 16; ++g) {
             const int key = kb0 + kt * 32 + (g & 3) + 8 * (g >> 2) + 4 * h;
-            if (key > q_abs || key >= kv_len) sacc[kt][g] = -INFINITY;
+            if (key > key_max) sacc[kt][g] = -INFINITY;
           }
       }
       float mx = -INFINITY;
