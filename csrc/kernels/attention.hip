@@ -952,14 +952,14 @@ extern "C" int dnn_qkv_split(const void* qkv, void* q, void* kc, void* vc, int B
   return (int)hipGetLastError();
 }
 
-// Two key groups: at most one workgroup a CU and a chain of a few blocks.  us, one :
-// two groups: GPT-2 200 tokens 7.2 : 6.6, 3 x 357 10.0 : 8.8, 960 19.2 : 14.7, 4 x 600
-// 14.6 : 11.8, but 100 5.3 : 5.7; XL 8 x 256 (400 workgroups) 9.4 : 12.9; Llama-3 700
-// 21.4 : 19.2, 1000 29.6 : 26.1, 300 11.2 : 11.5.
+// Two key groups: at most one workgroup a CU and a chain of a few blocks of 64 keys: from 4
+// (8 at hd 128).  us, one : two groups: GPT-2 161 tokens 5.8 : 6.0, 192 6.0 : 6.1, 193 6.9 :
+// 6.6, 3 x 357 9.4 : 8.6, 960 18.0 : 14.6, 4 x 600 13.7 : 11.6; XL 8 x 256 (400 workgroups)
+// 9.4 : 12.9; Llama-3 449 15.2 : 14.7, 700 20.6 : 18.9, 1000 27.9 : 24.8, 300 11.2 : 11.5.
 constexpr int FA_KS_WGS = 256;
 template <int HD>
 static bool flash_two_groups(long wgs, int T) {
-  return wgs <= FA_KS_WGS && T > (HD == 64 ? 160 : 448);
+  return wgs <= FA_KS_WGS && T > (HD == 64 ? 192 : 448);
 }
 template <int HD, bool QKV, bool KV8>
 static void launch_flash(dim3 grid, hipStream_t st, const bf16_t* q, const bf16_t* kc, const bf16_t* vc, bf16_t* o,

@@ -192,7 +192,7 @@ def test_flash_attn_spike_rescale():
     assert _rel(out, ref) < 2e-2
 
 
-@pytest.mark.parametrize("B,Tn,H,Hkv,hd,pos0,S", [(1, 161, 3, 3, 64, 0, 161), (2, 200, 4, 2, 64, 33, 240), (1, 320, 2, 2, 64, 0, 300),
+@pytest.mark.parametrize("B,Tn,H,Hkv,hd,pos0,S", [(1, 193, 3, 3, 64, 0, 193), (2, 200, 4, 2, 64, 33, 240), (1, 320, 2, 2, 64, 0, 300),
                                                   (1, 449, 4, 2, 128, 0, 512), (1, 513, 2, 1, 128, 70, 600)])
 def test_flash_two_key_groups(B, Tn, H, Hkv, hd, pos0, S, monkeypatch):
     """Every other key block in a group of its own (the default on small grids) against
