@@ -84,18 +84,26 @@ MidPlan mid_plan(int M, int N, int K, long long ws_bytes, unsigned kind) {
   return e.plan;
 }
 
-// Decode kernels (gemm_skinny.hip) on more than 64 rows: every 16 rows read the
-// weights once more (from the cache).  us beside the tiles, a folded norm that rides
-// along (its launch takes 2.5 beside them): 66 rows x 768 x 768 4.1 : 5.3, 192 x 768 x 3072 13.6
-// : 10.3, 66 x 2048 x 7680 25.4 : 15.3, 256 x 4096 x 4096 88 : 18; with the norm 66 x 2304
-// x 768 6.7 : 8.0, 128 rows 8.2 : 8.0, 256 rows 11.0 : 8.1.  `frag`: the weight has its
-// fragment-order copy.
+// Decode kernels (gemm_skinny.hip) on more than 64 rows against the tiles.  They take 16 rows
+// and 32 columns a workgroup (16 up to 1024 columns), which share a CU and add up: the
+// time is that of the fullest CU, in steps.  `frag`: the weight has its fragment-order
+// copy; without it a step costs 1.6 times as much.  A folded norm rides along for 1 us; the
+// tiles need a launch that adds 3.3, and at K below 1024 they take 0.8 longer than their
+// estimate.  us, decode kernels : tiles: 132 rows x 768 x 768 5.3 : 5.8, 192 6.6 : 5.9; row-
+// major 70 4.8 : 5.3; 192 x 768 x 3072 row-major 19.4 : 12.1; 70 x 1600 x 1600 7.1 : 7.1, 85
+// 9.0 : 8.5; 256 x 4096 x 4096 88 : 18; with a norm 128 x 3072 x 768 9.0 : 9.7, 146 10.4 : 9.8,
+// 135 x 2304 x 768 8.6 : 9.2, 167 9.6 : 9.1, 128 x 2816 x 512 6.4 : 7.4, 189 8.1 : 7.6, 256 x 1536 x
+// 512 6.4 : 7.1, 65 x 4800 x 1600 12.8 : 11.7.
 bool mid_skinny(int M, int N, int K, bool norm, bool frag, long long ws_bytes) {
   if (M <= 64) return true;
   if (M > 256) return false;
-  const float nk = (float)N * K;
-  return 3.8f + nk * 2.f / 4.27e6f + (frag ? 2.1e-7f : 3.2e-7f) * nk * ((M + 15) / 16) <
-         mid_plan(M, N, K, ws_bytes, MID_BF16).us + (norm ? 2.5f : 0.f);
+  const bool one = N <= 1024;
+  const int n = ((M + 15) / 16 * ((N + (one ? 15 : 31)) / (one ? 16 : 32)) + 255) / 256;
+  const float base = one ? 2.9f + 0.0002f * K : 3.6f + 0.0006f * K;
+  const float step = frag ? (one ? 0.45f + 0.0009f * K : 0.15f + 0.00152f * K)
+                          : (one ? 0.4f + 0.0016f * K : 0.2f + 0.0025f * K);
+  return base + n * step + (norm ? 1.f : 0.f) <
+         mid_plan(M, N, K, ws_bytes, MID_BF16).us + (K < 1024 ? 0.8f : 0.f) + (norm ? 3.3f : 0.f);
 }
 
 template <class T, MidOut OUT>
