@@ -432,10 +432,6 @@ extern "C" int dnn_gemm_set_mid(int tile, int splits) {
   g_mid_splits = splits;
   return 0;
 }
-extern "C" int dnn_gemm_is_skinny(int M, int N, int K, int norm, int frag, long long ws_bytes) {
-  return g_gemm_tile == 0 && g_mid_tile < 0 ? mid_skinny(M, N, K, norm != 0, frag != 0, ws_bytes - 4096) : M <= 64;
-}
-
 // Rows up to which every bf16 GEMM streams its weights on the skinny kernels
 // (A/B switch).  At M = 64 a wide-N head with warm weights runs faster on the
 // 128^2 MFMA tiles (GPT-2 50304 x 768: 28.3 -> 22.5 us, x 1600: 52.7 -> 33.6,
@@ -448,6 +444,14 @@ extern "C" int dnn_gemm_set_skinny_max_m(int m) {
   if (m < 0 || m > 64) return -1;
   g_skinny_max_m = m;
   return 0;
+}
+
+// The decode kernels' rows: all up to g_skinny_max_m, beyond by estimate unless a tile is pinned
+static bool skinny(int M, int N, int K, bool norm, bool frag, long long part_bytes) {
+  return M <= g_skinny_max_m || (g_gemm_tile == 0 && g_mid_tile < 0 && mid_skinny(M, N, K, norm, frag, part_bytes));
+}
+extern "C" int dnn_gemm_is_skinny(int M, int N, int K, int norm, int frag, long long ws_bytes) {
+  return skinny(M, N, K, norm != 0, frag != 0, ws_bytes - 4096);
 }
 
 // 256^2 epilogue: residual rows loaded ahead of the outputs (1) or per output row group (0)
@@ -523,13 +527,10 @@ static int launch_gemm(const void* A, int lda, const void* W, int ldw, void* C, 
   // GEMM (rowstat) always takes the tile kernels: the skinny path folds its norm
   // itself, dnn_gemm_skinny_norm
   const long long part_bytes = mid_ws(ws, ws_bytes);
-  const bool pinned = g_gemm_tile != 0 || g_mid_tile >= 0;
   // up to 256 rows what the small tiles cannot stage (dma_rows) goes to the decode kernels, whose loads are plain
   const bool narrow = lda < 1 << 23 && ldw < 1 << 23;  // the small tiles address a tile's rows with 32 bits
-  if (rowstat == nullptr &&
-      (M <= g_skinny_max_m || (M > 64 && M <= 256 && !pinned &&
-                               (!narrow || !dma_rows(A, lda, W, ldw) ||
-                                mid_skinny(M, N, K, false, Wsh != nullptr, part_bytes))))) {
+  if (rowstat == nullptr && (skinny(M, N, K, false, Wsh != nullptr, part_bytes) ||
+                             (M <= 256 && (!narrow || !dma_rows(A, lda, W, ldw))))) {
     return dnn_gemm_skinny(A, lda, nullptr, W, ldw, nullptr, C, ldc, bias, R, ldr, M, N, K, ACT, F32 ? 1 : 0, 0, st, Wsh,
                            ws, ws_bytes);
   }

@@ -95,7 +95,6 @@ MidPlan mid_plan(int M, int N, int K, long long ws_bytes, unsigned kind) {
 // 135 x 2304 x 768 8.6 : 9.2, 167 9.6 : 9.1, 128 x 2816 x 512 6.4 : 7.4, 189 8.1 : 7.6, 256 x 1536 x
 // 512 6.4 : 7.1, 65 x 4800 x 1600 12.8 : 11.7.
 bool mid_skinny(int M, int N, int K, bool norm, bool frag, long long ws_bytes) {
-  if (M <= 64) return true;
   if (M > 256) return false;
   const bool one = N <= 1024;
   const int n = ((M + 15) / 16 * ((N + (one ? 15 : 31)) / (one ? 16 : 32)) + 255) / 256;

@@ -63,6 +63,7 @@ def set_skinny_max_m(m: int = 64) -> None:
     global SKINNY_ALWAYS_M
     check(lib().gemm_set_skinny_max_m(int(m)), "gemm_set_skinny_max_m")
     SKINNY_ALWAYS_M = int(m)
+    _is_skinny.cache_clear()
 _ACTS = {None: ACT_NONE, "none": ACT_NONE, "relu": ACT_RELU, "gelu": ACT_GELU, "silu_mul": ACT_SILU_MUL,
          "gelu_tanh_mul": ACT_GELU_TANH_MUL}
 

@@ -1,0 +1,26 @@
+"""Which rows take the decode kernels (the library's host side: no GPU needed)."""
+import pytest
+
+from distributed_neural_networks_amd.ops import gemm as G
+
+
+@pytest.fixture
+def max_m():
+    yield G.set_skinny_max_m
+    G.set_skinny_max_m()
+
+
+def test_set_skinny_max_m_governs_folded_norms(max_m):
+    """Rows past the switch go by estimate, below 65 too: a head of 50304 columns is then the tiles'."""
+    head = (50304, False, 768, True)
+    assert all(G.skinny_rows(M, *head) for M in (1, 33, 48, 64)) and not G.skinny_rows(65, *head)
+    max_m(32)
+    assert G.skinny_rows(32, *head) and not any(G.skinny_rows(M, *head) for M in (33, 48, 64))
+    assert G.skinny_rows(48, 768, False, 768, True)  # 16 workgroups of 128 x 128: still the decode kernels'
+    max_m(64)
+    assert G.skinny_rows(48, *head)  # no answer of the other setting is kept
+
+
+def test_fp8_rows():
+    assert G.skinny_rows(64, 50304, True) and G.skinny_rows(256, 12160, True) and not G.skinny_rows(65, 24576, True)
+    assert not G.skinny_rows(257, 128, True)
