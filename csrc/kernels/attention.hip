@@ -19,6 +19,7 @@
 #include "common.h"
 
 #include <algorithm>
+#include <cfloat>
 #include <cstdlib>
 
 namespace dnn {

@@ -175,8 +175,9 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
     }
   }
 
-  // softmax state: G = 1, of the lane's row group; MF, of head hj over the wave (l: over the lane's keys)
-  float m = -INFINITY, l = 0.f, acc[G][8];
+  // softmax state: G = 1, of the lane's row group; MF, of head hj over the wave (l: over the lane's keys).
+  // The maximum starts finite: against -inf, scores that are -inf would make exp2(-inf + inf)
+  float m = -FLT_MAX, l = 0.f, acc[G][8];
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
@@ -215,7 +216,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
           s[t][r] = t * 16 + r < last ? s[t][r] * scale_log2 : -INFINITY;
           mx = fmaxf(mx, s[t][r]);
         }
-      const float mn = fmaxf(m, max_over_quarters(mx)), base = mn == -INFINITY ? 0.f : mn;  // no finite score yet: all 0
+      const float mn = fmaxf(m, max_over_quarters(mx));
       const float al = mn == m ? 1.f : __builtin_amdgcn_exp2f(m - mn);
       m = mn;
       float sum = 0.f;
@@ -223,7 +224,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
       for (int t = 0; t < NT16; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float p = __builtin_amdgcn_exp2f(s[t][r] - base);
+          const float p = __builtin_amdgcn_exp2f(s[t][r] - mn);
           sum += p;
           const int row = t * 16 + c4 * 4 + r, u = row / RG;
           if (hj < G) pl[wave][((row % RG) * (U / 2) + (u >> 1)) * G * 2 + hj * 2 + (u & 1)] = f2bf(p);
@@ -271,12 +272,12 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
 #pragma unroll
       for (int u = 0; u < U; ++u)
         if (u * RG < last) mn = fmaxf(mn, p[u]);
-      const float al = mn == m ? 1.f : __builtin_amdgcn_exp2f(m - mn), base = mn == -INFINITY ? 0.f : mn;
+      const float al = mn == m ? 1.f : __builtin_amdgcn_exp2f(m - mn);
       m = mn;
       float sum = 0.f;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        p[u] = u * RG < last ? __builtin_amdgcn_exp2f(p[u] - base) : 0.f;
+        p[u] = u * RG < last ? __builtin_amdgcn_exp2f(p[u] - mn) : 0.f;
         sum += p[u];
       }
       l = l * al + sum;
@@ -316,7 +317,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
     __builtin_amdgcn_sched_barrier(0);
   }
 
-  // the wave's row groups, then the waves: a group without rows carries m = -inf, l = 0
+  // the wave's row groups, then the waves: a group without rows carries the lowest m, l = 0
   float mw = m, f = 1.f;
   if constexpr (!MF) {
 #pragma unroll
