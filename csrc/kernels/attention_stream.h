@@ -2,11 +2,13 @@
 // Decode attention that keeps the K/V stream running: every wave walks its own
 // blocks of rows with the next block's keys in flight while it folds the values of
 // this one, and no wave waits for another before the end.  Bound by the bytes of the
-// caches: Llama-3 8B B=32 of 690 to 1100 keys 38.4 -> 22.8 us (5.7 TB/s; batches of keys,
-// softmax over the split, batches of values before), of 540 19.5 -> 13.3 (all of a
-// split's rows in flight at once before), B=64 of 1000 49.9 -> 39.9, B=1 of 2048 18.3 ->
-// 9.6; GPT-2 B=64 of 512 18.1 -> 16.9, XL B=64 of 288 24.5 -> 19.3.  Blocks of twice the
-// rows: 0.5 us either way.
+// caches: Llama-3 8B B=32 of 820 to 1100 keys 39.0 -> 24.3 us (5.2 TB/s; batches of keys,
+// softmax over the split, batches of values before), of 560 21.7 -> 15.5 (all of a
+// split's rows in flight at once before), B=64 of 1000 55 -> 42, B=1 of 2048 18.7 -> 10.2;
+// GPT-2 B=64 of 385 to 512 18.5 -> 18.0, XL B=64 of 217 to 288 25.0 -> 20.0, of 60 17.6 -> 8.8;
+// caches that memory holds, not the last-level cache.  Slower than before: 16384 keys of 25
+// ungrouped heads, B=4, 80 -> 83, 32 ungrouped heads of 128, B=16 of 1024, 42.3 -> 43.2 (no
+// model here has either).  Blocks of twice the rows: 0.5 us either way.
 //
 // Included by attention.hip inside namespace dnn (load_head8, bf16x2v).
 //

@@ -1,7 +1,7 @@
 // bf16 GEMM for row counts between decode and large prefill (65 to a few thousand
 // rows, where 256 x 256 tiles leave most CUs idle): tiles of 64 to 256 rows with a
 // deep LDS pipeline, and the K range over several workgroups where the tiles alone
-// do not fill the chip (gemm_bf16.hip mid_plan chooses).
+// do not fill the chip (gemm_mid.hip mid_plan chooses).
 #pragma once
 #include "common.h"
 #include "gemm_epilogue.h"

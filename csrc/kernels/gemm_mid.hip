@@ -6,10 +6,11 @@ namespace dnn {
 
 // Tile table: rows, columns, whether two workgroups share a CU, and the two
 // constants of a tile's time in us: a (launch, first loads, epilogue) and s (a
-// K-tile of 64).  Fitted to 310 shapes (65 to 32768 rows, 768 to 28672 columns, K of
-// 768 to 18432, weights cold) that every tile ran, with 1 to 8 splits: the estimate
-// is off by 9 % (rms), and what it picks is within 1 % of the best measured on
-// average, 20 % at worst.  The last entry is the 256 x 256 kernel (gemm_tile.h).
+// K-tile of 64).  Over 191 shapes (66 to 9419 rows, 768 to 28672 columns, K of 768 to
+// 21504, weights cold) that every tile ran with 1 to 8 splits, 4139 times, the estimate is
+// off by 10 % (rms); what it picks takes 2 % longer than the best measured on average
+// (0.1 % in the median, 25 % at worst: 1022 x 2048 x 7680 52.7 us, 42.2 as 256 x 128 in 4;
+// profiles/gemm_mid_estimate.md).  The last entry is the 256 x 256 kernel (gemm_tile.h).
 struct MidCost {
   int bm, bn, pairs;
   float a, s;

@@ -6,6 +6,11 @@ from distributed_neural_networks_amd.ops import gemm as G
 
 @pytest.fixture
 def max_m():
+    from distributed_neural_networks_amd.ops._lib import lib
+    try:
+        lib()
+    except RuntimeError as e:
+        pytest.skip(f"kernel library: {e}")
     yield G.set_skinny_max_m
     G.set_skinny_max_m()
 
