@@ -130,13 +130,13 @@ extern "C" int dnn_token_gate(const void* x, int ldx, const void* w, int ldw, co
   if (ldx % 8 != 0 || ldw % 8 != 0 || ldx < K || ldw < K || ldg % 4 != 0 || ldg < np || wsh == nullptr) return -1;
   if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)wsh) & 15) != 0 || ((uintptr_t)g & 7) != 0) return -1;
   const TokenGate t{(const bf16_t*)table, tok, (bf16_t*)g, ldt, off, V, ldg, M, n};
-  // Few rows: rounds of 256 workgroups of 16 x 16 outputs, 6.4 us each for K up to
-  // 4096 (512 x 256 x 4096: 13.9 us, as tiles 17.0); tiles: 0.225 us a K-tile of 64
-  // (1024 x 256 x 4096: 16.9 us, as rounds 26.5; 30 with the six-stage loop of its own
-  // that read a tile's fragments between two barriers)
+  // Few rows: rounds of 256 workgroups of 16 x 16 outputs, 6.4 us each for K up to 4096;
+  // tiles 0.166 us a K-tile of 64 beside 4.9.  us, rounds : tiles: 100 x 64 x 512 7.1 : 6.2, 100 x
+  // 256 x 1024 7.1 : 7.5, 512 x 256 x 4096 13.6 : 15.4, 1024 x 256 x 4096 26.5 : 15.7 (30 with the
+  // six-stage loop of its own that read a tile's fragments between two barriers)
   const float rounds = (float)(((M + 15) / 16 * (np / 16) + 255) / 256), passes = (float)((K + 4095) / 4096);
   const bool narrow = ldx < 1 << 23 && ldw < 1 << 23;  // the tiles address their 64 rows with 32 bits
-  if (M <= 64 || !narrow || 1.f + 6.4f * rounds * passes < 2.5f + 0.225f * K / 64) {
+  if (M <= 64 || !narrow || 0.7f + 6.4f * rounds * passes < 4.9f + 0.166f * K / 64) {
     hipLaunchKernelGGL(token_gate_skinny_kernel, dim3(np / 16, (M + 15) / 16), dim3(64 * (TG_WAVES + 1)), 0, st,
                        (const bf16_t*)x, ldx, (const uint8_t*)wsh, K, t);
   } else {
