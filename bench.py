@@ -1,11 +1,11 @@
 #!/usr/bin/env python3
 """Flagship benchmark: CIFAR-10 ConvNet 2-stage pipeline inference, images/s.
 
-Metric/config from BASELINE.json (the reference's only measured headline:
-CIFAR-10 2-stage images/s; 3.40-4.15 k img/s on CPU over localhost gRPC,
-BASELINE.md).  Synthetic fp32 images, random-init weights of the reference
-architecture.  Precision: the reference's fp32 contract, computed as **fp32
-(bf16x3 split emulation, ~2^-16 relative per product, fp32 accumulation)**:
+Metric and configuration: the reference's only measured headline
+(CIFAR-10 2-stage images/s; 3.40-4.15 k img/s on CPU over localhost gRPC).
+Synthetic fp32 images, random-init weights of the reference architecture.
+Precision: the reference's fp32 contract, computed as **fp32 (bf16x3 split
+emulation, ~2^-16 relative per product, fp32 accumulation)**:
 every product is three bf16 MFMA terms (ops/cifar.py); the line reports the
 measured max|dprob| against fp32 torch on 4096 images (outside the timed
 region).  ``--precision bf16`` is the reduced-precision variant (extra keys).
@@ -57,7 +57,7 @@ import sys
 
 import torch
 
-BASELINE_IMG_S = 4150.0  # reference CIFAR-10 2-stage, best batch (255), CPU gRPC
+BASELINE_IMG_S = 4150.0  # the reference's CIFAR-10 2-stage, best batch (255), CPU gRPC
 METRIC = "images/sec CIFAR-10 2-stage"
 DTYPE_LABEL = {"fp32": "fp32 (bf16x3 split emulation, ~2^-16 per product)", "bf16": "bf16"}
 CPU_DTYPE_LABEL = "fp32 (torch CPU golden stages over gloo: schedule test, not a measurement)"
@@ -276,7 +276,7 @@ def bench_interleaved(args, info):
 
 
 def bench_pp2(args, info):
-    """BASELINE config 2 on N GPUs: the reference's 2-stage pipeline with its
+    """The image workload on N GPUs: the reference's 2-stage pipeline with its
     cut (conv | fc1+fc2+softmax, ``cifar_model_parts.py:29-58``), one stage per
     GPU.  Rank 2p runs stage 0 and rank 2p+1 stage 1 (pipeline p of N/2).
     The fp32 boundary (16 KiB/img) crosses a bipartite hop: every stage-0 GPU
@@ -363,7 +363,7 @@ def hop_bandwidth(info, nbytes: int, reps: int = 4, timeout_s: float = 60.0) -> 
     and the ranks agree on their outcome through the store before any
     collective: one rank's failure skips the measurement on every rank
     (raising the same error everywhere) instead of leaving the others in the
-    timing barrier (ADVICE r4)."""
+    timing barrier."""
     from distributed_neural_networks_amd.parallel.links import make_link
     from distributed_neural_networks_amd.parallel import rccl
     r, N, dev = info.rank, info.world, info.device
@@ -485,8 +485,8 @@ def golden_probs(dev, x: torch.Tensor) -> torch.Tensor:
 
 
 def pp2_verify(info, s0, s1, n_img: int = VERIFY_IMAGES) -> dict:
-    """The answer that crossed the hops, checked (the
-    reference's one check is the prediction that comes back over the hop,
+    """The answer that crossed the hops, checked (the reference's one
+    check is the prediction that comes back over the hop,
     ``node.py:58-68``, ``node.py:184-192``).  Every stage-0 GPU pushes a fixed
     seeded set of ``n_img`` images through the *distributed* pipeline the
     headline measured: its stage-0 kernel, the bipartite ``SplitLink`` hop to
@@ -660,7 +660,7 @@ def extra_keys(args, info):
     pipeline at reduced (bf16) precision when the headline is fp32."""
     out = {}
     if getattr(args, "gpt", True):
-        # GPT-2 small 4-stage pipeline (BASELINE.json metric, second half): all
+        # GPT-2 small 4-stage pipeline (tokens/s beside the images/s): all
         # 4 stages on this GPU, bf16, B=64 sequences x 512-token prompts,
         # microbatched decode ring with one HIP graph per microbatch
         sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "bench"))
@@ -692,7 +692,7 @@ def extra_keys(args, info):
             out[key + "_decode_ms_per_step"] = g["ms_per_step"]
         out["gpt2_4stage_kv8_dtype"] = "bf16 weights/activations, fp8-e4m3 KV cache"
     if getattr(args, "gpt", True) and not args.no_big:
-        # BASELINE.json configs 4 and 5 on this GPU (all stages colocated): Llama-3
+        # the larger workloads on this GPU (all stages colocated): Llama-3
         # 8B bf16 8-stage microbatched decode and GPT-2 XL 8-stage with fp8
         # weights; a failure only drops these keys
         for key, argv, cfg in (
@@ -720,7 +720,7 @@ def extra_keys(args, info):
             except Exception as e:  # noqa: BLE001
                 out[key + "_error"] = f"{type(e).__name__}: {e}"[:200]
             torch.cuda.empty_cache()
-        # the bf16 comparator of config 5's prefill: the same
+        # the bf16 comparator of the fp8 prefill above: the same
         # GPT-2 XL 8-stage B=64 x 512 prefill with bf16 weights
         try:
             g = gpt_bench.run(gpt_bench.parse(["--gpus", "1", "--steps", "2", "--warmup", "1", "--prefill_iters", "1",
@@ -730,7 +730,7 @@ def extra_keys(args, info):
         except Exception as e:  # noqa: BLE001
             out["gpt2xl_bf16_8stage_b64_prefill_error"] = f"{type(e).__name__}: {e}"[:200]
         torch.cuda.empty_cache()
-        # what fp8 weights cost at the model level (VERDICT r4 item 8): the XL
+        # what fp8 weights cost at the model level: the XL
         # stage against the fp32 golden on the ORIGINAL unquantised weights,
         # logits error and greedy-token agreement over 8 decode steps
         try:
@@ -741,7 +741,7 @@ def extra_keys(args, info):
         except Exception as e:  # noqa: BLE001
             out["gpt2xl_fp8_vs_unquantised_fp32_error"] = f"{type(e).__name__}: {e}"[:200]
         torch.cuda.empty_cache()
-        # config 5's prefill on split activations (e4m3 hi + residual planes,
+        # the fp8 prefill on split activations (e4m3 hi + residual planes,
         # bf16-equivalent MFMA work; the former default, kept as a key)
         try:
             g = gpt_bench.run(gpt_bench.parse(["--gpus", "1", "--steps", "4", "--warmup", "1", "--prefill_iters", "1",

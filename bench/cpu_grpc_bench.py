@@ -1,15 +1,15 @@
 #!/usr/bin/env python3
-"""BASELINE config 1 on the reference's own terms: CIFAR-10 2-stage on CPU over
+"""The CPU workload on the reference's own terms: CIFAR-10 2-stage on CPU over
 localhost gRPC, both stages this framework's ``node.py`` processes (CPU fp32
 torch stages, the gRPC data path with the wire schema of
-``/root/reference/node_service.proto``), measured as BASELINE.md's survey
-measured the reference: per request, stage 0's forward + the SendTensor hop +
-stage 1 + the result back; p50 / p99 over the requests, images/s = B / p50.
+``/root/reference/node_service.proto``), measured as the reference's
+own figures were: per request, stage 0's forward + the SendTensor hop + stage 1 +
+the result back; p50 / p99 over the requests, images/s = B / p50.
 
 Differences from the reference are this framework's, not the harness's: one
 persistent channel per hop instead of a new channel per request
-(``node.py:170``), lifted 4 MiB message caps (the reference fails at B >= 256,
-BASELINE.md), the compute off the event loop.
+(``node.py:170``), lifted 4 MiB message caps (the reference fails at B >= 256),
+the compute off the event loop.
 
     python bench/cpu_grpc_bench.py [--batches 1,255,1024] [--requests 60] [--threads 4]
 

@@ -93,7 +93,7 @@ def _build_group(model, ranges, stage_ids, dev, max_batch, max_seq, fp8, kv="bf1
 
 
 def verify_ring(args, info, ring, grp, rep, groups, M, B, V, ranges, max_seq, fp8, kv, sync) -> dict:
-    """The tokens that crossed the hops, checked (VERDICT r5 item 1): the
+    """The tokens that crossed the hops, checked: the
     distributed ring generates ``--verify_steps`` greedy tokens for fixed
     seeded prompts (every microbatch, ``--verify_prompt`` tokens each), then
     rank 0 builds every stage of the model on its own device (same weights:

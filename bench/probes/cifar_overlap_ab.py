@@ -2,7 +2,7 @@
 """A/B: the colocated CIFAR 2-stage step serial (one stream, one graph: the
 bench headline) vs stage 1 (fc1 + fc2/softmax/argmax) of microbatch m running
 on a second stream under stage 0 of microbatch m+1, with the persistent
-stage-0 grid leaving ``spare`` CUs free for fc1 (VERDICT r3 item 7).  Both
+stage-0 grid leaving ``spare`` CUs free for fc1.  Both
 arms are single HIP graphs (the overlapped one forks/joins streams inside the
 capture), fp32 (bf16x3) precision, B = 65536 images per step, interleaved
 rounds in one process.  Outputs must be identical to the serial arm.

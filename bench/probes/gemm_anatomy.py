@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Anatomy of a 256^2 prefill GEMM tile (VERDICT r5 items 4 / 5): the same
+"""Anatomy of a 256^2 prefill GEMM tile: the same
 launch with the epilogue's stores skipped (probe bit 1), with the main loop
 skipped (bit 2: prologue DMAs, their wait and the epilogue), and both (3),
 against the product launch (0), interleaved ``--rounds`` times.  Per shape:

@@ -12,7 +12,7 @@ decode projection at B = 64, timed whole and with parts removed —
     empty     the launch alone (every wave returns at once)
     no_red    no cross-wave reduction through LDS (each wave's partial stored)
     no_ld_no_red  neither loads nor the reduction
-    counted_wait  the round-4/5 image wait (vmcnt(weights after the image)
+    counted_wait  the earlier image wait (vmcnt(weights after the image)
                   instead of vmcnt(0)): with two steps, step 0 computes while
                   step 1's weights land — racy (gemm_oneshot.h "Retiring the
                   image"), measured here only for what the fix costs

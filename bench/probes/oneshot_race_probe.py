@@ -1,5 +1,5 @@
-"""Root-cause probe of the one-shot decode GEMM race (
-csrc/kernels/gemm_oneshot.h "Retiring the image").
+"""Root-cause probe of the one-shot decode GEMM race
+(csrc/kernels/gemm_oneshot.h "Retiring the image").
 
 Symptom (profiles/r5_oneshot_race_screen_*.jsonl): in ~2 % of forced
 LN + GELU calls at 2/1/1 (288 or 384 workgroups, two per CU) one workgroup's
@@ -15,7 +15,7 @@ Each experiment compares ``--iters`` calls bit for bit with a settled
 reference of the same launch; every call follows a call on other activations
 (the LDS holds someone else's bytes).  Probe bits (gemm_oneshot.h) select
 instrumented or alternative image syncs; profiles/r6_oneshot_race_root_cause.md
-tells the story of the round-6 runs (LDS floors 0 / 72 / 82 KB, an entry
+tells the story of these runs (LDS floors 0 / 72 / 82 KB, an entry
 barrier, a detector, CK's split waits, ck_tile's vmcnt-only wait, a short
 s_sleep, a second barrier, register-staged images, the dump, the SLP A/B).
 One JSON line per experiment."""

@@ -1,5 +1,5 @@
-"""Host issue cost of the decode ring per microbatch item vs its device time
-(VERDICT r4 item 7): can one Python rank keep its GPU busy at N = 4 / 8?
+"""Host issue cost of the decode ring per microbatch item vs its device time:
+can one Python rank keep its GPU busy at N = 4 / 8?
 
 One rank of a multi-GPU decode ring does, per microbatch item
 (``runtime/scheduler.py DecodeRing.decode_rounds``): wait on the input

@@ -146,7 +146,7 @@ __device__ __forceinline__ int k_swz(int key, int chunk) {
 // two score accumulators, so block j+1's S = K Q^T MFMAs are issued before
 // block j's softmax and P.V — the matrix pipe works through the softmax VALU
 // of the same wave instead of waiting on the S -> max -> exp -> P.V chain
-// (VERDICT r4 item 6; PMC before: MFMA 0.14 busy, profiles/r4_pmc_flash_lpt.md).
+// (PMC before: MFMA 0.14 busy, profiles/r4_pmc_flash_lpt.md).
 // Measured slower, so off by default: GPT-2 B=64 T=512 0.0950 -> 0.1075 ms,
 // B=8 T=2048 0.0851 -> 0.0986, 4-stage prefill 4.21 -> 4.13 M tok/s
 // (profiles/r5_flash_pipe_ab.jsonl): the second accumulator takes the kernel

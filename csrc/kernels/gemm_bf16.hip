@@ -567,7 +567,7 @@ static int launch_gemm(const void* A, int lda, const void* W, int ldw, void* C, 
                        rowstat, colsum);
     return (int)hipGetLastError();
   }
-  // Tail split (round 4): when the 256^2 grid is full rounds plus a last
+  // Tail split: when the 256^2 grid is full rounds plus a last
   // column of tiles that fills at most one more round as 256x128 tiles (GPT-2's
   // 768-wide O / c_proj at M = 32768: 256 tiles + a 128-tile column), the
   // first N - 256 columns run as 256^2 tiles and the last 256 as 256x128 tiles

@@ -172,7 +172,7 @@ __device__ __forceinline__ void epi_t4_pre(f32x4 v, int m, int n, void* __restri
 }
 
 // Row-statistics partial of one 16-column output tile, produced in the
-// epilogue of a residual-writing decode GEMM (VERDICT r4 item 2) so that the
+// epilogue of a residual-writing decode GEMM so that the
 // next pre-norm projection merges ~N/16 partials per row instead of
 // re-deriving the statistics from its activations in every column-tile
 // workgroup.  Transposed-accumulator layout: lane (fr = l & 15, fg = l >> 4)

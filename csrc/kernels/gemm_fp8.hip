@@ -1,5 +1,5 @@
 // FP8 (OCP e4m3fn) GEMM on the CDNA4 block-scaled MFMA, plus the per-token
-// activation quantizer. North-star config 5 (GPT-2 XL, fp8 weights).
+// activation quantizer. GPT-2 XL, fp8 weights.
 //
 //   C[M,N] = act( (Aq[M,K] . Wq[N,K]^T) * sa[m] * sw[n] + bias[n] ) (+ R[M,N])
 //

@@ -1,5 +1,5 @@
 // Decode vocabulary head with the greedy argmax's first pass ("head" kernel,
-// round 4: the tied 50304-wide head toward its byte floor).
+// the tied 50304-wide head toward its byte floor).
 //
 //   logits[m, n] = bf16( rstd[m] (A[m,:] . W'[n,:] - mean[m] colsum[n]) + bias'[n] )
 //   part[m, wg]  = argmax over this workgroup's columns of logits[m, :]

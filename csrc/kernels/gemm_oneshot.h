@@ -28,7 +28,7 @@
 //   * the A rows are issued first, then the weights step-major; the folded
 //     norm's row statistics are taken from the image once every load has
 //     landed and the workgroup has synchronised ("Retiring the image"
-//     below; the round-4 version took them under the weight flight, measured
+//     below; an earlier version took them under the weight flight, measured
 //     neutral against taking them from the MFMA fragments,
 //     profiles/r4_oneshot_norm_ab*.jsonl);
 //   * MFMAs from LDS fragments x register weights; the 4
@@ -58,13 +58,13 @@ constexpr int os_lds_bytes() {
 // ABL (probe only, bench/probes/oneshot_anatomy.py; 0 in every product launch):
 // bit 1 no weight loads, 2 no activation image, 4 no MFMAs, 8 no epilogue
 // stores, 32 return at once (the launch alone), 64 no cross-wave reduction
-// (each wave's own partial goes to the epilogue), 128 the round-4/5 counted
+// (each wave's own partial goes to the epilogue), 128 the earlier counted
 // image wait (racy, below) — what each part costs.
 //
 // Retiring the image.  The image is read only after composable_kernel's
 // direct-load sequence (block_sync_lds_direct_load: vmcnt(0), lgkmcnt(0),
 // s_barrier), not after a count of the weights issued behind it: an LDS-DMA is
-// not ordered with the plain loads that follow it.  The round-4/5 counted wait
+// not ordered with the plain loads that follow it.  The earlier counted wait
 // stays as the probe bit ABL 128; the sync costs nothing measurable
 // (oneshot_anatomy.py counted_wait arm within +-0.13 us,
 // profiles/r5_oneshot_anatomy_imagesync.jsonl).  Plain loads issued before

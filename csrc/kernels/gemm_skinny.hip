@@ -425,7 +425,7 @@ using namespace dnn;
 
 constexpr int SKINNY_MAX_M = 256;  // M > 64 only through the M split (medium-batch decode)
 
-// Producer-side row statistics (VERDICT r4 item 2, gemm_epilogue.h
+// Producer-side row statistics (gemm_epilogue.h
 // epi_rowstat16 / rowstat_merge): dnn_gemm_rowstats() arms the NEXT decode
 // GEMM call of this thread — ``out`` (float2 [M][ld], ld >= ceil(N/16)): the
 // call's kernel writes per-16-column-tile partials of its bf16 output rows;

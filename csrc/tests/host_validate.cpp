@@ -1,6 +1,6 @@
 // Host-side validation of the kernel C ABI under AddressSanitizer / UBSan
 // (tests/test_host_sanitizer.py builds this with `-Xarch_host -fsanitize=...`:
-// the GPU sanitizer is not available on this pool, so the host half of every
+// the GPU sanitizer is not available here, so the host half of every
 // entry point — shape checks, config tables, the guards that keep a kernel
 // from being launched with operands its grid does not cover — is what runs
 // instrumented).  Every call below must be REJECTED before any launch, so the

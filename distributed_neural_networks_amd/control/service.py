@@ -3,7 +3,7 @@
 Wire-compatible with the reference service (``node_service.proto:4-8``,
 method paths ``/node_service.NodeService/{SendMessage,HealthCheck,SendTensor}``)
 so a reference ``node.py`` peer can talk to this one.  Differences from the
-reference servicer (``node.py:34-133``), all deliberate (SURVEY A.5):
+reference servicer (``node.py:34-133``), all deliberate:
 
 * message-size caps lifted (the reference's default 4 MiB receive cap makes
   CIFAR batches >= 256 and GPT logits > ~20 tokens fail);

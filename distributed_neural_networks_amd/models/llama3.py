@@ -1,4 +1,4 @@
-"""Llama-3 golden model and stage modules (north-star config 4; not in the reference).
+"""Llama-3 golden model and stage modules (not in the reference).
 
 RMSNorm, RoPE (theta 500000, rotate-half convention as HF), grouped-query
 attention (32 q / 8 kv heads of 128 for 8B), SwiGLU MLP, untied ``lm_head``.

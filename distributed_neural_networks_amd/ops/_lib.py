@@ -107,7 +107,7 @@ def check(rc: int, what: str) -> None:
     """Raise on a rejected/failed launch.  With ``DNN_DEBUG_SYNC=1`` every kernel
     is followed by a device sync so an asynchronous fault (bad address, hang)
     is attributed to the launch that caused it (race/fault triage mode; the
-    GPU-side sanitizer is not available on this pool)."""
+    GPU-side sanitizer is not available)."""
     if rc != 0:
         raise RuntimeError(f"{what}: HIP launch failed with code {rc}")
     if DEBUG_SYNC:

@@ -9,7 +9,7 @@ Rendezvous: ``torchrun``-style env (``RANK``/``WORLD_SIZE``/``MASTER_ADDR``/
 ``MASTER_PORT``) when present; otherwise derived from the pipeline config —
 rank = ``part_index``, world = ``num_parts``, master = stage 0's host and its
 port + ``PORT_OFFSET`` (the gRPC control plane keeps the configured port).
-The reference has no collective runtime at all (SURVEY §0.3); its only
+The reference has no collective runtime at all; its only
 "barrier" is ``asyncio.sleep(2)`` (``node.py:203-207``) — process-group init
 is a real barrier.
 """

@@ -1,6 +1,6 @@
 """Native RCCL data plane: Python face of ``csrc/comm/p2p.cpp``.
 
-The SURVEY §7.1 data plane: stage hops go straight to RCCL
+The data plane: stage hops go straight to RCCL
 (``ncclSend``/``ncclRecv``) on channels this package owns, not through
 ProcessGroupNCCL's P2P.
 

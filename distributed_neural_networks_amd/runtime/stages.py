@@ -6,7 +6,7 @@
   packed once at load (``ops/cifar.py``; fp32 by default, the reference's
   precision, or bf16); no torch op runs in ``forward``.
 * ``TorchStage`` — the golden torch module on CPU (fp32): the data path of the
-  reference's CPU/gRPC configuration (``BASELINE.json`` configs[0]) and the
+  reference's CPU/gRPC configuration and the
   oracle in tests.  It is never used on a GPU device.
 
 The GPT-2 / Llama stages live in ``runtime/transformer.py`` (same interface).

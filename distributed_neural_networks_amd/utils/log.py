@@ -1,7 +1,7 @@
 """Logging: the reference prints ``[node_id] ...`` lines to stdout
 (``node.py:38-39,62,192``) and its output is block-buffered when piped; here
 every line is flushed so multi-process runs interleave readably, and the key
-reference lines keep their exact text (SURVEY Appendix A.4)."""
+reference lines keep their exact text."""
 from __future__ import annotations
 
 import sys

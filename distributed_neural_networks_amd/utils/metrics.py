@@ -1,6 +1,6 @@
 """Per-stage metrics: counters and latency samples, emitted as one JSON line.
 
-The reference only prints (metrics/logging).  A ``StageMetrics``
+The reference only prints.  A ``StageMetrics``
 object is owned by each stage loop / servicer; ``summary()`` gives requests,
 items, throughput and p50/p99 latency, and ``emit()`` prints
 ``METRICS {...}`` (one line, machine-readable) — enabled by ``--metrics`` or

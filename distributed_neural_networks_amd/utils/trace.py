@@ -1,7 +1,7 @@
 """Tracing: host spans + device-timed spans -> Chrome trace JSON, plus roctx
 ranges so ``rocprofv3 --marker-trace`` timelines show the same phases.
 
-The reference has no tracing (SURVEY §5).  Enable with ``DNN_TRACE=out.json``
+The reference has no tracing.  Enable with ``DNN_TRACE=out.json``
 (or ``trace.enable(path)``); every ``span(name)`` then records
 ``[start, end)`` on the host clock and, when a CUDA/HIP device is given, a
 pair of ``hipEvent``s whose device timestamps are resolved at flush (no

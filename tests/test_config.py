@@ -165,7 +165,7 @@ def test_rccl_device_mapping_validated(tmp_path):
 
 
 def test_fp8_prefill_default_is_mx_e4m3(tmp_path):
-    """ADVICE r5: the fp8 prefill default is the one-byte MX path ("e4m3");
+    """The fp8 prefill default is the one-byte MX path ("e4m3");
     its end-to-end error budget against the unquantised model is pinned on
     the GPU by tests/test_transformer_gpu.py::test_fp8_fidelity_vs_unquantised
     (prefill logits < 0.13 rel, greedy agreement >= 0.6 on GPT-2 XL blocks)

@@ -1,4 +1,4 @@
-"""BASELINE config 1 harness (bench/cpu_grpc_bench.py): two node.py processes on
+"""CPU workload's harness (bench/cpu_grpc_bench.py): two node.py processes on
 CPU over localhost gRPC, stage 0 recording each request's end-to-end latency
 (--metrics), at the reference's batch 1 and past its 4 MiB message cap."""
 import json

@@ -248,7 +248,7 @@ def _bench_cpu(n, *extra, timeout=420, launcher="torchrun", gpus=None):
     if launcher == "torchrun":
         cmd = [sys.executable, "-m", "torch.distributed.run", "--nnodes=1", "--nproc-per-node", str(n),
                "--master-addr", "127.0.0.1", "--master-port", str(free_port()), *args]
-    else:  # exactly as the driver invokes it: no launcher, bench.py spawns its own ranks
+    else:  # invoked without a launcher, bench.py spawns its own ranks
         cmd = [sys.executable, *args]
     env = dict(ENV, OMP_NUM_THREADS="1")
     for k in ("RANK", "WORLD_SIZE", "LOCAL_RANK", "MASTER_ADDR", "MASTER_PORT"):
@@ -262,11 +262,11 @@ def _bench_cpu(n, *extra, timeout=420, launcher="torchrun", gpus=None):
 
 @pytest.mark.parametrize("n,launcher", [(2, "torchrun"), (4, "self"), (8, "torchrun")])
 def test_bench_pp2_schedule_cpu(n, launcher):
-    """bench.py's N > 1 headline with gloo on CPU (the driver's N = 2/4/8
+    """bench.py's N > 1 headline with gloo on CPU (N = 2/4/8
     scaling runs use the same schedule over RCCL): the reference cut and
     metric at every N, a real p50 through the hop and back, and the extra
-    keys of BASELINE configs 3-5 (decode rings with per-token p50).  N = 4
-    runs as the driver launches it, ``python bench.py --gpus 4`` with no
+    keys of the decode rings (with per-token p50).  N = 4
+    runs as ``python bench.py --gpus 4`` with no
     launcher: bench.py must spawn the 4 ranks itself."""
     d = _bench_cpu(n, launcher=launcher)
     assert d["n_gpus"] == n and d["value"] > 0 and d["metric"] == "images/sec CIFAR-10 2-stage"
@@ -286,7 +286,7 @@ def test_bench_pp2_schedule_cpu(n, launcher):
     assert "hop_GBps_error" not in d and d["hop_GBps_per_pair"] > 0
     assert d["hop_bound_images_per_s"] == pytest.approx((n // 2) * d["hop_GBps_per_pair"] * 1e9 / 16384, rel=0.02)
     assert "extras_error" not in d and d["fc1cut_images_per_s"] > 0
-    # the answer that crossed the hops (VERDICT r5 item 1): every stage-0 rank's
+    # the answer that crossed the hops: every stage-0 rank's
     # images through the distributed pipeline and back, against fp32 torch
     assert "dist_verify_error" not in d, d.get("dist_verify_error")
     assert d["dist_argmax_agreement_vs_fp32_torch"] == 1.0

@@ -1,6 +1,5 @@
-"""Host AddressSanitizer + UBSan run of the kernel library's C ABI (SURVEY §5,
-race detection / sanitizers).  GPU-side ASan / xnack+ builds are not available
-on this pool, so the HOST half of every kernel source is compiled with the
+"""Host AddressSanitizer + UBSan run of the kernel library's C ABI.
+GPU-side ASan / xnack+ builds are not available, so the HOST half of every kernel source is compiled with the
 sanitizers (``--offload-host-only -Xarch_host -fsanitize=...``; the device half
 is never run here and would take minutes to compile) and linked with
 ``csrc/tests/host_validate.cpp``, which drives every entry point with shapes

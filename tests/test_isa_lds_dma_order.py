@@ -10,7 +10,7 @@ reads the assembly of the product instantiations (the planned GPT-2 / GPT-2
 XL decode configurations and the forced test shapes) and of the fused LM head
 (gemm_head.h, one image per K pass) and asserts, on every control-flow path,
 that no LDS read follows an LDS-DMA without a vmcnt(0) and then an s_barrier
-in between.  The round-4/5 counted-wait variant (probe bit ABL 128) is
+in between.  The earlier counted-wait variant (probe bit ABL 128) is
 compiled too and must be flagged, so the check is known to see what it
 guards.
 

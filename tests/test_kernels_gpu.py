@@ -301,7 +301,7 @@ def test_cifar_fp32_stage0_and_head(B):
 
 @pytest.mark.parametrize("boundary", ["fp32", "split"])
 def test_cifar_fp32_pipeline_4096_images_matches_reference(boundary):
-    """Acceptance (VERDICT r1 item 1): the 2-stage pipeline at the reference's
+    """Acceptance: the 2-stage pipeline at the reference's
     precision on 4096 images: max |dprob| <= 1e-5 vs fp32 torch
     (cifar_model_parts.py:7-26) and 100 % argmax agreement (rows whose golden
     top-2 probabilities tie within 1e-6 are excluded as numerically undecidable)."""

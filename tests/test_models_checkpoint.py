@@ -11,7 +11,7 @@ from distributed_neural_networks_amd.parallel.partition import balanced_ranges, 
 
 
 def test_cifar_split_equals_full():
-    # reference property: ModelPart1(ModelPart0(x)) == NeuralNetwork(x) (SURVEY §0.7)
+    # reference property: ModelPart1(ModelPart0(x)) == NeuralNetwork(x)
     torch.manual_seed(0)
     full = cifar.NeuralNetwork().eval()
     sd = full.state_dict()

@@ -1,5 +1,5 @@
-"""Multi-GPU paths over RCCL/xGMI (SURVEY §4.2 item 5): one process per GPU,
-launched exactly the way the driver launches the bench — ``python3 bench.py
+"""Multi-GPU paths over RCCL/xGMI: one process per GPU,
+launched the way a user launches the bench — ``python3 bench.py
 --gpus N`` with no launcher, so bench.py spawns its own ranks
 (``parallel/selflaunch.py``).  Skipped below 2 visible GPUs (conftest:
 ``multigpu``); RCCL refuses two ranks on one device, so the 1-GPU box cannot
@@ -31,7 +31,7 @@ def _port():
 
 
 def _bench(*args, timeout=600):
-    """``python3 bench.py ...`` as the driver runs it; returns rank 0's one JSON line."""
+    """``python3 bench.py ...``; returns rank 0's one JSON line."""
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), *args], env=ENV, capture_output=True,
                        text=True, timeout=timeout, cwd=ROOT)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-3000:]
@@ -62,7 +62,7 @@ def _check_dist_verify(d, n):
 def test_bench_pp2_headline(n):
     """The N > 1 headline: the reference cut, one stage per GPU, the hop over
     this package's native RCCL channels (not a ProcessGroupNCCL fallback);
-    at 4 and 8 GPUs the bipartite SplitLink hop the driver's scaling run takes.
+    at 4 and 8 GPUs the bipartite SplitLink hop a scaling run takes.
     The line must carry the distributed correctness keys at 1.0."""
     _need(n)
     d = _bench("--gpus", str(n), "--steps", "3", "--warmup", "1", "--batch", "8192", "--latency_iters", "5",
@@ -85,8 +85,8 @@ def test_bench_fc1cut_two_gpus():
 
 @pytest.mark.parametrize("n", [2, 4, 8])
 def test_bench_full_line(n):
-    """The complete multi-GPU line the driver records: headline plus the
-    fc1-cut and the BASELINE config 3/4/5 decode rings over RCCL, each ring's
+    """The complete multi-GPU line: headline plus the
+    fc1-cut and the three decode rings over RCCL, each ring's
     greedy tokens equal to the same stages colocated on rank 0's GPU."""
     _need(n)
     d = _bench("--gpus", str(n), "--steps", "5", "--warmup", "2", timeout=1100)

@@ -186,7 +186,7 @@ def test_preflight_pattern_distinguishes_messages():
 def test_nested_empty_scopes_close_their_own_frames(fake_rccl):
     """Two nested scopes that both open nothing new (equal, empty frames):
     the inner one's exit must pop the inner frame, so a channel the outer
-    block opens afterwards is still closed by the outer scope (ADVICE r4)."""
+    block opens afterwards is still closed by the outer scope."""
     rccl = fake_rccl
     dev = torch.device("cpu")
     st = _FakeStore()

@@ -6,7 +6,7 @@ caller's stream, completion tokens, HIP graph capture of a hop, counters —
 and a 2-process pair channel on the same GPU runs the real pair bootstrap
 through the TCP store (RCCL may refuse two ranks on one device; that refusal
 must then surface as a clean init error, not a hang).  Cross-GPU hops over
-xGMI run in the driver's multi-GPU bench.
+xGMI run in the multi-GPU bench.
 """
 import os
 import socket

@@ -1,4 +1,4 @@
-"""End-to-end pipeline tests on one MI355X (SURVEY §4.2 items 4 and 7.5).
+"""End-to-end pipeline tests on one MI355X.
 
 * the minimum slice through the reference CLI: ``node.py`` with a colocated
   2-stage CIFAR config, a real ``.pth`` and a PNG, prediction == torch golden;

@@ -202,7 +202,7 @@ def test_cli_cifar_3_stages_microbatched_gloo(tmp_path):
 
 def test_cli_return_to_middle_stage_gloo(tmp_path):
     """return_to_node_id naming a middle stage: predictions arrive there (the
-    round-1 CLI sent them to a rank that never received, and hung)."""
+    first CLI sent them to a rank that never received, and hung)."""
     from distributed_neural_networks_amd.checkpoint import make_full_checkpoint
     ck = tmp_path / "c.pth"
     make_full_checkpoint("cifar10", str(ck), 4)

@@ -341,7 +341,7 @@ def test_epilogue_prefetch_bit_identical(path, N, K, w8, epi):
 
 @pytest.mark.parametrize("N,floor_kb", [(3072, 0), (2304, 0), (3072, 72)])
 def test_oneshot_coresident_race_screen(N, floor_kb):
-    """VERDICT r5 item 2 regression: the forced one-shot LN + GELU grid with
+    """Regression: the forced one-shot LN + GELU grid with
     TWO workgroups per CU (LDS floor 0, or a 72 KB floor: padded but still two
     per CU), every call after a poisoning call on other activations, bit-
     identical to the settled reference in all 3000 calls.  The SLP build of

@@ -1249,7 +1249,7 @@ def test_llama3_8b_two_blocks_full_width_vs_golden(B, T):
     gains: a prefill (256^2 GEMMs, flash attention, qkv_split RoPE) and 8
     KV-cached decode steps (decode GEMMs, MFMA GQA decode attention) against
     the fp32 torch golden, logits within 2e-2 relative.  B = 32, T = 512 is
-    the bench's shape (config 4): 16 K-row prefill GEMMs, 32-row decode
+    the bench's shape: 16 K-row prefill GEMMs, 32-row decode
     GEMMs (the stream / one-shot kernels) and the decode attention
     over 512+ keys."""
     from distributed_neural_networks_amd import checkpoint as ckpt
@@ -1420,7 +1420,7 @@ def test_fp8_split_activation_planes(M, K):
 @pytest.mark.parametrize("N", [400, 1040, 272])
 @pytest.mark.parametrize("w8", [False, True])
 def test_rowstats_partial_width(N, w8):
-    """widths that are not a multiple of the kernels' column tiles
+    """Widths that are not a multiple of the kernels' column tiles
     (16 NT / 16 NTW): a surplus tile past the row must write no partial (it
     used to write NaN into the next row's partial 0).  Every partial of the
     row's ceil(N/16) tiles matches torch; a guard row past M stays untouched."""
@@ -1461,7 +1461,7 @@ def test_rowstats_partial_width(N, w8):
                                       (64, 1600, 6400, 6400), (48, 768, 768, 2304)])
 @pytest.mark.parametrize("w8", [False, True])
 def test_rowstats_producer_consumer(M, N, K, N2, w8):
-    """Producer-side decode row statistics (VERDICT r4 item 2): a residual-
+    """Producer-side decode row statistics: a residual-
     writing projection (one-shot / skinny kernel) writes {mean, M2} per 16-
     column tile of its bf16 output rows — checked against torch on the stored
     output, including rows with |mean| / std >= 50 — and the next folded-LN
@@ -1632,7 +1632,7 @@ def test_gemm_fp8_mx(M, N, K, act, res):
 
 
 def test_fp8_fidelity_vs_unquantised():
-    """what fp8 weights cost against the model itself — the
+    """What fp8 weights cost against the model itself — the
     GPT-2 XL fp8 stage (2 full-width blocks + head) against the fp32 golden on
     the ORIGINAL unquantised weights, both prefill modes, plus the bf16 stage
     as the floor.  Bounds sit above the measured 2-block values (B=64, T=512:
