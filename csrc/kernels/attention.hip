@@ -957,6 +957,11 @@ extern "C" int dnn_qkv_split(const void* qkv, void* q, void* kc, void* vc, int B
 // (8 at hd 128).  us, one : two groups: GPT-2 161 tokens 5.8 : 6.0, 192 6.0 : 6.1, 193 6.9 :
 // 6.6, 3 x 357 9.4 : 8.6, 960 18.0 : 14.6, 4 x 600 13.7 : 11.6; XL 8 x 256 (400 workgroups)
 // 9.4 : 12.9; Llama-3 449 15.2 : 14.7, 700 20.6 : 18.9, 1000 27.9 : 24.8, 300 11.2 : 11.5.
+//
+// `one_group` (the caller's): where e4m3 activations follow.  They make a step of 1/8 to 1/16
+// of what rounds differently in bf16: with the keys in another order a GPT-2 XL pass of 490
+// tokens (6 blocks) differs by 4.4 %, as much as either order from 64 bits, and takes 481 us
+// in place of 492.
 constexpr int FA_KS_WGS = 256;
 template <int HD>
 static bool flash_two_groups(long wgs, int T) {
@@ -964,7 +969,8 @@ static bool flash_two_groups(long wgs, int T) {
 }
 template <int HD, bool QKV, bool KV8>
 static void launch_flash(dim3 grid, hipStream_t st, const bf16_t* q, const bf16_t* kc, const bf16_t* vc, bf16_t* o,
-                         int T, int H, int Hkv, int S, const int* pos, float sl2, int ldq, bf16_t* kco, bf16_t* vco) {
+                         int T, int H, int Hkv, int S, const int* pos, float sl2, int ldq, bf16_t* kco, bf16_t* vco,
+                         bool one_group) {
   // double-buffered K/V LDS, one barrier per block (default): GPT-2 B=64 T=512 0.1075 -> 0.1063 ms,
   // hd 128 T=512 0.251 -> 0.243, T=4096 1.123 -> 1.092 (profiles/r3_flash_double_buffer.jsonl);
   // DNN_FLASH_DB=0 keeps the single buffer (A/B)
@@ -978,7 +984,7 @@ static void launch_flash(dim3 grid, hipStream_t st, const bf16_t* q, const bf16_
     }
   }
   const long wgs = (long)grid.x * grid.y * grid.z;
-  if (e == nullptr && flash_two_groups<HD>(wgs, T))  // DNN_FLASH_DB pins a one-group variant
+  if (e == nullptr && !one_group && flash_two_groups<HD>(wgs, T))  // DNN_FLASH_DB pins a one-group variant
     hipLaunchKernelGGL((flash_attn_kernel<HD, QKV, KV8, true, false, 2>), grid, dim3(512), 0, st, q, kc, vc, o, T, H,
                        Hkv, S, pos, sl2, ldq, kco, vco);
   else if (e == nullptr || atoi(e) != 0)
@@ -990,7 +996,7 @@ static void launch_flash(dim3 grid, hipStream_t st, const bf16_t* q, const bf16_
 }
 
 extern "C" int dnn_flash_attn(const void* q, const void* kc, const void* vc, void* o, int B, int T, int H, int Hkv,
-                              int hd, int S, const int* pos, float scale, hipStream_t st, int kv8) {
+                              int hd, int S, const int* pos, float scale, hipStream_t st, int kv8, int one_group) {
   if (H % Hkv != 0) return -1;
   dim3 grid(H, B, (T + FA_QB - 1) / FA_QB);
   const float sl2 = scale * 1.4426950408889634f;
@@ -998,15 +1004,15 @@ extern "C" int dnn_flash_attn(const void* q, const void* kc, const void* vc, voi
   bf16_t* o_ = (bf16_t*)o;
   if (kv8) {  // e4m3 cache: every key / value row widened as it is fetched
     if (hd == 64)
-      launch_flash<64, false, true>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, 0, nullptr, nullptr);
+      launch_flash<64, false, true>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, 0, nullptr, nullptr, one_group != 0);
     else if (hd == 128)
-      launch_flash<128, false, true>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, 0, nullptr, nullptr);
+      launch_flash<128, false, true>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, 0, nullptr, nullptr, one_group != 0);
     else
       return -2;
   } else if (hd == 64) {
-    launch_flash<64, false, false>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, 0, nullptr, nullptr);
+    launch_flash<64, false, false>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, 0, nullptr, nullptr, one_group != 0);
   } else if (hd == 128) {
-    launch_flash<128, false, false>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, 0, nullptr, nullptr);
+    launch_flash<128, false, false>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, 0, nullptr, nullptr, one_group != 0);
   } else {
     return -2;
   }
@@ -1015,7 +1021,8 @@ extern "C" int dnn_flash_attn(const void* q, const void* kc, const void* vc, voi
 
 // Prefill straight from the c_attn output (no RoPE): see flash_attn_kernel<HD, true>.
 extern "C" int dnn_flash_attn_qkv(const void* qkv, int ldqkv, void* kc, void* vc, void* o, int B, int T, int H,
-                                  int Hkv, int hd, int S, const int* pos, float scale, hipStream_t st, int kv8) {
+                                  int Hkv, int hd, int S, const int* pos, float scale, hipStream_t st, int kv8,
+                                  int one_group) {
   if (H % Hkv != 0 || ldqkv < (H + 2 * Hkv) * hd || (ldqkv % 8) != 0) return -1;
   dim3 grid(H, B, (T + FA_QB - 1) / FA_QB);
   const float sl2 = scale * 1.4426950408889634f;
@@ -1023,15 +1030,15 @@ extern "C" int dnn_flash_attn_qkv(const void* qkv, int ldqkv, void* kc, void* vc
   bf16_t *o_ = (bf16_t*)o, *ko = (bf16_t*)kc, *vo = (bf16_t*)vc;
   if (kv8) {  // e4m3 cache (unit scale)
     if (hd == 64)
-      launch_flash<64, true, true>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, ldqkv, ko, vo);
+      launch_flash<64, true, true>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, ldqkv, ko, vo, one_group != 0);
     else if (hd == 128)
-      launch_flash<128, true, true>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, ldqkv, ko, vo);
+      launch_flash<128, true, true>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, ldqkv, ko, vo, one_group != 0);
     else
       return -2;
   } else if (hd == 64) {
-    launch_flash<64, true, false>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, ldqkv, ko, vo);
+    launch_flash<64, true, false>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, ldqkv, ko, vo, one_group != 0);
   } else if (hd == 128) {
-    launch_flash<128, true, false>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, ldqkv, ko, vo);
+    launch_flash<128, true, false>(grid, st, q_, k_, v_, o_, T, H, Hkv, S, pos, sl2, ldqkv, ko, vo, one_group != 0);
   } else {
     return -2;
   }

@@ -152,6 +152,7 @@ struct PrefillPass {
   int run(const std::vector<PrefillBlock>& blocks) {
     const void* in = x;
     const int nq = (H + 2 * Hkv) * hd;
+    const int one_group = fp8 && rows() > skinny_max;  // e4m3 activations follow (attention.hip flash_two_groups)
     const bool up_quant = fp8 && act == 2 && !skinny(n_up, d, true, true, 0);
     for (size_t i = 0; i < blocks.size(); ++i) {
       const PrefillBlock& L = blocks[i];
@@ -160,18 +161,18 @@ struct PrefillPass {
       if (scattered(in, L.qkv, k, v, rc)) {
         if (rc) return rc;
         what = "flash_attn";
-        rc = dnn_flash_attn(q, k, v, att, B, T, H, Hkv, hd, S, pos, scale, st);
+        rc = dnn_flash_attn(q, k, v, att, B, T, H, Hkv, hd, S, pos, scale, st, 0, one_group);
       } else {
         if (rc) return rc;
         if ((rc = norm_proj(in, L.qkv, qkv, nq, nq, 0, true, false))) return rc;
         if (cosT == nullptr) {
           what = "flash_attn_qkv";
-          rc = dnn_flash_attn_qkv(qkv, nq, k, v, att, B, T, H, Hkv, hd, S, pos, scale, st);
+          rc = dnn_flash_attn_qkv(qkv, nq, k, v, att, B, T, H, Hkv, hd, S, pos, scale, st, 0, one_group);
         } else {
           what = "qkv_split";
           if ((rc = dnn_qkv_split(qkv, q, k, v, B, T, H, Hkv, hd, S, pos, cosT, sinT, 1, st))) return rc;
           what = "flash_attn";
-          rc = dnn_flash_attn(q, k, v, att, B, T, H, Hkv, hd, S, pos, scale, st);
+          rc = dnn_flash_attn(q, k, v, att, B, T, H, Hkv, hd, S, pos, scale, st, 0, one_group);
         }
       }
       if (rc) return rc;

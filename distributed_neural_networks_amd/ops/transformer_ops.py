@@ -140,20 +140,23 @@ def qkv_split(qkv: torch.Tensor, q: torch.Tensor, kc: torch.Tensor, vc: torch.Te
 
 
 def flash_attn(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, out: torch.Tensor, B: int, T: int, H: int,
-               Hkv: int, hd: int, pos: torch.Tensor, scale: Optional[float] = None) -> torch.Tensor:
+               Hkv: int, hd: int, pos: torch.Tensor, scale: Optional[float] = None,
+               one_group: bool = False) -> torch.Tensor:
     """Causal attention of T new queries per sequence against the cache
-    (positions 0..pos[b]+T-1). q (B,H,T,hd); out (B*T, H*hd)."""
+    (positions 0..pos[b]+T-1). q (B,H,T,hd); out (B*T, H*hd).  ``one_group``: the keys in
+    one order whatever the grid (attention.hip flash_two_groups)."""
     if hd not in (64, 128):
         raise ValueError(f"flash_attn: head_dim {hd} unsupported (64/128)")
     S = kc.shape[2]
     scale = scale if scale is not None else 1.0 / math.sqrt(hd)
     check(lib().flash_attn(ptr(q), ptr(kc), ptr(vc), ptr(out), B, T, H, Hkv, hd, S, ptr(pos), scale, stream_ptr(),
-                           kv8=_kv8(kc, vc)), "flash_attn")
+                           kv8=_kv8(kc, vc), one_group=int(one_group)), "flash_attn")
     return out
 
 
 def flash_attn_qkv(qkv: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, out: torch.Tensor, B: int, T: int, H: int,
-                   Hkv: int, hd: int, pos: torch.Tensor, scale: Optional[float] = None) -> torch.Tensor:
+                   Hkv: int, hd: int, pos: torch.Tensor, scale: Optional[float] = None,
+                   one_group: bool = False) -> torch.Tensor:
     """Causal prefill straight from the c_attn output (no RoPE): qkv (B*T, ld)
     rows [q | k | v]; the new keys/values are written into the cache rows
     pos[b].. as a side effect (what qkv_split would have done)."""
@@ -168,7 +171,7 @@ def flash_attn_qkv(qkv: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, out: t
         raise ValueError("flash_attn_qkv: cache slices must be contiguous")
     scale = scale if scale is not None else 1.0 / math.sqrt(hd)
     check(lib().flash_attn_qkv(ptr(qkv), qkv.stride(0), ptr(kc), ptr(vc), ptr(out), B, T, H, Hkv, hd, S, ptr(pos),
-                               scale, stream_ptr(), kv8=_kv8(kc, vc)), "flash_attn_qkv")
+                               scale, stream_ptr(), kv8=_kv8(kc, vc), one_group=int(one_group)), "flash_attn_qkv")
     return out
 
 

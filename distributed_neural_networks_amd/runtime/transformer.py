@@ -453,6 +453,7 @@ class TransformerStage(StageCompute):
         # of every column-tile workgroup re-deriving them
         rs = self.rowstat[r0:r1] if (T == 1 and self.fuse_norm and G_.ROWSTATS) else None
         have_rs = False
+        one_group = self.fp8 and ntok > G_.SKINNY_MAX_M  # e4m3 activations follow the attention
         one_call = T > 1 and self._prefill_blocks(h_in, pos, B, T, b0)
         for li, L in enumerate(() if one_call else self.layers):
             kc, vc = self.kc[li, b0:b0 + B], self.vc[li, b0:b0 + B]
@@ -469,15 +470,15 @@ class TransformerStage(StageCompute):
                 T_.layernorm(h_in, L.ln1_w, L.ln1_b, a, self.eps, self.rms, rows=ntok)
                 qkv, _ = self._lin(a, L.w_qkv, L.b_qkv, out=self.buf_qkv[r0:r1])
             if scattered:
-                T_.flash_attn(self.buf_q, kc, vc, att, B, T, self.H, self.Hkv, self.hd, pos)
+                T_.flash_attn(self.buf_q, kc, vc, att, B, T, self.H, self.Hkv, self.hd, pos, one_group=one_group)
             elif T == 1:  # decode: split/RoPE/cache write fused into the attention launch
                 T_.attn_decode_qkv(qkv, kc, vc, att, B, self.H, self.Hkv, self.hd, pos, ws, self.splits,
                                    self.cos, self.sin)
             elif self.cos is None:  # no RoPE (GPT-2): attention reads the c_attn output directly
-                T_.flash_attn_qkv(qkv, kc, vc, att, B, T, self.H, self.Hkv, self.hd, pos)
+                T_.flash_attn_qkv(qkv, kc, vc, att, B, T, self.H, self.Hkv, self.hd, pos, one_group=one_group)
             else:
                 T_.qkv_split(qkv, self.buf_q, kc, vc, B, T, self.H, self.Hkv, self.hd, pos, self.cos, self.sin)
-                T_.flash_attn(self.buf_q, kc, vc, att, B, T, self.H, self.Hkv, self.hd, pos)
+                T_.flash_attn(self.buf_q, kc, vc, att, B, T, self.H, self.Hkv, self.hd, pos, one_group=one_group)
             _, have_rs = self._lin(att, L.w_o, L.b_o, residual=h_in, out=h, w_shuf=L.w_o_s, ws=gws, rs_out=rs)
             up_act = ACT_GELU if self.family == "gpt2" else ACT_SILU_MUL
             mx_f = None

@@ -1743,3 +1743,22 @@ def test_prefill_rows_off_16_bytes(T):
         flat[off:off + T * st.d] = torch.linspace(-2, 2, T * st.d, device=DEV).sin().bfloat16()
         outs.append(st.step(flat[off:off + T * st.d].view(T, st.d), pos, 1, T).clone())
     assert _rel(outs[1], outs[0]) < 1e-2
+
+
+@pytest.mark.parametrize("dtype,T,same", [("fp8", 300, True), ("fp8", 257, True), ("bf16", 300, False)])
+@pytest.mark.parametrize("one_call", [True, False])
+def test_prefill_key_order_before_e4m3(dtype, T, same, one_call, monkeypatch):
+    """Where e4m3 activations follow the attention its keys keep one order on small grids too: the
+    bits of the pinned one-group kernel.  bf16 activations: two groups, another order."""
+    from distributed_neural_networks_amd import checkpoint as ckpt
+    from distributed_neural_networks_amd.runtime import transformer as R
+    sd = ckpt.random_stage_state_dict("gpt2", 1, 3, False, False, 3, nontrivial=True)
+    st = R.build_device_stage("gpt2", sd, 1, 3, False, False, DEV, max_batch=1, max_seq=T + 4, max_tokens=T, dtype=dtype)
+    if not one_call:
+        monkeypatch.setattr(R.TransformerStage, "_prefill_blocks", lambda *a: False)
+    x = torch.linspace(-2, 2, T * st.d, device=DEV).sin().bfloat16().view(T, st.d)
+    pos, outs = torch.zeros(1, dtype=torch.int32, device=DEV), []
+    for pin in (None, "1"):
+        monkeypatch.setenv("DNN_FLASH_DB", pin) if pin else monkeypatch.delenv("DNN_FLASH_DB", raising=False)
+        outs.append(st.step(x, pos, 1, T).clone())
+    assert torch.equal(*outs) == same
