@@ -46,9 +46,9 @@ __device__ __forceinline__ i32x8_t f8_cat(const bf16x8& lo, const bf16x8& hi) {
   return r;
 }
 
-template <int MI, int NJ>
+template <int MI, int NJ, bool WAIT = true>
 __device__ __forceinline__ void bg_mfma_f8(f32x4 (&acc)[MI][NJ], const bf16x8 (&a)[MI][2], const bf16x8 (&b)[NJ][2]) {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  if constexpr (WAIT) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_setprio(1);
 #pragma unroll
   for (int i = 0; i < MI; ++i)
@@ -63,11 +63,11 @@ __device__ __forceinline__ void bg_mfma_f8(f32x4 (&acc)[MI][NJ], const bf16x8 (&
 // mx_index: one dword per lane per 128-row half-tile and K-tile, byte i =
 // fragment i): acc carries the activation scales, the epilogue only the
 // weight channel scale.
-template <int MI, int NJ>
+template <int MI, int NJ, bool WAIT = true>
 __device__ __forceinline__ void bg_mfma_f8x(f32x4 (&acc)[MI][NJ], const bf16x8 (&a)[MI][2], const bf16x8 (&b)[NJ][2],
                                             uint32_t s) {
   static_assert(MI == 4, "one op_sel byte per A fragment");
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  if constexpr (WAIT) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_setprio(1);
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_256_kernel(
   static_assert(!QOUT || (MXA && ACT == ACT_GELU && !SCATTER), "quantised output: the MX c_fc");
   constexpr int TN = 128 * NQ;  // NQ = 1: the 256x128 variant (tail-split launches), as the bf16 kernel's
   __shared__ __attribute__((aligned(1024))) char smem[8 * BG_HALF + EPI_LDS];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ntn = (N + TN - 1) / TN, ntm = (M + BG_M - 1) / BG_M;
   int tm, tn;
   tile_coords(xcd_remap(blockIdx.x, ntm * ntn), ntm, ntn, tm, tn);
@@ -136,13 +136,20 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_256_kernel(
         for (int j = 0; j < 2; ++j) acc[a][b][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   auto half = [&](int u, int h) { return smem + (u * 4 + h) * BG_HALF; };
+  BgRows ra, rb;
+  if constexpr (NQ == 2) {
+    ra.init(A, lda, m0, M, wave, lane);
+    rb.init(W, ldw, n0, N, wave, lane);
+  }
   auto stA = [&](int u, int h, int t) {
     t = t < nk ? t : nk - 1;
-    stage_half(A, lda, m0 + h * 128, M, t * BG_K, half(u, h), wave, lane);
+    if constexpr (NQ == 2) ra.stage(h, t, half(u, h), wave);
+    else stage_half(A, lda, m0 + h * 128, M, t * BG_K, half(u, h), wave, lane);
   };
   auto stB = [&](int u, int h, int t) {
     t = t < nk ? t : nk - 1;
-    stage_half(W, ldw, n0 + h * 128, N, t * BG_K, half(u, 2 + h), wave, lane);
+    if constexpr (NQ == 2) rb.stage(h, t, half(u, 2 + h), wave);
+    else stage_half(W, ldw, n0 + h * 128, N, t * BG_K, half(u, 2 + h), wave, lane);
   };
 
   bf16x8 af[4][2], b0[2][2], b1[2][2];
@@ -181,56 +188,66 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_256_kernel(
     if (t < nk) ktile1(t, std::integral_constant<int, 0>{});
   } else {
   // MXA: the scale dwords of K-tile t (half-tiles 0 / 1 of A) in scl[t & 1];
-  // tile t + 1's are loaded in tile t's first phase, so the phase-4 vmcnt(4)
-  // (which retires everything but the last four DMAs) has retired them too
+  // tile t + 1's are loaded in tile t's first phase: two more loads that a wait
+  // for DMAs finds behind what it waits for
   uint32_t scl[2][2] = {{0x7f7f7f7fu, 0x7f7f7f7fu}, {0x7f7f7f7fu, 0x7f7f7f7fu}};
   const int nb64 = mx_mpad(M) >> 6;
   auto ldsx = [&](int t, uint32_t (&d)[2]) {
     t = t < nk ? t : nk - 1;
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      d[h] = sx[((size_t)t * nb64 + min((m0 >> 6) + 2 * h + wr, nb64 - 1)) * 16 + (lane & 15)];
+    for (int h = 0; h < 2; ++h) {
+      const GLB_AS uint32_t* p = (const GLB_AS uint32_t*)(sx + ((size_t)t * nb64 + min((m0 >> 6) + 2 * h + wr, nb64 - 1)) * 16);
+      asm("" : "+s"(p));  // scalar base (BgRows::stage)
+      d[h] = p[lane & 15];
+    }
   };
+  bf16x8 a1[4][2];
+  constexpr int FLY = MXA ? 12 : 10;  // the schedule of gemm_tile.h
   if constexpr (MXA) ldsx(0, scl[0]);
   stA(0, 0, 0);
+  stB(0, 0, 0);
   stB(0, 1, 0);
   stA(0, 1, 0);
-  stB(0, 0, 0);
   stA(1, 0, 1);
+  stB(1, 0, 1);
   stB(1, 1, 1);
-  asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+  bg_landed<10>();
   bg_barrier();
   if (wr == 1) bg_barrier();
+  bg_read<4>(af, half(0, 0), arow, lane);
 
-  auto mm = [&](f32x4 (&c)[4][2], const bf16x8 (&bb)[2][2], uint32_t s) {
-    if constexpr (MXA) bg_mfma_f8x<4, 2>(c, af, bb, s);
-    else bg_mfma_f8<4, 2>(c, af, bb);
+  auto mm = [&](f32x4 (&c)[4][2], const bf16x8 (&aa)[4][2], const bf16x8 (&bb)[2][2], uint32_t s, auto wait) {
+    constexpr bool W = decltype(wait)::value;
+    if constexpr (MXA) bg_mfma_f8x<4, 2, W>(c, aa, bb, s);
+    else bg_mfma_f8<4, 2, W>(c, aa, bb);
   };
   auto ktile = [&](const int t, auto ucst) {
     constexpr int u = decltype(ucst)::value;
     bg_read<2>(b0, half(u, 2), brow, lane);
-    __builtin_amdgcn_sched_barrier(0);
-    bg_read<4>(af, half(u, 0), arow, lane);
     stA(u ^ 1, 1, t + 1);
     if constexpr (MXA) ldsx(t + 1, scl[u ^ 1]);
+    bg_landed<FLY>();
     bg_barrier();
-    mm(acc[0][0], b0, scl[u][0]);
+    mm(acc[0][0], af, b0, scl[u][0], std::true_type{});
     bg_barrier();
     bg_read<2>(b1, half(u, 3), brow, lane);
-    stB(u ^ 1, 0, t + 1);
-    bg_barrier();
-    mm(acc[0][1], b1, scl[u][0]);
-    bg_barrier();
-    bg_read<4>(af, half(u, 1), arow, lane);
     stA(u, 0, t + 2);
+    bg_landed<FLY>();
     bg_barrier();
-    mm(acc[1][1], b1, scl[u][1]);
+    mm(acc[0][1], af, b1, scl[u][0], std::true_type{});
     bg_barrier();
-    bg_read<2>(b0, half(u, 2), brow, lane);
+    bg_read<4>(a1, half(u, 1), arow, lane);
+    stB(u, 0, t + 2);
+    bg_landed<FLY>();
+    bg_barrier();
+    mm(acc[1][1], a1, b1, scl[u][1], std::true_type{});
+    bg_barrier();
+    bg_read<4>(af, half(u ^ 1, 0), arow, lane);
     stB(u, 1, t + 2);
-    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    bg_landed<FLY>();
     bg_barrier();
-    mm(acc[1][0], b0, scl[u][1]);
+    mm(acc[1][0], a1, b0, scl[u][1], std::false_type{});
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     bg_barrier();
   };
   int t = (gan & 2) ? nk : 0;
@@ -559,7 +576,7 @@ static int launch_gemm(const void* A, int lda, const void* W, int ldw, void* C, 
     return mid_launch(plan.tile, a, nullptr, st);
   }
   const int tilesH = ((M + BG_M - 1) / BG_M) * ((N + 127) / 128);
-  const bool half = g_gemm_tile == 255 ||
+  const bool half = g_gemm_tile == 255 || !bg_narrow(lda) || !bg_narrow(ldw) ||
                     (g_gemm_tile == 0 && (float)((tilesH + 255) / 256) * g_half_cost < (float)((tiles256 + 255) / 256));
   if (half) {
     hipLaunchKernelGGL((gemm_bf16_256_kernel<ACT, F32, false, 1>), dim3(tilesH), dim3(512), 0, st, (const bf16_t*)A,
@@ -663,6 +680,12 @@ extern "C" int dnn_gemm_bf16_qkv_scatter(const void* A, int lda, const void* W, 
     }
   }
   if (M < 256) return -3;
+  if (!bg_narrow(lda) || !bg_narrow(ldw)) {  // the 256 x 128 tiles address rows with 64 bits
+    hipLaunchKernelGGL((gemm_bf16_256_kernel<ACT_NONE, false, true, 1>), dim3((M + BG_M - 1) / BG_M * ((N + 127) / 128)),
+                       dim3(512), 0, st, (const bf16_t*)A, lda, (const bf16_t*)W, ldw, q, hd, bias, (const bf16_t*)nullptr, 0,
+                       M, N, K, 0, reinterpret_cast<const float2*>(rowstat), colsum, sc);
+    return (int)hipGetLastError();
+  }
   // tail split as launch_gemm's (GPT-2 c_attn at M = 32768: 1024 + 128 tiles
   // -> 4 rounds of 256^2 + 1 round of 256x128); the bias is indexed by the
   // global column (c_off), the folded norm's colsum by the launch's own

@@ -28,15 +28,22 @@ __device__ __forceinline__ bf16x8 lds_frag(const char* tile, int row, int chunk)
 //   wave's output quadrant-row h, so a wave's 128x64 output is 2x2 quadrants of
 //   64x32 and each phase is one quadrant x K=64 = 16 MFMAs:
 //
-//     ph1: read B0 (4 ds_read_b128), A0 (8)  | stage A1[t+1] -> buf^1 | C00
-//     ph2: read B1 (4)                       | stage B0[t+1] -> buf^1 | C01
-//     ph3: read A1 (8)                       | stage A0[t+2] -> buf   | C11
-//     ph4: read B0 (4)                       | stage B1[t+2] -> buf   | C10
-//          + s_waitcnt vmcnt(4)  (retires everything of tile t+1)
+//     ph1: read B0 (4 ds_read_b128) of t   | stage A1[t+1] -> buf^1 | C00
+//     ph2: read B1 (4) of t                | stage A0[t+2] -> buf   | C01
+//     ph3: read A1 (8) of t                | stage B0[t+2] -> buf   | C11
+//     ph4: read A0 (8) of t + 1            | stage B1[t+2] -> buf   | C10
+//          each + s_waitcnt vmcnt(10): the half-tile that the next phase reads
 //
-//   Every restage lands >= 2 phases after the last read of that half-tile
-//   (WAR), every read is >= 1 phase after the vmcnt+barrier that retired its
-//   DMA (RAW).  Each phase = [ds_reads + 2 glds] s_barrier [lgkmcnt(0),
+//   Every fragment is read once (A0 and A1 have registers of their own, B0 lives
+//   from ph1 to ph4).  Every restage lands >= 2 phases after the last read of
+//   that half-tile (WAR; A0's reads are waited for at the end of ph4, not at the
+//   next ph1), every read is >= 1 phase after the vmcnt+barrier that retired its
+//   DMA (RAW), and a DMA has 5 phases until it is waited for: six half-tiles, 96
+//   of the 128 KiB, are in flight.  (With B0 read again in ph4 and DMAs 2 to 3
+//   phases ahead: 8192 x 28672 x 4096 1378 us, now 1311; 8192 x 4096 x 14336 658 :
+//   623; one round of tiles, weights from HBM: 512 x 21504 x 4096 91.9 : 87.6; 2048 x
+//   6400 x 1600 43.5 : 41.8.)
+//   Each phase = [ds_reads + 2 glds, vmcnt] s_barrier [lgkmcnt(0),
 //   setprio(1), 16 MFMA] s_barrier; waves of M-row 1 run one barrier behind
 //   M-row 0, so on every SIMD one wave issues LDS reads while its partner
 //   issues MFMAs.  glds stays in flight across barriers (raw s_barrier, counted
@@ -60,6 +67,36 @@ __device__ __forceinline__ void stage_half(const bf16_t* __restrict__ src, int l
     glds16(src + (size_t)r * ld + k0 + cs * 8, dst + piece * 1024);
   }
 }
+
+// The 4 pieces (8 rows of 128 B) of an operand that a wave stages: piece x & 1 of
+// half-tile x >> 1.  Uniform row bases and a lane offset: per-lane 64-bit addresses
+// would take 16 registers that the 256 x 256 schedule needs for fragments.
+struct BgRows {
+  const char* base[4];
+  uint32_t lim[4];          // the lane's row offset is clamped to it (rows past the matrix)
+  uint32_t lrow, lchunk;    // byte offsets of the lane's row and (swizzled) chunk
+  // ld in elements; 8 rows are addressed with 32 bits (host: bg_narrow)
+  __device__ __forceinline__ void init(const bf16_t* src, int ld, int r0, int nrows, int wave, int lane) {
+    const uint32_t ldb = (uint32_t)ld * 2u;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int r = min(r0 + (x >> 1) * 128 + ((x & 1) * 8 + wave) * 8, nrows - 1);
+      base[x] = reinterpret_cast<const char*>(src) + (size_t)r * ldb;
+      lim[x] = (uint32_t)min(7, nrows - 1 - r) * ldb;
+    }
+    lrow = (uint32_t)(lane >> 3) * ldb;
+    lchunk = (uint32_t)((lane & 7) ^ ((wave & 1) * 4 + (lane >> 4))) * 16u;
+  }
+  __device__ __forceinline__ void stage(int h, int t, char* dst, int wave) const {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const char* p = base[2 * h + i] + (size_t)t * (BG_K * 2);
+      asm("" : "+s"(p));  // scalar base, 32-bit lane offset: not folded into per-lane addresses ahead of the loop
+      glds16(p + (min(lrow, lim[2 * h + i]) + lchunk), dst + (i * 8 + wave) * 1024);
+    }
+  }
+};
+inline bool bg_narrow(int ld) { return ld < 1 << 28; }
 
 // The same from a weight in fragment order (blocks of 16 rows x 32 columns): a
 // wave-instruction reads eight 128-B pieces, one per 8 columns of its 8 rows.
@@ -118,9 +155,16 @@ __device__ __forceinline__ void bg_barrier() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-template <int MI, int NJ>
+// At most N of this wave's DMAs outstanding
+template <int N>
+__device__ __forceinline__ void bg_landed() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// WAIT: the operands were read in this phase
+template <int MI, int NJ, bool WAIT = true>
 __device__ __forceinline__ void bg_mfma(f32x4 (&acc)[MI][NJ], const bf16x8 (&a)[MI][2], const bf16x8 (&b)[NJ][2]) {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  if constexpr (WAIT) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_setprio(1);
 #pragma unroll
   for (int s = 0; s < 2; ++s)
@@ -225,7 +269,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_256_kernel(
   static_assert(NQ == 1 || NQ == 2, "256x256 or 256x128 tiles");
   constexpr int TN = 128 * NQ;
   __shared__ __attribute__((aligned(1024))) char smem[8 * BG_HALF + EPI_LDS];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ntn = (N + TN - 1) / TN;
   int tm, tn;
   int ga[4] = {};  // GRP: the A rows this thread stages (2 of either half-tile)
@@ -269,6 +313,11 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_256_kernel(
 
   // half-tile h of buffer u: A0=0, A1=1, B0=2, B1=3
   auto half = [&](int u, int h) { return smem + (u * 4 + h) * BG_HALF; };
+  BgRows ra, rb;
+  if constexpr (NQ == 2 && !GRP) {
+    ra.init(A, lda, m0, M, wave, lane);
+    rb.init(W, ldw, n0, N, wave, lane);
+  }
   auto stA = [&](int u, int h, int t) {
     t = t < nk ? t : nk - 1;
     if constexpr (GRP) {
@@ -278,6 +327,8 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_256_kernel(
         glds16(A + (size_t)(h == 0 ? ga[i] : ga[2 + i]) * lda + t * BG_K + ((lane & 7) ^ swz_chunk(piece * 8 + (lane >> 3))) * 8,
                half(u, h) + piece * 1024);
       }
+    } else if constexpr (NQ == 2) {
+      ra.stage(h, t, half(u, h), wave);
     } else {
       stage_half(A, lda, m0 + h * 128, M, t * BG_K, half(u, h), wave, lane);
     }
@@ -285,6 +336,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_256_kernel(
   auto stB = [&](int u, int h, int t) {
     t = t < nk ? t : nk - 1;
     if constexpr (GRP) stage_half_frag(W, K, n0 + h * 128, N, t * BG_K, half(u, 2 + h), wave, lane);
+    else if constexpr (NQ == 2) rb.stage(h, t, half(u, 2 + h), wave);
     else stage_half(W, ldw, n0 + h * 128, N, t * BG_K, half(u, 2 + h), wave, lane);
   };
 
@@ -325,16 +377,19 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_256_kernel(
     }
     if (t < nk) ktile1(t, std::integral_constant<int, 0>{});
   } else {
-  // prologue: tile 0 complete, A0/B1 of tile 1 in flight
+  // prologue: A0 and B0 of tile 0 landed, five half-tiles in flight
+  bf16x8 a1[4][2];
   stA(0, 0, 0);
+  stB(0, 0, 0);
   stB(0, 1, 0);
   stA(0, 1, 0);
-  stB(0, 0, 0);
   stA(1, 0, 1);
+  stB(1, 0, 1);
   stB(1, 1, 1);
-  asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+  bg_landed<10>();
   bg_barrier();
   if (wr == 1) bg_barrier();
+  bg_read<4>(af, half(0, 0), arow, lane);
 
   // One K-tile; the loop runs two per iteration so the buffer index u is a
   // compile-time constant and every LDS address an immediate offset.
@@ -342,30 +397,32 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_256_kernel(
     constexpr int u = decltype(ucst)::value;
     // ph1
     bg_read<2>(b0, half(u, 2), brow, lane);
-    __builtin_amdgcn_sched_barrier(0);
-    bg_read<4>(af, half(u, 0), arow, lane);
     stA(u ^ 1, 1, t + 1);
+    bg_landed<10>();
     bg_barrier();
     bg_mfma<4, 2>(acc[0][0], af, b0);
     bg_barrier();
     // ph2
     bg_read<2>(b1, half(u, 3), brow, lane);
-    stB(u ^ 1, 0, t + 1);
+    stA(u, 0, t + 2);
+    bg_landed<10>();
     bg_barrier();
     bg_mfma<4, 2>(acc[0][1], af, b1);
     bg_barrier();
     // ph3
-    bg_read<4>(af, half(u, 1), arow, lane);
-    stA(u, 0, t + 2);
+    bg_read<4>(a1, half(u, 1), arow, lane);
+    stB(u, 0, t + 2);
+    bg_landed<10>();
     bg_barrier();
-    bg_mfma<4, 2>(acc[1][1], af, b1);
+    bg_mfma<4, 2>(acc[1][1], a1, b1);
     bg_barrier();
-    // ph4
-    bg_read<2>(b0, half(u, 2), brow, lane);
+    // ph4: the products' operands are in registers; the next tile's A0 arrives behind them
+    bg_read<4>(af, half(u ^ 1, 0), arow, lane);
     stB(u, 1, t + 2);
-    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    bg_landed<10>();
     bg_barrier();
-    bg_mfma<4, 2>(acc[1][0], af, b0);
+    bg_mfma<4, 2, false>(acc[1][0], a1, b0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     bg_barrier();
   };
   int t = (gan & 2) ? nk : 0;

@@ -1762,3 +1762,28 @@ def test_prefill_key_order_before_e4m3(dtype, T, same, one_call, monkeypatch):
         monkeypatch.setenv("DNN_FLASH_DB", pin) if pin else monkeypatch.delenv("DNN_FLASH_DB", raising=False)
         outs.append(st.step(x, pos, 1, T).clone())
     assert torch.equal(*outs) == same
+
+
+@pytest.mark.parametrize("K", [64, 128, 192, 320])
+@pytest.mark.parametrize("M,N", [(256, 256), (257, 264), (511, 1000)])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_gemm_256_k_tiles(M, N, K, out_dtype):
+    """The 256 x 256 kernel from one K-tile on (its DMAs run up to two tiles ahead and
+    past the end) and at ragged borders, operands in rows of more than K columns,
+    against 64 bits; every call gives the same bits.  A bf16 result is rounded by at
+    most 2^-9, the fp32 sum of K products is off by less than K 2^-24."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    torch.manual_seed(M + K)
+    x = torch.randn(M, K + 64, device=DEV).bfloat16()[:, :K]
+    w = torch.randn(N, K + 8, device=DEV).mul_(K ** -0.5).bfloat16()[:, :K]
+    b = torch.randn(N, device=DEV)
+    r = torch.randn(M, N, device=DEV).bfloat16()
+    G.set_gemm_tile(256)
+    try:
+        y = [G.linear(x, w, b, residual=r, out_dtype=out_dtype).clone() for _ in range(4)]
+    finally:
+        G.set_gemm_tile(0)
+    ref = x.cpu().double() @ w.cpu().double().t() + b.cpu().double() + r.cpu().double()
+    err = ((y[0].cpu().double() - ref).norm() / ref.norm()).item()
+    assert err < (2.0 ** -9 if out_dtype == torch.bfloat16 else 0.0) + K * 2.0 ** -24
+    assert all(torch.equal(y[0], t) for t in y[1:])
