@@ -106,7 +106,7 @@ class Engine:
         x = None
         for s in self.stages:
             x = s.step_batch(b, x)
-        self._pos = b.pos[b.want.long()].contiguous() if b.n_want else None
+        self._pos = b.want_pos
         return x
 
     def end(self, seq_id: Hashable) -> None:

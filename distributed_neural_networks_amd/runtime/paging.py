@@ -85,7 +85,8 @@ class StepBatch:
     the sequences that bring two tokens or more; ``dec_rows``: rows of the
     sequences that bring one; ``ent``: {first row, tokens, slot, 0} of all of
     them, the chunks first; ``start`` / ``last``: per row, the first and last row
-    of its sequence; ``max_len``: the longest sequence after the step.
+    of its sequence; ``max_len``: the longest sequence after the step; ``want_pos``:
+    the positions of the wanted rows.
     ``tiles``: attention workgroups by key (``tile_lists``)."""
     M: int
     pos: torch.Tensor
@@ -102,6 +103,7 @@ class StepBatch:
     want: Optional[torch.Tensor] = None
     n_want: int = 0
     tiles: Optional[Dict[object, torch.Tensor]] = None
+    want_pos: Optional[torch.Tensor] = None
 
 
 KEY_ROWS = 1 << 15    # most keys of a step that are projected to heads
@@ -166,7 +168,11 @@ def tile_lists(groups: Sequence, chunks: Sequence[tuple], ones: Sequence[tuple],
 def build_batch(entries: Sequence[tuple], table: np.ndarray, groups: Sequence[int], device) -> StepBatch:
     """``entries``: (token ids, first position, slot, wanted places) per
     sequence.  ``groups``: the kinds of attention of the model's layers
-    (``tile_lists``).  Everything travels in one host-to-device copy."""
+    (``tile_lists``).  Everything travels in one host-to-device copy, from pinned
+    memory: a copy from pageable memory holds the host until every earlier launch of
+    the stream has run, so the device then waits for the next step's first launches
+    (Kozusun, nine steps of up to 512 tokens: 4130 us a pass so, 3650 of them kernels).
+    The caching allocator keeps the pinned block until the copy has run."""
     ids, pos, slots, dec, want, chunks, starts, start, last = [], [], [], [], [], [], [], [], []
     for toks, p0, slot, places in entries:
         n, row = len(toks), len(ids)
@@ -190,17 +196,20 @@ def build_batch(entries: Sequence[tuple], table: np.ndarray, groups: Sequence[in
               ("last", np.array(last, dtype=np.int32)),
               ("ids", np.array(ids, dtype=np.int32)), ("pos", np.array(pos, dtype=np.int32)),
               ("slots", np.array(slots, dtype=np.int32)), ("dec", np.array(dec, dtype=np.int32)),
-              ("want", np.array(want, dtype=np.int32)), ("table", table.reshape(-1))]
+              ("want", np.array(want, dtype=np.int32)), ("want_pos", np.array([pos[w] for w in want], dtype=np.int32)),
+              ("table", table.reshape(-1))]
     off, total = {}, 0
     for name, a in parts:
         off[name] = total
         total += -(-a.size // 4) * 4  # 16-byte aligned starts
-    host = np.zeros(total, dtype=np.int32)
+    host = torch.zeros(total, dtype=torch.int32, pin_memory=torch.device(device).type == "cuda")
+    flat = host.numpy()
     for name, a in parts:
-        host[off[name]:off[name] + a.size] = a
-    dev = torch.from_numpy(host).to(device)
+        flat[off[name]:off[name] + a.size] = a
+    dev = host.to(device, non_blocking=True)
     v = {name: dev[off[name]:off[name] + a.size] for name, a in parts}
     return StepBatch(M=len(ids), pos=v["pos"], slots=v["slots"], table=v["table"].view(table.shape),
                      dec_rows=v["dec"] if dec else None, n_dec=len(dec), chunks=chunks,
                      max_len=max(pos) + 1, ent=v["ent"].view(-1, 4), start=v["start"], last=v["last"], ids=v["ids"],
-                     want=v["want"] if want else None, n_want=len(want), tiles={k: v[k].view(-1, 4) for k in tiles})
+                     want=v["want"] if want else None, n_want=len(want), tiles={k: v[k].view(-1, 4) for k in tiles},
+                     want_pos=v["want_pos"] if want else None)

@@ -556,3 +556,27 @@ def test_refusals():
     with pytest.raises(ValueError, match="holds"):
         st[0].step(torch.zeros((2, 1), dtype=torch.int32, device=dev()),
                    torch.zeros(2, dtype=torch.int32, device=dev()), 2, 1)
+
+
+@pytest.mark.parametrize("tokens", [1, 70])
+def test_build_batch_does_not_wait_and_keeps_its_own_rows(tokens):
+    """Batches built one behind the other while the stream is busy: the host does not
+    wait for it, and each arrives with its own ids, positions and wanted rows."""
+    from distributed_neural_networks_amd.runtime.paging import PageTable, build_batch
+    table = PageTable(16, 4)
+    slot = table.admit()
+    build_batch([([1] * tokens, 0, slot, [])], table.table, [1], dev())  # the pinned block exists
+    a = torch.randn(8192, 8192, device=dev())
+    torch.cuda.synchronize()
+    for _ in range(20):
+        a @ a
+    busy = torch.cuda.Event()
+    busy.record()
+    got = [build_batch([([7 * i + j for j in range(tokens)], 3 * i, slot, [tokens - 1])], table.table, [1], dev())
+           for i in range(12)]
+    assert not busy.query()
+    torch.cuda.synchronize()
+    for i, b in enumerate(got):
+        assert b.ids.tolist() == [7 * i + j for j in range(tokens)]
+        assert b.pos.tolist() == list(range(3 * i, 3 * i + tokens))
+        assert b.want_pos.tolist() == [3 * i + tokens - 1] == b.pos[b.want.long()].tolist()
