@@ -213,11 +213,14 @@ using namespace x3;
 
 // SPLIT_OUT: the boundary leaves in the blocked hi/lo encoding
 // (cifar_split_blocked_kernel) that cifar_fc1_x3_kernel<true> stages by DMA.
+// keep: where given, a copy of the images is left there, from the registers they are
+// split in; the kernel is bound by its products and HBM has room.  A copy kernel of
+// its own in front took 301 us of a pass of 65536 images.
 template <bool WIDE, bool SPLIT_OUT>
 __global__ __launch_bounds__(512, 1) void cifar_stage0_x3_kernel(
     const float* __restrict__ x, float* __restrict__ out, const bf16_t* __restrict__ w1h,
     const bf16_t* __restrict__ w1l, const float* __restrict__ b1, const bf16_t* __restrict__ w2h,
-    const bf16_t* __restrict__ w2l, const float* __restrict__ b2, int B) {
+    const bf16_t* __restrict__ w2l, const float* __restrict__ b2, float* __restrict__ keep, int B) {
   __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -268,6 +271,13 @@ __global__ __launch_bounds__(512, 1) void cifar_stage0_x3_kernel(
         const int o = ((yy + 1) * XW + xx + 1) * 8;
         *reinterpret_cast<uint2*>(xh + o) = vh;
         *reinterpret_cast<uint2*>(xl + o) = vl;
+      }
+      if (keep != nullptr) {
+        float* kb = keep + (size_t)(blockIdx.x + (size_t)k * gridDim.x) * 3072;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int c = 0; c < 3; ++c) kb[c * 1024 + rt + 256 * i] = pf[i][c];
       }
     };
     if (n > 0) {
@@ -387,7 +397,7 @@ template <bool SPLIT_OUT>
 __global__ __launch_bounds__(512, 1) void cifar_stage0_x3_band_kernel(
     const float* __restrict__ x, float* __restrict__ out, const bf16_t* __restrict__ w1h,
     const bf16_t* __restrict__ w1l, const float* __restrict__ b1, const bf16_t* __restrict__ w2h,
-    const bf16_t* __restrict__ w2l, const float* __restrict__ b2) {
+    const bf16_t* __restrict__ w2l, const float* __restrict__ b2, float* __restrict__ keep) {
   constexpr int A1 = 2 * XPL;  // xin hi | lo, pooled map hi | lo
   __shared__ __attribute__((aligned(16))) char smem[A1 + 2 * A1PL];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -411,6 +421,10 @@ __global__ __launch_bounds__(512, 1) void cifar_stage0_x3_band_kernel(
     split2(px[i][2], 0.f, vh.y, vl.y);
     *reinterpret_cast<uint2*>(smem + o) = vh;
     *reinterpret_cast<uint2*>(smem + XPL + o) = vl;
+    if (keep != nullptr && (p >> 8) == ty2) {  // every band a quarter of the pixels
+#pragma unroll
+      for (int c = 0; c < 3; ++c) keep[img * 3072 + c * 1024 + p] = px[i][c];
+    }
   }
   if (wave < 4) {
     bf16x8 w1hf[3], w1lf[3];
@@ -951,34 +965,37 @@ extern "C" int dnn_cifar_s0_set_wide_store(int on) {
 
 template <bool SPLIT_OUT>
 static int launch_stage0_x3(const float* x, float* out, const void* w1h, const void* w1l, const float* b1,
-                            const void* w2h, const void* w2l, const float* b2, int B, int grid, hipStream_t st) {
+                            const void* w2h, const void* w2l, const float* b2, float* keep, int B, int grid,
+                            hipStream_t st) {
   if (g_s0_wide_store)
     hipLaunchKernelGGL((cifar_stage0_x3_kernel<true, SPLIT_OUT>), dim3(grid), dim3(512), 0, st, x, out,
-                       (const bf16_t*)w1h, (const bf16_t*)w1l, b1, (const bf16_t*)w2h, (const bf16_t*)w2l, b2, B);
+                       (const bf16_t*)w1h, (const bf16_t*)w1l, b1, (const bf16_t*)w2h, (const bf16_t*)w2l, b2, keep, B);
   else
     hipLaunchKernelGGL((cifar_stage0_x3_kernel<false, SPLIT_OUT>), dim3(grid), dim3(512), 0, st, x, out,
-                       (const bf16_t*)w1h, (const bf16_t*)w1l, b1, (const bf16_t*)w2h, (const bf16_t*)w2l, b2, B);
+                       (const bf16_t*)w1h, (const bf16_t*)w1l, b1, (const bf16_t*)w2h, (const bf16_t*)w2l, b2, keep, B);
   return (int)hipGetLastError();
 }
 
 // split_out = 1: the (B,4096) boundary in the blocked hi/lo encoding, else fp32.
+// keep (null: none): (B,3,32,32), receives a copy of x; must not overlap x.
 extern "C" int dnn_cifar_stage0_x3(const float* x, float* out, const void* w1h, const void* w1l, const float* b1,
                                    const void* w2h, const void* w2l, const float* b2, int B, int grid,
-                                   hipStream_t st, int split_out) {
+                                   hipStream_t st, int split_out, float* keep) {
   if (B <= 0) return 0;
+  if (keep == x) keep = nullptr;
   if (grid <= 0) grid = 256;
   if (4L * B <= grid) {
     if (split_out)
       hipLaunchKernelGGL(cifar_stage0_x3_band_kernel<true>, dim3(4 * B), dim3(512), 0, st, x, out, (const bf16_t*)w1h,
-                         (const bf16_t*)w1l, b1, (const bf16_t*)w2h, (const bf16_t*)w2l, b2);
+                         (const bf16_t*)w1l, b1, (const bf16_t*)w2h, (const bf16_t*)w2l, b2, keep);
     else
       hipLaunchKernelGGL(cifar_stage0_x3_band_kernel<false>, dim3(4 * B), dim3(512), 0, st, x, out, (const bf16_t*)w1h,
-                         (const bf16_t*)w1l, b1, (const bf16_t*)w2h, (const bf16_t*)w2l, b2);
+                         (const bf16_t*)w1l, b1, (const bf16_t*)w2h, (const bf16_t*)w2l, b2, keep);
     return (int)hipGetLastError();
   }
   if (grid > B) grid = B;
-  return split_out ? launch_stage0_x3<true>(x, out, w1h, w1l, b1, w2h, w2l, b2, B, grid, st)
-                   : launch_stage0_x3<false>(x, out, w1h, w1l, b1, w2h, w2l, b2, B, grid, st);
+  return split_out ? launch_stage0_x3<true>(x, out, w1h, w1l, b1, w2h, w2l, b2, keep, B, grid, st)
+                   : launch_stage0_x3<false>(x, out, w1h, w1l, b1, w2h, w2l, b2, keep, B, grid, st);
 }
 
 extern "C" int dnn_cifar_fc1_x3(const float* A, int lda, const void* Wh, const void* Wl, int ldw, const float* bias,

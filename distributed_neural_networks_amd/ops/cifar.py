@@ -194,9 +194,10 @@ def decode_boundary(h: torch.Tensor, out: Optional[torch.Tensor] = None) -> torc
 
 
 def stage0_forward(x: torch.Tensor, w: CifarStage0Weights, out: Optional[torch.Tensor] = None,
-                   grid: int = 0, boundary: str = "fp32") -> torch.Tensor:
+                   grid: int = 0, boundary: str = "fp32", keep: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Units 0-1: x (B,3,32,32) fp32 contiguous -> (B,4096) fp32 (or bf16 in bf16 mode;
-    ``boundary="split"``: the blocked hi/lo encoding in the fp32 tensor)."""
+    ``boundary="split"``: the blocked hi/lo encoding in the fp32 tensor).  ``keep``
+    (fp32 precision; apart from x): receives a copy of x in the same launch."""
     split = _split_boundary(boundary, w.precision)
     grid = grid or STAGE0_GRID
     _check_act(x, (3, 32, 32), torch.float32, "stage0 input")
@@ -206,9 +207,15 @@ def stage0_forward(x: torch.Tensor, w: CifarStage0Weights, out: Optional[torch.T
         out = torch.empty((B, 4096), dtype=dt, device=x.device)
     if tuple(out.shape) != (B, 4096) or out.dtype != dt or not out.is_contiguous():
         raise ValueError("stage0: bad output buffer")
+    if keep is not None:
+        if w.precision != "fp32":
+            raise ValueError("stage0: keep exists for the fp32 precision only")
+        _check_act(keep, (3, 32, 32), torch.float32, "stage0 keep")
+        if keep.shape[0] != B or keep.untyped_storage().data_ptr() == x.untyped_storage().data_ptr():
+            raise ValueError("stage0: keep must be as large as x and apart from it")
     if w.precision == "fp32":
         check(lib().cifar_stage0_x3(ptr(x), ptr(out), ptr(w.w1h), ptr(w.w1l), ptr(w.b1), ptr(w.w2h), ptr(w.w2l),
-                                    ptr(w.b2), B, grid, stream_ptr(), split), "cifar_stage0_x3")
+                                    ptr(w.b2), B, grid, stream_ptr(), split, ptr(keep)), "cifar_stage0_x3")
     else:
         check(lib().cifar_stage0_v4(ptr(x), ptr(out), ptr(w.w1), ptr(w.b1), ptr(w.w2), ptr(w.b2), B, grid,
                                     stream_ptr()), "cifar_stage0_v4")

@@ -28,19 +28,32 @@ class ColocatedPipeline:
             self.bufs.append(torch.empty(oshp, dtype=odt, device=dev))
         self._graph: Optional[GraphedStep] = None
 
-    def _step(self):
+    def _step(self, x: Optional[torch.Tensor] = None):
         h = self.x
-        for s, b in zip(self.stages, self.bufs):
-            h = s.forward(h, b)
+        for i, (s, b) in enumerate(zip(self.stages, self.bufs)):
+            h = s.forward(x, b, keep=self.x) if i == 0 and x is not None else s.forward(h, b)
         return h
 
     def capture(self) -> None:
         self._graph = GraphedStep(self._step, self.stages[0].device)
 
+    def _reads(self, x: torch.Tensor) -> bool:
+        """Can the first stage read ``x`` where it lies?  Its launch then leaves the
+        copy in ``self.x`` that a later call without an input runs on."""
+        return (getattr(self.stages[0], "keeps_input", False) and type(x) is torch.Tensor and x.is_cuda
+                and x.device == self.x.device and x.device.index == torch.cuda.current_device() and x.dtype == self.x.dtype
+                and x.shape == self.x.shape and x.is_contiguous() and not x.requires_grad
+                and x.untyped_storage().data_ptr() != self.x.untyped_storage().data_ptr())
+
     def __call__(self, x: Optional[torch.Tensor] = None) -> StageOutput:
-        if x is not None:
+        # an input read in place: no copy kernel in front (301 of 2718 us at 65536 images),
+        # and the few launches of a pass go out before the device has run the first
+        direct = x is not None and self._reads(x)
+        if x is not None and not direct:
             self.x.copy_(x, non_blocking=True)
         with trace.span("pipeline_step", "compute", device=self.x.device, batch=self.batch):
+            if direct:
+                return self._step(x)
             if self._graph is not None:
                 return self._graph()
             return self._step()

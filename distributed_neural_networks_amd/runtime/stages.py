@@ -117,7 +117,12 @@ class CifarHipStage(StageCompute):
             self._scratch[batch] = b
         return b
 
-    def forward(self, x, out=None):
+    @property
+    def keeps_input(self) -> bool:
+        """``forward(keep=)``: the launch that reads the images can leave a copy of them."""
+        return self.first and self.precision == "fp32"
+
+    def forward(self, x, out=None, keep=None):
         B = x.shape[0]
         buf = self._buf(B)
         h = x
@@ -125,7 +130,7 @@ class CifarHipStage(StageCompute):
             if h.dtype != torch.float32:
                 h = h.float()
             h = self._cops.stage0_forward(h.contiguous(), self.w0, buf["mid"] if self.end >= 2 else out,
-                                          boundary=self.boundary)
+                                          boundary=self.boundary, keep=keep)
             if self.end == 1:
                 return h
         elif h.dtype != self.adt:

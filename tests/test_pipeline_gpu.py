@@ -184,3 +184,34 @@ def test_microbatched_stream_equals_per_microbatch():
     mono = ColocatedPipeline(st, 512)(x).probs
     torch.cuda.synchronize()
     assert (torch.cat(parts) - mono).abs().max().item() < 2e-2
+
+
+@pytest.mark.parametrize("batch", [1, 5, 64, 65, 300])
+@pytest.mark.parametrize("captured", [True, False])
+def test_colocated_reads_its_input_in_place(batch, captured):
+    """An input on the device is read where it lies (bands of few images and the
+    persistent kernel: 4 B <= 256 and beyond): the bits of a copied input, the copy is
+    left behind for a call without one, and the input itself is not kept."""
+    from distributed_neural_networks_amd.models.cifar import NeuralNetwork
+    from distributed_neural_networks_amd.runtime.pipeline import ColocatedPipeline
+    from distributed_neural_networks_amd.runtime.stages import CifarHipStage
+    dev = torch.device("cuda", 0)
+    torch.manual_seed(3)
+    sd = NeuralNetwork().eval().state_dict()
+    pipe = ColocatedPipeline([CifarHipStage(sd, 0, 1, dev), CifarHipStage(sd, 2, 3, dev)], batch)
+    if captured:
+        pipe.capture()
+    xs = [torch.randn(batch, 3, 32, 32, device=dev) for _ in range(2)]
+    xs.append(torch.randn(batch, 32, 32, 3, device=dev).permute(0, 3, 1, 2))  # strided, host, other type: copied
+    xs += [torch.randn(batch, 3, 32, 32), torch.randn(batch, 3, 32, 32, device=dev, dtype=torch.float64)]
+    for x in xs:
+        pipe.x.copy_(x)
+        want = pipe().probs.clone()
+        pipe.x.zero_()
+        got = pipe(x)
+        assert torch.equal(got.probs, want) and torch.equal(pipe.x, x.to(pipe.x))
+        if x.is_cuda:
+            x.zero_()
+        assert torch.equal(pipe().probs, want)
+    pipe.x.copy_(xs[3])
+    assert torch.equal(pipe(pipe.x).probs, pipe().probs)  # its own buffer
