@@ -24,9 +24,9 @@
 //    (four 16-lane groups) conflict-free; conv2 results leave straight from
 //    the accumulators as 8-B fp32 stores (no LDS staging).
 //  * cifar_fc1_x3_kernel: fc1 + bias + ReLU on the fp32 boundary tensor, the
-//    split done in registers while staging A (no split copy in HBM): 256x256x32
-//    tiles, 8 waves of 128x64, per k32 step 3 x 32 mfma_f32_16x16x32_bf16 per
-//    wave (A_hi W_hi + A_hi W_lo + A_lo W_hi) on 24 conflict-free ds_read_b128.
+//    split done in registers between LDS and the MFMAs (no split copy in HBM):
+//    256x256x32 tiles, 8 waves of 64x128, per k32 step 3 x 32
+//    mfma_f32_16x16x32_bf16 per wave (A_hi W_hi + A_hi W_lo + A_lo W_hi).
 //  * cifar_split3_kernel: fp32 (B,K) -> bf16 (B,3K) = [hi | hi | lo], the A
 //    operand of the mid-batch fc1 (one bf16 GEMM over K' = 3K against
 //    W' = [W_hi | W_lo | W_hi]) when the 256^2 tiles cannot fill the chip.
@@ -37,15 +37,18 @@
 #include <type_traits>
 
 #include "gemm_epilogue.h"
+#include "gemm_tile.h"
 
 namespace dnn {
 namespace x3 {
 
-// 2 floats -> packed bf16 hi pair and lo pair (element a in the low half)
+// 2 floats -> packed bf16 hi pair and lo pair (element a in the low half).  Converted as
+// pairs: 6 vector instructions, 10 where the compiler converts them one by one.
 __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
-  hi = pack2bf(a, b);
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf2));
   const float ah = __uint_as_float(hi << 16), bh = __uint_as_float(hi & 0xffff0000u);
-  lo = pack2bf(a - ah, b - bh);
+  lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a - ah, b - bh}, bf2));
 }
 
 __device__ __forceinline__ int dpp_xor1(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false); }
@@ -470,201 +473,230 @@ __global__ __launch_bounds__(512, 1) void cifar_stage0_x3_band_kernel(
 
 // ---------------------------------------------------------------------------
 // fc1 at fp32 precision: C = relu(A . W^T + bias), A fp32 [M][K], W = W_hi + W_lo
-// (bf16 [N][K] each), C fp32.  A is read from HBM once per tile pair as fp32 and
-// split in registers (global_load_dwordx4 -> split2 -> ds_write_b128) while the
-// W halves stream into LDS by DMA (global_load_lds, source-side swizzle).  LDS:
-// 2 buffers x [A_hi A_lo W_hi W_lo] planes of 256 rows x 32 k (64-B rows, 16 KiB)
-// = 128 KiB.  The 16-B chunk c of row r is stored at c ^ ((r >> 2) & 2): the
-// four ds_read_b128 lane groups ({0-3,12-15,20-27}, ...) of a fragment read
-// (lane: row l & 15, chunk l >> 4) then hit 16 distinct slots, and the A
-// writes (8 contiguous lanes = 2 rows x 4 chunks) 8 distinct ds_write slots.
-// One barrier per k32 step: the step's next-tile loads are issued before its
-// MFMAs and land in the other buffer.
+// (bf16 [N][K] each), C fp32.  256 x 256 tiles, 8 waves (4 M x 2 N) of 2 x 2
+// quadrants of 32 x 64, k-steps of 32.  Both operands come by LDS-DMA in half-tiles
+// of 128 rows (16 KiB: A as the fp32 it is, W as a hi and a lo plane of 64-byte
+// rows), and the waves of column 1 run one barrier behind those of column 0, so that
+// on every SIMD one wave reads and splits while the other multiplies.  A phase is one
+// quadrant, 24 MFMAs:
+//
+//   ph1: read B0, fetch A1       | split A0 | stage B1[t+1] | C00
+//   ph2:                         | split A1 | stage A0[t+2] | C10
+//   ph3: read B1                 |          | stage B0[t+2] | C11
+//   ph4: fetch A0[t+1]           |          | stage A1[t+2] | C01
+//
+// A wave fetches its 32 rows of a half of A as fp32 and splits them in registers in the
+// next phase; two waves split the same rows.  (With 2 M x 4 N waves four do: the kernel
+// is at the card's power limit, and the fewer vector operations count: 657 us at 65536
+// x 512 x 4096, here 624.  Splitting once in LDS, in place, costs as much in LDS traffic:
+// 640.  With A loaded to registers, split and written to LDS between two barriers: 681.
+// A that arrives split: 549.)  A half-tile is staged again at the earliest two phases
+// behind its last read, and a DMA has four to five phases until it is waited for.
+//
+// A's 16-byte chunk c (4 floats) of a row lies in slot ((c >> 1 | (c & 1) << 2) ^
+// swz_chunk(row)): a lane's 8 floats are then slots g and 4 + g, which are read without
+// conflicts.  W's chunk c of a 64-byte row lies at c ^ ((r >> 2) & 2).
+//
+// SPLIT_IN: A arrives pre-split in the blocked boundary encoding (see
+// cifar_split_blocked_kernel: per row and 32-k block, 32 bf16 hi then 32 bf16
+// lo, the same 128 bytes), and nothing is split here.
 // ---------------------------------------------------------------------------
-constexpr int F1_T = 256, F1_K = 32, F1_PLANE = 256 * 64;
+constexpr int F1_T = 256, F1_K = 32;
 
 __device__ __forceinline__ int f1_swz(int r) { return (r >> 2) & 2; }
-
-__device__ __forceinline__ bf16x8 f1_frag(const char* plane, int row, int chunk) {
-  return *reinterpret_cast<const bf16x8*>(plane + row * 64 + ((chunk ^ f1_swz(row)) << 4));
-}
 
 __device__ __forceinline__ void f1_tile_coords(int logical, int ntm, int ntn, int& tm, int& tn) {
   // M fastest inside groups of 8 M-tiles: the ntn column tiles of one A panel
   // run close together on one XCD, so A's second read hits L2 / MALL
-  constexpr int G = 8;
+  constexpr int G = 1;
   const int per = G * ntn, grp = logical / per, first = grp * G;
   const int gm = min(ntm - first, G), r = logical - grp * per;
   tm = first + r % gm;
   tn = r / gm;
 }
 
-// A goes to registers one k-step ahead.  Measured alternatives, dropped: A by
-// DMA into a 32 KiB fp32 staging area two k-steps ahead (5 % slower), the
-// split+store between the two MFMA halves (flat), a second register set for A
-// two k-steps ahead once the loads were coalesced (flat, 6 spilled VGPRs).  Probes
-// (profiles/archive/r2_cifar_fc1_probes.jsonl): without the A stream the kernel runs
-// 0.51 ms, without any load 0.45 ms (1.8 PF/s), with both 0.80 ms.
-//
-// SPLIT_IN: A arrives pre-split in the blocked boundary encoding (see
-// cifar_split_blocked_kernel: per row and 32-k block, 32 bf16 hi then 32 bf16
-// lo — the same 4 bytes per element as fp32, the same hi/lo this kernel would
-// form in registers), so A is staged by DMA exactly like W: no VGPR round
-// trip, no split ALU, no vmcnt stall on A inside the k loop.
+// The 24 products of a phase, between barriers: hi.hi, then W_lo A_hi, then W_hi A_lo of
+// every accumulator
+__device__ __forceinline__ void f1_mfma(f32x4 (&acc)[2][4], const bf16x8 (&a)[2][2], const bf16x8 (&b)[4][2]) {
+  bg_barrier();
+  __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+  for (int jp = 0; jp < 4; jp += 2)  // the first fragments of W to arrive first
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+      for (int j = jp; j < jp + 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j][s == 1], a[i][s == 2], acc[i][j], 0, 0, 0);
+  __builtin_amdgcn_s_setprio(0);
+  bg_barrier();
+}
+
 template <bool SPLIT_IN>
 __global__ __launch_bounds__(512, 1) void cifar_fc1_x3_kernel(const float* __restrict__ A, int lda,
                                                               const bf16_t* __restrict__ Wh,
                                                               const bf16_t* __restrict__ Wl, int ldw,
                                                               const float* __restrict__ bias, float* __restrict__ C,
                                                               int ldc, int M, int N, int K) {
-  __shared__ __attribute__((aligned(1024))) char smem[2 * 4 * F1_PLANE];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ __attribute__((aligned(1024))) char smem[8 * BG_HALF];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ntn = N / F1_T, ntm = (M + F1_T - 1) / F1_T;
   int tm, tn;
   f1_tile_coords(xcd_remap(blockIdx.x, ntm * ntn), ntm, ntn, tm, tn);
   const int m0 = tm * F1_T, n0 = tn * F1_T;
-  const int wr = wave >> 2, wc = wave & 3;
+  const int wr = wave & 3, wc = wave >> 2, fr = lane & 15, fg = lane >> 4;
   const int nk = K / F1_K;
-  auto plane = [&](int u, int p) { return smem + (u * 4 + p) * F1_PLANE; };  // p: 0 A_hi, 1 A_lo, 2 W_hi, 3 W_lo
+  auto half = [&](int u, int h) { return smem + (u * 4 + h) * BG_HALF; };  // h: A0, A1, B0, B1
 
-  // A: 2 chunks (8 fp32 each) per thread; chunk q = tid + 512 i -> row q >> 2, k-chunk q & 3
-  // A: 4 pieces of 16 B per thread; piece k: row (tid >> 3) + 64 k, floats
-  // 4 (tid & 7) .. +3, so every wave load instruction reads 8 whole 128-B row
-  // segments and the split halves land as ds_write_b64 into half of a 16-B LDS
-  // chunk.  (The first mapping, 32 contiguous bytes per lane in two loads,
-  // touched every 128-B line twice per wave: 0.85 -> 0.68 ms.)
-  float4 ar[4];
-  auto load_a = [&](int t, auto) {
+  // A: pieces of 8 rows of 128 bytes, 2 of either half a wave: uniform row bases, the
+  // lane's row (clamped for rows past the matrix) and chunk as 32-bit offsets
+  const uint32_t ldb = (uint32_t)lda * 4u;
+  const char* abase[4];
+  uint32_t alim[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int row = min(m0 + (tid >> 3) + 64 * k, M - 1);
-      ar[k] = *reinterpret_cast<const float4*>(A + (size_t)row * lda + t * F1_K + (tid & 7) * 4);
+  for (int x = 0; x < 4; ++x) {
+    const int r = min(m0 + (x >> 1) * 128 + ((x & 1) * 8 + wave) * 8, M - 1);
+    abase[x] = reinterpret_cast<const char*>(A) + (size_t)r * ldb;
+    alim[x] = (uint32_t)min(7, M - 1 - r) * ldb;
+  }
+  const int slot = (lane & 7) ^ ((wave & 1) * 4 + (lane >> 4));  // swz_chunk of the lane's row in its piece
+  const uint32_t arow_off = (uint32_t)(lane >> 3) * ldb, achunk = (SPLIT_IN ? slot : (slot & 3) << 1 | slot >> 2) * 16u;
+  auto stA = [&](int u, int h, int t) {
+    t = t < nk ? t : nk - 1;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const char* p = abase[2 * h + i] + (size_t)t * 128;
+      asm("" : "+s"(p));  // scalar base, 32-bit lane offset: not folded into per-lane addresses ahead of the loop
+      glds16(p + (min(arow_off, alim[2 * h + i]) + achunk), half(u, h) + (i * 8 + wave) * 1024);
     }
   };
-  auto store_a = [&](int u, auto) {
+  // W: a wave stages 16 rows of 64 bytes of a half's hi and of its lo plane
+  const char* wbase[2];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int r = (tid >> 3) + 64 * k, c = (tid & 7) >> 1, half = tid & 1;
-      uint2 hi, lo;
-      split2(ar[k].x, ar[k].y, hi.x, lo.x);
-      split2(ar[k].z, ar[k].w, hi.y, lo.y);
-      const int o = r * 64 + ((c ^ f1_swz(r)) << 4) + half * 8;
-      *reinterpret_cast<uint2*>(plane(u, 0) + o) = hi;
-      *reinterpret_cast<uint2*>(plane(u, 1) + o) = lo;
-    }
-  };
-  // W: per plane 16 pieces of 16 rows (1 KiB per wave instruction), 2 per wave
-  // SPLIT_IN: A hi / lo planes by DMA, 2 pieces of 16 rows per wave and plane (as W)
-  auto stage_a = [&](int u, int t) {
-    const char* Ab = reinterpret_cast<const char*>(A);
+  for (int p = 0; p < 2; ++p)
+    wbase[p] = reinterpret_cast<const char*>(p ? Wl : Wh) + (size_t)(n0 + wave * 16) * ldw * 2;
+  const uint32_t woff = (uint32_t)(lane >> 2) * (uint32_t)ldw * 2u + (uint32_t)((lane & 3) ^ f1_swz(lane >> 2)) * 16u;
+  auto stB = [&](int u, int h, int t) {
+    t = t < nk ? t : nk - 1;
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
+      const char* s = wbase[p] + (size_t)h * 256 * ldw + (size_t)t * 64;
+      asm("" : "+s"(s));
+      glds16(s + woff, half(u, 2 + h) + p * (BG_HALF / 2) + wave * 1024);
+    }
+  };
+
+  f32x4 acc[2][2][2][4];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int piece = wave * 2 + j, rl = piece * 16 + (lane >> 2);
-        const int c = (lane & 3) ^ f1_swz(rl);
-        const int row = min(m0 + rl, M - 1);
-        glds16(Ab + (size_t)row * lda * 4 + t * 128 + p * 64 + c * 16, plane(u, p) + piece * 1024);
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[a][b][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  bf16x8 a0[2][2], a1[2][2], bb[4][2];
+  f32x4 raw[2][2];
+  const int arow = wr * 32 + fr, brow = wc * 64 + fr;
+  // LDS offsets of the lane's fragments, moved from buffer to buffer: 128 KiB are more
+  // than a read's immediate offset reaches, and registers for both would spill
+  uint32_t ao[2], bo = 2 * BG_HALF + brow * 64 + ((fg ^ f1_swz(brow)) << 4);
+#pragma unroll
+  for (int s = 0; s < 2; ++s) ao[s] = arow * 128 + (((s * 4 + fg) ^ swz_chunk(arow)) << 4);
+  auto fetch = [&](int h) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) raw[i][s] = *reinterpret_cast<const f32x4*>(smem + ao[s] + (h * BG_HALF + i * 2048));
+  };
+  auto fetched = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+  auto split = [&](bf16x8 (&a)[2][2]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if constexpr (SPLIT_IN) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) a[i][s] = __builtin_bit_cast(bf16x8, raw[i][s]);
+      } else {
+        uint4 hi, lo;
+        split2(raw[i][0][0], raw[i][0][1], hi.x, lo.x);
+        split2(raw[i][0][2], raw[i][0][3], hi.y, lo.y);
+        split2(raw[i][1][0], raw[i][1][1], hi.z, lo.z);
+        split2(raw[i][1][2], raw[i][1][3], hi.w, lo.w);
+        a[i][0] = __builtin_bit_cast(bf16x8, hi);
+        a[i][1] = __builtin_bit_cast(bf16x8, lo);
       }
     }
+    __builtin_amdgcn_sched_barrier(0);  // the next fragments take raw's registers
   };
-  auto stage_w = [&](int u, int t) {
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      const bf16_t* W = p ? Wl : Wh;
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int piece = wave * 2 + j, rl = piece * 16 + (lane >> 2);
-        const int c = (lane & 3) ^ f1_swz(rl);
-        glds16(W + (size_t)(n0 + rl) * ldw + t * F1_K + c * 8, plane(u, 2 + p) + piece * 1024);
-      }
-    }
-  };
-
-  f32x4 acc[8][4];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  using I0 = std::integral_constant<int, 0>;
-  if constexpr (SPLIT_IN) {
-    stage_a(0, 0);
-    stage_w(0, 0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  } else {
-    load_a(0, I0{});
-    stage_w(0, 0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    store_a(0, I0{});
-  }
-  __syncthreads();
-
-  const int fr = lane & 15, fc = lane >> 4;
-  auto compute = [&](int u) {
-    const char* ah_p = plane(u, 0);
-    const char* al_p = plane(u, 1);
-    const char* bh_p = plane(u, 2);
-    const char* bl_p = plane(u, 3);
-    bf16x8 bh[4], bl[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      bh[j] = f1_frag(bh_p, wc * 64 + j * 16 + fr, fc);
-      bl[j] = f1_frag(bl_p, wc * 64 + j * 16 + fr, fc);
-    }
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      bf16x8 ah[4], al[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        ah[i] = f1_frag(ah_p, wr * 128 + (h * 4 + i) * 16 + fr, fc);
-        al[i] = f1_frag(al_p, wr * 128 + (h * 4 + i) * 16 + fr, fc);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          f32x4& a = acc[h * 4 + i][j];
-          a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[j], ah[i], a, 0, 0, 0);
-          a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl[j], ah[i], a, 0, 0, 0);
-          a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[j], al[i], a, 0, 0, 0);
-        }
-    }
-  };
-  // raw barrier (lgkmcnt for this step's LDS writes; the DMAs were waited
-  // above): 6 % faster than __syncthreads here
-  auto barrier = [&]() {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  for (int t = 0; t < nk; ++t) {
-    const int u = t & 1;
-    if (t + 1 < nk) {
-      if constexpr (SPLIT_IN)
-        stage_a(u ^ 1, t + 1);
-      else
-        load_a(t + 1, I0{});
-      stage_w(u ^ 1, t + 1);
-    }
-    compute(u);
-    if (t + 1 < nk) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if constexpr (!SPLIT_IN) store_a(u ^ 1, I0{});
-    }
-    barrier();
-  }
-
-  // epilogue (transposed accumulators): row m0 + wr*128 + i*16 + (lane & 15), cols n..n+3
-  const bool vec = epi_vec_ok(C, ldc, bias, nullptr, 0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int m = m0 + wr * 128 + i * 16 + fr;
+  auto readB = [&](int h) {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      epi_t4<ACT_RELU, true>(acc[i][j], m, n0 + wc * 64 + j * 16 + fc * 4, M, N, C, ldc, bias, nullptr, 0, vec);
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        bb[j][p] = *reinterpret_cast<const bf16x8*>(smem + bo + (h * BG_HALF + p * (BG_HALF / 2) + j * 1024));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // prologue: A0, B0 and A1 of tile 0 landed, four half-tiles in flight
+  stA(0, 0, 0);
+  stB(0, 0, 0);
+  stA(0, 1, 0);
+  stB(0, 1, 0);
+  stA(1, 0, 1);
+  stB(1, 0, 1);
+  stA(1, 1, 1);
+  bg_landed<8>();
+  bg_barrier();
+  if (wc == 1) bg_barrier();
+  fetch(0);
+
+  for (int t = 0, u = 0; t < nk; ++t, u ^= 1) {
+    // ph1
+    fetched();
+    readB(0);
+    split(a0);
+    fetch(1);
+    stB(u ^ 1, 1, t + 1);
+    f1_mfma(acc[0][0], a0, bb);
+    // ph2
+    fetched();
+    split(a1);
+    stA(u, 0, t + 2);
+    bg_landed<10>();  // B1 of tile t
+    f1_mfma(acc[1][0], a1, bb);
+    // ph3
+    readB(1);
+    stB(u, 0, t + 2);
+    bg_landed<10>();  // A0 of tile t + 1
+    f1_mfma(acc[1][1], a1, bb);
+    // ph4
+    fetched();
+    ao[0] ^= 4 * BG_HALF, ao[1] ^= 4 * BG_HALF, bo ^= 4 * BG_HALF;
+    fetch(0);
+    stA(u, 1, t + 2);
+    bg_landed<8>();  // B0 and A1 of tile t + 1
+    f1_mfma(acc[0][1], a0, bb);
   }
+  fetched();
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (wc == 0) bg_barrier();
+
+  // epilogue (transposed accumulators): row m0 + mq 128 + wr 32 + i 16 + (lane & 15), cols n..n+3
+  const bool vec = epi_vec_ok(C, ldc, bias, nullptr, 0);
+#pragma unroll
+  for (int mq = 0; mq < 2; ++mq)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int m = m0 + mq * 128 + arow + i * 16;
+#pragma unroll
+      for (int nq = 0; nq < 2; ++nq)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          epi_t4<ACT_RELU, true>(acc[mq][nq][i][j], m, n0 + nq * 128 + wc * 64 + j * 16 + fg * 4, M, N, C, ldc, bias,
+                                 nullptr, 0, vec);
+    }
 }
 
 // Blocked boundary encoding of an fp32 (M,K) tensor, in place of the same
@@ -1002,6 +1034,7 @@ extern "C" int dnn_cifar_fc1_x3(const float* A, int lda, const void* Wh, const v
                                 float* C, int ldc, int M, int N, int K, hipStream_t st, int a_split) {
   if (M <= 0) return 0;
   if (N % F1_T != 0 || K % F1_K != 0 || lda % 4 != 0 || ldw % 8 != 0 || ldc % 4 != 0) return -1;
+  if (lda >= 1 << 27 || ldw >= 1 << 27) return -1;  // 8 rows of A and 16 of W are addressed with 32 bits
   const int blocks = ((M + F1_T - 1) / F1_T) * (N / F1_T);
   if (a_split)
     hipLaunchKernelGGL(cifar_fc1_x3_kernel<true>, dim3(blocks), dim3(512), 0, st, A, lda, (const bf16_t*)Wh,

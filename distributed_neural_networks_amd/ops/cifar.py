@@ -7,19 +7,17 @@ fp32 modules to the device):
   Every fp32 operand is split into bf16 hi + lo and each product is three bf16
   MFMAs (hi*hi + hi*lo + lo*hi) accumulated in fp32.  Stage boundary tensor
   ``(B,4096)`` fp32 exactly as the reference ships it (``node.py:45-48``).
-  fc1 at large batch is ``cifar_fc1_x3``: the fp32 boundary rows are split in
-  registers while staged to LDS (A read once as fp32, no split copy); at small
+  fc1 at large batch is ``cifar_fc1_x3``: the fp32 boundary rows come to LDS as they
+  are and are split in registers on their way to the MFMAs (no split copy); at small
   batch (too few 256-row tiles to fill the chip) it runs as ONE skinny/128^2
   bf16 GEMM over K' = 3*4096 on ``[A_hi | A_hi | A_lo]`` x ``[W_hi | W_lo | W_hi]``.
   Optional boundary encoding ``boundary="split"`` (fp32 only, both ends of
   the hop must be these kernels): the same 16 KiB/img, each row as 32-k blocks
   of 32 bf16 hi then 32 bf16 lo — the very hi/lo operands the x3 MFMAs consume
   (hi + lo = the fp32 value to ~2^-17) — written by the stage-0 epilogue and
-  staged into LDS by DMA in fc1 (no register split pass): fc1 0.710 -> 0.632
-  ms at B=65536 with bit-identical outputs (profiles/r3_fc1_split_ab.jsonl),
-  but the split stores cost the stage-0 epilogue as much, so the 2-stage step
-  is unchanged (2.541 vs 2.548 ms, profiles/r3_boundary_ab.jsonl) and the
-  pipelines keep plain fp32 (also the wire format a reference peer expects).
+  read as they lie in fc1: 0.624 -> 0.549 ms at B=65536 with bit-identical
+  outputs, but the split stores cost the stage-0 epilogue as much, so the 2-stage
+  step is unchanged (2.41 vs 2.43 ms) and the pipelines keep plain fp32 (also the wire format a reference peer expects).
   ``decode_boundary`` / ``encode_boundary`` convert.
 * ``bf16``: ``csrc/kernels/cifar_fused.hip`` (v4 persistent kernel), bf16
   boundary, an explicitly reduced-precision mode.
@@ -145,9 +143,10 @@ def act_dtype(precision: str) -> torch.dtype:
 
 
 STAGE0_GRID = 0  # persistent stage-0 workgroups; 0 = one per CU (256)
-# fused fp32 fc1 from this batch on: 2 x B/256 tiles of 128 k32 steps each need
-# >= 128 tiles to occupy the chip; below, split3 + the K-concat GEMM is faster
-FC1_X3_MIN_ROWS = 16384
+# fused fp32 fc1 from this batch on: 2 x B/256 tiles of 128 k32 steps each, one round up to
+# 32768 rows whatever the batch.  us, split3 and the K-concat GEMM : fused: 8192 rows 197 :
+# 237, 9216 251 : 230, 12288 291 : 232, 16384 324 : 235
+FC1_X3_MIN_ROWS = 8704
 # fp32 head up to this batch: fc1 in slices of K and a finish of one workgroup a row
 # (pipeline pass, us, with and without: 1 row 27.7 / 44.3, 64 29.7 / 57.4, 256 50.6 /
 # 84.9, 512 79.1 / 88.3, 768 104.4 / 96.2: each 32 rows are a round of every workgroup)

@@ -365,6 +365,33 @@ def test_cifar_fc1_x3_kernel(M, N, K, split_in):
     assert err <= 2e-5 * ref.abs().max().item(), err
 
 
+@pytest.mark.parametrize("split_in", [0, 1])
+@pytest.mark.parametrize("M,N,K,pad", [(1, 256, 32, 0), (255, 256, 64, 4), (257, 512, 96, 32), (600, 512, 160, 0)])
+def test_cifar_fc1_x3_edges(M, N, K, pad, split_in):
+    """One to five k-steps (the DMAs run up to two ahead and refill the last one past
+    the end), rows past the matrix, rows of a wider tensor, the widest range of values
+    a split takes.  Two terms of a product are off by 2^-16 of it, and K fp32 sums by
+    K 2^-24: within 2^-14 of the sum of magnitudes."""
+    from distributed_neural_networks_amd.ops import _lib
+    from distributed_neural_networks_amd.ops.cifar import encode_boundary, split_bf16
+    torch.manual_seed(M)
+    a = torch.randn(M, K, device=DEV) * torch.exp2(torch.randint(-40, 40, (M, 1), device=DEV).float())
+    w = torch.randn(N, K, device=DEV)
+    b = torch.zeros(N, device=DEV)
+    wh, wl = split_bf16(w)
+    rows = torch.full((M, K + pad), float("nan"), device=DEV)
+    rows[:, :K] = encode_boundary(a) if split_in else a
+    out = torch.full((M + 1, N), 7.0, device=DEV)
+    rc = _lib.lib().cifar_fc1_x3(rows.data_ptr(), K + pad, wh.data_ptr(), wl.data_ptr(), K, b.data_ptr(), out.data_ptr(),
+                                 N, M, N, K, torch.cuda.current_stream().cuda_stream, split_in)
+    assert rc == 0
+    torch.cuda.synchronize()
+    ref = torch.relu(a.double() @ w.double().t())
+    bound = a.double().abs() @ w.double().abs().t() * 2 ** -14
+    assert ((out[:M].double() - ref).abs() <= bound).all()
+    assert (out[M] == 7).all()
+
+
 @pytest.mark.parametrize("boundary", ["fp32", "split"])
 @pytest.mark.parametrize("B", [1, 2, 15, 16, 17, 32, 33, 64, 65, 500, 512])
 def test_cifar_few_images(B, boundary):
