@@ -274,6 +274,28 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_256_kernel(
     return;
   }
 
+  // Channel scales and (QOUT, or where the LDS copy is whole) bias of the lane's columns, once:
+  // looked up at every product they put three paths and a wait around each, and the epilogue
+  // of 2048 x 4800 x 1600 took as long as its 13 K-tiles (31.3 us; 26.5 with the scatter's
+  // addresses formed once as well, 2048 x 6400 x 1600 with GELU 39.0 : 37.6).
+  f32x4 cs[NQ][2], bs[NQ][2];
+#pragma unroll
+  for (int nq = 0; nq < NQ; ++nq)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int n = n0 + nq * 128 + wc * 32 + j * 16 + (lane >> 4) * 4;
+      bs[nq][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (epv) {  // the LDS copy (columns past N are not stored)
+        cs[nq][j] = *reinterpret_cast<const f32x4*>(epi + EPI_C + 4 * (n - n0));
+        if (bias != nullptr) bs[nq][j] = *reinterpret_cast<const f32x4*>(epi + EPI_B + 4 * (n - n0));
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          cs[nq][j][r] = n + r < N ? sw[n + r] : 0.f;
+          if (QOUT) bs[nq][j][r] = (bias != nullptr && n + r < N) ? bias[n + r] : 0.f;
+        }
+      }
+    }
   if constexpr (QOUT) {
     // bias + GELU in place, then per (row, 128-column half nq) amax: the lane's
     // 8 columns, the 4 lane rows of the wave (xor 16 / 32), the 4 waves of the
@@ -290,23 +312,7 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_256_kernel(
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
             const int n = n0 + nq * 128 + wc * 32 + j * 16 + (lane >> 4) * 4;
-            // 16-B channel-scale / bias loads (per-element ones were 8 scalar
-            // loads per quad)
-            f32x4 cs, bs = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (epv) {  // the LDS copy (columns past N are zeroed below)
-              cs = *reinterpret_cast<const f32x4*>(epi + EPI_C + 4 * (n - n0));
-              if (bias != nullptr) bs = *reinterpret_cast<const f32x4*>(epi + EPI_B + 4 * (n - n0));
-            } else if (n + 3 < N) {
-              cs = *reinterpret_cast<const f32x4*>(sw + n);
-              if (bias != nullptr) bs = *reinterpret_cast<const f32x4*>(bias + n);
-            } else {
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                cs[r] = n + r < N ? sw[n + r] : 0.f;
-                bs[r] = (bias != nullptr && n + r < N) ? bias[n + r] : 0.f;
-              }
-            }
-            f32x4 v = acc[mq][nq][i][j] * cs + bs;
+            f32x4 v = acc[mq][nq][i][j] * cs[nq][j] + bs[nq][j];
             const f32x2 g0 = gelu_erf2(f32x2{v[0], v[1]}), g1 = gelu_erf2(f32x2{v[2], v[3]});
             v = f32x4{g0[0], g0[1], g1[0], g1[1]};
 #pragma unroll
@@ -351,13 +357,23 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_256_kernel(
   }
   const bool badd = epv && bias != nullptr && !is_glu(ACT);  // uniform: bias added from the LDS copy
   const float* bias_e = badd ? nullptr : bias;
-  // SCATTER: the cache positions of the lane's 8 rows, loaded before any store (qkv_row_pos)
-  int spos[2][4] = {};
+  // SCATTER: the destinations' parts (qkv_row), before any store; bias that is not in LDS
+  QkvRow srow[2][4];
+  QkvCol scol[NQ];
   if constexpr (SCATTER) {
 #pragma unroll
     for (int mq = 0; mq < 2; ++mq)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) spos[mq][i] = qkv_row_pos(scat, min(m0 + mq * 128 + arow + i * 16 + (lane & 15), M - 1));
+      for (int i = 0; i < 4; ++i) srow[mq][i] = qkv_row(scat, min(m0 + mq * 128 + arow + i * 16 + (lane & 15), M - 1));
+#pragma unroll
+    for (int nq = 0; nq < NQ; ++nq) {
+      const int nb = n0 + nq * 128 + wc * 32 + scat.c_off;
+      scol[nq] = qkv_col(scat, pair_col(nb, lane));
+      if (bias_e != nullptr && nb - scat.c_off < N) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) bs[nq][j] = *reinterpret_cast<const f32x4*>(bias_e + nb + j * 16 + (lane >> 4) * 4);
+      }
+    }
   }
   const bool vec = epi_vec_ok(C, ldc, bias, R, ldr);
   const bool pair = vec && epi_pair_ok(C, ldc, bias, R, ldr);
@@ -396,21 +412,12 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_256_kernel(
         f32x4 v[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          const int n = nb + j * 16 + (lane >> 4) * 4;
-          f32x4 cs;
-          if (epv) {
-            cs = *reinterpret_cast<const f32x4*>(epi + EPI_C + 4 * (n - n0));
-          } else if (n + 3 < N) {
-            cs = *reinterpret_cast<const f32x4*>(sw + n);
-          } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) cs[r] = n + r < N ? sw[n + r] : 0.f;
-          }
-          v[j] = acc[mq][nq][i][j] * (cs * rs);
-          if (badd) v[j] += *reinterpret_cast<const f32x4*>(epi + EPI_B + 4 * (n - n0));
+#pragma clang fp contract(off)  // the product is rounded before the bias, on every path
+          v[j] = acc[mq][nq][i][j] * (cs[nq][j] * rs);
+          if (badd || (SCATTER && bias != nullptr)) v[j] += bs[nq][j];
         }
         if (SCATTER) {
-          if (nb < N) epi_pair_scatter(v[0], v[1], m, nb + scat.c_off, M, bias_e, lane, scat, spos[mq][i]);
+          if (nb < N) epi_pair_scatter(v[0], v[1], m, M, srow[mq][i], scol[nq]);
         } else if (is_glu(ACT)) {
           epi_glu_pair<ACT, false>(v[0], v[1], m, nb / 2, M, N / 2, C, ldc, vec, lane);
         } else if (rdma) {

@@ -53,6 +53,12 @@ __device__ __forceinline__ f32x4 mid_act(f32x4 v, const f32x2& xc) {
   return v;
 }
 
+// Whether a wave's whole columns leave as pairs of 16-byte stores (uniform).
+__device__ __forceinline__ bool mid_pair(const MidRows& p, int nw, int J) {
+  return !p.f32 && epi_vec_ok(p.C, p.ldc, p.bias, p.R, p.ldr) && epi_pair_ok(p.C, p.ldc, p.bias, p.R, p.ldr) &&
+         nw + J * 16 <= p.N;
+}
+
 // 4 finished columns of a row: residual and store, bf16 or fp32.
 __device__ __forceinline__ void epi_t4_any(const f32x4& v, int m, int n, int M, int N, const MidRows& p, const bf16_t* R,
                                            bool vec) {
@@ -60,16 +66,51 @@ __device__ __forceinline__ void epi_t4_any(const f32x4& v, int m, int n, int M, 
   else epi_t4<ACT_NONE, false>(v, m, n, M, N, p.C, p.ldc, nullptr, R, p.ldr, vec);
 }
 
-// Bias and an elementwise activation on a wave's accumulators.
-template <int I, int J, bool ALL = true>
-__device__ __forceinline__ void mid_bias_act(f32x4 (&acc)[I][J], const float* bias, int act, int n0, int N) {
-  if (bias != nullptr) {
+// What the epilogue of a wave reads, loaded ahead of the loop: behind it statistics and
+// column sums, bias, then residual rows were up to three trips to memory, 0.5 us each, of
+// kernels that take 6 to 40 (with residual, 1071 x 768 x 768 and x 3072: 11.8 us on average,
+// now 10.8).  The residual only where there are registers for it.
+template <int I, int J>
+struct MidPre {
+  static constexpr bool RES = I * J <= 8;
+  float2 rs[I];
+  f32x4 cs[J], bs[J];
+  bf16x4 rr[RES ? I : 1][J / 2][2];
+  bool res;  // rr is loaded
+  // rows m of this lane from mw on, the wave's columns from nw on; `scale`: per column (colsum, channel scale) or null
+  __device__ __forceinline__ void load(const MidRows& p, const float2* rowstat, const float* scale, int mw, int nw, int lane,
+                                       bool rows) {
+    const int M = p.M, N = p.N, n = nw + (lane >> 4) * 4;
+#pragma unroll
+    for (int i = 0; i < I; ++i) rs[i] = rowstat != nullptr ? rowstat[min(mw + i * 16, M - 1)] : float2{1.f, 0.f};
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-      const f32x4 b4 = mid_cols(bias, n0 + j * 16, N);
-#pragma unroll
-      for (int i = 0; i < I; ++i) acc[i][j] += b4;
+      cs[j] = scale != nullptr ? mid_cols(scale, n + j * 16, N) : f32x4{0.f, 0.f, 0.f, 0.f};
+      bs[j] = p.bias != nullptr && !is_glu(p.act) ? mid_cols(p.bias, n + j * 16, N) : f32x4{0.f, 0.f, 0.f, 0.f};
     }
+    res = false;
+    if constexpr (RES) {
+      if (rows && p.R != nullptr && !is_glu(p.act) && mid_pair(p, nw, J)) {
+        res = true;
+#pragma unroll
+        for (int i = 0; i < I; ++i)
+#pragma unroll
+          for (int jp = 0; jp < J / 2; ++jp)
+            epi_pair_res_load(mw + i * 16, nw + jp * 32, M, p.R, p.ldr, lane, rr[i][jp][0], rr[i][jp][1]);
+      }
+    }
+  }
+};
+
+// Bias and an elementwise activation on a wave's accumulators.
+template <int I, int J, bool ALL = true>
+__device__ __forceinline__ void mid_bias_act(f32x4 (&acc)[I][J], const float* bias, const f32x4 (&bs)[J], int act, int N) {
+#pragma clang fp contract(off)  // a product in front (norm, channel scale) is rounded before the bias
+  if (bias != nullptr) {
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+      for (int i = 0; i < I; ++i) acc[i][j] += bs[j];
   }
   if (act == ACT_GELU) {
 #pragma unroll
@@ -128,23 +169,27 @@ struct MidSource {
 
 // A wave's accumulators to head-major q / K / V (host: N % 32 == 0).
 template <int I, int J>
-__device__ __forceinline__ void mid_scatter(const f32x4 (&acc)[I][J], int mw, int nw, int M, int N, const float* bias, int lane,
-                                            const QkvScatter& scat) {
-  int spos[I];
+__device__ __forceinline__ void mid_scatter(f32x4 (&acc)[I][J], int mw, int nw, int M, int N, const float* bias,
+                                            const f32x4 (&bs)[J], int lane, const QkvScatter& scat) {
+  QkvRow row[I];
+  QkvCol col[J / 2];
 #pragma unroll
-  for (int i = 0; i < I; ++i) spos[i] = qkv_row_pos(scat, min(mw + i * 16, M - 1));
+  for (int i = 0; i < I; ++i) row[i] = qkv_row(scat, min(mw + i * 16, M - 1));
+#pragma unroll
+  for (int jp = 0; jp < J / 2; ++jp) col[jp] = qkv_col(scat, pair_col(nw + jp * 32, lane));
+  mid_bias_act<I, J, false>(acc, bias, bs, ACT_NONE, N);
 #pragma unroll
   for (int i = 0; i < I; ++i)
 #pragma unroll
     for (int jp = 0; jp < J / 2; ++jp)
-      if (nw + jp * 32 < N)
-        epi_pair_scatter(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, nw + jp * 32, M, bias, lane, scat, spos[i]);
+      if (nw + jp * 32 < N) epi_pair_scatter(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, M, row[i], col[jp]);
 }
 
 // A wave's accumulators (rows mw + 16 i of this lane, columns from nw on) through the epilogue to C.
 // ALL: with fp32 rows and the activations that only bf16 weights have.
 template <int I, int J, bool ALL = true>
-__device__ __forceinline__ void mid_rows(f32x4 (&acc)[I][J], int mw, int nw, int lane, const MidRows& p) {
+__device__ __forceinline__ void mid_rows(f32x4 (&acc)[I][J], int mw, int nw, int lane, const MidRows& p,
+                                         const MidPre<I, J>& pre) {
   const int M = p.M, N = p.N, fg = lane >> 4;
   const bool f32 = ALL && p.f32;
   const bool vec = epi_vec_ok(p.C, p.ldc, p.bias, p.R, p.ldr);
@@ -161,10 +206,17 @@ __device__ __forceinline__ void mid_rows(f32x4 (&acc)[I][J], int mw, int nw, int
       }
     return;
   }
-  mid_bias_act<I, J, ALL>(acc, p.bias, p.act, nw + fg * 4, N);
+  mid_bias_act<I, J, ALL>(acc, p.bias, pre.bs, p.act, N);
   bf16_t* C = reinterpret_cast<bf16_t*>(p.C);
-  const bool pair = vec && !f32 && epi_pair_ok(p.C, p.ldc, p.bias, p.R, p.ldr) && nw + J * 16 <= N;
-  if (pair && p.R != nullptr) {  // every residual load before the first output
+  const bool pair = mid_pair(p, nw, J);
+  if (MidPre<I, J>::RES && pre.res) {
+#pragma unroll
+    for (int i = 0; i < (MidPre<I, J>::RES ? I : 1); ++i)
+#pragma unroll
+      for (int jp = 0; jp < J / 2; ++jp)
+        epi_pair_bf16<ACT_NONE, true>(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, nw + jp * 32, M, C, p.ldc, nullptr,
+                                      p.R, p.ldr, lane, pre.rr[i][jp][0], pre.rr[i][jp][1]);
+  } else if (!MidPre<I, J>::RES && pair && p.R != nullptr) {  // every residual load before the first output
     bf16x4 rr[I][J / 2][2];
 #pragma unroll
     for (int i = 0; i < I; ++i)
@@ -301,6 +353,9 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvS
   MidSource<T> src;
   src.init(reinterpret_cast<const char*>(p.A), p.lda * 2, m0, M, reinterpret_cast<const char*>(p.W), p.ldw * 2, n0, N, k0,
            nk, smem, wave, lane);
+  const int mw = m0 + wm * (I * 16) + fr, nw = n0 + wn * (J * 16);  // the lane's first row, the wave's first column
+  MidPre<I, J> pre;
+  if constexpr (!PART) pre.load(p, p.rowstat, p.colsum, mw, nw, lane, OUT == MID_ROWS);
   f32x4 acc[I][J];
   mid_loop<T>(src, wm, wn, lane, acc);
 
@@ -317,22 +372,14 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvS
     }
     return;
   }
-  const int mw = m0 + wm * (I * 16) + fr, nw = n0 + wn * (J * 16);  // the lane's first row, the wave's first column
   if (p.rowstat != nullptr) {  // the folded norm, in the 256 x 256 kernel's order of operations
-    float2 rs[I];
-    f32x4 cs[J];
-#pragma unroll
-    for (int i = 0; i < I; ++i) rs[i] = p.rowstat[min(mw + i * 16, M - 1)];
-#pragma unroll
-    for (int j = 0; j < J; ++j)
-      cs[j] = p.colsum != nullptr ? mid_cols(p.colsum, nw + j * 16 + fg * 4, N) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < I; ++i)
 #pragma unroll
-      for (int j = 0; j < J; ++j) acc[i][j] = acc[i][j] * rs[i].x + rs[i].y * cs[j];
+      for (int j = 0; j < J; ++j) acc[i][j] = acc[i][j] * pre.rs[i].x + pre.rs[i].y * pre.cs[j];
   }
-  if constexpr (OUT == MID_SCATTER) mid_scatter<I, J>(acc, mw, nw, M, N, p.bias, lane, scat);
-  else mid_rows<I, J>(acc, mw, nw, lane, p);
+  if constexpr (OUT == MID_SCATTER) mid_scatter<I, J>(acc, mw, nw, M, N, p.bias, pre.bs, lane, scat);
+  else mid_rows<I, J>(acc, mw, nw, lane, p, pre);
 }
 
 // Sum of the parts and the epilogue.  A thread: 4 columns of one row (gated: 4
@@ -363,7 +410,8 @@ __global__ __launch_bounds__(256) void gemm_mid_reduce(MidArgs p) {
     return;
   }
   f32x4 a[1][1] = {{v}};
-  mid_bias_act<1, 1>(a, p.bias, p.act, n, N);
+  const f32x4 b[1] = {p.bias != nullptr ? mid_cols(p.bias, n, N) : f32x4{0.f, 0.f, 0.f, 0.f}};
+  mid_bias_act<1, 1>(a, p.bias, b, p.act, N);
   epi_t4_any(a[0][0], m, n, M, N, p, p.R, vec);
 }
 

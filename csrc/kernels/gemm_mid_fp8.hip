@@ -57,6 +57,9 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_fp8_kernel(Mid8Args p,
   const int ao[2] = {arow * 128 + ((fg ^ swz_chunk(arow)) << 4), arow * 128 + (((4 + fg) ^ swz_chunk(arow)) << 4)};
   const int bo[2] = {T::BM * 128 + brow * 128 + ((fg ^ swz_chunk(brow)) << 4),
                      T::BM * 128 + brow * 128 + (((4 + fg) ^ swz_chunk(brow)) << 4)};
+  const int mw = m0 + wm * (I * 16) + fr, nw = n0 + wn * (J * 16);
+  MidPre<I, J> pre;  // cs: the channel scales
+  pre.load(p, nullptr, p.sw, mw, nw, lane, OUT == MID8_ROWS);
   bf16x8 fa[2][I][2], fb[2][J][2];
   uint32_t fs[2];
   auto read = [&](auto uc, int buf) {
@@ -125,10 +128,6 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_fp8_kernel(Mid8Args p,
   if (t < nk) ktile(t, c0);
   __builtin_amdgcn_s_waitcnt(wait_imm(0, 0));
 
-  const int mw = m0 + wm * (I * 16) + fr, nw = n0 + wn * (J * 16);
-  f32x4 cs[J];
-#pragma unroll
-  for (int j = 0; j < J; ++j) cs[j] = mid_cols(p.sw, nw + j * 16 + fg * 4, N);
   if constexpr (OUT == MID8_QUANT) {
     // bias + GELU, then e4m3 with a scale per row and 128 columns: the columns of the
     // lane, of its four lane rows, and of the waves beside it through LDS
@@ -142,8 +141,7 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_fp8_kernel(Mid8Args p,
 #pragma unroll
       for (int j = 0; j < J; ++j) {
         const int n = nw + j * 16 + fg * 4;
-        const f32x4 bs = p.bias != nullptr ? mid_cols(p.bias, n, N) : f32x4{0.f, 0.f, 0.f, 0.f};
-        f32x4 v = mid_act<ACT_GELU>(acc[i][j] * cs[j] + bs, f32x2{});
+        f32x4 v = mid_act<ACT_GELU>(acc[i][j] * pre.cs[j] + pre.bs[j], f32x2{});
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           v[r] = n + r < N ? v[r] : 0.f;
@@ -184,9 +182,9 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_fp8_kernel(Mid8Args p,
 #pragma unroll
   for (int i = 0; i < I; ++i)
 #pragma unroll
-    for (int j = 0; j < J; ++j) acc[i][j] *= cs[j];
-  if constexpr (OUT == MID8_SCATTER) mid_scatter<I, J>(acc, mw, nw, M, N, p.bias, lane, scat);
-  else mid_rows<I, J, false>(acc, mw, nw, lane, p);
+    for (int j = 0; j < J; ++j) acc[i][j] *= pre.cs[j];
+  if constexpr (OUT == MID8_SCATTER) mid_scatter<I, J>(acc, mw, nw, M, N, p.bias, pre.bs, lane, scat);
+  else mid_rows<I, J, false>(acc, mw, nw, lane, p, pre);
 }
 
 template <class T, Mid8Out OUT>

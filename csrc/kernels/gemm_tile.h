@@ -208,43 +208,44 @@ __device__ __forceinline__ int qkv_batch(const QkvScatter& sc, int m) {
   b += (b + 1) * sc.T <= m ? 1 : 0;
   return b;
 }
-// the cache position of row m (pos[b] + t), loaded for a lane's 8 rows before
-// the epilogue's first store: loaded per 32-column pair it waited, through the
-// in-order vmcnt, for every store issued before it
-__device__ __forceinline__ int qkv_row_pos(const QkvScatter& sc, int m) {
-  const int b = qkv_batch(sc, m);
-  return sc.pos[b] + (m - b * sc.T);
+// A destination is a part of the row and a part of the 8 columns: element offsets of row
+// m in q (head 0) and, at position pos[b] + t, in the caches; formed for a lane's rows
+// before the epilogue's first store (a position loaded behind one waits for it through
+// the in-order vmcnt), so a store costs one 64-bit addition.
+struct QkvRow {
+  size_t q, kv;
+  bool in;  // false: past the cache capacity, k and v are dropped, as in qkv_split
+};
+__device__ __forceinline__ QkvRow qkv_row(const QkvScatter& sc, int m) {
+  const int b = qkv_batch(sc, m), t = m - b * sc.T, p = sc.pos[b] + t;
+  return QkvRow{((size_t)b * sc.H * sc.T + t) << sc.hd_shift, ((size_t)b * sc.Hkv * sc.S + p) << sc.hd_shift, p < sc.S};
 }
-__device__ __forceinline__ bf16_t* qkv_dest(const QkvScatter& sc, int m, int c, int p) {
-  const int b = qkv_batch(sc, m);
-  const int t = m - b * sc.T;
+struct QkvCol {
+  bf16_t* base;
+  bool q;
+};
+// columns c .. c + 7 (one head)
+__device__ __forceinline__ QkvCol qkv_col(const QkvScatter& sc, int c) {
   const int hs = sc.hd_shift, hmask = (1 << hs) - 1;
   const int qw = sc.H << hs, kw = sc.Hkv << hs;
-  if (c < qw) return sc.q + ((((size_t)b * sc.H + (c >> hs)) * sc.T + t) << hs) + (c & hmask);
-  if (p >= sc.S) return nullptr;  // past the cache capacity: dropped, as in qkv_split
+  if (c < qw) return QkvCol{sc.q + (((size_t)(c >> hs) * sc.T) << hs) + (c & hmask), true};
   const bool isk = c < qw + kw;
   const int cc = isk ? c - qw : c - qw - kw;
-  return (isk ? sc.k : sc.v) + ((((size_t)b * sc.Hkv + (cc >> hs)) * sc.S + p) << hs) + (cc & hmask);
+  return QkvCol{(isk ? sc.k : sc.v) + (((size_t)(cc >> hs) * sc.S) << hs) + (cc & hmask), false};
 }
+// the column of the 8 that lane row q = lane >> 4 stores of the pair from nb on (epi_pair_bf16)
+__device__ __forceinline__ int pair_col(int nb, int lane) { return nb + (((lane >> 4) & 1) << 4) + ((lane >> 5) << 3); }
 
 // One widened 16-B store per lane (as epi_pair_bf16) of a whole 32-column pair
-// to its head-major / cache destination (bias added first, no activation).
-__device__ __forceinline__ void epi_pair_scatter(f32x4 a0, f32x4 a1, int m, int nb, int M,
-                                                 const float* __restrict__ bias, int lane, const QkvScatter& sc,
-                                                 int p) {
-  const int q = lane >> 4;
-  if (bias != nullptr) {
-    a0 += *reinterpret_cast<const f32x4*>(bias + nb + q * 4);
-    a1 += *reinterpret_cast<const f32x4*>(bias + nb + 16 + q * 4);
-  }
+// to its head-major / cache destination.
+__device__ __forceinline__ void epi_pair_scatter(const f32x4& a0, const f32x4& a1, int m, int M, const QkvRow& row,
+                                                 const QkvCol& col) {
   const uint32_t x0 = pack2bf(a0[0], a0[1]), x1 = pack2bf(a0[2], a0[3]);
   const uint32_t y0 = pack2bf(a1[0], a1[1]), y1 = pack2bf(a1[2], a1[3]);
   const auto s0 = __builtin_amdgcn_permlane16_swap(x0, y0, false, false);
   const auto s1 = __builtin_amdgcn_permlane16_swap(x1, y1, false, false);
-  if (m < M) {
-    bf16_t* d = qkv_dest(sc, m, nb + ((q & 1) << 4) + ((q >> 1) << 3), p);
-    if (d != nullptr) *reinterpret_cast<uint4*>(d) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
-  }
+  if (m < M && (col.q || row.in))
+    *reinterpret_cast<uint4*>(col.base + (col.q ? row.q : row.kv)) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
 }
 
 // NQ = 2: 256x256 tiles (4 phases per K-tile, below).  NQ = 1: 256x128 tiles
@@ -495,13 +496,30 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_256_kernel(
       }
   }
   const float* bias_e = badd ? nullptr : bias;
-  // SCATTER: the cache positions of the lane's 8 rows, loaded before any store (qkv_row_pos)
-  int spos[2][4] = {};
+  // SCATTER: the destinations' parts (qkv_row), before any store; bias that is not in LDS
+  QkvRow srow[2][4];
+  QkvCol scol[NQ];
   if constexpr (SCATTER) {
 #pragma unroll
     for (int mq = 0; mq < 2; ++mq)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) spos[mq][i] = qkv_row_pos(scat, min(m0 + mq * 128 + arow + i * 16 + (lane & 15), M - 1));
+      for (int i = 0; i < 4; ++i) srow[mq][i] = qkv_row(scat, min(m0 + mq * 128 + arow + i * 16 + (lane & 15), M - 1));
+#pragma unroll
+    for (int nq = 0; nq < NQ; ++nq) scol[nq] = qkv_col(scat, pair_col(n0 + nq * 128 + wc * 32 + scat.c_off, lane));
+    if (bias_e != nullptr) {
+#pragma unroll
+      for (int nq = 0; nq < NQ; ++nq) {
+        if (n0 + nq * 128 + wc * 32 >= N) continue;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const f32x4 b4 = *reinterpret_cast<const f32x4*>(bias_e + scat.c_off + n0 + nq * 128 + wc * 32 + j * 16 + (lane >> 4) * 4);
+#pragma unroll
+          for (int mq = 0; mq < 2; ++mq)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[mq][nq][i][j] += b4;
+        }
+      }
+    }
   }
   const bool vec = epi_vec_ok(Cv, ldc, bias, R, ldr);
   const bool pair = vec && epi_pair_ok(Cv, ldc, bias, R, ldr);
@@ -569,9 +587,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_256_kernel(
           // destination of the lane's 8 columns (host: ACT_NONE, bf16 out, no
           // residual, N % 32 == 0, hd % 8 == 0 -> a 32-column pair is whole or
           // past N, wave-uniformly)
-          if (nb < N)
-            epi_pair_scatter(acc[mq][nq][i][0], acc[mq][nq][i][1], m, nb + scat.c_off, M, bias_e, lane, scat,
-                             spos[mq][i]);
+          if (nb < N) epi_pair_scatter(acc[mq][nq][i][0], acc[mq][nq][i][1], m, M, srow[mq][i], scol[nq]);
         } else if (!OUT_F32 && pair && nb + 31 < N) {
           epi_pair_bf16<ACT>(acc[mq][nq][i][0], acc[mq][nq][i][1], m, nb, (gan & 8) ? 0 : M, reinterpret_cast<bf16_t*>(Cv), ldc,
                              bias_e, R, ldr, lane, {}, {}, xc);
