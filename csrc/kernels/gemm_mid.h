@@ -10,10 +10,12 @@
 
 namespace dnn {
 
-template <int BM_, int BN_, int WM_, int WN_, int S_>
+template <int BM_, int BN_, int WM_, int WN_, int S_, int PW_ = 0>
 struct MidTile {
-  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, S = S_;
-  static constexpr int NW = WM * WN;                           // waves
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, S = S_, PW = PW_;
+  static constexpr int CW = WM * WN;                           // waves that multiply
+  static constexpr int NW = PW ? PW : CW;                      // waves that stage: PW > 0, others than those
+  static constexpr int THREADS = (CW + PW) * 64;
   static constexpr int I = BM / WM / 16, J = BN / WN / 16;      // 16 x 16 tiles of a wave
   static constexpr int PA = BM / 8 / NW, PB = BN / 8 / NW;      // 1-KiB pieces a wave stages of either operand
   static constexpr int STAGE = (BM + BN) * 128;                 // bytes of one K-tile of both operands
@@ -26,6 +28,22 @@ typedef MidTile<128, 64, 2, 2, 6> Mid1;
 typedef MidTile<128, 128, 2, 4, 4> Mid2;
 typedef MidTile<256, 128, 4, 2, 3> Mid3;
 typedef MidTile<128, 256, 2, 4, 3> Mid4;
+// The same where K is split: four waves that only stage (mid_stage), so that no product
+// waits for a request to be taken.  us with and without, parts and their sum: 512 x 4096 x
+// 18432 in 4 77.8 : 83.8, 500 x 4096 x 21504 in 4 89.4 : 94.0, 700 x 4096 x 14336 in 2 97.6 :
+// 101.9.  Smaller tiles gain nothing, and whole ones lack the registers for their epilogue.
+template <class T>
+struct MidSplit {
+  typedef T type;
+};
+template <>
+struct MidSplit<Mid3> {
+  typedef MidTile<256, 128, 4, 2, 3, 4> type;
+};
+template <>
+struct MidSplit<Mid4> {
+  typedef MidTile<128, 256, 2, 4, 3, 4> type;
+};
 
 // s_waitcnt operand: at most `vm` vector-memory and `lgkm` LDS operations outstanding
 constexpr int wait_imm(int vm, int lgkm) { return (vm & 15) | (vm >> 4) << 14 | 7 << 4 | lgkm << 8; }
@@ -261,8 +279,11 @@ __device__ __forceinline__ void mid_rows(f32x4 (&acc)[I][J], int mw, int nw, int
 // take 0.22 and its LDS traffic 0.33; larger tiles need fewer bytes per product but
 // more splits.  Touching later lines from a wave of its own, waves of 64 x 32 in
 // place of 64 x 64, or padded rows did not change that.
+//
+// T::PW > 0: other waves stage, and `src` only says where (mid_stage keeps the same barriers).
 template <class T>
 __device__ __forceinline__ void mid_loop(const MidSource<T>& src, int wm, int wn, int lane, f32x4 (&acc)[T::I][T::J]) {
+  constexpr bool OWN = T::PW == 0;
   constexpr int I = T::I, J = T::J, S = T::S, L = T::PA + T::PB;
   // fragment reads: lane (r, g) reads 16 B of row r at chunks g and 4 + g
   const int fr = lane & 15, fg = lane >> 4;
@@ -291,9 +312,11 @@ __device__ __forceinline__ void mid_loop(const MidSource<T>& src, int wm, int wn
   };
   constexpr auto h0 = std::integral_constant<int, 0>{};
   constexpr auto h1 = std::integral_constant<int, 1>{};
+  if constexpr (OWN) {
 #pragma unroll
-  for (int q = 0; q < S - 1; ++q) src.stage(q, q, 0, 1);
-  __builtin_amdgcn_s_waitcnt(wait_imm((S - 2) * L, 0));
+    for (int q = 0; q < S - 1; ++q) src.stage(q, q, 0, 1);
+    __builtin_amdgcn_s_waitcnt(wait_imm((S - 2) * L, 0));
+  }
   bg_barrier();
   read(h0, 0);
   int cur = 0;
@@ -305,10 +328,11 @@ __device__ __forceinline__ void mid_loop(const MidSource<T>& src, int wm, int wn
       mma(h0, i);
       __builtin_amdgcn_sched_barrier(0);
       if (i == 0) read(h1, cur);
-      src.stage(t + S - 1, prev, i, I);
+      if constexpr (OWN) src.stage(t + S - 1, prev, i, I);
       __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_s_waitcnt(wait_imm((S - 2) * L, 0));  // tile t + 1 landed, tile t read
+    if constexpr (OWN) __builtin_amdgcn_s_waitcnt(wait_imm((S - 2) * L, 0));  // tile t + 1 landed, tile t read
+    else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                   // tile t read
     bg_barrier();
 #pragma unroll
     for (int i = 0; i < I; ++i) {
@@ -323,11 +347,31 @@ __device__ __forceinline__ void mid_loop(const MidSource<T>& src, int wm, int wn
   __builtin_amdgcn_s_waitcnt(wait_imm(0, 0));
 }
 
+// The waves that only stage: tile t + S - 1 goes to the buffer that tile t - 1 left at the
+// barrier before, tile t + 1 has landed at the next one; as many barriers as mid_loop.
+template <class T>
+__device__ __forceinline__ void mid_stage(const MidSource<T>& src) {
+  constexpr int S = T::S, L = T::PA + T::PB;
+#pragma unroll
+  for (int q = 0; q < S - 1; ++q) src.stage(q, q, 0, 1);
+  __builtin_amdgcn_s_waitcnt(wait_imm((S - 2) * L, 0));
+  bg_barrier();
+  int prev = S - 1;
+  for (int t = 0; t < src.nk; ++t) {
+    src.stage(t + S - 1, prev, 0, 1);
+    __builtin_amdgcn_s_waitcnt(wait_imm((S - 2) * L, 0));
+    bg_barrier();
+    prev = prev == S - 1 ? 0 : prev + 1;
+  }
+  __builtin_amdgcn_s_waitcnt(wait_imm(0, 0));
+}
+
 enum MidOut { MID_ROWS = 0, MID_SCATTER = 1, MID_PART = 2 };
 
 template <class T, MidOut OUT>
-__global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvScatter scat) {
+__global__ __launch_bounds__(T::THREADS, 2) void gemm_mid_kernel(MidArgs p, QkvScatter scat) {
   constexpr bool PART = OUT == MID_PART;
+  static_assert(PART || T::PW == 0, "");
   constexpr int I = T::I, J = T::J;
   // S * STAGE bytes, given at launch: with the size in the kernel the compiler sees one
   // wave per SIMD and moves accumulators of the four-wave tiles to AGPRs and back in
@@ -344,7 +388,8 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvS
   int tm, tn;
   tile_coords(id, ntm, ntn, tm, tn);
   const int m0 = tm * T::BM, n0 = tn * T::BN;
-  const int wm = wave / T::WN, wn = wave % T::WN, fr = lane & 15, fg = lane >> 4;
+  const int cw = wave - T::PW;  // < 0: stages
+  const int wm = cw / T::WN, wn = cw % T::WN, fr = lane & 15, fg = lane >> 4;
   int nk = p.K >> 6, k0 = 0;
   if constexpr (PART) {
     k0 = (int)((long long)nk * sp / p.splits);
@@ -353,6 +398,12 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_kernel(MidArgs p, QkvS
   MidSource<T> src;
   src.init(reinterpret_cast<const char*>(p.A), p.lda * 2, m0, M, reinterpret_cast<const char*>(p.W), p.ldw * 2, n0, N, k0,
            nk, smem, wave, lane);
+  if constexpr (T::PW > 0) {
+    if (cw < 0) {
+      mid_stage<T>(src);
+      return;
+    }
+  }
   const int mw = m0 + wm * (I * 16) + fr, nw = n0 + wn * (J * 16);  // the lane's first row, the wave's first column
   MidPre<I, J> pre;
   if constexpr (!PART) pre.load(p, p.rowstat, p.colsum, mw, nw, lane, OUT == MID_ROWS);

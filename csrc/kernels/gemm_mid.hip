@@ -113,7 +113,7 @@ static int start(const MidArgs& a, const QkvScatter& scat, hipStream_t st) {
       hipFuncSetAttribute((const void*)gemm_mid_kernel<T, OUT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   if (room != hipSuccess) return (int)room;
   const int tiles = ((a.M + T::BM - 1) / T::BM) * ((a.N + T::BN - 1) / T::BN);
-  hipLaunchKernelGGL((gemm_mid_kernel<T, OUT>), dim3(tiles * a.splits), dim3(T::NW * 64), LDS, st, a, scat);
+  hipLaunchKernelGGL((gemm_mid_kernel<T, OUT>), dim3(tiles * a.splits), dim3(T::THREADS), LDS, st, a, scat);
   return (int)hipGetLastError();
 }
 
@@ -121,7 +121,7 @@ template <class T>
 static int launch(const MidArgs& a, const QkvScatter* scat, hipStream_t st) {
   if (scat != nullptr) return start<T, MID_SCATTER>(a, *scat, st);
   if (a.splits == 1) return start<T, MID_ROWS>(a, QkvScatter{}, st);
-  if (const int rc = start<T, MID_PART>(a, QkvScatter{}, st)) return rc;
+  if (const int rc = start<typename MidSplit<T>::type, MID_PART>(a, QkvScatter{}, st)) return rc;
   const bool glu = is_glu(a.act);
   const dim3 grid(((glu ? a.N / 2 : a.N) / 4 + 255) / 256, a.M);
   if (glu) hipLaunchKernelGGL((gemm_mid_reduce<1>), grid, dim3(256), 0, st, a);
