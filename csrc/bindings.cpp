@@ -134,10 +134,12 @@ PYBIND11_MODULE(_dnn_hip, m) {
   }, py::arg("a"), py::arg("lda"), py::arg("o"), py::arg("ldo"), py::arg("M"), py::arg("K"), py::arg("st"),
         py::arg("blocked") = 0);
   m.def("cifar_fc1_x3", [](u64 a, int lda, u64 wh, u64 wl, int ldw, u64 bias, u64 c, int ldc, int M, int N, int K,
-                           u64 st, int a_split) {
-    return dnn_cifar_fc1_x3(CFP(a), lda, CP(wh), CP(wl), ldw, CFP(bias), FP(c), ldc, M, N, K, ST(st), a_split);
+                           u64 st, int a_split, int splits, u64 part) {
+    return dnn_cifar_fc1_x3(CFP(a), lda, CP(wh), CP(wl), ldw, CFP(bias), FP(c), ldc, M, N, K, ST(st), a_split, splits,
+                            FP(part));
   }, py::arg("a"), py::arg("lda"), py::arg("wh"), py::arg("wl"), py::arg("ldw"), py::arg("bias"), py::arg("c"),
-        py::arg("ldc"), py::arg("M"), py::arg("N"), py::arg("K"), py::arg("st"), py::arg("a_split") = 0);
+        py::arg("ldc"), py::arg("M"), py::arg("N"), py::arg("K"), py::arg("st"), py::arg("a_split") = 0,
+        py::arg("splits") = 1, py::arg("part") = 0);
   m.def("cifar_split_blocked", [](u64 a, u64 o, int M, int K, int dir, u64 st) {
     return dnn_cifar_split_blocked(CFP(a), FP(o), M, K, dir, ST(st));
   });

@@ -26,10 +26,11 @@
 //  * cifar_fc1_x3_kernel: fc1 + bias + ReLU on the fp32 boundary tensor, the
 //    split done in registers between LDS and the MFMAs (no split copy in HBM):
 //    256x256x32 tiles, 8 waves of 64x128, per k32 step 3 x 32
-//    mfma_f32_16x16x32_bf16 per wave (A_hi W_hi + A_hi W_lo + A_lo W_hi).
+//    mfma_f32_16x16x32_bf16 per wave (A_hi W_hi + A_hi W_lo + A_lo W_hi); K in
+//    ranges where the tiles do not fill the chip, summed by cifar_fc1_sum_kernel.
 //  * cifar_split3_kernel: fp32 (B,K) -> bf16 (B,3K) = [hi | hi | lo], the A
-//    operand of the mid-batch fc1 (one bf16 GEMM over K' = 3K against
-//    W' = [W_hi | W_lo | W_hi]) when the 256^2 tiles cannot fill the chip.
+//    operand of fc1 into strided or typed outputs (one bf16 GEMM over K' = 3K
+//    against W' = [W_hi | W_lo | W_hi]).
 //  * cifar_stage0_x3_band_kernel, cifar_fc1_few_kernel, cifar_head_few_kernel: the
 //    same stages where the batch is too small to fill the chip with whole images.
 //  * cifar_head_tail_x3_kernel: fc2 (512->10) + bias + softmax + per-row argmax
@@ -500,6 +501,8 @@ __global__ __launch_bounds__(512, 1) void cifar_stage0_x3_band_kernel(
 // SPLIT_IN: A arrives pre-split in the blocked boundary encoding (see
 // cifar_split_blocked_kernel: per row and 32-k block, 32 bf16 hi then 32 bf16
 // lo, the same 128 bytes), and nothing is split here.
+//
+// splits > 1: K in that many ranges over the workgroups, whose sums are left in `part` [splits][M][N].
 // ---------------------------------------------------------------------------
 constexpr int F1_T = 256, F1_K = 32;
 
@@ -538,15 +541,17 @@ __global__ __launch_bounds__(512, 1) void cifar_fc1_x3_kernel(const float* __res
                                                               const bf16_t* __restrict__ Wh,
                                                               const bf16_t* __restrict__ Wl, int ldw,
                                                               const float* __restrict__ bias, float* __restrict__ C,
-                                                              int ldc, int M, int N, int K) {
+                                                              int ldc, int M, int N, int K, int splits,
+                                                              float* __restrict__ part) {
   __shared__ __attribute__((aligned(1024))) char smem[8 * BG_HALF];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ntn = N / F1_T, ntm = (M + F1_T - 1) / F1_T;
   int tm, tn;
-  f1_tile_coords(xcd_remap(blockIdx.x, ntm * ntn), ntm, ntn, tm, tn);
+  const int id = xcd_remap(blockIdx.x, ntm * ntn * splits), sp = id / (ntm * ntn);
+  f1_tile_coords(id - sp * ntm * ntn, ntm, ntn, tm, tn);
   const int m0 = tm * F1_T, n0 = tn * F1_T;
   const int wr = wave & 3, wc = wave >> 2, fr = lane & 15, fg = lane >> 4;
-  const int nk = K / F1_K;
+  const int nkall = K / F1_K, k0 = nkall * sp / splits, nk = nkall * (sp + 1) / splits - k0;  // host: splits <= nkall
   auto half = [&](int u, int h) { return smem + (u * 4 + h) * BG_HALF; };  // h: A0, A1, B0, B1
 
   // A: pieces of 8 rows of 128 bytes, 2 of either half a wave: uniform row bases, the
@@ -557,7 +562,7 @@ __global__ __launch_bounds__(512, 1) void cifar_fc1_x3_kernel(const float* __res
 #pragma unroll
   for (int x = 0; x < 4; ++x) {
     const int r = min(m0 + (x >> 1) * 128 + ((x & 1) * 8 + wave) * 8, M - 1);
-    abase[x] = reinterpret_cast<const char*>(A) + (size_t)r * ldb;
+    abase[x] = reinterpret_cast<const char*>(A) + (size_t)r * ldb + (size_t)k0 * 128;
     alim[x] = (uint32_t)min(7, M - 1 - r) * ldb;
   }
   const int slot = (lane & 7) ^ ((wave & 1) * 4 + (lane >> 4));  // swz_chunk of the lane's row in its piece
@@ -575,7 +580,7 @@ __global__ __launch_bounds__(512, 1) void cifar_fc1_x3_kernel(const float* __res
   const char* wbase[2];
 #pragma unroll
   for (int p = 0; p < 2; ++p)
-    wbase[p] = reinterpret_cast<const char*>(p ? Wl : Wh) + (size_t)(n0 + wave * 16) * ldw * 2;
+    wbase[p] = reinterpret_cast<const char*>(p ? Wl : Wh) + (size_t)(n0 + wave * 16) * ldw * 2 + (size_t)k0 * 64;
   const uint32_t woff = (uint32_t)(lane >> 2) * (uint32_t)ldw * 2u + (uint32_t)((lane & 3) ^ f1_swz(lane >> 2)) * 16u;
   auto stB = [&](int u, int h, int t) {
     t = t < nk ? t : nk - 1;
@@ -684,6 +689,23 @@ __global__ __launch_bounds__(512, 1) void cifar_fc1_x3_kernel(const float* __res
   if (wc == 0) bg_barrier();
 
   // epilogue (transposed accumulators): row m0 + mq 128 + wr 32 + i 16 + (lane & 15), cols n..n+3
+  if (splits > 1) {  // this range's sums: cifar_fc1_sum_kernel finishes
+    float* d = part + (size_t)sp * M * N;
+#pragma unroll
+    for (int mq = 0; mq < 2; ++mq)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int m = m0 + mq * 128 + arow + i * 16;
+        if (m < M) {
+#pragma unroll
+          for (int nq = 0; nq < 2; ++nq)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              *reinterpret_cast<f32x4*>(d + (size_t)m * N + n0 + nq * 128 + wc * 64 + j * 16 + fg * 4) = acc[mq][nq][i][j];
+        }
+      }
+    return;
+  }
   const bool vec = epi_vec_ok(C, ldc, bias, nullptr, 0);
 #pragma unroll
   for (int mq = 0; mq < 2; ++mq)
@@ -697,6 +719,21 @@ __global__ __launch_bounds__(512, 1) void cifar_fc1_x3_kernel(const float* __res
           epi_t4<ACT_RELU, true>(acc[mq][nq][i][j], m, n0 + nq * 128 + wc * 64 + j * 16 + fg * 4, M, N, C, ldc, bias,
                                  nullptr, 0, vec);
     }
+}
+
+// relu(sum of the parts + bias), 4 columns a thread; bound by reading the parts.
+__global__ __launch_bounds__(256) void cifar_fc1_sum_kernel(const float* __restrict__ part, const float* __restrict__ bias,
+                                                            float* __restrict__ C, int ldc, int M, int N, int splits) {
+  const int n4 = N / 4, e = blockIdx.x * 256 + threadIdx.x, m = e / n4, n = (e - m * n4) * 4;
+  if (m >= M) return;
+  const float* d = part + (size_t)m * N + n;
+  f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = 0; s < splits; ++s) v += *reinterpret_cast<const f32x4*>(d + (size_t)s * M * N);
+  v += *reinterpret_cast<const f32x4*>(bias + n);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.f);
+  *reinterpret_cast<f32x4*>(C + (size_t)m * ldc + n) = v;
 }
 
 // Blocked boundary encoding of an fp32 (M,K) tensor, in place of the same
@@ -1031,17 +1068,25 @@ extern "C" int dnn_cifar_stage0_x3(const float* x, float* out, const void* w1h, 
 }
 
 extern "C" int dnn_cifar_fc1_x3(const float* A, int lda, const void* Wh, const void* Wl, int ldw, const float* bias,
-                                float* C, int ldc, int M, int N, int K, hipStream_t st, int a_split) {
+                                float* C, int ldc, int M, int N, int K, hipStream_t st, int a_split, int splits,
+                                float* part) {
   if (M <= 0) return 0;
+  if (splits < 1 || splits > K / F1_K || (splits > 1 && part == nullptr)) return -1;
+  // the sum takes 16 bytes at a time, and 32-bit indices
+  if (splits > 1 && ((((uintptr_t)C | (uintptr_t)bias | (uintptr_t)part) & 15) != 0 || M > 1 << 22)) splits = 1;
   if (N % F1_T != 0 || K % F1_K != 0 || lda % 4 != 0 || ldw % 8 != 0 || ldc % 4 != 0) return -1;
   if (lda >= 1 << 27 || ldw >= 1 << 27) return -1;  // 8 rows of A and 16 of W are addressed with 32 bits
-  const int blocks = ((M + F1_T - 1) / F1_T) * (N / F1_T);
+  const int blocks = ((M + F1_T - 1) / F1_T) * (N / F1_T) * splits;
   if (a_split)
     hipLaunchKernelGGL(cifar_fc1_x3_kernel<true>, dim3(blocks), dim3(512), 0, st, A, lda, (const bf16_t*)Wh,
-                       (const bf16_t*)Wl, ldw, bias, C, ldc, M, N, K);
+                       (const bf16_t*)Wl, ldw, bias, C, ldc, M, N, K, splits, part);
   else
     hipLaunchKernelGGL(cifar_fc1_x3_kernel<false>, dim3(blocks), dim3(512), 0, st, A, lda, (const bf16_t*)Wh,
-                       (const bf16_t*)Wl, ldw, bias, C, ldc, M, N, K);
+                       (const bf16_t*)Wl, ldw, bias, C, ldc, M, N, K, splits, part);
+  if (const hipError_t e = hipGetLastError()) return (int)e;
+  if (splits > 1)
+    hipLaunchKernelGGL(cifar_fc1_sum_kernel, dim3(((long)M * (N / 4) + 255) / 256), dim3(256), 0, st, part, bias, C, ldc, M, N,
+                       splits);
   return (int)hipGetLastError();
 }
 

@@ -8,9 +8,9 @@ fp32 modules to the device):
   MFMAs (hi*hi + hi*lo + lo*hi) accumulated in fp32.  Stage boundary tensor
   ``(B,4096)`` fp32 exactly as the reference ships it (``node.py:45-48``).
   fc1 at large batch is ``cifar_fc1_x3``: the fp32 boundary rows come to LDS as they
-  are and are split in registers on their way to the MFMAs (no split copy); at small
-  batch (too few 256-row tiles to fill the chip) it runs as ONE skinny/128^2
-  bf16 GEMM over K' = 3*4096 on ``[A_hi | A_hi | A_lo]`` x ``[W_hi | W_lo | W_hi]``.
+  are and are split in registers on their way to the MFMAs (no split copy), K in ranges over
+  the workgroups where its 256-row tiles would not fill the chip; a strided or typed
+  output is ONE bf16 GEMM over K' = 3*4096 on ``[A_hi | A_hi | A_lo]`` x ``[W_hi | W_lo | W_hi]``.
   Optional boundary encoding ``boundary="split"`` (fp32 only, both ends of
   the hop must be these kernels): the same 16 KiB/img, each row as 32-k blocks
   of 32 bf16 hi then 32 bf16 lo — the very hi/lo operands the x3 MFMAs consume
@@ -32,6 +32,8 @@ The flatten order is the reference's NCHW ``c*64 + h*8 + w`` (``cifar_model_part
 """
 from __future__ import annotations
 
+import functools
+import math
 from dataclasses import dataclass
 from typing import Dict, Optional, Tuple
 
@@ -83,8 +85,8 @@ class CifarStage0Weights:
 @dataclass
 class CifarHeadWeights:
     precision: str
-    w_fc1: torch.Tensor = None   # bf16: [512][4096]; fp32: [512][3*4096] = [hi | lo | hi] (small batch)
-    w_fc1h: torch.Tensor = None  # fp32 path, large batch: W hi / lo [512][4096] each (cifar_fc1_x3)
+    w_fc1: torch.Tensor = None   # bf16: [512][4096]; fp32: [512][3*4096] = [hi | lo | hi] (strided outputs)
+    w_fc1h: torch.Tensor = None  # fp32 path: W hi / lo [512][4096] each (cifar_fc1_x3)
     w_fc1l: torch.Tensor = None
     b_fc1: torch.Tensor = None
     w_fc2: torch.Tensor = None   # bf16: [16][512]
@@ -143,9 +145,9 @@ def act_dtype(precision: str) -> torch.dtype:
 
 
 STAGE0_GRID = 0  # persistent stage-0 workgroups; 0 = one per CU (256)
-# fused fp32 fc1 from this batch on: 2 x B/256 tiles of 128 k32 steps each, one round up to
-# 32768 rows whatever the batch.  us, split3 and the K-concat GEMM : fused: 8192 rows 197 :
-# 237, 9216 251 : 230, 12288 291 : 232, 16384 324 : 235
+# a strided or typed output below this batch is written by the GEMM over [hi | hi | lo] rows;
+# from it on the fused fc1, without a split of K, is the faster one (us, GEMM : fused: 8192
+# rows 197 : 237, 9216 251 : 230, 16384 324 : 235)
 FC1_X3_MIN_ROWS = 8704
 # fp32 head up to this batch: fc1 in slices of K and a finish of one workgroup a row
 # (pipeline pass, us, with and without: 1 row 27.7 / 44.3, 64 29.7 / 57.4, 256 50.6 /
@@ -240,17 +242,45 @@ def _fc1_scratch(scratch: Optional[torch.Tensor], B: int, device) -> torch.Tenso
     return scratch
 
 
+@functools.lru_cache(maxsize=256)
+def _fc1_splits(B: int) -> int:
+    """Ranges of K of the fused fc1, so that its tiles fill one round of 256 CUs: a k-step
+    takes 1.75 us, a workgroup 5 around its steps, the sum of the parts a launch and their way
+    out and in at 4 TB/s.  us, GEMM over [hi | hi | lo] rows : this (whole): 520 rows 46.8 : 38.2
+    (226), 2000 57.4 : 52.7 (228), 4000 92.6 : 66.2 (230), 8192 195 : 97.5 (231), 12288 291 : 149
+    (232), 16384 328 : 176 (252)."""
+    tiles, best, splits = -(-B // 256) * 2, math.inf, 1
+    for s in range(1, 13):  # 12: the parts of a row in the 24 KB of its scratch
+        if s > 1 and tiles * s > 256:
+            break
+        us = -(-tiles * s // 256) * (5 + 1.75 * -(-128 // s)) + (4 + s * B * 4096 / 4e6 if s > 1 else 0)
+        if us < best:
+            best, splits = us, s
+    return splits
+
+
+def fc1_scratch_rows(B: int) -> int:
+    """Rows of 24 KB that ``fc1_forward`` of a batch takes as ``scratch`` (0: none)."""
+    if B < FC1_X3_MIN_ROWS:
+        return B
+    s = _fc1_splits(B)
+    return -(-B * s // 12) if s > 1 else 0
+
+
+def _plain(hid: Optional[torch.Tensor], B: int) -> bool:
+    return hid is None or (tuple(hid.shape) == (B, 512) and hid.dtype == torch.float32 and hid.is_contiguous())
+
+
 def _few_rows(h: torch.Tensor, w: CifarHeadWeights, hid: Optional[torch.Tensor]) -> bool:
     """One row a workgroup of the finish; a strided or typed ``hid`` is the GEMM's."""
     B = h.shape[0]
-    return w.precision == "fp32" and 0 < B <= FC1_FEW_ROWS and (
-        hid is None or (tuple(hid.shape) == (B, 512) and hid.dtype == torch.float32 and hid.is_contiguous()))
+    return w.precision == "fp32" and 0 < B <= FC1_FEW_ROWS and _plain(hid, B)
 
 
 def fc1_forward(h: torch.Tensor, w: CifarHeadWeights, out: Optional[torch.Tensor] = None,
                 scratch: Optional[torch.Tensor] = None, boundary: str = "fp32") -> torch.Tensor:
     """Unit 2: (B,4096) -> relu(fc1) (B,512) on the MFMA GEMM (fp32: split operand,
-    ``scratch`` = (>=B, 12288) bf16 for the [hi | hi | lo] rows; ``boundary``:
+    ``scratch`` = (>= fc1_scratch_rows(B), 12288) bf16 for parts or [hi | hi | lo] rows; ``boundary``:
     the encoding of ``h``)."""
     split = _split_boundary(boundary, w.precision)
     dt = act_dtype(w.precision)
@@ -258,15 +288,17 @@ def fc1_forward(h: torch.Tensor, w: CifarHeadWeights, out: Optional[torch.Tensor
     B = h.shape[0]
     if w.precision == "bf16":
         return linear(h, w.w_fc1, w.b_fc1, act=ACT_RELU, out=out)
-    if B >= FC1_X3_MIN_ROWS:
-        if out is None:
-            out = torch.empty((B, 512), dtype=torch.float32, device=h.device)
-        check(lib().cifar_fc1_x3(ptr(h), 4096, ptr(w.w_fc1h), ptr(w.w_fc1l), 4096, ptr(w.b_fc1), ptr(out), 512,
-                                 B, 512, 4096, stream_ptr(), split), "cifar_fc1_x3")
-        return out
     if _few_rows(h, w, out):
         out = torch.empty((B, 512), dtype=torch.float32, device=h.device) if out is None else out
         _head_few(h, w, out, None, None, scratch, split)
+        return out
+    if B >= FC1_X3_MIN_ROWS or (B > FC1_FEW_ROWS and _plain(out, B)):
+        if out is None:
+            out = torch.empty((B, 512), dtype=torch.float32, device=h.device)
+        s = _fc1_splits(B)
+        part = _fc1_scratch(scratch, -(-B * s // 12), h.device) if s > 1 else None
+        check(lib().cifar_fc1_x3(ptr(h), 4096, ptr(w.w_fc1h), ptr(w.w_fc1l), 4096, ptr(w.b_fc1), ptr(out), 512,
+                                 B, 512, 4096, stream_ptr(), split, s, ptr(part)), "cifar_fc1_x3")
         return out
     a3 = _fc1_scratch(scratch, B, h.device)[:B]
     check(lib().cifar_split3(ptr(h), 4096, ptr(a3), 3 * 4096, B, 4096, stream_ptr(), split), "cifar_split3")

@@ -109,8 +109,9 @@ class CifarHipStage(StageCompute):
             b = {}
             if self.first and self.end >= 2:
                 b["mid"] = torch.empty((batch, 4096), dtype=self.adt, device=d)
-            if self.start <= 2 <= self.end and self.precision == "fp32" and batch < self._cops.FC1_X3_MIN_ROWS:
-                b["split"] = torch.empty((batch, 3 * 4096), dtype=torch.bfloat16, device=d)
+            rows = self._cops.fc1_scratch_rows(batch) if self.start <= 2 <= self.end and self.precision == "fp32" else 0
+            if rows:
+                b["split"] = torch.empty((rows, 3 * 4096), dtype=torch.bfloat16, device=d)
             if self.last:
                 b["hid"] = torch.empty((batch, 512), dtype=self.adt, device=d)
                 b["pred"] = torch.empty((batch,), dtype=torch.int32, device=d)

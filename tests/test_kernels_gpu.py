@@ -392,6 +392,50 @@ def test_cifar_fc1_x3_edges(M, N, K, pad, split_in):
     assert (out[M] == 7).all()
 
 
+@pytest.mark.parametrize("split_in", [0, 1])
+@pytest.mark.parametrize("M,K,splits", [(1, 96, 3), (257, 160, 2), (600, 4096, 12), (1000, 416, 5)])
+def test_cifar_fc1_x3_ranges(M, K, splits, split_in):
+    """K in ranges of unequal and of one k-step, rows past the matrix; parts behind the
+    ones asked for stay as they are.  Bound: test_cifar_fc1_x3_edges."""
+    from distributed_neural_networks_amd.ops import _lib
+    from distributed_neural_networks_amd.ops.cifar import encode_boundary, split_bf16
+    torch.manual_seed(M)
+    N = 256
+    a, w, b = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV), torch.randn(N, device=DEV)
+    wh, wl = split_bf16(w)
+    a_in = encode_boundary(a) if split_in else a
+    out, part = torch.full((M + 1, N), 7.0, device=DEV), torch.full((splits * M * N + 64,), 7.0, device=DEV)
+    rc = _lib.lib().cifar_fc1_x3(a_in.data_ptr(), K, wh.data_ptr(), wl.data_ptr(), K, b.data_ptr(), out.data_ptr(), N, M,
+                                 N, K, torch.cuda.current_stream().cuda_stream, split_in, splits, part.data_ptr())
+    assert rc == 0
+    torch.cuda.synchronize()
+    ref = torch.relu(a.double() @ w.double().t() + b.double())
+    bound = (a.double().abs() @ w.double().abs().t() + b.double().abs()) * 2 ** -14
+    assert ((out[:M].double() - ref).abs() <= bound).all()
+    assert (out[M] == 7).all() and (part[splits * M * N:] == 7).all()
+
+
+@pytest.mark.parametrize("B", [513, 1000, 8700, 9000, 16400])
+def test_cifar_fc1_batches(B):
+    """fc1 on every side of its rules, with the stage's scratch, its own and a strided output."""
+    from distributed_neural_networks_amd.ops import cifar as cops
+    torch.manual_seed(B)
+    w = cops.pack_head({"fc1.weight": torch.randn(512, 4096) / 64, "fc1.bias": torch.randn(512), "fc2.weight": torch.randn(10, 512),
+                        "fc2.bias": torch.randn(10)}, DEV)
+    h = torch.rand(B, 4096, device=DEV)
+    ref = torch.relu(h.double() @ (w.w_fc1h.double() + w.w_fc1l.double()).t() + w.b_fc1.double())
+    rows = cops.fc1_scratch_rows(B)
+    own = torch.empty((rows, 3 * 4096), dtype=torch.bfloat16, device=DEV) if rows else None
+    outs = [cops.fc1_forward(h, w, scratch=own), cops.fc1_forward(h, w)]
+    assert torch.equal(*outs)
+    if B < cops.FC1_X3_MIN_ROWS:
+        wide = torch.zeros(B, 520, device=DEV)
+        outs.append(cops.fc1_forward(h, w, out=wide[:, :512]))
+        assert (wide[:, 512:] == 0).all()
+    for y in outs:
+        assert (y.double() - ref).abs().max().item() <= 2e-5 * ref.abs().max().item()
+
+
 @pytest.mark.parametrize("boundary", ["fp32", "split"])
 @pytest.mark.parametrize("B", [1, 2, 15, 16, 17, 32, 33, 64, 65, 500, 512])
 def test_cifar_few_images(B, boundary):
