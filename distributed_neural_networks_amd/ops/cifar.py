@@ -145,9 +145,9 @@ def act_dtype(precision: str) -> torch.dtype:
 
 
 STAGE0_GRID = 0  # persistent stage-0 workgroups; 0 = one per CU (256)
-# a strided or typed output below this batch is written by the GEMM over [hi | hi | lo] rows;
-# from it on the fused fc1, without a split of K, is the faster one (us, GEMM : fused: 8192
-# rows 197 : 237, 9216 251 : 230, 16384 324 : 235)
+# strided fp32 rows below this batch are written by the GEMM over [hi | hi | lo] rows; from it
+# on the fused fc1, without a split of K, is the faster one (us, GEMM : fused: 8192 rows 197 :
+# 237, 9216 251 : 230, 16384 324 : 235).  Outputs of another type or layout are the GEMM's.
 FC1_X3_MIN_ROWS = 8704
 # fp32 head up to this batch: fc1 in slices of K and a finish of one workgroup a row
 # (pipeline pass, us, with and without: 1 row 27.7 / 44.3, 64 29.7 / 57.4, 256 50.6 /
@@ -271,6 +271,12 @@ def _plain(hid: Optional[torch.Tensor], B: int) -> bool:
     return hid is None or (tuple(hid.shape) == (B, 512) and hid.dtype == torch.float32 and hid.is_contiguous())
 
 
+def _fp32_rows(out: torch.Tensor, B: int) -> bool:
+    """Can the fused fc1 write these rows, at a distance of their own?"""
+    return (tuple(out.shape) == (B, 512) and out.dtype == torch.float32 and out.stride(1) == 1
+            and out.stride(0) >= 512 and out.stride(0) % 4 == 0)
+
+
 def _few_rows(h: torch.Tensor, w: CifarHeadWeights, hid: Optional[torch.Tensor]) -> bool:
     """One row a workgroup of the finish; a strided or typed ``hid`` is the GEMM's."""
     B = h.shape[0]
@@ -292,13 +298,15 @@ def fc1_forward(h: torch.Tensor, w: CifarHeadWeights, out: Optional[torch.Tensor
         out = torch.empty((B, 512), dtype=torch.float32, device=h.device) if out is None else out
         _head_few(h, w, out, None, None, scratch, split)
         return out
-    if B >= FC1_X3_MIN_ROWS or (B > FC1_FEW_ROWS and _plain(out, B)):
+    plain = _plain(out, B)
+    if (plain and B > FC1_FEW_ROWS) or (B >= FC1_X3_MIN_ROWS and _fp32_rows(out, B)):
         if out is None:
             out = torch.empty((B, 512), dtype=torch.float32, device=h.device)
-        s = _fc1_splits(B)
+        s = _fc1_splits(B) if plain else 1
         part = _fc1_scratch(scratch, -(-B * s // 12), h.device) if s > 1 else None
-        check(lib().cifar_fc1_x3(ptr(h), 4096, ptr(w.w_fc1h), ptr(w.w_fc1l), 4096, ptr(w.b_fc1), ptr(out), 512,
-                                 B, 512, 4096, stream_ptr(), split, s, ptr(part)), "cifar_fc1_x3")
+        check(lib().cifar_fc1_x3(ptr(h), 4096, ptr(w.w_fc1h), ptr(w.w_fc1l), 4096, ptr(w.b_fc1), ptr(out),
+                                 512 if plain else out.stride(0), B, 512, 4096, stream_ptr(), split, s, ptr(part)),
+              "cifar_fc1_x3")
         return out
     a3 = _fc1_scratch(scratch, B, h.device)[:B]
     check(lib().cifar_split3(ptr(h), 4096, ptr(a3), 3 * 4096, B, 4096, stream_ptr(), split), "cifar_split3")

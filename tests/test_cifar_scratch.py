@@ -17,3 +17,58 @@ def test_fc1_scratch():
     for dt in (torch.uint8, torch.float16, torch.float32):  # the few-row head keeps 16 KB of partial sums a row in it
         with pytest.raises(TypeError):
             cops._fc1_scratch(torch.empty((3, K3), dtype=dt), 3, cpu)
+
+
+@pytest.fixture
+def fc1_calls(monkeypatch):
+    """fc1_forward on tensors without memory: what it would launch, with the row distance of the output."""
+    calls = []
+
+    class Lib:
+        def cifar_fc1_x3(self, a, lda, wh, wl, ldw, bias, c, ldc, *rest):
+            calls.append(("fused", ldc, rest[5]))
+            return 0
+
+        def cifar_split3(self, *args):
+            return 0
+
+        def cifar_head_few(self, *args):
+            calls.append(("few", 512, 1))
+            return 0
+
+    monkeypatch.setattr(cops, "lib", lambda: Lib())
+    monkeypatch.setattr(cops, "stream_ptr", lambda: 0)
+
+    def linear(x, w, bias, act, out):
+        calls.append(("gemm", out.stride(0), 1))
+        return out
+
+    monkeypatch.setattr(cops, "linear", linear)
+    return calls
+
+
+def _head(device="meta"):
+    bf = dict(dtype=torch.bfloat16, device=device)
+    return cops.CifarHeadWeights("fp32", w_fc1=torch.empty((512, K3), **bf), w_fc1h=torch.empty((512, 4096), **bf),
+                                 w_fc1l=torch.empty((512, 4096), **bf), b_fc1=torch.empty(512, device=device))
+
+
+@pytest.mark.parametrize("B", [1, 512, 513, 8703, 8704, 9000, 16383, 16400, 65536])
+def test_fc1_honours_its_output(B, fc1_calls):
+    """Strided rows keep their distance, another type or layout is the GEMM's, on every side of the rules."""
+    h, w = torch.empty((B, 4096), device="meta"), _head()
+    wide = dict(device="meta")
+    rows = {"plain": torch.empty((B, 512), **wide), "wide": torch.empty((B, 520), **wide)[:, :512],
+            "odd": torch.empty((B, 517), **wide)[:, :512], "typed": torch.empty((B, 512), dtype=torch.bfloat16, **wide),
+            "columns": torch.empty((512, B), **wide).t(), "more": torch.empty((B + 1, 512), **wide)}
+    got = {}
+    for name, out in rows.items():
+        assert cops.fc1_forward(h, w, out=out) is out
+        got[name] = fc1_calls.pop()
+        assert not fc1_calls
+    assert got["plain"][0] == ("few" if B <= 512 else "fused") and got["plain"][1] == 512
+    if B > 1:  # one row has no distance
+        assert got["wide"][:2] == ("fused" if B >= cops.FC1_X3_MIN_ROWS else "gemm", 520)
+        assert got["odd"][:2] == ("gemm", 517) and got["columns"][0] == "gemm"
+    assert got["wide"][2] == 1
+    assert got["typed"][0] == "gemm" and got["more"][0] == "gemm"
