@@ -734,7 +734,7 @@ extern "C" int dnn_gemm_fp8_qkv_scatter(const void* A8, const float* sa, const v
                                         int H, int Hkv, int hd, int S, int Kb, hipStream_t st) {
   const int M = B * T, N = (H + 2 * Hkv) * hd;
   if (Kb % 128 != 0 || M <= 0 || hd % 8 != 0 || sa == nullptr || sw == nullptr) return -1;
-  if (N % 32 != 0 || M < 256 || ((uintptr_t)bias & 15) != 0) return -3;
+  if (N % 32 != 0 || M < 256 || ((uintptr_t)bias & 15) != 0 || !bg_narrow(Kb / 2)) return -3;
   const int tiles = ((M + BG_M - 1) / BG_M) * ((N + BG_N - 1) / BG_N);
   if ((hd & (hd - 1)) != 0 || M >= (1 << 24)) return -3;
   QkvScatter sc{(bf16_t*)q, (bf16_t*)kc, (bf16_t*)vc, pos, T, H, Hkv, __builtin_ctz(hd), S, 1.0f / (float)T};
@@ -758,12 +758,13 @@ extern "C" int dnn_gemm_fp8_qkv_scatter(const void* A8, const float* sa, const v
 
 // fp8 256^2 GEMM (see gemm_fp8_256_kernel); Kb = row bytes of A and W (multiple
 // of 128), sa per-row, sw per-column scales.  Called by dnn_gemm_fp8 when the
-// 256^2 tiles fill the chip.
+// 256^2 tiles fill the chip.  -3: rows too wide for the tiles' 32-bit row offsets.
 extern "C" int dnn_gemm_fp8_256(const void* A, const float* sa, const void* W, const float* sw, void* C, int ldc,
                                 const float* bias, const void* R, int ldr, int M, int N, int Kb, int act,
                                 hipStream_t st) {
   if (Kb % 128 != 0 || M <= 0 || N <= 0 || sa == nullptr || sw == nullptr) return -1;
   if (is_glu(act) && N % 16 != 0) return -1;
+  if (!bg_narrow(Kb / 2)) return -3;
   const int tiles = ((M + BG_M - 1) / BG_M) * ((N + BG_N - 1) / BG_N);
   // tail split (as launch_gemm's): GPT-2 XL O / c_proj (N = 1600) and c_fc (N = 6400) at M = 32768
   const int Na = !is_glu(act) ? tail_split_cols(M, N, true) : 0;
@@ -808,7 +809,7 @@ extern "C" int dnn_gemm_fp8_mx(const void* A8, const void* sx, const void* W8, c
                                const float* bias, const void* R, int ldr, int M, int N, int Kb, int act, void* qo,
                                int ldq, void* sxo, int kpo, hipStream_t st) {
   if (Kb % 128 != 0 || M <= 0 || N <= 0 || sx == nullptr || sw == nullptr) return -1;
-  if (M < 256 || N < 256) return -3;
+  if (M < 256 || N < 256 || !bg_narrow(Kb / 2)) return -3;
   if (qo != nullptr && (act != ACT_GELU || sxo == nullptr || kpo % 128 != 0 || kpo < N || ldq < kpo ||
                         (ldq & 7) != 0 || ((uintptr_t)qo & 7) != 0))
     return -1;
@@ -846,7 +847,7 @@ extern "C" int dnn_gemm_fp8_qkv_scatter_mx(const void* A8, const void* sx, const
                                            int H, int Hkv, int hd, int S, int Kb, hipStream_t st) {
   const int M = B * T, N = (H + 2 * Hkv) * hd;
   if (Kb % 128 != 0 || M <= 0 || hd % 8 != 0 || sx == nullptr || sw == nullptr) return -1;
-  if (N % 32 != 0 || M < 256 || N < 256 || ((uintptr_t)bias & 15) != 0) return -3;
+  if (N % 32 != 0 || M < 256 || N < 256 || ((uintptr_t)bias & 15) != 0 || !bg_narrow(Kb / 2)) return -3;
   if ((hd & (hd - 1)) != 0 || M >= (1 << 24)) return -3;
   QkvScatter sc{(bf16_t*)q, (bf16_t*)kc, (bf16_t*)vc, pos, T, H, Hkv, __builtin_ctz(hd), S, 1.0f / (float)T};
   const int mid = mx_mid_tile(M, N, Kb, false);

@@ -235,8 +235,10 @@ extern "C" int dnn_gemm_fp8(const void* A, const float* sa, const void* W, const
     return (double)t / ((double)w * slots);
   };
   if (g_fp8_tile != 128 && M >= 256 && N >= 256 &&
-      (g_fp8_tile == 256 || 1.4 * fill(tiles256, 256) > fill(tiles, 512)))
-    return dnn_gemm_fp8_256(A, sa, W, sw, C, ldc, bias, R, ldr, M, N, K, act, st);
+      (g_fp8_tile == 256 || 1.4 * fill(tiles256, 256) > fill(tiles, 512))) {
+    const int rc = dnn_gemm_fp8_256(A, sa, W, sw, C, ldc, bias, R, ldr, M, N, K, act, st);
+    if (rc != -3) return rc;  // -3: rows too wide for it
+  }
 #define F8(a)                                                                                                        \
   if (act == a) {                                                                                                    \
     hipLaunchKernelGGL((gemm_fp8_kernel<a>), dim3(tiles), dim3(256), 0, st, (const uint8_t*)A, sa, (const uint8_t*)W, \

@@ -289,6 +289,14 @@ int main() {
   expect_reject(dnn_gemm_skinny_sweep(p, 64, p, 64, nullptr, p, 8, 4, 16, 64, 1, 2, 16, 0, 0, st), "sweep ks>8");
   expect_reject(dnn_gemm_fp8(p, f, p, f, p, 8, nullptr, nullptr, 0, 128, 128, 96, 0, st), "fp8 K%128");
   expect_reject(dnn_gemm_fp8(p, f, p, f, p, 8, nullptr, nullptr, 0, 128, 24, 128, 3, st), "fp8 silu N%16");
+  const int wide = 1 << 29;  // 7 rows of it are the 32-bit row offsets of the 256 x 256 tiles
+  expect_reject(dnn_gemm_fp8_256(p, f, p, f, p, 256, nullptr, nullptr, 0, 256, 256, wide, 0, st), "fp8 256 x 256 wide rows");
+  expect_reject(dnn_gemm_fp8_mx(p, p, p, f, p, 256, nullptr, nullptr, 0, 256, 256, wide, 0, nullptr, 0, nullptr, 0, st),
+                "MX wide rows");
+  expect_reject(dnn_gemm_fp8_qkv_scatter(p, f, p, f, nullptr, p, p, p, ip, 1, 256, 2, 1, 64, 256, wide, st),
+                "fp8 scatter wide rows");
+  expect_reject(dnn_gemm_fp8_qkv_scatter_mx(p, p, p, f, nullptr, p, p, p, ip, 1, 256, 2, 1, 64, 256, wide, st),
+                "MX scatter wide rows");
   expect_reject(dnn_quant_fp8_rows(p, 12, p, f, 4, 12, 128, st), "quant K%8");
   expect_reject(dnn_quant_fp8_rows(p, 256, p, f, 4, 256, 128, st), "quant kpad<K");
   // norms / embedding
