@@ -1075,6 +1075,7 @@ extern "C" int dnn_cifar_fc1_x3(const float* A, int lda, const void* Wh, const v
   // the sum takes 16 bytes at a time, and 32-bit indices
   if (splits > 1 && ((((uintptr_t)C | (uintptr_t)bias | (uintptr_t)part) & 15) != 0 || M > 1 << 22)) splits = 1;
   if (N % F1_T != 0 || K % F1_K != 0 || lda % 4 != 0 || ldw % 8 != 0 || ldc % 4 != 0) return -1;
+  if ((((uintptr_t)A | (uintptr_t)Wh | (uintptr_t)Wl) & 15) != 0) return -1;  // 16-byte LDS-DMA
   if (lda >= 1 << 27 || ldw >= 1 << 27) return -1;  // 8 rows of A and 16 of W are addressed with 32 bits
   const int blocks = ((M + F1_T - 1) / F1_T) * (N / F1_T) * splits;
   if (a_split)

@@ -30,7 +30,7 @@ static void expect_noop(int rc, const char* what) {
 }
 
 int main() {
-  char buf[64] = {0};
+  alignas(16) char buf[64] = {0};
   void* p = buf;
   float* f = reinterpret_cast<float*>(buf);
   int* ip = reinterpret_cast<int*>(buf);
@@ -325,6 +325,12 @@ int main() {
   expect_reject(dnn_cifar_set_v4_pt(36), "v4 pt>32");
   expect_noop(dnn_cifar_stage0_v4(f, p, p, f, p, f, 0, 0, st), "stage0 B=0");
   expect_noop(dnn_cifar_head_tail(p, p, f, f, ip, 0, st), "head B=0");
+  for (int off = 0; off < 3; ++off) {  // rows or weights that 16-byte LDS-DMA does not fetch
+    char* q[3] = {buf, buf, buf};
+    q[off] += 4;
+    expect_reject(dnn_cifar_fc1_x3(reinterpret_cast<float*>(q[0]), 4096, q[1], q[2], 4096, f, f, 512, 600, 512, 4096, st),
+                  "fc1 operands off 16 bytes");
+  }
   if (g_fail) {
     std::printf("host_validate FAILED (%d)\n", g_fail);
     return 1;

@@ -277,6 +277,11 @@ def _fp32_rows(out: torch.Tensor, B: int) -> bool:
             and out.stride(0) >= 512 and out.stride(0) % 4 == 0)
 
 
+def _dma_rows(h: torch.Tensor, w: CifarHeadWeights) -> bool:
+    """The fused fc1 fetches rows and weights by 16-byte LDS-DMA; split3 and the GEMM take any ``h``."""
+    return (ptr(h) | ptr(w.w_fc1h) | ptr(w.w_fc1l)) % 16 == 0
+
+
 def _few_rows(h: torch.Tensor, w: CifarHeadWeights, hid: Optional[torch.Tensor]) -> bool:
     """One row a workgroup of the finish; a strided or typed ``hid`` is the GEMM's."""
     B = h.shape[0]
@@ -299,7 +304,7 @@ def fc1_forward(h: torch.Tensor, w: CifarHeadWeights, out: Optional[torch.Tensor
         _head_few(h, w, out, None, None, scratch, split)
         return out
     plain = _plain(out, B)
-    if (plain and B > FC1_FEW_ROWS) or (B >= FC1_X3_MIN_ROWS and _fp32_rows(out, B)):
+    if ((plain and B > FC1_FEW_ROWS) or (B >= FC1_X3_MIN_ROWS and _fp32_rows(out, B))) and _dma_rows(h, w):
         if out is None:
             out = torch.empty((B, 512), dtype=torch.float32, device=h.device)
         s = _fc1_splits(B) if plain else 1

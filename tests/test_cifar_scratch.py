@@ -72,3 +72,13 @@ def test_fc1_honours_its_output(B, fc1_calls):
         assert got["odd"][:2] == ("gemm", 517) and got["columns"][0] == "gemm"
     assert got["wide"][2] == 1
     assert got["typed"][0] == "gemm" and got["more"][0] == "gemm"
+
+
+@pytest.mark.parametrize("B", [513, 9000, 16400])
+def test_fc1_rows_off_16_bytes(B, fc1_calls, monkeypatch):
+    """Rows or weights that 16-byte LDS-DMA does not fetch are the GEMM's, whose split reads them with plain loads."""
+    h, w = torch.empty((B, 4096), device="meta"), _head()
+    for off in (None, h, w.w_fc1h, w.w_fc1l):
+        monkeypatch.setattr(cops, "ptr", lambda t: 4 if t is not None and t is off else 0)
+        cops.fc1_forward(h, w)
+        assert fc1_calls.pop()[0] == ("fused" if off is None else "gemm")

@@ -442,6 +442,26 @@ def test_cifar_fc1_batches(B):
 
 
 @pytest.mark.parametrize("boundary", ["fp32", "split"])
+@pytest.mark.parametrize("B", [513, 8704])
+def test_cifar_fc1_rows_off_16_bytes(B, boundary):
+    """Boundary rows that start one float behind a 16-byte address, against 64 bits
+    (bound: test_cifar_fc1_x3_edges)."""
+    from distributed_neural_networks_amd.ops import cifar as cops
+    torch.manual_seed(B)
+    w = cops.pack_head({"fc1.weight": torch.randn(512, 4096) / 64, "fc1.bias": torch.randn(512), "fc2.weight": torch.randn(10, 512),
+                        "fc2.bias": torch.randn(10)}, DEV)
+    a = torch.rand(B, 4096, device=DEV)
+    h = torch.empty(B * 4096 + 1, device=DEV)[1:].view(B, 4096)
+    h.copy_(cops.encode_boundary(a) if boundary == "split" else a)
+    assert h.is_contiguous() and h.data_ptr() % 16 == 4
+    y = cops.fc1_forward(h, w, boundary=boundary)
+    W = w.w_fc1h.double() + w.w_fc1l.double()
+    ref = torch.relu(a.double() @ W.t() + w.b_fc1.double())
+    bound = (a.double() @ W.abs().t() + w.b_fc1.double().abs()) * 2 ** -14
+    assert ((y.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("boundary", ["fp32", "split"])
 @pytest.mark.parametrize("B", [1, 2, 15, 16, 17, 32, 33, 64, 65, 500, 512])
 def test_cifar_few_images(B, boundary):
     """Bands of one image against whole images a workgroup (the same bits) and the
