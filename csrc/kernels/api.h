@@ -93,6 +93,7 @@ int dnn_cifar_stage0_x3(const float* x, float* out, const void* w1h, const void*
                         float* keep = nullptr);
 int dnn_cifar_s0_set_wide_store(int on);
 int dnn_cifar_split3(const float* a, int lda, void* o, int ldo, int M, int K, hipStream_t st, int blocked = 0);
+int dnn_cifar_fc1_ranges(int M, int N, int splits, const float* C, const float* bias, const float* part);
 int dnn_cifar_fc1_x3(const float* A, int lda, const void* Wh, const void* Wl, int ldw, const float* bias, float* C,
                      int ldc, int M, int N, int K, hipStream_t st, int a_split = 0, int splits = 1,
                      float* part = nullptr);

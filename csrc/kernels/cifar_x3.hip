@@ -35,6 +35,7 @@
 //    same stages where the batch is too small to fill the chip with whole images.
 //  * cifar_head_tail_x3_kernel: fc2 (512->10) + bias + softmax + per-row argmax
 //    on fp32 hidden rows, 3-term split on mfma_f32_16x16x32_bf16.
+#include <climits>
 #include <type_traits>
 
 #include "gemm_epilogue.h"
@@ -1067,13 +1068,19 @@ extern "C" int dnn_cifar_stage0_x3(const float* x, float* out, const void* w1h, 
                    : launch_stage0_x3<false>(x, out, w1h, w1l, b1, w2h, w2l, b2, keep, B, grid, st);
 }
 
+// The ranges of K that dnn_cifar_fc1_x3 takes of those asked for: cifar_fc1_sum_kernel reads 16
+// bytes at a time and counts quads of columns, whole workgroups of them, with 32 bits.
+extern "C" int dnn_cifar_fc1_ranges(int M, int N, int splits, const float* C, const float* bias, const float* part) {
+  const bool sum = (((uintptr_t)C | (uintptr_t)bias | (uintptr_t)part) & 15) == 0 && (long)M * (N / 4) <= INT_MAX - 255;
+  return sum ? splits : 1;
+}
+
 extern "C" int dnn_cifar_fc1_x3(const float* A, int lda, const void* Wh, const void* Wl, int ldw, const float* bias,
                                 float* C, int ldc, int M, int N, int K, hipStream_t st, int a_split, int splits,
                                 float* part) {
   if (M <= 0) return 0;
   if (splits < 1 || splits > K / F1_K || (splits > 1 && part == nullptr)) return -1;
-  // the sum takes 16 bytes at a time, and 32-bit indices
-  if (splits > 1 && ((((uintptr_t)C | (uintptr_t)bias | (uintptr_t)part) & 15) != 0 || M > 1 << 22)) splits = 1;
+  splits = dnn_cifar_fc1_ranges(M, N, splits, C, bias, part);
   if (N % F1_T != 0 || K % F1_K != 0 || lda % 4 != 0 || ldw % 8 != 0 || ldc % 4 != 0) return -1;
   if ((((uintptr_t)A | (uintptr_t)Wh | (uintptr_t)Wl) & 15) != 0) return -1;  // 16-byte LDS-DMA
   if (lda >= 1 << 27 || ldw >= 1 << 27) return -1;  // 8 rows of A and 16 of W are addressed with 32 bits

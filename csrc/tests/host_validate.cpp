@@ -29,6 +29,13 @@ static void expect_noop(int rc, const char* what) {
   }
 }
 
+static void expect_eq(int got, int want, const char* what) {
+  if (got != want) {
+    std::printf("%s: %d, not %d\n", what, got, want);
+    ++g_fail;
+  }
+}
+
 int main() {
   alignas(16) char buf[64] = {0};
   void* p = buf;
@@ -331,6 +338,10 @@ int main() {
     expect_reject(dnn_cifar_fc1_x3(reinterpret_cast<float*>(q[0]), 4096, q[1], q[2], 4096, f, f, 512, 600, 512, 4096, st),
                   "fc1 operands off 16 bytes");
   }
+  expect_eq(dnn_cifar_fc1_ranges(16384, 512, 2, f, f, f), 2, "fc1 ranges");
+  expect_eq(dnn_cifar_fc1_ranges(1 << 22, 2048, 2, f, f, f), 1, "fc1 ranges of 2^31 quads of columns");
+  expect_eq(dnn_cifar_fc1_ranges(1 << 20, 4096, 2, f, f, f), 2, "fc1 ranges of 2^30 quads of columns");
+  expect_eq(dnn_cifar_fc1_ranges(600, 512, 2, f + 1, f, f), 1, "fc1 ranges into rows off 16 bytes");
   if (g_fail) {
     std::printf("host_validate FAILED (%d)\n", g_fail);
     return 1;
