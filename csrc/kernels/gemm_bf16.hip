@@ -274,28 +274,33 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_256_kernel(
     return;
   }
 
-  // Channel scales and (QOUT, or where the LDS copy is whole) bias of the lane's columns, once:
-  // looked up at every product they put three paths and a wait around each, and the epilogue
-  // of 2048 x 4800 x 1600 took as long as its 13 K-tiles (31.3 us; 26.5 with the scatter's
-  // addresses formed once as well, 2048 x 6400 x 1600 with GELU 39.0 : 37.6).
+  // Channel scales and (QOUT, or where the LDS copy is whole) bias of the lane's columns, held
+  // from here on: looked up at every product they put three paths and a wait around each, and
+  // the epilogue of 2048 x 4800 x 1600 took as long as its 13 K-tiles (31.3 us; 26.5 with the
+  // scatter's addresses formed once as well, 2048 x 6400 x 1600 with GELU 39.0 : 37.6; without
+  // activation 31.4 : 28.5, 8192 rows 108.7 : 99.5).  MX with ReLU looks them up: where it holds
+  // them, the compiler spills operands in every K-tile (2048 x 1600 x 6400 59 : 84).
+  constexpr bool HELD = !(MXA && ACT == ACT_RELU);
   f32x4 cs[NQ][2], bs[NQ][2];
+  if constexpr (HELD) {
 #pragma unroll
-  for (int nq = 0; nq < NQ; ++nq)
+    for (int nq = 0; nq < NQ; ++nq)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int n = n0 + nq * 128 + wc * 32 + j * 16 + (lane >> 4) * 4;
-      bs[nq][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (epv) {  // the LDS copy (columns past N are not stored)
-        cs[nq][j] = *reinterpret_cast<const f32x4*>(epi + EPI_C + 4 * (n - n0));
-        if (bias != nullptr) bs[nq][j] = *reinterpret_cast<const f32x4*>(epi + EPI_B + 4 * (n - n0));
-      } else {
+      for (int j = 0; j < 2; ++j) {
+        const int n = n0 + nq * 128 + wc * 32 + j * 16 + (lane >> 4) * 4;
+        bs[nq][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (epv) {  // the LDS copy (columns past N are not stored)
+          cs[nq][j] = *reinterpret_cast<const f32x4*>(epi + EPI_C + 4 * (n - n0));
+          if (bias != nullptr) bs[nq][j] = *reinterpret_cast<const f32x4*>(epi + EPI_B + 4 * (n - n0));
+        } else {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          cs[nq][j][r] = n + r < N ? sw[n + r] : 0.f;
-          if (QOUT) bs[nq][j][r] = (bias != nullptr && n + r < N) ? bias[n + r] : 0.f;
+          for (int r = 0; r < 4; ++r) {
+            cs[nq][j][r] = n + r < N ? sw[n + r] : 0.f;
+            if (QOUT) bs[nq][j][r] = (bias != nullptr && n + r < N) ? bias[n + r] : 0.f;
+          }
         }
       }
-    }
+  }
   if constexpr (QOUT) {
     // bias + GELU in place, then per (row, 128-column half nq) amax: the lane's
     // 8 columns, the 4 lane rows of the wave (xor 16 / 32), the 4 waves of the
@@ -413,8 +418,22 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_256_kernel(
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
 #pragma clang fp contract(off)  // the product is rounded before the bias, on every path
-          v[j] = acc[mq][nq][i][j] * (cs[nq][j] * rs);
-          if (badd || (SCATTER && bias != nullptr)) v[j] += bs[nq][j];
+          const int n = nb + j * 16 + (lane >> 4) * 4;
+          f32x4 c4;
+          if constexpr (HELD) {
+            c4 = cs[nq][j];
+          } else if (epv) {
+            c4 = *reinterpret_cast<const f32x4*>(epi + EPI_C + 4 * (n - n0));
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) c4[r] = n + r < N ? sw[n + r] : 0.f;
+          }
+          v[j] = acc[mq][nq][i][j] * (c4 * rs);
+          if constexpr (HELD) {
+            if (badd || (SCATTER && bias != nullptr)) v[j] += bs[nq][j];
+          } else {
+            if (badd) v[j] += *reinterpret_cast<const f32x4*>(epi + EPI_B + 4 * (n - n0));
+          }
         }
         if (SCATTER) {
           if (nb < N) epi_pair_scatter(v[0], v[1], m, M, srow[mq][i], scol[nq]);
