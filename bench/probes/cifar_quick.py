@@ -29,8 +29,8 @@ def main():
         x = torch.randn(B, 3, 32, 32, device="cuda")
         mid = torch.empty(B, 4096, dtype=adt, device="cuda")
         hid = torch.empty(B, 512, dtype=adt, device="cuda")
-        spl = (torch.empty(B, 3 * 4096, dtype=torch.bfloat16, device="cuda")
-               if a.precision == "fp32" and B < cops.FC1_X3_MIN_ROWS else None)
+        rows = cops.fc1_scratch_rows(B) if a.precision == "fp32" else 0
+        spl = torch.empty(rows, 3 * 4096, dtype=torch.bfloat16, device="cuda") if rows else None
         probs = torch.empty(B, 10, device="cuda")
         pred = torch.empty(B, dtype=torch.int32, device="cuda")
 

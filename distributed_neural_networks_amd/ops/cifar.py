@@ -260,8 +260,9 @@ def _fc1_splits(B: int) -> int:
 
 
 def fc1_scratch_rows(B: int) -> int:
-    """Rows of 24 KB that ``fc1_forward`` of a batch takes as ``scratch`` (0: none)."""
-    if B < FC1_X3_MIN_ROWS:
+    """Rows of 24 KB that ``fc1_forward`` of a batch into a plain output takes as ``scratch`` (0:
+    none); into another one it takes ``B``, and brings its own where it is given fewer."""
+    if B <= FC1_FEW_ROWS:
         return B
     s = _fc1_splits(B)
     return -(-B * s // 12) if s > 1 else 0
@@ -291,8 +292,8 @@ def _few_rows(h: torch.Tensor, w: CifarHeadWeights, hid: Optional[torch.Tensor])
 def fc1_forward(h: torch.Tensor, w: CifarHeadWeights, out: Optional[torch.Tensor] = None,
                 scratch: Optional[torch.Tensor] = None, boundary: str = "fp32") -> torch.Tensor:
     """Unit 2: (B,4096) -> relu(fc1) (B,512) on the MFMA GEMM (fp32: split operand,
-    ``scratch`` = (>= fc1_scratch_rows(B), 12288) bf16 for parts or [hi | hi | lo] rows; ``boundary``:
-    the encoding of ``h``)."""
+    ``scratch`` = (>= fc1_scratch_rows(B), 12288) bf16 for parts, or (>= B, 12288) for [hi | hi | lo]
+    rows; ``boundary``: the encoding of ``h``)."""
     split = _split_boundary(boundary, w.precision)
     dt = act_dtype(w.precision)
     _check_act(h, (4096,), dt, "fc1 input")

@@ -82,3 +82,19 @@ def test_fc1_rows_off_16_bytes(B, fc1_calls, monkeypatch):
         monkeypatch.setattr(cops, "ptr", lambda t: 4 if t is not None and t is off else 0)
         cops.fc1_forward(h, w)
         assert fc1_calls.pop()[0] == ("fused" if off is None else "gemm")
+
+
+@pytest.mark.parametrize("B", [1, 512, 513, 1000, 4096, 8703, 8704, 16384, 65536])
+def test_fc1_scratch_rows(B, fc1_calls, monkeypatch):
+    """What a stage keeps for its head is what the pass takes: nothing is allocated, and of more than
+    512 rows no more than the parts of the ranges of K."""
+    took = []
+    scratch = cops._fc1_scratch
+    monkeypatch.setattr(cops, "_fc1_scratch", lambda t, rows, dev: took.append((t, rows)) or scratch(t, rows, dev))
+    rows = cops.fc1_scratch_rows(B)
+    own = torch.empty((rows, K3), dtype=torch.bfloat16, device="meta") if rows else None
+    cops.fc1_forward(torch.empty((B, 4096), device="meta"), _head(), scratch=own)
+    assert took == ([(own, rows)] if rows else [])
+    if B > 512:
+        kind, _, splits = fc1_calls.pop()
+        assert kind == "fused" and rows * K3 * 2 < (splits * B * 512 * 4 if splits > 1 else 0) + 2 * K3
