@@ -418,8 +418,8 @@ def test_cifar_fc1_x3_ranges(M, K, splits, split_in):
 @pytest.mark.parametrize("B", [513, 1000, 8700, 9000, 16400])
 def test_cifar_fc1_batches(B):
     """fc1 on every side of its rules, with the stage's scratch and its own, into plain, strided
-    (16 bytes apart and not) and bf16 rows; what lies beside them stays.  A bf16 result is rounded
-    by at most 2^-9 of itself."""
+    (16 bytes apart and not) and bf16 rows; what lies beside them stays.  bf16 has 8 significant
+    bits: a result is rounded by at most 2^-8 of itself."""
     from distributed_neural_networks_amd.ops import cifar as cops
     torch.manual_seed(B)
     w = cops.pack_head({"fc1.weight": torch.randn(512, 4096) / 64, "fc1.bias": torch.randn(512), "fc2.weight": torch.randn(10, 512),
@@ -436,7 +436,7 @@ def test_cifar_fc1_batches(B):
         assert (wide[:, 512:] == 7).all() and (wide[B] == 7).all()
     typed = torch.full((B + 1, 512), 7.0, device=DEV, dtype=torch.bfloat16)
     y = cops.fc1_forward(h, w, out=typed[:B])
-    assert ((y.double() - ref).abs() <= ref * 2 ** -9 + 2e-5 * ref.abs().max()).all() and (typed[B] == 7).all()
+    assert ((y.double() - ref).abs() <= ref * 2 ** -8 + 2e-5 * ref.abs().max()).all() and (typed[B] == 7).all()
     for y in outs:
         assert (y.double() - ref).abs().max().item() <= 2e-5 * ref.abs().max().item()
 
