@@ -10,6 +10,7 @@ from typing import List, Optional, Sequence
 
 import torch
 
+from ..ops._lib import apart
 from ..utils import trace
 from .graph import GraphedStep
 from .stages import StageCompute, StageOutput
@@ -39,11 +40,13 @@ class ColocatedPipeline:
 
     def _reads(self, x: torch.Tensor) -> bool:
         """Can the first stage read ``x`` where it lies?  Its launch then leaves the
-        copy in ``self.x`` that a later call without an input runs on."""
+        copy in ``self.x`` that a later call without an input runs on.  Not what shares
+        memory with a buffer the pass writes, nor a tensor whose values are not the
+        bytes at its address (negated views, zeros without memory)."""
         return (getattr(self.stages[0], "keeps_input", False) and type(x) is torch.Tensor and x.is_cuda
                 and x.device == self.x.device and x.device.index == torch.cuda.current_device() and x.dtype == self.x.dtype
                 and x.shape == self.x.shape and x.is_contiguous() and not x.requires_grad
-                and x.untyped_storage().data_ptr() != self.x.untyped_storage().data_ptr())
+                and not x.is_neg() and not x._is_zerotensor() and all(apart(x, b) for b in (self.x, *self.bufs)))
 
     def __call__(self, x: Optional[torch.Tensor] = None) -> StageOutput:
         # an input read in place: no copy kernel in front (301 of 2718 us at 65536 images),

@@ -214,4 +214,36 @@ def test_colocated_reads_its_input_in_place(batch, captured):
             x.zero_()
         assert torch.equal(pipe().probs, want)
     pipe.x.copy_(xs[3])
-    assert torch.equal(pipe(pipe.x).probs, pipe().probs)  # its own buffer
+    want = pipe().probs.clone()
+    for own in (pipe.x, torch.from_dlpack(pipe.x)):  # its own buffer, also as a storage of another object
+        pipe.bufs[-1].zero_()
+        assert torch.equal(pipe(own).probs, want) and torch.equal(pipe.x, xs[3].to(dev))
+
+
+@pytest.mark.parametrize("batch", [5, 65, 300])
+def test_colocated_copies_what_it_cannot_read(batch):
+    """Images inside a buffer that the pass writes, a negated view and zeros without memory
+    are copied first."""
+    from distributed_neural_networks_amd.models.cifar import NeuralNetwork
+    from distributed_neural_networks_amd.runtime.pipeline import ColocatedPipeline
+    from distributed_neural_networks_amd.runtime.stages import CifarHipStage
+    dev = torch.device("cuda", 0)
+    torch.manual_seed(4)
+    sd = NeuralNetwork().eval().state_dict()
+    stages = [CifarHipStage(sd, 0, 1, dev), CifarHipStage(sd, 2, 3, dev)]
+    pipe = ColocatedPipeline(stages, batch)
+    x = torch.randn(batch, 3, 32, 32, device=dev)
+
+    def copied(t):
+        pipe.x.copy_(t)
+        return pipe().probs.clone()
+
+    want = copied(x)
+    inside = pipe.bufs[0].view(-1)[8:8 + x.numel()].view_as(x)
+    inside.copy_(x)
+    assert not pipe._reads(inside) and torch.equal(pipe(inside).probs, want)
+    for t, values in ((torch._neg_view(x), -x), (torch._efficientzerotensor(x.shape, device=dev), torch.zeros_like(x))):
+        assert not pipe._reads(t)
+        want_t = copied(values)
+        assert torch.equal(pipe(t).probs, want_t) and torch.equal(pipe.x, values)
+    assert pipe._reads(x) and torch.equal(pipe(x).probs, want)
