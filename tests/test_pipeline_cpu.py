@@ -10,3 +10,19 @@ def test_apart():
     for a, b in ((m[:9], m[8:16]), (m, m[8:16]), (m[8:16], m), (m, m), (m, torch.from_dlpack(m))):
         assert not apart(a, b) and not apart(b, a)
     assert apart(m, torch.zeros(64))
+
+
+def test_wrapped_forward_is_given_no_keep():
+    from distributed_neural_networks_amd.models.cifar import NeuralNetwork
+    from distributed_neural_networks_amd.runtime.stages import CifarHipStage
+    sd = NeuralNetwork().state_dict()
+    cpu = torch.device("cpu")
+
+    class Wrapped(CifarHipStage):
+        def forward(self, x, out=None):
+            return super().forward(x, out)
+
+    plain, patched = CifarHipStage(sd, 0, 1, cpu), CifarHipStage(sd, 0, 1, cpu)
+    patched.forward = lambda x, out=None: out
+    assert plain.keeps_input and not Wrapped(sd, 0, 1, cpu).keeps_input and not patched.keeps_input
+    assert not CifarHipStage(sd, 2, 3, cpu).keeps_input and not CifarHipStage(sd, 0, 1, cpu, precision="bf16").keeps_input

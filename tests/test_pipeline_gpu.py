@@ -223,7 +223,7 @@ def test_colocated_reads_its_input_in_place(batch, captured):
 @pytest.mark.parametrize("batch", [5, 65, 300])
 def test_colocated_copies_what_it_cannot_read(batch):
     """Images inside a buffer that the pass writes, a negated view and zeros without memory
-    are copied first."""
+    are copied first; a stage whose forward takes no ``keep`` is given none."""
     from distributed_neural_networks_amd.models.cifar import NeuralNetwork
     from distributed_neural_networks_amd.runtime.pipeline import ColocatedPipeline
     from distributed_neural_networks_amd.runtime.stages import CifarHipStage
@@ -247,3 +247,10 @@ def test_colocated_copies_what_it_cannot_read(batch):
         want_t = copied(values)
         assert torch.equal(pipe(t).probs, want_t) and torch.equal(pipe.x, values)
     assert pipe._reads(x) and torch.equal(pipe(x).probs, want)
+
+    class Wrapped(CifarHipStage):
+        def forward(self, x, out=None):
+            return super().forward(x, out)
+
+    pipe = ColocatedPipeline([Wrapped(sd, 0, 1, dev), stages[1]], batch)
+    assert not pipe._reads(x) and torch.equal(pipe(x).probs, want)
