@@ -12,6 +12,21 @@ def test_apart():
     assert apart(m, torch.zeros(64))
 
 
+def test_input_apart_from_what_the_pass_writes():
+    """One byte of the input buffer or of a stage's output is enough, on either side."""
+    from distributed_neural_networks_amd.runtime.pipeline import ColocatedPipeline
+    from distributed_neural_networks_amd.runtime.stages import TorchStage
+    from distributed_neural_networks_amd.models.cifar import NeuralNetwork
+    sd = NeuralNetwork().state_dict()
+    pipe = ColocatedPipeline([TorchStage("cifar10", sd, 0, 1, True, False), TorchStage("cifar10", sd, 2, 3, False, True)], 2)
+    n = pipe.x.nbytes
+    for b in (pipe.x, *pipe.bufs):
+        at = b.data_ptr()
+        assert not any(pipe._apart(at + d) for d in (0, 1 - n, b.nbytes - 1, (b.nbytes - n) // 2))
+    first, last = (f(b.data_ptr() + (f is max) * b.nbytes for b in (pipe.x, *pipe.bufs)) for f in (min, max))
+    assert pipe._apart(first - n) and pipe._apart(last)
+
+
 def test_wrapped_forward_is_given_no_keep():
     from distributed_neural_networks_amd.models.cifar import NeuralNetwork
     from distributed_neural_networks_amd.runtime.stages import CifarHipStage
