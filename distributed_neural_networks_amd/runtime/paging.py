@@ -172,7 +172,11 @@ def build_batch(entries: Sequence[tuple], table: np.ndarray, groups: Sequence[in
     memory: a copy from pageable memory holds the host until every earlier launch of
     the stream has run, so the device then waits for the next step's first launches
     (Kozusun, nine steps of up to 512 tokens: 4130 us a pass so, 3650 of them kernels).
-    The caching allocator keeps the pinned block until the copy has run."""
+    The caching allocator keeps the pinned block until the copy has run.  Not inside a
+    graph's capture: a replay would copy whatever the block holds by then."""
+    pinned = torch.device(device).type == "cuda"
+    if pinned and torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("a step's batch cannot be captured into a graph: its ids and positions come from the host")
     ids, pos, slots, dec, want, chunks, starts, start, last = [], [], [], [], [], [], [], [], []
     for toks, p0, slot, places in entries:
         n, row = len(toks), len(ids)
@@ -202,7 +206,7 @@ def build_batch(entries: Sequence[tuple], table: np.ndarray, groups: Sequence[in
     for name, a in parts:
         off[name] = total
         total += -(-a.size // 4) * 4  # 16-byte aligned starts
-    host = torch.zeros(total, dtype=torch.int32, pin_memory=torch.device(device).type == "cuda")
+    host = torch.zeros(total, dtype=torch.int32, pin_memory=pinned)
     flat = host.numpy()
     for name, a in parts:
         flat[off[name]:off[name] + a.size] = a

@@ -280,3 +280,15 @@ def test_oracle_gelu():
     z = torch.linspace(-4, 4, 33, dtype=torch.float64)
     assert torch.allclose(O.gelu_tanh(z), torch.nn.functional.gelu(z, approximate="tanh"))
     assert math.isclose(O.rms_norm(torch.full((4,), 2.0, dtype=torch.float64), 0.0)[0].item(), 1.0)
+
+
+def test_batch_is_not_captured(monkeypatch):
+    """A captured copy from pinned memory would read it again at every replay."""
+    from distributed_neural_networks_amd.runtime.paging import PageTable, build_batch
+    table = PageTable(4, 2)
+    entries = [([1, 2], 0, table.admit(), [1])]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    with pytest.raises(RuntimeError, match="captured"):
+        build_batch(entries, table.table, [1], torch.device("cuda"))
+    b = build_batch(entries, table.table, [1], torch.device("cpu"))
+    assert b.ids.tolist() == [1, 2] and b.want_pos.tolist() == [1]
