@@ -29,8 +29,8 @@
 //    mfma_f32_16x16x32_bf16 per wave (A_hi W_hi + A_hi W_lo + A_lo W_hi); K in
 //    ranges where the tiles do not fill the chip, summed by cifar_fc1_sum_kernel.
 //  * cifar_split3_kernel: fp32 (B,K) -> bf16 (B,3K) = [hi | hi | lo], the A
-//    operand of fc1 into strided or typed outputs (one bf16 GEMM over K' = 3K
-//    against W' = [W_hi | W_lo | W_hi]).
+//    operand of fc1 where the kernel above does not write the output or fetch the
+//    rows (one bf16 GEMM over K' = 3K against W' = [W_hi | W_lo | W_hi]).
 //  * cifar_stage0_x3_band_kernel, cifar_fc1_few_kernel, cifar_head_few_kernel: the
 //    same stages where the batch is too small to fill the chip with whole images.
 //  * cifar_head_tail_x3_kernel: fc2 (512->10) + bias + softmax + per-row argmax
@@ -509,16 +509,6 @@ constexpr int F1_T = 256, F1_K = 32;
 
 __device__ __forceinline__ int f1_swz(int r) { return (r >> 2) & 2; }
 
-__device__ __forceinline__ void f1_tile_coords(int logical, int ntm, int ntn, int& tm, int& tn) {
-  // M fastest inside groups of 8 M-tiles: the ntn column tiles of one A panel
-  // run close together on one XCD, so A's second read hits L2 / MALL
-  constexpr int G = 1;
-  const int per = G * ntn, grp = logical / per, first = grp * G;
-  const int gm = min(ntm - first, G), r = logical - grp * per;
-  tm = first + r % gm;
-  tn = r / gm;
-}
-
 // The 24 products of a phase, between barriers: hi.hi, then W_lo A_hi, then W_hi A_lo of
 // every accumulator
 __device__ __forceinline__ void f1_mfma(f32x4 (&acc)[2][4], const bf16x8 (&a)[2][2], const bf16x8 (&b)[4][2]) {
@@ -547,9 +537,10 @@ __global__ __launch_bounds__(512, 1) void cifar_fc1_x3_kernel(const float* __res
   __shared__ __attribute__((aligned(1024))) char smem[8 * BG_HALF];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ntn = N / F1_T, ntm = (M + F1_T - 1) / F1_T;
-  int tm, tn;
-  const int id = xcd_remap(blockIdx.x, ntm * ntn * splits), sp = id / (ntm * ntn);
-  f1_tile_coords(id - sp * ntm * ntn, ntm, ntn, tm, tn);
+  // columns fastest: the tiles of one panel of A run close together on one XCD, and its second
+  // read hits L2 or the last-level cache (panels in groups of 8, rows fastest: no difference)
+  const int id = xcd_remap(blockIdx.x, ntm * ntn * splits), sp = id / (ntm * ntn), tile = id - sp * ntm * ntn;
+  const int tm = tile / ntn, tn = tile - tm * ntn;
   const int m0 = tm * F1_T, n0 = tn * F1_T;
   const int wr = wave & 3, wc = wave >> 2, fr = lane & 15, fg = lane >> 4;
   const int nkall = K / F1_K, k0 = nkall * sp / splits, nk = nkall * (sp + 1) / splits - k0;  // host: splits <= nkall
@@ -776,7 +767,8 @@ __global__ __launch_bounds__(256) void cifar_split_blocked_kernel(const float* _
   }
 }
 
-// fp32 (M,K) -> bf16 (M,3K) rows [hi | hi | lo]; K % 8 == 0, 16-B aligned rows.
+// fp32 (M,K) -> bf16 (M,3K) rows [hi | hi | lo]; K % 8 == 0, plain loads: rows of a may start
+// at any float.
 // blocked = 1: a is in the blocked hi/lo encoding (the split is already done).
 __global__ __launch_bounds__(256) void cifar_split3_kernel(const float* __restrict__ a, int lda,
                                                            bf16_t* __restrict__ o, int ldo, int M, int K,

@@ -6,13 +6,14 @@ namespace dnn {
 
 // Tile table: rows, columns, whether two workgroups share a CU, and the two
 // constants of a tile's time in us: a (launch, first loads, epilogue) and s (a
-// K-tile of 64).  Over 191 shapes (66 to 9419 rows, 768 to 28672 columns, K of 768 to
-// 21504, weights cold) that every tile ran with 1 to 8 splits, 4139 times, the estimate is
-// off by 10 % (rms); what it picks takes 2 % longer than the best measured on average
-// (0.1 % in the median, 25 % at worst: 1022 x 2048 x 7680 52.7 us, 42.2 as 256 x 128 in 4;
-// profiles/gemm_mid_estimate.md).  The last entry is the 256 x 256 kernel (gemm_tile.h).
-// (Measured without the staging waves of MidSplit: split 256 x 128 and 128 x 256 tiles run 6
-// to 10 % faster than estimated.)
+// K-tile of 64).  Over 406 shapes (66 to 9400 rows, 768 to 28672 columns, K of 768 to
+// 21504, weights cold) that every tile ran with 1 to 8 splits, 7564 times, the estimate is
+// off by 10 % (rms); what it picks takes 1.7 % longer than the best measured on average
+// (0.4 % in the median, 17 % at worst: 75 x 6144 x 4096 22.5 us, 19.2 as 128 x 128 in 4;
+// profiles/gemm_mid_estimate.md).  The constants are those of the kernels before the staging
+// waves of MidSplit and the 256 x 256 schedule of gemm_tile.h: split 256 x 128 and 128 x 256
+// tiles run 7 and 6 % faster than estimated, the 256 x 256 kernel (the last entry) 6 %; 12 of the
+// 406 shapes would run over 2 % faster as such a split tile than as picked.
 struct MidCost {
   int bm, bn, pairs;
   float a, s;

@@ -9,8 +9,9 @@ fp32 modules to the device):
   ``(B,4096)`` fp32 exactly as the reference ships it (``node.py:45-48``).
   fc1 at large batch is ``cifar_fc1_x3``: the fp32 boundary rows come to LDS as they
   are and are split in registers on their way to the MFMAs (no split copy), K in ranges over
-  the workgroups where its 256-row tiles would not fill the chip; a strided or typed
-  output is ONE bf16 GEMM over K' = 3*4096 on ``[A_hi | A_hi | A_lo]`` x ``[W_hi | W_lo | W_hi]``.
+  the workgroups where its 256-row tiles would not fill the chip; a typed output, a strided one
+  of fewer rows, or rows off 16 bytes are ONE bf16 GEMM over K' = 3*4096 on ``[A_hi | A_hi | A_lo]``
+  x ``[W_hi | W_lo | W_hi]``.
   Optional boundary encoding ``boundary="split"`` (fp32 only, both ends of
   the hop must be these kernels): the same 16 KiB/img, each row as 32-k blocks
   of 32 bf16 hi then 32 bf16 lo — the very hi/lo operands the x3 MFMAs consume
@@ -85,7 +86,7 @@ class CifarStage0Weights:
 @dataclass
 class CifarHeadWeights:
     precision: str
-    w_fc1: torch.Tensor = None   # bf16: [512][4096]; fp32: [512][3*4096] = [hi | lo | hi] (strided outputs)
+    w_fc1: torch.Tensor = None   # bf16: [512][4096]; fp32: [512][3*4096] = [hi | lo | hi] (typed, strided outputs)
     w_fc1h: torch.Tensor = None  # fp32 path: W hi / lo [512][4096] each (cifar_fc1_x3)
     w_fc1l: torch.Tensor = None
     b_fc1: torch.Tensor = None

@@ -1,7 +1,9 @@
 """Colocated pipeline: every stage on one GPU (the 1-GPU measurement point).
 
-Stage forwards are chained on one stream over preallocated buffers and the
-whole step is captured into one HIP graph.  The multi-rank schedules (GPipe
+Stage forwards are chained on one stream over preallocated buffers.  A step on
+the images in ``ColocatedPipeline.x`` can be captured into one HIP graph (``capture``);
+a step on images that the first stage reads where they lie is launched, captured
+or not.  The multi-rank schedules (GPipe
 stream, CLI request stream, decode ring) live in ``runtime/scheduler.py``.
 """
 from __future__ import annotations
