@@ -121,10 +121,5 @@ def ptr(t) -> int:
     return 0 if t is None else t.data_ptr()
 
 
-def apart(a: torch.Tensor, b: torch.Tensor) -> bool:
-    """Do two contiguous tensors share no byte?"""
-    return a.data_ptr() + a.nbytes <= b.data_ptr() or b.data_ptr() + b.nbytes <= a.data_ptr()
-
-
 def library_path() -> str:
     return os.path.abspath(lib().__file__)

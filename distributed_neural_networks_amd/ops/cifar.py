@@ -40,7 +40,7 @@ from typing import Dict, Optional, Tuple
 
 import torch
 
-from ._lib import apart, check, lib, ptr, stream_ptr
+from ._lib import check, lib, ptr, stream_ptr
 from .gemm import ACT_RELU, linear
 
 PRECISIONS = ("fp32", "bf16")
@@ -213,7 +213,7 @@ def stage0_forward(x: torch.Tensor, w: CifarStage0Weights, out: Optional[torch.T
         if w.precision != "fp32":
             raise ValueError("stage0: keep exists for the fp32 precision only")
         _check_act(keep, (3, 32, 32), torch.float32, "stage0 keep")
-        if keep.shape[0] != B or not apart(keep, x):
+        if keep.shape[0] != B or abs(ptr(keep) - ptr(x)) < x.nbytes:
             raise ValueError("stage0: keep must be as large as x and apart from it")
     if w.precision == "fp32":
         check(lib().cifar_stage0_x3(ptr(x), ptr(out), ptr(w.w1h), ptr(w.w1l), ptr(w.b1), ptr(w.w2h), ptr(w.w2l),

@@ -28,7 +28,8 @@ class ColocatedPipeline:
         for s in self.stages:
             oshp, odt = s.out_spec(batch)
             self.bufs.append(torch.empty(oshp, dtype=odt, device=dev))
-        self._bytes = [b.nbytes for b in (self.x, *self.bufs)]
+        self._in = (self.x.get_device(), dt, self.x.shape)
+        self._writes = [(b.data_ptr(), b.nbytes) for b in (self.x, *self.bufs)]
         self._graph: Optional[GraphedStep] = None
 
     def _step(self, x: Optional[torch.Tensor] = None):
@@ -45,16 +46,16 @@ class ColocatedPipeline:
         copy in ``self.x`` that a later call without an input runs on.  Not what shares
         memory with a buffer the pass writes, nor a tensor whose values are not the
         bytes at its address (negated views, zeros without memory)."""
-        return (getattr(self.stages[0], "keeps_input", False) and type(x) is torch.Tensor and x.is_cuda
-                and x.device == self.x.device and x.device.index == torch.cuda.current_device() and x.dtype == self.x.dtype
-                and x.shape == self.x.shape and x.is_contiguous() and not x.requires_grad
+        return (type(x) is torch.Tensor and x.is_cuda and getattr(self.stages[0], "keeps_input", False)
+                and x.get_device() == self._in[0] == torch.cuda.current_device() and x.dtype == self._in[1]
+                and x.shape == self._in[2] and x.is_contiguous() and not x.requires_grad
                 and not x.is_neg() and not x._is_zerotensor() and self._apart(x.data_ptr()))
 
     def _apart(self, at: int) -> bool:
         """Does an input at this address share no byte with a buffer the pass writes?"""
-        n = self._bytes[0]
-        for b, size in zip((self.x, *self.bufs), self._bytes):
-            if -n < at - b.data_ptr() < size:
+        n = self._writes[0][1]
+        for start, size in self._writes:
+            if -n < at - start < size:
                 return False
         return True
 

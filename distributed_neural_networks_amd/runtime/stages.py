@@ -122,8 +122,8 @@ class CifarHipStage(StageCompute):
     def keeps_input(self) -> bool:
         """``forward(keep=)``: the launch that reads the images can leave a copy of them.  A
         ``forward`` that was replaced or wrapped need not know of it."""
-        return (self.first and self.precision == "fp32"
-                and getattr(self.forward, "__func__", None) is CifarHipStage.forward)
+        return (self.first and self.precision == "fp32" and type(self).forward is CifarHipStage.forward
+                and "forward" not in self.__dict__)
 
     def forward(self, x, out=None, keep=None):
         B = x.shape[0]

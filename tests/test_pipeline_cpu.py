@@ -1,15 +1,6 @@
 """Which inputs the colocated pipeline's first stage may read in place (CPU: the rule alone)."""
+import pytest
 import torch
-
-from distributed_neural_networks_amd.ops._lib import apart
-
-
-def test_apart():
-    m = torch.zeros(64)
-    assert apart(m[:8], m[8:16]) and apart(m[8:16], m[:8])
-    for a, b in ((m[:9], m[8:16]), (m, m[8:16]), (m[8:16], m), (m, m), (m, torch.from_dlpack(m))):
-        assert not apart(a, b) and not apart(b, a)
-    assert apart(m, torch.zeros(64))
 
 
 def test_input_apart_from_what_the_pass_writes():
@@ -25,6 +16,24 @@ def test_input_apart_from_what_the_pass_writes():
         assert not any(pipe._apart(at + d) for d in (0, 1 - n, b.nbytes - 1, (b.nbytes - n) // 2))
     first, last = (f(b.data_ptr() + (f is max) * b.nbytes for b in (pipe.x, *pipe.bufs)) for f in (min, max))
     assert pipe._apart(first - n) and pipe._apart(last)
+
+
+def test_keep_shares_no_byte_with_the_images(monkeypatch):
+    from distributed_neural_networks_amd.models.cifar import NeuralNetwork
+    from distributed_neural_networks_amd.ops import cifar as cops
+    w = cops.pack_stage0(NeuralNetwork().state_dict(), torch.device("cpu"))
+    launched = []
+    monkeypatch.setattr(cops, "lib", lambda: type("L", (), {"cifar_stage0_x3": staticmethod(lambda *a: launched.append(a) or 0)}))
+    monkeypatch.setattr(cops, "stream_ptr", lambda: 0)
+    n = 2 * 3072
+    m = torch.zeros(3 * n)
+    x = m[n:2 * n].view(2, 3, 32, 32)
+    for start in (n, 1, n - 1, n + 1, 2 * n - 1):
+        with pytest.raises(ValueError, match="apart"):
+            cops.stage0_forward(x, w, keep=m[start:start + n].view_as(x))
+    for start in (0, 2 * n):
+        cops.stage0_forward(x, w, keep=m[start:start + n].view_as(x))
+    assert len(launched) == 2
 
 
 def test_wrapped_forward_is_given_no_keep():
