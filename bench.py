@@ -4,9 +4,9 @@
 Metric and configuration: the reference's only measured headline
 (CIFAR-10 2-stage images/s; 3.40-4.15 k img/s on CPU over localhost gRPC).
 Synthetic fp32 images, random-init weights of the reference architecture.
-Precision: the reference's fp32 contract, computed as **fp32 (bf16x3 split
-emulation, ~2^-16 relative per product, fp32 accumulation)**:
-every product is three bf16 MFMA terms (ops/cifar.py); the line reports the
+Precision: the reference's fp32 contract, computed as **fp32 emulated by 3
+products of 16-bit terms (~2^-16 relative per product, fp32 accumulation)**:
+two bf16 terms an operand, two fp16 terms in conv2 (ops/cifar.py); the line reports the
 measured max|dprob| against fp32 torch on 4096 images (outside the timed
 region).  ``--precision bf16`` is the reduced-precision variant (extra keys).
 Every timed step runs the complete forward of both stages (conv stage +
@@ -59,7 +59,7 @@ import torch
 
 BASELINE_IMG_S = 4150.0  # the reference's CIFAR-10 2-stage, best batch (255), CPU gRPC
 METRIC = "images/sec CIFAR-10 2-stage"
-DTYPE_LABEL = {"fp32": "fp32 (bf16x3 split emulation, ~2^-16 per product)", "bf16": "bf16"}
+DTYPE_LABEL = {"fp32": "fp32 (emulated by 3 products of 16-bit terms, ~2^-16 per product)", "bf16": "bf16"}
 CPU_DTYPE_LABEL = "fp32 (torch CPU golden stages over gloo: schedule test, not a measurement)"
 FP8_LABEL = ("fp8-e4m3 weights (W8A16 decode; prefill W8A8 on the scaled fp8 MFMA, e4m3 activations with "
              "MX e8m0 block scales per row x 128 columns), "

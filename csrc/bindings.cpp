@@ -128,6 +128,11 @@ PYBIND11_MODULE(_dnn_hip, m) {
                                ST(st), split_out, FP(keep));
   }, py::arg("x"), py::arg("out"), py::arg("w1h"), py::arg("w1l"), py::arg("b1"), py::arg("w2h"), py::arg("w2l"),
         py::arg("b2"), py::arg("B"), py::arg("grid"), py::arg("st"), py::arg("split_out") = 0, py::arg("keep") = 0);
+  m.def("cifar_stage0_wino", [](u64 x, u64 out, u64 w1h, u64 w1l, u64 b1, u64 w2h, u64 w2l, u64 u2h, u64 u2l, u64 b2,
+                                u64 sc, int B, int grid, u64 st, int split_out, u64 keep) {
+    return dnn_cifar_stage0_wino(CFP(x), FP(out), CP(w1h), CP(w1l), CFP(b1), CP(w2h), CP(w2l), CP(u2h), CP(u2l), CFP(b2),
+                                 CFP(sc), B, grid, ST(st), split_out, FP(keep));
+  });
   m.def("cifar_s0_set_wide_store", [](int on) { return dnn_cifar_s0_set_wide_store(on); });
   m.def("cifar_split3", [](u64 a, int lda, u64 o, int ldo, int M, int K, u64 st, int blocked) {
     return dnn_cifar_split3(CFP(a), lda, P(o), ldo, M, K, ST(st), blocked);

@@ -91,6 +91,9 @@ int dnn_cifar_set_v4_pt(int pt);
 int dnn_cifar_stage0_x3(const float* x, float* out, const void* w1h, const void* w1l, const float* b1, const void* w2h,
                         const void* w2l, const float* b2, int B, int grid, hipStream_t st, int split_out = 0,
                         float* keep = nullptr);
+int dnn_cifar_stage0_wino(const float* x, float* out, const void* w1h, const void* w1l, const float* b1, const void* w2h,
+                          const void* w2l, const void* u2h, const void* u2l, const float* b2, const float* sc, int B, int grid,
+                          hipStream_t st, int split_out, float* keep);
 int dnn_cifar_s0_set_wide_store(int on);
 int dnn_cifar_split3(const float* a, int lda, void* o, int ldo, int M, int K, hipStream_t st, int blocked = 0);
 int dnn_cifar_fc1_ranges(int M, int N, int splits, const float* C, const float* bias, const float* part);

@@ -36,6 +36,7 @@ NO_PACKED_FP32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 PER_FILE_FLAGS = {"cifar_fused.hip": ["-ffast-math"],
                   # fp32-accurate split path: keep IEEE rounding, only drop NaN canonicalisation in fmaxf
                   "cifar_x3.hip": ["-fno-honor-nans"],
+                  "cifar_wino.hip": ["-fno-honor-nans"] + NO_SLP,
                   # flash / decode softmax maxima over MFMA results: no v_max canonicalise
                   # per score (52 -> 17 v_max per GPT-2 flash block); -inf masking is kept
                   "attention.hip": ["-fno-honor-nans"] + NO_SLP,

@@ -5,7 +5,8 @@ fp32 modules to the device):
 
 * ``fp32`` (the reference's precision, default): ``csrc/kernels/cifar_x3.hip``.
   Every fp32 operand is split into bf16 hi + lo and each product is three bf16
-  MFMAs (hi*hi + hi*lo + lo*hi) accumulated in fp32.  Stage boundary tensor
+  MFMAs (hi*hi + hi*lo + lo*hi) accumulated in fp32; from three images a workgroup on conv2 is
+  Winograd's F(2 x 2, 3 x 3) on two fp16 terms (``cifar_wino.hip``).  Stage boundary tensor
   ``(B,4096)`` fp32 exactly as the reference ships it (``node.py:45-48``).
   fc1 at large batch is ``cifar_fc1_x3``: the fp32 boundary rows come to LDS as they
   are and are split in registers on their way to the MFMAs (no split copy), K in ranges over
@@ -64,6 +65,25 @@ def _conv2_k288(sd) -> torch.Tensor:
     return sd["conv2.weight"].float().permute(0, 2, 3, 1).reshape(64, 288)  # (oc, ky, kx, c)
 
 
+def _conv2_winograd(sd) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """U = G g G^T of every conv2 filter, times a power of two per output channel that brings its largest
+    number into [2^9, 2^10), as two fp16 terms [4 i + j][oc][c]; and the inverse scales."""
+    G = torch.tensor([[1, 0, 0], [.5, .5, .5], [.5, -.5, .5], [0, 0, 1]], dtype=torch.float64)
+    u = G @ sd["conv2.weight"].detach().cpu().double() @ G.t()  # (oc, c, i, j)
+    top = torch.nan_to_num(u.abs(), nan=0.0, posinf=0.0).amax((1, 2, 3))
+    k = torch.where(top > 0, 10 - torch.frexp(top).exponent, 0).clamp(-110, 110)
+    u = (u * 2.0 ** k.double()[:, None, None, None]).permute(2, 3, 0, 1).reshape(16, 64, 32)
+    hi = u.half()
+    return hi, (u - hi.double()).half(), (2.0 ** -k.double()).float()
+
+
+def _conv1_bound(sd) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(l1, b): conv1 of an image of magnitudes up to m stays within l1 m + b.  What is not finite does
+    not count: its channel is lost whatever the scale."""
+    w, b = (torch.nan_to_num(sd[f"conv1.{n}"].detach().cpu().double().abs(), nan=0.0, posinf=0.0) for n in ("weight", "bias"))
+    return (w.sum((1, 2, 3)).max() * (1 + 2.0 ** -12)).float(), b.max().float()
+
+
 def _fc2_pad(sd) -> torch.Tensor:
     w = torch.zeros(16, 512)
     w[:10] = sd["fc2.weight"].float()
@@ -81,6 +101,9 @@ class CifarStage0Weights:
     w1l: torch.Tensor = None
     w2h: torch.Tensor = None
     w2l: torch.Tensor = None
+    u2h: torch.Tensor = None   # fp32 path, Winograd's conv2: [16][64][32] fp16, two terms
+    u2l: torch.Tensor = None
+    sc: torch.Tensor = None    # its scales: bound of conv1's weights and biases, 64 inverse scales of u2
 
 
 @dataclass
@@ -113,7 +136,12 @@ def pack_stage0(sd: Dict[str, torch.Tensor], device, precision: str = "fp32") ->
                                   w2=w2.to(device=device, dtype=torch.bfloat16).contiguous())
     (w1h, w1l), (w2h, w2l) = split_bf16(w1), split_bf16(w2)
     dv = lambda t: t.to(device).contiguous()  # noqa: E731
-    return CifarStage0Weights("fp32", b1, b2, w1h=dv(w1h), w1l=dv(w1l), w2h=dv(w2h), w2l=dv(w2l))
+    w = CifarStage0Weights("fp32", b1, b2, w1h=dv(w1h), w1l=dv(w1l), w2h=dv(w2h), w2l=dv(w2l))
+    l1, b = _conv1_bound(sd)
+    if WINO_RANGE * b >= 32 * l1:  # images up to a magnitude of 32 are within the range of one scale
+        u2h, u2l, inv = _conv2_winograd(sd)
+        w.u2h, w.u2l, w.sc = dv(u2h), dv(u2l), dv(torch.cat([torch.stack([l1, b]), inv]))
+    return w
 
 
 def pack_head(sd: Dict[str, torch.Tensor], device, fc1: bool = True, fc2: bool = True,
@@ -146,6 +174,11 @@ def act_dtype(precision: str) -> torch.dtype:
 
 
 STAGE0_GRID = 0  # persistent stage-0 workgroups; 0 = one per CU (256)
+# conv2 by Winograd (cifar_wino.hip) beyond this many images a workgroup (us, direct : this: 256 images 12.9 :
+# 13.6, 512 19.2 : 18.1, 600 23.9 : 22.2, 1000 32.5 : 28.3, 8192 228 : 192, 65536 1796 : 1475).  Up to two images the
+# results are those of the bands of few images, bit by bit.
+WINO_ROUNDS = 2
+WINO_RANGE = 65536  # its fp16 terms hold a range of this much beside conv1's biases; wider images go the direct way there
 # strided fp32 rows below this batch are written by the GEMM over [hi | hi | lo] rows; from it
 # on the fused fc1, without a split of K, is the faster one (us, GEMM : fused: 8192 rows 197 :
 # 237, 9216 251 : 230, 16384 324 : 235).  Outputs of another type or layout are the GEMM's.
@@ -215,7 +248,11 @@ def stage0_forward(x: torch.Tensor, w: CifarStage0Weights, out: Optional[torch.T
         _check_act(keep, (3, 32, 32), torch.float32, "stage0 keep")
         if keep.shape[0] != B or abs(ptr(keep) - ptr(x)) < x.nbytes:
             raise ValueError("stage0: keep must be as large as x and apart from it")
-    if w.precision == "fp32":
+    if w.precision == "fp32" and B > WINO_ROUNDS * (grid or 256) and w.u2h is not None:
+        check(lib().cifar_stage0_wino(ptr(x), ptr(out), ptr(w.w1h), ptr(w.w1l), ptr(w.b1), ptr(w.w2h), ptr(w.w2l),
+                                      ptr(w.u2h), ptr(w.u2l), ptr(w.b2), ptr(w.sc), B, grid, stream_ptr(), split, ptr(keep)),
+              "cifar_stage0_wino")
+    elif w.precision == "fp32":
         check(lib().cifar_stage0_x3(ptr(x), ptr(out), ptr(w.w1h), ptr(w.w1l), ptr(w.b1), ptr(w.w2h), ptr(w.w2l),
                                     ptr(w.b2), B, grid, stream_ptr(), split, ptr(keep)), "cifar_stage0_x3")
     else:

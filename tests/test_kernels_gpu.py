@@ -494,6 +494,81 @@ def test_cifar_few_images(B, boundary):
     assert torch.equal(pred.long(), probs.argmax(1))
 
 
+def _stage0_in_64_bits(sd, x):
+    """(units 0-1, the sums of magnitudes behind them, conv1's share of those) in float64."""
+    def conv(t, w, b):
+        n, _, h, _ = t.shape
+        u = torch.nn.functional.pad(t, (1, 1, 1, 1)).unfold(2, 3, 1).unfold(3, 3, 1)
+        y = u.permute(0, 2, 3, 1, 4, 5).reshape(n * h * h, -1) @ w.reshape(w.shape[0], -1).t() + b
+        return y.view(n, h, h, -1).permute(0, 3, 1, 2)
+    W = {k: v.to(DEV).double() for k, v in sd.items()}
+    x = x.to(DEV).double()
+    pool = torch.nn.functional.max_pool2d
+    a = pool(conv(x, W["conv1.weight"], W["conv1.bias"]).relu(), 2)
+    mag = pool(conv(x.abs(), W["conv1.weight"].abs(), W["conv1.bias"].abs()), 2)
+    y = pool(conv(a, W["conv2.weight"], W["conv2.bias"]).relu(), 2)
+    own = conv(mag, W["conv2.weight"].abs(), W["conv2.bias"].abs())
+    # the 4 x 4 patch of every output: F(2 x 2, 3 x 3) meets all of it
+    patch = torch.nn.functional.max_pool2d(torch.nn.functional.pad(mag, (1, 1, 1, 1)), 4, 2)
+    wide = patch.permute(0, 2, 3, 1) @ W["conv2.weight"].abs().sum((2, 3)).t()
+    return y.flatten(1), pool(own, 2).flatten(1), wide.permute(0, 3, 1, 2).flatten(1)
+
+
+@pytest.mark.parametrize("boundary", ["fp32", "split"])
+@pytest.mark.parametrize("B,grid,kind", [(3, 1, "plain"), (5, 2, "plain"), (7, 2, "holes"), (7, 3, "wide"), (513, 0, "plain"),
+                                         (1025, 256, "holes"), (4, 1, "huge"), (6, 2, "flat")])
+def test_cifar_winograd(B, grid, kind, boundary):
+    """conv2 by Winograd against 64 bits and against the direct form: workgroups with 3 and more images, and
+    with unequal numbers of them; infinities and NaN (what they reach is 0 in both forms); a range too wide for
+    one scale (the direct form's bits); images of magnitudes near the range's ends.  Bound: conv1 is off by 3 * 2^-17
+    of its magnitudes; a product of conv2 by 2^-19, of which an output sums 9 of operands up to 4 times the patch's."""
+    from distributed_neural_networks_amd.ops import cifar as cops
+    g = torch.Generator().manual_seed(B)
+    sd, _, _, _ = _cifar_golden(B, 1)
+    x = torch.randn(B, 3, 32, 32, generator=g) * {"huge": 500.0, "flat": 1e-6}.get(kind, 1.0)
+    if kind == "holes":
+        x[0, 1, 0, 0], x[1, 0, 31, 31], x[2, 2, 13, 18], x[-1, 1, 16, 7] = float("inf"), float("nan"), -float("inf"), float("nan")
+    if kind == "wide":
+        x[::2, :, :16] *= 1e6
+    w0, x = cops.pack_stage0(sd, DEV), x.to(DEV)
+    assert w0.u2h is not None and B > cops.WINO_ROUNDS * (grid or 256)
+    keep, h = torch.zeros_like(x), torch.full((B, 4096), float("nan"), device=DEV)
+    cops.stage0_forward(x, w0, h, grid=grid, boundary=boundary, keep=keep)
+    assert torch.equal(keep.view(torch.int32), x.view(torch.int32))
+    direct = cops.stage0_forward(x, w0, grid=B, boundary=boundary)  # one image a workgroup
+    if boundary == "split":
+        plain = cops.stage0_forward(x, w0, grid=grid)
+        assert torch.equal(cops.encode_boundary(plain).view(torch.int32), h.view(torch.int32))
+        h, direct = plain, cops.decode_boundary(direct)
+    if kind == "wide":
+        assert torch.equal(h[::2], cops.stage0_forward(x, w0, grid=B)[::2])
+    if kind == "holes":
+        clean = torch.nan_to_num(x, nan=0.0, posinf=0.0, neginf=0.0)
+        touched = torch.nn.functional.pad((x != clean).any(1, keepdim=True).float(), (1, 2, 1, 1))
+        touched = torch.nn.functional.max_pool2d(touched, (3, 4), 1)  # conv1's windows, whose rows are padded to 4 with zeros
+        touched = torch.nn.functional.max_pool2d(touched, 2)
+        touched = torch.nn.functional.max_pool2d(torch.nn.functional.max_pool2d(touched, 3, 1, 1), 2)
+        away = (touched == 0).expand(B, 64, 8, 8).reshape(B, 4096)
+        ref, own, wide = _stage0_in_64_bits(sd, clean)
+        assert ((h - direct).abs() <= own * 3 * 2.0 ** -16 + wide * 36 * 2.0 ** -18).all()  # 0 for 0 where they reach
+        ref, own, wide = (t * away for t in (ref, own, wide))
+        h, direct = h * away, direct * away
+    else:
+        ref, own, wide = _stage0_in_64_bits(sd, x)
+    assert ((h.double() - ref).abs() <= own * 3 * 2.0 ** -17 + wide * 36 * 2.0 ** -19).all()
+    assert (h.double() - ref).norm() <= 1.05 * (direct.double() - ref).norm()  # no further off than the direct form
+
+
+def test_cifar_without_biases_stays_direct():
+    """Without biases beside them, small parts of an image have no floor: the direct form, the same bits."""
+    from distributed_neural_networks_amd.ops import cifar as cops
+    sd, x, _, _ = _cifar_golden(5, 5)
+    sd = {k: torch.zeros_like(v) if k == "conv1.bias" else v for k, v in sd.items()}
+    w0, x = cops.pack_stage0(sd, DEV), x.to(DEV)
+    assert w0.u2h is None
+    assert torch.equal(cops.stage0_forward(x, w0, grid=1), cops.stage0_forward(x, w0, grid=5))
+
+
 @pytest.mark.parametrize("boundary", ["fp32", "split"])
 def test_cifar_fp32_pipeline_large_batch_fused_fc1(boundary):
     """The large-batch fp32 head (fused fc1) on 20000 images: max |dprob| <= 1e-5
