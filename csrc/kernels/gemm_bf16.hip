@@ -480,7 +480,7 @@ static int g_gemm_tile = 0;
 // Forced tile of gemm_mid.h's table and K split (tests, A/B); -1: chosen
 static int g_mid_tile = -1, g_mid_splits = 1;
 extern "C" int dnn_gemm_set_mid(int tile, int splits) {
-  if (tile < -1 || tile > 4 || splits < 1 || splits > 16) return -1;
+  if (tile < -1 || tile > 6 || splits < 1 || splits > 16) return -1;
   g_mid_tile = tile;
   g_mid_splits = splits;
   return 0;
@@ -813,7 +813,7 @@ extern "C" int dnn_gemm_fp8_256(const void* A, const float* sa, const void* W, c
 // bytes takes a tile as long as the bf16 kernel's K-tile of 64: the same estimate.
 static int mx_mid_tile(int M, int N, int Kb, bool quant) {
   if (g_gemm_tile != 0 || Kb >= 1 << 24) return -1;  // the small tiles address a tile's rows with 32 bits
-  if (g_mid_tile >= 0) return quant && g_mid_tile < 2 ? 2 : g_mid_tile;
+  if (g_mid_tile >= 0 && g_mid_tile < 5) return quant && g_mid_tile < 2 ? 2 : g_mid_tile;
   return mid_plan(M, N, Kb / 2, 0, quant ? MID_MX_QUANT : MID_MX).tile;
 }
 

@@ -22,16 +22,21 @@ struct MidTile {
   static_assert(J % 2 == 0 && PA >= 1 && PB >= 1 && S >= 2, "");
 };
 
-// The tile table (costs: gemm_mid.hip MID)
+// The tile table (costs: gemm_mid.hip MID).  Heights of 192 and 96 rows: between the powers of two a
+// row count leaves half a tile empty or a chip half full, and 192 x 128 has room for four K-tiles where 256 x 128
+// has for three.  us, the best of the others : these: 700 x 6144 x 4096 51.8 : 43.4, 1500 x 4096 x 4096 57.0 : 49.9, 1400 x
+// 3072 x 768 17.4 : 14.9, 700 x 4096 x 14336 in 2 95.2 : 86; 96 rows: 380 x 6144 x 4096 38.3 : 35.0, 700 x 4096 x 4096 34.3 : 33.0.
+// (192 x 64, 128 x 192 and 192 x 192 are best nowhere by more than 2 %.)
 typedef MidTile<64, 64, 2, 2, 4> Mid0;
 typedef MidTile<128, 64, 2, 2, 6> Mid1;
 typedef MidTile<128, 128, 2, 4, 4> Mid2;
 typedef MidTile<256, 128, 4, 2, 3> Mid3;
 typedef MidTile<128, 256, 2, 4, 3> Mid4;
+typedef MidTile<192, 128, 4, 2, 4> Mid5;
+typedef MidTile<96, 128, 2, 2, 5> Mid6;
 // The same where K is split: four waves that only stage (mid_stage), so that no product
 // waits for a request to be taken.  us with and without, parts and their sum: 512 x 4096 x
-// 18432 in 4 77.8 : 83.8, 500 x 4096 x 21504 in 4 89.4 : 94.0, 700 x 4096 x 14336 in 2 97.6 :
-// 101.9.  Smaller tiles gain nothing, and whole ones lack the registers for their epilogue.
+// 18432 in 4 77.8 : 83.8, 500 x 4096 x 21504 in 4 89.4 : 94.0; split 192 x 128 tiles 3 to 5 %.  Smaller tiles gain nothing, and whole ones lack the registers for their epilogue.
 template <class T>
 struct MidSplit {
   typedef T type;
@@ -43,6 +48,10 @@ struct MidSplit<Mid3> {
 template <>
 struct MidSplit<Mid4> {
   typedef MidTile<128, 256, 2, 4, 3, 4> type;
+};
+template <>
+struct MidSplit<Mid5> {
+  typedef MidTile<192, 128, 4, 2, 4, 4> type;
 };
 
 // s_waitcnt operand: at most `vm` vector-memory and `lgkm` LDS operations outstanding

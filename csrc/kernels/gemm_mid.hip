@@ -4,45 +4,54 @@
 
 namespace dnn {
 
-// Tile table: rows, columns, whether two workgroups share a CU, and the two
-// constants of a tile's time in us: a (launch, first loads, epilogue) and s (a
-// K-tile of 64).  Over 406 shapes (66 to 9400 rows, 768 to 28672 columns, K of 768 to
-// 21504, weights cold) that every tile ran with 1 to 8 splits, 7564 times, the estimate is
-// off by 10 % (rms); what it picks takes 1.7 % longer than the best measured on average
-// (0.4 % in the median, 17 % at worst: 75 x 6144 x 4096 22.5 us, 19.2 as 128 x 128 in 4;
-// profiles/gemm_mid_estimate.md).  The constants are those of the kernels before the staging
-// waves of MidSplit and the 256 x 256 schedule of gemm_tile.h: split 256 x 128 and 128 x 256
-// tiles run 7 and 6 % faster than estimated, the 256 x 256 kernel (the last entry) 6 %; 12 of the
-// 406 shapes would run over 2 % faster as such a split tile than as picked.
+// Tile table: rows, columns, whether two workgroups share a CU, and the constants of a
+// tile's time in us: a (launch, first loads, epilogue), s (a K-tile of 64) and p (of s, where K is
+// split: no epilogue, and waves that only stage), fitted to 1174 shapes.  Over 590 others (66 to 9400 rows, 768 to
+// 28672 columns, K of 768 to 21504, weights cold), every tile with 1 to 8 splits, the estimate is off by 10 % (rms);
+// what it picks takes 1.3 % longer than the best measured on average, 0.4 % in the median (profiles/gemm_mid_estimate.md).
 struct MidCost {
   int bm, bn, pairs;
-  float a, s;
+  float a, s, p;
 };
-static constexpr MidCost MID[] = {{64, 64, 1, 1.89f, 0.252f},   {128, 64, 0, 2.78f, 0.332f},
-                                  {128, 128, 0, 2.99f, 0.472f}, {256, 128, 0, 4.14f, 0.707f},
-                                  {128, 256, 0, 4.07f, 0.754f}, {256, 256, 0, 4.93f, 1.198f}};
-static constexpr int MID_TILES = 5, CUS = 256;
+static constexpr MidCost MID[] = {{64, 64, 1, 2.97f, 0.220f, 0.83f},    {128, 64, 0, 3.04f, 0.332f, 0.94f},
+                                  {128, 128, 0, 3.18f, 0.454f, 1.03f},  {256, 128, 0, 4.14f, 0.747f, 0.88f},
+                                  {128, 256, 0, 3.88f, 0.752f, 0.92f},  {192, 128, 0, 3.67f, 0.602f, 0.92f},
+                                  {96, 128, 0, 3.67f, 0.446f, 0.89f}};
+static constexpr MidCost MID_256 = {256, 256, 0, 6.33f, 1.172f, 1.f};
+// The e4m3 kernels on the first five and as 256 x 256, whole
+static constexpr MidCost MID8[] = {{64, 64, 1, 1.89f, 0.252f, 1.f},   {128, 64, 0, 2.78f, 0.332f, 1.f},
+                                   {128, 128, 0, 2.99f, 0.472f, 1.f}, {256, 128, 0, 4.14f, 0.707f, 1.f},
+                                   {128, 256, 0, 4.07f, 0.754f, 1.f}};
+static constexpr MidCost MID8_256 = {256, 256, 0, 4.93f, 1.198f, 1.f};
+static constexpr int CUS = 256;
 
-// Time of one tile size and split: K-tiles of the fullest CU, beside the time that
-// reading the weights (4.3 TB/s) and moving the activations (2 TB/s) takes; a split
-// adds its sum (one more launch, and the parts written and read at 3.2 TB/s).
-static float mid_time(const MidCost& c, int M, int N, int K, int splits) {
+// Bytes a microsecond: weights, activations in and out, parts of a split
+struct MidRates {
+  float w, x, part;
+};
+static constexpr MidRates RATES = {7.3e6f, 1.9e6f, 3.2e6f}, RATES8 = {4.27e6f, 2.0e6f, 3.16e6f};
+
+// Time of one tile size and split: K-tiles of the fullest CU, beside the time that reading the
+// weights and moving the activations takes; a split adds its sum (one more launch, and the
+// parts written and read).
+static float mid_time(const MidCost& c, const MidRates& r, int M, int N, int K, int splits) {
   const long long wgs = (long long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * splits;
   const int kt = (K / 64 + splits - 1) / splits, n = (int)((wgs + CUS - 1) / CUS);
   const float rounds = c.pairs ? (n / 2) * 1.73f + (n & 1) : (float)n;
   const float a = c.pairs ? c.a : c.a * (1.f + 0.5f * (n - 1));
-  const float t = rounds * kt * c.s, w = (float)N * K * 2.f / 4.27e6f + (float)M * (K + N) * 2.f / 2.0e6f;
+  const float t = rounds * kt * (splits > 1 ? c.s * c.p : c.s), w = (float)N * K * 2.f / r.w + (float)M * (K + N) * 2.f / r.x;
   const float us = a + cbrtf(t * t * t + w * w * w);
-  return splits == 1 ? us : us + 4.f + (splits + 0.5f) * M * N * 4.f / 3.16e6f;
+  return splits == 1 ? us : us + 4.12f + (splits + 0.5f) * M * N * 4.f / r.part;
 }
 
 // The best tile and split of M x N, at most `best`.
 static MidPlan best_tile(int M, int N, int K, long long ws_bytes, unsigned kind, MidPlan best) {
-  for (int i = 0; i < MID_TILES; ++i) {
-    if (kind == MID_MX_QUANT && MID[i].bn < 128) continue;
+  const bool mx = kind >= MID_MX;
+  for (int i = 0; i < (mx ? 5 : 7); ++i) {
+    if (kind == MID_MX_QUANT && MID8[i].bn < 128) continue;
     for (int s = 1; s <= 8; ++s) {
       if (s > 1 && (N % 4 != 0 || M > 65535 || K / 64 / s < 3 || (long long)s * M * N * 4 > ws_bytes)) break;
-      const float t = mid_time(MID[i], M, N, K, s);
+      const float t = mx ? mid_time(MID8[i], RATES8, M, N, K, s) : mid_time(MID[i], RATES, M, N, K, s);
       if (t < best.us) best = {i, s, t, 0};
     }
   }
@@ -52,9 +61,9 @@ static MidPlan best_tile(int M, int N, int K, long long ws_bytes, unsigned kind,
 static MidPlan best_plan(int M, int N, int K, long long ws_bytes, unsigned kind) {
   // the 256 x 256 kernel needs to be 5 % slower to lose: the estimate's error at
   // its sizes (12352 columns of 3000 rows: 257 us, 267 as 256 x 128)
-  const MidCost& big = MID[MID_TILES];
-  MidPlan best = best_tile(M, N, K, ws_bytes, kind,
-                           {-1, 1, M < 256 || N < 256 ? 1e30f : 0.95f * mid_time(big, M, N, K, 1), 0});
+  const bool mx = kind >= MID_MX;
+  const float whole = mx ? mid_time(MID8_256, RATES8, M, N, K, 1) : mid_time(MID_256, RATES, M, N, K, 1);
+  MidPlan best = best_tile(M, N, K, ws_bytes, kind, {-1, 1, M < 256 || N < 256 ? 1e30f : 0.95f * whole, 0});
   // Full rounds of 256 x 256 tiles and the columns that are left on the tile that
   // suits them: a last round that fills a third of the chip costs a whole one.  us as
   // the best single tile and in two: 700 x 28672 x 4096 168 : 155, 1700 rows 356 : 320,
@@ -64,7 +73,7 @@ static MidPlan best_plan(int M, int N, int K, long long ws_bytes, unsigned kind)
     const int cols = (int)(tiles / CUS * CUS / ntm) * 256;
     if (cols > 0 && cols < N) {
       MidPlan two = best_tile(M, N - cols, K, ws_bytes, kind, {-1, 1, 1e30f, 0});
-      two.us += mid_time(big, M, cols, K, 1);
+      two.us += mid_time(MID_256, RATES, M, cols, K, 1);
       two.cols = cols;
       if (two.us < 0.95f * best.us) best = two;
     }
@@ -72,7 +81,7 @@ static MidPlan best_plan(int M, int N, int K, long long ws_bytes, unsigned kind)
   return best;
 }
 
-// The same by sizes: 48 estimates take 3 us of host time, a table entry (per thread)
+// The same by sizes: some 50 estimates take 3 us of host time, a table entry (per thread)
 // nothing beside a launch.
 MidPlan mid_plan(int M, int N, int K, long long ws_bytes, unsigned kind) {
   struct Entry {
@@ -92,8 +101,7 @@ MidPlan mid_plan(int M, int N, int K, long long ws_bytes, unsigned kind) {
 // and 32 columns a workgroup (16 up to 1024 columns), which share a CU and add up: the
 // time is that of the fullest CU, in steps.  `frag`: the weight has its fragment-order
 // copy; without it a step costs 1.6 times as much.  A folded norm rides along for 1 us; the
-// tiles need a launch that adds 3.3, and at K below 1024 they take 0.8 longer than their
-// estimate.  us, decode kernels : tiles: 132 rows x 768 x 768 5.3 : 5.8, 192 6.6 : 5.9; row-
+// tiles need a launch that adds 3.3.  us, decode kernels : tiles: 132 rows x 768 x 768 5.3 : 5.8, 192 6.6 : 5.9; row-
 // major 70 4.8 : 5.3; 192 x 768 x 3072 row-major 19.4 : 12.1; 70 x 1600 x 1600 7.1 : 7.1, 85
 // 9.0 : 8.5; 256 x 4096 x 4096 88 : 18; with a norm 128 x 3072 x 768 9.0 : 9.7, 146 10.4 : 9.8,
 // 135 x 2304 x 768 8.6 : 9.2, 167 9.6 : 9.1, 128 x 2816 x 512 6.4 : 7.4, 189 8.1 : 7.6, 256 x 1536 x
@@ -106,7 +114,7 @@ bool mid_skinny(int M, int N, int K, bool norm, bool frag, long long ws_bytes) {
   const float step = frag ? (one ? 0.45f + 0.0009f * K : 0.15f + 0.00152f * K)
                           : (one ? 0.4f + 0.0016f * K : 0.2f + 0.0025f * K);
   return base + n * step + (norm ? 1.f : 0.f) <
-         mid_plan(M, N, K, ws_bytes, MID_BF16).us + (K < 1024 ? 0.8f : 0.f) + (norm ? 3.3f : 0.f);
+         mid_plan(M, N, K, ws_bytes, MID_BF16).us + (norm ? 3.3f : 0.f);
 }
 
 template <class T, MidOut OUT>
@@ -142,6 +150,8 @@ int mid_launch(int tile, const MidArgs& a, const QkvScatter* scat, hipStream_t s
     case 2: return launch<Mid2>(a, scat, st);
     case 3: return launch<Mid3>(a, scat, st);
     case 4: return launch<Mid4>(a, scat, st);
+    case 5: return launch<Mid5>(a, scat, st);
+    case 6: return launch<Mid6>(a, scat, st);
   }
   return -1;
 }

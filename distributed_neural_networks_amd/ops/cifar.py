@@ -248,13 +248,14 @@ def stage0_forward(x: torch.Tensor, w: CifarStage0Weights, out: Optional[torch.T
         _check_act(keep, (3, 32, 32), torch.float32, "stage0 keep")
         if keep.shape[0] != B or abs(ptr(keep) - ptr(x)) < x.nbytes:
             raise ValueError("stage0: keep must be as large as x and apart from it")
-    if w.precision == "fp32" and B > WINO_ROUNDS * (grid or 256) and w.u2h is not None:
-        check(lib().cifar_stage0_wino(ptr(x), ptr(out), ptr(w.w1h), ptr(w.w1l), ptr(w.b1), ptr(w.w2h), ptr(w.w2l),
-                                      ptr(w.u2h), ptr(w.u2l), ptr(w.b2), ptr(w.sc), B, grid, stream_ptr(), split, ptr(keep)),
-              "cifar_stage0_wino")
-    elif w.precision == "fp32":
-        check(lib().cifar_stage0_x3(ptr(x), ptr(out), ptr(w.w1h), ptr(w.w1l), ptr(w.b1), ptr(w.w2h), ptr(w.w2l),
-                                    ptr(w.b2), B, grid, stream_ptr(), split, ptr(keep)), "cifar_stage0_x3")
+    if w.precision == "fp32":
+        if B > WINO_ROUNDS * (grid or 256) and w.u2h is not None:
+            check(lib().cifar_stage0_wino(ptr(x), ptr(out), ptr(w.w1h), ptr(w.w1l), ptr(w.b1), ptr(w.w2h), ptr(w.w2l),
+                                          ptr(w.u2h), ptr(w.u2l), ptr(w.b2), ptr(w.sc), B, grid, stream_ptr(), split,
+                                          ptr(keep)), "cifar_stage0_wino")
+        else:
+            check(lib().cifar_stage0_x3(ptr(x), ptr(out), ptr(w.w1h), ptr(w.w1l), ptr(w.b1), ptr(w.w2h), ptr(w.w2l),
+                                        ptr(w.b2), B, grid, stream_ptr(), split, ptr(keep)), "cifar_stage0_x3")
     else:
         check(lib().cifar_stage0_v4(ptr(x), ptr(out), ptr(w.w1), ptr(w.b1), ptr(w.w2), ptr(w.b2), B, grid,
                                     stream_ptr()), "cifar_stage0_v4")

@@ -226,7 +226,7 @@ def set_gemm_tile(tile: int = 0) -> None:
 
 
 def set_gemm_mid(tile: int = -1, splits: int = 1) -> None:
-    """Force a tile of gemm_mid.h's table (0..4) and a K split for GEMMs above the
+    """Force a tile of gemm_mid.h's table (0..6) and a K split for GEMMs above the
     decode sizes (tests, A/B probes); -1 restores the choice by estimated time."""
     check(lib().gemm_set_mid(int(tile), int(splits)), "gemm_set_mid")
     _is_skinny.cache_clear()

@@ -699,7 +699,7 @@ def test_fp8_gemm_tail_split_matches_single_grid(N, K, split, act, res):
     assert err < (3e-2 if split else 8e-2), err
 
 
-MID_TILES = ((64, 64), (128, 64), (128, 128), (256, 128), (128, 256))  # csrc/kernels/gemm_mid.hip MID
+MID_TILES = ((64, 64), (128, 64), (128, 128), (256, 128), (128, 256), (192, 128), (96, 128))  # csrc/kernels/gemm_mid.hip MID
 
 
 def _mid_reference(x, w, b, r, act, norm, consts):
@@ -755,6 +755,14 @@ def test_gemm_mid_tiles(tile, splits, dm, dn, K):
     finally:
         G.set_gemm_mid()
     assert not ws[-4096:].any()  # the tickets of a decode workspace are not parts
+
+
+@pytest.mark.parametrize("tile", [5, 6])
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("dm,dn,K", [(1, 36, 192), (0, 0, 448), (-1, -8, 576), (-97, 20, 4096), (-47, 100, 320)])
+def test_gemm_mid_tiles_between(tile, splits, dm, dn, K):
+    """The tiles of 192 and 96 rows: as test_gemm_mid_tiles, and with rows that end in any wave's part."""
+    test_gemm_mid_tiles(tile, splits, max(dm, 1 - MID_TILES[tile][0]), dn, K)
 
 
 @pytest.mark.parametrize("M,N,K", [(65, 768, 3072), (96, 4096, 14336), (200, 6144, 4096), (256, 768, 768), (257, 4800, 1600),
@@ -909,3 +917,29 @@ def test_qkv_scatter_small_prefill(B, T, H, Hkv, hd, pos0, S):
         keep = pos0 + torch.arange(T, device=DEV) < S
         assert torch.equal(q.view(B, H, T, hd)[:, :, keep], q2.view(B, H, T, hd)[:, :, keep])
         assert torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3])
+
+
+@pytest.mark.parametrize("tile", [5, 6])
+@pytest.mark.parametrize("B,T,H,Hkv,hd,pos0,S", [(1, 193, 12, 12, 64, 0, 200), (3, 43, 4, 2, 128, 5, 60), (2, 97, 25, 25, 64, 9, 100)])
+def test_qkv_scatter_tiles_between(tile, B, T, H, Hkv, hd, pos0, S):
+    """The scatter epilogue of the tiles of 192 and 96 rows == qkv rows + qkv_split."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    from distributed_neural_networks_amd.ops import transformer_ops as T_
+    g = torch.Generator(device=DEV).manual_seed(B * T)
+    d, N = 320, (H + 2 * Hkv) * hd
+    x = torch.randn(B * T, d, device=DEV, generator=g).bfloat16()
+    f = G.fold_norm(torch.randn(N, d, device=DEV, generator=g) * 0.05, torch.ones(d, device=DEV), torch.zeros(d, device=DEV),
+                    torch.randn(N, device=DEV, generator=g) * 0.02, False, 1e-5, DEV)
+    std, pos = torch.empty(B * T, d, device=DEV, dtype=torch.bfloat16), torch.full((B,), pos0, device=DEV, dtype=torch.int32)
+    caches = [torch.zeros(B, Hkv, S, hd, device=DEV).bfloat16() for _ in range(4)]
+    q, q2 = (torch.empty(B * H * T * hd, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    G.set_gemm_mid(tile)
+    try:
+        assert G.qkv_scatter_norm(x, f, std, q, caches[0], caches[1], pos, B, T, H, Hkv, hd)
+        qkv = G.linear_norm(x, f, std_buf=std, ones=torch.ones(d, device=DEV))
+    finally:
+        G.set_gemm_mid()
+    T_.qkv_split(qkv, q2, caches[2], caches[3], B, T, H, Hkv, hd, pos)
+    keep = pos0 + torch.arange(T, device=DEV) < S
+    assert torch.equal(q.view(B, H, T, hd)[:, :, keep], q2.view(B, H, T, hd)[:, :, keep])
+    assert torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3])
