@@ -307,7 +307,7 @@ __global__ __launch_bounds__(256 * KS, 2) void flash_attn_kernel(const bf16_t* _
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
         for (int g = 0; g < 16; g += 2) mx = fmax_nan(mx, fmax_nan(sacc[kt][g], sacc[kt][g + 1]));
-      mx = fmax_nan(mx, __shfl_xor(mx, 32, 64));
+      mx = max32_nan(mx);
       const float m_new = fmax_nan(m_i, mx * scale_log2);
       const float m_use = m_new == -INFINITY ? 0.f : m_new;
       const float alpha = __builtin_amdgcn_exp2f(m_i - m_use);
@@ -327,7 +327,7 @@ __global__ __launch_bounds__(256 * KS, 2) void flash_attn_kernel(const bf16_t* _
           rs2 += pv;
         }
       float rs = rs2[0] + rs2[1];
-      rs += __shfl_xor(rs, 32, 64);
+      rs = add32(rs);
       l_i = l_i * alpha + rs;
       m_i = m_new;
       // hd 64 (VALU-bound): the running max rarely moves once the first blocks

@@ -26,12 +26,7 @@
 //    the wave.
 typedef uint16_t u16x2v __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ float max_over_quarters(float v) {  // lanes l, l ^ 16, l ^ 32, l ^ 48
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
+__device__ __forceinline__ float max_over_quarters(float v) { return max32(max16(v)); }  // lanes l, l ^ 16, l ^ 32, l ^ 48
 
 // Sums of v[0..N) over the wave's row groups (LPK lanes apart), spread: quarter rr = lane
 // >> 4 ends with values at(rr) .. at(rr) + N / 4 in v[0..N / 4): a swap and an add halve
@@ -62,6 +57,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
     const float* __restrict__ sinT, float scale_log2, bf16_t* __restrict__ o_direct) {
   constexpr bool FUSED = FM != 0, ROPE = FM == 2;
   constexpr int LPK = HD / 8, RG = 64 / LPK, R = U * RG;
+  static_assert(LPK == 8 || LPK == 16, "sums over row groups");
   constexpr bool MF = G > 1;
   constexpr int NT16 = R / 16, NKC = HD / 32;  // MF: key tiles of a block, k-steps of a tile
   static_assert(U % 2 == 0, "P.V folds row pairs");
@@ -322,13 +318,13 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
   // the wave's row groups, then the waves: a group without rows carries the lowest m, l = 0
   float mw = m, f = 1.f;
   if constexpr (!MF) {
-#pragma unroll
-    for (int off = LPK; off < 64; off <<= 1) mw = fmaxf(mw, __shfl_xor(mw, off, 64));
+    if constexpr (LPK == 8) mw = fmaxf(mw, dpp_f<0x128>(mw));  // row_ror:8
+    mw = max_over_quarters(mw);
     f = m == mw ? 1.f : __builtin_amdgcn_exp2f(m - mw);
   }
   float ls = l * f;
-#pragma unroll
-  for (int off = MF ? 16 : LPK; off < 64; off <<= 1) ls += __shfl_xor(ls, off, 64);
+  if constexpr (!MF && LPK == 8) ls += dpp_f<0x128>(ls);
+  ls = add32(add16(ls));
   if (lane < G) {
     mred[wave * G + lane] = mw;
     lred[wave * G + lane] = ls;

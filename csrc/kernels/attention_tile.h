@@ -30,7 +30,7 @@ __device__ __forceinline__ float pa_softmax(f32x16 (&s)[NT], float sc, float& m_
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int g = 0; g < 16; g += 2) mx = fmax_nan(mx, fmax_nan(s[t][g], s[t][g + 1]));
-  mx = fmax_nan(mx, __shfl_xor(mx, 32, 64));
+  mx = max32_nan(mx);
   const float m_new = fmax_nan(m_i, mx * sc);
   const float m_use = m_new == -INFINITY ? 0.f : m_new;
   const float alpha = __builtin_amdgcn_exp2f(m_i - m_use);
@@ -42,7 +42,7 @@ __device__ __forceinline__ float pa_softmax(f32x16 (&s)[NT], float sc, float& m_
       s[t][g] = __builtin_amdgcn_exp2f(fmaf(s[t][g], sc, -m_use));
       rs += s[t][g];
     }
-  rs += __shfl_xor(rs, 32, 64);
+  rs = add32(rs);
   l_i = fmaf(l_i, alpha, rs);
   m_i = m_new;
   return alpha;

@@ -820,8 +820,8 @@ __global__ __launch_bounds__(256) void cifar_head_few_kernel(const float* __rest
         z = fmaf(hv[2 * e + 1], __uint_as_float(ph[e] & 0xffff0000u) + __uint_as_float(pl[e] & 0xffff0000u), z);
       }
     }
-    z += __shfl_xor(z, 16, 64);
-    z += __shfl_xor(z, 32, 64);
+    z = add16(z);
+    z = add32(z);
     if ((tid & 63) < 16) zs[tid >> 6][cls] = z;
     __syncthreads();
     if (tid < 16) {

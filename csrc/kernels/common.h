@@ -11,6 +11,7 @@ namespace dnn {
 typedef uint16_t bf16_t;
 typedef short bf16x8 __attribute__((ext_vector_type(8)));
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -56,7 +57,6 @@ __device__ __forceinline__ float gelu_erf(float x) {
 // products go through v_pk_fma_f32 / v_pk_mul_f32 (two lanes' worth per
 // instruction), only the reciprocal, the exponential, |x| and the sign select
 // stay per element — a GEMM epilogue applies it to 128 outputs per thread.
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ f32x2 gelu_erf2(f32x2 x) {
   const f32x2 z = f32x2{fabsf(x[0]), fabsf(x[1])} * 0.70710678118654752f;
   const f32x2 d = z * 0.3275911f + 1.0f;
@@ -89,6 +89,26 @@ __device__ __forceinline__ float dpp_f(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
 }
 
+// The values of this lane and of the one 16 (32) away, in the order of the lanes: one
+// v_permlane16_swap (32_swap) where a __shfl_xor is a round trip through the LDS unit, some 130
+// clocks of a chain: the launches of one to 64 rows are chains of a few microseconds with two to
+// four of these in each (a GPT-2 decode step of one row 288.8 -> 283.6 us, of 64 rows 543 -> 537,
+// of 64 rows in fp8 359.0 -> 351.5).  The bits are those of the shuffles.  Every lane of the wave
+// (16: of its half) must call it.
+__device__ __forceinline__ f32x2 lanes16(float v) {
+  const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f32x2{__uint_as_float(s[0]), __uint_as_float(s[1])};
+}
+__device__ __forceinline__ f32x2 lanes32(float v) {
+  const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f32x2{__uint_as_float(s[0]), __uint_as_float(s[1])};
+}
+__device__ __forceinline__ float add16(float v) { const f32x2 p = lanes16(v); return p[0] + p[1]; }
+__device__ __forceinline__ float add32(float v) { const f32x2 p = lanes32(v); return p[0] + p[1]; }
+__device__ __forceinline__ float max16(float v) { const f32x2 p = lanes16(v); return fmaxf(p[0], p[1]); }
+__device__ __forceinline__ float max32(float v) { const f32x2 p = lanes32(v); return fmaxf(p[0], p[1]); }
+__device__ __forceinline__ float max32_nan(float v) { const f32x2 p = lanes32(v); return fmax_nan(p[0], p[1]); }
+
 // Sum / max over aligned groups of L lanes (L = 1..64); every lane of the group
 // gets the result.
 template <int L>
@@ -97,8 +117,8 @@ __device__ __forceinline__ float group_sum(float v) {
   if constexpr (L >= 4) v += dpp_f<0x4E>(v);
   if constexpr (L >= 8) v += dpp_f<0x141>(v);
   if constexpr (L >= 16) v += dpp_f<0x140>(v);
-  if constexpr (L >= 32) v += __shfl_xor(v, 16, 64);
-  if constexpr (L >= 64) v += __shfl_xor(v, 32, 64);
+  if constexpr (L >= 32) v = add16(v);
+  if constexpr (L >= 64) v = add32(v);
   return v;
 }
 template <int L>
@@ -107,8 +127,8 @@ __device__ __forceinline__ float group_max(float v) {
   if constexpr (L >= 4) v = fmaxf(v, dpp_f<0x4E>(v));
   if constexpr (L >= 8) v = fmaxf(v, dpp_f<0x141>(v));
   if constexpr (L >= 16) v = fmaxf(v, dpp_f<0x140>(v));
-  if constexpr (L >= 32) v = fmaxf(v, __shfl_xor(v, 16, 64));
-  if constexpr (L >= 64) v = fmaxf(v, __shfl_xor(v, 32, 64));
+  if constexpr (L >= 32) v = max16(v);
+  if constexpr (L >= 64) v = max32(v);
   return v;
 }
 

@@ -228,8 +228,8 @@ __global__ __launch_bounds__(PIPE ? 512 : 256, 1) void delta_chunks_kernel(Delta
         const float x = bf2f_s(f[i][j >> 2][j & 3]);
         s = fmaf(x, x, s);
       }
-    s += __shfl_xor(s, 16, 64);
-    s += __shfl_xor(s, 32, 64);
+    s = add16(s);
+    s = add32(s);
     return 1.0f / sqrtf(s + a.unit_eps);
   };
   // what was fetched, of this wave's block, to LDS; v waits for the set of its chunk

@@ -327,8 +327,8 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_256_kernel(
             }
             acc[mq][nq][i][j] = v;
           }
-          am = fmaxf(am, __shfl_xor(am, 16, 64));
-          am = fmaxf(am, __shfl_xor(am, 32, 64));
+          am = max16(am);
+          am = max32(am);
           if (lane < 16) red[((((mq * 2 + nq) * 4 + i) * 2 + wr) * 16 + lane) * 4 + wc] = am;
         }
     __syncthreads();

@@ -188,8 +188,8 @@ __device__ __forceinline__ void epi_rowstat16(const f32x4& x, int m, int n0, int
   float s = 0.f;
 #pragma unroll
   for (int r = 0; r < 4; ++r) s += r < nv ? x[r] : 0.f;
-  s += __shfl_xor(s, 16, 64);
-  s += __shfl_xor(s, 32, 64);
+  s = add16(s);
+  s = add32(s);
   const float mean = s / (float)nt;
   float q = 0.f;
 #pragma unroll
@@ -197,8 +197,8 @@ __device__ __forceinline__ void epi_rowstat16(const f32x4& x, int m, int n0, int
     const float d = r < nv ? x[r] - mean : 0.f;
     q = fmaf(d, d, q);
   }
-  q += __shfl_xor(q, 16, 64);
-  q += __shfl_xor(q, 32, 64);
+  q = add16(q);
+  q = add32(q);
   if (lane < 16 && m < M) rs[(size_t)m * ld + (n0 >> 4)] = make_float2(mean, q);
 }
 
@@ -225,12 +225,9 @@ __device__ __forceinline__ float2 rowstat_merge(const float2 (&p)[SPT], float2 p
       sm += p[i].y;
     }
   }
-#pragma unroll
-  for (int o = 1; o < TPR; o <<= 1) {
-    s1 += __shfl_xor(s1, o, 64);
-    s2 += __shfl_xor(s2, o, 64);
-    sm += __shfl_xor(sm, o, 64);
-  }
+  s1 = group_sum<TPR>(s1);
+  s2 = group_sum<TPR>(s2);
+  sm = group_sum<TPR>(sm);
   const float invk = 1.f / (float)K;
   const float var = NORM == 2 ? fmaxf((sm + s2 - s1 * s1 * invk) * invk, 0.f) : (sm + s2) * invk;
   return make_float2(NORM == 2 ? c + s1 * invk : 0.f, rsqrtf(var + eps));

@@ -243,11 +243,8 @@ __global__ __launch_bounds__(512, 1) void gemm_head_kernel(const uint8_t* __rest
 
   // ---- row statistics -> LDS
   if constexpr (NORM != 0) {
-#pragma unroll
-    for (int o = 1; o < 8; o <<= 1) {
-      s1 += __shfl_xor(s1, o, 64);
-      s2 += __shfl_xor(s2, o, 64);
-    }
+    s1 = group_sum<8>(s1);
+    s2 = group_sum<8>(s2);
     if (ssub == 0) {
       const float invk = 1.f / (float)kelems, d = s1 * invk;
       const float var = NORM == 2 ? fmaxf(s2 * invk - d * d, 0.f) : s2 * invk;

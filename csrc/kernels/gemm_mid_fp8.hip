@@ -149,8 +149,8 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_fp8_kernel(Mid8Args p,
         }
         acc[i][j] = v;
       }
-      am = fmaxf(am, __shfl_xor(am, 16, 64));
-      am = fmaxf(am, __shfl_xor(am, 32, 64));
+      am = max16(am);
+      am = max32(am);
       if (lane < 16) red[(wm * (I * 16) + i * 16 + lane) * T::WN + wn] = am;
     }
     __syncthreads();

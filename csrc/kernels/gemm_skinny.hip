@@ -320,10 +320,10 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const uint8_t* __restr
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
       float a = st1[t], q = st2[t];
-      a += __shfl_xor(a, 16, 64);
-      a += __shfl_xor(a, 32, 64);
-      q += __shfl_xor(q, 16, 64);
-      q += __shfl_xor(q, 32, 64);
+      a = add16(a);
+      a = add32(a);
+      q = add16(q);
+      q = add32(q);
       if (lane < 16) {
         sk_st[((wave * MT + t) * 2 + 0) * 16 + lane] = a;
         sk_st[((wave * MT + t) * 2 + 1) * 16 + lane] = q;

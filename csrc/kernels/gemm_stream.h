@@ -397,10 +397,10 @@ __global__ __launch_bounds__(256, 1) void gemm_stream_kernel(const uint8_t* __re
 
   // ---- statistics of this wave's M tile: the 4 lane groups hold disjoint k
   if constexpr (NORM != 0) {
-    s1 += __shfl_xor(s1, 16, 64);
-    s1 += __shfl_xor(s1, 32, 64);
-    s2 += __shfl_xor(s2, 16, 64);
-    s2 += __shfl_xor(s2, 32, 64);
+    s1 = add16(s1);
+    s1 = add32(s1);
+    s2 = add16(s2);
+    s2 = add32(s2);
   }
 
   if constexpr (SPLIT) {

@@ -254,7 +254,7 @@ __global__ __launch_bounds__(512, 1) void latent_attn_kernel(LatentAttnArgs a, c
     float mx = -INFINITY;
 #pragma unroll
     for (int e = 0; e < EN; ++e) mx = fmaxf(mx, s[e]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max32(mx);
     if (h == 0) red[wave * 32 + r32] = mx;
     __syncthreads();
     float al[RH], mu = 0.f, mine = 1.f;
@@ -277,7 +277,7 @@ __global__ __launch_bounds__(512, 1) void latent_attn_kernel(LatentAttnArgs a, c
       s[e] = __builtin_amdgcn_exp2f(fmaf(s[e], sc, -mu));
       rs += s[e];
     }
-    rs += __shfl_xor(rs, 32, 64);
+    rs = add32(rs);
     l_i = fmaf(l_i, mine, rs);
     {  // fragment of 16 keys: this lane's 8, of which a wave has EN
       char* d = ps + ((rh * 4 + kh * 2 + kq * EN / 8) * 64 + lane) * 16;

@@ -370,14 +370,14 @@ __global__ __launch_bounds__(PIPE ? 512 : 256, 1) void wkv_chunks_kernel(WkvArgs
 #pragma unroll
             for (int j = 0; j < 8; ++j)
               v = fmaf(r[j] * __shfl(k[j], src, 64), __builtin_amdgcn_exp2f(fminf(E[j] - __shfl(Lc[j], src, 64), 0.f)), v);
-            v += __shfl_xor(v, 16, 64);
-            v += __shfl_xor(v, 32, 64);
+            v = add16(v);
+            v = add32(v);
             if (g == sq) A[i] += v;
           }
       }
     }
-    own += __shfl_xor(own, 16, 64);
-    own += __shfl_xor(own, 32, 64);
+    own = add16(own);
+    own = add32(own);
     float m[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) m[i] = 4 * g + i < t16 ? A[i] : 4 * g + i == t16 ? own : 0.f;
