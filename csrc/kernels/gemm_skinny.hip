@@ -871,6 +871,22 @@ static int launch_skinny_cfg(const void* A, int lda_b, const float* sa, const vo
   return (int)hipGetLastError();
 }
 
+// Waves and chunks a batch of a workgroup that owns one 16 x 16 tile: as few waves as take K in one
+// batch each, and the batch that leaves fewer requests past a wave's range (those are made all the
+// same, and short products are bound by their requests, W and A).  us, 4 chunks on 8 waves : this, bf16 in
+// fragment order, weights from memory: 1 row, 768 x 768 3.20 : 2.84, 2304 x 768 3.48 : 3.13, 3072 x 768 3.62 :
+// 3.26, 1536 x 512 3.26 : 2.82, 1280 x 1280 4.10 : 3.64; 16 rows, 768 x 768 4.04 : 3.54, 1536 x 512 3.91 : 3.25;
+// 64 rows (4 chunks on 4 waves), 768 x 768 4.31 : 3.99.  The same from 49 chunks on, but for 65 to 72, 4.78 : 4.53.
+struct Few {
+  int u, ks;
+};
+static Few few_plan(bool w8, int kbytes) {
+  const int nch = kbytes / 64;
+  if (w8) return {4, 8};
+  const int ks = nch <= 24 ? 4 : 8, per = (nch + ks - 1) / ks;
+  return {nch <= 48 && (per + 5) / 6 * 6 < (per + 3) / 4 * 4 ? 6 : 4, ks};
+}
+
 template <int ACT, bool F32, bool FP8, int NORM = NORM_NONE, bool W8 = false>
 static int launch_skinny(const void* A, int lda_b, const float* sa, const void* W, int ldw_b, const float* sw,
                          void* C, int ldc, const float* bias, const void* R, int ldr, int M, int N, int kbytes,
@@ -939,18 +955,23 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
     if (N <= 1024) CFG_MS(1, 4, false, 4);
     CFG_MS(2, 2, false, 4);
   }
+  const Few few = few_plan(FP8 || W8, kbytes);
   if (M <= 8) {
     // batch 1-8: the fragment-order copy (Wsh) is streamed whenever the layer
     // attached one; per shape class: QKV-sized N 1 tile x 4 chunks on 4 waves
     // (Llama-3 8B fp8 decode graph 12.25 -> 10.33 us), the rest below
-    if (!FP8 && Wsh != nullptr && N > 4096 && N < 16384 && kbytes <= 8192) CFG(1, 1, 4, false, 4);
+    if (!FP8 && Wsh != nullptr && N > 4096 && N < 16384 && kbytes <= 8192) {
+      if (few.u == 6 && few.ks == 4) CFG(1, 1, 6, false, 4);
+      CFG(1, 1, 4, false, 4);
+    }
     // fp8 vocabulary head (128K x 4K, fragment order): 2 column tiles per wave
     // 83.3 -> 75.8 us, 6.9 TB/s (profiles/archive/r2_skinny_sweep_w8_m1.jsonl)
     if (W8 && Wsh != nullptr && N >= 65536) CFG(1, 2, 4, false, 8);
     // fp8 gate|up (28K x 4K) with the fused RMSNorm: 2 column tiles x 2 chunks
     // on 2 waves 23.3 -> 21.3 us (profiles/archive/r2_w8_decode_projections.jsonl)
     if (W8 && Wsh != nullptr && N >= 16384) CFG(1, 2, 2, false, 2);
-    CFG(1, 1, 4, false, 8);
+    if (few.u == 6) CFG(1, 1, 6, false, few.ks);
+    CFG(1, 1, 4, false, few.ks);
   }
   if (M <= 16) {
     // narrow N: one column tile a workgroup, as for M <= 8.  Two put 64 to 128 workgroups
@@ -958,7 +979,10 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
     // : 9.1, 768 x 3072 8.9 : 6.8, 2304 x 768 5.8 : 5.1; row-major 4096 x 14336 50.4 : 33.3,
     // 2048 x 7680 30.4 : 19.8; e4m3 4096 x 14336 23.9 : 19.0, 1600 x 6400 11.9 : 10.4 (the
     // last four on 4 waves: 8 are up to 10 % slower there and faster above)
-    if (!FP8 && N <= 4096) CFG(1, 1, 4, false, (W8 || Wsh == nullptr) ? 4 : 8);
+    if (!FP8 && N <= 4096) {
+      if (few.u == 6) CFG(1, 1, 6, false, few.ks);
+      CFG(1, 1, 4, false, (W8 || Wsh == nullptr) ? 4 : few.ks);
+    }
     // wide N in fragment order, K from 2048: 28672 x 4096, 12 rows 45.9 : 40.7, 16 rows
     // 45.2 : 44.0, 32768 x 4096 49.9 : 46.2 (50257 x 768 the other way, 19.8 : 23.2)
     if (!FP8 && !W8 && wide && Wsh != nullptr && kbytes >= 4096) CFG(1, 1, 4, false, 4);
@@ -981,7 +1005,10 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
       if (M <= 32) CFG(2, 4, 2, false, 2);
       CFG(4, 4, 2, false, 2);
     }
-    if (N <= 1024) CFG_MS(1, 4, false, 4);
+    if (N <= 1024) {
+      if (few.u == 6 && few.ks == 4) CFG_MS(1, 6, false, 4);
+      CFG_MS(1, 4, false, 4);
+    }
     // (8-wave variants of the Llama-3 8B B=32 QKV / O rules below measured within
     // noise in one process, decode_ab.py --switch skinny_pin, profiles/r6_skinny_pin_ab.jsonl)
     if (!W8 && N > 4096 && M <= 32) CFG(2, 2, 2, true, 4);  // Llama QKV (6144)

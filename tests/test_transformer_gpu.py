@@ -863,6 +863,28 @@ def test_attn_decode_qkv_fused(B, H, Hkv, hd, S, pos, rope, splits):
         assert _rel(out[b], ref) < 2e-2, b
 
 
+@pytest.mark.parametrize("M,N", [(1, 40), (3, 4112), (16, 768), (64, 200)])
+@pytest.mark.parametrize("K", [256, 512, 576, 768, 832, 1024, 1088, 1536, 1600])
+def test_skinny_batches(M, N, K):
+    """Waves and chunks a batch by the length of K (16, 24, 32 and 48 chunks of 32 are the edges), a slice of a wave
+    whole, short and empty: against float64 on the same bf16 values.  Bound: the sum in fp32 (K roundings of the sum of
+    magnitudes) and one rounding to bf16."""
+    from distributed_neural_networks_amd.ops.gemm import fold_norm, linear, linear_norm, shuffle_weight
+    torch.manual_seed(K + M)
+    x = torch.randn(M, K, device=DEV).bfloat16()
+    w = (torch.randn(N, K, device=DEV) / math.sqrt(K)).bfloat16()
+    ref, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    bound = ref.abs() * 2.0 ** -8 + mag * K * 2.0 ** -24
+    for shuf in (None, shuffle_weight(w)):
+        assert bool(((linear(x, w, w_shuf=shuf).double() - ref).abs() <= bound).all())
+    f = fold_norm(w.float(), torch.ones(K, device=DEV), None, None, True, 0.0, DEV)
+    f.ws = shuffle_weight(f.w)
+    r = torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True))
+    # rstd: a sum of squares in fp32, its reciprocal root to 1 ulp
+    bound = (ref * r).abs() * (2.0 ** -8 + K * 2.0 ** -24) + mag * r * K * 2.0 ** -24
+    assert bool(((linear_norm(x, f).double() - ref * r).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
 @pytest.mark.parametrize("N,K", [(100, 128), (2304, 768), (1600, 1600), (6144, 4096), (16400, 256)])
 def test_skinny_shuffled_weights_match(M, N, K):
