@@ -1233,12 +1233,14 @@ static int head_cus() {
   return cus[dev];
 }
 
-template <bool W8, int NORM, int NCH, int CPP, int GS>
+template <bool W8, int NORM, int MT, int NCH, int CPP, int GS>
 static int launch_head_cfg(const void* A, int lda_b, const void* Wsh, const float* sw, const float* colsum,
                            const float* bias, float eps, void* C, int ldc, int M, int N, int K, int grid, void* part,
                            hipStream_t st) {
-  constexpr size_t smem = head_lds_bytes<W8, NCH, CPP, GS>();
-  hipLaunchKernelGGL((gemm_head_kernel<W8, NORM, NCH, CPP, GS>), dim3(grid), dim3(512), smem, st, (const uint8_t*)A, lda_b, (const uint8_t*)Wsh, sw, colsum,
+  constexpr size_t smem = HeadCfg<W8, MT, NCH, CPP, GS>::LDS;
+  const int waves = std::max(2 * MT, ((N + 15) / 16 + grid - 1) / grid);  // <= HEAD_WAVES (dnn_gemm_head)
+  hipLaunchKernelGGL((gemm_head_kernel<W8, NORM, MT, NCH, CPP, GS>), dim3(grid), dim3(64 * waves), smem, st,
+                     (const uint8_t*)A, lda_b, (const uint8_t*)Wsh, sw, colsum,
                      bias, eps, (bf16_t*)C, ldc, M, N, K, (int2*)part);
   return (int)hipGetLastError();
 }
@@ -1247,22 +1249,25 @@ template <int NORM>
 static int launch_head(bool w8, int nch, const void* A, int lda_b, const void* Wsh, const float* sw,
                        const float* colsum, const float* bias, float eps, void* C, int ldc, int M, int N, int K,
                        int grid, void* part, hipStream_t st) {
-  // (weight chunks, chunks per K pass, chunks per load group): the LDS image is
-  // 64 rows x CPP chunks of activations (<= 128 KiB); GPT-2 family widths
-#define HEADC(W8V, NCHV, CPPV, GSV)                                                                             \
+  // Weight chunks; chunks per K pass and per load group for 64 rows, whose LDS image of a pass is at most 128 KiB, and
+  // chunks per group for 16 rows in one pass.  GPT-2 family widths.  A group of 7 (bf16, 1600) or 5 (e4m3, 1600)
+  // chunks of 64 rows spills at 128 registers a wave: 51 us, 39.7 as here.
+#define HEADC(W8V, NCHV, CPPV, GSV, GS1V)                                                                         \
   if (w8 == W8V && nch == NCHV)                                                                                 \
-    return launch_head_cfg<W8V, NORM, NCHV, CPPV, GSV>(A, lda_b, Wsh, sw, colsum, bias, eps, C, ldc, M, N, K, grid, \
-                                                      part, st);
-  HEADC(false, 8, 8, 8)     // gpt2-tiny (d 256)
-  HEADC(false, 24, 24, 12)  // gpt2 (d 768)
-  HEADC(false, 32, 32, 8)   // gpt2-medium (d 1024)
-  HEADC(false, 40, 20, 10)  // gpt2-large (d 1280), 2 K passes
-  HEADC(false, 50, 28, 7)   // gpt2-xl bf16 (d 1600), 2 K passes
-  HEADC(true, 4, 4, 4)      // gpt2-tiny fp8
-  HEADC(true, 12, 12, 4)    // gpt2 fp8
-  HEADC(true, 16, 16, 4)    // gpt2-medium fp8
-  HEADC(true, 20, 10, 5)    // gpt2-large fp8, 2 K passes
-  HEADC(true, 25, 14, 5)    // gpt2-xl fp8 (d 1600), 2 K passes
+    return M <= 16 ? launch_head_cfg<W8V, NORM, 1, NCHV, (NCHV + 3) / 4 * 4, GS1V>(                               \
+                         A, lda_b, Wsh, sw, colsum, bias, eps, C, ldc, M, N, K, grid, part, st)                   \
+                   : launch_head_cfg<W8V, NORM, 4, NCHV, CPPV, GSV>(A, lda_b, Wsh, sw, colsum, bias, eps, C, ldc, M, N, \
+                                                                    K, grid, part, st);
+  HEADC(false, 8, 8, 8, 8)     // gpt2-tiny (d 256)
+  HEADC(false, 24, 24, 8, 8)   // gpt2 (d 768)
+  HEADC(false, 32, 32, 8, 8)   // gpt2-medium (d 1024)
+  HEADC(false, 40, 20, 5, 8)   // gpt2-large (d 1280)
+  HEADC(false, 50, 20, 5, 10)  // gpt2-xl bf16 (d 1600)
+  HEADC(true, 4, 4, 4, 4)      // gpt2-tiny fp8
+  HEADC(true, 12, 12, 4, 4)    // gpt2 fp8
+  HEADC(true, 16, 16, 4, 4)    // gpt2-medium fp8
+  HEADC(true, 20, 12, 4, 5)    // gpt2-large fp8
+  HEADC(true, 25, 14, 4, 5)    // gpt2-xl fp8 (d 1600)
 #undef HEADC
   return -3;
 }
@@ -1284,7 +1289,7 @@ extern "C" int dnn_gemm_head(const void* A, int lda, const void* Wsh, const floa
   if (cus <= 0) return -1;
   int grid = (ntile16 + 7) / 8;
   grid = grid < cus ? grid : cus;
-  if ((long long)grid * 16 < ntile16 || grid > part_cap) return -1;  // at most two column tiles per wave
+  if ((long long)grid * HEAD_WAVES < ntile16 || grid > part_cap) return -1;  // a column tile a wave
   int rc;
   if (norm == NORM_LN)
     rc = launch_head<NORM_LN>(w8 != 0, nch, A, lda * 2, Wsh, sw, colsum, bias, eps, C, ldc, M, N, K, grid, part, st);

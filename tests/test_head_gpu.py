@@ -78,6 +78,34 @@ def test_head_matches_golden_and_unfused(M, K, N, w8, rms):
     assert torch.equal(o2, out)
 
 
+@pytest.mark.parametrize("M", [1, 16, 17])
+@pytest.mark.parametrize("K,N,w8", [(768, 16, False), (768, 1003, False), (1024, 33010, False), (1600, 50257, True),
+                                    (1280, 20481, True)])
+def test_head_row_tiles_and_waves(M, K, N, w8):
+    """One row tile (16 rows) and four, workgroups with 1 to 13 tiles, a ragged last one, and rows that are all -inf
+    (first index): logits against float64 on the weights as held, the ids against the logits."""
+    from distributed_neural_networks_amd.ops.gemm import HEAD_PART_PER_ROW, head_argmax
+    x, f, _ = _setup(M, K, N, w8, seed=N + M)
+    ldc = (N + 7) // 8 * 8
+    logits = torch.full((M, ldc), float("nan"), device=DEV, dtype=torch.bfloat16)
+    part = torch.empty(2 * HEAD_PART_PER_ROW * M, dtype=torch.int32, device=DEV)
+    out = torch.empty(M, dtype=torch.int32, device=DEV)
+    assert head_argmax(x, f, logits[:, :N], part, out)
+    wd = (f.w.q[:, :K].double() * f.w.scale[:, None].double()) if w8 else f.w.double()
+    xd = x.double()
+    xn = (xd - xd.mean(1, keepdim=True)) * torch.rsqrt(xd.var(1, unbiased=False, keepdim=True) + f.eps)
+    ref = xn @ wd.t() + f.bias.double()
+    # bf16 of the logit, and fp32 sums over the raw rows (their offset cancels: x W - mean colsum)
+    rstd = torch.rsqrt(xd.var(1, unbiased=False, keepdim=True) + f.eps)
+    bound = ref.abs() * 2.0 ** -8 + (xd.abs() @ wd.abs().t()) * rstd * K * 2.0 ** -24 + 2.0 ** -20
+    lg = logits[:, :N]
+    assert bool(((lg.double() - ref).abs() <= bound).all())
+    assert torch.equal(out, lg.float().argmax(1).int())
+    f.bias.fill_(float("-inf"))
+    assert head_argmax(x, f, logits[:, :N], part, out)
+    assert bool((out == 0).all())
+
+
 def test_head_ties_take_smallest_index():
     """Identical columns make exact ties across workgroups: the merge keeps the
     smallest index, as argmax_rows / numpy."""
