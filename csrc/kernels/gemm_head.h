@@ -123,8 +123,8 @@ __device__ __forceinline__ void head_amax(float& best, int& bi, float v, int i) 
   }
 }
 
-// NORM: 0 none, 1 RMSNorm, 2 LayerNorm (folded; colsum for LN).
-template <bool W8, int NORM, int MT, int NCH, int CPP, int GS>
+// NORM: 0 none, 1 RMSNorm, 2 LayerNorm (folded; colsum for LN).  MT: row tiles of 16, 1 or 4.
+template <bool W8, int NORM, int NCH, int CPP, int GS, int MT = 4>
 __global__ __launch_bounds__(HEAD_WAVES * 64, 1) void gemm_head_kernel(const uint8_t* __restrict__ A, int lda_b,
                                                            const uint8_t* __restrict__ Wsh,
                                                            const float* __restrict__ sw,
@@ -196,8 +196,7 @@ __global__ __launch_bounds__(HEAD_WAVES * 64, 1) void gemm_head_kernel(const uin
       glds16(A + (size_t)row * lda_b + kb, hd_lds + q * 1024);
     }
     if (ng > 1) head_wload<NCH, GS>(wb, Wsh, tile, pc0 + GS, pc1, lane);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ng > 1 ? GS : 0) : "memory");
-    __syncthreads();
+    __syncthreads();  // waits for all of them: an LDS-DMA is not ordered with plain loads behind it
 
     // statistics of this pass's K range
     if (stats) {

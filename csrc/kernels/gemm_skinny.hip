@@ -1239,7 +1239,7 @@ static int launch_head_cfg(const void* A, int lda_b, const void* Wsh, const floa
                            hipStream_t st) {
   constexpr size_t smem = HeadCfg<W8, MT, NCH, CPP, GS>::LDS;
   const int waves = std::max(2 * MT, ((N + 15) / 16 + grid - 1) / grid);  // <= HEAD_WAVES (dnn_gemm_head)
-  hipLaunchKernelGGL((gemm_head_kernel<W8, NORM, MT, NCH, CPP, GS>), dim3(grid), dim3(64 * waves), smem, st,
+  hipLaunchKernelGGL((gemm_head_kernel<W8, NORM, NCH, CPP, GS, MT>), dim3(grid), dim3(64 * waves), smem, st,
                      (const uint8_t*)A, lda_b, (const uint8_t*)Wsh, sw, colsum,
                      bias, eps, (bf16_t*)C, ldc, M, N, K, (int2*)part);
   return (int)hipGetLastError();
