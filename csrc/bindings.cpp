@@ -107,6 +107,24 @@ PYBIND11_MODULE(_dnn_hip, m) {
     return dnn_gemm_bf16_qkv_scatter(CP(A), lda, CP(W), ldw, CFP(bias), CFP(rowstat), CFP(colsum), P(q), P(kc), P(vc),
                                      CIP(pos), B, T, H, Hkv, hd, S, K, ST(st));
   });
+  m.def("gemm_takes_parts", [](int M, int N, int K, int act, int scatter, long long ws_bytes) {
+    return dnn_gemm_takes_parts(M, N, K, act, scatter, ws_bytes) != 0;
+  });
+  // (code, whether the output's partials were written)
+  m.def("gemm_bf16_parts", [](u64 A, int lda, u64 W, int ldw, u64 C, int ldc, u64 bias, u64 R, int ldr, int M, int N, int K,
+                              int act, u64 st, u64 wsh, int norm, float eps, u64 stats, u64 parts, u64 colsum,
+                              u64 parts_out, u64 ws, long long ws_bytes) {
+    int wrote = 0;
+    const int rc = dnn_gemm_bf16_parts(CP(A), lda, CP(W), ldw, P(C), ldc, CFP(bias), CP(R), ldr, M, N, K, act, ST(st), CP(wsh),
+                                       norm, eps, FP(stats), CP(parts), CFP(colsum), P(parts_out), &wrote, P(ws), ws_bytes);
+    return py::make_tuple(rc, wrote != 0);
+  });
+  m.def("gemm_bf16_qkv_scatter_parts", [](u64 A, int lda, u64 W, int ldw, u64 bias, int norm, float eps, u64 stats, u64 parts,
+                                          u64 colsum, u64 q, u64 kc, u64 vc, u64 pos, int B, int T, int H, int Hkv, int hd,
+                                          int S, int K, u64 st) {
+    return dnn_gemm_bf16_qkv_scatter_parts(CP(A), lda, CP(W), ldw, CFP(bias), norm, eps, FP(stats), CP(parts), CFP(colsum),
+                                           P(q), P(kc), P(vc), CIP(pos), B, T, H, Hkv, hd, S, K, ST(st));
+  });
   m.def("gemm_fp8_qkv_scatter", [](u64 A8, u64 sa, u64 W8, u64 sw, u64 bias, u64 q, u64 kc, u64 vc, u64 pos, int B,
                                    int T, int H, int Hkv, int hd, int S, int Kb, u64 st) {
     return dnn_gemm_fp8_qkv_scatter(CP(A8), CFP(sa), CP(W8), CFP(sw), CFP(bias), P(q), P(kc), P(vc), CIP(pos), B, T, H,
@@ -161,16 +179,17 @@ PYBIND11_MODULE(_dnn_hip, m) {
   });
 #ifdef DNN_HAVE_TRANSFORMER
   // blocks: 20 pointers each (qkv, o, up, down x weight, scale, bias, row sums, fragment copy); returns
-  // (code, launch that failed); -100: not a pass of this kind, nothing launched
+  // (code, launch that failed, whether the partials of the last rows were written); -100: not a pass of this kind, nothing launched
   m.def("prefill_blocks", [](const std::vector<int>& n, const std::vector<u64>& b, float eps, float scale,
                              long long kv_block, long long ws_bytes, u64 st,
                              const std::vector<u64>& blocks) -> py::tuple {
-    if (n.size() != 15 || b.size() != 19 || blocks.size() % 20 != 0)
+    if (n.size() != 17 || b.size() != 20 || blocks.size() % 20 != 0)
       throw std::runtime_error("prefill_blocks: ragged arguments");
     dnn::PrefillPass a{};
     int* dims[] = {&a.B, &a.T, &a.d, &a.H, &a.Hkv, &a.hd, &a.S, &a.ffn, &a.n_up, &a.act, &a.norm, &a.skinny_rows,
-                   &a.skinny_max, &a.fp8, &a.scatter};
-    for (size_t i = 0; i < n.size(); ++i) *dims[i] = n[i];
+                   &a.skinny_max, &a.fp8, &a.scatter, &a.more};
+    for (size_t i = 0; i < 16; ++i) *dims[i] = n[i];
+    a.have = n[16] != 0;
     void** bufs[] = {&a.h, &a.a, &a.qkv, &a.q, &a.att, &a.f, &a.q8, &a.sx, &a.q8b, &a.sxb, &a.ws};
     for (size_t i = 0; i < 11; ++i) *bufs[i] = P(b[i]);
     a.x = CP(b[11]);
@@ -181,6 +200,7 @@ PYBIND11_MODULE(_dnn_hip, m) {
     a.cosT = CFP(b[16]);
     a.sinT = CFP(b[17]);
     a.s8 = FP(b[18]);
+    a.parts = P(b[19]);
     a.eps = eps;
     a.scale = scale;
     a.kv_block = kv_block;
@@ -194,13 +214,13 @@ PYBIND11_MODULE(_dnn_hip, m) {
         *p[j] = {CP(w[0]), CFP(w[1]), CFP(w[2]), CFP(w[3]), CP(w[4])};
       }
     }
-    if (!a.covered()) return py::make_tuple(-100, "");
+    if (!a.covered()) return py::make_tuple(-100, "", false);
     int rc;
     {
       py::gil_scoped_release nogil;
       rc = a.run(L);
     }
-    return py::make_tuple(rc, a.what);
+    return py::make_tuple(rc, a.what, a.have);
   });
   m.def("row_stats", [](u64 x, int ldx, u64 stats, int M, int N, float eps, int rms, u64 st) {
     return dnn_row_stats(CP(x), ldx, FP(stats), M, N, eps, rms, ST(st));

@@ -64,6 +64,16 @@ int dnn_gemm_head(const void* A, int lda, const void* Wsh, const float* sw, cons
 // hist (optional, with pos_inc): hist[row * hist_ld + pos_inc[row]] = id before the advance (token history)
 int dnn_argmax_final(const void* part, int S, int M, int* out, int* out2, int* pos_inc, hipStream_t st,
                      int* hist = nullptr, int hist_ld = 0);
+// folded norm from partials of the row statistics, and partials of the output's (gemm_mid.h): whether a product of these
+// sizes reads them; the product; QKV scattered
+int dnn_gemm_takes_parts(int M, int N, int K, int act, int scatter, long long ws_bytes);
+int dnn_gemm_bf16_parts(const void* A, int lda, const void* W, int ldw, void* C, int ldc, const float* bias, const void* R,
+                        int ldr, int M, int N, int K, int act, hipStream_t st, const void* Wsh, int norm, float eps,
+                        float* stats, const void* parts, const float* colsum, void* parts_out, int* wrote, void* ws,
+                        long long ws_bytes);
+int dnn_gemm_bf16_qkv_scatter_parts(const void* A, int lda, const void* W, int ldw, const float* bias, int norm, float eps,
+                                    float* stats, const void* parts, const float* colsum, void* q, void* kc, void* vc,
+                                    const int* pos, int B, int T, int H, int Hkv, int hd, int S, int K, hipStream_t st);
 // prefill: 256^2 + 256x128 tail split (gemm_bf16.hip launch_gemm)
 int dnn_gemm_set_split_tail(int on);
 // MX-scaled W8A8 prefill (e8m0 per (row, 128 columns), common.h mx_index)

@@ -567,6 +567,20 @@ extern "C" int dnn_gemm_set_half_cost(float c) {
   return 0;
 }
 
+// Partials of the row statistics for one call (dnn_gemm_bf16_parts, its scatter): what launch_gemm shall read in
+// place of rowstat and write beside C; `wrote`: it did.
+struct PartsReq {
+  const float2* in = nullptr;
+  float2* out = nullptr;
+  float eps = 0.f;
+  int rms = 0, wrote = 0;
+};
+static thread_local PartsReq g_parts;
+struct PartsScope {
+  explicit PartsScope(const PartsReq& r) { g_parts = r; }
+  ~PartsScope() { g_parts = PartsReq{}; }
+};
+
 // Rows that 16-byte LDS-DMA may fetch.
 static bool dma_rows(const void* A, int lda, const void* W, int ldw) {
   return (((uintptr_t)A | (uintptr_t)W) & 15) == 0 && lda % 8 == 0 && ldw % 8 == 0;
@@ -582,7 +596,7 @@ static int launch_gemm(const void* A, int lda, const void* W, int ldw, void* C, 
   const long long part_bytes = mid_ws(ws, ws_bytes);
   // up to 256 rows what the small tiles cannot stage (dma_rows) goes to the decode kernels, whose loads are plain
   const bool narrow = lda < 1 << 23 && ldw < 1 << 23;  // the small tiles address a tile's rows with 32 bits
-  if (rowstat == nullptr && (skinny(M, N, K, false, Wsh != nullptr, part_bytes) ||
+  if (rowstat == nullptr && g_parts.in == nullptr && (skinny(M, N, K, false, Wsh != nullptr, part_bytes) ||
                              (M <= 256 && (!narrow || !dma_rows(A, lda, W, ldw))))) {
     return dnn_gemm_skinny(A, lda, nullptr, W, ldw, nullptr, C, ldc, bias, R, ldr, M, N, K, ACT, F32 ? 1 : 0, 0, st, Wsh,
                            ws, ws_bytes);
@@ -597,7 +611,13 @@ static int launch_gemm(const void* A, int lda, const void* W, int ldw, void* C, 
     plan = mid_plan(M, N, K, part_bytes, has_consts(ACT) ? MID_BF16_WHOLE : MID_BF16);  // constants lie behind all N
   if (plan.tile >= 0) {
     MidArgs a{{C, bias, (const bf16_t*)R, ldc, ldr, M, N, ACT, F32 ? 1 : 0}, (const bf16_t*)A, (const bf16_t*)W,
-              rowstat, colsum, (float*)ws, lda, ldw, K, plan.splits};
+              rowstat, colsum, nullptr, g_parts.in, g_parts.eps, g_parts.rms, (float*)ws, lda, ldw, K, plan.splits};
+    // partials beside rows that leave as pairs of 16-byte stores with a residual (mid_rows)
+    if (g_parts.out != nullptr && !F32 && ACT == ACT_NONE && R != nullptr && plan.cols == 0 && N % MID_PARTS_N == 0 &&
+        (((uintptr_t)C | (uintptr_t)R | (uintptr_t)bias) & 15) == 0 && ldc % 8 == 0 && ldr % 8 == 0) {
+      a.parts_out = g_parts.out;
+      g_parts.wrote = 1;
+    }
     if (const int n = plan.cols) {  // disjoint columns
       hipLaunchKernelGGL((gemm_bf16_256_kernel<ACT, F32>), dim3(((M + BG_M - 1) / BG_M) * (n / BG_N)), dim3(512), 0, st,
                          a.A, lda, a.W, ldw, C, ldc, bias, a.R, ldr, M, n, K, g_res_prefetch, rowstat, colsum);
@@ -655,7 +675,7 @@ extern "C" int dnn_gemm_bf16(const void* A, int lda, const void* W, int ldw, voi
                              const void* Wsh, const float* rowstat, const float* colsum, void* ws,
                              long long ws_bytes) {
   if (K % 64 != 0 || M <= 0 || N <= 0) return -1;
-  if (colsum != nullptr && rowstat == nullptr) return -1;
+  if (colsum != nullptr && rowstat == nullptr && g_parts.in == nullptr) return -1;
   const float2* rs = reinterpret_cast<const float2*>(rowstat);
 #define DISPATCH(a)                                                                                  \
   if (act == a) {                                                                                    \
@@ -684,6 +704,57 @@ extern "C" int dnn_gemm_bf16(const void* A, int lda, const void* W, int ldw, voi
 }
 
 #ifndef DNN_DECODER_ONLY
+// Whether a folded norm of these sizes can take its statistics from partials: one launch of the small tiles, K whole.
+static bool takes_parts(int M, int N, int K, long long part_bytes, int act, bool scatter) {
+  if (g_gemm_tile != 0 || K % 64 != 0 || K > MID_PARTS_K) return false;
+  if (scatter && tail_split_cols(M, N) != 0) return false;
+  if (g_mid_tile >= 0) return scatter || g_mid_splits == 1;
+  if (!is_glu(act) && tail_split_cols(M, N) != 0) return false;
+  const MidPlan p = mid_plan(M, N, K, scatter ? 0 : part_bytes, scatter || has_consts(act) ? MID_BF16_WHOLE : MID_BF16);
+  return p.tile >= 0 && p.cols == 0 && p.splits == 1;
+}
+
+extern "C" int dnn_gemm_takes_parts(int M, int N, int K, int act, int scatter, long long ws_bytes) {
+  return takes_parts(M, N, K, ws_bytes - 4096, act, scatter != 0);
+}
+
+// GPT-2, 3 x 357 tokens: a statistics launch of 3.4 us ahead of every c_attn and c_fc, 784 a pass; as partials, which
+// cost their writers 0.2 and their readers 0.6 each, 749.  Rows wider than MID_PARTS_K keep the launch: the
+// partials of 4096 columns are as many bytes a workgroup as two of its K-tiles, and 700 rows' launch is 5 of 340 a block.
+// dnn_gemm_bf16 with a folded norm (norm 1 RMS, 2 LayerNorm, 0 none) whose statistics come from `parts` (partials of A's
+// rows, [M][K / 32]) where these sizes take them, else from a pass over A into `stats`; the partials
+// of C's rows go to `parts_out` (null: none) where they can, `wrote` says whether.
+extern "C" int dnn_gemm_bf16_parts(const void* A, int lda, const void* W, int ldw, void* C, int ldc, const float* bias,
+                                   const void* R, int ldr, int M, int N, int K, int act, hipStream_t st, const void* Wsh,
+                                   int norm, float eps, float* stats, const void* parts, const float* colsum,
+                                   void* parts_out, int* wrote, void* ws, long long ws_bytes) {
+  const bool read = norm != 0 && parts != nullptr && takes_parts(M, N, K, mid_ws(ws, ws_bytes), act, false);
+  *wrote = 0;
+  if (norm != 0 && !read) {
+    if (stats == nullptr) return -1;
+    if (const int rc = dnn_row_stats(A, lda, stats, M, K, eps, norm == 1, st)) return rc;
+  }
+  PartsScope scope({read ? (const float2*)parts : nullptr, (float2*)parts_out, eps, norm == 1, 0});
+  const int rc = dnn_gemm_bf16(A, lda, W, ldw, C, ldc, bias, R, ldr, M, N, K, act, 0, st, Wsh,
+                               norm != 0 && !read ? stats : nullptr, norm != 0 ? colsum : nullptr, ws, ws_bytes);
+  *wrote = g_parts.wrote;
+  return rc;
+}
+
+extern "C" int dnn_gemm_bf16_qkv_scatter_parts(const void* A, int lda, const void* W, int ldw, const float* bias, int norm,
+                                               float eps, float* stats, const void* parts, const float* colsum, void* q,
+                                               void* kc, void* vc, const int* pos, int B, int T, int H, int Hkv, int hd,
+                                               int S, int K, hipStream_t st) {
+  const int N = (H + 2 * Hkv) * hd;
+  const bool read = parts != nullptr && N % 32 == 0 && takes_parts(B * T, N, K, 0, ACT_NONE, true);
+  if (!read) {
+    if (const int rc = dnn_row_stats(A, lda, stats, B * T, K, eps, norm == 1, st)) return rc;
+  }
+  PartsScope scope({read ? (const float2*)parts : nullptr, nullptr, eps, norm == 1, 0});
+  return dnn_gemm_bf16_qkv_scatter(A, lda, W, ldw, bias, read ? nullptr : stats, colsum, q, kc, vc, pos, B, T, H, Hkv, hd, S,
+                                   K, st);
+}
+
 extern "C" int dnn_silu_mul_packed(const void* gu, int ld_in, void* out, int ld_out, int M, int F, hipStream_t st) {
   const int n = M * F;
   hipLaunchKernelGGL(silu_mul_packed_kernel, dim3((n + 255) / 256), dim3(256), 0, st, (const bf16_t*)gu, ld_in,
@@ -701,7 +772,7 @@ extern "C" int dnn_gemm_bf16_qkv_scatter(const void* A, int lda, const void* W, 
                                          const int* pos, int B, int T, int H, int Hkv, int hd, int S, int K,
                                          hipStream_t st) {
   const int M = B * T, N = (H + 2 * Hkv) * hd;
-  if (K % 64 != 0 || M <= 0 || hd % 8 != 0 || (colsum != nullptr && rowstat == nullptr)) return -1;
+  if (K % 64 != 0 || M <= 0 || hd % 8 != 0 || (colsum != nullptr && rowstat == nullptr && g_parts.in == nullptr)) return -1;
   if (N % 32 != 0 || ((uintptr_t)bias & 15) != 0 || (M < 256 && !dma_rows(A, lda, W, ldw))) return -3;
   const int tiles = ((M + BG_M - 1) / BG_M) * ((N + BG_N - 1) / BG_N);
   if ((hd & (hd - 1)) != 0 || M >= (1 << 24)) return -3;
@@ -711,7 +782,8 @@ extern "C" int dnn_gemm_bf16_qkv_scatter(const void* A, int lda, const void* W, 
     if (g_mid_tile >= 0) plan.tile = g_mid_tile;
     if (plan.tile >= 0) {
       const MidArgs a{{q, bias, nullptr, hd, 0, M, N, ACT_NONE, 0}, (const bf16_t*)A, (const bf16_t*)W,
-                      reinterpret_cast<const float2*>(rowstat), colsum, nullptr, lda, ldw, K, 1};
+                      reinterpret_cast<const float2*>(rowstat), colsum, nullptr, g_parts.in, g_parts.eps, g_parts.rms,
+                      nullptr, lda, ldw, K, 1};
       return mid_launch(plan.tile, a, &sc, st);
     }
   }

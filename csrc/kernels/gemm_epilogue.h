@@ -283,7 +283,7 @@ __device__ __forceinline__ void epi_pair_bf16(f32x4 a0, f32x4 a1, int m, int nb,
                                               int ldc, const float* __restrict__ bias,
                                               const bf16_t* __restrict__ R, int ldr, int lane,
                                               bf16x4 rp0 = bf16x4{}, bf16x4 rp1 = bf16x4{},
-                                              const f32x2& xc = f32x2{}) {
+                                              const f32x2& xc = f32x2{}, uint4* stored = nullptr) {
   const int q = lane >> 4;
   const int n0 = nb + q * 4, n1 = n0 + 16;
   if (bias != nullptr) {
@@ -319,6 +319,7 @@ __device__ __forceinline__ void epi_pair_bf16(f32x4 a0, f32x4 a1, int m, int nb,
   }
   uint32_t x0 = pack2bf(a0[0], a0[1]), x1 = pack2bf(a0[2], a0[3]);
   uint32_t y0 = pack2bf(a1[0], a1[1]), y1 = pack2bf(a1[2], a1[3]);
+  if (stored != nullptr) *stored = make_uint4(x0, x1, y0, y1);
   const auto s0 = __builtin_amdgcn_permlane16_swap(x0, y0, false, false);
   const auto s1 = __builtin_amdgcn_permlane16_swap(x1, y1, false, false);
   if (m >= M) return;

@@ -194,6 +194,84 @@ struct MidSource {
   }
 };
 
+// {mean, sum of squared deviations} of 32 stored columns of a row, 8 of them in each of the lanes l, l ^ 16, l ^ 32, l ^ 48.
+__device__ __forceinline__ void mid_part_out(const uint4& x, int m, int nb, const MidRows& p, float2* out, int lane) {
+  const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+  float v[8], s = 0.f, q = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    v[i] = __uint_as_float(i & 1 ? w[i >> 1] & 0xffff0000u : w[i >> 1] << 16);
+    s += v[i];
+  }
+  const float mean = add32(add16(s)) * (1.f / 32.f);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) q = fmaf(v[i] - mean, v[i] - mean, q);
+  q = add32(add16(q));
+  if (lane < 16 && m < p.M) out[(size_t)m * (p.N >> 5) + (nb >> 5)] = make_float2(mean, q);
+}
+
+// The rows' {rstd, -mean rstd} from their partials, TPR lanes a row and two partials a load.  As rowstat_merge
+// (gemm_epilogue.h): shifted by the first partial's mean, so that no |mean| / std cancels.  load() ahead of the first
+// requests, merge() behind them; the rows go to their lanes by way of LDS: behind the K-tiles where there is room
+// (written ahead of the loop's first barrier), else where they were, behind the loop.
+template <class T>
+struct MidParts {
+  static constexpr int TPR = T::THREADS / T::BM >= 4 ? 4 : 2, B = 4;  // lanes a row, loads a lane and batch
+  static constexpr int TILES = T::S * T::STAGE;
+  static constexpr bool ROOM = TILES + T::BM * 8 <= 160 * 1024;
+  static constexpr int LDS = TILES + (ROOM ? T::BM * 8 : 0);
+  f32x4 p[B];
+  float2 r;
+  const f32x4* row;
+  int n2, sub;
+  __device__ __forceinline__ void batch(int b) {
+#pragma unroll
+    for (int i = 0; i < B; ++i) p[i] = row[min(sub + (b + i) * TPR, n2 - 1)];
+  }
+  __device__ __forceinline__ void load(const MidArgs& a, int m0, int tid) {
+    n2 = a.K >> 6, sub = tid % TPR;
+    row = reinterpret_cast<const f32x4*>(a.parts) + (size_t)min(m0 + min(tid / TPR, T::BM - 1), a.M - 1) * n2;
+    batch(0);
+  }
+  __device__ __forceinline__ void put(char* lds, int tid) const {
+    if (sub == 0 && tid / TPR < T::BM) reinterpret_cast<float2*>(lds)[tid / TPR] = r;
+  }
+  __device__ __forceinline__ void merge(const MidArgs& a, char* lds, int tid) {
+    const float c = a.rms ? 0.f : dpp_f<TPR == 4 ? 0x00 : 0xA0>(p[0][0]);  // quad_perm: the row's first lane
+    float s1 = 0.f, s2 = 0.f, sm = 0.f;
+    for (int b = 0;; b += B) {
+#pragma unroll
+      for (int i = 0; i < B; ++i) {
+        const bool in = sub + (b + i) * TPR < n2;
+        const float d = in ? p[i][0] - c : 0.f, e = in ? p[i][2] - c : 0.f;
+        s1 += d + e;
+        s2 = fmaf(d, d, fmaf(e, e, s2));
+        sm += in ? p[i][1] + p[i][3] : 0.f;
+      }
+      if ((b + B) * TPR >= n2) break;  // uniform
+      batch(b + B);
+    }
+    s1 = group_sum<TPR>(s1) * 32.f;
+    s2 = group_sum<TPR>(s2) * 32.f;
+    sm = group_sum<TPR>(sm);
+    const float invk = 1.f / (float)a.K, d = a.rms ? 0.f : s1 * invk;
+    const float rstd = rsqrtf(fmax_nan((sm + s2) * invk - d * d, 0.f) + a.eps);
+    r = make_float2(rstd, a.rms ? 0.f : -(c + d) * rstd);
+    if constexpr (ROOM) put(lds + TILES, tid);
+  }
+  template <int I>
+  __device__ __forceinline__ void share(char* lds, int tid, int row0, float2 (&rs)[I]) const {
+    if constexpr (!ROOM) {
+      __syncthreads();
+      put(lds, tid);
+      __syncthreads();
+    }
+    const float2* st = reinterpret_cast<const float2*>(lds + (ROOM ? TILES : 0));
+#pragma unroll
+    for (int i = 0; i < I; ++i) rs[i] = st[row0 + i * 16];
+  }
+};
+
 // A wave's accumulators to head-major q / K / V (host: N % 32 == 0).
 template <int I, int J>
 __device__ __forceinline__ void mid_scatter(f32x4 (&acc)[I][J], int mw, int nw, int M, int N, const float* bias,
@@ -216,7 +294,7 @@ __device__ __forceinline__ void mid_scatter(f32x4 (&acc)[I][J], int mw, int nw, 
 // ALL: with fp32 rows and the activations that only bf16 weights have.
 template <int I, int J, bool ALL = true>
 __device__ __forceinline__ void mid_rows(f32x4 (&acc)[I][J], int mw, int nw, int lane, const MidRows& p,
-                                         const MidPre<I, J>& pre) {
+                                         const MidPre<I, J>& pre, float2* parts_out = nullptr) {
   const int M = p.M, N = p.N, fg = lane >> 4;
   const bool f32 = ALL && p.f32;
   const bool vec = epi_vec_ok(p.C, p.ldc, p.bias, p.R, p.ldr);
@@ -240,9 +318,12 @@ __device__ __forceinline__ void mid_rows(f32x4 (&acc)[I][J], int mw, int nw, int
 #pragma unroll
     for (int i = 0; i < (MidPre<I, J>::RES ? I : 1); ++i)
 #pragma unroll
-      for (int jp = 0; jp < J / 2; ++jp)
+      for (int jp = 0; jp < J / 2; ++jp) {
+        uint4 x;
         epi_pair_bf16<ACT_NONE, true>(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, nw + jp * 32, M, C, p.ldc, nullptr,
-                                      p.R, p.ldr, lane, pre.rr[i][jp][0], pre.rr[i][jp][1]);
+                                      p.R, p.ldr, lane, pre.rr[i][jp][0], pre.rr[i][jp][1], f32x2{}, &x);
+        if (parts_out != nullptr) mid_part_out(x, mw + i * 16, nw + jp * 32, p, parts_out, lane);
+      }
   } else if (!MidPre<I, J>::RES && pair && p.R != nullptr) {  // every residual load before the first output
     bf16x4 rr[I][J / 2][2];
 #pragma unroll
@@ -253,9 +334,12 @@ __device__ __forceinline__ void mid_rows(f32x4 (&acc)[I][J], int mw, int nw, int
 #pragma unroll
     for (int i = 0; i < I; ++i)
 #pragma unroll
-      for (int jp = 0; jp < J / 2; ++jp)
+      for (int jp = 0; jp < J / 2; ++jp) {
+        uint4 x;
         epi_pair_bf16<ACT_NONE, true>(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, nw + jp * 32, M, C, p.ldc, nullptr,
-                                      p.R, p.ldr, lane, rr[i][jp][0], rr[i][jp][1]);
+                                      p.R, p.ldr, lane, rr[i][jp][0], rr[i][jp][1], f32x2{}, &x);
+        if (parts_out != nullptr) mid_part_out(x, mw + i * 16, nw + jp * 32, p, parts_out, lane);
+      }
   } else if (pair) {
 #pragma unroll
     for (int i = 0; i < I; ++i)
@@ -290,8 +374,13 @@ __device__ __forceinline__ void mid_rows(f32x4 (&acc)[I][J], int mw, int nw, int
 // place of 64 x 64, or padded rows did not change that.
 //
 // T::PW > 0: other waves stage, and `src` only says where (mid_stage keeps the same barriers).
-template <class T>
-__device__ __forceinline__ void mid_loop(const MidSource<T>& src, int wm, int wn, int lane, f32x4 (&acc)[T::I][T::J]) {
+// `behind`: run behind the first requests.
+struct MidNone {
+  __device__ __forceinline__ void operator()() const {}
+};
+template <class T, class F = MidNone>
+__device__ __forceinline__ void mid_loop(const MidSource<T>& src, int wm, int wn, int lane, f32x4 (&acc)[T::I][T::J],
+                                         F behind = F{}) {
   constexpr bool OWN = T::PW == 0;
   constexpr int I = T::I, J = T::J, S = T::S, L = T::PA + T::PB;
   // fragment reads: lane (r, g) reads 16 B of row r at chunks g and 4 + g
@@ -324,6 +413,7 @@ __device__ __forceinline__ void mid_loop(const MidSource<T>& src, int wm, int wn
   if constexpr (OWN) {
 #pragma unroll
     for (int q = 0; q < S - 1; ++q) src.stage(q, q, 0, 1);
+    behind();
     __builtin_amdgcn_s_waitcnt(wait_imm((S - 2) * L, 0));
   }
   bg_barrier();
@@ -377,12 +467,14 @@ __device__ __forceinline__ void mid_stage(const MidSource<T>& src) {
 
 enum MidOut { MID_ROWS = 0, MID_SCATTER = 1, MID_PART = 2 };
 
-template <class T, MidOut OUT>
+// MERGE: the folded norm's statistics from partials (a variant of its own: a load under a branch is waited for where
+// the branch ends, ahead of the first request)
+template <class T, MidOut OUT, bool MERGE>
 __global__ __launch_bounds__(T::THREADS, 2) void gemm_mid_kernel(MidArgs p, QkvScatter scat) {
   constexpr bool PART = OUT == MID_PART;
-  static_assert(PART || T::PW == 0, "");
+  static_assert(PART ? !MERGE : T::PW == 0, "");
   constexpr int I = T::I, J = T::J;
-  // S * STAGE bytes, given at launch: with the size in the kernel the compiler sees one
+  // S * STAGE bytes (MERGE: MidParts::LDS), given at launch: with the size in the kernel the compiler sees one
   // wave per SIMD and moves accumulators of the four-wave tiles to AGPRs and back in
   // the loop (a tile of 192 x 128 rows at 700 x 6144 x 4096: 47 -> 78 us)
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -417,7 +509,14 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_mid_kernel(MidArgs p, QkvS
   MidPre<I, J> pre;
   if constexpr (!PART) pre.load(p, p.rowstat, p.colsum, mw, nw, lane, OUT == MID_ROWS);
   f32x4 acc[I][J];
-  mid_loop<T>(src, wm, wn, lane, acc);
+  MidParts<T> parts;
+  if constexpr (MERGE) {
+    parts.load(p, m0, tid);
+    mid_loop<T>(src, wm, wn, lane, acc, [&]() { parts.merge(p, smem, tid); });
+    parts.share(smem, tid, wm * (I * 16) + fr, pre.rs);
+  } else {
+    mid_loop<T>(src, wm, wn, lane, acc);
+  }
 
   if constexpr (PART) {
     float* d = p.part + (size_t)sp * M * N;
@@ -432,14 +531,14 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_mid_kernel(MidArgs p, QkvS
     }
     return;
   }
-  if (p.rowstat != nullptr) {  // the folded norm, in the 256 x 256 kernel's order of operations
+  if (MERGE || p.rowstat != nullptr) {  // the folded norm, in the 256 x 256 kernel's order of operations
 #pragma unroll
     for (int i = 0; i < I; ++i)
 #pragma unroll
       for (int j = 0; j < J; ++j) acc[i][j] = acc[i][j] * pre.rs[i].x + pre.rs[i].y * pre.cs[j];
   }
   if constexpr (OUT == MID_SCATTER) mid_scatter<I, J>(acc, mw, nw, M, N, p.bias, pre.bs, lane, scat);
-  else mid_rows<I, J>(acc, mw, nw, lane, p, pre);
+  else mid_rows<I, J>(acc, mw, nw, lane, p, pre, p.parts_out);
 }
 
 // Sum of the parts and the epilogue.  A thread: 4 columns of one row (gated: 4
@@ -472,6 +571,15 @@ __global__ __launch_bounds__(256) void gemm_mid_reduce(MidArgs p) {
   f32x4 a[1][1] = {{v}};
   const f32x4 b[1] = {p.bias != nullptr ? mid_cols(p.bias, n, N) : f32x4{0.f, 0.f, 0.f, 0.f}};
   mid_bias_act<1, 1>(a, p.bias, b, p.act, N);
+  if (p.parts_out != nullptr) {  // host: bf16, whole groups of 8 threads
+    f32x4 x;
+    epi_t4<ACT_NONE, false>(a[0][0], m, n, M, N, p.C, p.ldc, nullptr, p.R, p.ldr, vec, nullptr, 1.f, &x);
+    const float mean = group_sum<8>(x[0] + x[1] + (x[2] + x[3])) * (1.f / 32.f);
+    x -= mean;
+    const float s = group_sum<8>(x[0] * x[0] + x[1] * x[1] + (x[2] * x[2] + x[3] * x[3]));
+    if ((threadIdx.x & 7) == 0) p.parts_out[(size_t)m * (N >> 5) + (n >> 5)] = make_float2(mean, s);
+    return;
+  }
   epi_t4_any(a[0][0], m, n, M, N, p, p.R, vec);
 }
 

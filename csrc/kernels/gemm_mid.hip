@@ -117,19 +117,25 @@ bool mid_skinny(int M, int N, int K, bool norm, bool frag, long long ws_bytes) {
          mid_plan(M, N, K, ws_bytes, MID_BF16).us + (norm ? 3.3f : 0.f);
 }
 
-template <class T, MidOut OUT>
+template <class T, MidOut OUT, bool MERGE = false>
 static int start(const MidArgs& a, const QkvScatter& scat, hipStream_t st) {
-  constexpr int LDS = T::S * T::STAGE;
+  constexpr int LDS = MERGE ? MidParts<T>::LDS : T::S * T::STAGE;
   static const hipError_t room =
-      hipFuncSetAttribute((const void*)gemm_mid_kernel<T, OUT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+      hipFuncSetAttribute((const void*)gemm_mid_kernel<T, OUT, MERGE>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   if (room != hipSuccess) return (int)room;
   const int tiles = ((a.M + T::BM - 1) / T::BM) * ((a.N + T::BN - 1) / T::BN);
-  hipLaunchKernelGGL((gemm_mid_kernel<T, OUT>), dim3(tiles * a.splits), dim3(T::THREADS), LDS, st, a, scat);
+  hipLaunchKernelGGL((gemm_mid_kernel<T, OUT, MERGE>), dim3(tiles * a.splits), dim3(T::THREADS), LDS, st, a, scat);
   return (int)hipGetLastError();
 }
 
 template <class T>
 static int launch(const MidArgs& a, const QkvScatter* scat, hipStream_t st) {
+#ifndef DNN_DECODER_ONLY
+  if (a.parts != nullptr) {
+    if (a.splits != 1) return -1;
+    return scat != nullptr ? start<T, MID_SCATTER, true>(a, *scat, st) : start<T, MID_ROWS, true>(a, QkvScatter{}, st);
+  }
+#endif
   if (scat != nullptr) return start<T, MID_SCATTER>(a, *scat, st);
   if (a.splits == 1) return start<T, MID_ROWS>(a, QkvScatter{}, st);
   if (const int rc = start<typename MidSplit<T>::type, MID_PART>(a, QkvScatter{}, st)) return rc;

@@ -18,6 +18,12 @@ struct MidArgs : MidRows {
   const bf16_t* W;
   const float2* rowstat;
   const float* colsum;
+  // Row statistics by way of partials {mean, sum of squared deviations} of 32 columns of a row: written with the
+  // bf16 output [M][N / 32], or read for the folded norm instead of rowstat [M][K / 32]
+  float2* parts_out;
+  const float2* parts;
+  float eps;
+  int rms;
   float* part;  // splits > 1: fp32 parts [splits][M][N]
   int lda, ldw, K, splits;
 };
@@ -39,6 +45,8 @@ MidPlan mid_plan(int M, int N, int K, long long ws_bytes, unsigned kind);
 bool mid_skinny(int M, int N, int K, bool norm, bool frag, long long ws_bytes);
 // Bytes of a decode workspace that parts may use: its last 4 KiB hold the decode stream kernel's tickets.
 inline long long mid_ws(const void* ws, long long bytes) { return ws == nullptr ? 0 : bytes - 4096; }
+// Widest rows whose partials a workgroup merges, and what the columns of a product with partials divide by.
+constexpr int MID_PARTS_K = 2048, MID_PARTS_N = 64;
 int mid_launch(int tile, const MidArgs& a, const QkvScatter* scat, hipStream_t st);  // a.splits workgroups over K
 
 }  // namespace dnn

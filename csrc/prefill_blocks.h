@@ -34,6 +34,7 @@ struct PrefillPass {
   void *h, *a, *qkv, *q, *att, *f;
   void *q8, *sx, *q8b, *sxb;    // fp8: MX activations and scales, those of the c_fc output
   float* s8;                    // fp8: row scales of activations that are not MX
+  void* parts;                  // partials of the row statistics of h, [rows][d / 32], or null
   const float* ones;
   char *kc, *vc;                // this stage's caches at the first sequence, one block's bytes apart
   long long kv_block;
@@ -42,6 +43,8 @@ struct PrefillPass {
   void* ws;
   long long ws_bytes;
   hipStream_t st;
+  int more;                     // another call runs the blocks behind these
+  bool have;                    // `parts` holds the partials of x; after run(), of h
   const char* what = "";
 
   int rows() const { return B * T; }
@@ -55,10 +58,6 @@ struct PrefillPass {
   }
   bool mx(int N) const { return rows() >= 256 && N >= 256; }
 
-  int stats(const void* in) {
-    what = "row_stats";
-    return dnn_row_stats(in, d, (float*)a, rows(), d, eps, norm == 1, st);
-  }
   int quant_norm(const void* in) {
     what = "layernorm_q8_mx";
     return dnn_layernorm_q8_mx(in, d, ones, nullptr, q8, kpad(d), sx, rows(), d, kpad(d), eps, norm == 1, st);
@@ -88,19 +87,24 @@ struct PrefillPass {
       return dnn_gemm_fp8_mx(q8, sx, p.w, p.scale, out, ldo, p.bias, nullptr, 0, M, N, kpad(d), act_,
                              quant ? q8b : nullptr, quant ? kpad(N) : 0, quant ? sxb : nullptr, quant ? kpad(N) : 0, st);
     }
-    if (const int rc = stats(in)) return rc;
-    what = "gemm_bf16";
-    return dnn_gemm_bf16(in, d, p.w, d, out, ldo, p.bias, nullptr, 0, M, N, d, act_, 0, st, nullptr, (const float*)a,
-                         p.colsum, ws, ws_bytes);
+    what = "gemm_bf16_parts";
+    int wrote;
+    return dnn_gemm_bf16_parts(in, d, p.w, d, out, ldo, p.bias, nullptr, 0, M, N, d, act_, st, nullptr, norm, eps,
+                               (float*)a, have ? parts : nullptr, p.colsum, nullptr, &wrote, ws, ws_bytes);
   }
 
-  // h = in W^T + bias + res, in (rows, K); quantised: in lies in q8b / sxb already
-  int res_proj(const void* in, const PrefillProj& p, const void* res, int K, bool quantised) {
+  // h = in W^T + bias + res, in (rows, K); quantised: in lies in q8b / sxb already; read: the next projection
+  // takes h's partials (`have`: they were written)
+  int res_proj(const void* in, const PrefillProj& p, const void* res, int K, bool quantised, bool read) {
     const int M = rows();
+    have = false;
     if (!fp8) {
-      what = "gemm_bf16";
-      return dnn_gemm_bf16(in, K, p.w, K, h, d, p.bias, res, d, M, d, K, 0, 0, st, p.frag, nullptr, nullptr, ws,
-                           ws_bytes);
+      what = "gemm_bf16_parts";
+      int wrote = 0;
+      const int rc = dnn_gemm_bf16_parts(in, K, p.w, K, h, d, p.bias, res, d, M, d, K, 0, st, p.frag, 0, 0.f, nullptr,
+                                         nullptr, nullptr, read ? parts : nullptr, &wrote, ws, ws_bytes);
+      have = wrote != 0;
+      return rc;
     }
     if (skinny(d, K, false, true, ws_bytes)) {
       what = "gemm_skinny_w8";
@@ -128,10 +132,9 @@ struct PrefillPass {
       rc = dnn_gemm_fp8_qkv_scatter_mx(q8, sx, p.w, p.scale, p.bias, q, k, v, pos, B, T, H, Hkv, hd, S, kpad(d), st);
       return 1;
     }
-    if ((rc = stats(in))) return 0;
-    what = "gemm_bf16_qkv_scatter";
-    rc = dnn_gemm_bf16_qkv_scatter(in, d, p.w, d, p.bias, (const float*)a, p.colsum, q, k, v, pos, B, T, H, Hkv, hd, S,
-                                   d, st);
+    what = "gemm_bf16_qkv_scatter_parts";
+    rc = dnn_gemm_bf16_qkv_scatter_parts(in, d, p.w, d, p.bias, norm, eps, (float*)a, have ? parts : nullptr, p.colsum, q, k,
+                                         v, pos, B, T, H, Hkv, hd, S, d, st);
     if (rc == -3) {  // off the tiles with the scatter epilogue: projection rows instead
       rc = 0;
       return 0;
@@ -154,6 +157,9 @@ struct PrefillPass {
     const int nq = (H + 2 * Hkv) * hd;
     const int one_group = fp8 && rows() > skinny_max;  // e4m3 activations follow (attention.hip flash_two_groups)
     const bool up_quant = fp8 && act == 2 && !skinny(n_up, d, true, true, 0);
+    const bool part = parts != nullptr && !fp8;  // who reads h's partials
+    const bool read_up = part && dnn_gemm_takes_parts(rows(), n_up, d, act, 0, ws_bytes);
+    const bool read_qkv = part && scatter && cosT == nullptr && dnn_gemm_takes_parts(rows(), nq, d, 0, 1, 0);
     for (size_t i = 0; i < blocks.size(); ++i) {
       const PrefillBlock& L = blocks[i];
       void *k = kc + i * kv_block, *v = vc + i * kv_block;
@@ -176,9 +182,9 @@ struct PrefillPass {
         }
       }
       if (rc) return rc;
-      if ((rc = res_proj(att, L.o, in, H * hd, false))) return rc;
+      if ((rc = res_proj(att, L.o, in, H * hd, false, read_up))) return rc;
       if ((rc = norm_proj(h, L.up, f, ffn, n_up, act, false, up_quant))) return rc;
-      if ((rc = res_proj(f, L.down, h, ffn, up_quant))) return rc;
+      if ((rc = res_proj(f, L.down, h, ffn, up_quant, read_qkv && (more || i + 1 < blocks.size())))) return rc;
       in = h;
     }
     return 0;

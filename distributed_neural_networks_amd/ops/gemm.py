@@ -162,18 +162,34 @@ def _ws_args(ws: Optional[torch.Tensor]):
     return (0, 0) if ws is None else (ws.data_ptr(), ws.nbytes)
 
 
+def parts_buffer(rows: int, width: int, device) -> Optional[torch.Tensor]:
+    """Partials of the row statistics of prefill activations, {mean, sum of squared deviations} of 32 columns: written
+    by the projection that makes the rows and merged by the next folded norm (gemm_mid.h).  None for widths without."""
+    if width % 64 or width > 2048:
+        return None
+    return torch.empty((rows, width // 16), dtype=torch.float32, device=device)
+
+
+def takes_parts(M: int, N: int, K: int, act: int = 0, ws: Optional[torch.Tensor] = None, scatter: bool = False) -> bool:
+    """Whether a folded norm of these sizes merges partials (else it needs ``row_stats``)."""
+    return bool(lib().gemm_takes_parts(M, N, K, act, int(scatter), 0 if ws is None else ws.nbytes))
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, act=None,
            residual: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None,
            out_dtype: torch.dtype = torch.bfloat16, w_shuf: Optional[torch.Tensor] = None,
            rowstat: Optional[torch.Tensor] = None, colsum: Optional[torch.Tensor] = None,
-           ws: Optional[torch.Tensor] = None, rs_out: Optional[torch.Tensor] = None) -> torch.Tensor:
+           ws: Optional[torch.Tensor] = None, rs_out: Optional[torch.Tensor] = None,
+           parts: Optional[tuple] = None, parts_out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``w_shuf``: ``shuffle_weight(w)``, streamed instead of ``w`` on the skinny path (``skinny_rows``).
     ``rs_out`` (decode): row-statistics partials of the output (``rowstats_buffer``);
     ``rowstats_written()`` tells whether the kernel that ran wrote them.
     ``ws``: ``decode_workspace`` (``prefill_workspace``) for the partials of a K split.
     ``rowstat`` ((M, 2) fp32 from ``transformer_ops.row_stats``) / ``colsum``: a
     folded pre-norm applied in the epilogue, ``rstd (x W^T) - mean rstd colsum``
-    (MFMA tile kernels only).  ``ACT_XIELU``: c0 z^2 + z / 2 above zero, c1 (exp(z) - 1 - z) + z / 2
+    (MFMA tile kernels only).  ``parts`` = (``parts_buffer`` of x, eps, norm): the folded norm with its statistics
+    merged from partials, sizes of ``takes_parts`` only.  ``parts_out``: partials of the output where the kernel that
+    runs can write them (``rowstats_written()``).  ``ACT_XIELU``: c0 z^2 + z / 2 above zero, c1 (exp(z) - 1 - z) + z / 2
     below; ``bias`` has N + 2 entries, the last two are c0 and c1."""
     a = _ACTS[act] if not isinstance(act, int) else act
     x2 = x.reshape(-1, x.shape[-1]) if x.dim() != 2 else x
@@ -205,9 +221,23 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     if rowstat is not None and (rowstat.dtype != torch.float32 or rowstat.numel() < 2 * M
                                 or not rowstat.is_contiguous()):
         raise ValueError("linear: rowstat must be contiguous fp32 (M, 2)")
-    if colsum is not None and (rowstat is None or colsum.dtype != torch.float32 or colsum.numel() < N):
+    for t, width, nm in ((None if parts is None else parts[0], K, "parts"), (parts_out, N, "parts_out")):
+        if t is not None and (t.dtype != torch.float32 or not t.is_contiguous() or width % 32 or t.numel() < M * (width // 16)):
+            raise ValueError(f"linear: {nm}: contiguous fp32 with {M} x {width} / 16 entries expected")
+    if parts is not None and (rowstat is not None or not takes_parts(M, N, K, a, ws)):
+        raise ValueError("linear: these sizes do not take partials")
+    if colsum is not None and (rowstat is None and parts is None or colsum.dtype != torch.float32 or colsum.numel() < N):
         raise ValueError("linear: colsum needs rowstat and N fp32 entries")
     wsp, wsb = _ws_args(ws)
+    if parts is not None or parts_out is not None:
+        if o2.dtype != torch.bfloat16:
+            raise ValueError("linear: partials need bf16 output")
+        t, eps, norm = parts if parts is not None else (None, 0.0, 0)
+        rc, _LAST_RS[0] = lib().gemm_bf16_parts(ptr(x2), x2.stride(0), ptr(w), w.stride(0), ptr(o2), o2.stride(0), ptr(bias),
+                                                ptr(r2), 0 if r2 is None else r2.stride(0), M, N, K, a, stream_ptr(),
+                                                ptr(w_shuf), norm, eps, 0, ptr(t), ptr(colsum), ptr(parts_out), wsp, wsb)
+        check(rc, "gemm_bf16_parts")
+        return out
     rs = _RowStats(rs_out, None, M)
     try:
         check(lib().gemm_bf16(ptr(x2), x2.stride(0), ptr(w), w.stride(0), ptr(o2), o2.stride(0), ptr(bias),
@@ -313,8 +343,9 @@ def linear_norm(x: torch.Tensor, f: FoldedLinear, act=None, residual: Optional[t
                 ones: Optional[torch.Tensor] = None, q8: Optional[torch.Tensor] = None,
                 s8: Optional[torch.Tensor] = None, ws: Optional[torch.Tensor] = None,
                 rs_in: Optional[torch.Tensor] = None, sx: Optional[torch.Tensor] = None,
-                q_out: Optional[tuple] = None) -> torch.Tensor:
-    """``linear(norm(x), W, b)`` for a ``FoldedLinear``.  ``rs_in`` (decode):
+                q_out: Optional[tuple] = None, parts: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``linear(norm(x), W, b)`` for a ``FoldedLinear``.  ``parts`` (prefill): the partials of ``x``, in place of
+    a pass over it where the sizes take them.  ``rs_in`` (decode):
     the row-statistics partials of ``x`` written by its producer (``linear(...,
     rs_out=)``), merged instead of deriving the statistics from ``x``.  Decode-sized M (<= 64):
     one skinny-GEMM launch that accumulates the row statistics from the A
@@ -357,6 +388,8 @@ def linear_norm(x: torch.Tensor, f: FoldedLinear, act=None, residual: Optional[t
             # statistics only (8 B per row, carved from the front of std_buf), the
             # norm applied in the GEMM epilogue on the raw activations: no
             # normalised copy written and re-read (profiles/archive/r2_prefill_fold_norm_ab.jsonl)
+            if parts is not None and takes_parts(M, N, K, a, ws):
+                return linear(x, f.w, f.bias, a, residual, out, colsum=f.colsum, ws=ws, parts=(parts, f.eps, f.norm))
             from .transformer_ops import row_stats
             st = std_buf.reshape(-1)[:4 * M].view(torch.float32).view(M, 2)
             row_stats(x, st, f.eps, f.norm == NORM_RMS, rows=M, ldx=x.stride(0))
@@ -393,7 +426,8 @@ QKV_SCATTER = True  # prefill c_attn writes q / K / V head-major (A/B switch)
 def qkv_scatter_norm(x: torch.Tensor, f: FoldedLinear, std_buf: torch.Tensor, q: torch.Tensor, kc: torch.Tensor,
                      vc: torch.Tensor, pos: torch.Tensor, B: int, T: int, H: int, Hkv: int, hd: int,
                      ones: Optional[torch.Tensor] = None, q8: Optional[torch.Tensor] = None,
-                     s8: Optional[torch.Tensor] = None, sx: Optional[torch.Tensor] = None) -> bool:
+                     s8: Optional[torch.Tensor] = None, sx: Optional[torch.Tensor] = None,
+                     parts: Optional[torch.Tensor] = None) -> bool:
     """Prefill c_attn (folded pre-norm, no RoPE) with the QKV scatter epilogue
     (gemm_bf16.hip ``dnn_gemm_bf16_qkv_scatter``): q lands in ``q`` as (B, H, T,
     hd) and K / V straight in the bf16 caches at rows ``pos[b] + t``, so the head-
@@ -434,6 +468,14 @@ def qkv_scatter_norm(x: torch.Tensor, f: FoldedLinear, std_buf: torch.Tensor, q:
                                          ptr(f.bias), ptr(q), ptr(kc), ptr(vc), ptr(pos), B, T, H, Hkv, hd,
                                          kc.shape[2], 2 * kp if split else kp, stream_ptr()),
               "gemm_fp8_qkv_scatter")
+        return True
+    if parts is not None and takes_parts(M, N, K, scatter=True):
+        rc = lib().gemm_bf16_qkv_scatter_parts(ptr(x), x.stride(0), ptr(f.w), f.w.stride(0), ptr(f.bias), f.norm, f.eps,
+                                               ptr(std_buf), ptr(parts), ptr(f.colsum), ptr(q), ptr(kc), ptr(vc), ptr(pos),
+                                               B, T, H, Hkv, hd, kc.shape[2], K, stream_ptr())
+        if rc == -3:
+            return False
+        check(rc, "gemm_bf16_qkv_scatter_parts")
         return True
     from .transformer_ops import row_stats
     st = std_buf.reshape(-1)[:4 * M].view(torch.float32).view(M, 2)

@@ -350,6 +350,7 @@ class TransformerStage(StageCompute):
         self.head_part = (torch.empty((self.max_batch * 2 * HEAD_PART_PER_ROW,), dtype=torch.int32, device=dev)
                           if self.last else None)
         self.rowstat = G_.rowstats_buffer(self.max_batch, d, dev)  # decode rows only
+        self.rowparts = None if self.fp8 or not self.fuse_norm else G_.parts_buffer(ntok, d, dev)  # prefill rows
         self.pws = None if self.fp8 else G_.prefill_workspace(ntok, max((H + 2 * Hkv) * hd, d, ffn), dev)
         self.q8 = self.s8 = None
         self.sx8 = self.q8b = self.sx8b = None
@@ -371,8 +372,9 @@ class TransformerStage(StageCompute):
             self.next_ids = torch.empty((ntok,), dtype=torch.int32, device=dev)
 
     def _lin(self, x, w, b, act=ACT_NONE, residual=None, out=None, ncols=None, w_shuf=None, ws=None, rs_out=None,
-             mx_in=None):
+             mx_in=None, parts_out=None):
         """``rs_out``: decode row-statistics partials of the output (see ``step``);
+        ``parts_out``: prefill partials of the output;
         ``mx_in`` (fp8 prefill): (bytes, scales) of x already MX-quantised by its
         producer.  Returns (out, whether the row statistics were written)."""
         from ..ops.gemm import rowstats_written
@@ -384,8 +386,8 @@ class TransformerStage(StageCompute):
             if mx_in is not None:
                 return linear_fp8(x, w, b, act, residual, out, mx_in[0], None, prequantized=True, sx=mx_in[1]), False
             return linear_fp8(x, w, b, act, residual, out, self.q8, self.s8, sx=self.sx8), False
-        y = linear(x, w, b, act, residual, out, w_shuf=w_shuf, ws=ws, rs_out=rs_out)
-        return y, rs_out is not None and rowstats_written()
+        y = linear(x, w, b, act, residual, out, w_shuf=w_shuf, ws=ws, rs_out=rs_out, parts_out=parts_out)
+        return y, (rs_out is not None or parts_out is not None) and rowstats_written()
 
     # ------------------------------------------------------------------ specs
     act_dtype = torch.bfloat16  # stage-boundary hidden states
@@ -455,17 +457,26 @@ class TransformerStage(StageCompute):
         have_rs = False
         one_group = self.fp8 and ntok > G_.SKINNY_MAX_M  # e4m3 activations follow the attention
         one_call = T > 1 and self._prefill_blocks(h_in, pos, B, T, b0)
+        # prefill: the same by partials of 32 columns, where the projection that follows merges them
+        rp_up = rp_qkv = None
+        if T > 1 and not one_call and self.rowparts is not None and self.layers:
+            up, nq = self.layers[0].w_up, (self.H + 2 * self.Hkv) * self.hd
+            act = ACT_GELU if self.family == "gpt2" else ACT_SILU_MUL
+            rp_up = self.rowparts if G_.takes_parts(ntok, up.w.shape[0], d, act, gws) else None
+            rp_qkv = (self.rowparts if G_.QKV_SCATTER and self.cos is None and G_.takes_parts(ntok, nq, d, scatter=True)
+                      else None)
         for li, L in enumerate(() if one_call else self.layers):
             kc, vc = self.kc[li, b0:b0 + B], self.vc[li, b0:b0 + B]
             att = self.buf_att[r0:r1]
             scattered = (T > 1 and self.cos is None and self.fuse_norm and
                          qkv_scatter_norm(h_in, L.w_qkv, a, self.buf_q, kc, vc, pos, B, T, self.H, self.Hkv,
-                                          self.hd, ones=self.ones, q8=q8, s8=s8, sx=self.sx8 if T > 1 else None))
+                                          self.hd, ones=self.ones, q8=q8, s8=s8, sx=self.sx8 if T > 1 else None,
+                                          parts=rp_qkv if have_rs else None))
             if scattered:
                 pass  # prefill (no RoPE): c_attn wrote q head-major and K / V straight into the caches
             elif self.fuse_norm:
                 qkv = linear_norm(h_in, L.w_qkv, out=self.buf_qkv[r0:r1], std_buf=a, ones=self.ones, q8=q8,
-                                  s8=s8, ws=gws, rs_in=rs if have_rs else None)
+                                  s8=s8, ws=gws, rs_in=rs if have_rs else None, parts=rp_qkv if have_rs else None)
             else:
                 T_.layernorm(h_in, L.ln1_w, L.ln1_b, a, self.eps, self.rms, rows=ntok)
                 qkv, _ = self._lin(a, L.w_qkv, L.b_qkv, out=self.buf_qkv[r0:r1])
@@ -479,7 +490,8 @@ class TransformerStage(StageCompute):
             else:
                 T_.qkv_split(qkv, self.buf_q, kc, vc, B, T, self.H, self.Hkv, self.hd, pos, self.cos, self.sin)
                 T_.flash_attn(self.buf_q, kc, vc, att, B, T, self.H, self.Hkv, self.hd, pos, one_group=one_group)
-            _, have_rs = self._lin(att, L.w_o, L.b_o, residual=h_in, out=h, w_shuf=L.w_o_s, ws=gws, rs_out=rs)
+            _, have_rs = self._lin(att, L.w_o, L.b_o, residual=h_in, out=h, w_shuf=L.w_o_s, ws=gws, rs_out=rs,
+                                   parts_out=rp_up)
             up_act = ACT_GELU if self.family == "gpt2" else ACT_SILU_MUL
             mx_f = None
             if self.fuse_norm:
@@ -489,14 +501,14 @@ class TransformerStage(StageCompute):
                     mx_f = (self.q8b, self.sx8b)
                 f = linear_norm(h, L.w_up, act=up_act, out=self.buf_f[r0:r1], std_buf=a, ones=self.ones, q8=q8,
                                 s8=s8, ws=gws, rs_in=rs if have_rs else None,
-                                sx=self.sx8 if T > 1 else None, q_out=mx_f)
+                                sx=self.sx8 if T > 1 else None, q_out=mx_f, parts=rp_up if have_rs else None)
                 if mx_f is not None:
                     f = self.buf_f[r0:r1]  # shape only: c_proj reads the e4m3 bytes in mx_f
             else:
                 T_.layernorm(h, L.ln2_w, L.ln2_b, a, self.eps, self.rms, rows=ntok)
                 f, _ = self._lin(a, L.w_up, L.b_up, act=up_act, out=self.buf_f[r0:r1])
             _, have_rs = self._lin(f, L.w_down, L.b_down, residual=h, out=h, w_shuf=L.w_down_s, ws=gws, rs_out=rs,
-                                   mx_in=mx_f)
+                                   mx_in=mx_f, parts_out=rp_qkv)
             h_in = h
         if not self.last:
             if out is not None:
@@ -554,18 +566,20 @@ class TransformerStage(StageCompute):
         up = self.layers[0].w_up
         n = [B, T, self.d, self.H, self.Hkv, self.hd, self.kc.shape[3], self.buf_f.shape[1], up.w.shape[0],
              ACT_GELU if self.family == "gpt2" else ACT_SILU_MUL, up.norm, G_.SKINNY_ALWAYS_M, G_.SKINNY_MAX_M,
-             int(self.fp8), int(G_.QKV_SCATTER)]
+             int(self.fp8), int(G_.QKV_SCATTER), 0, 0]
         bufs = [_lib.ptr(t) for t in (self.buf_h, self.buf_a, self.buf_qkv, self.buf_q, self.buf_att, self.buf_f,
                                       self.q8, self.sx8, self.q8b, self.sx8b, self.pws, x, self.ones, self.kc[0, b0],
-                                      self.vc[0, b0], pos, self.cos, self.sin, self.s8)]
+                                      self.vc[0, b0], pos, self.cos, self.sin, self.s8, self.rowparts)]
         block, wsb = self.kc.stride(0) * 2, 0 if self.pws is None else self.pws.nbytes
         st = _lib.stream_ptr()
         # the first block by itself: the device works on it while the pointers of the rest are collected
-        for layers in (self.layers[:1], self.layers[1:]):
+        rest = self.layers[1:]
+        for layers in (self.layers[:1], rest):
             if not layers:
                 break
             w = [p for L in layers for p in self._block_ptrs(L)]
-            rc, what = _lib.lib().prefill_blocks(n, bufs, self.eps, 1.0 / math.sqrt(self.hd), block, wsb, st, w)
+            n[15] = int(layers is not rest and bool(rest))
+            rc, what, n[16] = _lib.lib().prefill_blocks(n, bufs, self.eps, 1.0 / math.sqrt(self.hd), block, wsb, st, w)
             if rc == -100:  # the same answer for every block
                 return False
             _lib.check(rc, what)

@@ -1752,6 +1752,49 @@ def test_prefill_one_call(model, dtype, B, T, monkeypatch):
     assert got[0][1][:, 1:1 + B].abs().sum() > 0 and got[0][1][:, 1 + B].abs().sum() == 0
 
 
+@pytest.mark.parametrize("tile,splits", [(t, 1) for t in range(7)] + [(0, 2), (2, 3), (5, 2)])
+@pytest.mark.parametrize("M,d,rms", [(65, 768, False), (200, 64, False), (333, 1600, True), (259, 2048, False)])
+def test_row_statistics_by_partials(tile, splits, M, d, rms):
+    """Partials of 32 columns beside a projection's rows, on every tile and from a split's sum, and a folded norm that
+    merges them: both against float64 on the rows as stored.  Rows far from zero (their mean cancels), one with an
+    infinity.  Bounds: a sum of n terms in fp32, n 2^-24 of their magnitude; the norm's two products cancel against
+    each other, so theirs is that of the raw rows."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    torch.manual_seed(M + d)
+    K0, N = 256, 192
+    x, w = torch.randn(M, K0, device=DEV).bfloat16(), (torch.randn(d, K0, device=DEV) / 16).bfloat16()
+    res = (torch.randn(M, d, device=DEV) + 20 * torch.randn(M, 1, device=DEV)).bfloat16()
+    h, parts = torch.empty(M, d, device=DEV, dtype=torch.bfloat16), G.parts_buffer(M, d, DEV)
+    ws = G.prefill_workspace(M, 2048, DEV)
+    f = G.fold_norm(torch.randn(N, d, device=DEV) / math.sqrt(d), torch.rand(d, device=DEV) + 0.5, None, None, rms, 1e-5, DEV)
+    std, ones = torch.empty(M, d, device=DEV, dtype=torch.bfloat16), torch.ones(d, device=DEV)
+    G.lib().gemm_set_mid(tile, splits)
+    try:
+        G.linear(x, w, None, residual=res, out=h, ws=ws, parts_out=parts)
+        assert G.rowstats_written()
+        assert torch.equal(h, G.linear(x, w, None, residual=res, ws=ws))
+        p, hd = parts.view(M, d // 32, 2).double(), h.double().view(M, d // 32, 32)
+        mean = hd.mean(2)
+        assert bool(((p[..., 0] - mean).abs() <= hd.abs().sum(2) * 2.0 ** -24).all())
+        m2 = (hd - mean[..., None]).pow(2).sum(2)
+        # the mean's rounding shifts every difference: 2 |x - mean| times it, and 32 roundings
+        assert bool(((p[..., 1] - m2).abs() <= m2 * 40 * 2.0 ** -24 + 32 * (hd.abs().sum(2) * 2.0 ** -24) ** 2 + 1e-12).all())
+        if splits == 1:
+            if M > 65:
+                h[1, 5], parts.view(M, -1, 2)[1, 0] = float("inf"), torch.tensor([float("inf"), float("nan")], device=DEV)
+            assert G.takes_parts(M, N, d, 0, ws)
+            y = G.linear(h, f.w, f.bias, colsum=f.colsum, ws=ws, parts=(parts, f.eps, f.norm)).double()
+            r = h.double()
+            mu = r.mean(1, keepdim=True) * (0 if rms else 1)
+            rstd = torch.rsqrt((r - mu).pow(2).mean(1, keepdim=True) + f.eps)
+            ref = ((r - mu) * rstd) @ f.w.double().t()
+            bound = ref.abs() * 2.0 ** -8 + (r.abs() @ f.w.double().abs().t()) * rstd * (d + 64) * 2.0 ** -24
+            ok = torch.isfinite(r).all(1)
+            assert bool(((y - ref).abs() <= bound)[ok].all()) and not bool(torch.isfinite(y[~ok]).any())
+    finally:
+        G.lib().gemm_set_mid(-1, 1)
+
+
 @pytest.mark.parametrize("T", [70, 200])
 def test_prefill_rows_off_16_bytes(T):
     """Hidden rows that start off 16 bytes: issued by the loop, whose kernels look at the alignment."""
