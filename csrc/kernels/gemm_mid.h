@@ -27,7 +27,9 @@ struct MidTile {
 // has for three.  us, the best of the others : these: 700 x 6144 x 4096 51.8 : 43.4, 1500 x 4096 x 4096 57.0 : 49.9, 1400 x
 // 3072 x 768 17.4 : 14.9, 700 x 4096 x 14336 in 2 95.2 : 86; 96 rows: 380 x 6144 x 4096 38.3 : 35.0, 700 x 4096 x 4096 34.3 : 33.0.
 // (192 x 64, 128 x 192 and 192 x 192 are best nowhere by more than 2 %.)
-typedef MidTile<64, 64, 2, 2, 4> Mid0;
+// 64 x 64: five K-tiles are what two workgroups a CU have room for.  us with four : five: 64 x 64 x 3072 11.1 : 10.6, 1071 x
+// 768 x 3072 13.5 : 12.8, 700 x 6144 x 4096 72.2 : 71.0; six and more (one workgroup a CU) gain nothing over five.
+typedef MidTile<64, 64, 2, 2, 5> Mid0;
 typedef MidTile<128, 64, 2, 2, 6> Mid1;
 typedef MidTile<128, 128, 2, 4, 4> Mid2;
 typedef MidTile<256, 128, 4, 2, 3> Mid3;
@@ -218,7 +220,8 @@ template <class T>
 struct MidParts {
   static constexpr int TPR = T::THREADS / T::BM >= 4 ? 4 : 2, B = 4;  // lanes a row, loads a lane and batch
   static constexpr int TILES = T::S * T::STAGE;
-  static constexpr bool ROOM = TILES + T::BM * 8 <= 160 * 1024;
+  static constexpr int CU = TILES > 80 * 1024 ? 160 * 1024 : 80 * 1024;  // as many workgroups a CU as without
+  static constexpr bool ROOM = TILES + T::BM * 8 <= CU;
   static constexpr int LDS = TILES + (ROOM ? T::BM * 8 : 0);
   f32x4 p[B];
   float2 r;
