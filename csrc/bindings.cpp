@@ -107,8 +107,8 @@ PYBIND11_MODULE(_dnn_hip, m) {
     return dnn_gemm_bf16_qkv_scatter(CP(A), lda, CP(W), ldw, CFP(bias), CFP(rowstat), CFP(colsum), P(q), P(kc), P(vc),
                                      CIP(pos), B, T, H, Hkv, hd, S, K, ST(st));
   });
-  m.def("gemm_takes_parts", [](int M, int N, int K, int act, int scatter, long long ws_bytes) {
-    return dnn_gemm_takes_parts(M, N, K, act, scatter, ws_bytes) != 0;
+  m.def("gemm_takes_parts", [](int M, int N, int K, int lda, int ldw, int act, int scatter, long long ws_bytes) {
+    return dnn_gemm_takes_parts(M, N, K, lda, ldw, act, scatter, ws_bytes) != 0;
   });
   // (code, whether the output's partials were written)
   m.def("gemm_bf16_parts", [](u64 A, int lda, u64 W, int ldw, u64 C, int ldc, u64 bias, u64 R, int ldr, int M, int N, int K,

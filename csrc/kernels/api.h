@@ -66,7 +66,7 @@ int dnn_argmax_final(const void* part, int S, int M, int* out, int* out2, int* p
                      int* hist = nullptr, int hist_ld = 0);
 // folded norm from partials of the row statistics, and partials of the output's (gemm_mid.h): whether a product of these
 // sizes reads them; the product; QKV scattered
-int dnn_gemm_takes_parts(int M, int N, int K, int act, int scatter, long long ws_bytes);
+int dnn_gemm_takes_parts(int M, int N, int K, int lda, int ldw, int act, int scatter, long long ws_bytes);
 int dnn_gemm_bf16_parts(const void* A, int lda, const void* W, int ldw, void* C, int ldc, const float* bias, const void* R,
                         int ldr, int M, int N, int K, int act, hipStream_t st, const void* Wsh, int norm, float eps,
                         float* stats, const void* parts, const float* colsum, void* parts_out, int* wrote, void* ws,

@@ -581,6 +581,9 @@ struct PartsScope {
   ~PartsScope() { g_parts = PartsReq{}; }
 };
 
+// The small tiles address a tile's rows with 32 bits.
+static bool mid_narrow(int lda, int ldw) { return lda < 1 << 23 && ldw < 1 << 23; }
+
 // Rows that 16-byte LDS-DMA may fetch.
 static bool dma_rows(const void* A, int lda, const void* W, int ldw) {
   return (((uintptr_t)A | (uintptr_t)W) & 15) == 0 && lda % 8 == 0 && ldw % 8 == 0;
@@ -595,7 +598,7 @@ static int launch_gemm(const void* A, int lda, const void* W, int ldw, void* C, 
   // itself, dnn_gemm_skinny_norm
   const long long part_bytes = mid_ws(ws, ws_bytes);
   // up to 256 rows what the small tiles cannot stage (dma_rows) goes to the decode kernels, whose loads are plain
-  const bool narrow = lda < 1 << 23 && ldw < 1 << 23;  // the small tiles address a tile's rows with 32 bits
+  const bool narrow = mid_narrow(lda, ldw);
   if (rowstat == nullptr && g_parts.in == nullptr && (skinny(M, N, K, false, Wsh != nullptr, part_bytes) ||
                              (M <= 256 && (!narrow || !dma_rows(A, lda, W, ldw))))) {
     return dnn_gemm_skinny(A, lda, nullptr, W, ldw, nullptr, C, ldc, bias, R, ldr, M, N, K, ACT, F32 ? 1 : 0, 0, st, Wsh,
@@ -609,6 +612,8 @@ static int launch_gemm(const void* A, int lda, const void* W, int ldw, void* C, 
   else if (g_gemm_tile == 128) plan.tile = 2;
   else if (g_gemm_tile == 0 && (is_glu(ACT) || has_consts(ACT) || tail_split_cols(M, N) == 0))
     plan = mid_plan(M, N, K, part_bytes, has_consts(ACT) ? MID_BF16_WHOLE : MID_BF16);  // constants lie behind all N
+  // partials are merged by one launch of the small tiles over all columns and all of K, and by nothing else
+  if (g_parts.in != nullptr && (plan.tile < 0 || plan.cols != 0 || plan.splits != 1)) return -4;
   if (plan.tile >= 0) {
     MidArgs a{{C, bias, (const bf16_t*)R, ldc, ldr, M, N, ACT, F32 ? 1 : 0}, (const bf16_t*)A, (const bf16_t*)W,
               rowstat, colsum, nullptr, g_parts.in, g_parts.eps, g_parts.rms, (float*)ws, lda, ldw, K, plan.splits};
@@ -704,9 +709,10 @@ extern "C" int dnn_gemm_bf16(const void* A, int lda, const void* W, int ldw, voi
 }
 
 #ifndef DNN_DECODER_ONLY
-// Whether a folded norm of these sizes can take its statistics from partials: one launch of the small tiles, K whole.
-static bool takes_parts(int M, int N, int K, long long part_bytes, int act, bool scatter) {
-  if (g_gemm_tile != 0 || K % 64 != 0 || K > MID_PARTS_K) return false;
+// Whether a folded norm of these sizes and distances of rows can take its statistics from partials: one launch of the
+// small tiles, K whole.
+static bool takes_parts(int M, int N, int K, int lda, int ldw, long long part_bytes, int act, bool scatter) {
+  if (g_gemm_tile != 0 || K % 64 != 0 || K > MID_PARTS_K || !mid_narrow(lda, ldw)) return false;
   if (scatter && tail_split_cols(M, N) != 0) return false;
   if (g_mid_tile >= 0) return scatter || g_mid_splits == 1;
   if (!is_glu(act) && tail_split_cols(M, N) != 0) return false;
@@ -714,8 +720,8 @@ static bool takes_parts(int M, int N, int K, long long part_bytes, int act, bool
   return p.tile >= 0 && p.cols == 0 && p.splits == 1;
 }
 
-extern "C" int dnn_gemm_takes_parts(int M, int N, int K, int act, int scatter, long long ws_bytes) {
-  return takes_parts(M, N, K, ws_bytes - 4096, act, scatter != 0);
+extern "C" int dnn_gemm_takes_parts(int M, int N, int K, int lda, int ldw, int act, int scatter, long long ws_bytes) {
+  return takes_parts(M, N, K, lda, ldw, ws_bytes - 4096, act, scatter != 0);
 }
 
 // GPT-2, 3 x 357 tokens: a statistics launch of 3.4 us ahead of every c_attn and c_fc, 784 a pass; as partials, which
@@ -728,7 +734,7 @@ extern "C" int dnn_gemm_bf16_parts(const void* A, int lda, const void* W, int ld
                                    const void* R, int ldr, int M, int N, int K, int act, hipStream_t st, const void* Wsh,
                                    int norm, float eps, float* stats, const void* parts, const float* colsum,
                                    void* parts_out, int* wrote, void* ws, long long ws_bytes) {
-  const bool read = norm != 0 && parts != nullptr && takes_parts(M, N, K, mid_ws(ws, ws_bytes), act, false);
+  const bool read = norm != 0 && parts != nullptr && takes_parts(M, N, K, lda, ldw, mid_ws(ws, ws_bytes), act, false);
   *wrote = 0;
   if (norm != 0 && !read) {
     if (stats == nullptr) return -1;
@@ -746,7 +752,7 @@ extern "C" int dnn_gemm_bf16_qkv_scatter_parts(const void* A, int lda, const voi
                                                void* kc, void* vc, const int* pos, int B, int T, int H, int Hkv, int hd,
                                                int S, int K, hipStream_t st) {
   const int N = (H + 2 * Hkv) * hd;
-  const bool read = parts != nullptr && N % 32 == 0 && takes_parts(B * T, N, K, 0, ACT_NONE, true);
+  const bool read = parts != nullptr && N % 32 == 0 && takes_parts(B * T, N, K, lda, ldw, 0, ACT_NONE, true);
   if (!read) {
     if (const int rc = dnn_row_stats(A, lda, stats, B * T, K, eps, norm == 1, st)) return rc;
   }
@@ -777,7 +783,7 @@ extern "C" int dnn_gemm_bf16_qkv_scatter(const void* A, int lda, const void* W, 
   const int tiles = ((M + BG_M - 1) / BG_M) * ((N + BG_N - 1) / BG_N);
   if ((hd & (hd - 1)) != 0 || M >= (1 << 24)) return -3;
   QkvScatter sc{(bf16_t*)q, (bf16_t*)kc, (bf16_t*)vc, pos, T, H, Hkv, __builtin_ctz(hd), S, 1.0f / (float)T};
-  if (g_gemm_tile == 0 && tail_split_cols(M, N) == 0 && lda < 1 << 23 && ldw < 1 << 23) {
+  if (g_gemm_tile == 0 && tail_split_cols(M, N) == 0 && mid_narrow(lda, ldw)) {
     MidPlan plan = mid_plan(M, N, K, 0, MID_BF16_WHOLE);
     if (g_mid_tile >= 0) plan.tile = g_mid_tile;
     if (plan.tile >= 0) {
@@ -787,6 +793,7 @@ extern "C" int dnn_gemm_bf16_qkv_scatter(const void* A, int lda, const void* W, 
       return mid_launch(plan.tile, a, &sc, st);
     }
   }
+  if (g_parts.in != nullptr) return -4;  // only the small tiles merge partials
   if (M < 256) return -3;
   if (!bg_narrow(lda) || !bg_narrow(ldw)) {  // the 256 x 128 tiles address rows with 64 bits
     hipLaunchKernelGGL((gemm_bf16_256_kernel<ACT_NONE, false, true, 1>), dim3((M + BG_M - 1) / BG_M * ((N + 127) / 128)),

@@ -158,8 +158,8 @@ struct PrefillPass {
     const int one_group = fp8 && rows() > skinny_max;  // e4m3 activations follow (attention.hip flash_two_groups)
     const bool up_quant = fp8 && act == 2 && !skinny(n_up, d, true, true, 0);
     const bool part = parts != nullptr && !fp8;  // who reads h's partials
-    const bool read_up = part && dnn_gemm_takes_parts(rows(), n_up, d, act, 0, ws_bytes);
-    const bool read_qkv = part && scatter && cosT == nullptr && dnn_gemm_takes_parts(rows(), nq, d, 0, 1, 0);
+    const bool read_up = part && dnn_gemm_takes_parts(rows(), n_up, d, d, d, act, 0, ws_bytes);
+    const bool read_qkv = part && scatter && cosT == nullptr && dnn_gemm_takes_parts(rows(), nq, d, d, d, 0, 1, 0);
     for (size_t i = 0; i < blocks.size(); ++i) {
       const PrefillBlock& L = blocks[i];
       void *k = kc + i * kv_block, *v = vc + i * kv_block;

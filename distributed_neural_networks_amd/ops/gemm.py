@@ -170,9 +170,11 @@ def parts_buffer(rows: int, width: int, device) -> Optional[torch.Tensor]:
     return torch.empty((rows, width // 16), dtype=torch.float32, device=device)
 
 
-def takes_parts(M: int, N: int, K: int, act: int = 0, ws: Optional[torch.Tensor] = None, scatter: bool = False) -> bool:
-    """Whether a folded norm of these sizes merges partials (else it needs ``row_stats``)."""
-    return bool(lib().gemm_takes_parts(M, N, K, act, int(scatter), 0 if ws is None else ws.nbytes))
+def takes_parts(M: int, N: int, K: int, act: int = 0, ws: Optional[torch.Tensor] = None, scatter: bool = False,
+                lda: int = 0, ldw: int = 0) -> bool:
+    """Whether a folded norm of these sizes, with rows this far apart (0: one behind the other), merges partials
+    (else it needs ``row_stats``)."""
+    return bool(lib().gemm_takes_parts(M, N, K, lda or K, ldw or K, act, int(scatter), 0 if ws is None else ws.nbytes))
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, act=None,
@@ -224,7 +226,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     for t, width, nm in ((None if parts is None else parts[0], K, "parts"), (parts_out, N, "parts_out")):
         if t is not None and (t.dtype != torch.float32 or not t.is_contiguous() or width % 32 or t.numel() < M * (width // 16)):
             raise ValueError(f"linear: {nm}: contiguous fp32 with {M} x {width} / 16 entries expected")
-    if parts is not None and (rowstat is not None or not takes_parts(M, N, K, a, ws)):
+    if parts is not None and (rowstat is not None or not takes_parts(M, N, K, a, ws, lda=x2.stride(0), ldw=w.stride(0))):
         raise ValueError("linear: these sizes do not take partials")
     if colsum is not None and (rowstat is None and parts is None or colsum.dtype != torch.float32 or colsum.numel() < N):
         raise ValueError("linear: colsum needs rowstat and N fp32 entries")
@@ -388,7 +390,7 @@ def linear_norm(x: torch.Tensor, f: FoldedLinear, act=None, residual: Optional[t
             # statistics only (8 B per row, carved from the front of std_buf), the
             # norm applied in the GEMM epilogue on the raw activations: no
             # normalised copy written and re-read (profiles/archive/r2_prefill_fold_norm_ab.jsonl)
-            if parts is not None and takes_parts(M, N, K, a, ws):
+            if parts is not None and takes_parts(M, N, K, a, ws, lda=x.stride(0), ldw=f.w.stride(0)):
                 return linear(x, f.w, f.bias, a, residual, out, colsum=f.colsum, ws=ws, parts=(parts, f.eps, f.norm))
             from .transformer_ops import row_stats
             st = std_buf.reshape(-1)[:4 * M].view(torch.float32).view(M, 2)
@@ -469,7 +471,7 @@ def qkv_scatter_norm(x: torch.Tensor, f: FoldedLinear, std_buf: torch.Tensor, q:
                                          kc.shape[2], 2 * kp if split else kp, stream_ptr()),
               "gemm_fp8_qkv_scatter")
         return True
-    if parts is not None and takes_parts(M, N, K, scatter=True):
+    if parts is not None and takes_parts(M, N, K, scatter=True, lda=x.stride(0), ldw=f.w.stride(0)):
         rc = lib().gemm_bf16_qkv_scatter_parts(ptr(x), x.stride(0), ptr(f.w), f.w.stride(0), ptr(f.bias), f.norm, f.eps,
                                                ptr(std_buf), ptr(parts), ptr(f.colsum), ptr(q), ptr(kc), ptr(vc), ptr(pos),
                                                B, T, H, Hkv, hd, kc.shape[2], K, stream_ptr())

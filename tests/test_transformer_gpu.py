@@ -1795,6 +1795,43 @@ def test_row_statistics_by_partials(tile, splits, M, d, rms):
         G.lib().gemm_set_mid(-1, 1)
 
 
+@pytest.mark.parametrize("far", ["rows", "weights"])
+@pytest.mark.parametrize("scatter", [False, True])
+def test_partials_of_rows_far_apart(far, scatter):
+    """Rows 2^23 elements apart leave the tiles that merge partials: with ``parts`` the norm is applied all the same (the
+    same launches as without, so the same bits), and a call that insists on partials is refused."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    torch.manual_seed(5)
+    B, T, H, hd, d = 1, 257, 4, 64, 256
+    M, N = B * T, 3 * H * hd
+    x = (3 * torch.randn(M, d, device=DEV) + 1).bfloat16()
+    f = G.fold_norm(torch.randn(N, d, device=DEV) / 16, torch.ones(d, device=DEV), torch.zeros(d, device=DEV), None, False, 1e-5, DEV)
+    assert G.takes_parts(M, N, d, scatter=scatter) and not G.takes_parts(M, N, d, scatter=scatter, lda=1 << 23)
+    held = torch.empty(M if far == "rows" else N, 1 << 23, device=DEV, dtype=torch.bfloat16)
+    view = held[:, :d]
+    view.copy_(x if far == "rows" else f.w)
+    if far == "rows":
+        x = view
+    else:
+        f.w = view
+    parts = G.parts_buffer(M, d, DEV)
+    r = x.float().view(M, d // 32, 32)
+    parts.view(M, d // 32, 2).copy_(torch.stack([r.mean(2), r.var(2, unbiased=False) * 32], 2))
+    std, ones = torch.empty(M, d, device=DEV, dtype=torch.bfloat16), torch.ones(d, device=DEV)
+    got = []
+    for p in (parts, None):
+        if scatter:
+            q, kc, vc = (torch.zeros(B, H, T, hd, device=DEV, dtype=torch.bfloat16) for _ in range(3))
+            pos = torch.zeros(B, device=DEV, dtype=torch.int32)
+            assert G.qkv_scatter_norm(x, f, std, q, kc, vc, pos, B, T, H, H, hd, parts=p)
+            got.append(torch.stack([q, kc, vc]))
+        else:
+            got.append(G.linear_norm(x, f, std_buf=std, ones=ones, parts=p))
+    assert torch.equal(*got)
+    with pytest.raises(ValueError):
+        G.linear(x, f.w, f.bias, colsum=f.colsum, parts=(parts, f.eps, f.norm))
+
+
 @pytest.mark.parametrize("T", [70, 200])
 def test_prefill_rows_off_16_bytes(T):
     """Hidden rows that start off 16 bytes: issued by the loop, whose kernels look at the alignment."""
