@@ -32,6 +32,7 @@ inline void bind_decoder(py::module_& m) {
      py::arg("st"), py::arg("wsh") = 0, py::arg("rowstat") = 0, py::arg("colsum") = 0, py::arg("ws") = 0,
      py::arg("ws_bytes") = 0);
   m.def("gemm_set_mid", [](int tile, int splits) { return dnn_gemm_set_mid(tile, splits); });
+  m.def("gemm_mid_blocks", [](int tile, int mx) { return dnn_gemm_mid_blocks(tile, mx); });
   m.def("gemm_is_skinny", [](int M, int N, int K, int norm, int frag, long long ws_bytes) {
     return dnn_gemm_is_skinny(M, N, K, norm, frag, ws_bytes);
   });

@@ -64,6 +64,7 @@ int dnn_gemm_head(const void* A, int lda, const void* Wsh, const float* sw, cons
 // hist (optional, with pos_inc): hist[row * hist_ld + pos_inc[row]] = id before the advance (token history)
 int dnn_argmax_final(const void* part, int S, int M, int* out, int* out2, int* pos_inc, hipStream_t st,
                      int* hist = nullptr, int hist_ld = 0);
+int dnn_gemm_mid_blocks(int tile, int mx);
 // folded norm from partials of the row statistics, and partials of the output's (gemm_mid.h): whether a product of these
 // sizes reads them; the product; QKV scattered
 int dnn_gemm_takes_parts(int M, int N, int K, int lda, int ldw, int act, int scatter, long long ws_bytes);

@@ -485,6 +485,13 @@ extern "C" int dnn_gemm_set_mid(int tile, int splits) {
   g_mid_splits = splits;
   return 0;
 }
+// Workgroups of a tile of that table (mx: of the e4m3 kernel's) that share a CU
+extern "C" int dnn_gemm_mid_blocks(int tile, int mx) {
+#ifndef DNN_DECODER_ONLY
+  if (mx) return mid8_blocks(tile);
+#endif
+  return mx ? -1 : mid_blocks(tile);
+}
 // Rows up to which every bf16 GEMM streams its weights on the skinny kernels
 // (A/B switch).  At M = 64 a wide-N head with warm weights runs faster on the
 // 128^2 MFMA tiles (GPT-2 50304 x 768: 28.3 -> 22.5 us, x 1600: 52.7 -> 33.6,

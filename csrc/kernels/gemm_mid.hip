@@ -146,6 +146,27 @@ static int launch(const MidArgs& a, const QkvScatter* scat, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
+template <class T>
+static int blocks() {
+  int n = 0;
+  const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void*)gemm_mid_kernel<T, MID_ROWS, false>,
+                                                                    T::THREADS, T::S * T::STAGE);
+  return e == hipSuccess ? n : -1;
+}
+
+int mid_blocks(int tile) {
+  switch (tile) {
+    case 0: return blocks<Mid0>();
+    case 1: return blocks<Mid1>();
+    case 2: return blocks<Mid2>();
+    case 3: return blocks<Mid3>();
+    case 4: return blocks<Mid4>();
+    case 5: return blocks<Mid5>();
+    case 6: return blocks<Mid6>();
+  }
+  return -1;
+}
+
 int mid_launch(int tile, const MidArgs& a, const QkvScatter* scat, hipStream_t st) {
   if (a.splits < 1 || (a.splits > 1 && (scat != nullptr || a.part == nullptr || a.N % 4 != 0 || a.K / 64 < a.splits ||
                                         a.M > 65535)))

@@ -47,6 +47,7 @@ bool mid_skinny(int M, int N, int K, bool norm, bool frag, long long ws_bytes);
 inline long long mid_ws(const void* ws, long long bytes) { return ws == nullptr ? 0 : bytes - 4096; }
 // Widest rows whose partials a workgroup merges, and what the columns of a product with partials divide by.
 constexpr int MID_PARTS_K = 2048, MID_PARTS_N = 64;
+int mid_blocks(int tile);  // workgroups of a tile (K whole) that share a CU
 int mid_launch(int tile, const MidArgs& a, const QkvScatter* scat, hipStream_t st);  // a.splits workgroups over K
 
 }  // namespace dnn

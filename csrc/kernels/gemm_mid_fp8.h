@@ -17,6 +17,7 @@ struct Mid8Args : MidRows {
   int Kb, ldq, kpo;
 };
 
+int mid8_blocks(int tile);  // workgroups of a tile that share a CU
 int mid8_launch(int tile, const Mid8Args& a, const QkvScatter* scat, hipStream_t st);
 
 }  // namespace dnn

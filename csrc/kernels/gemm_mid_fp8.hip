@@ -187,9 +187,37 @@ __global__ __launch_bounds__(T::NW * 64, 2) void gemm_mid_fp8_kernel(Mid8Args p,
   else mid_rows<I, J, false>(acc, mw, nw, lane, p, pre);
 }
 
+// 64 x 64: four K-tiles in flight.  With the scales' 1 KiB a K-tile five are 87,040 bytes, one workgroup a CU where the
+// estimate counts on two (gemm_mid.hip MID8).  us with five : four: 500 x 2304 x 768 8.5 :
+// 6.1, 1000 12.2 : 9.2, 1800 19.7 : 13.7, 1350 x 768 x 768 8.4 : 5.9, 820 x 4800 x 1600 22.6 : 15.6.
+typedef MidTile<64, 64, 2, 2, 4> Mid0Mx;
+
+template <class T>
+constexpr int mid8_lds() { return T::S * (T::STAGE + T::NW * 256); }
+static_assert(2 * mid8_lds<Mid0Mx>() <= 160 * 1024, "two workgroups a CU");
+
+template <class T>
+static int blocks() {
+  int n = 0;
+  const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void*)gemm_mid_fp8_kernel<T, MID8_ROWS>,
+                                                                    T::NW * 64, mid8_lds<T>());
+  return e == hipSuccess ? n : -1;
+}
+
+int mid8_blocks(int tile) {
+  switch (tile) {
+    case 0: return blocks<Mid0Mx>();
+    case 1: return blocks<Mid1>();
+    case 2: return blocks<Mid2>();
+    case 3: return blocks<Mid3>();
+    case 4: return blocks<Mid4>();
+  }
+  return -1;
+}
+
 template <class T, Mid8Out OUT>
 static int start(const Mid8Args& a, const QkvScatter& scat, hipStream_t st) {
-  constexpr int LDS = T::S * (T::STAGE + T::NW * 256);
+  constexpr int LDS = mid8_lds<T>();
   static const hipError_t room =
       hipFuncSetAttribute((const void*)gemm_mid_fp8_kernel<T, OUT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   if (room != hipSuccess) return (int)room;
@@ -209,7 +237,7 @@ static int launch(const Mid8Args& a, const QkvScatter* scat, hipStream_t st) {
 
 int mid8_launch(int tile, const Mid8Args& a, const QkvScatter* scat, hipStream_t st) {
   switch (tile) {
-    case 0: return launch<Mid0>(a, scat, st);
+    case 0: return launch<Mid0Mx>(a, scat, st);
     case 1: return launch<Mid1>(a, scat, st);
     case 2: return launch<Mid2>(a, scat, st);
     case 3: return launch<Mid3>(a, scat, st);

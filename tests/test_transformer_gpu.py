@@ -1673,6 +1673,13 @@ def test_fp8_fidelity_vs_unquantised():
     assert r["fp8-e4m3"]["prefill_logits_rel"] < 2 * r["fp8-split"]["prefill_logits_rel"]
 
 
+def test_two_small_tiles_a_cu():
+    """The estimate counts two workgroups of 64 x 64 a CU and one of every other tile, for bf16 and for e4m3."""
+    from distributed_neural_networks_amd.ops import _lib
+    for mx, tiles in ((0, 7), (1, 5)):
+        assert [_lib.lib().gemm_mid_blocks(t, mx) for t in range(tiles)] == [2] + [1] * (tiles - 1)
+
+
 @pytest.mark.parametrize("tile", range(5))
 @pytest.mark.parametrize("M,N,K", [(256, 256, 64), (257, 300, 200), (383, 520, 1600), (513, 388, 384)])
 def test_gemm_fp8_mx_small_tiles(tile, M, N, K):
