@@ -65,23 +65,38 @@ def _conv2_k288(sd) -> torch.Tensor:
     return sd["conv2.weight"].float().permute(0, 2, 3, 1).reshape(64, 288)  # (oc, ky, kx, c)
 
 
-def _conv2_winograd(sd) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+def _conv2_winograd(sd) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """U = G g G^T of every conv2 filter, times a power of two per output channel that brings its largest
-    number into [2^9, 2^10), as two fp16 terms [4 i + j][oc][c]; and the inverse scales."""
+    number into [2^9, 2^10), as two fp16 terms [4 i + j][oc][c]; the inverse scales; the largest number of a filter (oc, c)."""
     G = torch.tensor([[1, 0, 0], [.5, .5, .5], [.5, -.5, .5], [0, 0, 1]], dtype=torch.float64)
     u = G @ sd["conv2.weight"].detach().cpu().double() @ G.t()  # (oc, c, i, j)
-    top = torch.nan_to_num(u.abs(), nan=0.0, posinf=0.0).amax((1, 2, 3))
+    u_top = torch.nan_to_num(u.abs(), nan=0.0, posinf=0.0).amax((2, 3))
+    top = u_top.amax(1)
     k = torch.where(top > 0, 10 - torch.frexp(top).exponent, 0).clamp(-110, 110)
     u = (u * 2.0 ** k.double()[:, None, None, None]).permute(2, 3, 0, 1).reshape(16, 64, 32)
     hi = u.half()
-    return hi, (u - hi.double()).half(), (2.0 ** -k.double()).float()
+    return hi, (u - hi.double()).half(), (2.0 ** -k.double()).float(), u_top
 
 
-def _conv1_bound(sd) -> Tuple[torch.Tensor, torch.Tensor]:
-    """(l1, b): conv1 of an image of magnitudes up to m stays within l1 m + b.  What is not finite does
-    not count: its channel is lost whatever the scale."""
-    w, b = (torch.nan_to_num(sd[f"conv1.{n}"].detach().cpu().double().abs(), nan=0.0, posinf=0.0) for n in ("weight", "bias"))
-    return (w.sum((1, 2, 3)).max() * (1 + 2.0 ** -12)).float(), b.max().float()
+def _winograd_range(sd, u_top: torch.Tensor) -> Optional[torch.Tensor]:
+    """(l1, b, most): conv1 of an image of magnitudes up to m stays within l1 m + b; up to ``most`` that is at most
+    ``WINO_RANGE`` times what conv1's biases bring to every conv2 channel: their mean by the magnitudes of its
+    weights, each up to 4 times the median bias (one large bias lifts the scale of all channels, and may never pass
+    the ReLU).  None where one scale an image or an output channel would cost precision: ``most`` is
+    below ``WINO_IMAGES``; or a filter's numbers in U (``u_top``: the largest, (oc, c)), which keep 2^-34 of the
+    channel's largest, lie below 2^-16 of it, so that they keep fewer bits than a pair of bf16.
+    What is not finite does not count: its channel is lost whatever the scale."""
+    w1, b1, w2 = (torch.nan_to_num(sd[k].detach().cpu().double().abs(), nan=0.0, posinf=0.0)
+                  for k in ("conv1.weight", "conv1.bias", "conv2.weight"))
+    by = w2.sum((2, 3))
+    by = by[by.sum(1) > 0]
+    typical = b1.clamp(max=4 * b1.median())
+    floor = (by @ typical / by.sum(1)).min() if len(by) else b1.median()
+    l1, b = w1.sum((1, 2, 3)).max() * (1 + 2.0 ** -12), b1.max()
+    most = (WINO_RANGE * floor - b) / l1 if l1 > 0 else torch.tensor(math.inf, dtype=torch.float64)
+    if not most >= WINO_IMAGES or bool(((u_top > 0) & (u_top < u_top.amax(1, keepdim=True) * 2.0 ** -16)).any()):
+        return None
+    return torch.stack([l1, b, most]).float()
 
 
 def _fc2_pad(sd) -> torch.Tensor:
@@ -103,7 +118,7 @@ class CifarStage0Weights:
     w2l: torch.Tensor = None
     u2h: torch.Tensor = None   # fp32 path, Winograd's conv2: [16][64][32] fp16, two terms
     u2l: torch.Tensor = None
-    sc: torch.Tensor = None    # its scales: bound of conv1's weights and biases, 64 inverse scales of u2
+    sc: torch.Tensor = None    # its scales: _winograd_range, 64 inverse scales of u2
 
 
 @dataclass
@@ -137,10 +152,9 @@ def pack_stage0(sd: Dict[str, torch.Tensor], device, precision: str = "fp32") ->
     (w1h, w1l), (w2h, w2l) = split_bf16(w1), split_bf16(w2)
     dv = lambda t: t.to(device).contiguous()  # noqa: E731
     w = CifarStage0Weights("fp32", b1, b2, w1h=dv(w1h), w1l=dv(w1l), w2h=dv(w2h), w2l=dv(w2l))
-    l1, b = _conv1_bound(sd)
-    if WINO_RANGE * b >= 32 * l1:  # images up to a magnitude of 32 are within the range of one scale
-        u2h, u2l, inv = _conv2_winograd(sd)
-        w.u2h, w.u2l, w.sc = dv(u2h), dv(u2l), dv(torch.cat([torch.stack([l1, b]), inv]))
+    u2h, u2l, inv, u_top = _conv2_winograd(sd)
+    if (rng := _winograd_range(sd, u_top)) is not None:
+        w.u2h, w.u2l, w.sc = dv(u2h), dv(u2l), dv(torch.cat([rng, inv]))
     return w
 
 
@@ -179,6 +193,7 @@ STAGE0_GRID = 0  # persistent stage-0 workgroups; 0 = one per CU (256)
 # results are those of the bands of few images, bit by bit.
 WINO_ROUNDS = 2
 WINO_RANGE = 65536  # its fp16 terms hold a range of this much beside conv1's biases; wider images go the direct way there
+WINO_IMAGES = 256  # magnitudes that have to be in range, raw pixels among them, for weights to take it
 # strided fp32 rows below this batch are written by the GEMM over [hi | hi | lo] rows; from it
 # on the fused fc1, without a split of K, is the faster one (us, GEMM : fused: 8192 rows 197 :
 # 237, 9216 251 : 230, 16384 324 : 235).  Outputs of another type or layout are the GEMM's.

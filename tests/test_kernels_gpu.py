@@ -569,6 +569,55 @@ def test_cifar_without_biases_stays_direct():
     assert torch.equal(cops.stage0_forward(x, w0, grid=1), cops.stage0_forward(x, w0, grid=5))
 
 
+def _spread(kind, sd):
+    sd = {k: v.clone() for k, v in sd.items()}
+    if kind in ("bias", "dead"):  # one channel's bias, which half of the outputs do not read
+        sd["conv1.bias"][3] = 1e7 if kind == "bias" else -1e7
+        sd["conv2.weight"][::2, 3] = 0
+    if kind == "weights":  # one channel small in conv1 and large in conv2
+        for k in ("conv1.weight", "conv1.bias"):
+            sd[k][3] *= 2.0 ** -24
+        sd["conv2.weight"][:, 3] *= 2.0 ** 24
+    if kind == "little":  # images beyond 40 reach past the range beside these biases
+        sd["conv1.bias"] *= 0.02
+    if kind == "none":
+        sd["conv2.weight"].zero_()
+    if kind == "holes":  # a filter of zeros loses nothing, a lost channel bounds nothing
+        sd["conv2.weight"][5, 7] = 0
+        sd["conv1.weight"][9, 0, 1, 1], sd["conv1.bias"][11] = float("inf"), float("nan")
+    return sd
+
+
+@pytest.mark.parametrize("kind,takes", [("plain", True), ("none", True), ("holes", True), ("bias", False), ("dead", False),
+                                        ("weights", False), ("little", False)])
+def test_cifar_winograd_takes_weights(kind, takes):
+    """Weights of a spread that one scale an image or an output channel would cut bits of stay with the direct form; where
+    they do not, conv2 of few images and of many is as close to 64 bits (bounds: test_cifar_winograd)."""
+    from distributed_neural_networks_amd.ops import cifar as cops
+    sd, x, _, _ = _cifar_golden(5, 5)
+    sd = _spread(kind, sd)
+    w0, x = cops.pack_stage0(sd, DEV), x.to(DEV)
+    h = cops.stage0_forward(x, w0, grid=1)
+    if kind != "holes":
+        ref, own, wide = _stage0_in_64_bits(sd, x)
+        assert ((h.double() - ref).abs() <= own * 3 * 2.0 ** -17 + wide * 36 * 2.0 ** -19).all()
+    assert (w0.u2h is not None) == takes
+
+
+def test_cifar_winograd_raw_pixels():
+    """Images of 0 to 255 are in range: Winograd's form (other bits than the direct one), the bounds of test_cifar_winograd."""
+    from distributed_neural_networks_amd.ops import cifar as cops
+    sd, x, _, _ = _cifar_golden(6, 6)
+    x = torch.randint(0, 256, x.shape, generator=torch.Generator().manual_seed(6)).float()
+    x[:, :, 8:20, 8:20] = 0
+    w0, x = cops.pack_stage0(sd, DEV), x.to(DEV)
+    h, direct = (cops.stage0_forward(x, w0, grid=g) for g in (2, 6))
+    ref, own, wide = _stage0_in_64_bits(sd, x)
+    assert ((h.double() - ref).abs() <= own * 3 * 2.0 ** -17 + wide * 36 * 2.0 ** -19).all()
+    assert all(not torch.equal(a, b) for a, b in zip(h, direct))
+    assert (h.double() - ref).norm() <= 1.05 * (direct.double() - ref).norm()
+
+
 @pytest.mark.parametrize("boundary", ["fp32", "split"])
 def test_cifar_fp32_pipeline_large_batch_fused_fc1(boundary):
     """The large-batch fp32 head (fused fc1) on 20000 images: max |dprob| <= 1e-5
