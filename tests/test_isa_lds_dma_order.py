@@ -27,6 +27,7 @@ import re
 import shutil
 import subprocess
 import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 
@@ -47,8 +48,18 @@ CONFIGS = [
     (2, 4, "true", 0, "ACT_NONE", "true", 2),     # split-K slab variant
 ]
 
-# <W8, NORM, NCH, CPP, GS>: the GPT-2 and GPT-2 XL fp8 heads of the decode step
-HEADS = [("false", 2, 24, 24, 12), ("true", 2, 25, 14, 5)]
+
+def _heads():
+    """<W8, NORM, NCH, CPP, GS, MT> of every decode head that dnn_gemm_head launches: its table (gemm_skinny.hip HEADC:
+    W8, chunks, chunks a pass and a group for four row tiles, chunks a group for one in one pass) x the norms."""
+    with open(os.path.join(ROOT, "csrc", "kernels", "gemm_skinny.hip")) as f:
+        rows = re.findall(r"^  HEADC\((true|false), (\d+), (\d+), (\d+), (\d+)\)", f.read(), re.M)
+    out = []
+    for w8, nch, cpp, gs, gs1 in ((r[0], *map(int, r[1:])) for r in rows):
+        for norm in (0, 1, 2):
+            out += [(w8, norm, nch, cpp, gs, 4), (w8, norm, nch, (nch + 3) // 4 * 4, gs1, 1)]
+    return out
+
 
 SRC = """#include "kernels/gemm_oneshot.h"
 #include "kernels/gemm_head.h"
@@ -77,11 +88,14 @@ def _asm(extra=None):
 
 
 def _asm_build(extra):
-    items = ", ".join([f"(void*)&gemm_oneshot_kernel<{mt}, {ntw}, {w8}, {norm}, {act}, {split}, {steps}>"
-                       for mt, ntw, w8, norm, act, split, steps in CONFIGS] +
-                      [f"(void*)&gemm_oneshot_kernel<{mt}, {ntw}, {w8}, {norm}, {act}, {split}, {steps}, {abl}>"
-                       for mt, ntw, w8, norm, act, split, steps, abl in RACY] +
-                      [f"(void*)&gemm_head_kernel<{w8}, {norm}, {nch}, {cpp}, {gs}>" for w8, norm, nch, cpp, gs in HEADS])
+    return _compile([f"(void*)&gemm_oneshot_kernel<{mt}, {ntw}, {w8}, {norm}, {act}, {split}, {steps}>"
+                     for mt, ntw, w8, norm, act, split, steps in CONFIGS] +
+                    [f"(void*)&gemm_oneshot_kernel<{mt}, {ntw}, {w8}, {norm}, {act}, {split}, {steps}, {abl}>"
+                     for mt, ntw, w8, norm, act, split, steps, abl in RACY], extra)
+
+
+def _compile(kernels, extra):
+    items = ", ".join(kernels)
     d = tempfile.mkdtemp(prefix="dnn_isa_")
     src, out = os.path.join(d, "oneshot_isa.hip"), os.path.join(d, "oneshot_isa.s")
     with open(src, "w") as f:
@@ -200,19 +214,38 @@ def _unretired_reads(lines, barriers: int = 1):
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
 def test_lds_dma_images_retired_before_reads():
     text = _asm()
-    for kernel, n in (("gemm_oneshot_kernel", len(CONFIGS)), ("gemm_head_kernel", len(HEADS))):
-        ks = _product(_kernels(text, kernel, raw=True))
-        assert len(ks) == n, (kernel, sorted(ks))
-        for name, seq in ks.items():
-            assert any("global_load_lds" in t for t in seq), name
-            bad = _unretired_reads(seq, 1)
-            assert not bad, f"{name}: {len(bad)} LDS reads before the image DMA is retired: {bad[:3]}"
+    ks = _product(_kernels(text, raw=True))
+    assert len(ks) == len(CONFIGS), sorted(ks)
+    _assert_retired(ks)
     # the racy variants must be flagged (the check sees the bug): the counted
     # wait (ABL 128)
     racy = {n: q for n, q in _kernels(text, raw=True).items() if n not in _product({n: q})}
     assert len(racy) == len(RACY), sorted(racy)
     for name, seq in racy.items():
         assert _unretired_reads(seq, 1), f"{name}: counted-wait variant not flagged"
+
+
+def _assert_retired(ks):
+    for name, seq in ks.items():
+        assert any("global_load_lds" in t for t in seq), name
+        bad = _unretired_reads(seq, 1)
+        assert not bad, f"{name}: {len(bad)} LDS reads before the image DMA is retired: {bad[:3]}"
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+def test_head_images_retired_before_reads():
+    """The decode head as it is launched: every width, four row tiles and one, every norm."""
+    heads = _heads()
+    with open(os.path.join(ROOT, "csrc", "kernels", "gemm_skinny.hip")) as f:
+        src = f.read()
+    assert len(heads) == 6 * (src.count("HEADC(") - 1) and "NCHV, (NCHV + 3) / 4 * 4, GS1V>" in src  # as the table's macro has it
+    names = [f"(void*)&gemm_head_kernel<{', '.join(map(str, h))}>" for h in heads]
+    ks = {}
+    with ThreadPoolExecutor(4) as pool:  # threads that wait for compilers
+        for text in pool.map(lambda n: _compile(n, _lib_flags()), [names[i::4] for i in range(4)]):
+            ks.update(_kernels(text, "gemm_head_kernel", raw=True))
+    assert len(ks) == len(heads), sorted(ks)
+    _assert_retired(ks)
 
 PK_CROSS = re.compile(r"^v_pk_\w+_f32\b.*\bop_sel:\[")
 
