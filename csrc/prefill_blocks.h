@@ -157,11 +157,14 @@ struct PrefillPass {
     const int nq = (H + 2 * Hkv) * hd;
     const int one_group = fp8 && rows() > skinny_max;  // e4m3 activations follow (attention.hip flash_two_groups)
     const bool up_quant = fp8 && act == 2 && !skinny(n_up, d, true, true, 0);
-    const bool part = parts != nullptr && !fp8;  // who reads h's partials
-    const bool read_up = part && dnn_gemm_takes_parts(rows(), n_up, d, d, d, act, 0, ws_bytes);
-    const bool read_qkv = part && scatter && cosT == nullptr && dnn_gemm_takes_parts(rows(), nq, d, d, d, 0, 1, 0);
+    const bool part = parts != nullptr && !fp8;
     for (size_t i = 0; i < blocks.size(); ++i) {
       const PrefillBlock& L = blocks[i];
+      // who reads h's partials: not the decode kernels, and none is behind the last block
+      const bool read_up = part && !skinny(n_up, d, true, L.up.frag != nullptr, ws_bytes) &&
+                           dnn_gemm_takes_parts(rows(), n_up, d, d, d, act, 0, ws_bytes);
+      const bool read_qkv = part && scatter && cosT == nullptr && (more || i + 1 < blocks.size()) &&
+                            !skinny(nq, d, true, L.qkv.frag != nullptr, 0) && dnn_gemm_takes_parts(rows(), nq, d, d, d, 0, 1, 0);
       void *k = kc + i * kv_block, *v = vc + i * kv_block;
       int rc;
       if (scattered(in, L.qkv, k, v, rc)) {
@@ -184,7 +187,7 @@ struct PrefillPass {
       if (rc) return rc;
       if ((rc = res_proj(att, L.o, in, H * hd, false, read_up))) return rc;
       if ((rc = norm_proj(h, L.up, f, ffn, n_up, act, false, up_quant))) return rc;
-      if ((rc = res_proj(f, L.down, h, ffn, up_quant, read_qkv && (more || i + 1 < blocks.size())))) return rc;
+      if ((rc = res_proj(f, L.down, h, ffn, up_quant, read_qkv))) return rc;
       in = h;
     }
     return 0;

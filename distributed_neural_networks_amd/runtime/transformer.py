@@ -460,11 +460,13 @@ class TransformerStage(StageCompute):
         # prefill: the same by partials of 32 columns, where the projection that follows merges them
         rp_up = rp_qkv = None
         if T > 1 and not one_call and self.rowparts is not None and self.layers:
-            up, nq = self.layers[0].w_up, (self.H + 2 * self.Hkv) * self.hd
+            L, nq = self.layers[0], (self.H + 2 * self.Hkv) * self.hd
             act = ACT_GELU if self.family == "gpt2" else ACT_SILU_MUL
-            rp_up = self.rowparts if G_.takes_parts(ntok, up.w.shape[0], d, act, gws) else None
-            rp_qkv = (self.rowparts if G_.QKV_SCATTER and self.cos is None and G_.takes_parts(ntok, nq, d, scatter=True)
-                      else None)
+            if not G_._norm_skinny(h, L.w_up, act, True, gws) and G_.takes_parts(ntok, L.w_up.w.shape[0], d, act, gws):
+                rp_up = self.rowparts
+            if (G_.QKV_SCATTER and self.cos is None and not G_._norm_skinny(h, L.w_qkv, ACT_NONE, True)
+                    and G_.takes_parts(ntok, nq, d, scatter=True)):
+                rp_qkv = self.rowparts
         for li, L in enumerate(() if one_call else self.layers):
             kc, vc = self.kc[li, b0:b0 + B], self.vc[li, b0:b0 + B]
             att = self.buf_att[r0:r1]
@@ -508,7 +510,7 @@ class TransformerStage(StageCompute):
                 T_.layernorm(h, L.ln2_w, L.ln2_b, a, self.eps, self.rms, rows=ntok)
                 f, _ = self._lin(a, L.w_up, L.b_up, act=up_act, out=self.buf_f[r0:r1])
             _, have_rs = self._lin(f, L.w_down, L.b_down, residual=h, out=h, w_shuf=L.w_down_s, ws=gws, rs_out=rs,
-                                   mx_in=mx_f, parts_out=rp_qkv)
+                                   mx_in=mx_f, parts_out=rp_qkv if li + 1 < len(self.layers) else None)
             h_in = h
         if not self.last:
             if out is not None:

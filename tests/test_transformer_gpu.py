@@ -1802,6 +1802,28 @@ def test_row_statistics_by_partials(tile, splits, M, d, rms):
         G.lib().gemm_set_mid(-1, 1)
 
 
+def _three_blocks(B, T):
+    from distributed_neural_networks_amd import checkpoint as ckpt
+    from distributed_neural_networks_amd.runtime.transformer import build_device_stage
+    sd = ckpt.random_stage_state_dict("gpt2", 0, 2, True, False, 3, nontrivial=True)
+    st = build_device_stage("gpt2", sd, 0, 2, True, False, DEV, dtype="bf16", max_batch=B, max_seq=T, max_tokens=B * T)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    return st, torch.randint(0, 50257, (B, T), dtype=torch.int32, device=DEV, generator=g), torch.zeros(B, dtype=torch.int32, device=DEV)
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("B,T,read", [(1, 100, False), (3, 357, True)])
+def test_partials_written_where_read(B, T, read, native, monkeypatch):
+    """100 rows: the projections behind the norms run on the decode kernels, and nobody writes partials for them."""
+    from distributed_neural_networks_amd.runtime.transformer import TransformerStage
+    st, ids, pos = _three_blocks(B, T)
+    if not native:
+        monkeypatch.setattr(TransformerStage, "_prefill_blocks", lambda self, *a: False)
+    st.rowparts.fill_(float("nan"))
+    st.step(ids, pos, B, T)
+    assert bool(torch.isfinite(st.rowparts).any()) == read
+
+
 @pytest.mark.parametrize("far", ["rows", "weights"])
 @pytest.mark.parametrize("scatter", [False, True])
 def test_partials_of_rows_far_apart(far, scatter):
