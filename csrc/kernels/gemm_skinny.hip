@@ -96,8 +96,10 @@ __device__ __forceinline__ void sk_stats(const i32x4& a, float c, float& s1, flo
   }
 }
 
+// HV (host: 4 waves): a wave owns two slices of K, the lower and the upper half of a batch, each with sums of its own: 4 waves in place
+// of 8 and the sums of 8, bit by bit (a slice twice as long is 9 % further from 64 bits at K = 768).
 template <int ACT, bool OUT_F32, int MT, int NT, bool FP8, int U, bool PIPE = false, int NORM = NORM_NONE,
-          bool W8 = false, bool MS = false>
+          bool W8 = false, bool MS = false, bool HV = false>
 __global__ __launch_bounds__(512) void gemm_skinny_kernel(const uint8_t* __restrict__ A, int lda_b,
                                                            const float* __restrict__ sa, const uint8_t* __restrict__ W,
                                                            int ldw_b, const float* __restrict__ sw,
@@ -109,10 +111,12 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const uint8_t* __restr
                                                            float2* __restrict__ rs_out = nullptr, int rs_ld = 0,
                                                            int epi_pre = 1) {
   static_assert(NORM == NORM_NONE || !FP8, "fused norm needs bf16 activations");
+  static_assert(!HV || (!PIPE && U % 2 == 0), "a batch of two halves");
+  constexpr int G = HV ? 2 : 1;
   static_assert(!(FP8 && W8), "W8 = fp8 weights with bf16 activations; FP8 = both fp8");
   constexpr int AU = W8 ? 2 : 1;        // 16-B A loads per chunk per M tile (W8: a chunk is 64 k = 128 B of A)
   constexpr int ACH = W8 ? 128 : 64;    // A bytes per row per chunk
-  extern __shared__ __attribute__((aligned(16))) f32x4 sk_red[];  // [KS][NT*MT][64], then [KS][MT][16] x2 stats
+  extern __shared__ __attribute__((aligned(16))) f32x4 sk_red[];  // [KS * G][NT*MT][64], then [KS * G][MT][16] x2 stats
   // wave index via readfirstlane: the K-slice bounds and the surplus-chunk tests
   // below are then scalar (s_cbranch), not exec-masked VALU branches
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), KS = blockDim.x >> 6;
@@ -198,15 +202,18 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const uint8_t* __restr
                                                               : reinterpret_cast<const bf16_t*>(dummy));
     }
   }
-  f32x4 acc[NT][MT];
+  f32x4 acc[G][NT][MT];
 #pragma unroll
-  for (int j = 0; j < NT; ++j)
+  for (int g = 0; g < G; ++g)
 #pragma unroll
-    for (int t = 0; t < MT; ++t) acc[j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float st1[MT], st2[MT], shift[MT];  // shifted row statistics of this lane's A fragments (NORM)
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) acc[g][j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float st1[G][MT], st2[G][MT], shift[MT];  // shifted row statistics of this lane's A fragments (NORM)
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
-    st1[t] = st2[t] = 0.f;
+#pragma unroll
+    for (int g = 0; g < G; ++g) st1[g][t] = st2[g][t] = 0.f;
     shift[t] = 0.f;
     if constexpr (NORM == NORM_LN) {  // RMS has no subtraction to protect: c = 0
       int m = t * 16 + (lane & 15);
@@ -216,7 +223,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const uint8_t* __restr
   }
 
   const int nch = kbytes >> 6;
-  const int per = (nch + KS - 1) / KS;
+  const int per = (nch + KS * G - 1) / (KS * G) * G;
   const int c0 = wave * per, c1 = min(nch, c0 + per);
   // Batches of U chunks; the last batch of a wave is partial: its loads are
   // clamped in-bounds and the surplus chunks' weights zeroed, so every batch
@@ -252,6 +259,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const uint8_t* __restr
   auto comp = [&](int cc, i32x4(&wv)[NT][U], const i32x4(&av)[MT][U * AU]) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
+      const int g = HV && u >= U / 2 ? 1 : 0;
       if (cc + u >= c1) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) wv[j][u] = i32x4{0, 0, 0, 0};
@@ -259,7 +267,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const uint8_t* __restr
 #pragma unroll
         for (int t = 0; t < MT; ++t)
 #pragma unroll
-          for (int h = 0; h < AU; ++h) sk_stats<NORM>(av[t][u * AU + h], shift[t], st1[t], st2[t]);
+          for (int h = 0; h < AU; ++h) sk_stats<NORM>(av[t][u * AU + h], shift[t], st1[g][t], st2[g][t]);
       }
       if constexpr (W8) {
         // the lane's 16 weight bytes are k = 16g..16g+15 of the chunk; its two A
@@ -273,15 +281,15 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const uint8_t* __restr
             bf16x8 a0, a1;
             __builtin_memcpy(&a0, &av[t][2 * u], 16);
             __builtin_memcpy(&a1, &av[t][2 * u + 1], 16);
-            acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wlo, a0, acc[j][t], 0, 0, 0);
-            acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(whi, a1, acc[j][t], 0, 0, 0);
+            acc[g][j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wlo, a0, acc[g][j][t], 0, 0, 0);
+            acc[g][j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(whi, a1, acc[g][j][t], 0, 0, 0);
           }
         }
       } else {
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-          for (int t = 0; t < MT; ++t) acc[j][t] = sk_mma<FP8>(wv[j][u], av[t][u], acc[j][t]);
+          for (int t = 0; t < MT; ++t) acc[g][j][t] = sk_mma<FP8>(wv[j][u], av[t][u], acc[g][j][t]);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -311,28 +319,32 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const uint8_t* __restr
     }
   }
 #pragma unroll
-  for (int j = 0; j < NT; ++j)
+  for (int g = 0; g < G; ++g)
 #pragma unroll
-    for (int t = 0; t < MT; ++t) sk_red[(wave * NT * MT + j * MT + t) * 64 + lane] = acc[j][t];
-  float* sk_st = reinterpret_cast<float*>(sk_red + KS * NT * MT * 64);  // [KS][MT][2][16]
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) sk_red[((wave * G + g) * NT * MT + j * MT + t) * 64 + lane] = acc[g][j][t];
+  float* sk_st = reinterpret_cast<float*>(sk_red + KS * G * NT * MT * 64);  // [KS * G][MT][2][16]
   if constexpr (NORM != NORM_NONE) {
     // the 4 lane groups hold disjoint 16-B pieces of the same 16 rows
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      float a = st1[t], q = st2[t];
-      a = add16(a);
-      a = add32(a);
-      q = add16(q);
-      q = add32(q);
-      if (lane < 16) {
-        sk_st[((wave * MT + t) * 2 + 0) * 16 + lane] = a;
-        sk_st[((wave * MT + t) * 2 + 1) * 16 + lane] = q;
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        float a = st1[g][t], q = st2[g][t];
+        a = add16(a);
+        a = add32(a);
+        q = add16(q);
+        q = add32(q);
+        if (lane < 16) {
+          sk_st[(((wave * G + g) * MT + t) * 2 + 0) * 16 + lane] = a;
+          sk_st[(((wave * G + g) * MT + t) * 2 + 1) * 16 + lane] = q;
+        }
       }
-    }
   }
   __syncthreads();
 
-  // reduction over the KS waves + epilogue: wave w finishes M tiles t = w, w+KS, ...
+  // reduction over the waves' slices + epilogue: wave w finishes M tiles t = w, w+KS, ...
   const bool vec = epi_vec_ok(Cv, ldc, bias, R, ldr);
   const f32x2 xc = act_consts<ACT>(bias, N);
   for (int t = wave; t < MT; t += KS) {
@@ -340,6 +352,14 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const uint8_t* __restr
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       s[j] = sk_red[(j * MT + t) * 64 + lane];
+      if constexpr (HV) {  // all reads at once: a loop over the waves waits for each (8 slices 0.25 us)
+        f32x4 v[8];
+#pragma unroll
+        for (int w = 1; w < 8; ++w) v[w] = sk_red[(w * NT * MT + j * MT + t) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < 8; ++w) s[j] += v[w];
+        continue;
+      }
       for (int w = 1; w < KS; ++w) s[j] += sk_red[(w * NT * MT + j * MT + t) * 64 + lane];
     }
     const int m = t * 16 + (lane & 15);
@@ -361,7 +381,13 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const uint8_t* __restr
     }
     if constexpr (NORM != NORM_NONE) {
       float a = 0.f, q = 0.f;
-      for (int w = 0; w < KS; ++w) {
+      constexpr int SL = HV ? 8 : 0;
+#pragma unroll
+      for (int w = 0; w < SL; ++w) {
+        a += sk_st[((w * MT + t) * 2 + 0) * 16 + (lane & 15)];
+        q += sk_st[((w * MT + t) * 2 + 1) * 16 + (lane & 15)];
+      }
+      for (int w = SL; w < KS; ++w) {
         a += sk_st[((w * MT + t) * 2 + 0) * 16 + (lane & 15)];
         q += sk_st[((w * MT + t) * 2 + 1) * 16 + (lane & 15)];
       }
@@ -812,9 +838,9 @@ extern "C" int dnn_gemm_set_stream(int on, long long min_bytes, int fold) {
 // NT x MT MFMAs.  The configuration table below is fitted to
 // bench/skinny_sweep.py on MI355X (profiles/archive/r1_skinny_sweep.jsonl, weights
 // rotated past the 256 MB MALL):
-//   M <= 8     : 1 tile, 4 chunks in flight, 8 waves/WG (within 3% of the best
-//                row-major config on every Llama-3 / GPT-2 XL shape); with the
-//                fragment-order copy (Wsh) the per-class rules below
+//   M <= 8     : 1 tile, 8 slices of K: 4 or 6 chunks in flight on 8 waves (within 3% of the best
+//                row-major config on every Llama-3 / GPT-2 XL shape), short K in bf16 on 4 waves of two
+//                slices (CFG_EIGHT); with the fragment-order copy (Wsh) the per-class rules below
 //   M <= 16    : N <= 4096: as M <= 8; wide N (>= 16K): 4 tiles x 2 chunks, 2 waves; else 2 tiles x 2
 //                chunks pipelined, 4 waves
 //   M <= 64    : by N class (wide >= 16K / mid / narrow <= 4K): 4 / 2 / 1 column
@@ -855,36 +881,28 @@ static bool w8_rows64(int M, int N, int K, bool norm) {
   return t64 + (norm ? 0.7f : 0.f) < 0.98f * t16;
 }
 
-template <int ACT, bool F32, bool FP8, int MT, int NT, int U, bool PIPE, int NORM, bool W8, bool MS = false>
+template <int ACT, bool F32, bool FP8, int MT, int NT, int U, bool PIPE, int NORM, bool W8, bool MS = false, bool HV = false>
 static int launch_skinny_cfg(const void* A, int lda_b, const float* sa, const void* W, int ldw_b, const float* sw,
                              void* C, int ldc, const float* bias, const void* R, int ldr, int M, int N, int kbytes,
                              int ks, const float* colsum, float eps, hipStream_t st, const void* Wsh) {
   const int groups = (N + 16 * NT - 1) / (16 * NT) * (MS ? (M + 16 * MT - 1) / (16 * MT) : 1);
   while (ks > 1 && kbytes / 64 < ks) ks >>= 1;
-  size_t smem = (size_t)ks * NT * MT * 64 * sizeof(f32x4);
-  if (NORM != NORM_NONE) smem += (size_t)ks * MT * 2 * 16 * sizeof(float);
+  const size_t slices = HV ? 2 * ks : ks;
+  size_t smem = slices * NT * MT * 64 * sizeof(f32x4);
+  if (NORM != NORM_NONE) smem += slices * MT * 2 * 16 * sizeof(float);
   float2* rso = (!F32 && !FP8 && !is_glu(ACT)) ? g_rs_cur.out : nullptr;
-  hipLaunchKernelGGL((gemm_skinny_kernel<ACT, F32, MT, NT, FP8, U, PIPE, NORM, W8, MS>), dim3(groups), dim3(64 * ks), smem,
+  hipLaunchKernelGGL((gemm_skinny_kernel<ACT, F32, MT, NT, FP8, U, PIPE, NORM, W8, MS, HV>), dim3(groups), dim3(64 * ks), smem,
                      st, (const uint8_t*)A, lda_b, sa, (const uint8_t*)W, ldw_b, sw, C, ldc, bias, (const bf16_t*)R,
                      ldr, M, N, kbytes, colsum, eps, (const uint8_t*)Wsh, rso, g_rs_cur.out_ld, g_epi_pre);
   if (rso != nullptr) g_rs_written = 1;
   return (int)hipGetLastError();
 }
 
-// Waves and chunks a batch of a workgroup that owns one 16 x 16 tile: as few waves as take K in one
-// batch each, and the batch that leaves fewer requests past a wave's range (those are made all the
-// same, and short products are bound by their requests, W and A).  us, 4 chunks on 8 waves : this, bf16 in
-// fragment order, weights from memory: 1 row, 768 x 768 3.20 : 2.84, 2304 x 768 3.48 : 3.13, 3072 x 768 3.62 :
-// 3.26, 1536 x 512 3.26 : 2.82, 1280 x 1280 4.10 : 3.64; 16 rows, 768 x 768 4.04 : 3.54, 1536 x 512 3.91 : 3.25;
-// 64 rows (4 chunks on 4 waves), 768 x 768 4.31 : 3.99.  The same from 49 chunks on, but for 65 to 72, 4.78 : 4.53.
-struct Few {
-  int u, ks;
-};
-static Few few_plan(bool w8, int kbytes) {
-  const int nch = kbytes / 64;
-  if (w8) return {4, 8};
-  const int ks = nch <= 24 ? 4 : 8, per = (nch + ks - 1) / ks;
-  return {nch <= 48 && (per + 5) / 6 * 6 < (per + 3) / 4 * 4 ? 6 : 4, ks};
+// A workgroup that owns one 16 x 16 tile: the batch that leaves fewer requests past a wave's range (those are made all
+// the same, and short products are bound by their requests, W and A).  `ks` waves, 6 chunks a batch in place of 4?
+static bool few_six(int nch, int ks) {
+  const int per = (nch + ks - 1) / ks;
+  return nch <= 48 && (per + 5) / 6 * 6 < (per + 3) / 4 * 4;
 }
 
 template <int ACT, bool F32, bool FP8, int NORM = NORM_NONE, bool W8 = false>
@@ -920,6 +938,24 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
 #define CFG(MTV, NTV, UV, PV, KSV)                                                                                   \
   return launch_skinny_cfg<ACT, F32, FP8, MTV, NTV, UV, PV, NORM, W8>(A, lda_b, sa, W, ldw_b, sw, C, ldc, bias, R,   \
                                                                        ldr, M, N, kbytes, KSV, colsum, eps, st, Wsh)
+// One column tile, slices of K as of 8 waves: 8 to 24 chunks on 4 waves of two slices each (HV), a batch as long as both.
+// us, bf16 in fragment order, weights from memory, 4 chunks on 8 waves : this: 1 row, 768 x 768 3.28 :
+// 2.88, 2304 x 768 3.47 : 3.12, 3072 x 768 3.64 : 3.30, 1536 x 512 3.30 : 2.83, 768 x 256 3.13 : 2.59; 16 rows, 768 x 768 4.00 :
+// 3.51, 1536 x 512 3.93 : 3.34; 6 chunks on 8 waves, 1280 x 1280 4.16 : 3.72.
+#define CFG_EIGHT()                                                                                                   \
+  do {                                                                                                                \
+    if (nch >= 8 && nch <= 24) {                                                                                      \
+      if (nch > 16) CFG_HV(6);                                                                                        \
+      if (nch > 8) CFG_HV(4);                                                                                         \
+      CFG_HV(2);                                                                                                      \
+    }                                                                                                                 \
+    if (few_six(nch, 8)) CFG(1, 1, 6, false, 8);                                                                      \
+    CFG(1, 1, 4, false, 8);                                                                                           \
+  } while (0)
+#define CFG_HV(UV)                                                                                                    \
+  return launch_skinny_cfg<ACT, F32, FP8, 1, 1, UV, false, NORM, W8, false, true>(A, lda_b, sa, W, ldw_b, sw, C, ldc,  \
+                                                                                  bias, R, ldr, M, N, kbytes, 4,      \
+                                                                                  colsum, eps, st, Wsh)
 #define CFG_MS(NTV, UV, PV, KSV)                                                                                 \
   return launch_skinny_cfg<ACT, F32, FP8, 1, NTV, UV, PV, NORM, W8, true>(A, lda_b, sa, W, ldw_b, sw, C, ldc, bias, \
                                                                            R, ldr, M, N, kbytes, KSV, colsum, eps, st, \
@@ -955,13 +991,16 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
     if (N <= 1024) CFG_MS(1, 4, false, 4);
     CFG_MS(2, 2, false, 4);
   }
-  const Few few = few_plan(FP8 || W8, kbytes);
+  constexpr bool BF = !FP8 && !W8;
+  const int nch = kbytes / 64;
   if (M <= 8) {
     // batch 1-8: the fragment-order copy (Wsh) is streamed whenever the layer
-    // attached one; per shape class: QKV-sized N 1 tile x 4 chunks on 4 waves
+    // attached one; per shape class: QKV-sized N 1 tile x 4 or 6 chunks on 4 waves
     // (Llama-3 8B fp8 decode graph 12.25 -> 10.33 us), the rest below
     if (!FP8 && Wsh != nullptr && N > 4096 && N < 16384 && kbytes <= 8192) {
-      if (few.u == 6 && few.ks == 4) CFG(1, 1, 6, false, 4);
+      if constexpr (BF) {
+        if (few_six(nch, 4)) CFG(1, 1, 6, false, 4);
+      }
       CFG(1, 1, 4, false, 4);
     }
     // fp8 vocabulary head (128K x 4K, fragment order): 2 column tiles per wave
@@ -970,8 +1009,8 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
     // fp8 gate|up (28K x 4K) with the fused RMSNorm: 2 column tiles x 2 chunks
     // on 2 waves 23.3 -> 21.3 us (profiles/archive/r2_w8_decode_projections.jsonl)
     if (W8 && Wsh != nullptr && N >= 16384) CFG(1, 2, 2, false, 2);
-    if (few.u == 6) CFG(1, 1, 6, false, few.ks);
-    CFG(1, 1, 4, false, few.ks);
+    if constexpr (BF) CFG_EIGHT();
+    else CFG(1, 1, 4, false, 8);
   }
   if (M <= 16) {
     // narrow N: one column tile a workgroup, as for M <= 8.  Two put 64 to 128 workgroups
@@ -980,8 +1019,11 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
     // 2048 x 7680 30.4 : 19.8; e4m3 4096 x 14336 23.9 : 19.0, 1600 x 6400 11.9 : 10.4 (the
     // last four on 4 waves: 8 are up to 10 % slower there and faster above)
     if (!FP8 && N <= 4096) {
-      if (few.u == 6) CFG(1, 1, 6, false, few.ks);
-      CFG(1, 1, 4, false, (W8 || Wsh == nullptr) ? 4 : few.ks);
+      if constexpr (BF) {
+        if (Wsh != nullptr) CFG_EIGHT();
+        if (few_six(nch, 4)) CFG(1, 1, 6, false, 4);
+      }
+      CFG(1, 1, 4, false, 4);
     }
     // wide N in fragment order, K from 2048: 28672 x 4096, 12 rows 45.9 : 40.7, 16 rows
     // 45.2 : 44.0, 32768 x 4096 49.9 : 46.2 (50257 x 768 the other way, 19.8 : 23.2)
@@ -1006,7 +1048,9 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
       CFG(4, 4, 2, false, 2);
     }
     if (N <= 1024) {
-      if (few.u == 6 && few.ks == 4) CFG_MS(1, 6, false, 4);
+      if constexpr (BF) {
+        if (few_six(nch, 4)) CFG_MS(1, 6, false, 4);
+      }
       CFG_MS(1, 4, false, 4);
     }
     // (8-wave variants of the Llama-3 8B B=32 QKV / O rules below measured within
@@ -1022,6 +1066,8 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
   }
 #undef CFG_MS
 #undef CFG_MM
+#undef CFG_EIGHT
+#undef CFG_HV
   const bool deep = kbytes >= 16384;
   const bool narrow = N <= 4096;
   if (M <= 32) {

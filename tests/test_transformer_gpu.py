@@ -885,6 +885,21 @@ def test_skinny_batches(M, N, K):
     assert bool(((linear_norm(x, f).double() - ref * r).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("K", [640, 768])
+def test_skinny_slices_of_few_rows(K):
+    """Up to 16 rows sum K in eight slices, 64 rows in four: the first is nearer to 64 bits (chains of three products for six;
+    measured 0.91 of the distance, with slices of one length 1)."""
+    from distributed_neural_networks_amd.ops.gemm import linear, shuffle_weight
+    few = many = 0.0
+    for seed in range(6):
+        g = torch.Generator(device=DEV).manual_seed(seed)
+        x, w = torch.randn(64, K, device=DEV, generator=g).bfloat16(), torch.randn(768, K, device=DEV, generator=g).bfloat16()
+        ref, ws = (x.double() @ w.double().t())[:16], shuffle_weight(w)
+        few += (linear(x[:16], w, w_shuf=ws, out_dtype=torch.float32).double() - ref).pow(2).sum().item()
+        many += (linear(x, w, w_shuf=ws, out_dtype=torch.float32)[:16].double() - ref).pow(2).sum().item()
+    assert few ** 0.5 < 0.96 * many ** 0.5
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
 @pytest.mark.parametrize("N,K", [(100, 128), (2304, 768), (1600, 1600), (6144, 4096), (16400, 256)])
 def test_skinny_shuffled_weights_match(M, N, K):
