@@ -234,6 +234,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     if parts is not None or parts_out is not None:
         if o2.dtype != torch.bfloat16:
             raise ValueError("linear: partials need bf16 output")
+        if rs_out is not None:
+            raise ValueError("linear: rs_out (decode) and partials (prefill) exclude each other")
         t, eps, norm = parts if parts is not None else (None, 0.0, 0)
         rc, _LAST_RS[0] = lib().gemm_bf16_parts(ptr(x2), x2.stride(0), ptr(w), w.stride(0), ptr(o2), o2.stride(0), ptr(bias),
                                                 ptr(r2), 0 if r2 is None else r2.stride(0), M, N, K, a, stream_ptr(),
@@ -511,8 +513,8 @@ def head_argmax(x: torch.Tensor, f: FoldedLinear, logits: torch.Tensor, part: to
     the decode step tail (``also`` = copy of the ids, ``hist[row, advance]``
     = the id, ``advance += 1``).
     Returns False with nothing launched where it does not apply (more than 64
-    rows, a width without an instantiated config, a vocabulary over two
-    column tiles per wave): the caller then runs the GEMM and argmax_rows."""
+    rows, a width without an instantiated config, a vocabulary over 16
+    column tiles a compute unit): the caller then runs the GEMM and argmax_rows."""
     from .fp8 import Fp8Weight
     if not FUSED_HEAD or not isinstance(f, FoldedLinear):
         return False

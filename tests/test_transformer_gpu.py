@@ -1817,6 +1817,14 @@ def test_row_statistics_by_partials(tile, splits, M, d, rms):
         G.lib().gemm_set_mid(-1, 1)
 
 
+def test_linear_takes_one_kind_of_statistics():
+    """Decode's statistics and prefill's partials of the same rows in one call: refused, where rs_out was left unwritten."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    x, w = torch.randn(8, 64, device=DEV).bfloat16(), torch.randn(64, 64, device=DEV).bfloat16()
+    with pytest.raises(ValueError):
+        G.linear(x, w, rs_out=G.rowstats_buffer(8, 64, DEV), parts_out=G.parts_buffer(8, 64, DEV))
+
+
 def _three_blocks(B, T):
     from distributed_neural_networks_amd import checkpoint as ckpt
     from distributed_neural_networks_amd.runtime.transformer import build_device_stage
