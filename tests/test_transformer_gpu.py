@@ -1847,6 +1847,67 @@ def test_partials_written_where_read(B, T, read, native, monkeypatch):
     assert bool(torch.isfinite(st.rowparts).any()) == read
 
 
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("B,T", [(3, 357), (1, 259), (2, 500)])
+def test_prefill_by_partials(B, T, native, monkeypatch):
+    """Three blocks whose norms merge partials (written by the block before, across the two native calls too) against the
+    same blocks with a pass over the rows for their statistics.  Both are fp32 sums, so they differ where a rounding to
+    bf16 (1.1e-3 rms) falls the other way: at most in all of a block's four products, three blocks behind each
+    other, 1.1e-3 sqrt(12) = 4e-3.  Other rows' partials are off by far more."""
+    from distributed_neural_networks_amd.runtime.transformer import TransformerStage
+    st, ids, pos = _three_blocks(B, T)
+    if not native:
+        monkeypatch.setattr(TransformerStage, "_prefill_blocks", lambda self, *a: False)
+    got = []
+    for parts in (st.rowparts, None):
+        st.rowparts = parts
+        st.kc.zero_(), st.vc.zero_()
+        y = st.step(ids, pos, B, T)
+        got.append((y.clone(), st.kc.clone(), st.vc.clone()))
+    for a, b in zip(*got):
+        assert _rel(a, b) < 4e-3
+    assert not torch.equal(got[0][0], got[1][0])  # two routes
+
+
+@pytest.mark.parametrize("tile", range(7))
+@pytest.mark.parametrize("B,T,H,Hkv,hd,pos0,S,rms", [(1, 193, 12, 12, 64, 0, 200, False), (3, 43, 4, 2, 128, 5, 60, True),
+                                                     (2, 97, 25, 25, 64, 9, 100, False), (1, 66, 2, 1, 64, 0, 66, True)])
+def test_qkv_scatter_by_partials(tile, B, T, H, Hkv, hd, pos0, S, rms):
+    """The scatter epilogue behind a norm that merges partials, on every tile: the rows of the same product + qkv_split, and
+    both against float64 on the rows (the bound of test_row_statistics_by_partials)."""
+    from distributed_neural_networks_amd.ops import gemm as G
+    from distributed_neural_networks_amd.ops import transformer_ops as T_
+    g = torch.Generator(device=DEV).manual_seed(B * T + tile)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    M, d, N = B * T, 320, (H + 2 * Hkv) * hd
+    x, parts = torch.empty(M, d, device=DEV, dtype=torch.bfloat16), G.parts_buffer(M, d, DEV)
+    f = G.fold_norm(rnd(N, d) / math.sqrt(d), torch.rand(d, device=DEV, generator=g) + 0.5, None, rnd(N) * 0.02, rms, 1e-5, DEV)
+    std, pos = torch.empty(M, d, device=DEV, dtype=torch.bfloat16), torch.full((B,), pos0, device=DEV, dtype=torch.int32)
+    caches = [torch.zeros(B, Hkv, S, hd, device=DEV).bfloat16() for _ in range(4)]
+    q, q2 = (torch.empty(M * H * hd, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    G.set_gemm_mid(tile)
+    try:
+        G.linear(rnd(M, 128).bfloat16(), (rnd(d, 128) / 12).bfloat16(), None, residual=(rnd(M, d) + 9 * rnd(M, 1)).bfloat16(), out=x,
+                 parts_out=parts)
+        assert G.rowstats_written() and G.takes_parts(M, N, d, scatter=True)
+        std.fill_(float("nan"))  # where a pass over the rows leaves its statistics
+        assert G.qkv_scatter_norm(x, f, std, q, caches[0], caches[1], pos, B, T, H, Hkv, hd, parts=parts)
+        qkv = G.linear(x, f.w, f.bias, colsum=f.colsum, parts=(parts, f.eps, f.norm))
+    finally:
+        G.set_gemm_mid()
+    T_.qkv_split(qkv, q2, caches[2], caches[3], B, T, H, Hkv, hd, pos)
+    assert bool(torch.isnan(std).all())
+    keep = pos0 + torch.arange(T, device=DEV) < S
+    assert torch.equal(q.view(B, H, T, hd)[:, :, keep], q2.view(B, H, T, hd)[:, :, keep])
+    assert torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3])
+    r = x.double()
+    mu = r.mean(1, keepdim=True) * (0 if rms else 1)
+    rstd = torch.rsqrt((r - mu).pow(2).mean(1, keepdim=True) + f.eps)
+    ref = ((r - mu) * rstd) @ f.w.double().t() + f.bias.double()
+    bound = ref.abs() * 2.0 ** -8 + ((r.abs() @ f.w.double().abs().t()) * rstd + f.bias.abs()) * (d + 64) * 2.0 ** -24
+    assert bool(((qkv.double() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("far", ["rows", "weights"])
 @pytest.mark.parametrize("scatter", [False, True])
 def test_partials_of_rows_far_apart(far, scatter):
