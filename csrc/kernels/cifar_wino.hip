@@ -28,7 +28,10 @@
 // of an image so that what conv1 can reach at most (its weights' sum of magnitudes times the image's
 // largest finite magnitude, plus the bias) lies below 2^13; V then stays below 2^15.  The scale of the
 // map rides in conv1's bias addition, both inverses in conv2's.  An image whose range is too wide for one
-// scale goes the direct way at the end (wide_range, direct_images).
+// scale goes the direct way at the end (wide_range, direct_images), weights of such a spread take the direct form
+// at all times (ops/cifar.py _winograd_range).  As every form that sums a patch before it multiplies: an output
+// beside a part of its 4 x 4 patch that its own window does not see is off by 2^-21 of that part, so small outputs along
+// an edge to values over 2^4 times theirs are further off than by the window, all of an image nearer.
 //
 // Work.  One workgroup a CU walks over images, 4 phases an image with one barrier each.  Waves 0-3
 // ("producers") run conv1 of image it, two of its tile rows a phase, stage the next image, a quarter a phase, and

@@ -92,8 +92,8 @@ __device__ __forceinline__ float dpp_f(float v) {
 // The values of this lane and of the one 16 (32) away, in the order of the lanes: one
 // v_permlane16_swap (32_swap) where a __shfl_xor is a round trip through the LDS unit, some 130
 // clocks of a chain: the launches of one to 64 rows are chains of a few microseconds with two to
-// four of these in each (a GPT-2 decode step of one row 288.8 -> 283.6 us, of 64 rows 543 -> 537,
-// of 64 rows in fp8 359.0 -> 351.5).  The bits are those of the shuffles.  Every lane of the wave
+// four of these in each (a GPT-2 decode step of one row 288.8 -> 283.6 us; steps of 64 rows within
+// their spread).  The bits are those of the shuffles.  Every lane of the wave
 // (16: of its half) must call it.
 __device__ __forceinline__ f32x2 lanes16(float v) {
   const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);

@@ -28,7 +28,8 @@ struct MidTile {
 // 3072 x 768 17.4 : 14.9, 700 x 4096 x 14336 in 2 95.2 : 86; 96 rows: 380 x 6144 x 4096 38.3 : 35.0, 700 x 4096 x 4096 34.3 : 33.0.
 // (192 x 64, 128 x 192 and 192 x 192 are best nowhere by more than 2 %.)
 // 64 x 64: five K-tiles are what two workgroups a CU have room for.  us with four : five: 64 x 64 x 3072 11.1 : 10.6, 1071 x
-// 768 x 3072 13.5 : 12.8, 700 x 6144 x 4096 72.2 : 71.0; six and more (one workgroup a CU) gain nothing over five.
+// 768 x 3072 13.5 : 12.8, 700 x 6144 x 4096 72.2 : 71.0; six and more (one workgroup a CU) gain nothing over five.  Exactly half
+// a CU's LDS: a kernel that keeps more beside its K-tiles needs a tile of its own (gemm_mid_fp8.hip).
 typedef MidTile<64, 64, 2, 2, 5> Mid0;
 typedef MidTile<128, 64, 2, 2, 6> Mid1;
 typedef MidTile<128, 128, 2, 4, 4> Mid2;

@@ -6,9 +6,11 @@ namespace dnn {
 
 // Tile table: rows, columns, whether two workgroups share a CU, and the constants of a
 // tile's time in us: a (launch, first loads, epilogue), s (a K-tile of 64) and p (of s, where K is
-// split: no epilogue, and waves that only stage), fitted to 1174 shapes.  Over 590 others (66 to 9400 rows, 768 to
+// split: no epilogue, and waves that only stage), fitted to 1174 shapes (64 x 64
+// with four K-tiles in flight).  As the kernels run now, over 589 other shapes (66 to 9400 rows, 768 to
 // 28672 columns, K of 768 to 21504, weights cold), every tile with 1 to 8 splits, the estimate is off by 10 % (rms);
-// what it picks takes 1.3 % longer than the best measured on average, 0.4 % in the median (profiles/gemm_mid_estimate.md).
+// what it picks takes 1.1 % longer than the best measured on average, 0.2 % in the median, 14 % at worst (67 x 6144 x
+// 4096 20.5, 18.0 as 96 x 128 in 4; profiles/gemm_mid_estimate.md).
 struct MidCost {
   int bm, bn, pairs;
   float a, s, p;
@@ -101,7 +103,7 @@ MidPlan mid_plan(int M, int N, int K, long long ws_bytes, unsigned kind) {
 // and 32 columns a workgroup (16 up to 1024 columns), which share a CU and add up: the
 // time is that of the fullest CU, in steps.  `frag`: the weight has its fragment-order
 // copy; without it a step costs 1.6 times as much.  A folded norm rides along for 1 us; the
-// tiles need a launch that adds 3.3.  us, decode kernels : tiles: 132 rows x 768 x 768 5.3 : 5.8, 192 6.6 : 5.9; row-
+// tiles need a launch that adds 3.3 (also counted where partials of the row statistics spare it).  us, decode kernels : tiles: 132 rows x 768 x 768 5.3 : 5.8, 192 6.6 : 5.9; row-
 // major 70 4.8 : 5.3; 192 x 768 x 3072 row-major 19.4 : 12.1; 70 x 1600 x 1600 7.1 : 7.1, 85
 // 9.0 : 8.5; 256 x 4096 x 4096 88 : 18; with a norm 128 x 3072 x 768 9.0 : 9.7, 146 10.4 : 9.8,
 // 135 x 2304 x 768 8.6 : 9.2, 167 9.6 : 9.1, 128 x 2816 x 512 6.4 : 7.4, 189 8.1 : 7.6, 256 x 1536 x
