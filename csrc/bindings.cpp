@@ -256,6 +256,10 @@ PYBIND11_MODULE(_dnn_hip, m) {
   }, py::arg("q"), py::arg("kc"), py::arg("vc"), py::arg("o"), py::arg("B"), py::arg("T"), py::arg("H"),
      py::arg("Hkv"), py::arg("hd"), py::arg("S"), py::arg("pos"), py::arg("scale"), py::arg("st"), py::arg("kv8") = 0,
      py::arg("one_group") = 0);
+  m.def("flash_attn_mx", [](u64 q, u64 kc, u64 vc, u64 q8, int ld8, u64 sx, int B, int T, int H, int Hkv, int hd, int S,
+                            u64 pos, float scale, u64 st) {
+    return dnn_flash_attn_mx(CP(q), CP(kc), CP(vc), P(q8), ld8, P(sx), B, T, H, Hkv, hd, S, CIP(pos), scale, ST(st));
+  });
   m.def("attn_decode", [](u64 q, u64 kc, u64 vc, u64 o, int B, int H, int Hkv, int hd, int S, u64 lens,
                           float scale, int splits, u64 ws, u64 st, int kv8) {
     return dnn_attn_decode(CP(q), CP(kc), CP(vc), P(o), B, H, Hkv, hd, S, CIP(lens), scale, splits, FP(ws), ST(st),

@@ -131,6 +131,8 @@ int dnn_qkv_split(const void* qkv, void* q, void* kc, void* vc, int B, int T, in
 int dnn_flash_attn_qkv(const void* qkv, int ldqkv, void* kc, void* vc, void* o, int B, int T, int H, int Hkv,
                        int hd, int S, const int* pos, float scale, hipStream_t st, int kv8 = 0,
                        int one_group = 0);
+int dnn_flash_attn_mx(const void* q, const void* kc, const void* vc, void* q8, int ld8, void* sx, int B, int T, int H,
+                      int Hkv, int hd, int S, const int* pos, float scale, hipStream_t st);
 int dnn_flash_attn(const void* q, const void* kc, const void* vc, void* o, int B, int T, int H, int Hkv, int hd, int S,
                    const int* pos, float scale, hipStream_t st, int kv8 = 0, int one_group = 0);
 int dnn_attn_decode_qkv(const void* qkv, int ldqkv, void* kc, void* vc, void* o, int B, int H, int Hkv, int hd, int S,

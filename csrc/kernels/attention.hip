@@ -157,37 +157,51 @@ __device__ __forceinline__ int k_swz(int key, int chunk) {
 // queries into buffers of their own and merge at the end.  A workgroup's blocks are
 // a chain (fetch, barrier, S, softmax, P.V: 1 us at hd 64) that nothing hides where
 // the grid leaves a workgroup a CU: FA_KS_WGS below.
-template <int HD, bool QKV = false, bool KV8 = false, bool DB = false, bool PIPE = false, int KS = 1>
+//
+// MXO (hd 64): a workgroup is 64 queries of two neighbouring heads, two waves each, the 128 columns that
+// share a scale of the projection behind (mx_index), and the rows leave as its e4m3 operand.  The quantiser's
+// launch and its pass over the rows (4 us and more) go, for keys and values staged for half as many queries:
+// us of both launches / of this, 25 heads, 8 x 256 14.8 / 10.4, 1 x 300 11.2 / 9.3, 1 x 960 23.3 / 23.4,
+// 8 x 960 54.9 / 50.6, 16 x 64 9.9 / 5.3.  With 128 queries a head, eight waves (8 x 256 13.3 in its pass, 12.3 so),
+// the longest tiles share a CU two and two.
+template <int HD, bool QKV = false, bool KV8 = false, bool DB = false, bool PIPE = false, int KS = 1, bool MXO = false>
 __global__ __launch_bounds__(256 * KS, 2) void flash_attn_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                                                             const bf16_t* __restrict__ vc, bf16_t* __restrict__ o, int T,
                                                             int H, int Hkv, int S, const int* __restrict__ pos,
                                                             float scale_log2, int ldq = 0,
                                                             bf16_t* __restrict__ kc_out = nullptr,
-                                                            bf16_t* __restrict__ vc_out = nullptr) {
+                                                            bf16_t* __restrict__ vc_out = nullptr,
+                                                            uint8_t* __restrict__ q8 = nullptr, int ld8 = 0,
+                                                            uint8_t* __restrict__ sx8 = nullptr) {
   using SM = FaSmem<HD>;
+  constexpr int NG = MXO ? 2 : KS;                  // groups of waves,
+  constexpr int TG = MXO ? 128 : 256, QB = TG / 2;  // their threads, a workgroup's queries
   // DB: two K/V buffers, one barrier per block (the block after next is staged
   // into the other buffer while this one is read)
-  __shared__ __attribute__((aligned(16))) char smem[SM::TOTAL * (PIPE ? 3 : DB ? 2 : 1) * KS];
-  static_assert(KS == 1 || (DB && !PIPE), "key groups have two buffers each");
-  const int kg = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);  // key group
+  __shared__ __attribute__((aligned(16))) char smem[SM::TOTAL * (PIPE ? 3 : DB ? 2 : 1) * NG];
+  static_assert(NG == 1 || (DB && !PIPE), "groups have two buffers each");
+  static_assert(!MXO || (HD == 64 && KS == 1 && !QKV), "two heads of 64 columns");
+  const int kg = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / TG);  // key group; MXO: head of the pair
   char* const buf0 = smem + kg * 2 * SM::TOTAL;
   char* ks = buf0;
   char* vs = buf0 + SM::K_BYTES;
   constexpr int NKS = HD / 16;  // k-steps of the QK^T contraction
   constexpr int NDT = HD / 32;  // 32-wide d tiles of O
   constexpr int CH = HD / 8;    // 16-B chunks per row
-  const int tid = KS == 1 ? threadIdx.x : threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+  const int tid = NG == 1 ? threadIdx.x : threadIdx.x & (TG - 1), lane = tid & 63, wave = tid >> 6;
   const int h = lane >> 5, r32 = lane & 31;
-  const int qb = (int)(gridDim.z - 1 - blockIdx.z), hh = blockIdx.x, b = blockIdx.y;
+  // MXO, odd number of heads: the last pair's second group repeats the first's and stores zeros
+  const int qb = (int)(gridDim.z - 1 - blockIdx.z), hh = MXO ? min(2 * (int)blockIdx.x + kg, H - 1) : (int)blockIdx.x;
+  const int b = blockIdx.y;
   const int kvh = hh / (H / Hkv);
   const int p0 = pos != nullptr ? pos[b] : 0;
   const int kv_len = min(p0 + T, S);  // rows of the cache: none past its end is fetched or counted
-  const int qrow0 = qb * FA_QB + wave * 32;            // this wave's first query (chunk-relative)
+  const int qrow0 = qb * QB + wave * 32;               // this wave's first query (chunk-relative)
   const int qrow = qrow0 + r32;                        // this lane's query
   const int key_max = min(p0 + min(qrow, T - 1), kv_len - 1);  // last key this lane's query attends
   const int wave_qmax = p0 + min(qrow0 + 31, T - 1);   // wave-uniform
   const int wave_qmin = p0 + min(qrow0, T - 1);
-  const int blk_qmax = p0 + min(qb * FA_QB + FA_QB - 1, T - 1);
+  const int blk_qmax = p0 + min(qb * QB + QB - 1, T - 1);
   const int kv_end = min(kv_len, blk_qmax + 1);
 
   const bf16_t* krow_new = nullptr;  // QKV: this sequence's new-key rows (position p0 + t = row b*T + t)
@@ -198,8 +212,8 @@ __global__ __launch_bounds__(256 * KS, 2) void flash_attn_kernel(const bf16_t* _
     if (hh % (H / Hkv) == 0) {  // cache write of rows t in [qb*128, qb*128+128), once per kv head
       bf16_t* kd = kc_out + ((size_t)b * Hkv + kvh) * S * HD;
       bf16_t* vd = vc_out + ((size_t)b * Hkv + kvh) * S * HD;
-      for (int e = threadIdx.x; e < FA_QB * CH; e += 256 * KS) {
-        const int t = qb * FA_QB + e / CH, c = e % CH;
+      for (int e = threadIdx.x; e < QB * CH; e += 256 * KS) {
+        const int t = qb * QB + e / CH, c = e % CH;
         if (t < T && p0 + t < S) {
           if constexpr (KV8) {
             uint8_t* kd8 = reinterpret_cast<uint8_t*>(kc_out) + ((size_t)b * Hkv + kvh) * S * HD;
@@ -241,12 +255,12 @@ __global__ __launch_bounds__(256 * KS, 2) void flash_attn_kernel(const bf16_t* _
   // prefill, 0.1058 -> 0.1051 ms, and slower at hd 128, 1.121 -> 1.218 ms at
   // T = 4096: profiles/r3_flash_prefetch_depth.jsonl.  The PMC there: MFMA
   // pipe 11 % busy, VALU ~30 %, waves waiting the rest.)
-  constexpr int NIT = (FA_KB * CH) / 256;
+  constexpr int NIT = (FA_KB * CH) / TG;
   i32x4 pkA[NIT], pvA[NIT];  // ext vectors: uint4 structs do not promote out of scratch
   auto fetch = [&](int kb0, i32x4(&pk)[NIT], i32x4(&pv)[NIT]) __attribute__((always_inline)) {
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
-      const int e = it * 256 + tid;
+      const int e = it * TG + tid;
       const int key = e / CH, c = e % CH;
       const int kk = min(kb0 + key, kv_len - 1);
       if (QKV && kk >= p0) {
@@ -267,7 +281,7 @@ __global__ __launch_bounds__(256 * KS, 2) void flash_attn_kernel(const bf16_t* _
     // ---- stage K (swizzled) and V (padded rows) from the prefetch registers ----
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
-      const int e = it * 256 + tid;
+      const int e = it * TG + tid;
       const int key = e / CH, c = e % CH;
       *reinterpret_cast<i32x4*>(ks + key * HD * 2 + (k_swz<HD>(key, c) << 4)) = pk[it];
       *reinterpret_cast<i32x4*>(vs + key * SM::V_STRIDE + c * 16) = pv[it];
@@ -425,7 +439,7 @@ __global__ __launch_bounds__(256 * KS, 2) void flash_attn_kernel(const bf16_t* _
       __syncthreads();
     }
   } else {
-    const int first = kg * FA_KB;
+    const int first = KS == 1 ? 0 : kg * FA_KB;
     constexpr int STEP = KS * FA_KB;
     if (first < kv_end) {
       fetch(first, pkA, pvA);
@@ -470,6 +484,45 @@ __global__ __launch_bounds__(256 * KS, 2) void flash_attn_kernel(const bf16_t* _
     for (int i = 0; i < NDT; ++i)
 #pragma unroll
       for (int g = 0; g < 16; ++g) oacc[i][g] = oacc[i][g] * f0 + mb[(2 + i * 16 + g) * 64] * f1;
+  }
+  if constexpr (MXO) {
+    // the bf16 values that the plain kernel stores, quantised as quant_fp8_mx_kernel does it
+    const float inv = l_i > 0.f ? 1.f / l_i : 0.f;
+    const bool there = 2 * (int)blockIdx.x + kg < H;
+    float am = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int g = 0; g < 16; ++g) {
+        oacc[dt][g] = there ? bf2f(f2bf(oacc[dt][g] * inv)) : 0.f;
+        am = fmaxf(am, fabsf(oacc[dt][g]));
+      }
+    am = max32(am);
+    float* red = reinterpret_cast<float*>(smem);  // [group][QB queries]
+    __syncthreads();                              // both groups are done with the key and value buffers
+    if (lane < 32) red[kg * QB + wave * 32 + lane] = am;
+    __syncthreads();
+    am = fmaxf(am, red[(kg ^ 1) * QB + wave * 32 + r32]);
+    float qi;
+    const uint32_t e = e8m0_of(am, qi);
+    const int m = b * T + qrow;
+    uint8_t* const dst = q8 + (size_t)m * ld8 + (2 * (int)blockIdx.x + kg) * HD;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {  // columns dt * 32 + 16 p + 0..15: lane h of a pair stores the 8 from 8 h on
+        int w[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int g = 4 * (2 * p + i);
+          w[i] = __builtin_amdgcn_cvt_pk_fp8_f32(oacc[dt][g] * qi, oacc[dt][g + 1] * qi, 0, false);
+          w[i] = __builtin_amdgcn_cvt_pk_fp8_f32(oacc[dt][g + 2] * qi, oacc[dt][g + 3] * qi, w[i], true);
+        }
+        const auto s = __builtin_amdgcn_permlane32_swap((uint32_t)w[0], (uint32_t)w[1], false, false);
+        if (qrow < T) *reinterpret_cast<uint2*>(dst + dt * 32 + 8 * (2 * p + h)) = make_uint2(s[0], s[1]);
+      }
+    if (kg == 0 && h == 0 && qrow < T) sx8[mx_index(m, blockIdx.x, mx_mpad(gridDim.y * T))] = (uint8_t)e;
+    return;
   }
   // ---- normalise + store: lane = query, regs = d ----
   if (qrow < T) {
@@ -1016,6 +1069,19 @@ extern "C" int dnn_flash_attn(const void* q, const void* kc, const void* vc, voi
   } else {
     return -2;
   }
+  return (int)hipGetLastError();
+}
+
+// The same with rows that leave as MX e4m3 (dnn_quant_fp8_mx of them, bit by bit): q8 rows of ld8 bytes, whole 128-column
+// blocks of H * hd written.  -3, nothing launched: not this shape, or a pinned variant.
+extern "C" int dnn_flash_attn_mx(const void* q, const void* kc, const void* vc, void* q8, int ld8, void* sx, int B, int T,
+                                 int H, int Hkv, int hd, int S, const int* pos, float scale, hipStream_t st) {
+  if (H % Hkv != 0 || ld8 % 8 != 0 || ld8 < (H + 1) / 2 * 128) return -1;
+  if (hd != 64 || getenv("DNN_FLASH_DB") != nullptr || getenv("DNN_FLASH_PIPE") != nullptr) return -3;
+  hipLaunchKernelGGL((flash_attn_kernel<64, false, false, true, false, 1, true>),
+                     dim3((H + 1) / 2, B, (T + 63) / 64), dim3(256), 0, st, (const bf16_t*)q, (const bf16_t*)kc,
+                     (const bf16_t*)vc, (bf16_t*)nullptr, T, H, Hkv, S, pos, scale * 1.4426950408889634f, 0,
+                     (bf16_t*)nullptr, (bf16_t*)nullptr, (uint8_t*)q8, ld8, (uint8_t*)sx);
   return (int)hipGetLastError();
 }
 

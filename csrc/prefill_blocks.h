@@ -93,9 +93,9 @@ struct PrefillPass {
                                (float*)a, have ? parts : nullptr, p.colsum, nullptr, &wrote, ws, ws_bytes);
   }
 
-  // h = in W^T + bias + res, in (rows, K); quantised: in lies in q8b / sxb already; read: the next projection
-  // takes h's partials (`have`: they were written)
-  int res_proj(const void* in, const PrefillProj& p, const void* res, int K, bool quantised, bool read) {
+  // h = in W^T + bias + res, in (rows, K); qin, sin: in as MX e4m3, where its producer left it so; read: the
+  // next projection takes h's partials (`have`: they were written)
+  int res_proj(const void* in, const PrefillProj& p, const void* res, int K, const void* qin, const void* sin, bool read) {
     const int M = rows();
     have = false;
     if (!fp8) {
@@ -111,12 +111,13 @@ struct PrefillPass {
       return dnn_gemm_skinny_w8(in, K, p.w, kpad(K), p.scale, h, d, p.bias, res, d, M, d, K, 0, 0, nullptr, 0.f, st,
                                 p.frag, ws, ws_bytes);
     }
-    if (!quantised) {
+    if (qin == nullptr) {
+      qin = q8, sin = sx;
       what = "quant_fp8_mx";
       if (const int rc = dnn_quant_fp8_mx(in, K, q8, kpad(K), sx, M, K, kpad(K), st)) return rc;
     }
     what = "gemm_fp8_mx";
-    return dnn_gemm_fp8_mx(quantised ? q8b : q8, quantised ? sxb : sx, p.w, p.scale, h, d, p.bias, res, d, M, d,
+    return dnn_gemm_fp8_mx(qin, sin, p.w, p.scale, h, d, p.bias, res, d, M, d,
                            kpad(K), 0, nullptr, 0, nullptr, 0, st);
   }
 
@@ -156,6 +157,8 @@ struct PrefillPass {
     const void* in = x;
     const int nq = (H + 2 * Hkv) * hd;
     const int one_group = fp8 && rows() > skinny_max;  // e4m3 activations follow (attention.hip flash_two_groups)
+    // the attention quantises its rows itself where the projection behind it takes MX rows
+    const bool att_quant = one_group && hd == 64 && !skinny(d, H * hd, false, true, ws_bytes);
     const bool up_quant = fp8 && act == 2 && !skinny(n_up, d, true, true, 0);
     const bool part = parts != nullptr && !fp8;
     for (size_t i = 0; i < blocks.size(); ++i) {
@@ -167,10 +170,18 @@ struct PrefillPass {
                             !skinny(nq, d, true, L.qkv.frag != nullptr, 0) && dnn_gemm_takes_parts(rows(), nq, d, d, d, 0, 1, 0);
       void *k = kc + i * kv_block, *v = vc + i * kv_block;
       int rc;
+      bool mx_att = false;
       if (scattered(in, L.qkv, k, v, rc)) {
         if (rc) return rc;
-        what = "flash_attn";
-        rc = dnn_flash_attn(q, k, v, att, B, T, H, Hkv, hd, S, pos, scale, st, 0, one_group);
+        if (att_quant) {
+          what = "flash_attn_mx";
+          rc = dnn_flash_attn_mx(q, k, v, q8, kpad(H * hd), sx, B, T, H, Hkv, hd, S, pos, scale, st);
+          mx_att = rc != -3;
+        }
+        if (!mx_att) {
+          what = "flash_attn";
+          rc = dnn_flash_attn(q, k, v, att, B, T, H, Hkv, hd, S, pos, scale, st, 0, one_group);
+        }
       } else {
         if (rc) return rc;
         if ((rc = norm_proj(in, L.qkv, qkv, nq, nq, 0, true, false))) return rc;
@@ -185,9 +196,9 @@ struct PrefillPass {
         }
       }
       if (rc) return rc;
-      if ((rc = res_proj(att, L.o, in, H * hd, false, read_up))) return rc;
+      if ((rc = res_proj(att, L.o, in, H * hd, mx_att ? q8 : nullptr, mx_att ? sx : nullptr, read_up))) return rc;
       if ((rc = norm_proj(h, L.up, f, ffn, n_up, act, false, up_quant))) return rc;
-      if ((rc = res_proj(f, L.down, h, ffn, up_quant, read_qkv))) return rc;
+      if ((rc = res_proj(f, L.down, h, ffn, up_quant ? q8b : nullptr, up_quant ? sxb : nullptr, read_qkv))) return rc;
       in = h;
     }
     return 0;
