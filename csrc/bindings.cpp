@@ -10,6 +10,7 @@
 #include <cstdint>
 
 #include "kernels/api.h"
+#include "kernels/attention_row.h"
 #include "comm/p2p.h"
 
 #include <string>
@@ -178,6 +179,23 @@ PYBIND11_MODULE(_dnn_hip, m) {
     return dnn_cifar_head_tail(CP(hid), CP(w2p), CFP(b2), FP(probs), IP(pred), B, ST(st));
   });
 #ifdef DNN_HAVE_TRANSFORMER
+  m.def("decode_row_parts", [](int M, int d, int H, int Hkv, int hd, int S) {
+    return dnn_decode_row_parts(M, d, H, Hkv, hd, S);
+  });
+  // blocks: the 10 pointers of RowBlock each; -3: not a step of this kind, nothing launched
+  m.def("decode_row_blocks", [](const std::vector<int>& n, const std::vector<u64>& b, float eps, float scale,
+                                long long kv_block, u64 st, const std::vector<u64>& blocks) {
+    if (n.size() != 6 || b.size() != 9 || blocks.empty() || blocks.size() % 10 != 0)
+      throw std::runtime_error("decode_row_blocks: ragged arguments");
+    std::vector<RowBlock> L(blocks.size() / 10);
+    for (size_t i = 0; i < L.size(); ++i) {
+      const u64* p = &blocks[i * 10];
+      L[i] = {CP(p[0]), CP(p[1]), CP(p[2]), CP(p[3]), CFP(p[4]), CFP(p[5]), CFP(p[6]), CFP(p[7]), CFP(p[8]), CFP(p[9])};
+    }
+    return dnn_decode_row_blocks(L.data(), (int)L.size(), CP(b[0]), P(b[1]), P(b[2]), P(b[3]), P(b[4]), FP(b[5]),
+                                 static_cast<char*>(P(b[6])), static_cast<char*>(P(b[7])), kv_block, n[0], n[1], n[2], n[3],
+                                 n[4], n[5], CIP(b[8]), scale, eps, ST(st));
+  });
   // blocks: 20 pointers each (qkv, o, up, down x weight, scale, bias, row sums, fragment copy); returns
   // (code, launch that failed, whether the partials of the last rows were written); -100: not a pass of this kind, nothing launched
   m.def("prefill_blocks", [](const std::vector<int>& n, const std::vector<u64>& b, float eps, float scale,

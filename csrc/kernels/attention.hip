@@ -16,6 +16,7 @@
 // as the B operand (no LDS round trip for P) and V^T fragments fetched with
 // ds_read_b64_tr_b16 (hardware transpose) from a row-padded V tile. K rows are
 // XOR-swizzled so the A-fragment ds_read_b128 reads are conflict-free.
+#include "attention_row.h"
 #include "common.h"
 
 #include <algorithm>
@@ -1181,6 +1182,15 @@ static int attn_stream_launch(const StreamArgs& a, int B, int hd, int splits, in
   STR(64, 1) STR(64, 2) STR(64, 4) STR(64, 8) STR(128, 1) STR(128, 2) STR(128, 4) STR(128, 8) { return -2; }
 #undef STR
   if (ns > 1) launch_decode_combine(a.ws, a.o, B, a.H, a.Hkv, hd, (int)ns, st);
+  return (int)hipGetLastError();
+}
+
+extern "C" int dnn_attn_decode_proj(const void* qkv, int ldq, void* kc, void* vc, const void* wo, float* part, int B, int H,
+                                    int S, const int* pos, float scale, hipStream_t st) {
+  if (B < 1 || H < 1 || S < 1 || ldq < 3 * H * 64 || ldq % 8 != 0) return -1;
+  hipLaunchKernelGGL((attn_decode_stream_kernel<64, 1, 1, false, 8, 4, true>), dim3(B * H, (H * 4 + 7) / 8), dim3(512), 0, st,
+                     (const bf16_t*)qkv, ldq, (bf16_t*)kc, (bf16_t*)vc, (float*)nullptr, H, H, S, pos, (const float*)nullptr,
+                     (const float*)nullptr, scale * 1.4426950408889634f, (bf16_t*)nullptr, (const uint8_t*)wo, part);
   return (int)hipGetLastError();
 }
 

@@ -50,11 +50,16 @@ __device__ __forceinline__ int sum_row_groups(float (&v)[N], int lane) {
   return ((lane >> 4) & 1) * (N / 2) + (lane >> 5) * (N / 4);
 }
 
-template <int HD, int G, int FM, bool NT, int NW, int U>
+// PROJ (heads of 64, one workgroup a head and NW column tiles, blockIdx.y): the head's output, rounded to bf16 as it
+// would be stored, times its 64 columns of W_o (wo, fragment order): part[head][row][N], N = 64 H.  The weights are
+// asked for with the first keys.  Every column group forms the head's output for itself.
+template <int HD, int G, int FM, bool NT, int NW, int U, bool PROJ = false>
 __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
     const bf16_t* __restrict__ q, int ldq, bf16_t* __restrict__ kc, bf16_t* __restrict__ vc, float* __restrict__ ws,
     int H, int Hkv, int S, const int* __restrict__ lens, const float* __restrict__ cosT,
-    const float* __restrict__ sinT, float scale_log2, bf16_t* __restrict__ o_direct) {
+    const float* __restrict__ sinT, float scale_log2, bf16_t* __restrict__ o_direct,
+    const uint8_t* __restrict__ wo = nullptr, float* __restrict__ part = nullptr) {
+  static_assert(!PROJ || (HD == 64 && G == 1), "two chunks of W_o a head");
   constexpr bool FUSED = FM != 0, ROPE = FM == 2;
   constexpr int LPK = HD / 8, RG = 64 / LPK, R = U * RG;
   static_assert(LPK == 8 || LPK == 16, "sums over row groups");
@@ -63,12 +68,12 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
   static_assert(U % 2 == 0, "P.V folds row pairs");
   static_assert(!MF || (R % 16 == 0 && G <= 16), "MF: blocks of whole tiles");
   // MF: probabilities of a wave [row group][row pair][head][2]; q, the new key, the new value
-  __shared__ __attribute__((aligned(16))) uint16_t pl[MF ? NW : 1][MF ? RG * U * G : 8];
+  __shared__ __attribute__((aligned(16))) uint16_t pl[MF ? NW : 1][MF ? RG * U * G : PROJ ? HD : 8];
   __shared__ __attribute__((aligned(16))) uint16_t qkv[MF ? G + 2 : 1][HD];
   __shared__ __attribute__((aligned(16))) float red[NW * G * HD];
   __shared__ float mred[NW * G], lred[NW * G];
 
-  const int bk = blockIdx.x, split = blockIdx.y, NS = gridDim.y;
+  const int bk = blockIdx.x, split = PROJ ? 0 : blockIdx.y, NS = PROJ ? 1 : gridDim.y;
   const int b = bk / Hkv, kvh = bk % Hkv;
   const int p_new = FUSED ? lens[b] : 0;
   const int len = FUSED ? min(p_new + 1, S) : min(lens[b], S);
@@ -78,8 +83,12 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int sub = lane % LPK, grp = lane / LPK;
   float* wsp = ws + ((size_t)bk * NS + split) * G * (HD + 2);
+  const int ct = blockIdx.y * NW + wave;  // PROJ: the wave's column tile, and where its 4 columns' sums go
+  float* const pdst = part + ((size_t)kvh * (gridDim.x / Hkv) + b) * (Hkv * HD) + ct * 16 + (lane >> 4) * 4;
   if (k0 >= k1) {  // nothing in this split (short context), or no key at all
-    if (NS == 1) {
+    if (PROJ) {
+      if (ct < Hkv * HD / 16 && (lane & 15) == 0) *reinterpret_cast<f32x4*>(pdst) = f32x4{0.f, 0.f, 0.f, 0.f};
+    } else if (NS == 1) {
       for (int i = tid; i < G * HD; i += NW * 64) o_direct[(size_t)b * H * HD + kvh * G * HD + i] = 0;
     } else {
       for (int i = tid; i < G * (HD + 2); i += NW * 64) wsp[i] = (i % (HD + 2)) == HD ? -INFINITY : 0.f;
@@ -171,6 +180,13 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
       load_head8<HD, false>(q + (size_t)b * ldq + (H + Hkv + kvh) * HD, sub, nullptr, nullptr, 0, t8);
       pack(nvp);
     }
+  }
+  i32x4 wo_r[2];
+  if constexpr (PROJ) {
+    const i32x4* wp = reinterpret_cast<const i32x4*>(wo) + ((size_t)min(ct, Hkv * HD / 16 - 1) * (Hkv * 2) + kvh * 2) * 64 + lane;
+    wo_r[0] = wp[0];
+    wo_r[1] = wp[64];
+    __builtin_amdgcn_sched_barrier(0);
   }
 
   // softmax state: G = 1, of the lane's row group; MF, of head hj over the wave (l: over the lane's keys).
@@ -356,7 +372,9 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
       s += red[(w * G + g) * HD + d] * f;
       ls += lred[w * G + g] * f;
     }
-    if (NS == 1) {
+    if constexpr (PROJ) {
+      pl[0][d] = f2bf(ls > 0.f ? s / ls : 0.f);
+    } else if (NS == 1) {
       o_direct[(size_t)b * H * HD + (kvh * G + g) * HD + d] = f2bf(ls > 0.f ? s / ls : 0.f);
     } else {
       wsp[g * (HD + 2) + d] = s;
@@ -366,8 +384,17 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_stream_kernel(
       }
     }
   }
+  if constexpr (PROJ) {
+    __syncthreads();
+    f32x4 y = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+      y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wo_r[c]),
+                                                  *reinterpret_cast<const bf16x8*>(&pl[0][c * 32 + (lane >> 4) * 8]), y, 0, 0, 0);
+    if (ct < Hkv * HD / 16 && (lane & 15) == 0) *reinterpret_cast<f32x4*>(pdst) = y;
+  }
   // the new row into the cache, behind every load of the workgroup
-  if (own_new && tid < LPK) {
+  if (own_new && tid < LPK && (!PROJ || blockIdx.y == 0)) {
     const size_t at = (((size_t)b * Hkv + kvh) * S + p_new) * HD + sub * 8;
     uint4 wk, wv;
     if constexpr (MF) {

@@ -352,6 +352,11 @@ class TransformerStage(StageCompute):
         self.rowstat = G_.rowstats_buffer(self.max_batch, d, dev)  # decode rows only
         self.rowparts = None if self.fp8 or not self.fuse_norm else G_.parts_buffer(ntok, d, dev)  # prefill rows
         self.pws = None if self.fp8 else G_.prefill_workspace(ntok, max((H + 2 * Hkv) * hd, d, ffn), dev)
+        # partials of a one- or two-row decode step (_decode_rows): a region per cache row, as the other scratch
+        self.rowpart = None
+        if not self.fp8 and self.fuse_norm and self.family == "gpt2" and self.device.type == "cuda":
+            per = _lib.lib().decode_row_parts(1, d, H, Hkv, hd, self.max_seq)
+            self.rowpart = torch.empty((self.max_batch, per), dtype=torch.float32, device=dev) if per else None
         self.q8 = self.s8 = None
         self.sx8 = self.q8b = self.sx8b = None
         if self.fp8:
@@ -467,6 +472,9 @@ class TransformerStage(StageCompute):
             if (G_.QKV_SCATTER and self.cos is None and not G_._norm_skinny(h, L.w_qkv, ACT_NONE, True)
                     and G_.takes_parts(ntok, nq, d, scatter=True)):
                 rp_qkv = self.rowparts
+        if T == 1 and self._decode_rows(h_in, pos, B, b0):
+            one_call, L = True, self.layers[-1]
+            self._lin(self.buf_f[r0:r1], L.w_down, L.b_down, residual=h, out=h, w_shuf=L.w_down_s, ws=gws)
         for li, L in enumerate(() if one_call else self.layers):
             kc, vc = self.kc[li, b0:b0 + B], self.vc[li, b0:b0 + B]
             att = self.buf_att[r0:r1]
@@ -587,6 +595,32 @@ class TransformerStage(StageCompute):
             _lib.check(rc, what)
             bufs[11] = bufs[0]  # the next block reads what this one wrote
             bufs[13], bufs[14] = bufs[13] + block, bufs[14] + block
+        return True
+
+    def _decode_rows(self, x: torch.Tensor, pos: torch.Tensor, B: int, b0: int) -> bool:
+        """A decode step of a row or two up to the last block's c_fc, by partial products
+        (csrc/kernels/decode_row.hip): four launches a block in one native call, from the
+        layers' weights as they are now.  False, with nothing launched, where the loop has
+        to issue them: other widths, more rows, e4m3 caches, no fragment-order copies."""
+        if (self.rowpart is None or B > 2 or not self.layers or self.kc.dtype != torch.bfloat16 or _lib.DEBUG_SYNC
+                or pos.dtype != torch.int32 or not pos.is_contiguous() or pos.numel() < B or x.dtype != torch.bfloat16
+                or not x.is_contiguous() or x.data_ptr() % 16):
+            return False
+        w = []
+        for L in self.layers:
+            q, u = L.w_qkv, L.w_up
+            w += [0 if t is None else t.data_ptr() for t in (q.ws, L.w_o_s, u.ws, L.w_down_s, q.colsum, q.bias, L.b_o,
+                                                             u.colsum, u.bias, L.b_down)]
+        if 0 in w:
+            return False
+        r = slice(b0, b0 + B)
+        bufs = [t.data_ptr() for t in (x, self.buf_a[r], self.buf_h[r], self.buf_qkv[r], self.buf_f[r], self.rowpart[r],
+                                       self.kc[0, b0], self.vc[0, b0], pos)]
+        rc = _lib.lib().decode_row_blocks([B, self.d, self.H, self.Hkv, self.hd, self.kc.shape[3]], bufs, self.eps,
+                                          1.0 / math.sqrt(self.hd), self.kc.stride(0) * 2, _lib.stream_ptr(), w)
+        if rc == -3:
+            return False
+        _lib.check(rc, "decode_row_blocks")
         return True
 
     def _block_ptrs(self, L: LayerW) -> List[int]:
