@@ -1,0 +1,269 @@
+// Decode projections of up to 64 rows whose slices of K lie in registers ("lean"):
+//   C[M,N] = epi(A[M,K] . W[N,K]^T), W in fragment order, bf16 or e4m3 (W8A16).
+//
+// At these sizes a launch in a decode step costs its start, one round trip for what it
+// reads and the code itself: every launch begins with a cold instruction cache, and 4 to 5
+// KB of a kernel that is laid out for every shape are 1 to 2 us of fetches (GPT-2's
+// 2304 x 768 of 64 rows: 5.0 us launched over and over by itself, 7.4 in its step).  So
+// the shape is compile-time down to the chunk: NW waves of NB batches of CB chunks are K, D
+// batches of a wave in flight straight to registers (a wave's slices of A and W are its own,
+// nothing is shared before the sums meet), one barrier, and the waves that finish a tile
+// have its epilogue's operands by then: 1.2 to 5.8 KB, of which the e4m3 c_fc's was 28.
+//
+// us a launch in the step, GPT-2 (bf16) of 64 rows 2304 x 768 7.4 -> 4.6, 3072 x 768 7.0 -> 5.1, 768 x 768 5.4
+// -> 4.8, 768 x 3072 7.1 -> 6.1; XL (e4m3) of 64 rows 4800 x 1600 10.7 -> 7.1, 6400 x 1600 11.2 -> 7.6,
+// 1600 x 1600 5.8 -> 5.0, 1600 x 6400 11.6 -> 10.5.  Batches in flight, waves and their chunks matter
+// little (within 1 % of the step from one batch to all of K, 4 to 8 waves); tiles do: lean_gemm.
+#include <utility>
+
+#include "gemm_lean.h"
+
+namespace dnn {
+
+template <int NW, int CB, int NB, int D, int MT, int NT, bool W8, int NORM, int ACT, bool RES>
+struct Lean {
+  static constexpr int K = NW * CB * NB * (W8 ? 64 : 32), ROWS = 16 * MT;
+  static constexpr int LPR = NW * 64 / ROWS;  // threads a row for the merge of its statistics
+  static constexpr int TPR = LPR >= 64 ? 64 : LPR >= 32 ? 32 : LPR >= 16 ? 16 : LPR >= 8 ? 8 : 4;
+  static constexpr int SPT = (K / 16 + TPR - 1) / TPR;
+};
+
+template <int NW, int CB, int NB, int D, int MT, int NT, bool W8, int NORM, int ACT, bool RES>
+__global__ __launch_bounds__(NW * 64) void gemm_lean_kernel(LeanArgs p) {
+  using L = Lean<NW, CB, NB, D, MT, NT, W8, NORM, ACT, RES>;
+  constexpr int AU = W8 ? 2 : 1, ACH = 64 * AU, TS = MT * NT, CH = CB * NB, TW = (TS + NW - 1) / NW;
+  static_assert(D <= NB, "batches in flight");
+  __shared__ f32x4 red[NW][TS][64];
+  __shared__ float2 st[NORM == NORM_LN ? L::ROWS : 1];
+  __shared__ float ss[NORM == NORM_RMS ? NW : 1][NORM == NORM_RMS ? L::ROWS : 1];
+  const int n0 = blockIdx.x * (16 * NT), m0 = blockIdx.y * (16 * MT);
+  if (n0 >= p.N) return;  // the grid is a multiple of 8 columns: the row tiles of a column tile on one XCD
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, c4 = lane >> 4;
+  float2 rp[L::SPT], rp0;
+  const int srow = tid / L::TPR, sub = tid % L::TPR;
+  if constexpr (NORM == NORM_LN) {
+    const float2* q = p.rs_in + (size_t)min(m0 + min(srow, L::ROWS - 1), p.M - 1) * p.rs_in_ld;
+    rp0 = q[0];
+#pragma unroll
+    for (int i = 0; i < L::SPT; ++i) rp[i] = q[min(sub + i * L::TPR, L::K / 16 - 1)];
+  }
+  i32x4 av[D][MT][CB * AU], wv[D][NT][CB];
+  const uint8_t* ap[MT];
+  const uint8_t* wp[NT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+    ap[t] = p.A + (size_t)min(m0 + t * 16 + r16, p.M - 1) * p.lda_b + wave * (CH * ACH) + c4 * (16 * AU);
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    wp[j] = p.W + ((size_t)min(n0 / 16 + j, p.N / 16 - 1) * (NW * CH) + wave * CH) * 1024 + lane * 16;
+  auto load = [&](auto bc) __attribute__((always_inline)) {
+    constexpr int b = decltype(bc)::value, d = b % D;
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int u = 0; u < CB; ++u)
+#pragma unroll
+        for (int h = 0; h < AU; ++h)
+          av[d][t][u * AU + h] = *reinterpret_cast<const i32x4*>(ap[t] + (b * CB + u) * ACH + h * 16);
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int u = 0; u < CB; ++u) wv[d][j][u] = *reinterpret_cast<const i32x4*>(wp[j] + (b * CB + u) * 1024);
+  };
+  [&]<int... B>(std::integer_sequence<int, B...>) __attribute__((always_inline)) {
+    (load(std::integral_constant<int, B>{}), ...);
+  }(std::make_integer_sequence<int, D>{});
+  // the tiles that this wave finishes, and their operands (absent ones from a dummy address)
+  f32x4 cs[TW], bs[TW], sc[TW];
+  bf16x4 rr[TW];
+  int n[TW], m[TW];
+#pragma unroll
+  for (int i = 0; i < TW; ++i) {
+    const int tile = min(wave + i * NW, TS - 1);
+    n[i] = min(n0 + tile / MT * 16, p.N - 16) + c4 * 4;
+    m[i] = m0 + tile % MT * 16 + r16;
+    bs[i] = *reinterpret_cast<const f32x4*>(p.bias != nullptr ? p.bias + n[i] : reinterpret_cast<const float*>(p.W));
+    if constexpr (NORM == NORM_LN) cs[i] = *reinterpret_cast<const f32x4*>(p.colsum + n[i]);
+    if constexpr (W8) sc[i] = *reinterpret_cast<const f32x4*>(p.sw + n[i]);
+    if constexpr (RES) rr[i] = *reinterpret_cast<const bf16x4*>(p.R + (size_t)min(m[i], p.M - 1) * p.ldr + n[i]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (NORM == NORM_LN) {
+    const float2 mr = rowstat_merge<NORM_LN, L::TPR, L::SPT>(rp, rp0, sub, L::K, p.eps);
+    if (sub == 0 && srow < L::ROWS) st[srow] = mr;
+  }
+  f32x4 acc[NT][MT];
+  float sq[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    sq[t] = 0.f;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  auto comp = [&](auto bc) __attribute__((always_inline)) {
+    constexpr int d = decltype(bc)::value % D;
+#pragma unroll
+    for (int u = 0; u < CB; ++u)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        bf16x8 w[AU];
+        if constexpr (W8) w8_to_bf16(wv[d][j][u], w[0], w[AU - 1]);
+        else w[0] = __builtin_bit_cast(bf16x8, wv[d][j][u]);
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+          for (int h = 0; h < AU; ++h)
+            acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[h], __builtin_bit_cast(bf16x8, av[d][t][u * AU + h]),
+                                                                acc[j][t], 0, 0, 0);
+      }
+    if constexpr (NORM == NORM_RMS) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int u = 0; u < CB * AU; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const bf16x2v v = __builtin_bit_cast(bf16x2v, (uint32_t)av[d][t][u][i]);
+            sq[t] = __builtin_amdgcn_fdot2_f32_bf16(v, v, sq[t], false);
+          }
+    }
+  };
+  [&]<int... B>(std::integer_sequence<int, B...>) __attribute__((always_inline)) {
+    (([&]() __attribute__((always_inline)) {
+       comp(std::integral_constant<int, B>{});
+       __builtin_amdgcn_sched_barrier(0);
+       if constexpr (B + D < NB) {
+         load(std::integral_constant<int, B + D>{});
+         __builtin_amdgcn_sched_barrier(0);
+       }
+     }()),
+     ...);
+  }(std::make_integer_sequence<int, NB>{});
+  if constexpr (NORM == NORM_RMS) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      const float s = add32(add16(sq[t]));
+      if (lane < 16) ss[wave][t * 16 + lane] = s;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) red[wave][j * MT + t][lane] = acc[j][t];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < TW; ++i) {
+    const int tile = wave + i * NW, nt = n0 + tile / MT * 16;
+    if (tile >= TS || nt >= p.N) return;
+    f32x4 v[NW];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) v[w] = red[w][tile][lane];
+    f32x4 y = v[0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) y += v[w];
+    if constexpr (W8) y *= sc[i];
+    if constexpr (NORM == NORM_LN) {
+      const float2 mr = st[m[i] - m0];
+      y = mr.y * (y - mr.x * cs[i]);
+    }
+    if constexpr (NORM == NORM_RMS) {
+      float q = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) q += ss[w][m[i] - m0];
+      y *= rsqrtf(q * (1.f / L::K) + p.eps);
+    }
+    if (p.bias != nullptr) y += bs[i];
+    if constexpr (ACT == ACT_GELU) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = gelu_erf(y[e]);
+    }
+    if constexpr (RES) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] += bf2f_s(rr[i][e]);
+    }
+    const uint2 o = make_uint2(pack2bf(y[0], y[1]), pack2bf(y[2], y[3]));
+    if (m[i] < p.M) *reinterpret_cast<uint2*>(p.C + (size_t)m[i] * p.ldc + n[i]) = o;
+    if (RES && p.rs_out != nullptr)
+      epi_rowstat16(f32x4{__uint_as_float(o.x << 16), __uint_as_float(o.x & 0xffff0000u), __uint_as_float(o.y << 16),
+                          __uint_as_float(o.y & 0xffff0000u)},
+                    m[i], nt, p.M, p.N, p.rs_out, p.rs_out_ld, lane);
+  }
+}
+
+template <int NW, int CB, int NB, int D, int MT, int NT, bool W8, int NORM, int ACT, bool RES>
+static void lean_launch(const LeanArgs& p, hipStream_t st) {
+  const int cols = (p.N / 16 + NT - 1) / NT;
+  hipLaunchKernelGGL((gemm_lean_kernel<NW, CB, NB, D, MT, NT, W8, NORM, ACT, RES>),
+                     dim3((cols + 7) / 8 * 8, (p.M + 16 * MT - 1) / (16 * MT)), dim3(NW * 64), 0, st, p);
+}
+
+// False, nothing done, where the shape is not one of those laid out.
+template <int ACT, int NORM, bool W8>
+static bool lean_gemm(const LeanArgs& p, int nch, hipStream_t st) {
+  constexpr bool RES = NORM == NORM_NONE;
+  if constexpr (!(NORM == NORM_LN && (ACT == ACT_NONE || ACT == ACT_GELU)) && !(RES && ACT == ACT_NONE) &&
+                !(NORM == NORM_RMS && ACT == ACT_NONE && !W8)) {
+    return false;
+  } else {
+    // The tiles, from whole steps (us; GPT-2 behind 100 tokens, XL behind 64, Llama-3 of 4 layers behind 100; before:
+    // gemm_skinny, gemm_oneshot):
+    //   GPT-2 QKV, c_fc        8 rows 302: 1 x 1 tiles 270, 1 x 2 272, 2 x 2 279; 32 rows 406: 358, 347, 364; 64 rows 422:
+    //                          409, 397, 389
+    //   its O, c_proj          1 x 1 at every number of rows (24 rows 389: 376, 372; 64 rows 422: 415, 403)
+    //   XL e4m3 QKV, c_fc      8 rows 183: 1 x 2 tiles 164, 1 x 4 166; 32 rows 286: 246, 230, 2 x 4 253; 64 rows 278: 300, 272, 267
+    //   its O, c_proj          32 rows 286: 1 x 1 275, 266, 1 x 2 279, 285; 64 rows 278: 289, 308; 275, 274
+    //   Llama-3 QKV, O         16 rows 410: 393, 400 (1 x 2, 1 x 1); from 17 rows the step is up to 3 % slower with tiles of
+    //                          32 rows: 16 rows of a load lie 8 KB apart, on one channel of the L2
+    // Two rows or fewer of GPT-2's widths: decode_row.hip.  Other widths have not been laid out or measured.
+    auto al = [](const void* x, int a) { return ((uintptr_t)x & (a - 1)) == 0; };
+    if (p.W == nullptr || p.M < 1 || p.M > 64 || p.N % 16 != 0 || p.N > (RES ? 4096 : 8192) || (p.R != nullptr) != RES ||
+        (!RES && p.rs_out != nullptr) || p.lda_b % 16 != 0 || p.ldc % 4 != 0 || !al(p.A, 16) || !al(p.C, 8) ||
+        !al(p.bias, 16) || !al(p.colsum, 16) || !al(p.sw, 16) || (RES && (p.ldr % 4 != 0 || !al(p.R, 8))) ||
+        (NORM == NORM_LN && (p.rs_in == nullptr || p.colsum == nullptr)))
+      return false;
+#define LEAN(NWV, CBV, NBV, DV, MTV, NTV) lean_launch<NWV, CBV, NBV, DV, MTV, NTV, W8, NORM, ACT, RES>(p, st)
+    const int M = p.M;
+    if constexpr (!W8 && NORM == NORM_LN) {
+      if (nch != 24) return false;
+      if (M <= 16) LEAN(4, 6, 1, 1, 1, 1);
+      else if (M <= 48) LEAN(4, 6, 1, 1, 1, 2);
+      else LEAN(4, 6, 1, 1, 2, 2);
+    } else if constexpr (!W8 && NORM == NORM_RMS) {
+      if (nch != 128 || M > 16) return false;
+      LEAN(8, 4, 4, 2, 1, 2);
+    } else if constexpr (!W8) {
+      if (nch == 24) LEAN(4, 6, 1, 1, 1, 1);
+      else if (nch == 96) LEAN(4, 6, 4, 3, 1, 1);
+      else if (nch == 128 && M <= 16) LEAN(8, 4, 4, 4, 1, 1);
+      else return false;
+    } else if constexpr (NORM == NORM_LN) {
+      if (nch != 25) return false;
+      if (M <= 16) LEAN(5, 5, 1, 1, 1, 2);
+      else if (M <= 48) LEAN(5, 1, 5, 2, 1, 4);
+      else LEAN(5, 1, 5, 1, 2, 4);
+    } else {
+      if (nch == 25) {
+        if (M <= 32) LEAN(5, 5, 1, 1, 1, 1);
+        else LEAN(5, 1, 5, 3, 1, 2);
+      } else if (nch == 100) {
+        if (M <= 32) LEAN(10, 1, 10, 4, 1, 1);
+        else LEAN(10, 1, 10, 2, 1, 2);
+      } else {
+        return false;
+      }
+    }
+#undef LEAN
+    return true;
+  }
+}
+
+bool dnn_gemm_lean(const LeanArgs& p, int nch, int act, int norm, bool w8, hipStream_t st) {
+#define LG(A, N)                                                                                  \
+  if (act == A && norm == N) return w8 ? lean_gemm<A, N, true>(p, nch, st) : lean_gemm<A, N, false>(p, nch, st);
+  LG(ACT_NONE, NORM_LN) LG(ACT_GELU, NORM_LN) LG(ACT_NONE, NORM_NONE) LG(ACT_NONE, NORM_RMS)
+#undef LG
+  return false;
+}
+
+}  // namespace dnn

@@ -32,6 +32,7 @@
 #include <cstdlib>
 #include "gemm_epilogue.h"
 #include "gemm_head.h"
+#include "gemm_lean.h"
 #include "gemm_oneshot.h"
 #include "gemm_stream.h"
 
@@ -52,25 +53,6 @@ __device__ __forceinline__ f32x4 sk_mma(const i32x4& w, const i32x4& a, f32x4 ac
     __builtin_memcpy(&ab, &a, 16);
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, ab, acc, 0, 0, 0);
   }
-}
-
-enum SkNorm { NORM_NONE = 0, NORM_RMS = 1, NORM_LN = 2 };
-
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-
-// 16 OCP e4m3 weight bytes -> 16 bf16 (exact: every e4m3 value is a bf16
-// value).  gfx950's v_cvt_scalef32_pk_bf16_fp8 (scale 1.0) turns two bytes into
-// a packed bf16 pair in one op: 8 VALU per 16 B instead of 8 fp32 converts + 8
-// repacks — the decode weight stream is VALU-paced at batch 1.
-__device__ __forceinline__ void w8_to_bf16(const i32x4& w, bf16x8& lo, bf16x8& hi) {
-  bf16x2v o[8];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    o[2 * i] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((uint32_t)w[i], 1.0f, false);
-    o[2 * i + 1] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((uint32_t)w[i], 1.0f, true);
-  }
-  __builtin_memcpy(&lo, &o[0], 16);
-  __builtin_memcpy(&hi, &o[4], 16);
 }
 
 // Shifted sum and sum of squares of the 8 bf16 of one A fragment: x - c with
@@ -921,6 +903,12 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
   const bool pin_any = g_skinny_pin.id != 0 && (g_skinny_pin.n == 0 || g_skinny_pin.n == N) &&
                        (g_skinny_pin.k == 0 || g_skinny_pin.k * 2 == kbytes);
   if constexpr (!F32 && !FP8 && ACT != ACT_RELU) if (!pin_any) {
+    if (g_os_on == 1 && dnn_gemm_lean({(const uint8_t*)A, lda_b, (const uint8_t*)Wsh, sw, (bf16_t*)C, ldc, bias,
+                                                  (const bf16_t*)R, ldr, M, N, colsum, eps, g_rs_cur.in, g_rs_cur.in_ld,
+                                                  g_rs_cur.out, g_rs_cur.out_ld}, kbytes / 64, ACT, NORM, W8, st)) {
+      if (R != nullptr && g_rs_cur.out != nullptr) g_rs_written = 1;
+      return (int)hipGetLastError();
+    }
     OsCfg oc;
     if (os_eligible<ACT, NORM, W8>(A, lda_b, Wsh, M, kbytes) && os_plan<W8>(M, N, kbytes, ws != nullptr, ws_bytes, oc))
       return launch_os<ACT, NORM, W8>(oc, A, lda_b, Wsh, sw, C, ldc, bias, R, ldr, M, N, kbytes, colsum, eps, st, ws);
