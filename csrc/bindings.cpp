@@ -170,6 +170,15 @@ PYBIND11_MODULE(_dnn_hip, m) {
   m.def("cifar_head_tail_x3", [](u64 hid, u64 w2h, u64 w2l, u64 b2, u64 probs, u64 pred, int B, u64 st) {
     return dnn_cifar_head_tail_x3(CFP(hid), CP(w2h), CP(w2l), CFP(b2), FP(probs), IP(pred), B, ST(st));
   });
+  // a pass on a few images: stage 0 and head, p = x, h, w1h, w1l, b1, w2h, w2l, b2, keep | fc1 h, l, bias, part,
+  // hid, fc2 h, l, bias, probs, pred
+  m.def("cifar_pass_few", [](const std::vector<u64>& p, int B, int grid, int split, u64 st) {
+    if (p.size() != 19) throw std::runtime_error("cifar_pass_few: ragged arguments");
+    const int rc = dnn_cifar_stage0_x3(CFP(p[0]), FP(p[1]), CP(p[2]), CP(p[3]), CFP(p[4]), CP(p[5]), CP(p[6]), CFP(p[7]), B,
+                                       grid, ST(st), split, FP(p[8]));
+    return rc ? rc : dnn_cifar_head_few(CFP(p[1]), split, CP(p[9]), CP(p[10]), CFP(p[11]), FP(p[12]), FP(p[13]), CP(p[14]),
+                                        CP(p[15]), CFP(p[16]), FP(p[17]), reinterpret_cast<int*>(P(p[18])), B, ST(st));
+  });
   m.def("cifar_head_few", [](u64 a, int blocked, u64 wh, u64 wl, u64 b1, u64 part, u64 hid, u64 w2h, u64 w2l, u64 b2,
                              u64 probs, u64 pred, int M, u64 st) {
     return dnn_cifar_head_few(CFP(a), blocked, CP(wh), CP(wl), CFP(b1), FP(part), FP(hid), CP(w2h), CP(w2l), CFP(b2),

@@ -265,7 +265,7 @@ def stage0_forward(x: torch.Tensor, w: CifarStage0Weights, out: Optional[torch.T
         if keep.shape[0] != B or abs(ptr(keep) - ptr(x)) < x.nbytes:
             raise ValueError("stage0: keep must be as large as x and apart from it")
     if w.precision == "fp32":
-        if B > WINO_ROUNDS * (grid or 256) and w.u2h is not None:
+        if not stage0_direct(B, w, grid):
             check(lib().cifar_stage0_wino(ptr(x), ptr(out), ptr(w.w1h), ptr(w.w1l), ptr(w.b1), ptr(w.w2h), ptr(w.w2l),
                                           ptr(w.u2h), ptr(w.u2l), ptr(w.b2), ptr(w.sc), B, grid, stream_ptr(), split,
                                           ptr(keep)), "cifar_stage0_wino")
@@ -276,6 +276,25 @@ def stage0_forward(x: torch.Tensor, w: CifarStage0Weights, out: Optional[torch.T
         check(lib().cifar_stage0_v4(ptr(x), ptr(out), ptr(w.w1), ptr(w.b1), ptr(w.w2), ptr(w.b2), B, grid,
                                     stream_ptr()), "cifar_stage0_v4")
     return out
+
+
+def stage0_direct(B: int, w: CifarStage0Weights, grid: int = 0) -> bool:
+    """fp32: conv2 as it is, not by Winograd."""
+    return B <= WINO_ROUNDS * (grid or STAGE0_GRID or 256) or w.u2h is None
+
+
+def plain(t: torch.Tensor, shape: tuple) -> bool:
+    return t.shape == shape and t.dtype == torch.float32 and t.is_contiguous()
+
+
+def pass_few(x: torch.Tensor, w0: CifarStage0Weights, h: torch.Tensor, keep: torch.Tensor, wh: CifarHeadWeights,
+             scratch: torch.Tensor, hid: torch.Tensor, probs: torch.Tensor, pred: torch.Tensor, boundary: str) -> None:
+    """``stage0_forward`` (``keep``) and ``head_forward`` of up to ``FC1_FEW_ROWS`` images, fp32, into plain buffers that are
+    as large as those take, by one native call."""
+    args = [0 if t is None else t.data_ptr() for t in (x, h, w0.w1h, w0.w1l, w0.b1, w0.w2h, w0.w2l, w0.b2, keep, wh.w_fc1h,
+                                                       wh.w_fc1l, wh.b_fc1, scratch, hid, wh.w_fc2h, wh.w_fc2l, wh.b_fc2,
+                                                       probs, pred)]
+    check(lib().cifar_pass_few(args, x.shape[0], STAGE0_GRID, int(boundary == "split"), stream_ptr()), "cifar_pass_few")
 
 
 def _head_few(h: torch.Tensor, w: CifarHeadWeights, hid: Optional[torch.Tensor], probs: Optional[torch.Tensor],

@@ -149,6 +149,24 @@ class CifarHipStage(StageCompute):
         return StageOutput(probs, pred)
 
 
+    def pass_few(self, last: "StageCompute", x: torch.Tensor, h: torch.Tensor, probs: torch.Tensor,
+                 keep: torch.Tensor) -> Optional[StageOutput]:
+        """This stage on ``x`` (float32, contiguous, as ``forward`` with ``keep``) and ``last`` on its output ``h``,
+        their three launches by one native call: the pass of one image is bound by the host (25 us of it, 15 of the
+        device's).  None, with nothing launched, where ``forward`` of both has to decide: more images, other ranges,
+        devices or encodings, a ``last`` that was replaced or wrapped, buffers that are not plain."""
+        B, c, wh = x.shape[0], self._cops, getattr(last, "wh", None)
+        if not (0 < B <= c.FC1_FEW_ROWS and type(last) is type(self) is CifarHipStage and "forward" not in last.__dict__
+                and (self.start, self.end, last.start, last.end) == (0, 1, 2, 3) and last.precision == "fp32"
+                and self.boundary == last.boundary and last.device == self.device
+                and c.stage0_direct(B, self.w0) and c.plain(h, (B, 4096)) and c.plain(probs, (B, 10))
+                and c.plain(keep, (B, 3, 32, 32)) and abs(keep.data_ptr() - x.data_ptr()) >= x.nbytes):
+            return None
+        buf = last._buf(B)
+        c.pass_few(x, self.w0, h, keep, wh, buf["split"], buf["hid"], probs, buf["pred"], self.boundary)
+        return StageOutput(probs, buf["pred"])
+
+
 class TorchStage(StageCompute):
     """Golden torch module as a stage (CPU fp32 plumbing path / tests)."""
 
