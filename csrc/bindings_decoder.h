@@ -229,6 +229,10 @@ inline void bind_decoder(py::module_& m) {
   m.def("paged_prefill", [](const PagedAttnArgs& a, u64 tiles, int ntiles, u64 st) {
     return dnn_paged_prefill(&a, CIP(tiles), ntiles, ST(st));
   });
+  m.def("paged_mixed", [](const PagedAttnArgs& a, u64 tiles, int ntiles, u64 rows, int nrows, int splits, u64 ws,
+                          long long ws_elems, u64 st) {
+    return dnn_paged_mixed(&a, CIP(tiles), ntiles, CIP(rows), nrows, splits, FP(ws), ws_elems, ST(st));
+  });
   m.def("paged_decode", [](const PagedAttnArgs& a, u64 rows, int nrows, int splits, u64 ws, long long ws_elems,
                            u64 st) {
     return dnn_paged_decode(&a, CIP(rows), nrows, splits, FP(ws), ws_elems, ST(st));

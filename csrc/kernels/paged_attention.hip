@@ -26,6 +26,9 @@
 // Scores, softmax and accumulation are fp32; S^T = K Q^T keeps a query on one
 // lane pair, so row maxima and sums are in registers, and O^T += V^T P^T takes
 // P from the score registers and V^T by transposing LDS reads.
+#include <algorithm>
+#include <climits>
+
 #include "attention_tile.h"
 #include "residual_api.h"
 
@@ -119,17 +122,14 @@ __device__ __forceinline__ float pa_gate(const PagedAttnArgs& a, int row, int he
 // ---------------------------------------------------------------- prefill
 // tiles: {first batch row of the chunk, its tokens, slot, first packed row}
 template <int DK, int DV>
-__global__ __launch_bounds__(256, (DK + DV <= 256) ? 2 : 1) void paged_prefill_kernel(PagedAttnArgs a,
-                                                                                      const int4* __restrict__ tiles) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+__device__ __forceinline__ void paged_prefill_tile(const PagedAttnArgs& a, const int4 t, const int g, char* smem) {
   char* ks = smem;
   char* vs = smem + PG * DK * 2;
   constexpr int NKS = DK / 16, NDT = DV / 32, CK = DK / 8, CV = DV / 8;
   constexpr int NIK = PG * CK / 256, NIV = PG * CV / 256;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int h = lane >> 5, r32 = lane & 31;
-  const int g = blockIdx.x, R = a.H / a.G;
-  const int4 t = tiles[blockIdx.y];
+  const int R = a.H / a.G;
   const int tok0 = t.x, n = t.y, slot = t.z, row0 = t.w;
   const int p0 = a.pos[tok0];
   const int last = n - 1;
@@ -243,56 +243,56 @@ __global__ __launch_bounds__(256, (DK + DV <= 256) ? 2 : 1) void paged_prefill_k
     }
 }
 
+template <int DK, int DV>
+__global__ __launch_bounds__(256, (DK + DV <= 256) ? 2 : 1) void paged_prefill_kernel(PagedAttnArgs a,
+                                                                                      const int4* __restrict__ tiles) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  paged_prefill_tile<DK, DV>(a, tiles[blockIdx.y], blockIdx.x, smem);
+}
+
 // ---------------------------------------------------------------- decode
-// grid (G * head tiles, sequences, splits); rows[e] = batch row of sequence e.
-// ws (splits > 1): [e][H][splits][DV + 2] = {max, sum, O} partials.
+// A workgroup of NW waves: 32 query heads (at most) of KV head g of sequence e, part z of ns of its keys; rows[e] = the
+// batch row.  ws (ns > 1): [e][H][ns][DV + 2] = {max, sum, O} partials.
+//
+// The token's own key and value are taken from the projection row by the wave that has their unit (the last one), and
+// stored behind everything else: a store that the wave then waits for and reads back is a round trip more, and
+// the page numbers of a wave are one load.  Eight waves where the launch leaves CUs idle: 32 heads over 8, 2 to 6
+// sequences of 150 to 400 keys, 11.4 to 13.3 us with four waves and the store, 8.7 to 11.4 so: four dependent reads
+// (row, slot, page, keys), 10 KB of code and two units of keys in turn.
 constexpr int DU = 32;  // keys per unit
 
-template <int DV>
+template <int DV, int NW>
 __host__ __device__ constexpr int pa_dec_lds(int rt_rows) {
-  const int v = 4 * DU * (DV * 2 + 64), m = 4 * rt_rows * (DV + 2) * 4;
+  const int v = NW * DU * (DV * 2 + 64), m = NW * rt_rows * (DV + 2) * 4;
   return v > m ? v : m;
 }
 
-template <int DK, int DV>
-__global__ __launch_bounds__(256, (DK + DV <= 256) ? 2 : 1) void paged_decode_kernel(PagedAttnArgs a,
-                                                                                     const int* __restrict__ rows,
-                                                                                     float* __restrict__ ws) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+template <int DK, int DV, int NW>
+__device__ __forceinline__ void paged_decode_part(const PagedAttnArgs& a, const int* __restrict__ rows,
+                                                  float* __restrict__ ws, const int grt, const int e, const int z,
+                                                  const int ns, const bool written, char* smem) {
   constexpr int NKS = DK / 16, NDT = DV / 32, CV = DV / 8;
   constexpr int NIV = DU * CV / 64;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, r32 = lane & 31;
   const int R = a.H / a.G, nrt = (R + 31) / 32;
-  const int g = blockIdx.x / nrt, rt = blockIdx.x % nrt;
+  const int g = grt / nrt, rt = grt % nrt;
   const int rr = min(R - rt * 32, 32);  // query heads of this workgroup
-  const int e = blockIdx.y, row = rows[e], ns = gridDim.z;
+  const int row = rows[e];
   const int slot = a.slots[row], p = a.pos[row];
   char* vs = smem + wave * DU * PaV<DV>::STRIDE;
 
   const Units u = pa_units(p, p, a.window, a.keep, DU);
-  const int ub = (int)((long)u.total * blockIdx.z / ns), ue = (int)((long)u.total * (blockIdx.z + 1) / ns);
+  const int ub = (int)((long)u.total * z / ns), ue = (int)((long)u.total * (z + 1) / ns);
 
   const bf16_t* rowp = reinterpret_cast<const bf16_t*>(a.qkv) + (size_t)row * a.ldq;
-  // the token's own key and value: the wave that reads their unit (the last of
-  // the list) stores them first
-  const int lastw = (u.total - 1 - ub) & 3;
-  if (!a.written && ue == u.total && wave == lastw) {
-    const int page = pa_page(a, slot, p / PG);
-    if (page >= 0) {
-      bf16_t* kd = reinterpret_cast<bf16_t*>(a.kp) + (((size_t)page * a.G + g) * PG + p % PG) * DK;
-      bf16_t* vd = reinterpret_cast<bf16_t*>(a.vp) + (((size_t)page * a.G + g) * PG + p % PG) * DV;
-      if (lane < DK / 8)
-        *reinterpret_cast<uint4*>(kd + lane * 8) =
-            *reinterpret_cast<const uint4*>(rowp + a.H * DK + g * DK + lane * 8);
-      if (lane < DV / 8)
-        *reinterpret_cast<uint4*>(vd + lane * 8) =
-            *reinterpret_cast<const uint4*>(rowp + (a.H + a.G) * DK + g * DV + lane * 8);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const bool own = !written && ue == u.total && ue > ub && wave == (u.total - 1 - ub) % NW;  // this wave has the token's unit
+  // pages of the wave's first 64 units, a lane each
+  int pages = 0;
+  {
+    const int i = ub + wave + lane * NW;
+    if (i < ue) pages = pa_page(a, slot, u.at(i) / (PG / DU));
   }
-
   bf16x8 qf[NKS];
   {
     const bf16_t* qp = rowp + (g * R + rt * 32 + min(r32, rr - 1)) * DK + 8 * h;
@@ -303,7 +303,7 @@ __global__ __launch_bounds__(256, (DK + DV <= 256) ? 2 : 1) void paged_decode_ke
 #pragma unroll
   for (int i = 0; i < NDT; ++i) o[i] = f32x16{};
   float m_i, l_i;  // one wave of a token's workgroups brings the sink
-  pa_begin(a, g * R + rt * 32 + min(r32, rr - 1), wave == 0 && blockIdx.z == 0, m_i, l_i);
+  pa_begin(a, g * R + rt * 32 + min(r32, rr - 1), wave == 0 && z == 0, m_i, l_i);
   const bool terms = pa_has_terms(a);
   const float sc0 = a.scale * LOG2E, sc = terms ? 1.f : sc0;
   const float slope = pa_slope(a, g * R + rt * 32 + min(r32, rr - 1));
@@ -312,25 +312,35 @@ __global__ __launch_bounds__(256, (DK + DV <= 256) ? 2 : 1) void paged_decode_ke
   i32x4 pv[NIV];
   f32x4 ksc[4];
   auto load = [&](int i) __attribute__((always_inline)) {
-    const int unit = u.at(i);
-    const int page = max(pa_page(a, slot, unit / (PG / DU)), 0);
+    const int unit = u.at(i), k = (i - ub) / NW;
+    const int page = max(k < 64 ? __builtin_amdgcn_readlane(pages, k) : pa_page(a, slot, unit / (PG / DU)), 0);
     const size_t k0 = ((size_t)page * a.G + g) * PG + (unit % (PG / DU)) * DU;
     const bf16_t* kb = reinterpret_cast<const bf16_t*>(a.kp) + (k0 + r32) * DK + 8 * h;
     const bf16_t* vb = reinterpret_cast<const bf16_t*>(a.vp) + k0 * DV;
+    const int at = own && i == ue - 1 ? p - unit * DU : -1;  // the token's own row of the tile
+    if (r32 == at) kb = rowp + (a.H + g) * DK + 8 * h;
     if (!a.shared) {
 #pragma unroll
       for (int s = 0; s < NKS; ++s) kf[s] = *reinterpret_cast<const bf16x8*>(kb + s * 16);
     }
 #pragma unroll
-    for (int it = 0; it < NIV; ++it) pv[it] = *reinterpret_cast<const i32x4*>(vb + (it * 64 + lane) * 8);
+    for (int it = 0; it < NIV; ++it) {
+      const int c = it * 64 + lane;
+      pv[it] = *reinterpret_cast<const i32x4*>(c / CV == at ? rowp + (a.H + a.G) * DK + g * DV + c % CV * 8 : vb + c * 8);
+    }
     if (terms) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) ksc[q] = pa_kscale4(a, page, (unit % (PG / DU)) * DU + 8 * q + 4 * h) * sc0;
     }
   };
   int i = ub + wave;
-  if (i < ue) load(i);
-  for (; i < ue; i += 4) {
+  constexpr bool AHEAD = NW == 4;  // eight waves have a unit or two each: the next one's loads ahead are code more than time
+  if (AHEAD && i < ue) load(i);
+  // the gate of the first value that this thread will store, ahead of the keys' arrival
+  const int h0 = min(g * R + rt * 32 + tid / DV, a.H - 1);
+  const float gate0 = pa_gate(a, row, h0) * pa_gate_el(a, row, h0 * DV + tid % DV);
+  for (; i < ue; i += NW) {
+    if constexpr (!AHEAD) load(i);
     const int kb0 = u.at(i) * DU;
     f32x16 s[1];
     s[0] = f32x16{};
@@ -360,7 +370,7 @@ __global__ __launch_bounds__(256, (DK + DV <= 256) ? 2 : 1) void paged_decode_ke
           s[0][4 * q + j] = fmaf(s[0][4 * q + j], ksc[q][j], fmaf(slope, (float)(8 * q + j), off));
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (i + 4 < ue) load(i + 4);
+    if (AHEAD && i + NW < ue) load(i + NW);
     if (kb0 + DU - 1 > p || !(p - kb0 < a.window || kb0 + DU <= a.keep)) {
 #pragma unroll
       for (int q = 0; q < 16; ++q)
@@ -375,7 +385,7 @@ __global__ __launch_bounds__(256, (DK + DV <= 256) ? 2 : 1) void paged_decode_ke
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
 
-  // merge the four waves: {m, l, O[DV]} of each query head
+  // merge the waves: {m, l, O[DV]} of each query head
   __syncthreads();
   float* mg = reinterpret_cast<float*>(smem);
   if (r32 < rr) {
@@ -390,14 +400,14 @@ __global__ __launch_bounds__(256, (DK + DV <= 256) ? 2 : 1) void paged_decode_ke
       for (int q = 0; q < 16; ++q) d[2 + t * 32 + (q & 3) + 8 * (q >> 2) + 4 * h] = o[t][q];
   }
   __syncthreads();
-  for (int x = tid; x < rr * DV; x += 256) {
+  for (int x = tid; x < rr * DV; x += NW * 64) {
     const int r = x / DV, c = x % DV, head = g * R + rt * 32 + r;
     float m = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) m = fmaxf(m, mg[(w * rr + r) * (DV + 2)]);
+    for (int w = 0; w < NW; ++w) m = fmaxf(m, mg[(w * rr + r) * (DV + 2)]);
     float l = 0.f, v = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < NW; ++w) {
       const float* d = mg + (w * rr + r) * (DV + 2);
       const float f = d[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(d[0] - m);
       l = fmaf(d[1], f, l);
@@ -405,9 +415,9 @@ __global__ __launch_bounds__(256, (DK + DV <= 256) ? 2 : 1) void paged_decode_ke
     }
     if (ns == 1) {
       reinterpret_cast<bf16_t*>(a.out)[(size_t)row * a.ldo + head * DV + c] =
-          f2bf((l > 0.f ? v / l : 0.f) * pa_gate(a, row, head) * pa_gate_el(a, row, head * DV + c));
+          f2bf((l > 0.f ? v / l : 0.f) * (x == tid ? gate0 : pa_gate(a, row, head) * pa_gate_el(a, row, head * DV + c)));
     } else {
-      float* d = ws + (((size_t)e * a.H + head) * ns + blockIdx.z) * (DV + 2);
+      float* d = ws + (((size_t)e * a.H + head) * ns + z) * (DV + 2);
       if (c == 0) {
         d[0] = m;
         d[1] = l;
@@ -415,6 +425,42 @@ __global__ __launch_bounds__(256, (DK + DV <= 256) ? 2 : 1) void paged_decode_ke
       d[2 + c] = v;
     }
   }
+  if (own) {  // behind every read of the page by this workgroup; another one of the same head takes the row's own as well
+    const int page = pa_page(a, slot, p / PG);
+    if (page < 0) return;
+    bf16_t* kd = reinterpret_cast<bf16_t*>(a.kp) + (((size_t)page * a.G + g) * PG + p % PG) * DK;
+    bf16_t* vd = reinterpret_cast<bf16_t*>(a.vp) + (((size_t)page * a.G + g) * PG + p % PG) * DV;
+    if (lane < DK / 8)
+      *reinterpret_cast<uint4*>(kd + lane * 8) = *reinterpret_cast<const uint4*>(rowp + a.H * DK + g * DK + lane * 8);
+    if (lane < DV / 8)
+      *reinterpret_cast<uint4*>(vd + lane * 8) = *reinterpret_cast<const uint4*>(rowp + (a.H + a.G) * DK + g * DV + lane * 8);
+  }
+}
+
+// grid (G * head tiles, sequences, splits)
+template <int DK, int DV, int NW>
+__global__ __launch_bounds__(NW * 64, (DK + DV <= 256) ? 2 : 1) void paged_decode_kernel(PagedAttnArgs a,
+                                                                                         const int* __restrict__ rows,
+                                                                                         float* __restrict__ ws) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  paged_decode_part<DK, DV, NW>(a, rows, ws, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, a.written != 0, smem);
+}
+
+// Portions and single tokens of one step (their keys and values are in the pages): the tiles, then the sequences' parts,
+// four waves each.  The few workgroups of the single tokens run beside the tiles instead of behind them: 128 to
+// 160 workgroups of both, 12 to 13 and 16.4 us one after the other, 17.4 together.
+template <int DK, int DV>
+__global__ __launch_bounds__(256, (DK + DV <= 256) ? 2 : 1) void paged_mixed_kernel(PagedAttnArgs a, const int4* __restrict__ tiles,
+                                                                                    int ntiles, const int* __restrict__ rows,
+                                                                                    int ns, float* __restrict__ ws) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int b = blockIdx.x, np = ntiles * a.G;
+  if (b < np) {
+    paged_prefill_tile<DK, DV>(a, tiles[b / a.G], b % a.G, smem);
+    return;
+  }
+  const int per = a.G * ((a.H / a.G + 31) / 32), x = b - np;
+  paged_decode_part<DK, DV, 4>(a, rows, ws, x % per, x / per / ns, x / per % ns, ns, true, smem);
 }
 
 // One workgroup per (sequence, head): the four waves take every fourth split.
@@ -558,18 +604,50 @@ extern "C" int dnn_paged_prefill(const PagedAttnArgs* a, const int* tiles, int n
   return (int)hipGetLastError();
 }
 
-extern "C" int dnn_paged_decode(const PagedAttnArgs* a, const int* rows, int nrows, int splits, float* ws,
-                                long long ws_elems, hipStream_t st) {
-  if (!pa_ok(*a, 2) || nrows <= 0 || nrows > 65535 || splits < 1 || splits > 256 || !(a->scale > 0.f)) return -1;
-  if (splits > 1 && (ws == nullptr || ws_elems < (long long)nrows * a->H * splits * (a->DV + 2))) return -1;
-  const int R = a->H / a->G, rr = R < 32 ? R : 32;
-  const dim3 grid(a->G * ((R + 31) / 32), nrows, splits);
-#define PD(K, V) \
-  hipLaunchKernelGGL((paged_decode_kernel<K, V>), grid, dim3(256), pa_dec_lds<V>(rr), st, *a, rows, ws);
-  PA_DISPATCH(PD)
-#undef PD
+static void launch_combine(const PagedAttnArgs* a, const int* rows, int nrows, int splits, const float* ws, hipStream_t st) {
   if (splits > 1)
     hipLaunchKernelGGL(paged_combine_kernel, dim3((unsigned)(nrows * a->H)), dim3(256), 0, st, *a, rows, splits, ws);
+}
+static bool pa_dec_ok(const PagedAttnArgs& a, int nrows, int splits, const float* ws, long long ws_elems) {
+  return pa_ok(a, 2) && nrows > 0 && nrows <= 65535 && splits >= 1 && splits <= 256 && a.scale > 0.f &&
+         (splits == 1 || (ws != nullptr && ws_elems >= (long long)nrows * a.H * splits * (a.DV + 2)));
+}
+
+extern "C" int dnn_paged_decode(const PagedAttnArgs* a, const int* rows, int nrows, int splits, float* ws,
+                                long long ws_elems, hipStream_t st) {
+  if (!pa_dec_ok(*a, nrows, splits, ws, ws_elems)) return -1;
+  const int R = a->H / a->G, rr = R < 32 ? R : 32;
+  const dim3 grid(a->G * ((R + 31) / 32), nrows, splits);
+  // eight waves a workgroup where there is a CU for each and their tiles fit half its LDS
+  const bool w8 = (long)grid.x * nrows * splits <= 256;
+#define PD(K, V)                                                                                                          \
+  {                                                                                                                       \
+    constexpr bool fit = K + V <= 256;                                                                                    \
+    if (fit && w8 && pa_dec_lds<V, 8>(rr) <= 80 * 1024)                                                                   \
+      hipLaunchKernelGGL((paged_decode_kernel<K, V, fit ? 8 : 4>), grid, dim3(512), (pa_dec_lds<V, 8>(rr)), st, *a, rows, ws); \
+    else                                                                                                                  \
+      hipLaunchKernelGGL((paged_decode_kernel<K, V, 4>), grid, dim3(256), (pa_dec_lds<V, 4>(rr)), st, *a, rows, ws);        \
+  }
+  PA_DISPATCH(PD)
+#undef PD
+  launch_combine(a, rows, nrows, splits, ws, st);
+  return (int)hipGetLastError();
+}
+
+// dnn_paged_prefill and dnn_paged_decode of one step whose rows' keys and values are written already, in one launch.
+extern "C" int dnn_paged_mixed(const PagedAttnArgs* a, const int* tiles, int ntiles, const int* rows, int nrows, int splits,
+                               float* ws, long long ws_elems, hipStream_t st) {
+  if (!pa_dec_ok(*a, nrows, splits, ws, ws_elems) || ntiles <= 0 || ((uintptr_t)tiles & 15) != 0) return -1;
+  const int R = a->H / a->G, rr = R < 32 ? R : 32;
+  const long long wgs = (long long)ntiles * a->G + (long long)a->G * ((R + 31) / 32) * nrows * splits;
+  if (wgs > INT_MAX) return -1;
+#define PM(K, V)                                                                                                          \
+  hipLaunchKernelGGL((paged_mixed_kernel<K, V>), dim3((unsigned)wgs), dim3(256),                                          \
+                     (std::max(PG * (K * 2 + PaV<V>::STRIDE), pa_dec_lds<V, 4>(rr))), st, *a, (const int4*)tiles, ntiles, rows, \
+                     splits, ws);
+  PA_DISPATCH(PM)
+#undef PM
+  launch_combine(a, rows, nrows, splits, ws, st);
   return (int)hipGetLastError();
 }
 

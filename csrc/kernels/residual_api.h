@@ -182,6 +182,8 @@ int dnn_gemm_f32(const float* A, int lda, const float* W, int ldw, float* C, int
                  int K, hipStream_t st);
 int dnn_paged_write(const PagedAttnArgs* a, int f32, hipStream_t st);
 int dnn_paged_prefill(const PagedAttnArgs* a, const int* tiles, int ntiles, hipStream_t st);
+int dnn_paged_mixed(const PagedAttnArgs* a, const int* tiles, int ntiles, const int* rows, int nrows, int splits, float* ws,
+                    long long ws_elems, hipStream_t st);
 int dnn_paged_decode(const PagedAttnArgs* a, const int* rows, int nrows, int splits, float* ws, long long ws_elems,
                      hipStream_t st);
 int dnn_paged_attn_f32(const PagedAttnArgs* a, hipStream_t st);

@@ -297,11 +297,15 @@ def paged_write(args, f32: bool) -> None:
     check(lib().paged_write(args, int(f32), stream_ptr()), "paged_write")
 
 
+def _tiles(tiles: torch.Tensor, what: str) -> None:
+    if tiles.dtype != torch.int32 or tiles.dim() != 2 or tiles.shape[1] != 4 or not tiles.is_contiguous():
+        raise ValueError(f"{what}: tiles must be contiguous int32 (n, 4)")
+
+
 def paged_prefill(args, tiles: torch.Tensor) -> None:
     """Attention of chunks of tokens already written to the cache.  ``tiles``
     (n, 4) int32: {first row, tokens, slot, first packed row} (``chunk_tiles``)."""
-    if tiles.dtype != torch.int32 or tiles.dim() != 2 or tiles.shape[1] != 4 or not tiles.is_contiguous():
-        raise ValueError("paged_prefill: tiles must be contiguous int32 (n, 4)")
+    _tiles(tiles, "paged_prefill")
     n = tiles.shape[0]
     for i in range(0, n, 65535):
         part = tiles[i:i + 65535]
@@ -324,12 +328,25 @@ def paged_splits(n_seq: int, H: int, G: int, keys: int, window: Optional[int], k
     return max(1, min(-(-512 // wgs), units // 8, 64))
 
 
+def _decode_parts(rows: torch.Tensor, n: int, splits: int, ws: Optional[torch.Tensor], what: str) -> None:
+    _index(rows, n, f"{what} rows")
+    if splits > 1 and (ws is None or ws.dtype != torch.float32 or not ws.is_contiguous()):
+        raise ValueError(f"{what}: splits > 1 needs an fp32 workspace")
+
+
+def paged_mixed(args, tiles: torch.Tensor, rows: torch.Tensor, n: int, splits: int, ws: Optional[torch.Tensor]) -> None:
+    """``paged_prefill`` of ``tiles`` and ``paged_decode`` of ``n`` sequences in one launch; every row's k / v is in the
+    cache already."""
+    _tiles(tiles, "paged_mixed")
+    _decode_parts(rows, n, splits, ws, "paged_mixed")
+    check(lib().paged_mixed(args, ptr(tiles), tiles.shape[0], ptr(rows), n, splits, ptr(ws), 0 if ws is None else ws.numel(),
+                            stream_ptr()), "paged_mixed")
+
+
 def paged_decode(args, rows: torch.Tensor, n: int, splits: int, ws: Optional[torch.Tensor]) -> None:
     """One token of each of ``n`` sequences (``rows``: their batch rows); also
     stores the tokens' k / v.  ``ws``: fp32, n * H * splits * (DV + 2) for splits > 1."""
-    _index(rows, n, "paged_decode rows")
-    if splits > 1 and (ws is None or ws.dtype != torch.float32 or not ws.is_contiguous()):
-        raise ValueError("paged_decode: splits > 1 needs an fp32 workspace")
+    _decode_parts(rows, n, splits, ws, "paged_decode")
     check(lib().paged_decode(args, ptr(rows), n, splits, ptr(ws), 0 if ws is None else ws.numel(), stream_ptr()),
           "paged_decode")
 

@@ -129,8 +129,11 @@ def run_attention(st, args, b: StepBatch, group: int, splits: int, ws, write: bo
     if b.chunks:
         if write:
             D_.paged_write(args, False)
-        D_.paged_prefill(args, b.tiles[group])
-    if b.n_dec:
+        if b.n_dec:
+            D_.paged_mixed(args, b.tiles[group], b.dec_rows, b.n_dec, splits, ws)
+        else:
+            D_.paged_prefill(args, b.tiles[group])
+    elif b.n_dec:
         D_.paged_decode(args, b.dec_rows, b.n_dec, splits, ws)
 
 
