@@ -96,6 +96,19 @@ __device__ __forceinline__ void epi_t4_any(const f32x4& v, int m, int n, int M, 
   else epi_t4<ACT_NONE, false>(v, m, n, M, N, p.C, p.ldc, nullptr, R, p.ldr, vec);
 }
 
+// Epilogues of their own (gemm_mid_plain.hip), where the host knows that every wave's columns are whole and leave as
+// pairs of 16-byte bf16 stores: an activation, and what else there is.  MID_ANY: whatever the arguments say.
+enum MidEpi { MID_ANY = -1, MID_RES = 8, MID_STAT = 16, MID_COLS = 32, MID_BIAS = 64, MID_STATS_OUT = 128 };
+constexpr int mid_epi_act(int epi) { return epi & 7; }
+
+// Whether rows leave as those epilogues store them (epi_vec_ok, epi_pair_ok), from waves of `cols` columns; at: more
+// vectors that are read 16 bytes at a time.
+inline bool mid_plain_ok(const MidRows& a, int cols, const float* at) {
+  const uintptr_t p = (uintptr_t)a.C | (uintptr_t)a.bias | (uintptr_t)a.R | (uintptr_t)at;
+  return !a.f32 && a.act >= 0 && a.act <= 7 && a.N % cols == 0 && (p & 15) == 0 && a.ldc % 8 == 0 &&
+         (a.R == nullptr || a.ldr % 4 == 0);
+}
+
 // What the epilogue of a wave reads, loaded ahead of the loop: behind it statistics and
 // column sums, bias, then residual rows were up to three trips to memory, 0.5 us each, of
 // kernels that take 6 to 40 (with residual, 1071 x 768 x 768 and x 3072: 11.8 us on average,
@@ -107,6 +120,28 @@ struct MidPre {
   f32x4 cs[J], bs[J];
   bf16x4 rr[RES ? I : 1][J / 2][2];
   bool res;  // rr is loaded
+  template <int EPI>
+  __device__ __forceinline__ void load_plain(const MidRows& p, const float2* rowstat, const float* scale, int mw, int nw, int lane) {
+    const int n = min(nw, p.N - J * 16) + (lane >> 4) * 4;  // a wave past the columns reads the last ones
+    if (rowstat != nullptr) {
+#pragma unroll
+      for (int i = 0; i < I; ++i) rs[i] = rowstat[min(mw + i * 16, p.M - 1)];
+    }
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      if constexpr ((EPI & MID_COLS) != 0) cs[j] = *reinterpret_cast<const f32x4*>(scale + n + j * 16);
+      if constexpr ((EPI & MID_BIAS) != 0) bs[j] = *reinterpret_cast<const f32x4*>(p.bias + n + j * 16);
+    }
+    if constexpr (RES && (EPI & MID_RES) != 0) res_load(p, mw, nw, lane, rr);
+  }
+  template <int R>
+  static __device__ __forceinline__ void res_load(const MidRows& p, int mw, int nw, int lane, bf16x4 (&r)[R][J / 2][2]) {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int jp = 0; jp < J / 2; ++jp)
+        epi_pair_res_load(mw + i * 16, min(nw, p.N - J * 16) + jp * 32, p.M, p.R, p.ldr, lane, r[i % R][jp][0], r[i % R][jp][1]);
+  }
   // rows m of this lane from mw on, the wave's columns from nw on; `scale`: per column (colsum, channel scale) or null
   __device__ __forceinline__ void load(const MidRows& p, const float2* rowstat, const float* scale, int mw, int nw, int lane,
                                        bool rows) {
@@ -366,6 +401,74 @@ __device__ __forceinline__ void mid_rows(f32x4 (&acc)[I][J], int mw, int nw, int
   }
 }
 
+// epi_glu_pair (gemm_epilogue.h) of whole columns in bf16.
+template <int ACT>
+__device__ __forceinline__ void mid_glu_plain(const f32x4& a0, const f32x4& a1, int m, int ncol0, const MidRows& p, int lane) {
+  f32x4 v;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(a0[r]), __float_as_uint(a1[r]), false, false);
+    const float g = __uint_as_float(s[0]), u = __uint_as_float(s[1]);
+    if constexpr (ACT == ACT_GELU_TANH_MUL) v[r] = gelu_tanh(g) * u;
+    else v[r] = g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f)) * u;
+  }
+  if (m < p.M)
+    *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(p.C) + (size_t)m * p.ldc + ncol0 + (lane >> 4) * 4) =
+        make_uint2(pack2bf(v[0], v[1]), pack2bf(v[2], v[3]));
+}
+
+// The same where the epilogue is known (MidEpi).
+template <int I, int J, int EPI>
+__device__ __forceinline__ void mid_rows_plain(f32x4 (&acc)[I][J], int mw, int nw, int lane, const MidRows& p,
+                                               const MidPre<I, J>& pre, float2* parts_out) {
+  constexpr int ACT = mid_epi_act(EPI);
+  constexpr bool PRE = MidPre<I, J>::RES;
+  if (nw >= p.N) return;
+  if constexpr (is_glu(ACT)) {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int jp = 0; jp < J / 2; ++jp)
+        mid_glu_plain<ACT>(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, (nw + jp * 32) / 2, p, lane);
+    return;
+  }
+  {
+#pragma clang fp contract(off)  // as mid_bias_act
+    if constexpr ((EPI & MID_BIAS) != 0) {
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int i = 0; i < I; ++i) acc[i][j] += pre.bs[j];
+    }
+  }
+  if constexpr (ACT != ACT_NONE) {
+    const f32x2 xc = act_consts<ACT>(p.bias, p.N);
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int j = 0; j < J; ++j) acc[i][j] = mid_act<ACT>(acc[i][j], xc);
+  }
+  constexpr bool RES = (EPI & MID_RES) != 0;
+  bf16x4 rl[RES && !PRE ? I : 1][J / 2][2];
+  if constexpr (RES && !PRE) MidPre<I, J>::res_load(p, mw, nw, lane, rl);  // every residual load before the first output
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int jp = 0; jp < J / 2; ++jp) {
+      const int m = mw + i * 16, nb = nw + jp * 32;
+      bf16_t* C = reinterpret_cast<bf16_t*>(p.C);
+      if constexpr (!RES) {
+        epi_pair_bf16<ACT_NONE>(acc[i][2 * jp], acc[i][2 * jp + 1], m, nb, p.M, C, p.ldc, nullptr, nullptr, 0, lane);
+      } else {
+        uint4 x;
+        const bf16x4 r0 = PRE ? pre.rr[PRE ? i : 0][jp][0] : rl[PRE ? 0 : i][jp][0], r1 = PRE ? pre.rr[PRE ? i : 0][jp][1] : rl[PRE ? 0 : i][jp][1];
+        epi_pair_bf16<ACT_NONE, true>(acc[i][2 * jp], acc[i][2 * jp + 1], m, nb, p.M, C, p.ldc, nullptr, p.R, p.ldr, lane, r0, r1,
+                                      f32x2{}, &x);
+        if constexpr ((EPI & MID_STATS_OUT) != 0) mid_part_out(x, m, nb, p, parts_out, lane);
+      }
+    }
+}
+
 // Loop: a K-tile of 64 is multiplied in two halves of 32; the second half's
 // fragments are read behind the first row of products of the first, the next
 // tile's first half behind the first row of the second, one barrier a tile.  The
@@ -473,9 +576,11 @@ enum MidOut { MID_ROWS = 0, MID_SCATTER = 1, MID_PART = 2 };
 
 // MERGE: the folded norm's statistics from partials (a variant of its own: a load under a branch is waited for where
 // the branch ends, ahead of the first request)
-template <class T, MidOut OUT, bool MERGE>
+// EPI: MidEpi
+template <class T, MidOut OUT, bool MERGE, int EPI = MID_ANY>
 __global__ __launch_bounds__(T::THREADS, 2) void gemm_mid_kernel(MidArgs p, QkvScatter scat) {
   constexpr bool PART = OUT == MID_PART;
+  static_assert(EPI == MID_ANY || (OUT == MID_ROWS && T::PW == 0 && (!MERGE || (EPI & MID_STAT) != 0)), "");
   static_assert(PART ? !MERGE : T::PW == 0, "");
   constexpr int I = T::I, J = T::J;
   // S * STAGE bytes (MERGE: MidParts::LDS), given at launch: with the size in the kernel the compiler sees one
@@ -511,7 +616,8 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_mid_kernel(MidArgs p, QkvS
   }
   const int mw = m0 + wm * (I * 16) + fr, nw = n0 + wn * (J * 16);  // the lane's first row, the wave's first column
   MidPre<I, J> pre;
-  if constexpr (!PART) pre.load(p, p.rowstat, p.colsum, mw, nw, lane, OUT == MID_ROWS);
+  if constexpr (EPI != MID_ANY) pre.template load_plain<EPI>(p, !MERGE && (EPI & MID_STAT) != 0 ? p.rowstat : nullptr, p.colsum, mw, nw, lane);
+  else if constexpr (!PART) pre.load(p, p.rowstat, p.colsum, mw, nw, lane, OUT == MID_ROWS);
   f32x4 acc[I][J];
   MidParts<T> parts;
   if constexpr (MERGE) {
@@ -533,6 +639,19 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_mid_kernel(MidArgs p, QkvS
         if (m < M && n < N) *reinterpret_cast<f32x4*>(d + (size_t)m * N + n) = acc[i][j];
       }
     }
+    return;
+  }
+  if constexpr (EPI != MID_ANY) {
+    if constexpr ((EPI & MID_STAT) != 0) {
+#pragma unroll
+      for (int i = 0; i < I; ++i)
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          if constexpr ((EPI & MID_COLS) != 0) acc[i][j] = acc[i][j] * pre.rs[i].x + pre.rs[i].y * pre.cs[j];
+          else acc[i][j] *= pre.rs[i].x;
+        }
+    }
+    mid_rows_plain<I, J, EPI>(acc, mw, nw, lane, p, pre, p.parts_out);
     return;
   }
   if (MERGE || p.rowstat != nullptr) {  // the folded norm, in the 256 x 256 kernel's order of operations
@@ -585,6 +704,17 @@ __global__ __launch_bounds__(256) void gemm_mid_reduce(MidArgs p) {
     return;
   }
   epi_t4_any(a[0][0], m, n, M, N, p, p.R, vec);
+}
+
+template <class T, MidOut OUT, bool MERGE = false, int EPI = MID_ANY>
+static int mid_start(const MidArgs& a, const QkvScatter& scat, hipStream_t st) {
+  constexpr int LDS = MERGE ? MidParts<T>::LDS : T::S * T::STAGE;
+  static const hipError_t room =
+      hipFuncSetAttribute((const void*)gemm_mid_kernel<T, OUT, MERGE, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  if (room != hipSuccess) return (int)room;
+  const int tiles = ((a.M + T::BM - 1) / T::BM) * ((a.N + T::BN - 1) / T::BN);
+  hipLaunchKernelGGL((gemm_mid_kernel<T, OUT, MERGE, EPI>), dim3(tiles * a.splits), dim3(T::THREADS), LDS, st, a, scat);
+  return (int)hipGetLastError();
 }
 
 }  // namespace dnn

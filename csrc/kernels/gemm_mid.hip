@@ -119,28 +119,17 @@ bool mid_skinny(int M, int N, int K, bool norm, bool frag, long long ws_bytes) {
          mid_plan(M, N, K, ws_bytes, MID_BF16).us + (norm ? 3.3f : 0.f);
 }
 
-template <class T, MidOut OUT, bool MERGE = false>
-static int start(const MidArgs& a, const QkvScatter& scat, hipStream_t st) {
-  constexpr int LDS = MERGE ? MidParts<T>::LDS : T::S * T::STAGE;
-  static const hipError_t room =
-      hipFuncSetAttribute((const void*)gemm_mid_kernel<T, OUT, MERGE>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-  if (room != hipSuccess) return (int)room;
-  const int tiles = ((a.M + T::BM - 1) / T::BM) * ((a.N + T::BN - 1) / T::BN);
-  hipLaunchKernelGGL((gemm_mid_kernel<T, OUT, MERGE>), dim3(tiles * a.splits), dim3(T::THREADS), LDS, st, a, scat);
-  return (int)hipGetLastError();
-}
-
 template <class T>
 static int launch(const MidArgs& a, const QkvScatter* scat, hipStream_t st) {
 #ifndef DNN_DECODER_ONLY
   if (a.parts != nullptr) {
     if (a.splits != 1) return -1;
-    return scat != nullptr ? start<T, MID_SCATTER, true>(a, *scat, st) : start<T, MID_ROWS, true>(a, QkvScatter{}, st);
+    return scat != nullptr ? mid_start<T, MID_SCATTER, true>(a, *scat, st) : mid_start<T, MID_ROWS, true>(a, QkvScatter{}, st);
   }
 #endif
-  if (scat != nullptr) return start<T, MID_SCATTER>(a, *scat, st);
-  if (a.splits == 1) return start<T, MID_ROWS>(a, QkvScatter{}, st);
-  if (const int rc = start<typename MidSplit<T>::type, MID_PART>(a, QkvScatter{}, st)) return rc;
+  if (scat != nullptr) return mid_start<T, MID_SCATTER>(a, *scat, st);
+  if (a.splits == 1) return mid_start<T, MID_ROWS>(a, QkvScatter{}, st);
+  if (const int rc = mid_start<typename MidSplit<T>::type, MID_PART>(a, QkvScatter{}, st)) return rc;
   const bool glu = is_glu(a.act);
   const dim3 grid(((glu ? a.N / 2 : a.N) / 4 + 255) / 256, a.M);
   if (glu) hipLaunchKernelGGL((gemm_mid_reduce<1>), grid, dim3(256), 0, st, a);
@@ -173,6 +162,9 @@ int mid_launch(int tile, const MidArgs& a, const QkvScatter* scat, hipStream_t s
   if (a.splits < 1 || (a.splits > 1 && (scat != nullptr || a.part == nullptr || a.N % 4 != 0 || a.K / 64 < a.splits ||
                                         a.M > 65535)))
     return -1;
+  if (scat == nullptr && a.splits == 1) {
+    if (const int rc = mid_plain_launch(tile, a, st); rc != -3) return rc;
+  }
   switch (tile) {
     case 0: return launch<Mid0>(a, scat, st);
     case 1: return launch<Mid1>(a, scat, st);

@@ -48,6 +48,8 @@ inline long long mid_ws(const void* ws, long long bytes) { return ws == nullptr 
 // Widest rows whose partials a workgroup merges, and what the columns of a product with partials divide by.
 constexpr int MID_PARTS_K = 2048, MID_PARTS_N = 64;
 int mid_blocks(int tile);  // workgroups of a tile (K whole) that share a CU
+// The same on a kernel with that epilogue alone (gemm_mid_plain.hip); -3, nothing launched: there is none.
+int mid_plain_launch(int tile, const MidArgs& a, hipStream_t st);
 int mid_launch(int tile, const MidArgs& a, const QkvScatter* scat, hipStream_t st);  // a.splits workgroups over K
 
 }  // namespace dnn

@@ -49,6 +49,7 @@ PER_FILE_FLAGS = {"cifar_fused.hip": ["-ffast-math"],
                   "gemm_skinny.hip": NO_SLP,
                   "gemm_lean.hip": NO_SLP,
                   "gemm_mid.hip": NO_SLP,
+                  "gemm_mid_plain.hip": NO_SLP,
                   "gemm_mid_fp8.hip": NO_SLP,
                   "gemm_bf16.hip": NO_SLP}
 
@@ -124,7 +125,7 @@ def _compile(src: str, force: bool, extra: List[str]) -> str:
 # runs (runtime/decoder.py), compiled without the other families' entry points,
 # for a first use in a checkout that has no library yet (``ensure``).
 SUBSETS = {"": ("_dnn_hip", None, []),
-           "decoder": ("_dnn_decoder", ("gemm_bf16.hip", "gemm_mid.hip", "gemm_skinny.hip", "gemm_lean.hip", "sampler.hip", "gemm_f32.hip",
+           "decoder": ("_dnn_decoder", ("gemm_bf16.hip", "gemm_mid.hip", "gemm_mid_plain.hip", "gemm_skinny.hip", "gemm_lean.hip", "sampler.hip", "gemm_f32.hip",
                                         "residual_rows.hip", "token_gate.hip", "paged_attention.hip",
                                         "qk_norm.hip", "recurrence.hip", "moe.hip", "token_shift.hip", "wkv.hip",
                                         "delta_rule.hip", "latent_attention.hip", "poly_norm.hip", "bindings_decoder.cpp"),
