@@ -40,36 +40,21 @@ __device__ __forceinline__ float fmax_nan(float a, float b) { return __builtin_e
 // Exact-erf GELU (nanoGPT's nn.GELU()) without the branchy libm erff: with
 // z = |x|/sqrt2, erf(z) = 1 - t*P(t)*exp(-z^2), t = 1/(1 + p z) (Abramowitz &
 // Stegun 7.1.26, |error| <= 1.5e-7), so
-//   gelu(x) = x - q  (x >= 0),   q  (x < 0),   q = 0.5 x t P(t) exp(-x^2/2).
-// Straight-line: 1 v_rcp + 1 v_exp + ~10 FMA/MUL, no divergence in an epilogue.
+//   gelu(x) = max(x, 0) - |x| r,   r = 0.5 t P(t) exp(-x^2/2).
+// Straight-line: v_rcp, v_exp and 11 others, the halves and log2 e in the constants (15 others with
+// x - q and q chosen by the sign; from 64 bits both are 7.1e-8 (rms) and 3.3e-7 (largest) over +-12).  A GEMM's
+// epilogue applies it to up to 128 values a thread, with no product beside it.
 __device__ __forceinline__ float gelu_erf(float x) {
-  const float z = fabsf(x) * 0.70710678118654752f;
-  const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, z, 1.0f));
-  float p = fmaf(1.061405429f, t, -1.453152027f);
-  p = fmaf(p, t, 1.421413741f);
-  p = fmaf(p, t, -0.284496736f);
-  p = fmaf(p, t, 0.254829592f);
-  const float e = __builtin_amdgcn_exp2f(-z * z * 1.44269504088896341f);
-  const float q = 0.5f * x * (p * t) * e;
-  return x >= 0.f ? x - q : q;
+  const float a = fabsf(x), w = a * 0.84932180028801904f;  // sqrt(log2 e / 2)
+  const float t = __builtin_amdgcn_rcpf(fmaf(a, 0.3275911f * 0.70710678118654752f, 1.0f));
+  float p = fmaf(t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
+  p = fmaf(p, t, 0.5f * 1.421413741f);
+  p = fmaf(p, t, 0.5f * -0.284496736f);
+  p = fmaf(p, t, 0.5f * 0.254829592f);
+  const float r = p * t * __builtin_amdgcn_exp2f(-(w * w));
+  return fmaf(-a, r, fmaxf(x, 0.f));
 }
-// Two GELUs at once on packed fp32 math: the polynomial, the squares and the
-// products go through v_pk_fma_f32 / v_pk_mul_f32 (two lanes' worth per
-// instruction), only the reciprocal, the exponential, |x| and the sign select
-// stay per element — a GEMM epilogue applies it to 128 outputs per thread.
-__device__ __forceinline__ f32x2 gelu_erf2(f32x2 x) {
-  const f32x2 z = f32x2{fabsf(x[0]), fabsf(x[1])} * 0.70710678118654752f;
-  const f32x2 d = z * 0.3275911f + 1.0f;
-  const f32x2 t = f32x2{__builtin_amdgcn_rcpf(d[0]), __builtin_amdgcn_rcpf(d[1])};
-  f32x2 p = t * 1.061405429f - 1.453152027f;
-  p = p * t + 1.421413741f;
-  p = p * t - 0.284496736f;
-  p = p * t + 0.254829592f;
-  const f32x2 a = (z * z) * -1.44269504088896341f;
-  const f32x2 e = f32x2{__builtin_amdgcn_exp2f(a[0]), __builtin_amdgcn_exp2f(a[1])};
-  const f32x2 q = (x * 0.5f) * (p * t) * e;
-  return f32x2{x[0] >= 0.f ? x[0] - q[0] : q[0], x[1] >= 0.f ? x[1] - q[1] : q[1]};
-}
+__device__ __forceinline__ f32x2 gelu_erf2(f32x2 x) { return f32x2{gelu_erf(x[0]), gelu_erf(x[1])}; }
 
 // tanh-form GELU: 0.5 x (1 + tanh(u)) = x / (1 + exp(-2 u)), u = sqrt(2 / pi)
 // (x + 0.044715 x^3); one v_exp and one v_rcp (results feed bf16 stores).

@@ -299,6 +299,12 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_256_kernel(
             if (QOUT) bs[nq][j][r] = (bias != nullptr && n + r < N) ? bias[n + r] : 0.f;
           }
         }
+        if constexpr (QOUT) {  // columns past N leave as zeros: here once, not at every value (with gelu_erf's form 2048 x 6400 x 1600 37.8 -> 35.5 us)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            if (n + r >= N) cs[nq][j][r] = bs[nq][j][r] = 0.f;
+          }
+        }
       }
   }
   if constexpr (QOUT) {
@@ -316,13 +322,10 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_256_kernel(
           float am = 0.f;
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
-            const int n = n0 + nq * 128 + wc * 32 + j * 16 + (lane >> 4) * 4;
             f32x4 v = acc[mq][nq][i][j] * cs[nq][j] + bs[nq][j];
-            const f32x2 g0 = gelu_erf2(f32x2{v[0], v[1]}), g1 = gelu_erf2(f32x2{v[2], v[3]});
-            v = f32x4{g0[0], g0[1], g1[0], g1[1]};
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              v[r] = n + r < N ? v[r] : 0.f;
+              v[r] = gelu_erf(v[r]);
               am = fmaxf(am, fabsf(v[r]));
             }
             acc[mq][nq][i][j] = v;

@@ -55,3 +55,31 @@ def test_one_epilogue(tile, kind, M, N, K):
     if kind in ("none", "res"):  # of bf16 storage and fp32 sums
         ref = x.double() @ w.double().t() + (kw["residual"].double() if "residual" in kw else 0)
         assert ((outs[0].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -17 * (x.double().abs() @ w.double().abs().t())).all()
+
+
+@pytest.mark.parametrize("tile", range(5))
+@pytest.mark.parametrize("M,N,K", [(256, 256, 128), (257, 320, 320), (300, 448, 640)])
+def test_one_epilogue_of_e4m3(tile, M, N, K):
+    from distributed_neural_networks_amd.ops import gemm as G
+    from distributed_neural_networks_amd.ops.fp8 import kpad_of, linear_fp8, mx_scale_bytes, quantize_weight
+    g = torch.Generator(device=DEV).manual_seed(tile + M)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
+    x, w, bias, res = r(M, K).bfloat16(), quantize_weight(r(N, K) / math.sqrt(K), DEV), r(N), r(M, N).bfloat16()
+    q, sx = (torch.empty(n, dtype=torch.uint8, device=DEV) for n in (M * kpad_of(K), mx_scale_bytes(M, kpad_of(K))))
+    outs, names = [], []
+    G.lib().gemm_set_mid(tile, 1)
+    try:
+        for ld in (N, N + 4):
+            out = torch.full((M + 1, ld), 7.0, device=DEV, dtype=torch.bfloat16)
+            with profile(activities=[ProfilerActivity.CUDA]) as p:
+                linear_fp8(x, w, bias, 0, res, out[:M, :N], q, None, sx=sx)
+                torch.cuda.synchronize()
+            names.append([e.key for e in p.key_averages() if "gemm_mid_fp8" in e.key])
+            assert (out[M] == 7).all() and (out[:, N:] == 7).all()
+            outs.append(out[:M, :N].clone())
+    finally:
+        G.lib().gemm_set_mid(-1, 1)
+    assert [len(n) for n in names] == [1, 1] and names[0] != names[1]
+    assert torch.equal(*outs)
+    ref = x.double() @ (w.q[:, :K].double() * w.scale.double()[:, None]).t() + bias.double() + res.double()
+    assert ((outs[0].double() - ref).norm() / ref.norm()).item() < 2.0 ** -4  # an activation's e4m3 rounding, at worst
