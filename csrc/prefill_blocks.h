@@ -60,7 +60,7 @@ struct PrefillPass {
 
   int quant_norm(const void* in) {
     what = "layernorm_q8_mx";
-    return dnn_layernorm_q8_mx(in, d, ones, nullptr, q8, kpad(d), sx, rows(), d, kpad(d), eps, norm == 1, st);
+    return dnn_layernorm_q8_mx(in, d, nullptr, nullptr, q8, kpad(d), sx, rows(), d, kpad(d), eps, norm == 1, st);
   }
 
   // out = act(norm(in) W^T + bias), in (rows, d).  fp8: row_scale: one scale a row, else MX; quant: the
