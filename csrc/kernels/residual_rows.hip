@@ -309,6 +309,105 @@ __global__ __launch_bounds__(256) void rows_update_kernel(RowsArgs a) {
   }
 }
 
+// rows_update in bf16 of rows 1024 NC wide with nothing extra: one row a workgroup, no bounds, everything loaded ahead
+// of the first sum, one barrier a sum.  IN: the row comes from a table, is a residual and an output, or is the residual
+// alone (by index).  YN: y is normed.  OUT: what is made of x' beside itself.
+// A row is a trip to memory and two sums, and the launch of a step begins with no instructions in the cache, so the
+// 0.5 to 2.3 KB of a form 4096 wide count against the general kernel's 4.1.  Within a step: 1 to 6 rows 4.2 to 4.8
+// us -> 2.3 to 4, 512 rows 7 -> 5.4 to 6.1; a step's rows of 512 move 14 MB to 20 MB (2 to 3 us).
+enum LeanIn { LEAN_TABLE = 0, LEAN_JOIN = 1, LEAN_ROWS = 2 };
+enum LeanOut { LEAN_X = 0, LEAN_NORM = 1, LEAN_COPY = 2 };
+
+template <int NC, int IN, bool YN, int OUT>
+__global__ __launch_bounds__(256) void rows_lean_kernel(const float* x_in, const bf16_t* y, const int* idx, int rows,
+                                                        const float* y_w, float* x_out, const float* n_w, bf16_t* out,
+                                                        int ldx, int ldy, int ldo, int N, float mult, float eps) {
+  __shared__ float red[8];
+  const int wave = threadIdx.x >> 6, c = threadIdx.x * 4;
+  const size_t m = blockIdx.x;
+  size_t in = m;
+  if constexpr (IN != LEAN_JOIN)
+    if (idx != nullptr) in = (size_t)min(max(idx[m], 0), rows - 1);
+  f32x4 xv[NC], yv[NC], yw[NC], nw[NC];
+  bf16x4 yb[NC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    if constexpr (IN != LEAN_ROWS) yb[i] = *reinterpret_cast<const bf16x4*>(y + in * ldy + c + 1024 * i);
+    if constexpr (IN != LEAN_TABLE) xv[i] = ld4(x_in + in * ldx + c + 1024 * i);
+    if constexpr (YN) yw[i] = ld4(y_w + c + 1024 * i);
+    if constexpr (OUT == LEAN_NORM) nw[i] = ld4(n_w + c + 1024 * i);
+  }
+#pragma unroll
+  for (int i = 0; i < NC; ++i)
+    if constexpr (IN != LEAN_ROWS) yv[i] = f32x4{bf2f_s(yb[i][0]), bf2f_s(yb[i][1]), bf2f_s(yb[i][2]), bf2f_s(yb[i][3])};
+  if constexpr (YN) {
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s = fmaf(yv[i][j], yv[i][j], s);
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) red[wave] = s;
+    __syncthreads();
+    const float r = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)N + eps);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) yv[i] = yv[i] * r * yw[i];
+  }
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if constexpr (IN != LEAN_ROWS) xv[i][j] = fmaf(mult, yv[i][j], IN == LEAN_JOIN ? xv[i][j] : 0.f);
+      if constexpr (OUT == LEAN_NORM) s = fmaf(xv[i][j], xv[i][j], s);
+    }
+    if constexpr (IN != LEAN_ROWS) st4(x_out + m * ldx + c + 1024 * i, xv[i]);
+    if constexpr (OUT == LEAN_COPY) st4(out + m * ldo + c + 1024 * i, xv[i]);
+  }
+  if constexpr (OUT == LEAN_NORM) {
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) red[4 + wave] = s;
+    __syncthreads();
+    const float r = 1.0f / sqrtf((red[4] + red[5] + red[6] + red[7]) / (float)N + eps);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) st4(out + m * ldo + c + 1024 * i, xv[i] * r * nw[i]);
+  }
+}
+
+// 1: not one of these forms.
+template <int NC>
+static int lean_launch(const RowsArgs& a, hipStream_t st) {
+#define LEAN(IN, YN, OUT)                                                                                               \
+  {                                                                                                                     \
+    hipLaunchKernelGGL((rows_lean_kernel<NC, IN, YN, OUT>), dim3(a.M), dim3(256), 0, st, a.x_in, (const bf16_t*)a.y,    \
+                       IN == LEAN_ROWS ? a.xidx : a.yidx, IN == LEAN_ROWS ? a.xrows : a.yrows, a.y_w, a.x_out, a.n_w,   \
+                       (bf16_t*)(OUT == LEAN_COPY ? a.copy : a.h), a.ldx, a.ldy, OUT == LEAN_COPY ? a.ldcopy : a.ldh,   \
+                       a.N, a.mult, a.eps);                                                                             \
+    return (int)hipGetLastError();                                                                                      \
+  }
+  const bool norm = a.n_w != nullptr, copy = a.copy != nullptr;
+  if (norm && copy) return 1;
+  if (a.y == nullptr) {
+    if (a.x_in == nullptr || a.x_out != nullptr || !norm) return 1;
+    LEAN(LEAN_ROWS, false, LEAN_NORM)
+  }
+  if (a.x_out == nullptr) return 1;
+  if (a.x_in == nullptr) {
+    if (a.y_w != nullptr || !norm) return 1;
+    LEAN(LEAN_TABLE, false, LEAN_NORM)
+  }
+  if (a.yidx != nullptr || a.xidx != nullptr) return 1;
+  if (a.y_w == nullptr) {
+    if (norm) LEAN(LEAN_JOIN, false, LEAN_NORM)
+    if (copy) LEAN(LEAN_JOIN, false, LEAN_COPY)
+    LEAN(LEAN_JOIN, false, LEAN_X)
+  }
+  if (norm) LEAN(LEAN_JOIN, true, LEAN_NORM)
+  if (copy) LEAN(LEAN_JOIN, true, LEAN_COPY)
+  LEAN(LEAN_JOIN, true, LEAN_X)
+#undef LEAN
+}
+
 constexpr int ROWS_GRID = 2048;  // workgroups of a launch of many rows: they loop, eight to a CU
 
 template <typename YT, typename OT, int PART>
@@ -392,6 +491,16 @@ extern "C" int dnn_rows_update(const RowsArgs* a, int y_f32, int out_f32, hipStr
     return more ? rows_launch<YT, OT, ROWS_MORE>(*a, st) : rows_launch<YT, OT, ROWS_PLAIN>(*a, st); \
   }
   if (y_f32 && out_f32) ROWS_PART(float, float)
+  // Up to as many rows as workgroups are in flight at once: past that the general kernel keeps the norms' weights
+  // over a workgroup's rows.
+  if (!y_f32 && !out_f32 && !more && a->y2 == nullptr && a->ys == nullptr && a->freq == nullptr && a->sh_mu == nullptr &&
+      a->M <= ROWS_GRID) {
+    const int rc = a->NP == 1024   ? lean_launch<1>(*a, st)
+                   : a->NP == 2048 ? lean_launch<2>(*a, st)
+                   : a->NP == 4096 ? lean_launch<4>(*a, st)
+                                   : 1;
+    if (rc <= 0) return rc;
+  }
   if (!y_f32 && !out_f32) ROWS_PART(bf16_t, bf16_t)
 #undef ROWS_PART
   if (!y_f32 || a->y2 != nullptr || a->ys != nullptr || a->freq != nullptr || a->sh_mu != nullptr || more) return -1;
