@@ -4,9 +4,10 @@
 // gemm_f32).  W has few rows (the side dimension, padded to 64), so a plain
 // GEMM grid would leave most CUs idle:
 //
-//   few rows    a workgroup takes 16 columns of 16 rows; eight waves split
+//   few rows    a workgroup takes 16 columns of 16 or 32 rows; eight waves split
 //               K (one round trip for K <= 4096) over W in fragment order
-//               (ops/gemm.py shuffle_weight) and reduce through LDS
+//               (ops/gemm.py shuffle_weight) and reduce through LDS; K of 1024, 2048
+//               and 4096 has kernels of its own
 //   more rows   64 x 64 tiles on the loop of gemm_mid.h
 #include "common.h"
 #include "gemm_mid.h"
@@ -76,6 +77,73 @@ __global__ __launch_bounds__(64 * (TG_WAVES + 1)) void token_gate_skinny_kernel(
   __syncthreads();
 }
 
+// grid (rows / 16 R, columns / 16): eight waves of CH chunks are K, in H parts, everything of a wave in flight at once;
+// wave r finishes the 16 rows r.  A wave reads its slice of every row whole (1 KB of K = 4096) and turns it to fragments
+// in LDS of its own: read as fragments, 16 pieces of 64 bytes of rows 8 KB apart, 16 rows took 6.3 us of it against 4.4
+// (one row, all lanes at one line: 3.6).  In XCDs' turns of rows, so an L2 holds 64 of 512 rows and W.
+template <int CH, int R, int H>
+struct TgLean {
+  static constexpr int CP = CH / H, STRIDE = CP * 64 + 16;  // chunks a part, bytes of a staged row: 16 rows meet all banks
+  static constexpr int LPR = CP * 4, RPI = 64 / LPR, NX = R * CP;  // lanes a row, rows a load, loads a part
+  static constexpr int WAVE = 16 * R * STRIDE, LDS = TG_WAVES * WAVE;
+};
+
+template <int CH, int R, int H>
+__global__ __launch_bounds__(64 * TG_WAVES) void token_gate_lean_kernel(const bf16_t* __restrict__ x, int ldx,
+                                                                        const uint8_t* __restrict__ ws, TokenGate t) {
+  using L = TgLean<CH, R, H>;
+  extern __shared__ __attribute__((aligned(16))) char tg_rows[];
+  __shared__ f32x4 red[TG_WAVES][R][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int mg = blockIdx.x * (16 * R), m0 = mg + (lane & 15), c4 = blockIdx.y * 16 + (lane >> 4) * 4;
+  float e[4];
+  if (wave < R) token_gate_row(t, m0 + wave * 16, c4, e);
+  const uint8_t* wp = ws + ((size_t)blockIdx.y * TG_WAVES + wave) * (CH * 1024) + lane * 16;
+  bf16x8 w[CH], xr[H][L::NX];
+  const int xl = wave * (CH * 32) + lane % L::LPR * 8, xrow = L::LPR == 64 ? 0 : lane / L::LPR;
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+#pragma unroll
+    for (int i = 0; i < L::NX; ++i)
+      xr[h][i] = *reinterpret_cast<const bf16x8*>(x + (size_t)min(mg + i * L::RPI + xrow, t.M - 1) * ldx + xl + h * (L::CP * 32));
+#pragma unroll
+    for (int u = 0; u < L::CP; ++u) w[h * L::CP + u] = *reinterpret_cast<const bf16x8*>(wp + (h * L::CP + u) * 1024);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  f32x4 acc[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  char* mine = tg_rows + wave * L::WAVE;
+  char* to = mine + xrow * L::STRIDE + lane % L::LPR * 16;
+  const char* from = mine + (lane & 15) * L::STRIDE + (lane >> 4) * 16;
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+#pragma unroll
+    for (int i = 0; i < L::NX; ++i) *reinterpret_cast<bf16x8*>(to + i * (L::RPI * L::STRIDE)) = xr[h][i];
+#pragma unroll
+    for (int u = 0; u < L::CP; ++u)
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            w[h * L::CP + u], *reinterpret_cast<const bf16x8*>(from + r * (16 * L::STRIDE) + u * 64), acc[r], 0, 0, 0);
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) red[wave][r][lane] = acc[r];
+  __syncthreads();
+  if (wave >= R) return;
+  f32x4 z = red[0][wave][lane];
+#pragma unroll
+  for (int v = 1; v < TG_WAVES; ++v) z += red[v][wave][lane];
+  token_gate_store(t, z, m0 + wave * 16, c4, e);
+}
+
+template <int CH, int R, int H>
+static int token_gate_lean(const TokenGate& t, const void* x, int ldx, const void* ws, int np, hipStream_t st) {
+  hipLaunchKernelGGL((token_gate_lean_kernel<CH, R, H>), dim3((t.M + 16 * R - 1) / (16 * R), np / 16), dim3(64 * TG_WAVES),
+                     (TgLean<CH, R, H>::LDS), st, (const bf16_t*)x, ldx, (const uint8_t*)ws, t);
+  return (int)hipGetLastError();
+}
+
 template <class T>
 __global__ __launch_bounds__(T::NW * 64, 2) void token_gate_tile_kernel(const bf16_t* __restrict__ x, int ldx,
                                                                         const bf16_t* __restrict__ w, int ldw, int np, int K,
@@ -130,7 +198,18 @@ extern "C" int dnn_token_gate(const void* x, int ldx, const void* w, int ldw, co
   if (ldx % 8 != 0 || ldw % 8 != 0 || ldx < K || ldw < K || ldg % 4 != 0 || ldg < np || wsh == nullptr) return -1;
   if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)wsh) & 15) != 0 || ((uintptr_t)g & 7) != 0) return -1;
   const TokenGate t{(const bf16_t*)table, tok, (bf16_t*)g, ldt, off, V, ldg, M, n};
-  // Few rows: rounds of 256 workgroups of 16 x 16 outputs, 6.4 us each for K up to 4096;
+  // A K that eight waves hold: up to one round of 16 x 16 outputs a workgroup, then up to two of 32 x 16 (a third is
+  // behind the tiles).  us, 16 x 16 : 32 x 16 : tiles, 256 columns: K 4096, 256 rows 4.7 : 6.2 : 7.0, 512 rows 8.0 :
+  // 7.1 : 13.3, 1024 rows 15 : 12.2 : 15; K 1024, 512 rows 3.7 : 3.4 : 7.3, 1024 rows 5.9 : 5.4 : 7.3; 512 columns, 768
+  // rows: K 2048 11.2 : 10.6 : 9.8, K 4096 22 : 19 : 16.
+  const int groups = (M + 15) / 16 * (np / 16), pairs = (M + 31) / 32 * (np / 16);
+  if (pairs <= 512 && (K == 4096 || K == 2048 || K == 1024)) {
+    const bool one = groups <= 256;
+    if (K == 4096) return one ? token_gate_lean<16, 1, 1>(t, x, ldx, wsh, np, st) : token_gate_lean<16, 2, 2>(t, x, ldx, wsh, np, st);
+    if (K == 2048) return one ? token_gate_lean<8, 1, 1>(t, x, ldx, wsh, np, st) : token_gate_lean<8, 2, 1>(t, x, ldx, wsh, np, st);
+    return one ? token_gate_lean<4, 1, 1>(t, x, ldx, wsh, np, st) : token_gate_lean<4, 2, 1>(t, x, ldx, wsh, np, st);
+  }
+  // Any K, few rows: rounds of 256 workgroups of 16 x 16 outputs, 6.4 us each for K up to 4096;
   // tiles 0.166 us a K-tile of 64 beside 4.9.  us, rounds : tiles: 100 x 64 x 512 7.1 : 6.2, 100 x
   // 256 x 1024 7.1 : 7.5, 512 x 256 x 4096 13.6 : 15.4, 1024 x 256 x 4096 26.5 : 15.7 (30 with the
   // six-stage loop of its own that read a tile's fragments between two barriers)
