@@ -10,9 +10,12 @@
 // nothing is shared before the sums meet), one barrier, and the waves that finish a tile
 // have its epilogue's operands by then: 1.2 to 5.8 KB, of which the e4m3 c_fc's was 28.
 //
-// us a launch in the step, GPT-2 (bf16) of 64 rows 2304 x 768 7.4 -> 4.6, 3072 x 768 7.0 -> 5.1, 768 x 768 5.4
-// -> 4.8, 768 x 3072 7.1 -> 6.1; XL (e4m3) of 64 rows 4800 x 1600 10.7 -> 7.1, 6400 x 1600 11.2 -> 7.6,
-// 1600 x 1600 5.8 -> 5.0, 1600 x 6400 11.6 -> 10.5.  Batches in flight, waves and their chunks matter
+// A wave reads its slice of every row whole and turns it to fragments in LDS of its own.  Read as fragments, a load is 16
+// pieces of 64 bytes of 16 rows, half a line each: GPT-2's step of 64 rows is 501 us so, 482 through LDS, XL's 326 and 310.
+//
+// us a launch in the step, GPT-2 (bf16) of 64 rows 2304 x 768 7.4 -> 4.6, 3072 x 768 7.0 -> 5.0, 768 x 768 5.4
+// -> 4.8, 768 x 3072 7.1 -> 4.9; XL (e4m3) of 64 rows 4800 x 1600 10.7 -> 6.3, 6400 x 1600 11.2 -> 6.6,
+// 1600 x 1600 5.8 -> 4.9, 1600 x 6400 11.6 -> 7.8.  Batches in flight, waves and their chunks matter
 // little (within 1 % of the step from one batch to all of K, 4 to 8 waves); tiles do: lean_gemm.
 #include <utility>
 
@@ -26,6 +29,8 @@ struct Lean {
   static constexpr int LPR = NW * 64 / ROWS;  // threads a row for the merge of its statistics
   static constexpr int TPR = LPR >= 64 ? 64 : LPR >= 32 ? 32 : LPR >= 16 ? 16 : LPR >= 8 ? 8 : 4;
   static constexpr int SPT = (K / 16 + TPR - 1) / TPR;
+  // a batch of a wave's rows on its way through LDS: pieces of 16 bytes a row, and an odd number of them between rows
+  static constexpr int PB = CB * (W8 ? 8 : 4), STRIDE = (PB + 1) * 16, NX = MT * PB / 4, WAVE = ROWS * STRIDE, LDS = NW * WAVE;
 };
 
 template <int NW, int CB, int NB, int D, int MT, int NT, bool W8, int NORM, int ACT, bool RES>
@@ -33,6 +38,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_lean_kernel(LeanArgs p) {
   using L = Lean<NW, CB, NB, D, MT, NT, W8, NORM, ACT, RES>;
   constexpr int AU = W8 ? 2 : 1, ACH = 64 * AU, TS = MT * NT, CH = CB * NB, TW = (TS + NW - 1) / NW;
   static_assert(D <= NB, "batches in flight");
+  extern __shared__ __attribute__((aligned(16))) char lean_rows[];
   __shared__ f32x4 red[NW][TS][64];
   __shared__ float2 st[NORM == NORM_LN ? L::ROWS : 1];
   __shared__ float ss[NORM == NORM_RMS ? NW : 1][NORM == NORM_RMS ? L::ROWS : 1];
@@ -48,24 +54,21 @@ __global__ __launch_bounds__(NW * 64) void gemm_lean_kernel(LeanArgs p) {
 #pragma unroll
     for (int i = 0; i < L::SPT; ++i) rp[i] = q[min(sub + i * L::TPR, L::K / 16 - 1)];
   }
-  i32x4 av[D][MT][CB * AU], wv[D][NT][CB];
-  const uint8_t* ap[MT];
+  i32x4 xr[D][L::NX], wv[D][NT][CB];
+  const uint8_t* xp[L::NX];
   const uint8_t* wp[NT];
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
-    ap[t] = p.A + (size_t)min(m0 + t * 16 + r16, p.M - 1) * p.lda_b + wave * (CH * ACH) + c4 * (16 * AU);
+  for (int i = 0; i < L::NX; ++i) {
+    const int q = lane + i * 64;
+    xp[i] = p.A + (size_t)min(m0 + q / L::PB, p.M - 1) * p.lda_b + wave * (CH * ACH) + q % L::PB * 16;
+  }
 #pragma unroll
   for (int j = 0; j < NT; ++j)
     wp[j] = p.W + ((size_t)min(n0 / 16 + j, p.N / 16 - 1) * (NW * CH) + wave * CH) * 1024 + lane * 16;
   auto load = [&](auto bc) __attribute__((always_inline)) {
     constexpr int b = decltype(bc)::value, d = b % D;
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-      for (int u = 0; u < CB; ++u)
-#pragma unroll
-        for (int h = 0; h < AU; ++h)
-          av[d][t][u * AU + h] = *reinterpret_cast<const i32x4*>(ap[t] + (b * CB + u) * ACH + h * 16);
+    for (int i = 0; i < L::NX; ++i) xr[d][i] = *reinterpret_cast<const i32x4*>(xp[i] + b * (CB * ACH));
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
@@ -101,10 +104,23 @@ __global__ __launch_bounds__(NW * 64) void gemm_lean_kernel(LeanArgs p) {
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
+  char* mine = lean_rows + wave * L::WAVE;
+  const char* from = mine + r16 * L::STRIDE + c4 * (16 * AU);
   auto comp = [&](auto bc) __attribute__((always_inline)) {
     constexpr int d = decltype(bc)::value % D;
 #pragma unroll
-    for (int u = 0; u < CB; ++u)
+    for (int i = 0; i < L::NX; ++i) {
+      const int q = lane + i * 64;
+      *reinterpret_cast<i32x4*>(mine + q / L::PB * L::STRIDE + q % L::PB * 16) = xr[d][i];
+    }
+#pragma unroll
+    for (int u = 0; u < CB; ++u) {
+      bf16x8 a[MT][AU];
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int h = 0; h < AU; ++h)
+          a[t][h] = *reinterpret_cast<const bf16x8*>(from + t * (16 * L::STRIDE) + u * ACH + h * 16);
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
         bf16x8 w[AU];
@@ -114,19 +130,21 @@ __global__ __launch_bounds__(NW * 64) void gemm_lean_kernel(LeanArgs p) {
         for (int t = 0; t < MT; ++t)
 #pragma unroll
           for (int h = 0; h < AU; ++h)
-            acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[h], __builtin_bit_cast(bf16x8, av[d][t][u * AU + h]),
-                                                                acc[j][t], 0, 0, 0);
+            acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[h], a[t][h], acc[j][t], 0, 0, 0);
       }
-    if constexpr (NORM == NORM_RMS) {
+      if constexpr (NORM == NORM_RMS) {
 #pragma unroll
-      for (int t = 0; t < MT; ++t)
+        for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int u = 0; u < CB * AU; ++u)
+          for (int h = 0; h < AU; ++h) {
+            const i32x4 v4 = __builtin_bit_cast(i32x4, a[t][h]);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const bf16x2v v = __builtin_bit_cast(bf16x2v, (uint32_t)av[d][t][u][i]);
-            sq[t] = __builtin_amdgcn_fdot2_f32_bf16(v, v, sq[t], false);
+            for (int i = 0; i < 4; ++i) {
+              const bf16x2v v = __builtin_bit_cast(bf16x2v, (uint32_t)v4[i]);
+              sq[t] = __builtin_amdgcn_fdot2_f32_bf16(v, v, sq[t], false);
+            }
           }
+      }
     }
   };
   [&]<int... B>(std::integer_sequence<int, B...>) __attribute__((always_inline)) {
@@ -195,7 +213,8 @@ template <int NW, int CB, int NB, int D, int MT, int NT, bool W8, int NORM, int 
 static void lean_launch(const LeanArgs& p, hipStream_t st) {
   const int cols = (p.N / 16 + NT - 1) / NT;
   hipLaunchKernelGGL((gemm_lean_kernel<NW, CB, NB, D, MT, NT, W8, NORM, ACT, RES>),
-                     dim3((cols + 7) / 8 * 8, (p.M + 16 * MT - 1) / (16 * MT)), dim3(NW * 64), 0, st, p);
+                     dim3((cols + 7) / 8 * 8, (p.M + 16 * MT - 1) / (16 * MT)), dim3(NW * 64),
+                     (Lean<NW, CB, NB, D, MT, NT, W8, NORM, ACT, RES>::LDS), st, p);
 }
 
 // False, nothing done, where the shape is not one of those laid out.
@@ -206,15 +225,11 @@ static bool lean_gemm(const LeanArgs& p, int nch, hipStream_t st) {
                 !(NORM == NORM_RMS && ACT == ACT_NONE && !W8)) {
     return false;
   } else {
-    // The tiles, from whole steps (us; GPT-2 behind 100 tokens, XL behind 64, Llama-3 of 4 layers behind 100; before:
-    // gemm_skinny, gemm_oneshot):
-    //   GPT-2 QKV, c_fc        8 rows 302: 1 x 1 tiles 270, 1 x 2 272, 2 x 2 279; 32 rows 406: 358, 347, 364; 64 rows 422:
-    //                          409, 397, 389
-    //   its O, c_proj          1 x 1 at every number of rows (24 rows 389: 376, 372; 64 rows 422: 415, 403)
-    //   XL e4m3 QKV, c_fc      8 rows 183: 1 x 2 tiles 164, 1 x 4 166; 32 rows 286: 246, 230, 2 x 4 253; 64 rows 278: 300, 272, 267
-    //   its O, c_proj          32 rows 286: 1 x 1 275, 266, 1 x 2 279, 285; 64 rows 278: 289, 308; 275, 274
-    //   Llama-3 QKV, O         16 rows 410: 393, 400 (1 x 2, 1 x 1); from 17 rows the step is up to 3 % slower with tiles of
-    //                          32 rows: 16 rows of a load lie 8 KB apart, on one channel of the L2
+    // The tiles, from whole steps (us; GPT-2 behind 100 tokens, XL behind 64, Llama-3 of 4 layers behind 100):
+    //   GPT-2 QKV, c_fc        16 rows 1 x 1 tiles 251, 1 x 2 259, 2 x 2 266; 32 rows 311, 307, 321; 64 rows 358, 352, 351
+    //   its O, c_proj          1 x 1 at every number of rows (64 rows, 1 x 2 and 2 x 1: 354; c_proj 367)
+    //   XL e4m3 QKV, c_fc      8 rows 1 x 2 tiles 138, 1 x 4 142; 24 rows 181, 159; 64 rows 266, 232, 2 x 4 230
+    //   its O, c_proj          48 rows 1 x 1 213, 212, 1 x 2 211, 211; 8 rows 138, 138; 139, 146
     // Two rows or fewer of GPT-2's widths: decode_row.hip.  Other widths have not been laid out or measured.
     auto al = [](const void* x, int a) { return ((uintptr_t)x & (a - 1)) == 0; };
     if (p.W == nullptr || p.M < 1 || p.M > 64 || p.N % 16 != 0 || p.N > (RES ? 4096 : 8192) || (p.R != nullptr) != RES ||
@@ -234,14 +249,14 @@ static bool lean_gemm(const LeanArgs& p, int nch, hipStream_t st) {
       LEAN(8, 4, 4, 2, 1, 2);
     } else if constexpr (!W8) {
       if (nch == 24) LEAN(4, 6, 1, 1, 1, 1);
-      else if (nch == 96) LEAN(4, 6, 4, 3, 1, 1);
+      else if (nch == 96) LEAN(4, 6, 4, 2, 1, 1);
       else if (nch == 128 && M <= 16) LEAN(8, 4, 4, 4, 1, 1);
       else return false;
     } else if constexpr (NORM == NORM_LN) {
       if (nch != 25) return false;
       if (M <= 16) LEAN(5, 5, 1, 1, 1, 2);
       else if (M <= 48) LEAN(5, 1, 5, 2, 1, 4);
-      else LEAN(5, 1, 5, 1, 2, 4);
+      else LEAN(5, 1, 5, 2, 2, 4);
     } else {
       if (nch == 25) {
         if (M <= 32) LEAN(5, 5, 1, 1, 1, 1);
