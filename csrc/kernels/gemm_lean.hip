@@ -33,7 +33,8 @@ struct Lean {
   static constexpr int PB = CB * (W8 ? 8 : 4), STRIDE = (PB + 1) * 16, NX = MT * PB / 4, WAVE = ROWS * STRIDE, LDS = NW * WAVE;
 };
 
-template <int NW, int CB, int NB, int D, int MT, int NT, bool W8, int NORM, int ACT, bool RES>
+// ST: W goes past the L2's order of use (bytes read once; us a step of Llama-3's 32 rows, QKV with and without 399 and 414).
+template <int NW, int CB, int NB, int D, int MT, int NT, bool W8, int NORM, int ACT, bool RES, bool ST>
 __global__ __launch_bounds__(NW * 64) void gemm_lean_kernel(LeanArgs p) {
   using L = Lean<NW, CB, NB, D, MT, NT, W8, NORM, ACT, RES>;
   constexpr int AU = W8 ? 2 : 1, ACH = 64 * AU, TS = MT * NT, CH = CB * NB, TW = (TS + NW - 1) / NW;
@@ -42,8 +43,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_lean_kernel(LeanArgs p) {
   __shared__ f32x4 red[NW][TS][64];
   __shared__ float2 st[NORM == NORM_LN ? L::ROWS : 1];
   __shared__ float ss[NORM == NORM_RMS ? NW : 1][NORM == NORM_RMS ? L::ROWS : 1];
-  const int n0 = blockIdx.x * (16 * NT), m0 = blockIdx.y * (16 * MT);
-  if (n0 >= p.N) return;  // the grid is a multiple of 8 columns: the row tiles of a column tile on one XCD
+  // the row tiles of a column tile follow each other on one XCD
+  const int n0 = (blockIdx.z * 8 + blockIdx.x) * (16 * NT), m0 = blockIdx.y * (16 * MT);
+  if (n0 >= p.N) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, c4 = lane >> 4;
   float2 rp[L::SPT], rp0;
@@ -72,7 +74,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_lean_kernel(LeanArgs p) {
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int u = 0; u < CB; ++u) wv[d][j][u] = *reinterpret_cast<const i32x4*>(wp[j] + (b * CB + u) * 1024);
+      for (int u = 0; u < CB; ++u) {
+        const i32x4* q = reinterpret_cast<const i32x4*>(wp[j] + (b * CB + u) * 1024);
+        wv[d][j][u] = ST ? __builtin_nontemporal_load(q) : *q;
+      }
   };
   [&]<int... B>(std::integer_sequence<int, B...>) __attribute__((always_inline)) {
     (load(std::integral_constant<int, B>{}), ...);
@@ -200,6 +205,17 @@ __global__ __launch_bounds__(NW * 64) void gemm_lean_kernel(LeanArgs p) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) y[e] += bf2f_s(rr[i][e]);
     }
+    if constexpr (is_glu(ACT)) {  // 8 gate columns, then their 8 up columns
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(y[e]), __float_as_uint(y[e]), false, false);
+        v[e] = glu_gate<ACT>(__uint_as_float(h[0])) * __uint_as_float(h[1]);
+      }
+      if (lane < 32 && m[i] < p.M)
+        *reinterpret_cast<uint2*>(p.C + (size_t)m[i] * p.ldc + nt / 2 + c4 * 4) = make_uint2(pack2bf(v[0], v[1]), pack2bf(v[2], v[3]));
+      continue;
+    }
     const uint2 o = make_uint2(pack2bf(y[0], y[1]), pack2bf(y[2], y[3]));
     if (m[i] < p.M) *reinterpret_cast<uint2*>(p.C + (size_t)m[i] * p.ldc + n[i]) = o;
     if (RES && p.rs_out != nullptr)
@@ -209,11 +225,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_lean_kernel(LeanArgs p) {
   }
 }
 
-template <int NW, int CB, int NB, int D, int MT, int NT, bool W8, int NORM, int ACT, bool RES>
+template <int NW, int CB, int NB, int D, int MT, int NT, bool W8, int NORM, int ACT, bool RES, bool ST = false>
 static void lean_launch(const LeanArgs& p, hipStream_t st) {
   const int cols = (p.N / 16 + NT - 1) / NT;
-  hipLaunchKernelGGL((gemm_lean_kernel<NW, CB, NB, D, MT, NT, W8, NORM, ACT, RES>),
-                     dim3((cols + 7) / 8 * 8, (p.M + 16 * MT - 1) / (16 * MT)), dim3(NW * 64),
+  hipLaunchKernelGGL((gemm_lean_kernel<NW, CB, NB, D, MT, NT, W8, NORM, ACT, RES, ST>),
+                     dim3(8, (p.M + 16 * MT - 1) / (16 * MT), (cols + 7) / 8), dim3(NW * 64),
                      (Lean<NW, CB, NB, D, MT, NT, W8, NORM, ACT, RES>::LDS), st, p);
 }
 
@@ -222,7 +238,7 @@ template <int ACT, int NORM, bool W8>
 static bool lean_gemm(const LeanArgs& p, int nch, hipStream_t st) {
   constexpr bool RES = NORM == NORM_NONE;
   if constexpr (!(NORM == NORM_LN && (ACT == ACT_NONE || ACT == ACT_GELU)) && !(RES && ACT == ACT_NONE) &&
-                !(NORM == NORM_RMS && ACT == ACT_NONE && !W8)) {
+                !(NORM == NORM_RMS && (ACT == ACT_NONE || ACT == ACT_SILU_MUL) && !W8)) {
     return false;
   } else {
     // The tiles, from whole steps (us; GPT-2 behind 100 tokens, XL behind 64, Llama-3 of 4 layers behind 100):
@@ -230,28 +246,41 @@ static bool lean_gemm(const LeanArgs& p, int nch, hipStream_t st) {
     //   its O, c_proj          1 x 1 at every number of rows (64 rows, 1 x 2 and 2 x 1: 354; c_proj 367)
     //   XL e4m3 QKV, c_fc      8 rows 1 x 2 tiles 138, 1 x 4 142; 24 rows 181, 159; 64 rows 266, 232, 2 x 4 230
     //   its O, c_proj          48 rows 1 x 1 213, 212, 1 x 2 211, 211; 8 rows 138, 138; 139, 146
+    //   Llama-3 QKV            16 rows 1 x 2 tiles 375, 1 x 3 378, 2 x 3 388; 32 rows 416, 398, 407, 2 x 2 399; 64 rows 514,
+    //                          502, 481, 504 (before: 383, 414, 541)
+    //   its O                  32 rows 1 x 1 424, 2 x 1 406; 64 rows 550, on 8 waves 523, on 4 520
+    //   its gate | up          8 rows 1 x 1 343 (before: 335), 16 rows 371 (383), 1 x 2 381; 32 rows 2 x 2 429 (gemm_stream 414)
+    //   its down               2 x 1 32 rows 419, 64 rows 603, 4 x 1 583 (gemm_stream 414, 541)
     // Two rows or fewer of GPT-2's widths: decode_row.hip.  Other widths have not been laid out or measured.
     auto al = [](const void* x, int a) { return ((uintptr_t)x & (a - 1)) == 0; };
-    if (p.W == nullptr || p.M < 1 || p.M > 64 || p.N % 16 != 0 || p.N > (RES ? 4096 : 8192) || (p.R != nullptr) != RES ||
+    if (p.W == nullptr || p.M < 1 || p.M > 64 || p.N % 16 != 0 || p.N > (RES ? 4096 : is_glu(ACT) ? 65536 : 8192) || (is_glu(ACT) && p.bias != nullptr) || (p.R != nullptr) != RES ||
         (!RES && p.rs_out != nullptr) || p.lda_b % 16 != 0 || p.ldc % 4 != 0 || !al(p.A, 16) || !al(p.C, 8) ||
         !al(p.bias, 16) || !al(p.colsum, 16) || !al(p.sw, 16) || (RES && (p.ldr % 4 != 0 || !al(p.R, 8))) ||
         (NORM == NORM_LN && (p.rs_in == nullptr || p.colsum == nullptr)))
       return false;
 #define LEAN(NWV, CBV, NBV, DV, MTV, NTV) lean_launch<NWV, CBV, NBV, DV, MTV, NTV, W8, NORM, ACT, RES>(p, st)
+#define LEAN_ONCE(NWV, CBV, NBV, DV, MTV, NTV) lean_launch<NWV, CBV, NBV, DV, MTV, NTV, W8, NORM, ACT, RES, true>(p, st)
     const int M = p.M;
     if constexpr (!W8 && NORM == NORM_LN) {
       if (nch != 24) return false;
       if (M <= 16) LEAN(4, 6, 1, 1, 1, 1);
       else if (M <= 48) LEAN(4, 6, 1, 1, 1, 2);
       else LEAN(4, 6, 1, 1, 2, 2);
+    } else if constexpr (!W8 && NORM == NORM_RMS && is_glu(ACT)) {
+      if (nch != 128 || M <= 8 || M > 16) return false;
+      LEAN_ONCE(4, 8, 4, 2, 1, 1);
     } else if constexpr (!W8 && NORM == NORM_RMS) {
-      if (nch != 128 || M > 16) return false;
-      LEAN(8, 4, 4, 2, 1, 2);
+      if (nch != 128) return false;
+      if (M <= 16) LEAN_ONCE(8, 4, 4, 2, 1, 2);
+      else if (M <= 32) LEAN_ONCE(8, 4, 4, 2, 1, 3);
+      else LEAN_ONCE(8, 4, 4, 2, 2, 3);
     } else if constexpr (!W8) {
       if (nch == 24) LEAN(4, 6, 1, 1, 1, 1);
       else if (nch == 96) LEAN(4, 6, 4, 2, 1, 1);
-      else if (nch == 128 && M <= 16) LEAN(8, 4, 4, 4, 1, 1);
-      else return false;
+      else if (nch != 128) return false;
+      else if (M <= 16) LEAN_ONCE(8, 4, 4, 4, 1, 1);
+      else if (M <= 32) LEAN(8, 4, 4, 3, 2, 1);
+      else LEAN_ONCE(4, 8, 4, 2, 2, 1);
     } else if constexpr (NORM == NORM_LN) {
       if (nch != 25) return false;
       if (M <= 16) LEAN(5, 5, 1, 1, 1, 2);
@@ -269,6 +298,7 @@ static bool lean_gemm(const LeanArgs& p, int nch, hipStream_t st) {
       }
     }
 #undef LEAN
+#undef LEAN_ONCE
     return true;
   }
 }
@@ -276,7 +306,7 @@ static bool lean_gemm(const LeanArgs& p, int nch, hipStream_t st) {
 bool dnn_gemm_lean(const LeanArgs& p, int nch, int act, int norm, bool w8, hipStream_t st) {
 #define LG(A, N)                                                                                  \
   if (act == A && norm == N) return w8 ? lean_gemm<A, N, true>(p, nch, st) : lean_gemm<A, N, false>(p, nch, st);
-  LG(ACT_NONE, NORM_LN) LG(ACT_GELU, NORM_LN) LG(ACT_NONE, NORM_NONE) LG(ACT_NONE, NORM_RMS)
+  LG(ACT_NONE, NORM_LN) LG(ACT_GELU, NORM_LN) LG(ACT_NONE, NORM_NONE) LG(ACT_NONE, NORM_RMS) LG(ACT_SILU_MUL, NORM_RMS)
 #undef LG
   return false;
 }

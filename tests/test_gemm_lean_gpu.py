@@ -60,8 +60,6 @@ def test_residual_projection(M, K, N, w8):
     """In place on the residual, with the statistics of the stored rows."""
     from distributed_neural_networks_amd.ops.fp8 import linear_w8, quantize_weight
     from distributed_neural_networks_amd.ops.gemm import attach_shuffled, linear, rowstats_buffer, rowstats_written
-    if K == 4096 and M > 16:
-        pytest.skip("from 17 rows the general kernels")
     g = torch.Generator(device=DEV).manual_seed(M + K)
     r = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
     x, h0, bias, W = r(M, K).bfloat16(), r(M + 1, N).bfloat16(), (None if K == 4096 else r(N)), r(N, K) * 0.02
@@ -83,25 +81,32 @@ def test_residual_projection(M, K, N, w8):
     assert torch.allclose(rs.view(M, -1, 2)[:, :N // 16, 1], (t - t.mean(-1, keepdim=True)).square().sum(-1), rtol=1e-5, atol=1e-5)
 
 
-@pytest.mark.parametrize("M", [1, 9, 16])
-def test_rms_projection(M):
+@pytest.mark.parametrize("M,N,act", [(m, n, 0) for m in (1, 9, 16, 17, 31, 32, 33, 48, 49, 64) for n in (6144, 80)]
+                         + [(9, 28672, 3), (16, 28672, 3), (13, 48, 3)])
+def test_rms_projection(M, N, act):
     from distributed_neural_networks_amd.ops.gemm import attach_shuffled, fold_norm, linear_norm
-    K, N = 4096, 6144
+    K = 4096
     g = torch.Generator(device=DEV).manual_seed(M)
     x = (torch.randn(M, K, generator=g, device=DEV) * torch.logspace(-2, 2, M, device=DEV)[:, None]).bfloat16()
     f = fold_norm(torch.randn(N, K, generator=g, device=DEV) * 0.02, torch.ones(K, device=DEV), None, None, True, 1e-5, DEV)
     attach_shuffled(f)
-    out = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
-    assert "gemm_lean" in _kernels(lambda: linear_norm(x, f, out=out))
+    NO = N // 2 if act else N
+    out = torch.full((M + 1, NO + 4), 7.0, device=DEV, dtype=torch.bfloat16)
+    assert "gemm_lean" in _kernels(lambda: linear_norm(x, f, act=act, out=out[:M, :NO]))
     xd = x.double() / (x.double().square().mean(-1, keepdim=True) + 1e-5).sqrt()
-    assert _err(out, xd @ f.w.double().t(), xd.abs() @ f.w.double().abs().t()) < 1
+    z, size = xd @ f.w.double().t(), xd.abs() @ f.w.double().abs().t()
+    if act:  # 8 gate columns, their 8 up columns; the derivative of silu is under 1.1
+        (gate, up), (sg, su) = (t.view(M, -1, 2, 8).transpose(1, 2).reshape(M, 2, NO).unbind(1) for t in (z, size))
+        z, size = torch.nn.functional.silu(gate) * up, 1.1 * sg * up.abs() + gate.abs() * su
+    assert _err(out[:M, :NO], z, size) < 1
+    assert (out[M:] == 7).all() and (out[:, NO:] == 7).all()
 
 
 def test_what_stays_with_the_general_kernels():
     """Rows off 16 bytes, outputs off 8, other widths and numbers of rows, no partials: the same results from elsewhere."""
     from distributed_neural_networks_amd.ops.gemm import attach_shuffled, linear
     g = torch.Generator(device=DEV).manual_seed(1)
-    for M, K, N, off in ((8, 768, 770, 0), (65, 768, 768, 0), (8, 832, 768, 0), (8, 768, 768, 1), (17, 4096, 4096, 0)):
+    for M, K, N, off in ((8, 768, 770, 0), (65, 768, 768, 0), (8, 832, 768, 0), (8, 768, 768, 1), (65, 4096, 4096, 0)):
         x, W = torch.randn(M, K, generator=g, device=DEV).bfloat16(), (torch.randn(N, K, generator=g, device=DEV) * 0.02).bfloat16()
         out, res = torch.empty(M, N + off, device=DEV, dtype=torch.bfloat16)[:, off:], torch.randn(M, N, generator=g, device=DEV).bfloat16()
         call = lambda: linear(x, W, None, None, res, out, w_shuf=attach_shuffled(W))  # noqa: E731
