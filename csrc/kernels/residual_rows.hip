@@ -408,6 +408,117 @@ static int lean_launch(const RowsArgs& a, hipStream_t st) {
 #undef LEAN
 }
 
+// The token shift of such rows (ROWS_SHIFT), a workgroup a row: it forms its own row and the one whose normed values it
+// needs beside it -- the row before, or the sequence's last one, for the state, where its own is the first -- and both
+// rows' loads are in flight and both rows' sums add up at once.  The general kernel's groups form theirs one after the other.  Bound as rows_lean_kernel is;
+// us of 4096 columns, general : this: 1 row 4.9 : 4.0, 506 rows 9.3 : 7.3, 640 11.0 : 8.5, 1300 17.4 : 14.5, 2048 23.1 : 19.4 (a
+// launch over and over; in a step 5 rows 7.3, 640 13.5 before).
+template <int NC, int IN, bool YN>
+__global__ __launch_bounds__(256) void rows_shift_kernel(RowsArgs a) {
+  __shared__ float red[16];
+  const int wave = threadIdx.x >> 6, c = threadIdx.x * 4, m = xcd_remap(blockIdx.x, gridDim.x);
+  f32x4 x[2][NC], yw[NC], nw[NC], mu[NC], prev[NC];
+  bf16x4 yb[2][NC];
+  auto load = [&](int k, int row) __attribute__((always_inline)) {
+    size_t yr = row;
+    if constexpr (IN == LEAN_TABLE)
+      if (a.yidx != nullptr) yr = (size_t)min(max(a.yidx[row], 0), a.yrows - 1);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      yb[k][i] = *reinterpret_cast<const bf16x4*>(reinterpret_cast<const bf16_t*>(a.y) + yr * a.ldy + c + 1024 * i);
+      if constexpr (IN == LEAN_JOIN) x[k][i] = ld4(a.x_in + (size_t)row * a.ldx + c + 1024 * i);
+    }
+  };
+  load(0, m);
+  load(1, max(m - 1, 0));
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    if constexpr (YN) yw[i] = ld4(a.y_w + c + 1024 * i);
+    nw[i] = ld4(a.n_w + c + 1024 * i);
+    mu[i] = ld4(a.sh_mu + c + 1024 * i);
+    prev[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const bool first = a.sh_start[m] == m;
+  const int last = min(max(a.sh_last[m], m), a.M - 1);
+  float* state = a.sh_state + (size_t)min(max(a.sh_slots[m], 0), a.sh_nslots - 1) * a.NP + c;
+  if (first) {
+    if (a.sh_pos[m] != 0) {
+#pragma unroll
+      for (int i = 0; i < NC; ++i) prev[i] = ld4(state + 1024 * i);
+    }
+    if (last != m) load(1, last);
+  }
+  f32x4 y[2][NC];
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int i = 0; i < NC; ++i) y[k][i] = f32x4{bf2f_s(yb[k][i][0]), bf2f_s(yb[k][i][1]), bf2f_s(yb[k][i][2]), bf2f_s(yb[k][i][3])};
+  // 1 / the root of the mean square of both rows
+  auto norms = [&](const f32x4 (&v)[2][NC], float* sums, float (&r)[2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      float s = 0.f;
+#pragma unroll
+      for (int i = 0; i < NC; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s = fmaf(v[k][i][j], v[k][i][j], s);
+      s = wave_sum(s);
+      if ((threadIdx.x & 63) == 0) sums[4 * k + wave] = s;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      r[k] = 1.0f / sqrtf((sums[4 * k] + sums[4 * k + 1] + sums[4 * k + 2] + sums[4 * k + 3]) / (float)a.N + a.eps);
+  };
+  float r[2];
+  if constexpr (YN) {
+    norms(y, red, r);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int i = 0; i < NC; ++i) y[k][i] = y[k][i] * r[k] * yw[i];
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[k][i][j] = fmaf(a.mult, y[k][i][j], IN == LEAN_JOIN ? x[k][i][j] : 0.f);
+      if (k == 0) st4(a.x_out + (size_t)m * a.ldx + c + 1024 * i, x[k][i]);
+    }
+  norms(x, red + 8, r);
+  const bool keeps = first && a.sh_last[last] == last;
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+#pragma clang fp contract(off)  // h is rounded before it is taken from the row before, as there
+    const f32x4 h = x[0][i] * r[0] * nw[i], o = x[1][i] * r[1] * nw[i], p = first || m == 0 ? prev[i] : o;
+    f32x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = fmaf(p[j] - h[j], mu[i][j], h[j]);
+    st4((bf16_t*)a.h + (size_t)m * a.ldh + c + 1024 * i, v);
+    if (keeps) st4(state + 1024 * i, last == m ? h : o);
+  }
+}
+
+// 1: not one of these forms.
+template <int NC>
+static int shift_launch(const RowsArgs& a, hipStream_t st) {
+  if (a.y == nullptr || a.x_out == nullptr || a.copy != nullptr || a.xidx != nullptr) return 1;
+#define SHIFT(IN, YN)                                                                       \
+  {                                                                                         \
+    hipLaunchKernelGGL((rows_shift_kernel<NC, IN, YN>), dim3(a.M), dim3(256), 0, st, a);     \
+    return (int)hipGetLastError();                                                          \
+  }
+  if (a.x_in == nullptr) {
+    if (a.y_w != nullptr) return 1;
+    SHIFT(LEAN_TABLE, false)
+  }
+  if (a.yidx != nullptr) return 1;
+  if (a.y_w != nullptr) SHIFT(LEAN_JOIN, true)
+  SHIFT(LEAN_JOIN, false)
+#undef SHIFT
+}
+
 constexpr int ROWS_GRID = 2048;  // workgroups of a launch of many rows: they loop, eight to a CU
 
 template <typename YT, typename OT, int PART>
@@ -493,11 +604,11 @@ extern "C" int dnn_rows_update(const RowsArgs* a, int y_f32, int out_f32, hipStr
   if (y_f32 && out_f32) ROWS_PART(float, float)
   // Up to as many rows as workgroups are in flight at once: past that the general kernel keeps the norms' weights
   // over a workgroup's rows.
-  if (!y_f32 && !out_f32 && !more && a->y2 == nullptr && a->ys == nullptr && a->freq == nullptr && a->sh_mu == nullptr &&
-      a->M <= ROWS_GRID) {
-    const int rc = a->NP == 1024   ? lean_launch<1>(*a, st)
-                   : a->NP == 2048 ? lean_launch<2>(*a, st)
-                   : a->NP == 4096 ? lean_launch<4>(*a, st)
+  if (!y_f32 && !out_f32 && !more && a->y2 == nullptr && a->ys == nullptr && a->freq == nullptr && a->M <= ROWS_GRID) {
+    const bool shift = a->sh_mu != nullptr;
+    const int rc = a->NP == 1024   ? shift ? shift_launch<1>(*a, st) : lean_launch<1>(*a, st)
+                   : a->NP == 2048 ? shift ? shift_launch<2>(*a, st) : lean_launch<2>(*a, st)
+                   : a->NP == 4096 ? shift ? shift_launch<4>(*a, st) : lean_launch<4>(*a, st)
                                    : 1;
     if (rc <= 0) return rc;
   }

@@ -157,7 +157,8 @@ class TokenShift:
         # neighbouring rows of a group of threads (a workgroup's; a wave's where rows
         # are short): more of them form fewer rows twice, but the rows of a group are a
         # chain, so only what four workgroups a CU leave over.  4096 wide: 640 rows
-        # 11 us (8 at a time 29), 2048 24 (37), 4096 38 (41), 8192 92 (one at a time 124)
+        # 11 us (8 at a time 29), 2048 24 (37), 4096 38 (41), 8192 92 (one at a time 124).  Up to 2048 bf16 rows of 1024,
+        # 2048 and 4096 columns have a kernel of their own (rows_shift_kernel), which does not ask.
         short = self.mu.numel() <= 1024
         a.sh_rows = min(4 if short else 8, -(-M // (4096 if short and M > 256 else 1024)))
 

@@ -73,3 +73,74 @@ def test_rows_lean(form, NP, N):
             tol = 1e-5 if k == "x_out" else 2.0 ** -8 + 1e-5
             err = (v.double().cpu() - want[k]).abs()
             assert (err <= tol * want[k].abs() + 2e-5).all(), (k, M, err.max())
+
+
+@pytest.mark.parametrize("NP,N", [(1024, 1000), (2048, 2048), (4096, 3997), (4096, 4096)])
+@pytest.mark.parametrize("form", ["table", "join", "y-norm"])
+@pytest.mark.parametrize("lengths", [(1,), (1, 1, 1, 1, 1), (3, 1, 250, 2), (1, 640, 7, 1399, 1)])
+def test_rows_shift(form, NP, N, lengths):
+    """The token shift, a workgroup a row: as the general kernel (more than 2048 rows) forms the same sequences, bit for bit
+    where both add in one order, fp64 otherwise; the states of fresh and going sequences before and after."""
+    from distributed_neural_networks_amd.ops import decoder_ops as D_
+
+    g = torch.Generator().manual_seed(NP + N + len(lengths) + len(form))
+    cols = torch.arange(NP) < N
+    M, S = sum(lengths), len(lengths)
+    assert M <= 2048
+    R = M + 2049
+
+    def noise(rows, std=1.0):
+        return (torch.randn(rows, NP, generator=g) * std * cols).cuda()
+
+    x, y, state0 = noise(R), noise(R, 3.0).bfloat16(), noise(S + 3)
+    yw, nw, mu = noise(1)[0], noise(1)[0], noise(1)[0]
+    ids = torch.randint(-2, R + 2, (R,), generator=g).int().cuda()  # clamped
+    slots = torch.randperm(S + 1, generator=g)[:S]
+    rows = [torch.zeros(R, dtype=torch.int32) for _ in range(4)]  # first, last row, slot, position
+    at = 0
+    for i, n in enumerate(list(lengths) + [R - M]):
+        slot, p0 = (slots[i].item(), 0 if i % 2 else 40 + i) if i < S else (S + 2, 5)
+        for t, v in zip(rows, (at, at + n - 1, slot, p0)):
+            t[at:at + n] = v
+        rows[3][at:at + n] += torch.arange(n, dtype=torch.int32)
+        at += n
+    rows = [t.cuda() for t in rows]
+
+    def call(M):
+        xo, h = torch.full((M + 1, NP), 7.0, device="cuda"), torch.full((M + 1, NP), 7.0, device="cuda", dtype=torch.bfloat16)
+        state = state0.clone()
+        kw = dict(y=y, yidx=ids[:M], mult=1.7) if form == "table" else dict(x_in=x[:M], y=y[:M], mult=0.6)
+        D_.rows_update(M, N, x_out=xo[:M], norm=nw, h=h[:M], y_norm=yw if form == "y-norm" else None, eps=1e-5,
+                       shift=D_.TokenShift(mu, state, *(t[:M].contiguous() for t in rows)), **kw)
+        assert (xo[M:] == 7).all() and (h[M:] == 7).all()
+        return xo[:M], h[:M], state
+
+    whole, got = call(R), call(M)
+    assert torch.equal(got[2][S + 1:], state0[S + 1:])
+    if NP > 1024:
+        for a, b in zip(got[:2], whole[:2]):
+            assert torch.equal(a, b[:M])
+        assert torch.equal(got[2][:S + 1], whole[2][:S + 1])
+    xd, yd = x.double().cpu(), y.double().cpu()
+    if form == "table":
+        z = 1.7 * yd[ids[:M].long().clamp(0, R - 1).cpu()]
+    else:
+        z = yd[:M]
+        if form == "y-norm":
+            z = z * torch.rsqrt((z * z).sum(1, keepdim=True) / N + 1e-5) * yw.double().cpu()
+        z = xd[:M] + 0.6 * z
+    hn = z * torch.rsqrt((z * z).sum(1, keepdim=True) / N + 1e-5) * nw.double().cpu()
+    prev, want_state, at = torch.cat([hn[:1], hn[:-1]]), state0.double().cpu(), 0
+    for i, n in enumerate(lengths):
+        prev[at] = 0 if i % 2 else want_state[slots[i]]
+        at += n
+    at = 0
+    for i, n in enumerate(lengths):
+        at += n
+        want_state[slots[i]] = hn[at - 1]
+    want = hn + (prev - hn) * mu.double().cpu()
+    # as above; the shift is one more rounding of values up to |prev| + |h|
+    assert ((got[0].double().cpu() - z).abs() <= 1e-5 * z.abs() + 2e-5).all()
+    assert ((got[2].double().cpu() - want_state).abs() <= 1e-5 * want_state.abs() + 2e-5).all()
+    size = hn.abs() + (prev.abs() + hn.abs()) * mu.double().cpu().abs()
+    assert ((got[1].double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * size + 2e-5).all()
