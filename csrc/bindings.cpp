@@ -120,6 +120,11 @@ PYBIND11_MODULE(_dnn_hip, m) {
                                        norm, eps, FP(stats), CP(parts), CFP(colsum), P(parts_out), &wrote, P(ws), ws_bytes);
     return py::make_tuple(rc, wrote != 0);
   });
+  m.def("gemm_bf16_qkv_rope", [](u64 A, int lda, u64 W, int ldw, float eps, u64 stats, u64 q, u64 kc, u64 vc, u64 pos, int B,
+                                 int T, int H, int Hkv, int hd, int S, int K, u64 cos, u64 sin, long long ws_bytes, u64 st) {
+    return dnn_gemm_bf16_qkv_rope(CP(A), lda, CP(W), ldw, eps, FP(stats), P(q), P(kc), P(vc), CIP(pos), B, T, H, Hkv, hd, S, K,
+                                  CFP(cos), CFP(sin), ws_bytes, ST(st));
+  });
   m.def("gemm_bf16_qkv_scatter_parts", [](u64 A, int lda, u64 W, int ldw, u64 bias, int norm, float eps, u64 stats, u64 parts,
                                           u64 colsum, u64 q, u64 kc, u64 vc, u64 pos, int B, int T, int H, int Hkv, int hd,
                                           int S, int K, u64 st) {

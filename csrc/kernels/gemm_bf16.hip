@@ -835,6 +835,45 @@ extern "C" int dnn_gemm_bf16_qkv_scatter(const void* A, int lda, const void* W, 
   return (int)hipGetLastError();
 }
 
+// The same with RoPE: x W^T under an RMS norm whose statistics this call takes (into `stats`), q and K rotated, heads of
+// 128.  A wave's 32 columns are 16 of a head's lower half and the same 16 of its upper half (the weight's rows are
+// staged in that order), so a rotation is within a lane, and the pass that split and rotated the stored rows goes (6.3 us for 700 rows of
+// 6144 columns, 33 for 8192, which is all but the traffic).  Four Llama-3 layers, us without and with: 700 rows 1410 : 1391, 4 x
+// 2048 11279 : 11199, 8 x 512 5280 : 5220, 1500 2500 : 2467; the same bits.
+// It needs tiles of 128 columns and all of K; where a split of K is the faster product by more than that pass takes, and
+// for all else: -3 with nothing launched.
+extern "C" int dnn_gemm_bf16_qkv_rope(const void* A, int lda, const void* W, int ldw, float eps, float* stats, void* q, void* kc,
+                                      void* vc, const int* pos, int B, int T, int H, int Hkv, int hd, int S, int K,
+                                      const float* cosT, const float* sinT, long long ws_bytes, hipStream_t st) {
+  const int M = B * T, N = (H + 2 * Hkv) * hd;
+  if (K % 64 != 0 || M <= 0 || cosT == nullptr || sinT == nullptr) return -1;
+  if (hd != 128 || M >= (1 << 24) || !dma_rows(A, lda, W, ldw) || !mid_narrow(lda, ldw) || tail_split_cols(M, N) != 0 ||
+      (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc | (uintptr_t)cosT | (uintptr_t)sinT) & 15) != 0)
+    return -3;
+  MidPlan plan = mid_plan(M, N, K, 0, MID_BF16);
+  if (g_mid_tile >= 0) plan = {g_mid_tile, 1, 0.f, 0};
+  else if (g_gemm_tile == 256) plan = {-1, 1, 0.f, 0};
+  else if (g_gemm_tile != 0 ||
+           plan.us > mid_plan(M, N, K, ws_bytes, MID_BF16).us + 3.f + (float)M * N * 4.f / 5.5e6f) return -3;
+  if (plan.tile == 0 || plan.tile == 1 || (plan.tile < 0 && M < 256)) return -3;
+  QkvScatter sc{(bf16_t*)q, (bf16_t*)kc, (bf16_t*)vc, pos, T, H, Hkv, 7, S, 1.0f / (float)T, 0, cosT, sinT};
+  if (const int rc = dnn_row_stats(A, lda, stats, M, K, eps, 1, st)) return rc;
+  const float2* rs = reinterpret_cast<const float2*>(stats);
+  const int n = plan.tile < 0 ? N : plan.cols;  // columns of the 256 x 256 kernel
+  if (n > 0) {
+    hipLaunchKernelGGL((gemm_bf16_256_kernel<ACT_NONE, false, true, 2, false, true>),
+                       dim3((M + BG_M - 1) / BG_M * ((n + BG_N - 1) / BG_N)), dim3(512), 0, st, (const bf16_t*)A, lda,
+                       (const bf16_t*)W, ldw, q, hd, (const float*)nullptr, (const bf16_t*)nullptr, 0, M, n, K, 0, rs,
+                       (const float*)nullptr, sc);
+    if (const hipError_t e = hipGetLastError()) return (int)e;
+  }
+  if (n == N) return 0;
+  sc.c_off = n;
+  const MidArgs a{{q, nullptr, nullptr, hd, 0, M, N - n, ACT_NONE, 0}, (const bf16_t*)A, (const bf16_t*)W + (size_t)n * ldw, rs,
+                  nullptr, nullptr, nullptr, eps, 1, nullptr, lda, ldw, K, 1};
+  return mid_launch(plan.tile, a, &sc, st);
+}
+
 // fp8 (W8A8) c_attn with the QKV scatter epilogue: A8 / sa the per-token
 // e4m3 activations (layernorm_q8), W8 / sw the e4m3 weight, Kb its row bytes.
 extern "C" int dnn_gemm_fp8_qkv_scatter(const void* A8, const float* sa, const void* W8, const float* sw,

@@ -205,6 +205,7 @@ struct MidSource {
   char* lds;
   int nk, wave;
   uint32_t oa[T::PA], ob[T::PB];
+  template <bool ROPE = false>  // ROPE: rope_row (gemm_tile.h), of whole 128s
   __device__ __forceinline__ void init(const char* A, int lda, int m0, int M, const char* W, int ldw, int n0, int N, int k0,
                                        int nk_, char* smem, int wave_, int lane) {
     a = A + (size_t)m0 * lda + (size_t)k0 * 128;
@@ -218,7 +219,7 @@ struct MidSource {
 #pragma unroll
     for (int q = 0; q < T::PB; ++q) {
       const int rl = (q * T::NW + wave) * 8 + (lane >> 3);
-      ob[q] = (uint32_t)min(rl, N - 1 - n0) * (uint32_t)ldw + (uint32_t)((lane & 7) ^ swz_chunk(rl)) * 16u;
+      ob[q] = (uint32_t)min(ROPE ? (rl & ~127) + rope_row(rl & 127) : rl, N - 1 - n0) * (uint32_t)ldw + (uint32_t)((lane & 7) ^ swz_chunk(rl)) * 16u;
     }
   }
   // Part i of n of K-tile t; past the end: a harmless refill, so that the waits count alike
@@ -327,6 +328,33 @@ __device__ __forceinline__ void mid_scatter(f32x4 (&acc)[I][J], int mw, int nw, 
 #pragma unroll
     for (int jp = 0; jp < J / 2; ++jp)
       if (nw + jp * 32 < N) epi_pair_scatter(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, M, row[i], col[jp]);
+}
+
+// The same with q and K rotated (host: heads of 128, no bias; rows staged by rope_row).
+template <int I, int J>
+__device__ __forceinline__ void mid_rope(f32x4 (&acc)[I][J], int mw, int nw, int M, int N, int lane, const QkvScatter& scat) {
+  QkvRow row[I];
+  QkvCol col[J / 2];
+  f32x4 co[I][J / 2], si[I][J / 2];
+#pragma unroll
+  for (int i = 0; i < I; ++i) row[i] = qkv_row(scat, min(mw + i * 16, M - 1));
+#pragma unroll
+  for (int jp = 0; jp < J / 2; ++jp) {
+    col[jp] = qkv_col(scat, rope_pair_col(nw + jp * 32 + scat.c_off, lane));
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      co[i][jp] = rope_load(scat.cosT, row[i].p, nw + jp * 32, lane);
+      si[i][jp] = rope_load(scat.sinT, row[i].p, nw + jp * 32, lane);
+    }
+  }
+  const int rotated = ((scat.H + scat.Hkv) << 7) - scat.c_off;
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int jp = 0; jp < J / 2; ++jp) {
+      if (nw + jp * 32 < rotated) rope_pair(acc[i][2 * jp], acc[i][2 * jp + 1], co[i][jp], si[i][jp]);
+      if (nw + jp * 32 < N) epi_pair_scatter(acc[i][2 * jp], acc[i][2 * jp + 1], mw + i * 16, M, row[i], col[jp]);
+    }
 }
 
 // A wave's accumulators (rows mw + 16 i of this lane, columns from nw on) through the epilogue to C.
@@ -572,7 +600,7 @@ __device__ __forceinline__ void mid_stage(const MidSource<T>& src) {
   __builtin_amdgcn_s_waitcnt(wait_imm(0, 0));
 }
 
-enum MidOut { MID_ROWS = 0, MID_SCATTER = 1, MID_PART = 2 };
+enum MidOut { MID_ROWS = 0, MID_SCATTER = 1, MID_PART = 2, MID_ROPE = 3 };
 
 // MERGE: the folded norm's statistics from partials (a variant of its own: a load under a branch is waited for where
 // the branch ends, ahead of the first request)
@@ -606,8 +634,8 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_mid_kernel(MidArgs p, QkvS
     nk = (int)((long long)nk * (sp + 1) / p.splits) - k0;
   }
   MidSource<T> src;
-  src.init(reinterpret_cast<const char*>(p.A), p.lda * 2, m0, M, reinterpret_cast<const char*>(p.W), p.ldw * 2, n0, N, k0,
-           nk, smem, wave, lane);
+  src.template init<OUT == MID_ROPE>(reinterpret_cast<const char*>(p.A), p.lda * 2, m0, M, reinterpret_cast<const char*>(p.W),
+                                     p.ldw * 2, n0, N, k0, nk, smem, wave, lane);
   if constexpr (T::PW > 0) {
     if (cw < 0) {
       mid_stage<T>(src);
@@ -617,6 +645,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_mid_kernel(MidArgs p, QkvS
   const int mw = m0 + wm * (I * 16) + fr, nw = n0 + wn * (J * 16);  // the lane's first row, the wave's first column
   MidPre<I, J> pre;
   if constexpr (EPI != MID_ANY) pre.template load_plain<EPI>(p, !MERGE && (EPI & MID_STAT) != 0 ? p.rowstat : nullptr, p.colsum, mw, nw, lane);
+  else if constexpr (OUT == MID_ROPE) pre.template load_plain<MID_STAT>(p, p.rowstat, nullptr, mw, nw, lane);
   else if constexpr (!PART) pre.load(p, p.rowstat, p.colsum, mw, nw, lane, OUT == MID_ROWS);
   f32x4 acc[I][J];
   MidParts<T> parts;
@@ -652,6 +681,14 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_mid_kernel(MidArgs p, QkvS
         }
     }
     mid_rows_plain<I, J, EPI>(acc, mw, nw, lane, p, pre, p.parts_out);
+    return;
+  }
+  if constexpr (OUT == MID_ROPE) {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int j = 0; j < J; ++j) acc[i][j] *= pre.rs[i].x;
+    mid_rope<I, J>(acc, mw, nw, M, N, lane, scat);
     return;
   }
   if (MERGE || p.rowstat != nullptr) {  // the folded norm, in the 256 x 256 kernel's order of operations

@@ -127,6 +127,12 @@ static int launch(const MidArgs& a, const QkvScatter* scat, hipStream_t st) {
     return scat != nullptr ? mid_start<T, MID_SCATTER, true>(a, *scat, st) : mid_start<T, MID_ROWS, true>(a, QkvScatter{}, st);
   }
 #endif
+#ifndef DNN_DECODER_ONLY
+  if (scat != nullptr && scat->cosT != nullptr) {
+    if constexpr (T::BN % 128 == 0) return mid_start<T, MID_ROPE>(a, *scat, st);
+    return -1;
+  }
+#endif
   if (scat != nullptr) return mid_start<T, MID_SCATTER>(a, *scat, st);
   if (a.splits == 1) return mid_start<T, MID_ROWS>(a, QkvScatter{}, st);
   if (const int rc = mid_start<typename MidSplit<T>::type, MID_PART>(a, QkvScatter{}, st)) return rc;

@@ -68,6 +68,10 @@ __device__ __forceinline__ void stage_half(const bf16_t* __restrict__ src, int l
   }
 }
 
+// ROPE: heads of 128, the weight's rows staged so that 32 columns of a tile are columns 16 i .. of the lower half of a
+// head and the same of its upper half: the two that a rotation takes lie in one lane.  Tile row b of 128 -> row of the head
+__device__ __forceinline__ int rope_row(int b) { return (b >> 5) << 4 | (b & 15) | (b & 16) << 2; }
+
 // The 4 pieces (8 rows of 128 B) of an operand that a wave stages: piece x & 1 of
 // half-tile x >> 1.  Uniform row bases and a lane offset: per-lane 64-bit addresses
 // would take 16 registers that the 256 x 256 schedule needs for fragments.
@@ -75,12 +79,13 @@ struct BgRows {
   const char* base[4];
   uint32_t lim[4];          // the lane's row offset is clamped to it (rows past the matrix)
   uint32_t lrow, lchunk;    // byte offsets of the lane's row and (swizzled) chunk
-  // ld in elements; 8 rows are addressed with 32 bits (host: bg_narrow)
+  // ld in elements; 8 rows are addressed with 32 bits (host: bg_narrow).  ROPE: rope_row, of whole 128s
+  template <bool ROPE = false>
   __device__ __forceinline__ void init(const bf16_t* src, int ld, int r0, int nrows, int wave, int lane) {
     const uint32_t ldb = (uint32_t)ld * 2u;
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
-      const int r = min(r0 + (x >> 1) * 128 + ((x & 1) * 8 + wave) * 8, nrows - 1);
+      const int b = ((x & 1) * 8 + wave) * 8, r = min(r0 + (x >> 1) * 128 + (ROPE ? rope_row(b) : b), nrows - 1);
       base[x] = reinterpret_cast<const char*>(src) + (size_t)r * ldb;
       lim[x] = (uint32_t)min(7, nrows - 1 - r) * ldb;
     }
@@ -196,6 +201,7 @@ struct QkvScatter {
   int T, H, Hkv, hd_shift, S;  // head dim = 1 << hd_shift
   float invT;                  // 1 / T (row -> sequence without an integer division)
   int c_off = 0;               // first qkv column of this launch (the tail-split launch covers the last 256)
+  const float *cosT = nullptr, *sinT = nullptr;  // rotary tables [position][hd / 2] (ROPE)
 };
 
 // 8 consecutive output columns c..c+7 (one head) of row m -> destination.  The
@@ -215,10 +221,11 @@ __device__ __forceinline__ int qkv_batch(const QkvScatter& sc, int m) {
 struct QkvRow {
   size_t q, kv;
   bool in;  // false: past the cache capacity, k and v are dropped, as in qkv_split
+  int p;    // position, within the capacity
 };
 __device__ __forceinline__ QkvRow qkv_row(const QkvScatter& sc, int m) {
   const int b = qkv_batch(sc, m), t = m - b * sc.T, p = sc.pos[b] + t;
-  return QkvRow{((size_t)b * sc.H * sc.T + t) << sc.hd_shift, ((size_t)b * sc.Hkv * sc.S + p) << sc.hd_shift, p < sc.S};
+  return QkvRow{((size_t)b * sc.H * sc.T + t) << sc.hd_shift, ((size_t)b * sc.Hkv * sc.S + p) << sc.hd_shift, p < sc.S, min(p, sc.S - 1)};
 }
 struct QkvCol {
   bf16_t* base;
@@ -235,6 +242,24 @@ __device__ __forceinline__ QkvCol qkv_col(const QkvScatter& sc, int c) {
 }
 // the column of the 8 that lane row q = lane >> 4 stores of the pair from nb on (epi_pair_bf16)
 __device__ __forceinline__ int pair_col(int nb, int lane) { return nb + (((lane >> 4) & 1) << 4) + ((lane >> 5) << 3); }
+
+// ROPE (rope_row): where the lane's store of a pair of 16 columns goes (tile columns from nb on)
+__device__ __forceinline__ int rope_pair_col(int nb, int lane) {
+  return (nb & ~127) + ((nb & 96) >> 1) + (((lane >> 4) & 1) << 6) + ((lane >> 5) << 3);
+}
+// The lane's entries of a table for that pair at position p
+__device__ __forceinline__ f32x4 rope_load(const float* table, int p, int nb, int lane) {
+  return *reinterpret_cast<const f32x4*>(table + (size_t)p * 64 + ((nb & 96) >> 1) + (lane >> 4) * 4);
+}
+// As qkv_split_kernel rotates a row that was stored in bf16
+__device__ __forceinline__ void rope_pair(f32x4& lo, f32x4& hi, const f32x4& co, const f32x4& si) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float a = bf2f(f2bf(lo[r])), c = bf2f(f2bf(hi[r]));
+    lo[r] = fmaf(a, co[r], -(c * si[r]));
+    hi[r] = fmaf(c, co[r], a * si[r]);
+  }
+}
 
 // One widened 16-B store per lane (as epi_pair_bf16) of a whole 32-column pair
 // to its head-major / cache destination.
@@ -261,7 +286,8 @@ __device__ __forceinline__ void epi_pair_scatter(const f32x4& a0, const f32x4& a
 // GRP: the rows are sorted by expert (grouped_tile.h): a tile belongs to one
 // expert's range of places, A rows are gathered, W holds every expert's weight
 // in fragment order (ops/gemm.py shuffle_weight) and C rows are places.
-template <int ACT, bool OUT_F32, bool SCATTER = false, int NQ = 2, bool GRP = false>
+// ROPE: with SCATTER, q and K rotated on their way (NQ = 2; host: heads of 128, no bias, no colsum).
+template <int ACT, bool OUT_F32, bool SCATTER = false, int NQ = 2, bool GRP = false, bool ROPE = false>
 __global__ __launch_bounds__(512, 1) void gemm_bf16_256_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int ldw, void* __restrict__ Cv,
     int ldc, const float* __restrict__ bias, const bf16_t* __restrict__ R, int ldr, int M, int N, int K,
@@ -317,7 +343,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_256_kernel(
   BgRows ra, rb;
   if constexpr (NQ == 2 && !GRP) {
     ra.init(A, lda, m0, M, wave, lane);
-    rb.init(W, ldw, n0, N, wave, lane);
+    rb.template init<ROPE>(W, ldw, n0, N, wave, lane);
   }
   auto stA = [&](int u, int h, int t) {
     t = t < nk ? t : nk - 1;
@@ -500,12 +526,34 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_256_kernel(
   QkvRow srow[2][4];
   QkvCol scol[NQ];
   if constexpr (SCATTER) {
+    if constexpr (ROPE) {
+      f32x4 co[2][4], si[2][4];
+#pragma unroll
+      for (int mq = 0; mq < 2; ++mq)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int p = qkv_row(scat, min(m0 + mq * 128 + arow + i * 16 + (lane & 15), M - 1)).p;
+          co[mq][i] = rope_load(scat.cosT, p, wc * 32, lane);
+          si[mq][i] = rope_load(scat.sinT, p, wc * 32, lane);
+        }
+#pragma unroll
+      for (int nq = 0; nq < NQ; ++nq) {
+        if ((n0 + nq * 128 + scat.c_off) >> 7 >= scat.H + scat.Hkv) continue;  // V
+#pragma unroll
+        for (int mq = 0; mq < 2; ++mq)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) rope_pair(acc[mq][nq][i][0], acc[mq][nq][i][1], co[mq][i], si[mq][i]);
+      }
+    }
 #pragma unroll
     for (int mq = 0; mq < 2; ++mq)
 #pragma unroll
       for (int i = 0; i < 4; ++i) srow[mq][i] = qkv_row(scat, min(m0 + mq * 128 + arow + i * 16 + (lane & 15), M - 1));
 #pragma unroll
-    for (int nq = 0; nq < NQ; ++nq) scol[nq] = qkv_col(scat, pair_col(n0 + nq * 128 + wc * 32 + scat.c_off, lane));
+    for (int nq = 0; nq < NQ; ++nq) {
+      const int nb = n0 + nq * 128 + wc * 32 + scat.c_off;
+      scol[nq] = qkv_col(scat, ROPE ? rope_pair_col(nb, lane) : pair_col(nb, lane));
+    }
     if (bias_e != nullptr) {
 #pragma unroll
       for (int nq = 0; nq < NQ; ++nq) {

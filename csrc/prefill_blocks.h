@@ -121,11 +121,20 @@ struct PrefillPass {
                            kpad(K), 0, nullptr, 0, nullptr, 0, st);
   }
 
-  // q, K and V of a block without RoPE straight to q and the caches: 1 done, 0 not this shape, < 0 or > 1 failed
+  // q, K and V of a block straight to q and the caches: 1 done, 0 not this shape, < 0 or > 1 failed
   int scattered(const void* in, const PrefillProj& p, void* k, void* v, int& rc) {
     const int N = (H + 2 * Hkv) * hd;
     rc = 0;
-    if (!scatter || cosT != nullptr || skinny(N, d, true, fp8 || p.frag != nullptr, 0)) return 0;
+    if (!scatter || skinny(N, d, true, fp8 || p.frag != nullptr, 0)) return 0;
+    if (cosT != nullptr) {
+      if (fp8 || norm != 1 || p.bias != nullptr || p.colsum != nullptr) return 0;
+      what = "gemm_bf16_qkv_rope";
+      rc = dnn_gemm_bf16_qkv_rope(in, d, p.w, d, eps, (float*)a, q, k, v, pos, B, T, H, Hkv, hd, S, d, cosT, sinT,
+                                  ws == nullptr ? 0 : ws_bytes - 4096, st);
+      if (rc != -3) return 1;
+      rc = 0;
+      return 0;
+    }
     if (fp8) {
       if (N % 32 != 0) return 0;
       if ((rc = quant_norm(in))) return 0;
