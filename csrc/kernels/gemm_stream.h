@@ -9,8 +9,8 @@
 // load path (guide §5, "x operand through LDS in full lines": fragment-shaped
 // x +18..45 %), and Llama-3 8B B=32 projections stream at 3-4.8 TB/s.
 // Here:
-//   * a workgroup owns BN = 64 NT output columns (4 waves x NT 16-column
-//     tiles) and ONE K range; the waves share the A rows of that range, staged
+//   * a workgroup owns BN output columns (NW waves x NT 16-column
+//     tiles: 128 as 4 x 2 or 8 x 1, 112 as 7 x 1) and ONE K range; the waves share the A rows of that range, staged
 //     through LDS in full 512-B row segments (global_load_dwordx4 -> ds_write),
 //     so A crosses the load path once per workgroup: A : W bytes = M : BN;
 //   * each wave streams its own weight tiles straight to VGPRs (guide: GEMV
@@ -200,8 +200,9 @@ __device__ __forceinline__ void str_combine_tile(const float* slab, int splitk, 
   }
 }
 
-template <int MT, int NT, bool W8, int NORM, int ACT, bool SPLIT, bool FOLD = false>
-__global__ __launch_bounds__(256, 1) void gemm_stream_kernel(const uint8_t* __restrict__ A, int lda_b,
+// NW waves (FOLD: 4).
+template <int MT, int NT, bool W8, int NORM, int ACT, bool SPLIT, bool FOLD = false, int NW = 4>
+__global__ __launch_bounds__(NW * 64, 1) void gemm_stream_kernel(const uint8_t* __restrict__ A, int lda_b,
                                                              const uint8_t* __restrict__ Wsh,
                                                              const float* __restrict__ sw, void* __restrict__ Cv,
                                                              int ldc, const float* __restrict__ bias,
@@ -211,9 +212,11 @@ __global__ __launch_bounds__(256, 1) void gemm_stream_kernel(const uint8_t* __re
                                                              unsigned* __restrict__ cnt = nullptr) {
   using Cfg = StrCfg<W8>;
   constexpr int ACH = Cfg::ACH, CS = Cfg::CS, AU = Cfg::AU;
+  static_assert(NW == 4 || !FOLD, "");
+  static_assert(NW >= MT, "a wave a row tile's statistics");
   constexpr int MP = MT * 16;
-  constexpr int BN = 64 * NT;
-  constexpr int APASS = MP * STR_SB / 4096;  // 16-B staging loads per thread per step
+  constexpr int BN = 16 * NW * NT;
+  constexpr int APASS = (MP * STR_SB + NW * 1024 - 1) / (NW * 1024);  // 16-B staging loads per thread per step
   __shared__ __attribute__((aligned(1024))) char lds[2 * MP * STR_SB + 4 * 16 * 2 * 4];
   float* st_lds = reinterpret_cast<float*>(lds + 2 * MP * STR_SB);  // [MT][2][16] row statistics (no SPLIT)
 
@@ -232,16 +235,16 @@ __global__ __launch_bounds__(256, 1) void gemm_stream_kernel(const uint8_t* __re
   const uint8_t* wp[NT];
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
-    int ct = tile * (4 * NT) + wave * NT + j;
+    int ct = tile * (NW * NT) + wave * NT + j;
     ct = ct < ntile16 ? ct : ntile16 - 1;
     wp[j] = Wsh + ((size_t)ct * nch + c0) * 1024 + lane * 16;
   }
-  // staging pass p: flat byte p*4096 + tid*16 of the step's [MP][512] A image
+  // staging pass p: flat byte p*NW*1024 + tid*16 of the step's [MP][512] A image (past its end: the last piece again)
   const uint8_t* ap[APASS];
   int aoff[APASS], aslot[APASS];
 #pragma unroll
   for (int p = 0; p < APASS; ++p) {
-    const int flat = p * 4096 + tid * 16, row = flat >> 9, slot = (flat & 511) >> 4;
+    const int flat = min(p * (NW * 1024) + tid * 16, MP * STR_SB - 16), row = flat >> 9, slot = (flat & 511) >> 4;
     ap[p] = A + (size_t)min(row, M - 1) * lda_b;
     aslot[p] = slot * 16;
     aoff[p] = row * STR_SB + ((slot ^ (row & 15)) << 4);

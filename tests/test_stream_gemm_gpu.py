@@ -383,3 +383,28 @@ def test_oneshot_coresident_race_screen(N, floor_kb):
         set_oneshot_gemm(1)
     print(f"N={N} floor={floor_kb} KB: mismatched calls of 3000: {counts}")
     assert counts["product"] == 0, counts
+
+
+@pytest.mark.parametrize("M", [17, 31, 33, 64])
+@pytest.mark.parametrize("N,K", [(16, 64), (112, 192), (128, 576), (240, 4096), (2064, 320), (28672, 256)])
+def test_stream_gated_seven_waves(force_stream, M, N, K):
+    """Gate and up behind an RMS norm as tiles of 112 columns (seven waves): columns and K that no tile or step divides,
+    nothing written past the rows, every value to the roundings."""
+    from distributed_neural_networks_amd.ops.gemm import attach_shuffled, fold_norm, linear_norm, pack_gate_up
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K, device=DEV, generator=g).bfloat16()
+    gate, up = (torch.randn(N // 2, K, device=DEV, generator=g) / math.sqrt(K) for _ in range(2))
+    gamma = torch.rand(K, device=DEV, generator=g) + 0.5
+    f = attach_shuffled(fold_norm(pack_gate_up(gate, up), gamma, None, None, True, 1e-5, DEV))
+    out = torch.full((M + 1, N // 2 + 8), 5.0, device=DEV, dtype=torch.bfloat16)
+    linear_norm(x, f, act="silu_mul", out=out[:M, :N // 2])
+    assert (out[M] == 5).all() and (out[:, N // 2:] == 5).all()
+    xd = x.double()
+    w = f.w.double().view(N // 16, 2, 8, K)
+    r = xd * torch.rsqrt((xd * xd).mean(1, keepdim=True) + 1e-5)
+    zg, zu = (r @ w[:, i].reshape(-1, K).t() for i in (0, 1))
+    ref = zg * torch.sigmoid(zg) * zu
+    # one rounding to bf16; fp32 sums of K products of size about |r| |w|: 1e-5 of either factor, silu's slope is under 1.1
+    size = [(r.abs() @ w[:, i].reshape(-1, K).abs().t()) for i in (0, 1)]
+    bound = 2.0 ** -8 * ref.abs() + 1e-5 * (1.1 * size[0] * zu.abs() + size[1] * (zg * torch.sigmoid(zg)).abs()) + 1e-6
+    assert ((out[:M, :N // 2].double() - ref).abs() <= bound).all()
