@@ -526,12 +526,13 @@ static int launch_stream_mt(const void* A, int lda_b, const void* Wsh, const flo
   const int kelems = W8 ? kbytes : kbytes / 2;
   const dim3 grid(ntiles * splitk), block(256);
   // Gate and up of Llama-3 (28672 columns): 224 workgroups of 128 columns leave 32 CUs idle, and a CU streams no faster for
-  // it; as 256 of 112 every CU has one.  us a step of 4 layers behind 100 tokens, without and with : 32 rows 395 : 386, 64 rows 499 : 461.
+  // it; as 256 of 112 every CU has one.  Steps of 256 bytes of K: the first and the last step have nothing beside them.  us a
+  // step of 4 layers behind 100 tokens, as 128 columns, as 112, with 256 bytes (1024): 32 rows 395, 386, 384 (394); 64 rows 499, 461, 454 (544).
   if constexpr (!W8 && NORM == NORM_RMS && ACT == ACT_SILU_MUL) {
     constexpr int W = 7, BN7 = 16 * W;
     const int n7 = (N + BN7 - 1) / BN7;
     if (splitk == 1 && (n7 + 255) / 256 * BN7 < (ntiles + 255) / 256 * BN) {
-      hipLaunchKernelGGL((gemm_stream_kernel<MT, 1, W8, NORM, ACT, false, false, W>), dim3(n7), dim3(W * 64), 0, st,
+      hipLaunchKernelGGL((gemm_stream_kernel<MT, 1, W8, NORM, ACT, false, false, W, 256>), dim3(n7), dim3(W * 64), 0, st,
                          (const uint8_t*)A, lda_b, (const uint8_t*)Wsh, sw, C, ldc, bias, (const bf16_t*)R, ldr, M, N, nch, cps,
                          colsum, eps, kelems, (float*)nullptr, (unsigned*)nullptr);
       return (int)hipGetLastError();
@@ -550,10 +551,11 @@ static int launch_stream_mt(const void* A, int lda_b, const void* Wsh, const flo
                        eps, kelems, (float*)ws, cnt);
     return (int)hipGetLastError();
   }
-  // eight waves of a tile for four of two: twice the waves that wait (down, 32 rows: 23.6 -> 22.8 us)
-  hipLaunchKernelGGL((gemm_stream_kernel<MT, 1, W8, NORM, ACT, true, false, 4 * NT>), grid, dim3(256 * NT), 0, st,
-                     (const uint8_t*)A, lda_b, (const uint8_t*)Wsh, sw, C, ldc, bias, (const bf16_t*)R, ldr, M, N, nch, cps, colsum, eps, kelems,
-                     (float*)ws, (unsigned*)nullptr);
+  // eight waves of a tile for four of two: twice the waves that wait (down, 32 rows: 23.6 -> 22.8 us); 256 bytes of K: 64
+  // rows, a step 454 -> 449
+  hipLaunchKernelGGL((gemm_stream_kernel<MT, 1, W8, NORM, ACT, true, false, 4 * NT, 256>), grid, dim3(256 * NT), 0, st,
+                     (const uint8_t*)A, lda_b, (const uint8_t*)Wsh, sw, C, ldc, bias, (const bf16_t*)R, ldr, M, N, nch, cps,
+                     colsum, eps, kelems, (float*)ws, (unsigned*)nullptr);
   const int NO = is_glu(ACT) ? N / 2 : N;
   const long long threads = (long long)M * ((NO + 3) / 4);
   hipLaunchKernelGGL((gemm_stream_reduce<ACT, NORM, W8>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,

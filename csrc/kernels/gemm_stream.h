@@ -36,7 +36,7 @@
 
 namespace dnn {
 
-constexpr int STR_SB = 512;  // A bytes per row per K-step (bf16: 8 chunks of 32 k; W8: 4 chunks of 64 k)
+constexpr int STR_SB = 512;  // A bytes per row per K-step (bf16: 8 chunks of 32 k; W8: 4 chunks of 64 k), halved with one tile a wave
 
 template <bool W8>
 struct StrCfg {
@@ -200,8 +200,8 @@ __device__ __forceinline__ void str_combine_tile(const float* slab, int splitk, 
   }
 }
 
-// NW waves (FOLD: 4).
-template <int MT, int NT, bool W8, int NORM, int ACT, bool SPLIT, bool FOLD = false, int NW = 4>
+// NW waves (FOLD: 4); SB: A bytes per row per K-step.
+template <int MT, int NT, bool W8, int NORM, int ACT, bool SPLIT, bool FOLD = false, int NW = 4, int SB = STR_SB>
 __global__ __launch_bounds__(NW * 64, 1) void gemm_stream_kernel(const uint8_t* __restrict__ A, int lda_b,
                                                              const uint8_t* __restrict__ Wsh,
                                                              const float* __restrict__ sw, void* __restrict__ Cv,
@@ -211,14 +211,14 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_stream_kernel(const uint8_t* 
                                                              float eps, int kelems, float* __restrict__ slab,
                                                              unsigned* __restrict__ cnt = nullptr) {
   using Cfg = StrCfg<W8>;
-  constexpr int ACH = Cfg::ACH, CS = Cfg::CS, AU = Cfg::AU;
+  constexpr int ACH = Cfg::ACH, CS = SB / ACH, AU = Cfg::AU;
   static_assert(NW == 4 || !FOLD, "");
   static_assert(NW >= MT, "a wave a row tile's statistics");
   constexpr int MP = MT * 16;
   constexpr int BN = 16 * NW * NT;
-  constexpr int APASS = (MP * STR_SB + NW * 1024 - 1) / (NW * 1024);  // 16-B staging loads per thread per step
-  __shared__ __attribute__((aligned(1024))) char lds[2 * MP * STR_SB + 4 * 16 * 2 * 4];
-  float* st_lds = reinterpret_cast<float*>(lds + 2 * MP * STR_SB);  // [MT][2][16] row statistics (no SPLIT)
+  constexpr int APASS = (MP * SB + NW * 1024 - 1) / (NW * 1024);  // 16-B staging loads per thread per step
+  __shared__ __attribute__((aligned(1024))) char lds[2 * MP * SB + 4 * 16 * 2 * 4];
+  float* st_lds = reinterpret_cast<float*>(lds + 2 * MP * SB);  // [MT][2][16] row statistics (no SPLIT)
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -244,10 +244,10 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_stream_kernel(const uint8_t* 
   int aoff[APASS], aslot[APASS];
 #pragma unroll
   for (int p = 0; p < APASS; ++p) {
-    const int flat = min(p * (NW * 1024) + tid * 16, MP * STR_SB - 16), row = flat >> 9, slot = (flat & 511) >> 4;
+    const int flat = min(p * (NW * 1024) + tid * 16, MP * SB - 16), row = flat / SB, slot = flat % SB >> 4;
     ap[p] = A + (size_t)min(row, M - 1) * lda_b;
     aslot[p] = slot * 16;
-    aoff[p] = row * STR_SB + ((slot ^ (row & 15)) << 4);
+    aoff[p] = row * SB + ((slot ^ (row & 15)) << 4);
   }
   const int a_last = c1 * ACH - 16;  // last valid 16 B of this slice's A rows (surplus chunks clamp here)
   // fragment read offsets (bytes inside a step image) for M tile t, chunk cc, piece h
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_stream_kernel(const uint8_t* 
   auto frag_off = [&](int t, int cc, int h) {
     const int row = 16 * t + fr;
     const int slot = (cc * ACH + fg * (ACH / 4) + 16 * h) >> 4;
-    return row * STR_SB + ((slot ^ (row & 15)) << 4);
+    return row * SB + ((slot ^ (row & 15)) << 4);
   };
 
   float shift = 0.f, s1 = 0.f, s2 = 0.f;  // statistics of row 16*wave + fr (waves < MT)
@@ -286,12 +286,12 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_stream_kernel(const uint8_t* 
       as[p] = *reinterpret_cast<const i32x4*>(ap[p] + min((c0 + s * CS) * ACH + aslot[p], a_last));
   };
   auto store_a = [&](int buf) {
-    char* base = lds + buf * (MP * STR_SB);
+    char* base = lds + buf * (MP * SB);
 #pragma unroll
     for (int p = 0; p < APASS; ++p) *reinterpret_cast<i32x4*>(base + aoff[p]) = as[p];
   };
   auto compute = [&](i32x4(&w)[NT][CS], int buf, int s) {
-    const char* base = lds + buf * (MP * STR_SB);
+    const char* base = lds + buf * (MP * SB);
 #pragma unroll
     for (int cc = 0; cc < CS; ++cc) {
       const bool valid = c0 + s * CS + cc < c1;  // wave-uniform
