@@ -118,6 +118,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_lean_kernel(LeanArgs p) {
       const int q = lane + i * 64;
       *reinterpret_cast<i32x4*>(mine + q / L::PB * L::STRIDE + q % L::PB * 16) = xr[d][i];
     }
+    // other lanes read what this one stored, and the next batch lies where this one did: the fences keep both orders (a
+    // wave's LDS operations run in them)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
     for (int u = 0; u < CB; ++u) {
       bf16x8 a[MT][AU];
@@ -151,6 +154,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_lean_kernel(LeanArgs p) {
           }
       }
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   };
   [&]<int... B>(std::integer_sequence<int, B...>) __attribute__((always_inline)) {
     (([&]() __attribute__((always_inline)) {

@@ -120,12 +120,16 @@ __global__ __launch_bounds__(64 * TG_WAVES) void token_gate_lean_kernel(const bf
   for (int h = 0; h < H; ++h) {
 #pragma unroll
     for (int i = 0; i < L::NX; ++i) *reinterpret_cast<bf16x8*>(to + i * (L::RPI * L::STRIDE)) = xr[h][i];
+    // other lanes read what this one stored, and the next part lies where this one did: the fences keep both orders (a
+    // wave's LDS operations run in them)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
     for (int u = 0; u < L::CP; ++u)
 #pragma unroll
       for (int r = 0; r < R; ++r)
         acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
             w[h * L::CP + u], *reinterpret_cast<const bf16x8*>(from + r * (16 * L::STRIDE) + u * 64), acc[r], 0, 0, 0);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) red[wave][r][lane] = acc[r];
