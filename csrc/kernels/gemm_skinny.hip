@@ -632,7 +632,7 @@ static bool os_plan(int M, int N, int kbytes, bool have_ws, long long ws_bytes, 
       // keep gemm_skinny / gemm_stream.
       // the 50304-wide heads measured slower (GPT-2 26.2 -> 36.3 us, XL W8
       // 38.3 -> 47.2 us, profiles/r4_oneshot_heads.jsonl): wide N stays skinny
-      if (M <= 32 || N >= 16384 || nch > 4 * (W8 ? 2 : 1) * CS) return false;
+      if (g_stream_on == 2 || M <= 32 || N >= 16384 || nch > 4 * (W8 ? 2 : 1) * CS) return false;
       c.splitk = 1;
       c.steps = W8 ? 2 : 1;
       const bool narrow = N <= (W8 ? 2048 : 1024);
@@ -918,9 +918,10 @@ static int launch_skinny(const void* A, int lda_b, const float* sa, const void* 
   const bool pin_any = g_skinny_pin.id != 0 && (g_skinny_pin.n == 0 || g_skinny_pin.n == N) &&
                        (g_skinny_pin.k == 0 || g_skinny_pin.k * 2 == kbytes);
   if constexpr (!F32 && !FP8 && ACT != ACT_RELU) if (!pin_any) {
-    if (g_os_on == 1 && dnn_gemm_lean({(const uint8_t*)A, lda_b, (const uint8_t*)Wsh, sw, (bf16_t*)C, ldc, bias,
-                                                  (const bf16_t*)R, ldr, M, N, colsum, eps, g_rs_cur.in, g_rs_cur.in_ld,
-                                                  g_rs_cur.out, g_rs_cur.out_ld}, kbytes / 64, ACT, NORM, W8, st)) {
+    const bool forced = g_os_on != 1 || g_os_pin[0] > 0 || g_os_probe_abl != 0 || g_stream_on == 2;  // one of the kernels below
+    if (!forced && dnn_gemm_lean({(const uint8_t*)A, lda_b, (const uint8_t*)Wsh, sw, (bf16_t*)C, ldc, bias, (const bf16_t*)R, ldr,
+                                  M, N, colsum, eps, g_rs_cur.in, g_rs_cur.in_ld, g_rs_cur.out, g_rs_cur.out_ld},
+                                 kbytes / 64, ACT, NORM, W8, st)) {
       if (R != nullptr && g_rs_cur.out != nullptr) g_rs_written = 1;
       return (int)hipGetLastError();
     }

@@ -183,6 +183,57 @@ def test_stream_fold_matches_reduce_launch(norm):
     assert int(tickets.abs().sum()) == 0  # every ticket re-armed
 
 
+def _kernels(f):
+    """Names of the kernels that ``f`` launches."""
+    from torch.profiler import ProfilerActivity, profile
+    f()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        f()
+        torch.cuda.synchronize()
+    return " ".join(e.key for e in p.key_averages())
+
+
+@pytest.mark.parametrize("M,N,K,norm", [(17, 3072, 4096, 0), (64, 3072, 4096, 0), (32, 4096, 4096, 0), (32, 4096, 4096, 1),
+                                        (64, 640, 1024, 0), (64, 2048, 2048, 2)])
+@pytest.mark.parametrize("what", ["stream", "stream split", "stream fold", "one-shot", "one-shot pinned"])
+def test_forced_kernels_run(M, N, K, norm, what):
+    """A forced kernel is the one that runs, also for the shapes that kernels of their own are laid out for."""
+    from distributed_neural_networks_amd.ops.gemm import (attach_shuffled, decode_workspace, fold_norm, linear, linear_norm,
+                                                          set_oneshot_gemm, set_stream_gemm, shuffle_weight)
+    g = torch.Generator(device=DEV).manual_seed(N + M)
+    x, W = torch.randn(M, K, device=DEV, generator=g).bfloat16(), torch.randn(N, K, device=DEV, generator=g) / math.sqrt(K)
+    R, xd = torch.randn(M, N, device=DEV, generator=g).bfloat16(), x.double()
+    ws = decode_workspace(DEV, 7) if what != "stream" else None
+    if norm:
+        f = attach_shuffled(fold_norm(W, torch.ones(K, device=DEV), None, None, norm == 1, 1e-5, DEV))
+        run = lambda: linear_norm(x, f, ws=ws)  # noqa: E731
+        xd = xd if norm == 1 else xd - xd.mean(-1, keepdim=True)
+        ref = xd / (xd.square().mean(-1, keepdim=True) + 1e-5).sqrt() @ W.bfloat16().double().t()
+    else:
+        Wb = W.bfloat16()
+        sh = shuffle_weight(Wb)
+        run = lambda: linear(x, Wb, residual=R, w_shuf=sh, ws=ws)  # noqa: E731
+        ref = xd @ Wb.double().t() + R.double()
+    try:
+        if what.startswith("stream"):
+            set_stream_gemm(2, 1, int(what == "stream fold"))
+        elif what == "one-shot":
+            set_oneshot_gemm(2)
+        else:
+            set_oneshot_gemm(1, 2, 1, 2, -(-K // 2048))
+        names, y = _kernels(run), run()
+        torch.cuda.synchronize()
+    finally:
+        set_stream_gemm(1, 8 << 20, 0)
+        set_oneshot_gemm(1)
+    assert ("gemm_stream_kernel" if what.startswith("stream") else "gemm_oneshot_kernel") in names, names
+    if what == "stream split":
+        assert "gemm_stream_reduce" in names, names
+    # both round a sum of products of unit rows to bf16, which is 2^-9 of it at most; the rest is fp32
+    assert ((y.double() - ref).norm() / ref.norm()).item() < 2.0 ** -8
+
+
 # ---------------------------------------------------------------- one-shot decode GEMM (gemm_oneshot.h)
 @pytest.mark.parametrize("M", [17, 32, 64])
 @pytest.mark.parametrize("N,K,w8", [(2304, 768, False), (768, 3072, False), (4800, 1600, True), (1600, 6400, True),
