@@ -65,8 +65,9 @@ class ColocatedPipeline:
         direct = x is not None and self._reads(x)
         if x is not None and not direct:
             self.x.copy_(x, non_blocking=True)
-        if direct and len(self.stages) == 2 and not trace.enabled():
-            out = self.stages[0].pass_few(self.stages[1], x, self.bufs[0], self.bufs[1], self.x)
+        few = getattr(self.stages[0], "pass_few", None) if direct and len(self.stages) == 2 and not trace.enabled() else None
+        if few is not None:
+            out = few(self.stages[1], x, self.bufs[0], self.bufs[1], self.x)
             if out is not None:
                 return out
         with trace.span("pipeline_step", "compute", device=self.x.device, batch=self.batch):

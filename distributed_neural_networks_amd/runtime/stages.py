@@ -122,8 +122,10 @@ class CifarHipStage(StageCompute):
     def keeps_input(self) -> bool:
         """``forward(keep=)``: the launch that reads the images can leave a copy of them.  A
         ``forward`` that was replaced or wrapped need not know of it."""
-        return (self.first and self.precision == "fp32" and type(self).forward is CifarHipStage.forward
-                and "forward" not in self.__dict__)
+        return self.first and self.precision == "fp32" and self._own_forward()
+
+    def _own_forward(self) -> bool:
+        return type(self).forward is _CIFAR_FORWARD and "forward" not in self.__dict__
 
     def forward(self, x, out=None, keep=None):
         B = x.shape[0]
@@ -148,15 +150,14 @@ class CifarHipStage(StageCompute):
             probs, pred = self._cops.head_tail(h.contiguous(), self.wh, out, buf["pred"])
         return StageOutput(probs, pred)
 
-
     def pass_few(self, last: "StageCompute", x: torch.Tensor, h: torch.Tensor, probs: torch.Tensor,
                  keep: torch.Tensor) -> Optional[StageOutput]:
         """This stage on ``x`` (float32, contiguous, as ``forward`` with ``keep``) and ``last`` on its output ``h``,
         their three launches by one native call: the pass of one image is bound by the host (25 us of it, 15 of the
         device's).  None, with nothing launched, where ``forward`` of both has to decide: more images, other ranges,
-        devices or encodings, a ``last`` that was replaced or wrapped, buffers that are not plain."""
+        devices or encodings, stages or forwards that were replaced or wrapped, buffers that are not plain."""
         B, c, wh = x.shape[0], self._cops, getattr(last, "wh", None)
-        if not (0 < B <= c.FC1_FEW_ROWS and type(last) is type(self) is CifarHipStage and "forward" not in last.__dict__
+        if not (0 < B <= c.FC1_FEW_ROWS and type(last) is type(self) is CifarHipStage and self._own_forward() and last._own_forward()
                 and (self.start, self.end, last.start, last.end) == (0, 1, 2, 3) and last.precision == "fp32"
                 and self.boundary == last.boundary and last.device == self.device
                 and c.stage0_direct(B, self.w0) and c.plain(h, (B, 4096)) and c.plain(probs, (B, 10))
@@ -165,6 +166,9 @@ class CifarHipStage(StageCompute):
         buf = last._buf(B)
         c.pass_few(x, self.w0, h, keep, wh, buf["split"], buf["hid"], probs, buf["pred"], self.boundary)
         return StageOutput(probs, buf["pred"])
+
+
+_CIFAR_FORWARD = CifarHipStage.forward  # as it stands here: a later one need not know of ``keep``
 
 
 class TorchStage(StageCompute):

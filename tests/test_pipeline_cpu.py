@@ -50,3 +50,50 @@ def test_wrapped_forward_is_given_no_keep():
     patched.forward = lambda x, out=None: out
     assert plain.keeps_input and not Wrapped(sd, 0, 1, cpu).keeps_input and not patched.keeps_input
     assert not CifarHipStage(sd, 2, 3, cpu).keeps_input and not CifarHipStage(sd, 0, 1, cpu, precision="bf16").keeps_input
+
+
+def _two(monkeypatch, first, last):
+    """A two-stage pipeline on the CPU whose first stage reads its input where it lies."""
+    from distributed_neural_networks_amd.runtime.pipeline import ColocatedPipeline
+    monkeypatch.setattr(ColocatedPipeline, "_reads", lambda self, x: True)
+    return ColocatedPipeline([first, last], 2)
+
+
+def test_a_first_stage_of_the_callers_own(monkeypatch):
+    """keeps_input says that ``forward`` takes ``keep``, and nothing of passes by one call."""
+    from distributed_neural_networks_amd.models.cifar import NeuralNetwork
+    from distributed_neural_networks_amd.runtime.stages import TorchStage
+
+    class Keeps(TorchStage):
+        keeps_input = True
+
+        def forward(self, x, out=None, keep=None):
+            if keep is not None:
+                keep.copy_(x)
+            return super().forward(x, out)
+
+    torch.manual_seed(2)
+    net = NeuralNetwork().eval()
+    sd = net.state_dict()
+    pipe = _two(monkeypatch, Keeps("cifar10", sd, 0, 1, True, False), TorchStage("cifar10", sd, 2, 3, False, True))
+    x = torch.randn(2, 3, 32, 32)
+    got = pipe(x).probs.clone()
+    assert torch.allclose(got, net(x), atol=1e-6) and torch.equal(pipe.x, x) and torch.equal(pipe().probs, got)
+
+
+@pytest.mark.parametrize("what", ["class", "first", "last"])
+def test_a_replaced_forward_is_not_passed_by(what, monkeypatch):
+    """On the class or on a stage, on either side of the cut: the native call leaves the pass to the forwards."""
+    from distributed_neural_networks_amd.models.cifar import NeuralNetwork
+    from distributed_neural_networks_amd.ops import cifar as cops
+    from distributed_neural_networks_amd.runtime.stages import CifarHipStage
+    native = []
+    monkeypatch.setattr(cops, "pass_few", lambda *a: native.append(1))
+    sd, cpu = NeuralNetwork().state_dict(), torch.device("cpu")
+    pipe = _two(monkeypatch, CifarHipStage(sd, 0, 1, cpu), CifarHipStage(sd, 2, 3, cpu))
+    few = lambda: pipe.stages[0].pass_few(pipe.stages[1], torch.zeros(2, 3, 32, 32), *pipe.bufs, pipe.x)  # noqa: E731
+    assert few() is not None and native == [1]  # as it is built
+    at = {"class": CifarHipStage, "first": pipe.stages[0], "last": pipe.stages[1]}[what]
+    monkeypatch.setattr(at, "forward", lambda *a, **kw: None)
+    assert few() is None and native == [1]
+    assert pipe.stages[0].keeps_input == (what == "last")
