@@ -162,9 +162,8 @@ __device__ __forceinline__ int k_swz(int key, int chunk) {
 // MXO (hd 64): a workgroup is 64 queries of two neighbouring heads, two waves each, the 128 columns that
 // share a scale of the projection behind (mx_index), and the rows leave as its e4m3 operand.  The quantiser's
 // launch and its pass over the rows (4 us and more) go, for keys and values staged for half as many queries:
-// us of both launches / of this, 25 heads, 8 x 256 14.8 / 10.4, 1 x 300 11.2 / 9.3, 1 x 960 23.3 / 23.4,
-// 8 x 960 54.9 / 50.6, 16 x 64 9.9 / 5.3.  With 128 queries a head, eight waves (8 x 256 13.3 in its pass, 12.3 so),
-// the longest tiles share a CU two and two.
+// us of both launches / of this, 25 heads, 8 x 256 14.6 / 10.1, 1 x 384 12.9 / 10.6, 16 x 64 9.8 / 5.3: flash_mx_pays.
+// With 128 queries a head, eight waves (8 x 256 13.3 in its pass, 12.3 so), the longest tiles share a CU two and two.
 template <int HD, bool QKV = false, bool KV8 = false, bool DB = false, bool PIPE = false, int KS = 1, bool MXO = false>
 __global__ __launch_bounds__(256 * KS, 2) void flash_attn_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                                                             const bf16_t* __restrict__ vc, bf16_t* __restrict__ o, int T,
@@ -1073,12 +1072,23 @@ extern "C" int dnn_flash_attn(const void* q, const void* kc, const void* vc, voi
   return (int)hipGetLastError();
 }
 
+// Whether that is faster than both launches: what it saves is one launch and a pass over T rows, what it pays is as many
+// stagings more as a tile has key blocks, T / 64.  us of both launches / of this (new sequences):
+//   768 tokens    12 heads, 1 sequence 18.0 / 17.6, 16 sequences 37.6 / 34.7; 25 heads 19.1 / 18.7, 72.6 / 71.3
+//   1024          few workgroups: 12 heads x 1 (96) 21.3 / 22.0, 16 x 1 (128) 21.6 / 22.1; between: 20 x 1 (160) 22.3 / 22.2,
+//                 16 x 4 (512) 26.6 / 24.4, 25 x 4 (832) 33.9 / 32.6; many: 25 x 8 (1664) 56.8 / 59.2, 25 x 16 112 / 121
+//   1280, 2048    25 x 1 29.1 / 29.4, 42.6 / 44.5; 25 x 4 45.4 / 46.8, 93 / 103; 20 x 8 64 / 66, 142 / 153
+static bool flash_mx_pays(int B, int T, int H) {
+  const long long wgs = (long long)(H + 1) / 2 * B * ((T + 63) / 64);
+  return T <= 768 || (T <= 1024 && wgs > 128 && wgs <= 1024);
+}
+
 // The same with rows that leave as MX e4m3 (dnn_quant_fp8_mx of them, bit by bit): q8 rows of ld8 bytes, whole 128-column
-// blocks of H * hd written.  -3, nothing launched: not this shape, or a pinned variant.
+// blocks of H * hd written.  -3, nothing launched: not this shape, a size at which both launches are faster, or a pinned variant.
 extern "C" int dnn_flash_attn_mx(const void* q, const void* kc, const void* vc, void* q8, int ld8, void* sx, int B, int T,
                                  int H, int Hkv, int hd, int S, const int* pos, float scale, hipStream_t st) {
   if (H % Hkv != 0 || ld8 % 8 != 0 || ld8 < (H + 1) / 2 * 128) return -1;
-  if (hd != 64 || getenv("DNN_FLASH_DB") != nullptr || getenv("DNN_FLASH_PIPE") != nullptr) return -3;
+  if (hd != 64 || !flash_mx_pays(B, T, H) || getenv("DNN_FLASH_DB") != nullptr || getenv("DNN_FLASH_PIPE") != nullptr) return -3;
   hipLaunchKernelGGL((flash_attn_kernel<64, false, false, true, false, 1, true>),
                      dim3((H + 1) / 2, B, (T + 63) / 64), dim3(256), 0, st, (const bf16_t*)q, (const bf16_t*)kc,
                      (const bf16_t*)vc, (bf16_t*)nullptr, T, H, Hkv, S, pos, scale * 1.4426950408889634f, 0,

@@ -29,3 +29,12 @@ def test_set_skinny_max_m_governs_folded_norms(max_m):
 def test_fp8_rows():
     assert G.skinny_rows(64, 50304, True) and G.skinny_rows(256, 12160, True) and not G.skinny_rows(65, 24576, True)
     assert not G.skinny_rows(257, 128, True)
+
+
+def test_attention_that_quantises_is_for_short_prefill(max_m):
+    """-3, nothing launched: long sequences, and launches of few or many workgroups of 769 tokens on, keep both launches."""
+    from distributed_neural_networks_amd.ops._lib import lib
+    call = lambda B, T, H: lib().flash_attn_mx(0, 0, 0, 0, -(-H // 2) * 128, 0, B, T, H, H, 64, T, 0, 0.125, 0)  # noqa: E731
+    for B, T, H in ((1, 1025, 25), (4, 1280, 20), (1, 2048, 12), (16, 4096, 16),  # 3 to 14 % slower
+                    (1, 769, 12), (1, 960, 16), (1, 1024, 12), (8, 960, 25), (16, 1024, 25), (8, 1024, 20)):
+        assert call(B, T, H) == -3, (B, T, H)
