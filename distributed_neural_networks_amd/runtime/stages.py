@@ -22,6 +22,7 @@ from typing import Dict, Optional, Tuple
 import torch
 
 from ..models import cifar, model_info
+from ..ops import _lib
 
 Spec = Tuple[Tuple[int, ...], torch.dtype]
 
@@ -157,7 +158,8 @@ class CifarHipStage(StageCompute):
         device's).  None, with nothing launched, where ``forward`` of both has to decide: more images, other ranges,
         devices or encodings, stages or forwards that were replaced or wrapped, buffers that are not plain."""
         B, c, wh = x.shape[0], self._cops, getattr(last, "wh", None)
-        if not (0 < B <= c.FC1_FEW_ROWS and type(last) is type(self) is CifarHipStage and self._own_forward() and last._own_forward()
+        if not (0 < B <= c.FC1_FEW_ROWS and not _lib.DEBUG_SYNC
+                and type(last) is type(self) is CifarHipStage and self._own_forward() and last._own_forward()
                 and (self.start, self.end, last.start, last.end) == (0, 1, 2, 3) and last.precision == "fp32"
                 and self.boundary == last.boundary and last.device == self.device
                 and c.stage0_direct(B, self.w0) and c.plain(h, (B, 4096)) and c.plain(probs, (B, 10))

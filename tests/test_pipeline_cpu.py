@@ -97,3 +97,16 @@ def test_a_replaced_forward_is_not_passed_by(what, monkeypatch):
     monkeypatch.setattr(at, "forward", lambda *a, **kw: None)
     assert few() is None and native == [1]
     assert pipe.stages[0].keeps_input == (what == "last")
+
+
+def test_a_sync_behind_every_kernel_needs_every_launch_by_itself(monkeypatch):
+    """DNN_DEBUG_SYNC names the launch that a fault is of."""
+    from distributed_neural_networks_amd.models.cifar import NeuralNetwork
+    from distributed_neural_networks_amd.ops import _lib, cifar as cops
+    from distributed_neural_networks_amd.runtime.stages import CifarHipStage
+    native = []
+    monkeypatch.setattr(cops, "pass_few", lambda *a: native.append(1))
+    monkeypatch.setattr(_lib, "DEBUG_SYNC", True)
+    sd, cpu = NeuralNetwork().state_dict(), torch.device("cpu")
+    pipe = _two(monkeypatch, CifarHipStage(sd, 0, 1, cpu), CifarHipStage(sd, 2, 3, cpu))
+    assert pipe.stages[0].pass_few(pipe.stages[1], torch.zeros(2, 3, 32, 32), *pipe.bufs, pipe.x) is None and not native
