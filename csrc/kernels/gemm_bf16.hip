@@ -846,8 +846,8 @@ extern "C" int dnn_gemm_bf16_qkv_rope(const void* A, int lda, const void* W, int
                                       void* vc, const int* pos, int B, int T, int H, int Hkv, int hd, int S, int K,
                                       const float* cosT, const float* sinT, long long ws_bytes, hipStream_t st) {
   const int M = B * T, N = (H + 2 * Hkv) * hd;
-  if (K % 64 != 0 || M <= 0 || cosT == nullptr || sinT == nullptr) return -1;
-  if (hd != 128 || M >= (1 << 24) || !dma_rows(A, lda, W, ldw) || !mid_narrow(lda, ldw) || tail_split_cols(M, N) != 0 ||
+  if (M <= 0 || cosT == nullptr || sinT == nullptr) return -1;
+  if (hd != 128 || K % 64 != 0 || M >= (1 << 24) || !dma_rows(A, lda, W, ldw) || !mid_narrow(lda, ldw) || tail_split_cols(M, N) != 0 ||
       (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc | (uintptr_t)cosT | (uintptr_t)sinT) & 15) != 0)
     return -3;
   MidPlan plan = mid_plan(M, N, K, 0, MID_BF16);

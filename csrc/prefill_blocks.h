@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "kernels/api.h"
+#include "kernels/gemm_mid_api.h"
 
 namespace dnn {
 
@@ -130,7 +131,7 @@ struct PrefillPass {
       if (fp8 || norm != 1 || p.bias != nullptr || p.colsum != nullptr) return 0;
       what = "gemm_bf16_qkv_rope";
       rc = dnn_gemm_bf16_qkv_rope(in, d, p.w, d, eps, (float*)a, q, k, v, pos, B, T, H, Hkv, hd, S, d, cosT, sinT,
-                                  ws == nullptr ? 0 : ws_bytes - 4096, st);
+                                  mid_ws(ws, ws_bytes), st);
       if (rc != -3) return 1;
       rc = 0;
       return 0;

@@ -38,3 +38,12 @@ def test_attention_that_quantises_is_for_short_prefill(max_m):
     for B, T, H in ((1, 1025, 25), (4, 1280, 20), (1, 2048, 12), (16, 4096, 16),  # 3 to 14 % slower
                     (1, 769, 12), (1, 960, 16), (1, 1024, 12), (8, 960, 25), (16, 1024, 25), (8, 1024, 20)):
         assert call(B, T, H) == -3, (B, T, H)
+
+
+def test_rotating_projection_leaves_other_shapes_to_the_rows(max_m):
+    """-3, nothing launched, also for a K that its tiles do not take; pointers that no kernel could use stay refused."""
+    from distributed_neural_networks_amd.ops._lib import lib
+    call = lambda K=256, hd=128, M=300, cos=16: lib().gemm_bf16_qkv_rope(  # noqa: E731
+        0, K, 0, K, 1e-5, 0, 0, 0, 0, 0, 1, M, 2, 1, hd, 512, K, cos, cos, 0, 0)
+    assert call(K=96) == call(K=4128) == call(hd=64) == -3
+    assert call(cos=0) == call(M=0) == -1
