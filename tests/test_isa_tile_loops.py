@@ -37,7 +37,7 @@ def test_no_spill_between_k_tiles():
                            text=True)
         assert r.returncode == 0, r.stderr[-2000:]
         asm = open(out).read()
-    for kernel, count in (("gemm_fp8_256_kernel", 16), ("gemm_bf16_256_kernel", 22)):
+    for kernel, count in (("gemm_fp8_256_kernel", 16), ("gemm_bf16_256_kernel", 23)):
         loops = list(main_loops(asm, kernel))
         assert len(loops) == count and all(sum("v_mfma" in ln for ln in lp) >= 32 for _, lp in loops)
         assert [n for n, lp in loops if any("scratch_" in ln for ln in lp)] == []
