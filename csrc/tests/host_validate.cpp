@@ -8,6 +8,7 @@
 #include <cstdio>
 
 #include "../kernels/api.h"
+#include "../kernels/attention_row.h"
 #include "../kernels/mixer_api.h"
 #include "../kernels/residual_api.h"
 
@@ -258,6 +259,7 @@ int main() {
     edit(b);
     expect_reject(dnn_paged_decode(&b, ip, 1, 1, nullptr, 0, st), what);
     expect_reject(dnn_paged_prefill(&b, ip, 1, st), what);
+    expect_reject(dnn_paged_mixed(&b, ip, 1, ip, 1, 1, nullptr, 0, st), what);
   };
   bad([](PagedAttnArgs& b) { b.DK = 96; }, "paged head size 96");
   bad([](PagedAttnArgs& b) { b.G = 2; }, "paged heads % kv heads");
@@ -271,6 +273,11 @@ int main() {
   expect_reject(dnn_paged_decode(&pa, ip, 1, 2, f, 4, st), "paged decode workspace too small");
   expect_reject(dnn_paged_decode(&pa, ip, 0, 1, nullptr, 0, st), "paged decode of nothing");
   expect_reject(dnn_paged_prefill(&pa, ip, 0, st), "paged prefill of nothing");
+  expect_reject(dnn_paged_mixed(&pa, ip, 0, ip, 1, 1, nullptr, 0, st), "paged launch of both without portions");
+  expect_reject(dnn_paged_mixed(&pa, ip, 1, ip, 0, 1, nullptr, 0, st), "paged launch of both without single tokens");
+  expect_reject(dnn_paged_mixed(&pa, ip + 1, 1, ip, 1, 1, nullptr, 0, st), "paged tiles off 16 bytes");
+  expect_reject(dnn_paged_mixed(&pa, ip, 1, ip, 1, 2, f, 4, st), "paged workspace of both too small");
+  expect_reject(dnn_paged_mixed(&pa, ip, 0x7fffffff, ip, 1, 1, nullptr, 0, st), "paged workgroups past an int");
   // GEMMs
   expect_reject(dnn_gemm_bf16(p, 96, p, 96, p, 8, nullptr, nullptr, 0, 128, 128, 96, 0, 0, st), "gemm K%64");
   expect_reject(dnn_gemm_bf16(p, 64, p, 64, p, 8, nullptr, nullptr, 0, 0, 128, 64, 0, 0, st), "gemm M=0");
@@ -311,7 +318,38 @@ int main() {
   expect_reject(dnn_layernorm(p, 16384, f, f, p, 16384, 4, 16384, 1e-5f, 1, st), "layernorm N>8192");
   expect_reject(dnn_embed_gpt2(ip, p, p, p, 1, 1, 12, ip, 8, 8, st), "embed d%8");
   expect_reject(dnn_embed_gpt2(ip, p, p, p, 1, 1, 16, ip, 0, 8, st), "embed empty vocab");
+  expect_reject(dnn_layernorm_q8_mx(p, 64, nullptr, f, p, 128, p, 4, 64, 128, 1e-5f, 0, st), "standardised rows with a shift");
+  expect_reject(dnn_layernorm_q8_mx(p, 68, nullptr, nullptr, p, 128, p, 4, 64, 128, 1e-5f, 0, st), "standardised rows ld%8");
+  expect_reject(dnn_layernorm_q8_mx(buf + 8, 64, nullptr, nullptr, p, 128, p, 4, 64, 128, 1e-5f, 0, st),
+                "standardised rows off 16 bytes");
   // attention
+  auto rope = [&](int K, int hd, int T, const float* table) {
+    return dnn_gemm_bf16_qkv_rope(p, K, p, K, 1e-5f, f, p, p, p, ip, 1, T, 2, 1, hd, 512, K, table, table, 0, st);
+  };
+  expect_eq(rope(96, 128, 300, f), -3, "rotating projection K%64");
+  expect_eq(rope(128, 64, 300, f), -3, "rotating projection hd=64");
+  expect_eq(rope(128, 128, 300, f + 1), -3, "rotating projection tables off 16 bytes");
+  expect_eq(rope(128, 128, 0, f), -1, "rotating projection of nothing");
+  expect_eq(rope(128, 128, 300, nullptr), -1, "rotating projection without tables");
+  auto mx = [&](int T, int H, int Hkv, int hd, int ld8) {
+    return dnn_flash_attn_mx(p, p, p, p, ld8, p, 1, T, H, Hkv, hd, T, ip, 0.1f, st);
+  };
+  expect_eq(mx(64, 6, 4, 64, 384), -1, "flash that quantises H%Hkv");
+  expect_eq(mx(64, 5, 5, 64, 320), -1, "flash that quantises, row too short");
+  expect_eq(mx(64, 4, 4, 128, 512), -3, "flash that quantises hd=128");
+  expect_eq(mx(2048, 4, 4, 64, 256), -3, "flash that quantises, long");
+  const RowBlock block = {p, p, p, p, f, f, f, f, f, f};
+  auto row = [&](int n, int M, int d, int H, int hd, int S) {
+    return dnn_decode_row_blocks(&block, n, p, p, p, p, p, f, buf, buf, 0, M, d, H, H, hd, S, ip, 0.1f, 1e-5f, st);
+  };
+  expect_eq(row(0, 1, 768, 12, 64, 64), -3, "row step without blocks");
+  expect_eq(row(1, 3, 768, 12, 64, 64), -3, "row step of three rows");
+  expect_eq(row(1, 1, 1280, 20, 64, 64), -3, "row step width 1280");
+  expect_eq(row(1, 1, 768, 6, 128, 64), -3, "row step hd=128");
+  expect_eq(row(1, 1, 768, 12, 64, 2048), -3, "row step of a split cache");
+  expect_reject(dnn_attn_decode_proj(p, 2304, p, p, p, f, 0, 12, 64, ip, 0.1f, st), "attention and projection of nothing");
+  expect_reject(dnn_attn_decode_proj(p, 2296, p, p, p, f, 1, 12, 64, ip, 0.1f, st), "attention and projection, row too short");
+  expect_reject(dnn_attn_decode_proj(p, 2308, p, p, p, f, 1, 12, 64, ip, 0.1f, st), "attention and projection ld%8");
   expect_reject(dnn_qkv_split(p, p, p, p, 1, 1, 4, 4, 24, 16, ip, nullptr, nullptr, 0, st), "qkv_split hd%16");
   expect_reject(dnn_qkv_split(p, p, p, p, 1, 1, 6, 4, 64, 16, ip, nullptr, nullptr, 0, st), "qkv_split H%Hkv");
   expect_reject(dnn_flash_attn(p, p, p, p, 1, 8, 6, 4, 64, 16, ip, 0.1f, st), "flash H%Hkv");

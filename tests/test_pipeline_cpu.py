@@ -99,6 +99,25 @@ def test_a_replaced_forward_is_not_passed_by(what, monkeypatch):
     assert pipe.stages[0].keeps_input == (what == "last")
 
 
+@pytest.mark.parametrize("buf", ["h", "probs", "keep"])
+def test_the_native_call_writes_plain_buffers_only(buf, monkeypatch):
+    """It checks nothing itself: each buffer by itself, of another type, shape or order, or a keep on the images."""
+    from distributed_neural_networks_amd.models.cifar import NeuralNetwork
+    from distributed_neural_networks_amd.ops import cifar as cops
+    from distributed_neural_networks_amd.runtime.stages import CifarHipStage
+    native = []
+    monkeypatch.setattr(cops, "pass_few", lambda *a: native.append(1))
+    sd, cpu = NeuralNetwork().state_dict(), torch.device("cpu")
+    first, last = CifarHipStage(sd, 0, 1, cpu), CifarHipStage(sd, 2, 3, cpu)
+    x, good = torch.zeros(4, 3, 32, 32), {"h": torch.zeros(4, 4096), "probs": torch.zeros(4, 10), "keep": torch.zeros(4, 3, 32, 32)}
+    assert first.pass_few(last, x, **good) is not None and native == [1]
+    t = good[buf]
+    bad = [t.double(), t[:3], t[..., :-1], torch.zeros(8, *t.shape[1:])[::2], torch.zeros(t.shape[::-1]).permute(*range(t.dim())[::-1])]
+    for b in bad + ([x, x.view(-1).as_strided(x.shape, x.stride())] if buf == "keep" else []):
+        assert first.pass_few(last, x, **{**good, buf: b}) is None, (b.dtype, b.shape, b.stride())
+    assert native == [1]
+
+
 def test_a_sync_behind_every_kernel_needs_every_launch_by_itself(monkeypatch):
     """DNN_DEBUG_SYNC names the launch that a fault is of."""
     from distributed_neural_networks_amd.models.cifar import NeuralNetwork
