@@ -11,17 +11,19 @@
 // Here:
 //   * a workgroup owns BN output columns (NW waves x NT 16-column
 //     tiles: 128 as 4 x 2 or 8 x 1, 112 as 7 x 1) and ONE K range; the waves share the A rows of that range, staged
-//     through LDS in full 512-B row segments (global_load_dwordx4 -> ds_write),
+//     through LDS in full row segments of SB bytes (global_load_dwordx4 -> ds_write),
 //     so A crosses the load path once per workgroup: A : W bytes = M : BN;
 //   * each wave streams its own weight tiles straight to VGPRs (guide: GEMV
 //     row — no LDS round trip), non-temporally (read once), two K-steps of
-//     weights in flight (16 KiB per wave);
+//     weights in flight (NT tiles x SB bytes of 16 rows: 16 KiB a step of a wave with
+//     4 x 2 tiles and SB 512, 4 with one tile and 256);
 //   * narrow N is split over K across workgroups (SPLIT): fp32 partial slabs
 //     [splitk][Mp][Ns] in a caller workspace, summed by gemm_stream_reduce with
 //     the epilogue (bias / act / residual / fused norm / fp8 channel scale).
 //
-// LDS image of one A step: Mp rows x 512 B, 16-B slot j of row r stored at
-// j ^ (r & 15): conflict-free for the 4 ds_read_b128 lane groups of every
+// LDS image of one A step: Mp rows x SB bytes (512, or 256 with one tile a wave), 16-B
+// slot j of row r stored at j ^ (r & 15), which stays in the row where rows are whole
+// groups of 16 slots: conflict-free for the 4 ds_read_b128 lane groups of every
 // fragment read (bf16: slot 4c+g, W8: 8c+2g+h) and for the ds_write_b128 of
 // the staging pass (checked exhaustively offline).
 //
@@ -36,12 +38,12 @@
 
 namespace dnn {
 
-constexpr int STR_SB = 512;  // A bytes per row per K-step (bf16: 8 chunks of 32 k; W8: 4 chunks of 64 k), halved with one tile a wave
+constexpr int STR_SB = 512;  // SB of two tiles a wave, and what a slice of K is whole steps of (bf16: 8 chunks of 32 k; W8: 4 of 64 k)
 
 template <bool W8>
 struct StrCfg {
   static constexpr int ACH = W8 ? 128 : 64;  // A bytes per row per 64-B weight chunk
-  static constexpr int CS = STR_SB / ACH;    // weight chunks per K-step
+  static constexpr int CS = STR_SB / ACH;    // weight chunks in STR_SB
   static constexpr int AU = W8 ? 2 : 1;      // 16-B A pieces per chunk per lane
 };
 
@@ -214,6 +216,7 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_stream_kernel(const uint8_t* 
   constexpr int ACH = Cfg::ACH, CS = SB / ACH, AU = Cfg::AU;
   static_assert(NW == 4 || !FOLD, "");
   static_assert(NW >= MT, "a wave a row tile's statistics");
+  static_assert(SB % 256 == 0, "a slot's place is in its row");
   constexpr int MP = MT * 16;
   constexpr int BN = 16 * NW * NT;
   constexpr int APASS = (MP * SB + NW * 1024 - 1) / (NW * 1024);  // 16-B staging loads per thread per step
@@ -239,7 +242,7 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_stream_kernel(const uint8_t* 
     ct = ct < ntile16 ? ct : ntile16 - 1;
     wp[j] = Wsh + ((size_t)ct * nch + c0) * 1024 + lane * 16;
   }
-  // staging pass p: flat byte p*NW*1024 + tid*16 of the step's [MP][512] A image (past its end: the last piece again)
+  // staging pass p: flat byte p*NW*1024 + tid*16 of the step's [MP][SB] A image (past its end: the last piece again)
   const uint8_t* ap[APASS];
   int aoff[APASS], aslot[APASS];
 #pragma unroll
