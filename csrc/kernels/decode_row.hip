@@ -20,7 +20,9 @@
 //
 // GPT-2, 12 blocks and the head, graph, us of the separate launches : this: one row behind 100 tokens 268 :
 // 186, behind 900 313 : 225; two rows 275 : 209, 318 : 242.  A row more is 20 us of partials: three
-// would take 230 (separate 280), four 255.
+// would take 230 (separate 280), four 255.  us a block, one row behind 100 and 1000 tokens, two rows behind both:
+// width 256 17.1 : 12.2, 20.6 : 15.0, 18.1 : 13.4, 20.8 : 16.0; 768 18.1 : 13.8, 20.7 : 17.4, 18.1 : 15.7, 20.8 : 18.8; 1024
+// 22.4 : 16.1, 26.2 : 19.1, 22.5 : 17.5, 26.5 : 20.4.
 //
 // The rows are rounded to bf16 where the separate launches store them, sums are fp32.
 #include "attention_row.h"
@@ -199,6 +201,10 @@ static void row_slices_d(int ch, const RowProj& p, hipStream_t st) {
 }
 
 // fp32 elements of `parts` that a step of M rows of width d uses, 0: not a step for these kernels.
+// Caches below 2048 keys: from there on the separate attention splits a head's keys over workgroups, this one never, and
+// each of a head's H / 2 groups of columns reads them again: 3.0 us more a block for 1000 keys more where the split one
+// pays 0.7 (width 768, one row, a cache of 2047 keys behind 2000 tokens 20.5, the split one of 4096 21.4 there and 22.7
+// behind 4000).  The cache's size is what the host knows.
 extern "C" long long dnn_decode_row_parts(int M, int d, int H, int Hkv, int hd, int S) {
   if (M < 1 || M > DECODE_ROWS || row_chunks(d) == 0 || hd != 64 || H * hd != d || H != Hkv || S < 1 || S >= 2048) return 0;
   return (long long)M * d * (H + RP_SLICES);

@@ -255,7 +255,8 @@ static bool lean_gemm(const LeanArgs& p, int nch, hipStream_t st) {
     //   its O                  32 rows 1 x 1 424, 2 x 1 406; 64 rows 550, on 8 waves 523, on 4 520
     //   its gate | up          8 rows 1 x 1 343 (before: 335), 16 rows 371 (383), 1 x 2 381; 32 rows 2 x 2 429 (gemm_stream 414)
     //   its down               2 x 1 32 rows 419, 64 rows 603, 4 x 1 583 (gemm_stream 414, 541)
-    // Two rows or fewer of GPT-2's widths: decode_row.hip.  Other widths have not been laid out or measured.
+    // Two rows or fewer of GPT-2's widths: decode_row.hip.  These are the widths of GPT-2, XL in e4m3 and Llama-3 8B; GPT-2 medium
+    // and large, XL in bf16 and others in e4m3 have not been laid out or measured, and run on the general kernels.
     auto al = [](const void* x, int a) { return ((uintptr_t)x & (a - 1)) == 0; };
     if (p.W == nullptr || p.M < 1 || p.M > 64 || p.N % 16 != 0 || p.N > (RES ? 4096 : is_glu(ACT) ? 65536 : 8192) || (is_glu(ACT) && p.bias != nullptr) || (p.R != nullptr) != RES ||
         (!RES && p.rs_out != nullptr) || p.lda_b % 16 != 0 || p.ldc % 4 != 0 || !al(p.A, 16) || !al(p.C, 8) ||

@@ -488,8 +488,9 @@ static long long g_stream_min_bytes = 8ll << 20;
 // fewer than 192 workgroups (most CUs idle), fewer than 6 K-steps per slice
 // (the prologue latency and the split's reduce launch not amortised), or an
 // unsplit K of fewer than 12 steps (small-K wide-N heads: the skinny kernel's
-// K-split waves ramp faster).  Measured wins: Llama-3 8B gate|up (no split,
-// 224 workgroups x 16 steps) and down (8 slices x 7 steps).
+// K-split waves ramp faster).  Steps are of STR_SB bytes and workgroups of 128 columns
+// here; what is launched may have more workgroups of fewer columns, and steps half as long
+// (launch_stream_mt).  Measured wins: Llama-3 8B gate|up (no split) and down (8 slices x 7 steps).
 static constexpr int STREAM_NT = 2, STREAM_MIN_STEPS = 6, STREAM_MIN_WGS = 192, STREAM_MAX_SPLIT = 16;
 
 template <bool W8>
@@ -525,8 +526,8 @@ static int launch_stream_mt(const void* A, int lda_b, const void* Wsh, const flo
   const int ntiles = (N + BN - 1) / BN, nch = kbytes / 64;
   const int kelems = W8 ? kbytes : kbytes / 2;
   const dim3 grid(ntiles * splitk), block(256);
-  // Gate and up of Llama-3 (28672 columns): 224 workgroups of 128 columns leave 32 CUs idle, and a CU streams no faster for
-  // it; as 256 of 112 every CU has one.  Steps of 256 bytes of K: the first and the last step have nothing beside them.  us a
+  // 112 columns where rounds of 256 workgroups end earlier with them.  Gate and up of Llama-3 (28672 columns): 224 workgroups
+  // of 128 columns leave 32 CUs idle, and a CU streams no faster for it; as 256 of 112 every CU has one.  Steps of 256 bytes of K: the first and the last step have nothing beside them.  us a
   // step of 4 layers behind 100 tokens, as 128 columns, as 112, with 256 bytes (1024): 32 rows 395, 386, 384 (394); 64 rows 499, 461, 454 (544).
   if constexpr (!W8 && NORM == NORM_RMS && ACT == ACT_SILU_MUL) {
     constexpr int W = 7, BN7 = 16 * W;
@@ -627,7 +628,10 @@ static bool os_plan(int M, int N, int kbytes, bool have_ws, long long ws_bytes, 
       // launches, weights rotated past the MALL): 33..64 rows, the whole K in
       // one slice — GPT-2 (bf16, K 768): QKV 5.39 -> 4.76, O 3.66 -> 3.10,
       // c_fc 5.46 -> 4.80 us; GPT-2 XL (W8, K 1600): QKV 9.69 -> 8.35, O
-      // 5.79 -> 5.00, c_fc 9.70 -> 8.71 us.  Split-K shapes (c_proj K 3072 /
+      // 5.79 -> 5.00, c_fc 9.70 -> 8.71 us.  Of these the lean kernels
+      // (gemm_lean.hip) take by now what has row partials or a residual; a
+      // first block's QKV, whose rows no projection made, and other widths
+      // come here.  Split-K shapes (c_proj K 3072 /
       // 6400, every Llama-3 8B projection at 32 rows) measured slower: they
       // keep gemm_skinny / gemm_stream.
       // the 50304-wide heads measured slower (GPT-2 26.2 -> 36.3 us, XL W8

@@ -3,9 +3,12 @@
 // A pass of a few hundred tokens is a chain of 5 to 9 launches a block of 3 to 10 us
 // each; issued one by one from Python (10 us a launch: argument checks, tensor views,
 // the call) the device waits for the host: GPT-2, 66 to 256 tokens, 680 us for 63
-// launches that run 300.  The sequence, the kernels and their arguments are those of
-// runtime/transformer.py TransformerStage.step with T > 1 and folded norms; weights come
-// as pointers of this call, read from the stage's layers.
+// launches that run 300.  The sequence and what it computes are those of
+// runtime/transformer.py TransformerStage.step with T > 1 and folded norms, and so are the
+// kernels but for two that only this call launches: the q | k | v product that rotates
+// (dnn_gemm_bf16_qkv_rope: the bits of product and pass) and the attention that quantises its
+// rows (dnn_flash_attn_mx: the bytes of attention and quantiser).  Weights come as pointers of
+// this call, read from the stage's layers.
 #pragma once
 #include <cstdint>
 #include <vector>
