@@ -275,14 +275,20 @@ static bool lean_gemm(const LeanArgs& p, int nch, hipStream_t st) {
       if (nch != 128 || M <= 8 || M > 16) return false;
       LEAN_ONCE(4, 8, 4, 2, 1, 1);
     } else if constexpr (!W8 && NORM == NORM_RMS) {
-      if (nch != 128) return false;
+      // Fewer columns leave CUs idle, each wave with an eighth of K to itself; more of them are a second round.  us a launch, general :
+      // this (two small launches of 8 with it), 16 rows N 4096 13.4 : 14.5, 4608 15.6 : 13.4, 8192 17.5 : 16.7; 1 row 4608
+      // 15.1 : 14.3, 6144 15.8 : 16.2 (in a step of 4 layers 4 to 12 less), 8192 17.4 : 19.2; 32 rows 4096 14.9 : 15.9, 4608 19.9 : 16.4,
+      // 6144 20 : 16.9, 6656 21 : 25; 48 rows 2560 14.5 : 17, 3072 20 : 17.7, 6144 25.6 : 19.3, 6656 26 : 28; 64 rows 2048 14.2 : 17.1,
+      // 2560 20.3 : 17.3, 8192 31 : 29.5.
+      if (nch != 128 || p.N <= (M <= 32 ? 4096 : M <= 48 ? 2560 : 2048) || (p.N > 6144 && (M <= 8 || (M > 16 && M <= 48))))
+        return false;
       if (M <= 16) LEAN_ONCE(8, 4, 4, 2, 1, 2);
       else if (M <= 32) LEAN_ONCE(8, 4, 4, 2, 1, 3);
       else LEAN_ONCE(8, 4, 4, 2, 2, 3);
     } else if constexpr (!W8) {
       if (nch == 24) LEAN(4, 6, 1, 1, 1, 1);
       else if (nch == 96) LEAN(4, 6, 4, 2, 1, 1);
-      else if (nch != 128) return false;
+      else if (nch != 128 || (M > 32 && p.N <= 1024)) return false;  // 64 rows, 64 columns 11.1 : 12.0, 768 12.5 : 12.9, 1280 13.8 : 13.0
       else if (M <= 16) LEAN_ONCE(8, 4, 4, 4, 1, 1);
       else if (M <= 32) LEAN(8, 4, 4, 3, 2, 1);
       else LEAN_ONCE(4, 8, 4, 2, 2, 1);

@@ -81,7 +81,7 @@ def test_residual_projection(M, K, N, w8):
     assert torch.allclose(rs.view(M, -1, 2)[:, :N // 16, 1], (t - t.mean(-1, keepdim=True)).square().sum(-1), rtol=1e-5, atol=1e-5)
 
 
-@pytest.mark.parametrize("M,N,act", [(m, n, 0) for m in (1, 9, 16, 17, 31, 32, 33, 48, 49, 64) for n in (6144, 80)]
+@pytest.mark.parametrize("M,N,act", [(m, n, 0) for m in (1, 9, 16, 17, 31, 32, 33, 48, 49, 64) for n in (6144, 5200)]
                          + [(9, 28672, 3), (16, 28672, 3), (13, 48, 3)])
 def test_rms_projection(M, N, act):
     from distributed_neural_networks_amd.ops.gemm import attach_shuffled, fold_norm, linear_norm
@@ -100,6 +100,34 @@ def test_rms_projection(M, N, act):
         z, size = torch.nn.functional.silu(gate) * up, 1.1 * sg * up.abs() + gate.abs() * su
     assert _err(out[:M, :NO], z, size) < 1
     assert (out[M:] == 7).all() and (out[:, NO:] == 7).all()
+
+
+@pytest.mark.parametrize("M,N,lean", [(1, 4096, False), (1, 4112, True), (8, 6144, True), (8, 6160, False), (9, 4096, False),
+                                      (9, 6160, True), (16, 8192, True), (17, 4096, False), (17, 6144, True), (17, 6160, False),
+                                      (33, 2560, False), (48, 2576, True), (48, 6160, False), (49, 2048, False), (49, 2064, True),
+                                      (64, 8192, True), (64, 64, False)])
+def test_rms_projection_lines(M, N, lean):
+    """Columns that leave CUs idle or start a second round stay with the general kernels."""
+    from distributed_neural_networks_amd.ops.gemm import attach_shuffled, decode_workspace, fold_norm, linear_norm
+    K = 4096
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    f = attach_shuffled(fold_norm(torch.randn(N, K, generator=g, device=DEV) * 0.02, torch.ones(K, device=DEV), None, None, True, 1e-5, DEV))
+    out = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    assert ("gemm_lean" in _kernels(lambda: linear_norm(x, f, out=out, ws=decode_workspace(DEV, 7)))) == lean
+    xd = x.double() / (x.double().square().mean(-1, keepdim=True) + 1e-5).sqrt()
+    assert _err(out, xd @ f.w.double().t(), xd.abs() @ f.w.double().abs().t()) < 1
+
+
+@pytest.mark.parametrize("M,N,lean", [(32, 64, True), (33, 1024, False), (33, 1040, True), (64, 64, False)])
+def test_residual_projection_lines(M, N, lean):
+    from distributed_neural_networks_amd.ops.gemm import decode_workspace, linear, shuffle_weight
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x, W = torch.randn(M, 4096, generator=g, device=DEV).bfloat16(), (torch.randn(N, 4096, generator=g, device=DEV) * 0.02).bfloat16()
+    out, res, sh = (torch.empty(M, N, device=DEV, dtype=torch.bfloat16), torch.randn(M, N, generator=g, device=DEV).bfloat16(),
+                    shuffle_weight(W))
+    assert ("gemm_lean" in _kernels(lambda: linear(x, W, None, None, res, out, w_shuf=sh, ws=decode_workspace(DEV, 7)))) == lean
+    assert _err(out, x.double() @ W.double().t() + res.double(), x.double().abs() @ W.double().abs().t()) < 1
 
 
 def test_what_stays_with_the_general_kernels():
