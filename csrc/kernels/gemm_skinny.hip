@@ -552,11 +552,23 @@ static int launch_stream_mt(const void* A, int lda_b, const void* Wsh, const flo
                        eps, kelems, (float*)ws, cnt);
     return (int)hipGetLastError();
   }
-  // eight waves of a tile for four of two: twice the waves that wait (down, 32 rows: 23.6 -> 22.8 us); 256 bytes of K: 64
-  // rows, a step 454 -> 449
-  hipLaunchKernelGGL((gemm_stream_kernel<MT, 1, W8, NORM, ACT, true, false, 4 * NT, 256>), grid, dim3(256 * NT), 0, st,
-                     (const uint8_t*)A, lda_b, (const uint8_t*)Wsh, sw, C, ldc, bias, (const bf16_t*)R, ldr, M, N, nch, cps,
-                     colsum, eps, kelems, (float*)ws, (unsigned*)nullptr);
+  // Eight waves of a tile for four of two: twice the waves that wait (down, 32 rows: 23.6 -> 22.8 us); 256 bytes of K: 64
+  // rows, a step 454 -> 449, and two workgroups that share a CU (7 slices of 40 tiles, 11008 x 5120, 32 rows 39.7 -> 35.5).  With a
+  // residual and a CU or less for each workgroup there is less in flight so: up to 32 rows of bf16, 224 workgroups and fewer, 512
+  // bytes again (11008 x 4096 four of two 26.5, 256 bytes 28, 512 bytes 26.2; 8192 x 5120 25.7, 27.4, 25.8; 256
+  // workgroups, 14336 x 4096, 29, 28.3, 28.4); e4m3, four waves of two (64 rows, 14336 x 4096 27.4, 30, eight of 512 28.4; 14336 x
+  // 8192 36.7, 43.7, 39.4; 288 workgroups, 11008 x 6144, 40.6, 36.8).
+  auto split = [&](auto nt, auto sb) {
+    constexpr int T = decltype(nt)::value, SB = decltype(sb)::value, NW = BN / (16 * T);
+    hipLaunchKernelGGL((gemm_stream_kernel<MT, T, W8, NORM, ACT, true, false, NW, SB>), grid, dim3(NW * 64), 0, st,
+                       (const uint8_t*)A, lda_b, (const uint8_t*)Wsh, sw, C, ldc, bias, (const bf16_t*)R, ldr, M, N, nch, cps,
+                       colsum, eps, kelems, (float*)ws, (unsigned*)nullptr);
+  };
+  constexpr int few = NORM != NORM_NONE ? 0 : W8 ? 256 : MT <= 2 ? 255 : 0;
+  if constexpr (few > 0) {
+    if ((int)grid.x <= few) split(std::integral_constant<int, W8 ? NT : 1>{}, std::integral_constant<int, STR_SB>{});
+  }
+  if ((int)grid.x > few) split(std::integral_constant<int, 1>{}, std::integral_constant<int, 256>{});
   const int NO = is_glu(ACT) ? N / 2 : N;
   const long long threads = (long long)M * ((NO + 3) / 4);
   hipLaunchKernelGGL((gemm_stream_reduce<ACT, NORM, W8>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,

@@ -194,6 +194,33 @@ def _kernels(f):
     return " ".join(e.key for e in p.key_averages())
 
 
+@pytest.mark.parametrize("M,N,K,w8,form", [(17, 4096, 10240, False, "8, 512>"), (32, 4096, 11008, False, "8, 512>"),
+                                           (32, 4096, 14336, False, "8, 256>"), (33, 4096, 10240, False, "8, 256>"),
+                                           (17, 8192, 8192, True, "4, 512>"), (64, 4096, 14336, True, "4, 512>"),
+                                           (64, 6144, 11008, True, "8, 256>")])
+def test_split_forms(M, N, K, w8, form):
+    """Waves and bytes of a row a step on both sides of a workgroup a CU, against float64: bf16 storage, and fp32 sums."""
+    from distributed_neural_networks_amd.ops.fp8 import linear_w8, quantize_weight
+    from distributed_neural_networks_amd.ops.gemm import attach_shuffled, decode_workspace, linear, shuffle_weight
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x, W = torch.randn(M, K, device=DEV, generator=g).bfloat16(), torch.randn(N, K, device=DEV, generator=g) / math.sqrt(K)
+    R, out = torch.randn(M, N, device=DEV, generator=g).bfloat16(), torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    ws = decode_workspace(DEV, 7)
+    if w8:
+        w = attach_shuffled(quantize_weight(W, DEV))
+        wd = w.q[:, :K].double() * w.scale.double()[:, None]
+        run = lambda: linear_w8(x, w, None, 0, R, out, ws=ws)  # noqa: E731
+    else:
+        w = W.bfloat16()
+        sh, wd = shuffle_weight(w), w.double()
+        run = lambda: linear(x, w, residual=R, out=out, w_shuf=sh, ws=ws)  # noqa: E731
+    names = _kernels(run)
+    assert "gemm_stream_kernel" in names and "gemm_stream_reduce" in names and form in names, names
+    ref = x.double() @ wd.t() + R.double()
+    size = x.double().abs() @ wd.abs().t()
+    assert ((out.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -17 * size).all()
+
+
 @pytest.mark.parametrize("M,N,K,norm", [(17, 3072, 4096, 0), (64, 3072, 4096, 0), (32, 4096, 4096, 0), (32, 4096, 4096, 1),
                                         (64, 640, 1024, 0), (64, 2048, 2048, 2)])
 @pytest.mark.parametrize("what", ["stream", "stream split", "stream fold", "one-shot", "one-shot pinned"])
