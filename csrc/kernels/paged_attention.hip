@@ -287,9 +287,28 @@ __device__ __forceinline__ void paged_decode_part(const PagedAttnArgs& a, const 
 
   const bf16_t* rowp = reinterpret_cast<const bf16_t*>(a.qkv) + (size_t)row * a.ldq;
   const bool own = !written && ue == u.total && ue > ub && wave == (u.total - 1 - ub) % NW;  // this wave has the token's unit
+  auto store_own = [&]() {
+    const int page = pa_page(a, slot, p / PG);
+    if (page < 0) return;
+    bf16_t* kd = reinterpret_cast<bf16_t*>(a.kp) + (((size_t)page * a.G + g) * PG + p % PG) * DK;
+    bf16_t* vd = reinterpret_cast<bf16_t*>(a.vp) + (((size_t)page * a.G + g) * PG + p % PG) * DV;
+    if (lane < DK / 8)
+      *reinterpret_cast<uint4*>(kd + lane * 8) = *reinterpret_cast<const uint4*>(rowp + a.H * DK + g * DK + lane * 8);
+    if (lane < DV / 8)
+      *reinterpret_cast<uint4*>(vd + lane * 8) = *reinterpret_cast<const uint4*>(rowp + (a.H + a.G) * DK + g * DV + lane * 8);
+  };
+  // Heads of 256 have no register left for the row's own addresses, the pages and the gate (31 spilled for 18; 4 heads over 2, us a
+  // launch and two small ones, 1 to 64 sequences of 300 keys 23 to 27 for 21 to 25, 32 of 4000 76 for 68): their token is stored
+  // first and read back.
+  constexpr bool WIDE = DK + DV >= 512;
+  if constexpr (WIDE) {
+    if (own) store_own();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
   // pages of the wave's first 64 units, a lane each
   int pages = 0;
-  {
+  if constexpr (!WIDE) {
     const int i = ub + wave + lane * NW;
     if (i < ue) pages = pa_page(a, slot, u.at(i) / (PG / DU));
   }
@@ -313,11 +332,11 @@ __device__ __forceinline__ void paged_decode_part(const PagedAttnArgs& a, const 
   f32x4 ksc[4];
   auto load = [&](int i) __attribute__((always_inline)) {
     const int unit = u.at(i), k = (i - ub) / NW;
-    const int page = max(k < 64 ? __builtin_amdgcn_readlane(pages, k) : pa_page(a, slot, unit / (PG / DU)), 0);
+    const int page = max(!WIDE && k < 64 ? __builtin_amdgcn_readlane(pages, k) : pa_page(a, slot, unit / (PG / DU)), 0);
     const size_t k0 = ((size_t)page * a.G + g) * PG + (unit % (PG / DU)) * DU;
     const bf16_t* kb = reinterpret_cast<const bf16_t*>(a.kp) + (k0 + r32) * DK + 8 * h;
     const bf16_t* vb = reinterpret_cast<const bf16_t*>(a.vp) + k0 * DV;
-    const int at = own && i == ue - 1 ? p - unit * DU : -1;  // the token's own row of the tile
+    const int at = !WIDE && own && i == ue - 1 ? p - unit * DU : -1;  // the token's own row of the tile
     if (r32 == at) kb = rowp + (a.H + g) * DK + 8 * h;
     if (!a.shared) {
 #pragma unroll
@@ -415,7 +434,7 @@ __device__ __forceinline__ void paged_decode_part(const PagedAttnArgs& a, const 
     }
     if (ns == 1) {
       reinterpret_cast<bf16_t*>(a.out)[(size_t)row * a.ldo + head * DV + c] =
-          f2bf((l > 0.f ? v / l : 0.f) * (x == tid ? gate0 : pa_gate(a, row, head) * pa_gate_el(a, row, head * DV + c)));
+          f2bf((l > 0.f ? v / l : 0.f) * (!WIDE && x == tid ? gate0 : pa_gate(a, row, head) * pa_gate_el(a, row, head * DV + c)));
     } else {
       float* d = ws + (((size_t)e * a.H + head) * ns + z) * (DV + 2);
       if (c == 0) {
@@ -425,16 +444,7 @@ __device__ __forceinline__ void paged_decode_part(const PagedAttnArgs& a, const 
       d[2 + c] = v;
     }
   }
-  if (own) {  // behind every read of the page by this workgroup; another one of the same head takes the row's own as well
-    const int page = pa_page(a, slot, p / PG);
-    if (page < 0) return;
-    bf16_t* kd = reinterpret_cast<bf16_t*>(a.kp) + (((size_t)page * a.G + g) * PG + p % PG) * DK;
-    bf16_t* vd = reinterpret_cast<bf16_t*>(a.vp) + (((size_t)page * a.G + g) * PG + p % PG) * DV;
-    if (lane < DK / 8)
-      *reinterpret_cast<uint4*>(kd + lane * 8) = *reinterpret_cast<const uint4*>(rowp + a.H * DK + g * DK + lane * 8);
-    if (lane < DV / 8)
-      *reinterpret_cast<uint4*>(vd + lane * 8) = *reinterpret_cast<const uint4*>(rowp + (a.H + a.G) * DK + g * DV + lane * 8);
-  }
+  if (!WIDE && own) store_own();  // behind every read of the page by this workgroup; another one of the same head takes the row's own as well
 }
 
 // grid (G * head tiles, sequences, splits)

@@ -41,3 +41,17 @@ def test_no_spill_between_k_tiles():
         loops = list(main_loops(asm, kernel))
         assert len(loops) == count and all(sum("v_mfma" in ln for ln in lp) >= 32 for _, lp in loops)
         assert [n for n, lp in loops if any("scratch_" in ln for ln in lp)] == []
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+def test_paged_decode_spills():
+    """Heads of 256 fill the registers: the row's own addresses and the pages beside them spilled 31 and took 10 % longer."""
+    from distributed_neural_networks_amd.ops import build as b
+    src = os.path.join(b.CSRC, "kernels", "paged_attention.hip")
+    with tempfile.TemporaryDirectory() as d:
+        r = subprocess.run([HIPCC] + b._flags(src) + ["-c", "--cuda-device-only", "-Rpass-analysis=kernel-resource-usage", src,
+                                                      "-o", os.path.join(d, "p.o")], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    spilled = {m.group(1): int(m.group(2)) for m in
+               re.finditer(r"Function Name: _ZN3dnn19paged_decode_kernelI(\S+?)EEE.*?VGPRs Spill: (\d+)", r.stderr, re.S)}
+    assert len(spilled) == 13 and spilled.pop("Li256ELi256ELi4") <= 20 and not any(spilled.values())
